@@ -198,5 +198,13 @@ def check(rc):
         raise WdError("wd error %d: %s" % (rc, load().wd_last_error().decode()))
 
 
+_fns = {}     # bound functions by name: a decode step makes hundreds of calls of a few microseconds each
+
+
 def call(name, *args):
-    check(getattr(load(), name)(*args))
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(load(), name)
+    rc = fn(*args)
+    if rc:
+        check(rc)
