@@ -1,0 +1,60 @@
+"""The layer dispatches at the sizes where the choice of a kernel or the end of a tile changes: super-blocks per gate/up row
+around the passes of eight and the two fetches, down rows around the 16-block passes, router rows of one and two waves,
+experts around the 64-logit registers of the selection, tensors that are only 2-byte aligned."""
+import numpy as np
+import pytest
+
+from warpdecode_amd import synth
+from test_gpu_layer import SEED, check_layer
+
+pytestmark = pytest.mark.gpu
+IQ3, IQ2, Q8, IQ4 = synth.IQ3_S, synth.IQ2_S, synth.Q8_0, synth.IQ4_NL
+
+
+@pytest.fixture(scope="module")
+def g():
+    import gpu_util
+    gpu_util.init()
+    return gpu_util
+
+
+SHAPES = [
+    (256, 64, 8, 8, IQ3, IQ4, True),         # one super-block, every expert selected
+    (1792, 1536, 136, 10, IQ2, Q8, False),   # a last pass of seven, down rows of 48 blocks
+    (2304, 544, 72, 9, IQ3, IQ4, True),      # nine super-blocks (a pass of one), an unpaired 17th down block
+    (2304, 800, 64, 8, IQ4, IQ4, True),      # 72 gate blocks: a second pass of eight
+    (2816, 1568, 264, 5, IQ4, IQ4, False),   # 49 down blocks: beyond what is held in flight
+    (3328, 160, 200, 7, Q8, Q8, True),       # five down blocks
+    (4096, 1056, 24, 3, IQ2, Q8, True),      # sixteen super-blocks, 33 down blocks
+    (4352, 64, 520, 2, IQ3, Q8, True),       # beyond the aligned fetch and the paired router rows
+    (1024, 96, 128, 15, IQ4, Q8, True),      # the largest selection of one wave
+    (3072, 1536, 16, 16, IQ3, IQ4, True),    # items beyond the device, 17 matrices
+]
+
+
+@pytest.mark.parametrize("H,F,E,k,gate,down,shared", SHAPES)
+def test_layer_shapes(g, oracle, H, F, E, k, gate, down, shared):
+    L = synth.make_layer(H, F, E, k, gate, down, shared, seed=SEED, layer=H + F, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 61, H + F), H)
+    check_layer(g, oracle, L, x)
+    ids = synth.rng_for(SEED, 62, H + F).permutation(E)[:k].astype(np.int32)   # known before the launch
+    check_layer(g, oracle, L, x, ids=ids, weights=np.linspace(0.3, 0.05, k).astype(np.float32), flags=1)
+
+
+@pytest.mark.parametrize("H,F,k", [(2048, 512, 16), (2560, 640, 4), (3072, 96, 3)])
+def test_tensors_on_two_byte_boundaries(g, oracle, monkeypatch, H, F, k):
+    import torch
+    E = 16
+    L = synth.make_layer(H, F, E, k, IQ3, Q8, True, seed=SEED, layer=H + 1, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 63, H), H)
+    aligned = g.dev
+
+    def dev(a):
+        if a.dtype != np.uint8:
+            return aligned(a)
+        t = torch.empty(a.size + 16, dtype=torch.uint8, device="cuda")[2:2 + a.size]
+        t.copy_(torch.from_numpy(np.ascontiguousarray(a).reshape(-1)))
+        return t
+
+    monkeypatch.setattr(g, "dev", dev)
+    check_layer(g, oracle, L, x)

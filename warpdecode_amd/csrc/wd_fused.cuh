@@ -1,10 +1,10 @@
 // Fused MoE layer: two dispatches per layer (three when the caller asks for the split form).
-//   AB router logits (+ shared-expert gate logit), one row per wave; the router workgroup that finishes last
+//   AB router logits (+ shared-expert gate logit), a wave or two per row; the router workgroup that finishes last
 //      runs softmax/top-k and publishes the ids inside the dispatch; the shared expert's gate/up + SwiGLU and
 //      the routed gate/up + SwiGLU run in the same launch: the routed workgroups quantise x and stage the
-//      codebooks while the router runs and pick the ids up as soon as they appear
-//      (k_layer_a + k_layer_b are the same work as two launches: ids given by the caller, IQ4_NL gate/up,
-//      or WD_MOE_SPLIT_AB)
+//      codebooks while the router runs and pick the ids up as soon as they appear - or request their weights at
+//      once when the ids are known before the launch (given by the caller, or by a routing trace).
+//      The same kernel with only the first or only the last of these parts is the split form.
 //   C  Q8_0 re-quantisation of the k+1 activations, all down projections, the ordered weighted
 //      sum, the gated shared branch and the optional residual update
 // Activation quantisation is redone by every workgroup that needs it (8 KB of f32 from L2 and a
@@ -38,8 +38,10 @@ struct LayerArgs {
     int hc, hc_round_half;
     int dry;                     // measurement aid: every workgroup returns at once
     int preselected;
-    int n_router_wgs;            // workgroups of dispatch A that take router rows
-    int n_routed_items;          // merged dispatch: (expert rung, group of eight rows) items shared by the routed workgroups
+    int n_router_wgs;            // workgroups of dispatch AB that take router rows,
+    int n_shared_wgs;            // those that take the shared expert's gate/up (the rest: routed gate/up)
+    int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
+    const int32_t *ids_known;    // null, or the k ids where they are known before the launch
     unsigned *arrive;            // device counter of finished router workgroups (zero between dispatches)
     uint32_t *ids_tagged;        // [kTagCopies][16] selected ids published inside the merged dispatch (kTagInvalid = not yet)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
@@ -130,8 +132,6 @@ WD_DEV void wave_quantize_q8_k_regs(const float4 &v, int8_t *qs256, float *d, in
 // Lanes 0..k-1 write ids/weights through the given pointers (LDS or global).
 // src/qwen38_moe.cuh:711-818: softmax over all experts with the per-8 sums accumulated in a double in
 // ascending order, k rungs of "largest remaining probability, lowest index on ties", renormalise.
-// COHERENT: the logits were written by other workgroups of the same dispatch; they are read with
-// device-scope atomic loads so that no stale cached copy can be seen.
 // Wave-wide exact sum of doubles (any order gives the same bits when the caller has made sure that the sum is
 // exact); the result is uniform.
 WD_DEV double wave_sum_exact_f64(double v) {
@@ -187,7 +187,7 @@ WD_DEV double sum_groups(const float (&gs)[M], int groups, int lane) {
 
 // Softmax of the row: lane l ends up with the probabilities of its 8-expert group(s) in v (or -inf everywhere
 // when every exponential vanished: `dead`).
-template <int M, bool COHERENT>
+template <int M>
 WD_DEV void softmax_probs(const float *logits, int n, int lane, float (&v)[8 * M], bool &dead) {
     const int groups = n >> 3;
     float mx = -INFINITY;
@@ -195,16 +195,10 @@ WD_DEV void softmax_probs(const float *logits, int n, int lane, float (&v)[8 * M
     for (int m = 0; m < M; ++m) {
         const int g = lane + 64 * m;
         if (g < groups) {
-            if (COHERENT) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    v[8 * m + i] = __hip_atomic_load(logits + g * 8 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                const float4 a = *reinterpret_cast<const float4 *>(logits + g * 8);
-                const float4 b = *reinterpret_cast<const float4 *>(logits + g * 8 + 4);
-                v[8 * m + 0] = a.x, v[8 * m + 1] = a.y, v[8 * m + 2] = a.z, v[8 * m + 3] = a.w;
-                v[8 * m + 4] = b.x, v[8 * m + 5] = b.y, v[8 * m + 6] = b.z, v[8 * m + 7] = b.w;
-            }
+            const float4 a = *reinterpret_cast<const float4 *>(logits + g * 8);
+            const float4 b = *reinterpret_cast<const float4 *>(logits + g * 8 + 4);
+            v[8 * m + 0] = a.x, v[8 * m + 1] = a.y, v[8 * m + 2] = a.z, v[8 * m + 3] = a.w;
+            v[8 * m + 4] = b.x, v[8 * m + 5] = b.y, v[8 * m + 6] = b.z, v[8 * m + 7] = b.w;
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[8 * m + i] = -INFINITY;
@@ -286,16 +280,28 @@ WD_DEV void finish_weights(float top_mine, int id_mine, int k, float w_scale, in
     }
 }
 
-template <int M, bool COHERENT>
+template <int M>
 WD_DEV void topk_wave_m(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
                         const int32_t *__restrict__ override_ids, int lane) {
     float v[8 * M];
     bool dead;
-    softmax_probs<M, COHERENT>(logits, n, lane, v, dead);
+    softmax_probs<M>(logits, n, lane, v, dead);
     float top_mine;
     int id_mine;
     rungs_on_probs<M>(v, k, lane, top_mine, id_mine);
     finish_weights(top_mine, id_mine, k, w_scale, ids, weights, override_ids, lane);
+}
+
+// The ids held by lanes 0..k-1 (k <= 16) into the `copies` replicas: into every row of 16 lanes first, then four replicas
+// per store instruction, so that the last replica goes out a quarter of the stores after the first.
+WD_DEV void publish_ids(int id_mine, int k, uint32_t *tagged, int copies, int lane) {
+    const wd_uint2v t16 = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(id_mine), static_cast<uint32_t>(id_mine), false, false);
+    const wd_uint2v t32 = __builtin_amdgcn_permlane32_swap(t16.x, t16.x, false, false);
+    const int j = lane & 15, c4 = lane >> 4;
+#pragma unroll 4
+    for (int c0 = 0; c0 < copies; c0 += 4)
+        if (j < k && c0 + c4 < copies)
+            __hip_atomic_store(tagged + (c0 + c4) * 16 + j, t32.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The same selection by a workgroup of eight waves (every thread must call it; it contains barriers).
@@ -449,15 +455,7 @@ WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *w
     const bool all_good = __builtin_amdgcn_ballot_w64(good) == ~0ull;
     int id_mine = override_ids ? id_given : idc;
     if (all_good && tagged) {
-        // the ids (lanes 0..k-1, k <= 16) into every row of 16 lanes, then four replicas per store instruction: the last
-        // replica goes out a quarter of the stores after the first
-        const wd_uint2v t16 = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(id_mine), static_cast<uint32_t>(id_mine), false, false);
-        const wd_uint2v t32 = __builtin_amdgcn_permlane32_swap(t16.x, t16.x, false, false);
-        const int j = lane & 15, c4 = lane >> 4;
-#pragma unroll 4
-        for (int c0 = 0; c0 < copies; c0 += 4)
-            if (j < k && c0 + c4 < copies)
-                __hip_atomic_store(tagged + (c0 + c4) * 16 + j, t32.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        publish_ids(id_mine, k, tagged, copies, lane);
     }
     WD_STAMP(6);
 
@@ -480,12 +478,7 @@ WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *w
             }
         rungs_on_probs<M>(v, k, lane, top_mine, id_mine);
         if (override_ids) id_mine = id_given;
-        if (tagged && lane < k) {
-#pragma unroll 4
-            for (int c = 0; c < copies; ++c)
-                __hip_atomic_store(tagged + c * 16 + lane, static_cast<uint32_t>(id_mine), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        }
+        if (tagged) publish_ids(id_mine, k, tagged, copies, lane);
     }
     finish_weights(top_mine, id_mine, k, w_scale, ids, weights, nullptr, lane);
     WD_STAMP(7);
@@ -518,31 +511,23 @@ WD_DEV void topk_block_m(const float *logits, int n, int k, float w_scale, int32
 #undef WD_STAMP
 }
 
-WD_DEV void topk_block(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
-                       const int32_t *__restrict__ override_ids, uint8_t *lds, int lane, int wave,
-                       unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
-    if (n <= 512)
-        topk_block_m<1>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-    else
-        topk_block_m<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-}
-
-template <bool COHERENT>
 WD_DEV void topk_wave(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
                       const int32_t *__restrict__ override_ids, int lane) {
     if (n <= 512)
-        topk_wave_m<1, COHERENT>(logits, n, k, w_scale, ids, weights, override_ids, lane);
+        topk_wave_m<1>(logits, n, k, w_scale, ids, weights, override_ids, lane);
     else
-        topk_wave_m<2, COHERENT>(logits, n, k, w_scale, ids, weights, override_ids, lane);
+        topk_wave_m<2>(logits, n, k, w_scale, ids, weights, override_ids, lane);
 }
 
-// ---- the same selection by ONE wave that holds eight logits per lane ------------------------------------------------
-// lv[j] is the logit of expert 64 j + lane (-inf at and beyond n; n <= 512, k <= 15).  A single wave pays for every trip
-// through LDS or the scalar unit with hundreds of idle cycles, so step A stays in the vector registers: every logit
-// becomes a 32-bit key - its bits mapped so that unsigned order is float order, the low nine bits replaced by
-// 511 - expert - , every lane sorts its eight keys (a network of 19 exchanges), and k + 1 rounds of "largest head of any
-// lane" (a DPP reduction; the lane that held it moves its keys up) give the k + 1 largest keys in order, key j in
-// lane j.  The keys order the logits up to their low nine bits, so the result is accepted as the selection only when
+// ---- the same selection by ONE wave that holds M = 1, 2, 4 or 8 logits per lane --------------------------------------
+// lv[j] is the logit of expert 64 j + lane (-inf at and beyond n; n <= 64 M, k <= 15).  A single wave's time is the length
+// of its dependent steps, so step A counts instead of searching: every logit becomes a 32-bit key - its bits mapped so that
+// unsigned order is float order, the low nine bits replaced by 511 - expert, so that keys are distinct -; the largest keys
+// of groups of lanes (pairs; quads when a lane has one key) are ranked among themselves by counting, one uniform read, a
+// compare and an add for each; T, the (k+1)-th largest of them, is a lower bound of the (k+1)-th largest key, and the keys
+// not below T - 16 or so of 512 - are compacted into LDS, one per lane, and ranked the same way.  (k + 1 rounds of "largest
+// head of any lane" over sorted lanes took 1.9 us for 512 experts, this 1.1.)
+// The keys order the logits up to their low nine bits, so the result is accepted as the selection only when
 //   * the keys' upper 23 bits are strictly decreasing over the k + 1 - any logit that was not taken then lies below
 //     the grid point at or below the k-th taken logit -, and
 //   * the exponentials e_0 > e_1 > ... > e_k of the k + 1 exact logits are strictly decreasing by a relative margin:
@@ -559,81 +544,81 @@ struct SelWaveState {
     bool fast;     // step A accepted the row (the same in every lane)
 };
 
-WD_DEV uint32_t wave_max_u32(uint32_t v) {  // the result is uniform
-    // (umax_step: written so that the shuffle and the maximum become one instruction)
-    v = umax_step<kDppXor1>(v);
-    v = umax_step<kDppXor2>(v);
-    v = umax_step<kDppRor4>(v);
-    v = umax_step<kDppRor8>(v);  // every lane: its row's largest
-    const wd_uint2v t = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    v = max(t.x, t.y);                                                                            // rows 0|2 and 1|3
-    return max(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 0)),
-               static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 16)));
-}
-
 // Step A.  Returns with st.fast, and for accepted rows the ids of the selection in lanes 0..k-1 of st.id.
-// Registers and cross-lane moves only: no LDS is written or read.
-WD_DEV void sel_wave_ids(const float (&lv)[8], int n, int k, int lane, SelWaveState &st) {
-    uint32_t h[8];
+// Of the scratch it uses the candidates' and the selection's places only (cl, cid, sel, selp).
+template <int M>
+WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s, int lane, SelWaveState &st) {
+    uint32_t h[M];
     bool odd = false;
     float lm = lv[0];
+    uint32_t head = 0u;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < M; ++j) {
         const int id = 64 * j + lane;
         odd = odd || lv[j] != lv[j];
         lm = __builtin_fmaxf(lm, lv[j]);
         const uint32_t b = f_bits(lv[j]);
         const uint32_t ord = b ^ ((b & 0x80000000u) ? 0xffffffffu : 0x80000000u);  // unsigned order = float order
         h[j] = id < n ? ((ord & ~0x1ffu) | static_cast<uint32_t>(511 - id)) : 0u;
+        head = max(head, h[j]);
     }
     const float mx = wave_max(lm);
-    auto exchange = [&](int i, int j) {  // the larger key to the lower register
-        const uint32_t hi = max(h[i], h[j]), lo = min(h[i], h[j]);
-        h[i] = hi, h[j] = lo;
-    };
-    exchange(0, 1), exchange(2, 3), exchange(4, 5), exchange(6, 7);
-    exchange(0, 2), exchange(1, 3), exchange(4, 6), exchange(5, 7);
-    exchange(1, 2), exchange(5, 6);
-    exchange(0, 4), exchange(1, 5), exchange(2, 6), exchange(3, 7);
-    exchange(2, 4), exchange(3, 5);
-    exchange(1, 2), exchange(3, 4), exchange(5, 6);
-    uint32_t mine = 0u;  // lane j: the j-th largest key of the row
-    for (int j = 0; j <= k; ++j) {
-        const uint32_t m = wave_max_u32(h[0]);
-        const bool won = h[0] == m;  // (keys are distinct: they end in the expert's number)
+    constexpr int kGroup = M == 1 ? 4 : 2;
+    head = umax_step<kDppXor1>(head);
+    if (M == 1) head = umax_step<kDppXor2>(head);
+    int larger = 0;
 #pragma unroll
-        for (int i = 0; i < 7; ++i) h[i] = won ? h[i + 1] : h[i];
-        h[7] = won ? 0u : h[7];
-        mine = lane == j ? m : mine;
+    for (int g = 0; g < 64 / kGroup; ++g) larger += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(head), g * kGroup)) > head ? 1 : 0;
+    // (with k groups or fewer that hold experts - at most 64 of these then - every key is a candidate)
+    const unsigned long long at = __builtin_amdgcn_ballot_w64(larger == k);
+    const uint32_t thr = at ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(head), __builtin_ctzll(at))) : 0u;
+    uint32_t *const ck = reinterpret_cast<uint32_t *>(s.cid);
+    int count = 0;
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+        const bool c = h[j] >= thr && h[j] != 0u;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(c);
+        const int pos = count + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u)));
+        if (c && pos < 64) ck[pos] = h[j], s.cl[pos] = lv[j];
+        count += static_cast<int>(__builtin_popcountll(m));
     }
-    // the exact logit behind key j: register idc / 64 of lane idc % 64
+    wave_lds_fence();
+    const uint32_t key = lane < count ? ck[lane] : 0u;
+    const float key_l = s.cl[lane];
+    int rank = 0;
+    const int steps = (min(count, 64) + 3) & ~3;  // lanes past the list hold zero, which is ahead of nothing
+    for (int src = 0; src < steps; src += 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) rank += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), src + u)) > key ? 1 : 0;
+    }
+    if (key != 0u && rank <= k) s.sel[rank] = static_cast<int>(key), s.selp[rank] = key_l;
+    wave_lds_fence();
+    const uint32_t mine = lane <= k && lane < count ? static_cast<uint32_t>(s.sel[lane & 15]) : 0u;  // lane j: the j-th largest key of the row
     const int idc = 511 - static_cast<int>(mine & 0x1ffu);
-    const bool have = lane <= k && mine != 0u && idc < n;
-    float l = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float from = __shfl(lv[j], idc & 63, kWave);
-        l = (have && (idc >> 6) == j) ? from : l;
-    }
+    const bool have = mine != 0u && idc < n;
+    const float l = have ? s.selp[lane & 15] : -INFINITY;
+    wave_lds_fence();
     const float e = (have && l > -INFINITY) ? exp_ggml(l - mx) : 0.0f;
     const float nxt = dpp_f<kDppShl1>(0.0f, e);  // k + 1 <= 16: these lanes are one row
     const uint32_t grid = mine >> 9, grid_nxt = static_cast<uint32_t>(dpp_i<kDppShl1>(0, static_cast<int>(grid)));
-    const bool good = lane > k || (have && l > -INFINITY &&
+    // (with every expert selected there is no (k+1)-th, and nothing left that could be above the last)
+    const bool good = lane > k || (lane == k && n == k) || (have && l > -INFINITY &&
                                    (lane == k || (grid > grid_nxt && e >= 0x1p-100f && e > nxt * (lane == k - 1 ? 1.000004f : 1.000001f))));
     st.mx = mx, st.e = e, st.id = idc;
-    st.fast = __builtin_amdgcn_ballot_w64(odd) == 0ull && mx < INFINITY && __builtin_amdgcn_ballot_w64(good) == ~0ull;
+    st.fast = count <= 64 && __builtin_amdgcn_ballot_w64(odd) == 0ull && mx < INFINITY && __builtin_amdgcn_ballot_w64(good) == ~0ull;
 }
 
 // Step B, first half (any wave that holds the logits; it need not be the wave of step A): every exponential into s.p,
 // the per-8 sums, and the row's 1/sum as the reference takes it (0 for a row whose exponentials all vanished: `dead`).
-WD_DEV float sel_wave_denominator(const float (&lv)[8], int n, const TopkLds<1> &s, int lane, bool &dead) {
+template <int M>
+WD_DEV float sel_wave_denominator(const float (&lv)[M], int n, const TopkLds<1> &s, int lane, bool &dead) {
     const int groups = n >> 3;
     float lm = lv[0];
 #pragma unroll
-    for (int j = 1; j < 8; ++j) lm = __builtin_fmaxf(lm, lv[j]);
+    for (int j = 1; j < M; ++j) lm = __builtin_fmaxf(lm, lv[j]);
     const float mx = wave_max(lm);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < M; ++j) {
         const int id = 64 * j + lane;
         const float e = (id < n) ? exp_ggml(lv[j] - mx) : 0.0f;
         const float gs = close_lanes8(e);
@@ -667,6 +652,62 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
     finish_weights(top_mine, ids_given ? id_given : id_mine, k, w_scale, ids, weights, nullptr, lane);
 }
 
+// The selection of a row of n <= 64 M logits, k <= 15, inside a dispatch that wrote the logits: wave 0 ranks and publishes
+// the ids, wave 1 takes the exponentials and the denominator meanwhile, and wave 0 forms the weights behind one barrier.
+// Every thread of the workgroup must call it.  ids, weights: LDS.
+template <int M>
+WD_DEV void topk_two_waves(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
+                           const int32_t *__restrict__ override_ids, uint8_t *lds, int lane, int wave, unsigned long long *stamps,
+                           uint32_t *tagged, int copies) {
+#define WD_STAMP(i) do { if (stamps && wave == 0 && lane == 0) stamps[i] = wall_clock64(); } while (0)
+    const TopkLds<1> s(lds);
+    WD_STAMP(0);
+    SelWaveState st;
+    int id_given = 0;
+    if (wave <= 1) {
+        if (override_ids && wave == 0 && lane < k) id_given = override_ids[lane];
+        float lv[M];
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+            lv[j] = (64 * j + lane < n) ? __hip_atomic_load(logits + 64 * j + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
+        if (wave == 0) {
+            sel_wave_ids(lv, n, k, s, lane, st);
+            WD_STAMP(3);
+            if (st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+            WD_STAMP(6);
+        } else {
+            bool dead;
+            const float inv = sel_wave_denominator(lv, n, s, lane, dead);
+            if (lane == 0) s.rest[0] = inv, s.rest[1] = dead ? 1.0f : 0.0f;
+        }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const bool fast = st.fast;
+        sel_wave_weights(n, k, w_scale, s, lane, st, s.rest[0], s.rest[1] != 0.0f, ids, weights, override_ids != nullptr, id_given);
+        if (!fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        WD_STAMP(7);
+    }
+#undef WD_STAMP
+}
+
+// Selection inside a dispatch by the workgroup that read the last logit's arrival; every thread must call it.  Two waves do
+// it where one can hold the row (n <= 512, k <= 15); ids and weights are left in LDS by wave 0.
+// (64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
+// there are experts to select its threshold excludes nobody -; 512 experts, top-10: 2.1, 2.2.)
+WD_DEV void topk_block(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
+                       const int32_t *__restrict__ override_ids, uint8_t *lds, int lane, int wave,
+                       unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
+    if (n <= 512 && k <= 15) {
+        if (n <= 64) topk_two_waves<1>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        else if (n <= 128) topk_two_waves<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        else if (n <= 256) topk_two_waves<4>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        else topk_two_waves<8>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+    } else {
+        topk_block_m<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+    }
+}
+
 // Stand-alone softmax/top-k dispatch: one wave (src/qwen38_moe.cuh:711-818).
 // If gate_logit != null, gate_logit[0] is replaced by sigmoid_ggml(gate_logit[0]) (shared expert gate).
 // If override_ids != null the selected ids are replaced by override_ids[0..k) after the weights are formed.
@@ -683,7 +724,7 @@ __global__ __launch_bounds__(64) void k_topk_softmax(const float *__restrict__ l
 #pragma unroll
         for (int j = 0; j < 8; ++j) lv[j] = (64 * j + lane < n) ? logits[64 * j + lane] : -INFINITY;
         SelWaveState st;
-        sel_wave_ids(lv, n, k, lane, st);
+        sel_wave_ids(lv, n, k, s, lane, st);
         int id_given = 0;
         if (override_ids && lane < k) id_given = override_ids[lane];
         bool dead;
@@ -691,61 +732,23 @@ __global__ __launch_bounds__(64) void k_topk_softmax(const float *__restrict__ l
         sel_wave_weights(n, k, w_scale, s, lane, st, inv, dead, ids, weights, override_ids != nullptr, id_given);
         return;
     }
-    topk_wave<false>(logits, n, k, w_scale, ids, weights, override_ids, lane);
+    topk_wave(logits, n, k, w_scale, ids, weights, override_ids, lane);
 }
 
-// ---- router rows: 32 lanes per row, 8 rows per 256-thread workgroup ---------------------------------
-// All loads of a 2048-column span are issued before the first multiply-add, so one HBM round trip
-// covers the span; the multiply-add chain of each accumulator still runs in ascending column order.
-// COHERENT: results are published with device-scope atomic stores (another workgroup of the same
-// dispatch reads them).
-template <bool COHERENT>
-WD_DEV void router_rows(const float *__restrict__ w, const float *__restrict__ x, float *logits, int rows, int cols,
-                        const float *__restrict__ extra_w, float *extra_out, int wg) {
-    const int t = threadIdx.x & 31;
-    const int row = wg * static_cast<int>(blockDim.x >> 5) + (threadIdx.x >> 5);
-    const int total = rows + (extra_w ? 1 : 0);
-    const bool on = row < total;
-    const float *wr = on ? (row < rows ? w + static_cast<size_t>(row) * cols : extra_w) : x;
-    const int np = cols & ~31;
-    float s = 0.0f;
-    if (on) {
-        for (int i0 = 0; i0 < np; i0 += 2048) {
-            float wv[64], xv[64];
-#pragma unroll
-            for (int u = 0; u < 64; ++u) {
-                const int i = i0 + 32 * u + t;
-                if (i0 + 32 * u < np) {
-                    wv[u] = wr[i];
-                    xv[u] = x[i];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 64; ++u)
-                if (i0 + 32 * u < np) s = __builtin_fmaf(wv[u], xv[u], s);
-        }
-    }
-    float o = __shfl_down(s, 16, 32);
-    if (t < 16) s = s + o;
-    o = __shfl_down(s, 8, 32);
-    if (t < 8) s = s + o;
-    o = __shfl_down(s, 4, 32);
-    if (t < 4) s = s + o;
-    o = __shfl_down(s, 1, 32);
-    if (t == 0 || t == 2) s = s + o;
-    o = __shfl_down(s, 2, 32);
-    float acc = s + o;
-    if (on && t == 0) {
-        for (int c = np; c < cols; ++c) acc = acc + wr[c] * x[c];
-        float *dst = (row < rows) ? logits + row : extra_out;
-        if (COHERENT)
-            __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else
-            *dst = acc;
-    }
+// ---- router rows -------------------------------------------------------------------------------------------
+// ggml's closing tree over the 32 accumulators of a row, held one per lane by lanes 0..31 or 32..63: the upper sixteen
+// onto the lower, then 8, 4, 1 and 2 further on (the order of src/qwen38_moe.cuh:198-245).  Lane moves inside the vector
+// unit instead of five trips through the LDS crossbar.  Valid in lanes 0 and 32.
+WD_DEV float router_close32(float s) {
+    const wd_uint2v w = __builtin_amdgcn_permlane16_swap(f_bits(s), f_bits(s), false, false);
+    s = bits_f(w.x) + bits_f(w.y);
+    s = s + dpp_f<0x108>(0.0f, s);  // row_shl:8
+    s = s + dpp_f<kDppShl4>(0.0f, s);
+    s = s + dpp_f<kDppShl1>(0.0f, s);
+    return s + dpp_f<kDppShl2>(0.0f, s);
 }
 
-// Router rows for the merged dispatch: one row per wave, x staged once per workgroup in LDS (f32 [cols]).
+// One row per wave, x staged once per workgroup in LDS (f32 [cols]).
 // Accumulator t (of ggml's 4 x 8) of the row lives in lanes t and t + 32: for every span of 2048 columns lane t
 // runs the multiply-adds of columns [span, span + 1024) and hands the value to lane t + 32, which continues with
 // [span + 1024, span + 2048) and hands it back for the next span, so each chain still sees its columns in
@@ -753,7 +756,7 @@ WD_DEV void router_rows(const float *__restrict__ w, const float *__restrict__ x
 // which lets three workgroups of the merged dispatch share a compute unit).
 // Every thread of the workgroup must call it (it contains a barrier).
 // SCALAR_ROW: keep the wave's row pointer in scalar registers (two vector registers fewer).
-template <bool COHERENT, bool SCALAR_ROW = false>
+template <bool SCALAR_ROW = false>
 WD_DEV void router_rows_wave(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *logits, int rows,
                              int cols, const float *__restrict__ extra_w, float *extra_out, int wg) {
     const int lane = threadIdx.x & 63, t = lane & 31;
@@ -825,23 +828,11 @@ WD_DEV void router_rows_wave(const float *__restrict__ w, const float *__restric
         }
     }
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
-    float o = __shfl_down(s, 16, 32);
-    if (t < 16) s = s + o;
-    o = __shfl_down(s, 8, 32);
-    if (t < 8) s = s + o;
-    o = __shfl_down(s, 4, 32);
-    if (t < 4) s = s + o;
-    o = __shfl_down(s, 1, 32);
-    if (t == 0 || t == 2) s = s + o;
-    o = __shfl_down(s, 2, 32);
-    float acc = s + o;
+    float acc = router_close32(s);
     if (on && lane == 32) {
         for (int c = np; c < cols; ++c) acc = acc + wr[c] * xs[c];
         float *dst = (row < rows) ? logits + row : extra_out;
-        if (COHERENT)
-            __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else
-            *dst = acc;
+        __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (another workgroup of the dispatch reads it)
     }
 }
 
@@ -912,16 +903,7 @@ WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__re
     }
     if (!second) return;
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
-    float o = __shfl_down(s, 16, 32);
-    if (t < 16) s = s + o;
-    o = __shfl_down(s, 8, 32);
-    if (t < 8) s = s + o;
-    o = __shfl_down(s, 4, 32);
-    if (t < 4) s = s + o;
-    o = __shfl_down(s, 1, 32);
-    if (t == 0 || t == 2) s = s + o;
-    o = __shfl_down(s, 2, 32);
-    float acc = s + o;
+    float acc = router_close32(s);
     if (on && lane == 32) {
         for (int c = np; c < cols; ++c) acc = acc + wr[c] * xs[c];
         float *dst = (row < rows) ? logits + row : extra_out;
@@ -929,86 +911,53 @@ WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__re
     }
 }
 
-// ---- dispatch A -----------------------------------------------------------------------------------------
-// grid = n_router_wgs + ceil(F / 8) (the second part only with a shared expert); 512 threads.
-// Router workgroups: 16 rows each.  Shared-expert workgroups: 8 (gate, up) row pairs, one per wave.
-// dynamic LDS: H bytes + H/32 halves for the Q8_0 copy of x.
+// ---- dispatch AB ------------------------------------------------------------------------------------------
+// Workgroups [0, n_router_wgs): router rows, the last one to finish selects the experts and publishes the ids;
+// then n_shared_wgs workgroups for the shared expert's gate/up; the rest for the routed gate/up, one (expert rung,
+// group of eight rows) item each: a (gate, up) row pair per wave.  The routed workgroups are dispatched after the router
+// ones (lower block index first), quantise x and stage the codebooks while the router runs, then poll the published ids;
+// as soon as these appear they request their weights.  This removes a launch, a round trip for the ids and the serial
+// activation set-up from the critical path of the layer.  Where the ids are known before the launch (ids_known: a routing
+// trace, or a selection that is in the scratch) nothing is waited for and the weights are requested ahead of the set-up.
 //
 // Hand-off to the selecting workgroup: logits are published with device-scope atomic stores, each
 // workgroup then waits for its stores to complete and bumps a counter with a relaxed device-scope
 // atomic; the workgroup that reads n_router_wgs - 1 knows every logit is complete and reads them
 // with device-scope atomic loads.  No cache-wide release/acquire is needed for 2 KB of data.
-__global__ __launch_bounds__(512) void k_layer_a(LayerArgs a) {
-    extern __shared__ __align__(16) uint8_t lds_a[];
-    __shared__ Q8RowTile tiles[8];
-    __shared__ int s_last;
-    const int wg = blockIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (a.dry) return;
-    mark(a, 0, 0);
-    if (wg < a.n_router_wgs) {
-        router_rows<true>(a.router, a.x, a.logits, a.preselected ? 0 : a.E, a.H, a.sh_inp, a.shared_gate, wg);
-        mark(a, 0, 1);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
-        __syncthreads();
-        if (threadIdx.x == 0)
-            s_last = (__hip_atomic_fetch_add(a.arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                      static_cast<unsigned>(a.n_router_wgs - 1));
-        __syncthreads();
-        if (s_last && wave == 0) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            if (a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 0] = wall_clock64();
-            if (!a.preselected) topk_wave<true>(a.logits, a.E, a.k, a.w_scale, a.ids, a.weights, a.ids_override, lane);
-            if (lane == 0) {
-                if (a.sh_inp) {
-                    const float g = __hip_atomic_load(a.shared_gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    a.shared_gate[0] = sigmoid_ggml(g);
-                }
-                a.arrive[0] = 0u;
-            }
-            if (a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
-        }
-        mark(a, 0, 2);
-        return;
-    }
-    int8_t *xq = reinterpret_cast<int8_t *>(lds_a);
-    uint16_t *xd = reinterpret_cast<uint16_t *>(lds_a + a.H);
-    const int r = (wg - a.n_router_wgs) * 8 + wave;
-    const int nb = a.H >> 5;
-    const size_t rb = static_cast<size_t>(nb) * 34;
-    const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
-    const uint8_t *const rows[2] = {a.sh_gate + off, a.sh_up + off};
-    float gu[2];
-    q8_row_wave<2>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
-        lds_quantize_q8_0(a.x, a.H, xq, xd, threadIdx.x, 512);
-        __syncthreads();
-        mark(a, 0, 2);
-    });
-    if (lane == 0 && r < a.F) a.act[static_cast<size_t>(a.k) * a.F + r] = silu_ggml(gu[0]) * gu[1];
-    mark(a, 0, 3);
-}
-
-// ---- dispatches A and B in one launch ---------------------------------------------------------------------
-// Workgroups [0, n_router_wgs): router rows, the last one to finish selects the experts and publishes the ids;
-// then ceil(F / 8) workgroups for the shared expert's gate/up; then k * ceil(F / 8) workgroups for the routed
-// gate/up.  The routed workgroups are dispatched after the router ones (lower block index first), quantise x and
-// stage the codebooks while the router runs, then poll the published ids; as soon as these appear they request
-// their weights.  This removes a launch, a round trip for the ids and the serial activation set-up from the
-// critical path of the layer.
 //
 // Publication: id j goes, as one 32-bit word, to ids_tagged[c][j] of every replica c with a device-scope atomic
 // store; a word other than kTagInvalid is the id itself, so a reader needs no second flag.  The words are reset
 // to kTagInvalid by dispatch C (or by the caller) before the next layer pass uses them.  The wait is bounded:
 // when it runs out the workgroup sets status[0] and returns.
-// COAL (IQ types): rows of eight super-blocks on 16-byte boundaries are fetched with one aligned 16-byte load per
-// lane and parked in LDS (iq_rows8_coal); dynamic LDS then has 8 * 2 * kIqStageBytes more bytes behind the 4 * H + 16.
-// NB (COAL only): super-blocks per row, 8 (hidden 2048) or 10 (hidden 2560).
-// LOOP: the grid has fewer routed workgroups than there are (expert rung, group of eight rows) items; they walk them
-// with the stride of their number.
-template <int TYPE, bool COAL, int NB = 8, bool LOOP = false, bool PART = false, bool TRACE = false>
-__global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
-    constexpr bool kIq = (TYPE == 21 || TYPE == 22);
+//
+// TYPE: gate/up tensor type (21 IQ3_S, 22 IQ2_S, 8 Q8_0, 20 IQ4_NL).
+// FETCH: how rows come in, and with it how the router's rows are taken:
+//   8   IQ rows of eight super-blocks on 16-byte boundaries (hidden 2048): one aligned 16-byte load per lane (iq_rows8_coal)
+//   10  IQ rows of ten (hidden 2560): iq_rows10_coal
+//   1   other hidden up to 2048: IQ rows as the 16-byte words that cover them, one load per lane (iq_rows_cover)
+//   2   hidden 2049..4096: the same with two loads per lane
+//   0   anything else (hidden beyond 4096, IQ tensors that do not start on 16-byte boundaries): fields loaded one by one
+//   Router rows of 2049..4096 columns take two waves each (10 and 2: at hidden 4096 a row by one wave, two dependent trips
+//   to memory, took 8.7 us of the dispatch, by two 3.3), others one.
+// dynamic LDS: the larger of 4 * H + 16 bytes (x of the router rows) and the quantised x (H bytes + scales, layer_ab_stage)
+// with the per-wave staging area of the IQ rows behind it (layer_ab_stage_bytes).
+// LOOP: the grid has fewer routed workgroups than there are items; they walk them with the stride of their number.
+__host__ __device__ inline uint32_t layer_ab_stage(int H) { return static_cast<uint32_t>(H + H / 16 + 15) & ~15u; }
+template <int TYPE, int FETCH>
+constexpr bool kAbIq = (TYPE == 21 || TYPE == 22);
+template <int TYPE, int FETCH>
+__host__ __device__ inline uint32_t layer_ab_stage_bytes(int H) {  // per wave
+    if (!kAbIq<TYPE, FETCH> || FETCH == 0) return 0;
+    if (FETCH == 8) return 2 * kIqStageBytes;
+    if (FETCH == 10) return 2 * kIqStage10Bytes;
+    return 2 * iq_cover_bytes<TYPE>(H >> 8);
+}
+
+template <int TYPE, int FETCH, bool LOOP = false, bool PART = false, bool TRACE = false>
+__global__ __launch_bounds__(512, FETCH == 0 ? 4 : 6) void k_layer_ab(LayerArgs a) {
+    constexpr bool kIq = kAbIq<TYPE, FETCH>, kWide = FETCH == 10 || FETCH == 2;
+    constexpr bool kTwoPasses = kWide;  // Q8_0 rows of 65..128 blocks
+    constexpr int kIqType = kIq ? TYPE : 21;
     extern __shared__ __align__(16) uint8_t lds_ab[];
     __shared__ __align__(16) uint8_t s_union[sizeof(Q8RowTile) * 8 > sizeof(IqTables) ? sizeof(Q8RowTile) * 8 : sizeof(IqTables)];
     __shared__ int s_last;
@@ -1016,15 +965,15 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (a.dry) return;
     const int groups = (a.F + 7) / 8;
-    const int n_shared_wgs = a.sh_inp ? groups : 0;
 
-    mark<TRACE>(a, wg < a.n_router_wgs + n_shared_wgs ? 0 : 1, 0);
+    mark<TRACE>(a, wg < a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);
     if (wg < a.n_router_wgs) {
-        if (COAL && NB == 10)  // rows of 2560 columns: two waves per row, four rows per workgroup (the host sizes the grid for it)
-            router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.logits, a.E,
+        const int rows = a.preselected ? 0 : a.E;
+        if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
+            router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.logits, rows,
                                   a.H, a.sh_inp, a.shared_gate, wg);
         else
-            router_rows_wave<true>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.logits, a.E, a.H, a.sh_inp,
+            router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.logits, rows, a.H, a.sh_inp,
                                    a.shared_gate, wg);
         mark<TRACE>(a, 0, 1);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -1037,28 +986,31 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
         if (s_last) {
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             if (TRACE && a.trace && threadIdx.x == 0) a.trace[(0 * 16 + 8) * 8 + 0] = wall_clock64();
-            // results land behind the selection's own scratch
-            static_assert(sizeof(s_union) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
-            int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
-            float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
-            // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
-            topk_block(a.logits, a.E, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
-                       (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_tagged, kTagCopies);
-            if (wave == 0) {
-                wave_lds_fence();
-                // the plain copies for dispatch C
-                if (lane < a.k) {
-                    a.ids[lane] = lds_ids[lane];
-                    a.weights[lane] = lds_w[lane];
-                }
-                if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
-            } else if (wave == 5 && lane == 0) {
+            if (wave == 5 && lane == 0) {
                 // off the selection's path: the shared expert's gate, and the counter for the next layer pass
                 if (a.sh_inp) {
                     const float g = __hip_atomic_load(a.shared_gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     a.shared_gate[0] = sigmoid_ggml(g);
                 }
                 a.arrive[0] = 0u;
+            }
+            if (!a.preselected) {
+                // results land behind the selection's own scratch
+                static_assert(sizeof(s_union) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
+                int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
+                float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
+                // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
+                topk_block(a.logits, a.E, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
+                           (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
+                if (wave == 0) {
+                    wave_lds_fence();
+                    // the plain copies for dispatch C
+                    if (lane < a.k) {
+                        a.ids[lane] = lds_ids[lane];
+                        a.weights[lane] = lds_w[lane];
+                    }
+                    if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
+                }
             }
         }
         mark<TRACE>(a, 0, 2);
@@ -1067,7 +1019,7 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
 
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ab);
     uint8_t *xscale = lds_ab + a.H;  // Q8_K: f32 [H/256]; Q8_0: f16 [H/32]
-    if (wg < a.n_router_wgs + n_shared_wgs) {
+    if (wg < a.n_router_wgs + a.n_shared_wgs) {
         Q8RowTile *tiles = reinterpret_cast<Q8RowTile *>(s_union);
         const int r = (wg - a.n_router_wgs) * 8 + wave;
         const int nb = a.H >> 5;
@@ -1075,7 +1027,7 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
         const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
         const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
         float gu[2];
-        q8_row_wave<2>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, [&]() {
+        q8_row_wave<0, 2, kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, [&]() {
             lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
             __syncthreads();
         });
@@ -1083,42 +1035,65 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
         return;
     }
 
-    // routed gate/up: set-up that does not need the ids
-    const int bw = wg - a.n_router_wgs - n_shared_wgs;
+    // routed gate/up
+    const int bw = wg - a.n_router_wgs - a.n_shared_wgs;
     IqTables &tables = *reinterpret_cast<IqTables *>(s_union);
-    if (kIq) {
-        stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, 512);
-        for (int b = wave; b < (a.H >> 8); b += 8)
-            wave_quantize_q8_k_block(a.x + b * 256, xq + b * 256, reinterpret_cast<float *>(xscale) + b, lane);
-    } else {
-        lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
-    }
-    mark<TRACE>(a, 1, 1);
+    auto set_up = [&]() {  // what does not need the ids
+        if (kIq) {
+            stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, 512);
+            for (int b = wave; b < (a.H >> 8); b += 8)
+                wave_quantize_q8_k_block(a.x + b * 256, xq + b * 256, reinterpret_cast<float *>(xscale) + b, lane);
+        } else {
+            lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
+        }
+        mark<TRACE>(a, 1, 1);
+    };
     __shared__ int s_expert;
-    const int n_routed_wgs = LOOP ? static_cast<int>(gridDim.x) - a.n_router_wgs - n_shared_wgs : 0;
+    const int n_routed_wgs = LOOP ? static_cast<int>(gridDim.x) - a.n_router_wgs - a.n_shared_wgs : 0;
+    // With known ids the set-up is done behind the requests of the first item (the variants named here have no registers
+    // to hold these meanwhile).
+    constexpr bool kBehind = FETCH != 0 && !(TYPE == 8 && LOOP);
+    bool pending = true;
+    if (!kBehind || !a.ids_known) {
+        set_up();
+        pending = false;
+    }
     int item = bw;
     do {  // one item per workgroup unless the grid was capped (LOOP)
         const int j = item / groups;
         const int rg = item - j * groups;
-        if (threadIdx.x == 0) {
-            const uint32_t *src = a.ids_tagged + (bw & (kTagCopies - 1)) * 16 + j;
-            uint32_t e = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            unsigned polls = 0;
-            while (e == kTagInvalid && ++polls < a.spin_limit) {
-                __builtin_amdgcn_s_sleep(4);
-                e = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        int e;
+        if (a.ids_known) {
+            e = sld_i32(a.ids_known + j);
+            if (!kBehind) __syncthreads();
+        } else {
+            if (threadIdx.x == 0) {
+                const uint32_t *src = a.ids_tagged + (bw & (kTagCopies - 1)) * 16 + j;
+                uint32_t id = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                unsigned polls = 0;
+                while (id == kTagInvalid && ++polls < a.spin_limit) {
+                    __builtin_amdgcn_s_sleep(4);
+                    id = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (id == kTagInvalid) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_expert = static_cast<int>(id);
             }
-            if (e == kTagInvalid) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            s_expert = static_cast<int>(e);
+            __syncthreads();
+            e = s_expert;
+            if (e < 0 || e >= a.E) return;  // the wait ran out (status is set): leave without touching memory
         }
-        __syncthreads();
         mark<TRACE>(a, 1, 2);
-        const int e = s_expert;
-        if (e < 0 || e >= a.E) return;  // the wait ran out (status is set): leave without touching memory
         const uint8_t *gate = mat_ptr_expert<0>(a.gate_up, e);
         const uint8_t *up = mat_ptr_expert<1>(a.gate_up, e);
         float *act = a.act + static_cast<size_t>(j) * a.F;
         const int r = rg * 8 + wave;
+        auto pre = [&]() {
+            if (kBehind && pending) {
+                set_up();
+                __syncthreads();
+                pending = false;
+            }
+        };
         float gu[2];
         if (kIq) {
             const int nb = a.H >> 8;
@@ -1128,22 +1103,23 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
             // (PART) the chunk sums of the pair: gate row r of rung j, the up row F rows further on
             const size_t pg = static_cast<size_t>(nb) * 8;
             int32_t *pp = PART ? a.gup_part + (static_cast<size_t>(j) * 2 * a.F + min(r, a.F - 1)) * pg : nullptr;
-            if (COAL && NB == 10)
-                iq_rows10_coal<(kIq ? TYPE : 21), 2, PART>(rows, tables, xq, reinterpret_cast<const float *>(xscale), lane, gu,
-                                                           lds_ab + ((4 * a.H + 16 + 15) & ~15) + wave * 2 * kIqStage10Bytes, pp, a.F * pg);
-            else if (COAL)
-                iq_rows8_coal<(kIq ? TYPE : 21), 2, PART>(rows, tables, xq, reinterpret_cast<const float *>(xscale), lane, gu,
-                                                          lds_ab + ((4 * a.H + 16 + 15) & ~15) + wave * 2 * kIqStageBytes, pp, a.F * pg);
+            uint8_t *const stage = lds_ab + layer_ab_stage(a.H) + wave * layer_ab_stage_bytes<TYPE, FETCH>(a.H);
+            const float *xd = reinterpret_cast<const float *>(xscale);
+            if (FETCH == 10)
+                iq_rows10_coal<kIqType, 2, PART>(rows, tables, xq, xd, lane, gu, stage, pp, a.F * pg, pre);
+            else if (FETCH == 8)
+                iq_rows8_coal<kIqType, 2, PART>(rows, tables, xq, xd, lane, gu, stage, pp, a.F * pg, pre);
+            else if (FETCH != 0)
+                iq_rows_cover<kIqType, 2, FETCH == 0 ? 1 : (FETCH > 2 ? 2 : FETCH), PART>(rows, nb, tables, xq, xd, lane, gu, stage, pp, a.F * pg, pre);
             else
-                iq_rows_q8k<(kIq ? TYPE : 21), 2, PART>(rows, nb, tables, xq, reinterpret_cast<const float *>(xscale), lane, gu, pp,
-                                                         a.F * pg);
+                iq_rows_q8k<kIqType, 2, PART>(rows, nb, tables, xq, xd, lane, gu, pp, a.F * pg, pre);
         } else {
             Q8RowTile *tiles = reinterpret_cast<Q8RowTile *>(s_union);
             const int nb = a.H >> 5;
-            const size_t rb = static_cast<size_t>(nb) * 34;
+            const size_t rb = static_cast<size_t>(nb) * (TYPE == 8 ? 34 : 18);
             const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
-            const uint8_t *const rows[2] = {gate + off, up + off};
-            q8_row_wave<2>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu);
+            const uint8_t *const rows[2] = {uniform_ptr(gate + off), uniform_ptr(up + off)};
+            q8_row_wave<(TYPE == 8 ? 0 : 1), 2, kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, pre);
         }
         if (lane == 0 && r < a.F) act[r] = silu_ggml(gu[0]) * gu[1];
         mark<TRACE>(a, 1, 3);
@@ -1154,119 +1130,94 @@ __global__ __launch_bounds__(512, 6) void k_layer_ab(LayerArgs a) {
     } while (LOOP && item < a.n_routed_items);
 }
 
-// ---- dispatch B -----------------------------------------------------------------------------------------
-// TYPE: gate/up tensor type (21 IQ3_S, 22 IQ2_S, 8 Q8_0, 20 IQ4_NL).
-// IQ types and Q8_0: 512-thread workgroups, one (gate,up) row pair per wave, grid = k * ceil(F / 8).
-// IQ4_NL: 256-thread workgroups, four row pairs per wave, grid = k * ceil(F / 16).
-// Every wave first requests its weight bytes; the workgroup then stages the codebooks and quantises x
-// while they are in flight.  dynamic LDS: quantised x (H bytes + scales).
-template <int TYPE, bool PART = false>
-__global__ __launch_bounds__(TYPE == 20 ? 256 : 512) void k_layer_b(LayerArgs a) {
-    constexpr bool kIq = (TYPE == 21 || TYPE == 22);
-    constexpr int kThreads = (TYPE == 20) ? 256 : 512;
-    constexpr int kRowsPerWg = (TYPE == 20) ? 16 : 8;
-    extern __shared__ __align__(16) uint8_t lds_b[];
-    __shared__ IqTables tables;
-    __shared__ Q8TileN<4> tiles4[TYPE == 20 ? 4 : 1];
-    __shared__ Q8RowTile tiles1[TYPE == 8 ? 8 : 1];
-    int8_t *xq = reinterpret_cast<int8_t *>(lds_b);
-    uint8_t *xscale = lds_b + a.H;  // f32 [H/256] or f16 [H/32]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (a.dry) return;
-    mark(a, 1, 0);
-
-    const int groups = (a.F + kRowsPerWg - 1) / kRowsPerWg;
-    const int j = blockIdx.x / groups;
-    const int rg = blockIdx.x - j * groups;
-    const int e = a.ids[j];
-    const uint8_t *gate = mat_ptr_expert<0>(a.gate_up, e);
-    const uint8_t *up = mat_ptr_expert<1>(a.gate_up, e);
-    float *act = a.act + static_cast<size_t>(j) * a.F;
-    if (kIq) {
-        const int nb = a.H >> 8;
-        const size_t rb = static_cast<size_t>(nb) * (TYPE == 21 ? 110 : 82);
-        const int r = rg * 8 + wave;
-        const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
-        const uint8_t *const rows[2] = {gate + off, up + off};
-        float gu[2];
-        const size_t pg = static_cast<size_t>(nb) * 8;
-        int32_t *pp = PART ? a.gup_part + (static_cast<size_t>(j) * 2 * a.F + min(r, a.F - 1)) * pg : nullptr;
-        iq_rows_q8k<(kIq ? TYPE : 21), 2, PART>(rows, nb, tables, xq, reinterpret_cast<const float *>(xscale), lane, gu,
-                                                 pp, a.F * pg, [&]() {
-            stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, kThreads);
-            for (int b = wave; b < (a.H >> 8); b += kThreads / 64)
-                wave_quantize_q8_k_block(a.x + b * 256, xq + b * 256, reinterpret_cast<float *>(xscale) + b, lane);
-            mark(a, 1, 1);
-            __syncthreads();
-            mark(a, 1, 2);
-        });
-        if (lane == 0 && r < a.F) act[r] = silu_ggml(gu[0]) * gu[1];
-        mark(a, 1, 3);
-    } else if (TYPE == 8) {
-        const int nb = a.H >> 5;
-        const size_t rb = static_cast<size_t>(nb) * 34;
-        const int r = rg * 8 + wave;
-        const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
-        const uint8_t *const rows[2] = {gate + off, up + off};
-        float gu[2];
-        q8_row_wave<2>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles1[TYPE == 8 ? wave : 0], lane, gu,
-                       [&]() {
-                           lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, kThreads);
-                           __syncthreads();
-                       });
-        if (lane == 0 && r < a.F) act[r] = silu_ggml(gu[0]) * gu[1];
-    } else {
-        const int nb = a.H >> 5;
-        const size_t rb = static_cast<size_t>(nb) * 18;
-        const int r0 = rg * 16 + wave * 4;
-        const int nrows = max(0, min(4, a.F - r0));
-        const size_t off = static_cast<size_t>(min(r0, a.F - 1)) * rb;
-        const uint8_t *const rows[2] = {gate + off, up + off};
-        float gu[2];
-        q8_rows4_multi<1, 2, 4, false>(rows, nrows, nb, xq, reinterpret_cast<const uint16_t *>(xscale),
-                                       tiles4[TYPE == 20 ? wave : 0], lane, gu, nullptr, 0, [&]() {
-                                           lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale),
-                                                             threadIdx.x, kThreads);
-                                           __syncthreads();
-                                       });
-        const int r4 = lane >> 4;
-        if ((lane & 15) == 0 && r4 < nrows) act[r0 + r4] = silu_ggml(gu[0]) * gu[1];
+// ---- the combine at the end of dispatch C ---------------------------------------------------------------------
+// The operands of one wave's four rows, requested when the dispatch begins: lane m keeps router weight m, lane 16 the shared
+// gate; the residual values that the rows' owner updates at its end (nothing else writes them meanwhile): lane 4c + r
+// holds stream c of row r0 + r.
+struct FoldOps {
+    float w = 0.0f, res = 0.0f, inject = 0.0f;
+    unsigned bad = 0u;  // a bounded wait of this layer pass ran out: the results below are replaced by NaN
+};
+WD_DEV FoldOps layer_c_fold_request(const LayerArgs &a, int r0, int nrows, int lane) {
+    FoldOps o;
+    o.bad = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane < a.k) o.w = a.weights[lane];
+    if (lane == 16 && a.sh_inp) o.w = a.shared_gate[0];
+    if (a.residual) {
+        const int c = a.hc > 0 ? min(lane >> 2, a.hc - 1) : 0;
+        o.res = a.residual[static_cast<size_t>(c) * a.H + r0 + min(lane & 3, nrows - 1)];
+        if (a.hc > 0) o.inject = a.hc_inject[c];
     }
-    __syncthreads();
+    return o;
+}
+// Rows r0 .. r0 + nrows - 1 (at most four): matrix m's result for row r0 + q at ybuf[m * stride + q].  One wave.
+WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *ybuf, int stride, int r0, int nrows, int lane) {
+    const bool shared = a.sh_inp != nullptr;
+    // every lane folds row r0 + (lane & 3); lanes 0..3 store it
+    const int row = r0 + lane;
+    const bool on = lane < nrows;
+    float acc = 0.0f;
+    for (int m = 0; m < a.k; ++m) {
+        const float wm = lane_get(ops.w, m);
+        const float y = ybuf[m * stride + (lane & 3)];
+        const float prod = y * wm;
+        acc = acc + prod;
+        if (a.expert_out && on) a.expert_out[static_cast<size_t>(m) * a.H + row] = y;
+    }
+    const float gate = lane_get(ops.w, 16);
+    float o = acc;
+    if (shared) {
+        const float y = ybuf[a.k * stride + (lane & 3)];
+        const float prod = y * gate;
+        o = acc + prod;
+        if (on) a.down_f32[row] = y;
+    }
+    // an expert without a slot was reported by the waves above (or by the dispatch before)
+    unsigned bad = ops.bad;
+    if (a.down.slot_of_expert) bad |= __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (bad) acc = o = __builtin_nanf("");  // the caller sees the failure in its data, without a synchronisation
+    if (on) {
+        a.accum[row] = acc;
+        a.out[row] = o;
+    }
+    if (a.residual) {
+        if (a.hc > 0) {
+            const int c = lane >> 2;
+            if (c < a.hc && (lane & 3) < nrows) {
+                const float weighted = o * hc_weight(ops.inject, a.hc);
+                const float v = ops.res + weighted;
+                a.residual[static_cast<size_t>(c) * a.H + r0 + (lane & 3)] = a.hc_round_half ? round_half(v) : v;
+            }
+        } else if (on) {
+            const float scaled = o * a.residual_scale;
+            a.residual[row] = ops.res + scaled;
+        }
+    }
 }
 
 // ---- dispatch C -----------------------------------------------------------------------------------------
-// KIND: down tensor kind (0 Q8_0, 1 IQ4_NL).  One workgroup per four output rows; wave m takes
-// matrix m (the k routed down tensors, then the shared one), so every weight byte of the four rows
-// is requested at once.  Each wave re-quantises the activation of its own matrix while its weights
-// are in flight.  The first four lanes of wave 0 then fold the k+1 results in the reference order.
-// grid = ceil(H / 4), block = 64 * min(k + 1, 16).
-// dynamic LDS per wave: F bytes + F/32 halves (+ pad), then [k+1][4] floats.
-// COAL: the rows are 16 blocks long, H is a multiple of 4 and every down tensor starts on a 16-byte boundary: the
-// four rows of a wave are fetched as aligned 16-byte words (q8_rows4_coal).
-// NB (COAL only): blocks per row, 16 or 20.  TWO (COAL only): the workgroup has half as many waves as matrices; a wave
-// requests the rows and the activations of its two matrices together and parks all of it in LDS before the dot
-// products, which keeps it within 80 registers: the waves of a workgroup go to the four SIMDs in turn, so three
-// workgroups of six waves need six wave slots on two of them.  dynamic LDS per wave: two quantised activations and a
-// staging area of 4 * NB * 34 bytes.
-template <int KIND, bool COAL, int NB = 16, bool TWO = false, bool PART = false, bool TRACE = false>
-__global__ __launch_bounds__(TWO ? 576 : 1024) __attribute__((amdgpu_waves_per_eu(TWO ? 6 : 4)))
-void k_layer_c(LayerArgs a) {
+// All down projections of a few output rows per workgroup, a wave per matrix (the k routed down tensors, then the shared
+// one); each wave re-quantises the activation of its own matrix while its weights are in flight, and the first waves then
+// fold the results in the reference order (layer_c_fold).
+// KIND: down tensor kind (0 Q8_0, 1 IQ4_NL); the shared expert's is always Q8_0.
+//
+// k_layer_c: four rows, pass by pass: rows of any length, any number of matrices (waves take the matrices in turn).
+// grid = ceil(H / 4), block = 64 * min(n_act, 16) with n_act = k + 1 matrices (k without the shared expert).
+// dynamic LDS per wave: F bytes + F/32 halves (+ pad), then [n_act][4] floats.
+template <int KIND, bool PART = false, bool TRACE = false>
+__global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
     extern __shared__ __align__(16) uint8_t lds_c[];
-    using Tile = typename std::conditional<COAL, Q8TileNB<NB>, Q8Tile>::type;
-    __shared__ Tile tiles[TWO ? 9 : 16];
-    const bool shared = a.sh_inp != nullptr;
-    const int n_act = a.k + (shared ? 1 : 0);
+    __shared__ Q8Tile tiles[16];
+    const int n_act = a.k + (a.sh_inp ? 1 : 0);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nwaves = blockDim.x >> 6;
     const size_t per_wave = (static_cast<size_t>(a.F) + a.F / 16 + 15) & ~static_cast<size_t>(15);
     int8_t *aq = reinterpret_cast<int8_t *>(lds_c + wave * per_wave);
     uint16_t *ad = reinterpret_cast<uint16_t *>(lds_c + wave * per_wave + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_c + nwaves * per_wave);  // [n_act][4] (behind larger per-wave areas if TWO)
+    float *ybuf = reinterpret_cast<float *>(lds_c + nwaves * per_wave);  // [n_act][4]
     const int r0 = blockIdx.x * 4;
     const int nrows = min(4, a.H - r0);
     const int nb = a.F >> 5;
-    const int r4 = lane >> 4;
     if (a.dry) return;
     // every routed workgroup of this layer pass finished with the previous dispatch: make the ids published
     // for them invalid again (this dispatch reads the plain copy)
@@ -1274,188 +1225,118 @@ void k_layer_c(LayerArgs a) {
         for (int i = threadIdx.x; i < kTagCopies * 16; i += blockDim.x)
             __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     mark<TRACE>(a, 2, 0);
-    // combine operands, requested early: lane m keeps router weight m, lane 16 the shared gate
-    float wreg = 0.0f, res_pre = 0.0f, inject = 0.0f;
-    unsigned bad = 0u;  // a bounded wait of this layer pass ran out: the results below are replaced by NaN
-    if (wave == 0) {
-        bad = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (lane < a.k) wreg = a.weights[lane];
-        if (lane == 16 && shared) wreg = a.shared_gate[0];
-        // the residual values this workgroup updates at its end (nothing else writes them meanwhile): lane 4c + r
-        // holds stream c of row r0 + r
-        if (a.residual) {
-            const int c = a.hc > 0 ? min(lane >> 2, a.hc - 1) : 0;
-            res_pre = a.residual[static_cast<size_t>(c) * a.H + r0 + min(lane & 3, nrows - 1)];
-            if (a.hc > 0) inject = a.hc_inject[c];
-        }
-    }
-    // COAL: the activation of one matrix in registers, values 8 lane .. 8 lane + 8 and, with 20 blocks, 512 .. 639 in
-    // lanes 0..15 (the others repeat them); its Q8_0 form into LDS
-    constexpr int kActRegs = (COAL && NB == 20) ? 4 : 2;
-    auto request_act = [&](int m, float4 (&v)[kActRegs]) {
-        const float *act = a.act + static_cast<size_t>(m) * (NB * 32);
-        v[0] = *reinterpret_cast<const float4 *>(act + lane * 8);
-        v[1] = *reinterpret_cast<const float4 *>(act + lane * 8 + 4);
-        if constexpr (kActRegs == 4) {
-            v[2] = *reinterpret_cast<const float4 *>(act + 512 + (lane & 15) * 8);
-            v[3] = *reinterpret_cast<const float4 *>(act + 512 + (lane & 15) * 8 + 4);
-        }
-    };
-    auto quantise_act = [&](const float4 (&v)[kActRegs], int8_t *qs, uint16_t *d) {
-        lds_quantize_q8_0_step(v[0], v[1], true, lane * 8, qs, d, lane);
-        if constexpr (kActRegs == 4) lds_quantize_q8_0_step(v[2], v[3], lane < 16, 512 + (lane & 15) * 8, qs, d, lane);
-    };
-    if constexpr (COAL && TWO) {
-        // Everything is requested at once; both activations are quantised and both row groups parked in LDS as they
-        // arrive (loads return in order), so that no fetched word stays in a register while the dot products run.
-        using RawQ8 = Q8CoalRaw<0, NB>;
-        using RawW = Q8CoalRaw<KIND, NB>;
-        constexpr size_t kStage = 4 * NB * 34;  // the larger of the two kinds
-        const int uw = __builtin_amdgcn_readfirstlane(wave);
-        uint8_t *const wbase = lds_c + wave * (2 * per_wave + kStage);
-        int8_t *const aq2[2] = {reinterpret_cast<int8_t *>(wbase), reinterpret_cast<int8_t *>(wbase + per_wave)};
-        uint16_t *const ad2[2] = {reinterpret_cast<uint16_t *>(wbase + a.F), reinterpret_cast<uint16_t *>(wbase + per_wave + a.F)};
-        uint8_t *const stage2[2] = {reinterpret_cast<uint8_t *>(&tiles[wave]), wbase + 2 * per_wave};
-        ybuf = reinterpret_cast<float *>(lds_c + nwaves * (2 * per_wave + kStage));
-        const bool second = uw + nwaves < n_act;  // wave-uniform; a wave without a second matrix repeats its first (not used)
-        RawQ8 raw[2];  // (the request of either kind: as many loads as Q8_0 rows need)
-        float4 v[2][kActRegs];
-        int mm[2], words[2];
-        bool sh[2];
-        // the activations first: their addresses need no expert id, and loads return in order - the quantisation
-        // below then runs while the weights are still on their way
-        int e[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            mm[q] = (q == 0 || second) ? uw + q * nwaves : uw;
-            sh[q] = mm[q] == a.k;
-            e[q] = sld_i32(a.ids + min(mm[q], a.k - 1));  // both ids asked for together (not used for the shared expert)
-        }
-#pragma unroll
-        for (int q = 0; q < 2; ++q) request_act(mm[q], v[q]);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const uint8_t *w = sh[q] ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, e[q]);
-            const bool q8 = KIND == 0 || sh[q];  // wave-uniform
-            words[q] = q8 ? RawQ8::kWords : RawW::kWords;
-            raw[q] = q8_rows4_coal_request_any<NB>(w + static_cast<size_t>(r0) * NB * (q8 ? 34 : RawW::kBlk), words[q], lane);
-        }
-        mark<TRACE>(a, 2, 1);
-        wave_lds_fence();
-#pragma unroll
-        for (int q = 0; q < 2; ++q) quantise_act(v[q], aq2[q], ad2[q]);
-        mark<TRACE>(a, 2, 6);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) q8_rows4_coal_stage_any<NB>(raw[q], stage2[q], words[q], lane);
-        wave_lds_fence();
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            if (q == 1 && !second) break;
-            float y;
-            if (PART && !sh[q]) {  // (the shared expert's sums are not part of the dump)
-                int32_t *pp = a.down_part + (static_cast<size_t>(mm[q]) * a.H + r0) * (NB * 8);
-                y = q8_rows4_coal_dots<KIND, NB, PART>(stage2[q], aq2[q], ad2[q], tiles[wave], lane, pp);
-            } else {
-                y = (KIND == 0 || sh[q]) ? q8_rows4_coal_dots<0, NB>(stage2[q], aq2[q], ad2[q], tiles[wave], lane)
-                                         : q8_rows4_coal_dots<KIND, NB>(stage2[q], aq2[q], ad2[q], tiles[wave], lane);
-            }
-            if ((lane & 15) == 0) ybuf[mm[q] * 4 + r4] = y;
-            mark<TRACE>(a, 2, q == 0 ? 2 : 5);
-        }
-    } else
+    FoldOps ops;
+    if (wave == 0) ops = layer_c_fold_request(a, r0, nrows, lane);
     for (int m = wave; m < n_act; m += nwaves) {
         const bool is_shared = m == a.k;
-        if constexpr (COAL) {
-            // the activation first: its address needs no expert id, and loads return in order - it is quantised while
-            // the weights are still on their way
-            float4 v[kActRegs];
-            request_act(m, v);
-            const uint8_t *w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m));
-            float y;
-            if (KIND == 0 || is_shared) {
-                const auto raw = q8_rows4_coal_request<0, NB>(w + static_cast<size_t>(r0) * NB * 34, lane);
-                wave_lds_fence();
-                quantise_act(v, aq, ad);
-                mark<TRACE>(a, 2, 1);
-                if (PART && !is_shared)
-                    y = q8_rows4_coal_finish<0, NB, PART>(raw, aq, ad, tiles[wave], lane, a.down_part + (static_cast<size_t>(m) * a.H + r0) * (NB * 8));
-                else
-                    y = q8_rows4_coal_finish<0, NB>(raw, aq, ad, tiles[wave], lane);
-            } else {
-                const auto raw = q8_rows4_coal_request<1, NB>(w + static_cast<size_t>(r0) * NB * 18, lane);
-                wave_lds_fence();
-                quantise_act(v, aq, ad);
-                mark<TRACE>(a, 2, 1);
-                y = q8_rows4_coal_finish<1, NB, PART>(raw, aq, ad, tiles[wave], lane,
-                                                      PART ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (NB * 8) : nullptr);
-            }
-            if ((lane & 15) == 0) ybuf[m * 4 + r4] = y;
-        } else {
-            // m is the same for the whole wave: the id comes through the scalar path
-            const uint8_t *w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m));
-            const size_t rb = static_cast<size_t>(nb) * ((KIND == 0 || is_shared) ? 34 : 18);
-            const uint8_t *const rows[1] = {w + r0 * rb};
-            float y[1];
-            auto quantise = [&]() {
-                wave_lds_fence();
-                lds_quantize_q8_0(a.act + static_cast<size_t>(m) * a.F, a.F, aq, ad, lane, 64);
-                wave_lds_fence();
-                mark<TRACE>(a, 2, 1);
-            };
-            int32_t *pp = (PART && !is_shared) ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;
-            if (PART && !is_shared && KIND == 0)
-                q8_rows4_multi<0, 1, 1, PART>(rows, nrows, nb, aq, ad, tiles[wave], lane, y, pp, 0, quantise);
-            else if (KIND == 0 || is_shared)
-                q8_rows4_multi<0, 1, 1, false>(rows, nrows, nb, aq, ad, tiles[wave], lane, y, nullptr, 0, quantise);
-            else
-                q8_rows4_multi<1, 1, 1, PART>(rows, nrows, nb, aq, ad, tiles[wave], lane, y, pp, 0, quantise);
-            if ((lane & 15) == 0) ybuf[m * 4 + r4] = y[0];
-        }
+        // m is the same for the whole wave: the id comes through the scalar path
+        const uint8_t *const w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m));
+        const bool q8 = KIND == 0 || is_shared;  // the same in every lane
+        const uint8_t *const rows = w + static_cast<size_t>(r0) * nb * (q8 ? 34 : 18);
+        auto quantise = [&]() {
+            wave_lds_fence();
+            lds_quantize_q8_0(a.act + static_cast<size_t>(m) * a.F, a.F, aq, ad, lane, 64);
+            wave_lds_fence();
+            mark<TRACE>(a, 2, 1);
+        };
+        int32_t *pp = (PART && !is_shared) ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;
+        float y;
+        if (PART && !is_shared) y = q8_rows4<KIND, true>(rows, nrows, nb, aq, ad, tiles[wave], lane, pp, quantise);
+        else if (q8) y = q8_rows4<0, false>(rows, nrows, nb, aq, ad, tiles[wave], lane, nullptr, quantise);
+        else y = q8_rows4<KIND, false>(rows, nrows, nb, aq, ad, tiles[wave], lane, nullptr, quantise);
+        if ((lane & 15) == 0) ybuf[m * 4 + (lane >> 4)] = y;
         mark<TRACE>(a, 2, 2);
     }
     __syncthreads();
     mark<TRACE>(a, 2, 3);
-    if (wave == 0) {
-        // every lane folds row r0 + (lane & 3); lanes 0..3 store it
-        const int row = r0 + lane;
-        const bool on = lane < nrows;
-        float acc = 0.0f;
-        for (int m = 0; m < a.k; ++m) {
-            const float wm = lane_get(wreg, m);
-            const float y = ybuf[m * 4 + (lane & 3)];
-            const float prod = y * wm;
-            acc = acc + prod;
-            if (a.expert_out && on) a.expert_out[static_cast<size_t>(m) * a.H + row] = y;
-        }
-        const float gate = lane_get(wreg, 16);
-        float o = acc;
-        if (shared) {
-            const float y = ybuf[a.k * 4 + (lane & 3)];
-            const float prod = y * gate;
-            o = acc + prod;
-            if (on) a.down_f32[row] = y;
-        }
-        // an expert without a slot was reported by the waves above (or by the dispatch before)
-        if (a.down.slot_of_expert) bad |= __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (bad) acc = o = __builtin_nanf("");  // the caller sees the failure in its data, without a synchronisation
-        if (on) {
-            a.accum[row] = acc;
-            a.out[row] = o;
-        }
-        if (a.residual) {
-            if (a.hc > 0) {
-                const int c = lane >> 2;
-                if (c < a.hc && (lane & 3) < nrows) {
-                    const float weighted = o * hc_weight(inject, a.hc);
-                    const float v = res_pre + weighted;
-                    a.residual[static_cast<size_t>(c) * a.H + r0 + (lane & 3)] = a.hc_round_half ? round_half(v) : v;
-                }
-            } else if (on) {
-                const float scaled = o * a.residual_scale;
-                a.residual[row] = res_pre + scaled;
-            }
-        }
+    if (wave == 0) layer_c_fold(a, ops, ybuf, 4, r0, nrows, lane);
+    mark<TRACE>(a, 2, 4);
+}
+
+// k_layer_c8: eight rows per workgroup and wave: half the waves to launch, half the activations to quantise and, per 64
+// blocks, half the chain steps of the four-row form; all bytes of the eight rows are requested at once, behind the activation.
+// PASSES: of eight blocks per row (F <= 256 PASSES).  grid = H / 8, block = 64 max(n_act, 2) with at most 16 matrices; waves 0
+// and 1 fold four rows each.  (Hidden 4096, eight experts with rows of 48 Q8_0 blocks, 53.5 MB: 25.7 us in the four-row form
+// with two matrices per wave, 16.3 so, 15.4 with WORDS - the bytes alone take 9 -; hidden 2560, ten IQ4_NL experts of 20
+// blocks and the shared one: 12.4, 10.9; hidden 2048, ten Q8_0 experts of 16: 6.0, 5.5.)
+// WORDS: the rows come through LDS as aligned words (Q8Rows8Fetch), otherwise a lane loads its own blocks (Q8Rows8Blocks).
+// dynamic LDS: per wave the tile (WORDS: the staging area, which it lies in) and the quantised activation (F bytes + F/32
+// halves, padded), then [n_act][8] floats.
+template <bool WORDS>
+__host__ __device__ inline uint32_t layer_c8_wave_bytes(int F) {
+    static_assert(sizeof(Q8Tile8) <= kQ8Rows8StageBytes, "the tile lies in the staging area");
+    return (WORDS ? kQ8Rows8StageBytes : static_cast<uint32_t>(sizeof(Q8Tile8))) + (static_cast<uint32_t>(F + F / 16 + 15) & ~15u);
+}
+template <int KIND, int PASSES, bool WORDS, bool PART = false, bool TRACE = false>
+__global__ __launch_bounds__(1024) void k_layer_c8(LayerArgs a) {
+    constexpr int STEPS = (PASSES + 1) / 2;  // of sixteen blocks
+    extern __shared__ __align__(16) uint8_t lds_c8[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int n_act = a.k + (a.sh_inp ? 1 : 0);
+    const uint32_t per_wave = layer_c8_wave_bytes<WORDS>(a.F);
+    uint8_t *stage = lds_c8 + wave * per_wave;
+    Q8Tile8 &tile = *reinterpret_cast<Q8Tile8 *>(stage);
+    int8_t *aq = reinterpret_cast<int8_t *>(stage + (WORDS ? kQ8Rows8StageBytes : sizeof(Q8Tile8)));
+    uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
+    float *ybuf = reinterpret_cast<float *>(lds_c8 + max(n_act, 2) * per_wave);
+    const int r0 = blockIdx.x * 8, nb = a.F >> 5;
+    if (a.dry) return;
+    if (a.clear_tagged && blockIdx.x == 0)  // (as in k_layer_c)
+        for (int i = threadIdx.x; i < kTagCopies * 16; i += 64 * n_act)
+            __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mark<TRACE>(a, 2, 0);
+    const int m = min(wave, n_act - 1);  // (a second wave without a matrix of its own repeats the first's)
+    const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;
+    // the activation first: its address needs no expert id, and loads return in order - it is quantised while the weights are
+    // still on their way
+    float4 v[2 * STEPS];
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+        const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
+        v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
     }
+    const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m))) +
+                                            static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
+    FoldOps ops;
+    auto run = [&](auto kind, auto part) {
+        constexpr int K = decltype(kind)::value;
+        constexpr bool P = decltype(part)::value;
+        typename std::conditional<WORDS, Q8Rows8Fetch<K, STEPS>, Q8Rows8Blocks<K, PASSES>>::type fetch;
+        fetch.request(rows, nb, lane);
+        if (wave < 2) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i)
+            lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
+        mark<TRACE>(a, 2, 1);
+        Q8Chain ch;
+        int32_t *pp = P ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;
+#pragma unroll
+        for (int q = 0; q < STEPS; ++q) {
+            Q8Block w0, w1;
+            if constexpr (WORDS) {
+                wave_lds_fence();  // the step before has been read
+                fetch.park(q, stage, lane);
+                wave_lds_fence();
+                // (both blocks of the step before the first pass: its tile takes the parked words' place)
+                w0 = q8_rows8_block<K>(stage, nb, lane >> 3, lane & 7), w1 = q8_rows8_block<K>(stage, nb, lane >> 3, 8 + (lane & 7));
+            } else {
+                if (q == 0) wave_lds_fence();
+                w0 = fetch.w[2 * q], w1 = fetch.w[min(2 * q + 1, PASSES - 1)];
+            }
+            q8_rows8_pass<K, P>(w0, 16 * q, nb, aq, ad, tile, lane, ch, pp);
+            if (2 * q + 1 < PASSES && 16 * q + 8 < nb) q8_rows8_pass<K, P>(w1, 16 * q + 8, nb, aq, ad, tile, lane, ch, pp);
+        }
+        return q8_rows8_close<K>(ch, nb, tile, lane);
+    };
+    float y;
+    if (PART && !is_shared) y = run(std::integral_constant<int, KIND>{}, std::integral_constant<bool, PART>{});
+    else if (q8) y = run(std::integral_constant<int, 0>{}, std::false_type{});
+    else y = run(std::integral_constant<int, KIND>{}, std::false_type{});
+    if (wave < n_act && (lane & 7) == 0) ybuf[m * 8 + (lane >> 3)] = y;
+    mark<TRACE>(a, 2, 2);
+    __syncthreads();
+    mark<TRACE>(a, 2, 3);
+    if (wave < 2) layer_c_fold(a, ops, ybuf + 4 * wave, 8, r0 + 4 * wave, 4, lane);
     mark<TRACE>(a, 2, 4);
 }
 

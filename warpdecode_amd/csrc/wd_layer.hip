@@ -453,7 +453,6 @@ int layer_staged(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_s
 LayerArgs fused_args(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
                      const int32_t *ids_override, float *residual, float residual_scale, int rec = 0,
                      const HcSpec *hc = nullptr) {
-    const bool shared = L->shared_gate_inp != nullptr;
     LayerArgs a{};
     a.H = L->hidden, a.F = L->expert_ffn, a.E = L->n_experts, a.k = L->top_k;
     a.w_scale = L->expert_scale;
@@ -473,8 +472,7 @@ LayerArgs fused_args(const wd_moe_layer *L, const float *d_x, float *d_out, wd_m
     if (hc) a.hc_inject = hc->inject, a.hc = hc->hc, a.hc_round_half = hc->round_half;
     a.preselected = (flags & WD_MOE_PRESELECTED) ? 1 : 0;
     a.dry = (flags & WD_MOE_DRY) ? 1 : 0;
-    const int router_rows_n = (a.preselected ? 0 : a.E) + (shared ? 1 : 0);
-    a.n_router_wgs = (router_rows_n + 15) / 16;
+    a.ids_known = ids_override;  // a routing trace: the ids do not depend on the router
     a.trace = s->trace, a.trace_wg = s->trace_wg;
     a.arrive = s->arrive;
     a.ids_tagged = s->tagged + static_cast<size_t>(rec % kTagRecords) * kTagCopies * 16;
@@ -488,44 +486,116 @@ LayerArgs fused_args(const wd_moe_layer *L, const float *d_x, float *d_out, wd_m
     return a;
 }
 
-// Dispatch A: router logits (+ selection by the last router workgroup) and the shared expert's gate/up.
-int launch_a(const LayerArgs &a, hipStream_t st) {
-    const int grid_a = a.n_router_wgs + (a.sh_inp ? (a.F + 7) / 8 : 0);
-    if (grid_a > 0) {
-        k_layer_a<<<dim3(grid_a), dim3(512), static_cast<size_t>(a.H) + a.H / 16, st>>>(a);
-        WD_LAUNCH_CHECK();
-    }
-    return WD_OK;
-}
-
-// One layer in three dispatches (router + shared gate/up, routed gate/up, down + combine).
-template <int TYPE, bool COAL, int NB>
-void launch_layer_ab(bool loop, dim3 grid, dim3 block, size_t lds, hipStream_t st, const LayerArgs &m) {
+// Dispatch AB (or the part of it that `m` describes) of one row fetch.
+template <int TYPE, int FETCH>
+void launch_layer_ab_fetch(bool loop, int grid, hipStream_t st, const LayerArgs &m) {
+    const size_t routed = layer_ab_stage(m.H) + 8 * static_cast<size_t>(layer_ab_stage_bytes<TYPE, FETCH>(m.H));
+    const size_t lds = std::max(sizeof(float) * static_cast<size_t>(m.H) + 16, routed);
+    const dim3 block(512);
     const bool part = m.gup_part != nullptr;  // the variants that also store the int32 chunk sums
     // (the time stamps are a variant of their own, so that the others run without their tests; no stamps are taken
     // while the chunk sums are exported)
     const bool trace = m.trace != nullptr && !part;
-    if (loop && part)
-        k_layer_ab<TYPE, COAL, NB, true, true><<<grid, block, lds, st>>>(m);
-    else if (loop && trace)
-        k_layer_ab<TYPE, COAL, NB, true, false, true><<<grid, block, lds, st>>>(m);
+    if constexpr (TYPE == 21 || TYPE == 22) {
+        if (loop && part) return k_layer_ab<TYPE, FETCH, true, true><<<grid, block, lds, st>>>(m);
+        if (part) return k_layer_ab<TYPE, FETCH, false, true><<<grid, block, lds, st>>>(m);
+    }
+    if (loop && trace)
+        k_layer_ab<TYPE, FETCH, true, false, true><<<grid, block, lds, st>>>(m);
     else if (loop)
-        k_layer_ab<TYPE, COAL, NB, true><<<grid, block, lds, st>>>(m);
-    else if (part)
-        k_layer_ab<TYPE, COAL, NB, false, true><<<grid, block, lds, st>>>(m);
+        k_layer_ab<TYPE, FETCH, true><<<grid, block, lds, st>>>(m);
     else if (trace)
-        k_layer_ab<TYPE, COAL, NB, false, false, true><<<grid, block, lds, st>>>(m);
+        k_layer_ab<TYPE, FETCH, false, false, true><<<grid, block, lds, st>>>(m);
     else
-        k_layer_ab<TYPE, COAL, NB, false><<<grid, block, lds, st>>>(m);
+        k_layer_ab<TYPE, FETCH, false><<<grid, block, lds, st>>>(m);
 }
-template <int KIND, bool COAL, int NB, bool TWO>
-void launch_layer_c(dim3 grid, dim3 block, size_t lds, hipStream_t st, const LayerArgs &a) {
+template <int TYPE>
+void launch_layer_ab(int fetch, bool loop, int grid, hipStream_t st, const LayerArgs &m) {
+    switch (fetch) {
+        case 8:
+            if constexpr (TYPE == 21 || TYPE == 22) return launch_layer_ab_fetch<TYPE, 8>(loop, grid, st, m);
+            [[fallthrough]];
+        case 10:
+            if constexpr (TYPE == 21 || TYPE == 22) return launch_layer_ab_fetch<TYPE, 10>(loop, grid, st, m);
+            [[fallthrough]];
+        case 1: return launch_layer_ab_fetch<TYPE, 1>(loop, grid, st, m);
+        case 2: return launch_layer_ab_fetch<TYPE, 2>(loop, grid, st, m);
+        default: return launch_layer_ab_fetch<TYPE, 0>(loop, grid, st, m);
+    }
+}
+// Dispatch AB: with `front` the router, the selection and the shared expert's gate/up, with `routed` the routed gate/up.
+int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s, bool front, bool routed, hipStream_t st) {
+    const int H = a.H, F = a.F, groups = (F + 7) / 8;
+    const bool iq = consumes_q8k(L->gate_type), shared = a.sh_inp != nullptr;
+    auto al16 = [](const void *p, size_t v) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && v % 16 == 0; };
+    // IQ tensors that start on 16-byte boundaries (F rows are whole 16-byte words, F being a multiple of 32)
+    const bool words = !iq || (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && L->slot_gate_bytes % 16 == 0
+                                                 : al16(L->gate, L->gate_stride) && al16(L->up, L->up_stride));
+    int fetch = !words || H > 4096 ? 0 : (H > 2048 ? 2 : 1);
+    if (iq && words && H == 2048) fetch = 8;
+    if (iq && words && H == 2560) fetch = 10;
+    const bool wide = fetch == 2 || fetch == 10;
+    LayerArgs m = a;
+    const int router_rows_n = front ? (a.preselected ? 0 : a.E) + (shared ? 1 : 0) : 0;
+    m.n_router_wgs = wide ? (router_rows_n + 3) / 4 : (router_rows_n + 7) / 8;  // two waves or one per row
+    m.n_shared_wgs = front && shared ? groups : 0;
+    m.n_routed_items = routed ? a.k * groups : 0;
+    if (!routed) m.ids_tagged = nullptr;  // nobody waits for them inside this launch
+    if (!front || a.preselected) m.ids_known = s->ids;
+    // A compute unit holds three of these workgroups (two without the aligned fetch).  The router and shared ones leave well before the ids are
+    // published, so a few routed ones that have to wait for their places still start in time.  But when the routed
+    // ones alone are more than the device holds at once (hidden 2560: 800 against 768), the surplus would start -
+    // quantise x, stage the codebooks - only after others have finished: the grid is then cut to what the device
+    // holds and the routed workgroups walk the items in a loop (measured at hidden 2560: 36.4 against 37.4 us per layer;
+    // there each router row has two waves, and the routed workgroups keep their number all the same).
+    const int fixed_wgs = (router_rows_n + 7) / 8 + m.n_shared_wgs;
+    const int capacity = (fetch == 0 ? 2 : 3) * s->compute_units;
+    const int routed_wgs = m.n_routed_items <= capacity - 8 ? m.n_routed_items
+                                                            : std::min(m.n_routed_items, std::max(capacity - fixed_wgs, groups));
+    const int grid = m.n_router_wgs + m.n_shared_wgs + routed_wgs;
+    if (grid == 0) return WD_OK;
+    const bool loop = routed_wgs < m.n_routed_items;
+    switch (L->gate_type) {
+        case WD_TYPE_IQ3_S: launch_layer_ab<21>(fetch, loop, grid, st, m); break;
+        case WD_TYPE_IQ2_S: launch_layer_ab<22>(fetch, loop, grid, st, m); break;
+        case WD_TYPE_Q8_0: launch_layer_ab<8>(fetch, loop, grid, st, m); break;
+        case WD_TYPE_IQ4_NL: launch_layer_ab<20>(fetch, loop, grid, st, m); break;
+        default: return fail(WD_ERR_UNSUPPORTED, "fused layer: unsupported gate/up type %d", L->gate_type);
+    }
+    WD_LAUNCH_CHECK();
+    return WD_OK;
+}
+template <int KIND>
+void launch_layer_c(hipStream_t st, const LayerArgs &a) {
+    const int n_act = a.k + (a.sh_inp ? 1 : 0), waves = std::min(n_act, 16);
+    const size_t per_wave = (static_cast<size_t>(a.F) + a.F / 16 + 15) & ~static_cast<size_t>(15);
+    const size_t lds = waves * per_wave + sizeof(float) * 4 * n_act;
+    const dim3 grid((a.H + 3) / 4), block(64 * waves);
     if (a.down_part)
-        k_layer_c<KIND, COAL, NB, TWO, true><<<grid, block, lds, st>>>(a);
+        k_layer_c<KIND, true><<<grid, block, lds, st>>>(a);
     else if (a.trace)
-        k_layer_c<KIND, COAL, NB, TWO, false, true><<<grid, block, lds, st>>>(a);
+        k_layer_c<KIND, false, true><<<grid, block, lds, st>>>(a);
     else
-        k_layer_c<KIND, COAL, NB, TWO><<<grid, block, lds, st>>>(a);
+        k_layer_c<KIND><<<grid, block, lds, st>>>(a);
+}
+template <int KIND, int PASSES, bool WORDS>
+void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
+    const int n_act = a.k + (a.sh_inp ? 1 : 0), waves = std::max(n_act, 2);
+    const size_t lds = waves * static_cast<size_t>(layer_c8_wave_bytes<WORDS>(a.F)) + sizeof(float) * 8 * n_act;
+    const dim3 grid(a.H / 8), block(64 * waves);
+    if (a.down_part)
+        k_layer_c8<KIND, PASSES, WORDS, true><<<grid, block, lds, st>>>(a);
+    else if (a.trace)
+        k_layer_c8<KIND, PASSES, WORDS, false, true><<<grid, block, lds, st>>>(a);
+    else
+        k_layer_c8<KIND, PASSES, WORDS><<<grid, block, lds, st>>>(a);
+}
+template <int KIND>
+void launch_layer_c8(bool words, hipStream_t st, const LayerArgs &a) {
+    if (a.F <= 512) launch_layer_c8<KIND, 2, false>(st, a);
+    else if (a.F <= 768) launch_layer_c8<KIND, 3, false>(st, a);
+    else if (a.F <= 1024) words ? launch_layer_c8<KIND, 4, true>(st, a) : launch_layer_c8<KIND, 4, false>(st, a);
+    else words ? launch_layer_c8<KIND, 6, true>(st, a) : launch_layer_c8<KIND, 6, false>(st, a);
 }
 
 int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
@@ -536,118 +606,37 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
     const LayerArgs a = fused_args(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, rec, hc);
     const unsigned only = flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B | WD_MOE_ONLY_C);
     const bool run_a = !only || (only & WD_MOE_ONLY_A), run_b = !only || (only & WD_MOE_ONLY_B);
-    const bool iq = consumes_q8k(L->gate_type);
     // router + selection + shared gate/up + routed gate/up in one launch (the routed workgroups wait for the ids
-    // inside the dispatch) unless the ids are given, the tensor type has no 512-thread kernel, or the caller
-    // asked for the two dispatches apart
-    const bool merged = run_a && run_b && !a.preselected && !(flags & WD_MOE_SPLIT_AB) &&
-                        (iq || L->gate_type == WD_TYPE_Q8_0);
+    // inside the dispatch) unless the caller asked for the two parts apart
+    const bool merged = run_a && run_b && !(flags & WD_MOE_SPLIT_AB);
     if (merged) {
         SiteScope site(WD_SITE_FUSED_AB, st);
-        LayerArgs m = a;
-        m.n_router_wgs = (a.E + (shared ? 1 : 0) + 7) / 8;  // one router row per wave in the merged dispatch
-        // A compute unit holds three of these workgroups.  The router and shared ones leave well before the ids are
-        // published, so a few routed ones that have to wait for their places still start in time.  But when the routed
-        // ones alone are more than the device holds at once (hidden 2560: 800 against 768), the surplus would start -
-        // quantise x, stage the codebooks - only after others have finished: the grid is then cut to what the device
-        // holds and the routed workgroups walk the items in a loop (measured at hidden 2560: 36.4 against 37.4 us per layer).
-        m.n_routed_items = k * ((F + 7) / 8);
-        const int fixed_wgs = m.n_router_wgs + (shared ? (F + 7) / 8 : 0);
-        const int capacity = 3 * s->compute_units;
-        const int routed_wgs = m.n_routed_items <= capacity - 8 ? m.n_routed_items
-                                                                : std::min(m.n_routed_items, std::max(capacity - fixed_wgs, (F + 7) / 8));
-        // rows of eight super-blocks on 16-byte boundaries: coalesced fetch with a per-wave staging area behind lds_ab
-        auto al16_ = [](const void *p_, size_t v) { return reinterpret_cast<uintptr_t>(p_) % 16 == 0 && v % 16 == 0; };
-        // (rows of ten super-blocks are 4-byte aligned then, and F rows end on a 16-byte boundary)
-        const bool coal_ab = iq && (H == 2048 || H == 2560) &&
-                             (L->slot_of_expert ? al16_(L->slot_pool, L->slot_bytes) && L->slot_gate_bytes % 16 == 0
-                                                : al16_(L->gate, L->gate_stride) && al16_(L->up, L->up_stride));
-        if (coal_ab && H == 2560) {
-            // these variants give a router row two waves, every weight of the row requested at once: twice the router
-            // workgroups (they leave long before the routed ones stop waiting, so the routed workgroups keep their number)
-            m.n_router_wgs = (a.E + (shared ? 1 : 0) + 3) / 4;
+        if (const int rc = launch_ab(a, L, s, true, true, st)) return rc;
+    } else {
+        if (run_a) {
+            SiteScope site(WD_SITE_FUSED_A, st);
+            if (const int rc = launch_ab(a, L, s, true, false, st)) return rc;
         }
-        const int grid_ab = m.n_router_wgs + (shared ? (F + 7) / 8 : 0) + routed_wgs;
-        const size_t lds_ab = sizeof(float) * static_cast<size_t>(H) + 16;  // f32 x of the router rows; the quantised x of the others fits inside
-        const size_t lds_stage = 16 + 8 * 2 * static_cast<size_t>(H == 2048 ? kIqStageBytes : kIqStage10Bytes);
-        const dim3 grid(grid_ab), block(512);
-        const bool loop = routed_wgs < m.n_routed_items;
-        switch (L->gate_type) {
-            case WD_TYPE_IQ3_S:
-                if (coal_ab && H == 2048) launch_layer_ab<21, true, 8>(loop, grid, block, lds_ab + lds_stage, st, m);
-                else if (coal_ab) launch_layer_ab<21, true, 10>(loop, grid, block, lds_ab + lds_stage, st, m);
-                else launch_layer_ab<21, false, 8>(loop, grid, block, lds_ab, st, m);
-                break;
-            case WD_TYPE_IQ2_S:
-                if (coal_ab && H == 2048) launch_layer_ab<22, true, 8>(loop, grid, block, lds_ab + lds_stage, st, m);
-                else if (coal_ab) launch_layer_ab<22, true, 10>(loop, grid, block, lds_ab + lds_stage, st, m);
-                else launch_layer_ab<22, false, 8>(loop, grid, block, lds_ab, st, m);
-                break;
-            default: launch_layer_ab<8, false, 8>(loop, grid, block, lds_ab, st, m); break;
+        if (run_b) {
+            SiteScope site(WD_SITE_FUSED_B, st);
+            if (const int rc = launch_ab(a, L, s, false, true, st)) return rc;
         }
-        WD_LAUNCH_CHECK();
-    } else if (run_a) {
-        SiteScope site(WD_SITE_FUSED_A, st);
-        if (const int rc = launch_a(a, st)) return rc;
-    }
-    const size_t lds_b = H + (iq ? sizeof(float) * (H / 256) : sizeof(uint16_t) * (H / 32));
-    const int grid_b = k * (L->gate_type == WD_TYPE_IQ4_NL ? (F + 15) / 16 : (F + 7) / 8);
-    if (run_b && !merged) {
-        SiteScope site(WD_SITE_FUSED_B, st);
-        switch (L->gate_type) {
-            case WD_TYPE_IQ3_S:
-                if (a.gup_part) k_layer_b<21, true><<<dim3(grid_b), dim3(512), lds_b, st>>>(a);
-                else k_layer_b<21><<<dim3(grid_b), dim3(512), lds_b, st>>>(a);
-                break;
-            case WD_TYPE_IQ2_S:
-                if (a.gup_part) k_layer_b<22, true><<<dim3(grid_b), dim3(512), lds_b, st>>>(a);
-                else k_layer_b<22><<<dim3(grid_b), dim3(512), lds_b, st>>>(a);
-                break;
-            case WD_TYPE_Q8_0: k_layer_b<8><<<dim3(grid_b), dim3(512), lds_b, st>>>(a); break;
-            case WD_TYPE_IQ4_NL: k_layer_b<20><<<dim3(grid_b), dim3(256), lds_b, st>>>(a); break;
-            default: return fail(WD_ERR_UNSUPPORTED, "fused layer: unsupported gate/up type %d", L->gate_type);
-        }
-        WD_LAUNCH_CHECK();
     }
     if (only && !(only & WD_MOE_ONLY_C)) return WD_OK;
-    const int n_act = k + (shared ? 1 : 0);
-    const int grid_c = (H + 3) / 4;
-    // One wave per matrix (k routed and the shared one).  A compute unit holds two such workgroups; when the grid has
-    // more than the chip holds at once (hidden > 2048), waves take two matrices each instead, so that the smaller
-    // workgroups all run together rather than in two rounds.
-    // (With k = 16 and a shared expert there are 17 matrices, more than the 16 waves of a workgroup: halved as well.)
-    int waves_c = n_act;
-    if (grid_c > 512 || n_act > 16) waves_c = (n_act + 1) / 2;
-    const size_t per_wave = (static_cast<size_t>(F) + F / 16 + 15) & ~static_cast<size_t>(15);
-    const bool two = waves_c < n_act;  // halved above: n_act <= 2 * waves_c
-    // such a wave keeps both quantised activations and the second row group (at most 4 rows of F / 32 34-byte blocks) in LDS
-    const size_t lds_c = waves_c * (two ? 2 * per_wave + static_cast<size_t>(4) * (F / 32) * 34 : per_wave) + sizeof(float) * 4 * n_act;
-    auto al16 = [](const void *p_, size_t v) { return reinterpret_cast<uintptr_t>(p_) % 16 == 0 && v % 16 == 0; };
-    // rows of 16 or 20 blocks in 16-byte aligned groups of four: the coalesced fetch
-    const bool coal = (F == 512 || F == 640) && H % 4 == 0 && al16(L->shared_down, 0) &&
-                      (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && (L->slot_gate_bytes + L->slot_up_bytes) % 16 == 0
-                                         : al16(L->down, L->down_stride));
-    const dim3 grid(grid_c), block(64 * waves_c);
-    const bool q8 = L->down_type == WD_TYPE_Q8_0;
     SiteScope site(WD_SITE_FUSED_C, st);
-    if (coal && two) {
-        if (waves_c > 9) return fail(WD_ERR_ARG, "fused layer: %d waves in the paired down dispatch (at most 9)", waves_c);
-        if (F == 512 && q8) launch_layer_c<0, true, 16, true>(grid, block, lds_c, st, a);
-        else if (F == 512) launch_layer_c<1, true, 16, true>(grid, block, lds_c, st, a);
-        else if (q8) launch_layer_c<0, true, 20, true>(grid, block, lds_c, st, a);
-        else launch_layer_c<1, true, 20, true>(grid, block, lds_c, st, a);
-    } else if (coal && F == 512 && q8)
-        launch_layer_c<0, true, 16, false>(grid, block, lds_c, st, a);
-    else if (coal && F == 512)
-        launch_layer_c<1, true, 16, false>(grid, block, lds_c, st, a);
-    else if (coal && q8)
-        launch_layer_c<0, true, 20, false>(grid, block, lds_c, st, a);
-    else if (coal)
-        launch_layer_c<1, true, 20, false>(grid, block, lds_c, st, a);
-    else if (q8)
-        launch_layer_c<0, false, 16, false>(grid, block, lds_c, st, a);
-    else
-        launch_layer_c<1, false, 16, false>(grid, block, lds_c, st, a);
+    const int n_act = k + (shared ? 1 : 0);
+    const bool q8 = L->down_type == WD_TYPE_Q8_0;
+    if (F <= 1536 && n_act <= 16) {
+        // The aligned fetch where every down tensor starts on a 16-byte boundary and the rows' bytes are what the dispatch
+        // waits for: 40 MB and more (53.5 MB: 15.4 us against 16.3; 21 MB: 9.5 against 9.0; 15 MB: 7.5 against 7.0).
+        auto al16 = [](const void *p, size_t v) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && v % 16 == 0; };
+        const bool words = static_cast<size_t>(n_act) * wd_tensor_bytes(L->down_type, H, F) >= (40u << 20) && al16(L->shared_down, 0) &&
+                           (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && (L->slot_gate_bytes + L->slot_up_bytes) % 16 == 0
+                                              : al16(L->down, L->down_stride));
+        q8 ? launch_layer_c8<0>(words, st, a) : launch_layer_c8<1>(words, st, a);
+    } else {
+        q8 ? launch_layer_c<0>(st, a) : launch_layer_c<1>(st, a);
+    }
     WD_LAUNCH_CHECK();
     return WD_OK;
 }

@@ -306,17 +306,7 @@ WD_DEV float res_router_dot(const float (&wv)[32], const float *xt, int lane) {
     if (!upper) s = run_half(0.0f);
     const wd_uint2v fwd = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
     if (upper) s = run_half(bits_f(fwd.x));
-    // the 32 accumulators are final in the upper half: ggml's closing tree
-    float o = __shfl_down(s, 16, 32);
-    if (t < 16) s = s + o;
-    o = __shfl_down(s, 8, 32);
-    if (t < 8) s = s + o;
-    o = __shfl_down(s, 4, 32);
-    if (t < 4) s = s + o;
-    o = __shfl_down(s, 1, 32);
-    if (t == 0 || t == 2) s = s + o;
-    o = __shfl_down(s, 2, 32);
-    return s + o;
+    return router_close32(s);  // the 32 accumulators are final in the upper half
 }
 
 // ---- LDS layout -----------------------------------------------------------------------------------------------
@@ -666,7 +656,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             if constexpr (kQ8) {
                 Q8RowTile &tile = *reinterpret_cast<Q8RowTile *>(c.area());
                 float acc[2] = {0.0f, 0.0f};
-                q8_row_wave_pass<2>(gb, true, lane, c.x0q(), c.x0d(), tile, lane, acc);
+                q8_row_wave_pass<0, 2>(gb, true, lane, c.x0q(), c.x0d(), tile, lane, acc, acc);
                 gu[0] = close_lanes8(acc[0]), gu[1] = close_lanes8(acc[1]);
             } else {
                 if (decoded) iq_rows8_kept_decoded_dots<kIq>(dec, kept, c.kept(), c.xq(), c.xd(), lane, gu);
@@ -804,7 +794,7 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             res_mark<STAMPS>(a, c, l, 2);
             Q8RowTile &tile = *reinterpret_cast<Q8RowTile *>(c.area());
             float acc[2] = {0.0f, 0.0f};
-            q8_row_wave_pass<2>(gb, true, lane, c.x0q(), c.x0d(), tile, lane, acc);
+            q8_row_wave_pass<0, 2>(gb, true, lane, c.x0q(), c.x0d(), tile, lane, acc, acc);
             const float g = close_lanes8(acc[0]), u = close_lanes8(acc[1]);
             act = silu_ggml(g) * u;
             res_mark<STAMPS>(a, c, l, 5);
@@ -970,7 +960,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         bool weights_out = false;
         if (r == 0 && !traced) {
             (void)gather_logits(true);
-            sel_wave_ids(lv, a.E, a.k, lane, st);
+            sel_wave_ids(lv, a.E, a.k, scratch, lane, st);
             if (st.fast) {
                 if (lane < a.k) lds_ids[lane] = st.id;
                 publish_ids();
@@ -1005,7 +995,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         if (r == 0 && !traced && !weights_out) weights_from_lds();
         if (r == 0 && traced) {
             if (!got) (void)gather_logits(true);
-            sel_wave_ids(lv, a.E, a.k, lane, st);
+            sel_wave_ids(lv, a.E, a.k, scratch, lane, st);
             res_mark<STAMPS>(a, c, l, 13);
         }
         __syncthreads();  // B3

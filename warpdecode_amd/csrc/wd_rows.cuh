@@ -318,9 +318,9 @@ WD_DEV void iq_rows_q8k(const uint8_t *const (&rows)[NR], int nb, const IqTables
 // the even super-blocks (block offset 110 sb or 82 sb is 0 mod 4 there, and every such field sits at 2 mod 4).
 constexpr int kIqStageBytes = 896;  // per row, 16-byte multiple >= 880
 
+// (sh: 2 when blk + 2 is not on a 4-byte boundary, 0 when it is)
 template <int TYPE>
-WD_DEV IqFields iq_fields_lds(const uint8_t *blk, int ib, int sb) {
-    const uint32_t sh = (sb & 1) ? 0u : 2u;
+WD_DEV IqFields iq_fields_shifted(const uint8_t *blk, int ib, uint32_t sh) {
     IqFields f;
     f.d = *reinterpret_cast<const uint16_t *>(blk);
     if (TYPE == 21) {
@@ -342,6 +342,11 @@ WD_DEV IqFields iq_fields_lds(const uint8_t *blk, int ib, int sb) {
         f.sc = blk[74 + ib];
     }
     return f;
+}
+
+template <int TYPE>
+WD_DEV IqFields iq_fields_lds(const uint8_t *blk, int ib, int sb) {
+    return iq_fields_shifted<TYPE>(blk, ib, (sb & 1) ? 0u : 2u);
 }
 
 // iq_rows_q8k<TYPE, NR, false> for nb == 8 and 16-byte aligned rows.  stage: NR * kIqStageBytes bytes of LDS owned by
@@ -561,10 +566,12 @@ WD_DEV void iq_rows8_coal_finish(const IqRows8Raw<TYPE, NR> &raw, const IqTables
     iq_rows8_coal_park<TYPE, NR>(raw, lane, stage);
     iq_rows8_coal_dots<TYPE, NR, PART>(t, act_qs, act_d, lane, y, stage, partials, pstride);
 }
-template <int TYPE, int NR, bool PART = false>
+// (`pre` in this and the next two: as in iq_rows_q8k, between the requests and the first use of what they bring)
+template <int TYPE, int NR, bool PART = false, typename Pre = NoPre>
 WD_DEV void iq_rows8_coal(const uint8_t *const (&rows)[NR], const IqTables &t, const int8_t *act_qs, const float *act_d,
-                          int lane, float (&y)[NR], uint8_t *stage, int32_t *partials = nullptr, size_t pstride = 0) {
+                          int lane, float (&y)[NR], uint8_t *stage, int32_t *partials = nullptr, size_t pstride = 0, Pre pre = Pre()) {
     const IqRows8Raw<TYPE, NR> raw = iq_rows8_coal_request<TYPE, NR>(rows, lane);
+    pre();
     iq_rows8_coal_finish<TYPE, NR, PART>(raw, t, act_qs, act_d, lane, y, stage, partials, pstride);
 }
 
@@ -604,9 +611,9 @@ struct IqRowFetch {
 // position 2 i (a row shift), two more steps follow, and the result moves back to the last position for the closing tree.
 // rows[i]: 4-byte aligned, inside a tensor whose end is 16-byte aligned.  stage: NR * kIqStage10Bytes bytes of LDS
 // owned by the wave, 16-byte aligned.  NR <= 4.
-template <int TYPE, int NR, bool PART = false>
+template <int TYPE, int NR, bool PART = false, typename Pre = NoPre>
 WD_DEV void iq_rows10_coal(const uint8_t *const (&rows)[NR], const IqTables &t, const int8_t *act_qs, const float *act_d,
-                           int lane, float (&y)[NR], uint8_t *stage, int32_t *partials = nullptr, size_t pstride = 0) {
+                           int lane, float (&y)[NR], uint8_t *stage, int32_t *partials = nullptr, size_t pstride = 0, Pre pre = Pre()) {
     static_assert(NR >= 1 && NR <= 4, "the tails of the rows share one pass of eight positions");
     constexpr int kBlk = (TYPE == 21) ? 110 : 82, kRow = 10 * kBlk;
     constexpr bool kTwoLoads = 12 + kRow > 1024;
@@ -623,6 +630,7 @@ WD_DEV void iq_rows10_coal(const uint8_t *const (&rows)[NR], const IqTables &t, 
             raw0[i] = gld_u128_aligned(base + 16 * min(lane, words[i] - 1));
             if (kTwoLoads) raw1[i] = gld_u128_aligned(base + 16 * min(64 + lane, words[i] - 1));
         }
+        pre();
 #pragma unroll
         for (int i = 0; i < NR; ++i) {  // lanes past the last word repeat it
             uint4 *st = reinterpret_cast<uint4 *>(stage + i * kIqStage10Bytes);
@@ -685,6 +693,77 @@ WD_DEV void iq_rows10_coal(const uint8_t *const (&rows)[NR], const IqTables &t, 
         if (NR > 2) acc[NR > 2 ? 2 : 0] = dpp_f<0x114>(0.0f, v9);
         // (NR == 4: row 3's result is already at position 7)
         if (NR > 3) acc[NR > 3 ? 3 : 0] = v9;
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+        const float r = close_chains_pairs(acc[i]);
+        y[i] = (TYPE == 22) ? 0.125f * r : r;
+    }
+}
+
+// iq_rows_q8k<TYPE, NR, PART> for any number of super-blocks with the aligned fetch: every row is fetched as the 16-byte
+// words that cover it, LOADS per lane (at most 64 LOADS words: 9 super-blocks for LOADS == 1, 18 for 2), all rows before
+// the first is used, and the passes of eight super-blocks pick their fields from LDS.  Lane layout and chain as in
+// iq_rows8_coal_dots; the chain's value moves from the last position of a pass to the first of the next (row_shl:14), and
+// positions past the row's end pass it through unchanged, fma(0, 0, acc) == acc.
+// rows[i]: 2-byte aligned, inside a tensor whose beginning and end are 16-byte aligned.  stage: NR * iq_cover_bytes(nb)
+// bytes of LDS owned by the wave, 16-byte aligned.
+template <int TYPE>
+__host__ __device__ constexpr uint32_t iq_cover_bytes(int nb) { return static_cast<uint32_t>(14 + nb * (TYPE == 21 ? 110 : 82) + 15) & ~15u; }
+template <int TYPE, int NR, int LOADS, bool PART = false, typename Pre = NoPre>
+WD_DEV void iq_rows_cover(const uint8_t *const (&rows)[NR], int nb, const IqTables &t, const int8_t *act_qs, const float *act_d,
+                          int lane, float (&y)[NR], uint8_t *stage, int32_t *partials = nullptr, size_t pstride = 0, Pre pre = Pre()) {
+    constexpr int kBlk = (TYPE == 21) ? 110 : 82;
+    const int ib = ((lane >> 4) << 1) | (lane & 1), pos = (lane >> 1) & 7;
+    const uint32_t stride = iq_cover_bytes<TYPE>(nb);
+    uint32_t lead[NR];
+    {
+        uint4 raw[NR][LOADS];
+        int words[NR];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            lead[i] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(rows[i])) & 15u;  // the same in every lane
+            words[i] = static_cast<int>((lead[i] + nb * kBlk + 15) >> 4);
+            const uint8_t *base = rows[i] - lead[i];
+#pragma unroll
+            for (int q = 0; q < LOADS; ++q) raw[i][q] = gld_u128_aligned(base + 16 * min(64 * q + lane, words[i] - 1));
+        }
+        pre();
+#pragma unroll
+        for (int i = 0; i < NR; ++i)  // lanes past the last word repeat it
+#pragma unroll
+            for (int q = 0; q < LOADS; ++q) reinterpret_cast<uint4 *>(stage + i * stride)[min(64 * q + lane, words[i] - 1)] = raw[i][q];
+    }
+    wave_lds_fence();
+    float acc[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) acc[i] = 0.0f;
+    for (int base = 0; base < nb; base += 8) {
+        const bool on = base + pos < nb;
+        const int sb = min(base + pos, nb - 1);  // positions past the row's end read its last super-block and contribute zero
+        const uint4 a0 = *reinterpret_cast<const uint4 *>(act_qs + sb * 256 + ib * 32);
+        const uint4 a1 = *reinterpret_cast<const uint4 *>(act_qs + sb * 256 + ib * 32 + 16);
+        const uint32_t a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        const float dx = on ? act_d[sb] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const uint32_t off = lead[i] + sb * kBlk;  // even
+            const IqFields f = iq_fields_shifted<TYPE>(stage + i * stride + off, ib, (off + 2) & 2u);
+            int p[8];
+            iq_chunks<TYPE>(f, ib, t, a, p);
+            const float ds = on ? h2f(f.d) * dx : 0.0f;
+            const int P = reduce_scatter_ib_pairs(p, lane);  // lane (c = ib, sb): chunk c of super-block sb
+            if (PART && on) partials[i * pstride + sb * 8 + ib] = P;
+            const float pf = on ? static_cast<float>(P) : 0.0f;
+            float up = base == 0 ? 0.0f : dpp_f<kDppShl14>(0.0f, acc[i]);
+            float v = __builtin_fmaf(ds, pf, up);
+#pragma unroll
+            for (int s = 1; s < 8; ++s) {
+                up = dpp_f<kDppShr2>(up, v);  // (the chain's first lanes have no source and keep the carry)
+                v = __builtin_fmaf(ds, pf, up);
+            }
+            acc[i] = v;
+        }
     }
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
@@ -839,12 +918,11 @@ WD_DEV float q6k_close(float v) {
 // Four rows per wave step: lane (r4 = lane >> 4, b = lane & 15) takes blocks b, b+16, ... of row r4.
 // The per-block chunk sums are handed to the chain lanes through a per-wave LDS tile so that every
 // chunk accumulator sees its blocks in ascending order.
-template <int CH>
-struct Q8TileN {
-    float pf[CH][4 * 136];  // [pass][r4][b][c], row stride padded to 136 floats (bank spread)
-    float ds[CH][64];       // [pass][r4][b]
+struct Q8Tile {
+    float pf[4 * 136];  // [r4][b][c], row stride padded to 136 floats (bank spread)
+    float ds[64];       // [r4][b]
+    float tail[4];      // IQ4_NL: the trailing unpaired block of every row
 };
-using Q8Tile = Q8TileN<1>;
 
 // kind: 0 = Q8_0 (34-byte blocks), 1 = IQ4_NL (18-byte blocks, codebook values)
 struct Q8Block {
@@ -890,117 +968,179 @@ WD_DEV void q8_chunks(const Q8Block &w, const uint32_t (&a)[8], int (&p)[8]) {
     }
 }
 
-// NM matrices, the same four consecutive rows of each (row stride = nb * block bytes), against one
-// Q8_0 activation.  rows[i]: first of the (up to) four rows of matrix i; nrows (0..4) rows are valid.
-// y[i] for row r4 valid in lane r4*16.  CH passes (16 blocks per row each) of every matrix are
-// loaded before the first one is decoded, and their chunk sums go through the tile together, so a
-// row of up to 16*CH blocks needs one hand-off.
-// partials (PART): int32 [4][nb][8] per matrix, matrices `pstride` ints apart.
-template <int KIND, int NM, int CH, bool PART, typename Pre = NoPre>
-WD_DEV void q8_rows4_multi(const uint8_t *const (&rows)[NM], int nrows, int nb, const int8_t *act_qs,
-                           const uint16_t *act_d, Q8TileN<CH> &tile, int lane, float (&y)[NM], int32_t *partials,
-                           size_t pstride, Pre pre = Pre()) {
-    constexpr int kBlk = (KIND == 0) ? 34 : 18;
-    const int r4 = lane >> 4, b = lane & 15, c = lane & 7;
-    const bool row_on = r4 < nrows;
-    const size_t row_off = static_cast<size_t>(r4) * nb * kBlk;
-    // IQ4_NL pairs blocks into an even and an odd accumulator and treats a trailing unpaired block
-    // apart (src/qwen38_cpu_moe.cuh:377-422).
-    float acc[NM], acc_odd[NM], tail[NM];
+// Four consecutive rows (row stride = nb * block bytes) of which nrows (1..4) are valid, against one Q8_0 activation.
+// One pass: blocks base .. base + 15 of every row (w: the lane's block, any block when it lies past the end), then sixteen
+// chain steps.  Slots of blocks past the end hold zeros: those steps are fma(0, 0, acc) == acc (acc is never -0).
+// IQ4_NL pairs blocks into an even and an odd accumulator; a trailing unpaired block is apart (src/qwen38_cpu_moe.cuh:377-422):
+// one rounded product with the whole-block integer sum, added after the closing tree.
+// partials (PART): int32 [4][nb][8].
+struct Q8Chain {
+    float acc = 0.0f, odd = 0.0f;
+};
+template <int KIND, bool PART>
+WD_DEV void q8_rows4_pass(const Q8Block &w, int base, int nrows, int nb, const int8_t *act_qs, const uint16_t *act_d, Q8Tile &tile,
+                          int lane, Q8Chain &ch, int32_t *partials) {
+    const int r4 = lane >> 4, b = lane & 15, c = lane & 7, bi = base + b;
+    const bool on = r4 < nrows && bi < nb;
+    int p[8];
+    float ds = 0.0f;
+    if (on) {
+        const uint4 a0 = *reinterpret_cast<const uint4 *>(act_qs + bi * 32);
+        const uint4 a1 = *reinterpret_cast<const uint4 *>(act_qs + bi * 32 + 16);
+        const uint32_t a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        q8_chunks<KIND>(w, a, p);
+        ds = h2f(w.d) * h2f(act_d[bi]);
+        if (PART) {
 #pragma unroll
-    for (int i = 0; i < NM; ++i) acc[i] = acc_odd[i] = tail[i] = 0.0f;
-    const int paired = (KIND == 1) ? (nb & ~1) : nb;
-    for (int base0 = 0; base0 < nb; base0 += 16 * CH) {
-        Q8Block wb[NM][CH];
-        uint4 a0[CH], a1[CH];
-        uint16_t dxh[CH];
-#pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            const int bi = base0 + 16 * ch + b;
-            if (row_on && bi < nb) {
-#pragma unroll
-                for (int i = 0; i < NM; ++i) wb[i][ch] = q8_load<KIND>(rows[i] + row_off + static_cast<size_t>(bi) * kBlk);
-            }
+            for (int j = 0; j < 8; ++j) partials[(static_cast<size_t>(r4) * nb + bi) * 8 + j] = p[j];
         }
-        if (base0 == 0) pre();
+    } else {
 #pragma unroll
-        for (int ch = 0; ch < CH; ++ch) {
-            const int bi = base0 + 16 * ch + b;
-            if (row_on && bi < nb) {
-                a0[ch] = *reinterpret_cast<const uint4 *>(act_qs + bi * 32);
-                a1[ch] = *reinterpret_cast<const uint4 *>(act_qs + bi * 32 + 16);
-                dxh[ch] = act_d[bi];
-            }
-        }
+        for (int j = 0; j < 8; ++j) p[j] = 0;
+    }
+    wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
+    if (KIND == 1 && (nb & 1) && bi == nb - 1) {
+        int tot = 0;  // (exact integers below 2^24)
 #pragma unroll
-        for (int i = 0; i < NM; ++i) {
-            wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
+        for (int j = 0; j < 8; ++j) tot += p[j], p[j] = 0;
+        tile.tail[r4] = ds * static_cast<float>(tot);
+        ds = 0.0f;
+    }
+    float4 *dst = reinterpret_cast<float4 *>(&tile.pf[r4 * 136 + b * 8]);
+    dst[0] = make_float4(static_cast<float>(p[0]), static_cast<float>(p[1]), static_cast<float>(p[2]), static_cast<float>(p[3]));
+    dst[1] = make_float4(static_cast<float>(p[4]), static_cast<float>(p[5]), static_cast<float>(p[6]), static_cast<float>(p[7]));
+    tile.ds[lane] = ds;
+    wave_lds_fence();
 #pragma unroll
-            for (int ch = 0; ch < CH; ++ch) {
-                const int bi = base0 + 16 * ch + b;
-                const bool on = row_on && bi < nb;
-                int p[8];
-                float ds = 0.0f;
-                if (on) {
-                    const uint32_t a[8] = {a0[ch].x, a0[ch].y, a0[ch].z, a0[ch].w, a1[ch].x, a1[ch].y, a1[ch].z, a1[ch].w};
-                    q8_chunks<KIND>(wb[i][ch], a, p);
-                    ds = h2f(wb[i][ch].d) * h2f(dxh[ch]);
-                    if (PART) {
+    for (int s = 0; s < 16; ++s) {
+        const float pv = tile.pf[r4 * 136 + s * 8 + c], dv = tile.ds[r4 * 16 + s];
+        float &acc = (KIND == 1 && (s & 1)) ? ch.odd : ch.acc;
+        acc = __builtin_fmaf(dv, pv, acc);
+    }
+}
+// y of row r4, valid in lane 16 r4
+template <int KIND>
+WD_DEV float q8_rows4_close(const Q8Chain &ch, int nb, const Q8Tile &tile, int lane) {
+    const float r = close_lanes8(KIND == 1 ? ch.acc + ch.odd : ch.acc);
+    return (KIND == 1 && (nb & 1)) ? r + tile.tail[lane >> 4] : r;
+}
+// ---- the same, eight rows per wave: lane (row = lane >> 3, b = lane & 7) takes blocks b, b + 8, ... -----------------------
+// A pass of 64 blocks is eight of every row, so that the chain step that follows - lane (row, c) - uses every lane as well
+// and a pass has eight chain steps instead of sixteen.
+struct Q8Tile8 {
+    static constexpr int kRow = 72;  // floats per row, padded (bank spread)
+    float pf[8 * kRow];              // [row][b][c]
+    float ds[8 * 8];                 // [row][b]
+    float tail[8];
+};
+// Every lane loads its own blocks of CH passes, all at once.  (A block past the row's end is read as the row's last and not
+// used, so that no request hangs on a branch.)
+template <int KIND, int CH>
+struct Q8Rows8Blocks {
+    Q8Block w[CH];
+    WD_DEV void request(const uint8_t *group, int nb, int lane) {
+        constexpr int kBlk = (KIND == 0) ? 34 : 18;
+        const int row = lane >> 3, b = lane & 7;
 #pragma unroll
-                        for (int j = 0; j < 8; ++j) partials[i * pstride + (static_cast<size_t>(r4) * nb + bi) * 8 + j] = p[j];
-                    }
-                } else {
+        for (int i = 0; i < CH; ++i) w[i] = q8_load<KIND>(group + static_cast<uint32_t>(row * nb + min(8 * i + b, nb - 1)) * kBlk);
+    }
+};
+// Or the rows come in as aligned 16-byte words: the eight rows are 8 nb blocks in a row, which is a whole number of words
+// whatever nb is, so a group of eight starts on a 16-byte boundary when the tensor does.  A step of sixteen blocks of every
+// row (two passes) is at most kSegWords words per row - rows themselves need not be aligned -, fetched by the lanes in turn
+// and parked with a row stride of that many words; a lane then cuts its block out of the parked words.  Loads of one block
+// per lane, 16 + 16 + 2 bytes at a stride of 34 on 2-byte boundaries, keep the memory pipeline of a compute unit busy several
+// times as long as aligned ones, which tells where it is that pipeline a dispatch waits for (k_layer_c8, wd_fused.cuh);
+// elsewhere the way through LDS costs more than it saves.
+template <int KIND>
+struct Q8Rows8 {
+    static constexpr int kBlk = (KIND == 0) ? 34 : 18;
+    static constexpr int kSegBytes = 16 * kBlk, kSegWords = (kSegBytes + 14 + 15) / 16, kLoads = (8 * kSegWords + 63) / 64;
+    static constexpr int kStageBytes = 8 * kSegWords * 16;
+};
+constexpr int kQ8Rows8StageBytes = Q8Rows8<0>::kStageBytes;  // serves both kinds
+template <int KIND, int STEPS>
+struct Q8Rows8Fetch {
+    using R = Q8Rows8<KIND>;
+    uint4 u[STEPS][R::kLoads];
+    // group: the first of the eight rows, on a 16-byte boundary
+    WD_DEV void request(const uint8_t *group, int nb, int lane) {
+        const uint32_t rb = static_cast<uint32_t>(nb * R::kBlk), last = 8 * rb - 16;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) p[j] = 0;
-                }
-                float4 *dst = reinterpret_cast<float4 *>(&tile.pf[ch][r4 * 136 + b * 8]);
-                dst[0] = make_float4(static_cast<float>(p[0]), static_cast<float>(p[1]), static_cast<float>(p[2]),
-                                     static_cast<float>(p[3]));
-                dst[1] = make_float4(static_cast<float>(p[4]), static_cast<float>(p[5]), static_cast<float>(p[6]),
-                                     static_cast<float>(p[7]));
-                tile.ds[ch][lane] = ds;
-            }
-            wave_lds_fence();
+        for (int i = 0; i < R::kLoads; ++i) {
+            const uint32_t idx = min(static_cast<uint32_t>(64 * i + lane), static_cast<uint32_t>(8 * R::kSegWords - 1));
+            const uint32_t row = idx / R::kSegWords, word = idx - row * R::kSegWords;
+            const uint32_t off = ((row * rb) & ~15u) + 16 * word;
 #pragma unroll
-            for (int ch = 0; ch < CH; ++ch) {
-                const int base = base0 + 16 * ch;
-#pragma unroll
-                for (int s = 0; s < 16; ++s) {
-                    if (KIND == 1) {
-                        const int blk_i = base + s;
-                        if (blk_i < paired) {
-                            const float pv = tile.pf[ch][r4 * 136 + s * 8 + c];
-                            const float dv = tile.ds[ch][r4 * 16 + s];
-                            if (blk_i & 1)
-                                acc_odd[i] = __builtin_fmaf(dv, pv, acc_odd[i]);
-                            else
-                                acc[i] = __builtin_fmaf(dv, pv, acc[i]);
-                        }
-                    } else {
-                        // every slot of the tile was written this pass, zeros for the blocks past the end of the row:
-                        // those steps are fma(0, 0, acc) == acc (acc is never -0), so the chain needs no test
-                        const float pv = tile.pf[ch][r4 * 136 + s * 8 + c];
-                        const float dv = tile.ds[ch][r4 * 16 + s];
-                        acc[i] = __builtin_fmaf(dv, pv, acc[i]);
-                    }
-                }
-                if (KIND == 1 && (nb & 1) && base < nb && base + 16 >= nb) {
-                    // trailing unpaired block: one rounded product with the whole-block integer sum
-                    // (every chunk value is an exact integer < 2^24), added after the closing tree
-                    const int s = (nb - 1) & 15;
-                    float tot = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) tot += tile.pf[ch][r4 * 136 + s * 8 + j];
-                    tail[i] = tile.ds[ch][r4 * 16 + s] * tot;
-                }
-            }
+            for (int q = 0; q < STEPS; ++q) u[q][i] = gld_u128_aligned(group + min(off + q * R::kSegBytes, last));  // (past the end: the last word, not used)
         }
     }
+    WD_DEV void park(int q, uint8_t *stage, int lane) const {
 #pragma unroll
-    for (int i = 0; i < NM; ++i) {
-        const float r = close_lanes8((KIND == 1) ? acc[i] + acc_odd[i] : acc[i]);
-        y[i] = (KIND == 1 && (nb & 1)) ? r + tail[i] : r;
+        for (int i = 0; i < R::kLoads; ++i) reinterpret_cast<uint4 *>(stage)[min(64 * i + lane, 8 * R::kSegWords - 1)] = u[q][i];
     }
+};
+// Block b (0..15) of the step, of row `row`, out of the parked words.
+template <int KIND>
+WD_DEV Q8Block q8_rows8_block(const uint8_t *stage, int nb, int row, int b) {
+    using R = Q8Rows8<KIND>;
+    const uint32_t off = static_cast<uint32_t>(row * (R::kSegWords * 16)) + ((row * nb * R::kBlk) & 15u) + b * R::kBlk, sh = (off + 2) & 2u;
+    Q8Block w;
+    w.d = *reinterpret_cast<const uint16_t *>(stage + off);
+    const uint32_t *sw = reinterpret_cast<const uint32_t *>(stage + (off + 2 - sh));
+    constexpr int kWords = (KIND == 0) ? 9 : 5;
+    uint32_t r[kWords];
+#pragma unroll
+    for (int j = 0; j < kWords; ++j) r[j] = sw[j];
+    w.q0.x = __builtin_amdgcn_alignbyte(r[1], r[0], sh), w.q0.y = __builtin_amdgcn_alignbyte(r[2], r[1], sh);
+    w.q0.z = __builtin_amdgcn_alignbyte(r[3], r[2], sh), w.q0.w = __builtin_amdgcn_alignbyte(r[4], r[3], sh);
+    if (KIND == 0) {
+        w.q1.x = __builtin_amdgcn_alignbyte(r[5], r[4], sh), w.q1.y = __builtin_amdgcn_alignbyte(r[6], r[5], sh);
+        w.q1.z = __builtin_amdgcn_alignbyte(r[7], r[6], sh), w.q1.w = __builtin_amdgcn_alignbyte(r[8], r[7], sh);
+    }
+    return w;
+}
+template <int KIND, bool PART>
+WD_DEV void q8_rows8_pass(const Q8Block &w, int base, int nb, const int8_t *act_qs, const uint16_t *act_d, Q8Tile8 &tile, int lane,
+                          Q8Chain &ch, int32_t *partials) {
+    const int row = lane >> 3, b = lane & 7, c = b, bi = base + b, bc = min(bi, nb - 1);
+    const uint4 a0 = *reinterpret_cast<const uint4 *>(act_qs + bc * 32);
+    const uint4 a1 = *reinterpret_cast<const uint4 *>(act_qs + bc * 32 + 16);
+    const uint32_t a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+    int p[8];
+    q8_chunks<KIND>(w, a, p);
+    if (PART && bi < nb) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) partials[(static_cast<size_t>(row) * nb + bi) * 8 + j] = p[j];
+    }
+    // (a block past the row's end: fma(0, finite, acc) == acc, the chain's value never being -0)
+    float ds = bi < nb ? h2f(w.d) * h2f(act_d[bc]) : 0.0f;
+    wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
+    if (KIND == 1 && (nb & 1) && bi == nb - 1) {
+        int tot = 0;  // (exact integers below 2^24)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) tot += p[j];
+        tile.tail[row] = ds * static_cast<float>(tot);
+        ds = 0.0f;
+    }
+    float4 *dst = reinterpret_cast<float4 *>(&tile.pf[row * Q8Tile8::kRow + b * 8]);
+    dst[0] = make_float4(static_cast<float>(p[0]), static_cast<float>(p[1]), static_cast<float>(p[2]), static_cast<float>(p[3]));
+    dst[1] = make_float4(static_cast<float>(p[4]), static_cast<float>(p[5]), static_cast<float>(p[6]), static_cast<float>(p[7]));
+    tile.ds[lane] = ds;
+    wave_lds_fence();
+    const float4 d0 = *reinterpret_cast<const float4 *>(&tile.ds[row * 8]), d1 = *reinterpret_cast<const float4 *>(&tile.ds[row * 8 + 4]);
+    const float dv[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        float &acc = (KIND == 1 && (s & 1)) ? ch.odd : ch.acc;
+        acc = __builtin_fmaf(dv[s], tile.pf[row * Q8Tile8::kRow + s * 8 + c], acc);
+    }
+}
+// y of the lane's row, valid in lane 8 row
+template <int KIND>
+WD_DEV float q8_rows8_close(const Q8Chain &ch, int nb, const Q8Tile8 &tile, int lane) {
+    const float r = close_lanes8(KIND == 1 ? ch.acc + ch.odd : ch.acc);
+    return (KIND == 1 && (nb & 1)) ? r + tile.tail[lane >> 3] : r;
 }
 
 // ---- Q8_0 / IQ4_NL x Q8_0, four rows of 16 or 20 blocks, aligned fetch -----------------------------------------
@@ -1059,21 +1199,6 @@ WD_DEV void q8_rows4_coal_stage(const Q8CoalRaw<KIND, NB> &raw, uint8_t *stage, 
 #pragma unroll
     for (int i = 0; i < Raw::kLoads; ++i) reinterpret_cast<uint4 *>(stage)[min(i * 64 + lane, Raw::kWords - 1)] = raw.u[i];
 }
-// Request and staging for a kind only known at run time (words: Q8CoalRaw<kind, NB>::kWords, the same in every lane):
-// always as many loads as Q8_0 rows need, the surplus ones repeating the last word, so that the number of loads in
-// flight does not depend on the kind.
-template <int NB>
-WD_DEV Q8CoalRaw<0, NB> q8_rows4_coal_request_any(const uint8_t *rows, int words, int lane) {
-    Q8CoalRaw<0, NB> raw;
-#pragma unroll
-    for (int i = 0; i < Q8CoalRaw<0, NB>::kLoads; ++i) raw.u[i] = gld_u128_aligned(rows + 16 * min(i * 64 + lane, words - 1));
-    return raw;
-}
-template <int NB>
-WD_DEV void q8_rows4_coal_stage_any(const Q8CoalRaw<0, NB> &raw, uint8_t *stage, int words, int lane) {
-#pragma unroll
-    for (int i = 0; i < Q8CoalRaw<0, NB>::kLoads; ++i) reinterpret_cast<uint4 *>(stage)[min(i * 64 + lane, words - 1)] = raw.u[i];
-}
 // The dot products of the four staged rows; `stage` may be the tile itself (its chunk-sum area is overwritten only
 // after the staged bytes have been read).  y of row r4 valid in lane 16 r4.  The float order is that of q8_rows4_multi.
 // partials (PART): int32 [4 rows][NB blocks][8 chunk lanes].
@@ -1126,25 +1251,22 @@ WD_DEV float q8_rows4_coal_finish(const Q8CoalRaw<KIND, NB> &raw, const int8_t *
     wave_lds_fence();
     return q8_rows4_coal_dots<KIND, NB, PART>(stage, act_qs, act_d, tile, lane, partials);
 }
-// rows: first of the four rows.  `pre` runs between the request and the first read of the activation.
-template <int KIND, int NB, typename Pre = NoPre>
-WD_DEV float q8_rows4_coal(const uint8_t *rows, const int8_t *act_qs, const uint16_t *act_d, Q8TileNB<NB> &tile, int lane,
-                           Pre pre = Pre()) {
-    const Q8CoalRaw<KIND, NB> raw = q8_rows4_coal_request<KIND, NB>(rows, lane);
-    pre();
-    return q8_rows4_coal_finish<KIND, NB>(raw, act_qs, act_d, tile, lane);
-}
-
-template <int KIND, bool PART>
+// Rows of any length, pass by pass.  `pre` runs once, behind the first pass's request.
+template <int KIND, bool PART, typename Pre = NoPre>
 WD_DEV float q8_rows4(const uint8_t *rows, int nrows, int nb, const int8_t *act_qs, const uint16_t *act_d,
-                      Q8Tile &tile, int lane, int32_t *partials) {
-    const uint8_t *const rr[1] = {rows};
-    float y[1];
-    q8_rows4_multi<KIND, 1, 1, PART, NoPre>(rr, nrows, nb, act_qs, act_d, tile, lane, y, partials, 0);
-    return y[0];
+                      Q8Tile &tile, int lane, int32_t *partials, Pre pre = Pre()) {
+    Q8Chain ch;
+    for (int base = 0; base < nb; base += 16) {
+        // (a block past the row's or the group's end is read as one inside and not used)
+        const int row = min(lane >> 4, nrows - 1), bi = min(base + (lane & 15), nb - 1);
+        const Q8Block w = q8_load<KIND>(rows + (static_cast<size_t>(row) * nb + bi) * (KIND == 0 ? 34 : 18));
+        if (base == 0) pre();
+        q8_rows4_pass<KIND, PART>(w, base, nrows, nb, act_qs, act_d, tile, lane, ch, partials);
+    }
+    return q8_rows4_close<KIND>(ch, nb, tile, lane);
 }
 
-// ---- Q8_0 x Q8_0, one row per wave ---------------------------------------------------------------------
+// ---- Q8_0 or IQ4_NL x Q8_0, one row per wave ------------------------------------------------------------
 // For long rows (gate/up projections): lane b takes blocks b, b + 64, ...  The chunk sums of a pass
 // are handed over transposed ([chunk][block]) so that the chain lanes read them four at a time.
 struct Q8RowTile {
@@ -1152,12 +1274,16 @@ struct Q8RowTile {
     float ds[64];
 };
 
-// rows[i]: the row of matrix i.  y[i] valid in lane 0 (every aligned group of 8 lanes runs the same chain).
 // One pass of the row chains: block `bi` of every matrix (wb[i], loaded by the caller; lanes with on == false
-// contribute nothing) against the activation; acc[i] is chunk lane (lane & 7)'s accumulator.
-template <int NM>
+// contribute nothing) against the activation; acc[i] is chunk lane (lane & 7)'s accumulator (IQ4_NL: of the even blocks,
+// acc_odd[i] that of the odd ones).  next(i) runs once the block of matrix i has been used: the place to request the
+// matrix's block of the next pass, so that it travels under this pass's chain.
+struct NoNext {
+    WD_DEV void operator()(int) const {}
+};
+template <int KIND, int NM, typename Next = NoNext>
 WD_DEV void q8_row_wave_pass(const Q8Block (&wb)[NM], bool on, int bi, const int8_t *act_qs, const uint16_t *act_d,
-                             Q8RowTile &tile, int lane, float (&acc)[NM]) {
+                             Q8RowTile &tile, int lane, float (&acc)[NM], float (&acc_odd)[NM], Next next = Next()) {
     const int c = lane & 7;
     uint32_t a[8];
     float dx = 0.0f;
@@ -1172,12 +1298,13 @@ WD_DEV void q8_row_wave_pass(const Q8Block (&wb)[NM], bool on, int bi, const int
         int p[8];
         float ds = 0.0f;
         if (on) {
-            q8_chunks<0>(wb[i], a, p);
+            q8_chunks<KIND>(wb[i], a, p);
             ds = h2f(wb[i].d) * dx;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) p[j] = 0;
         }
+        next(i);
         wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
 #pragma unroll
         for (int j = 0; j < 8; ++j) tile.pf[j][lane] = static_cast<float>(p[j]);
@@ -1189,34 +1316,50 @@ WD_DEV void q8_row_wave_pass(const Q8Block (&wb)[NM], bool on, int bi, const int
         for (int s4 = 0; s4 < 16; ++s4) {
             const float4 pv = *reinterpret_cast<const float4 *>(&tile.pf[c][4 * s4]);
             const float4 dv = *reinterpret_cast<const float4 *>(&tile.ds[4 * s4]);
+            float &odd = KIND == 1 ? acc_odd[i] : acc[i];
             acc[i] = __builtin_fmaf(dv.x, pv.x, acc[i]);
-            acc[i] = __builtin_fmaf(dv.y, pv.y, acc[i]);
+            odd = __builtin_fmaf(dv.y, pv.y, odd);
             acc[i] = __builtin_fmaf(dv.z, pv.z, acc[i]);
-            acc[i] = __builtin_fmaf(dv.w, pv.w, acc[i]);
+            odd = __builtin_fmaf(dv.w, pv.w, odd);
         }
     }
 }
 
 // rows[i]: the row of matrix i.  y[i] valid in lane 0 (every aligned group of 8 lanes runs the same chain).
-template <int NM, typename Pre = NoPre>
+// IQ4_NL: an even number of blocks (a trailing unpaired block would not be part of a chain).
+// TWO: rows of 65..128 blocks; the second pass's blocks of a matrix are requested as soon as its first ones have been used
+// (otherwise rows of any length, every pass waits for its own blocks).
+template <int KIND, int NM, bool TWO, typename Pre = NoPre>
 WD_DEV void q8_row_wave(const uint8_t *const (&rows)[NM], int nb, const int8_t *act_qs, const uint16_t *act_d,
                         Q8RowTile &tile, int lane, float (&y)[NM], Pre pre = Pre()) {
-    float acc[NM];
+    constexpr int kBlk = (KIND == 0) ? 34 : 18;
+    float acc[NM], acc_odd[NM];
 #pragma unroll
-    for (int i = 0; i < NM; ++i) acc[i] = 0.0f;
-    for (int base = 0; base < nb; base += 64) {
-        const int bi = base + lane;
-        const bool on = bi < nb;
-        Q8Block wb[NM];
-        if (on) {
+    for (int i = 0; i < NM; ++i) acc[i] = acc_odd[i] = 0.0f;
+    if constexpr (TWO) {
+        Q8Block wb[NM], wb2[NM];
 #pragma unroll
-            for (int i = 0; i < NM; ++i) wb[i] = q8_load<0>(rows[i] + static_cast<size_t>(bi) * 34);
+        for (int i = 0; i < NM; ++i) wb[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(lane) * kBlk);
+        pre();
+        // (blocks past the row's end are read as its last one and not used, so that no request hangs on a branch)
+        q8_row_wave_pass<KIND, NM>(wb, true, lane, act_qs, act_d, tile, lane, acc, acc_odd, [&](int i) {
+            wb2[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(min(64 + lane, nb - 1)) * kBlk);
+        });
+        q8_row_wave_pass<KIND, NM>(wb2, 64 + lane < nb, 64 + lane, act_qs, act_d, tile, lane, acc, acc_odd);
+    } else {
+        for (int base = 0; base < nb; base += 64) {
+            const int bi = base + lane;
+            Q8Block wb[NM];
+            if (bi < nb) {
+#pragma unroll
+                for (int i = 0; i < NM; ++i) wb[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(bi) * kBlk);
+            }
+            if (base == 0) pre();
+            q8_row_wave_pass<KIND, NM>(wb, bi < nb, bi, act_qs, act_d, tile, lane, acc, acc_odd);
         }
-        if (base == 0) pre();
-        q8_row_wave_pass<NM>(wb, on, bi, act_qs, act_d, tile, lane, acc);
     }
 #pragma unroll
-    for (int i = 0; i < NM; ++i) y[i] = close_lanes8(acc[i]);
+    for (int i = 0; i < NM; ++i) y[i] = close_lanes8(KIND == 1 ? acc[i] + acc_odd[i] : acc[i]);
 }
 
 // ---- dense Q4_0 x Q8_0 (src/warodecode.cu:1534-1562; no canonical float order) ------------

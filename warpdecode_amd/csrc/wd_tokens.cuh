@@ -87,7 +87,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     const TokenSlots &s = ta.tok[token];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wg < a.n_router_wgs) {
-        router_rows_wave<true, true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, a.preselected ? 0 : a.E, a.H,
+        router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, a.preselected ? 0 : a.E, a.H,
                                a.sh_inp, s.shared_gate, wg);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
@@ -129,7 +129,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
     const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
     float gu[2];
-    q8_row_wave<2>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
+    q8_row_wave<0, 2, false>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
         lds_quantize_q8_0(s.x, a.H, xq, xd, threadIdx.x, 512);
         __syncthreads();
     });
@@ -508,17 +508,17 @@ __global__ __launch_bounds__(1024) void k_tokens_c(TokenArgs ta) {
                     for (int q = 0; q < 8; ++q) p[q] = 0;
                 }
                 wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
-                float4 *dst = reinterpret_cast<float4 *>(&tile.pf[0][r4 * 136 + b * 8]);
+                float4 *dst = reinterpret_cast<float4 *>(&tile.pf[r4 * 136 + b * 8]);
                 dst[0] = make_float4(static_cast<float>(p[0]), static_cast<float>(p[1]), static_cast<float>(p[2]),
                                      static_cast<float>(p[3]));
                 dst[1] = make_float4(static_cast<float>(p[4]), static_cast<float>(p[5]), static_cast<float>(p[6]),
                                      static_cast<float>(p[7]));
-                tile.ds[0][lane] = ds;
+                tile.ds[lane] = ds;
                 wave_lds_fence();
                 float acc = 0.0f;
 #pragma unroll
                 for (int s = 0; s < 16; ++s)  // slots past the row's end hold zeros: fma(0, 0, acc) == acc
-                    acc = __builtin_fmaf(tile.ds[0][r4 * 16 + s], tile.pf[0][r4 * 136 + s * 8 + c], acc);
+                    acc = __builtin_fmaf(tile.ds[r4 * 16 + s], tile.pf[r4 * 136 + s * 8 + c], acc);
                 const float y = close_lanes8(acc);
                 if ((lane & 15) == 0) ybuf[(it_t[i] * (a.k + 1) + it_j[i]) * 8 + 4 * g + r4] = y;
             }
