@@ -58,3 +58,33 @@ def test_tensors_on_two_byte_boundaries(g, oracle, monkeypatch, H, F, k):
 
     monkeypatch.setattr(g, "dev", dev)
     check_layer(g, oracle, L, x)
+
+
+@pytest.mark.parametrize("H,F,E,k,gate,down,shared,T", [
+    (256, 32, 8, 2, Q8, Q8, False, 2),           # one block per lane row, one down block
+    (2048, 544, 24, 6, Q8, IQ4, True, 5),        # 64 gate blocks, an unpaired 17th down block
+    (2304, 768, 16, 4, IQ4, Q8, True, 8),        # 72 gate blocks: a second pass of eight; 24 down blocks
+    (1792, 512, 32, 5, IQ3, IQ4, False, 3),      # a pass of seven super-blocks
+    (2304, 640, 16, 3, IQ2, IQ4, True, 4),       # nine
+    (4096, 1056, 16, 3, IQ3, Q8, True, 7),       # sixteen, 33 down blocks
+    (3072, 1536, 16, 10, IQ4, IQ4, True, 2),     # 48 down blocks
+    (1024, 1568, 16, 2, IQ2, Q8, True, 6)])      # 49: the one-token dispatch per token
+def test_token_batch_shapes(g, oracle, H, F, E, k, gate, down, shared, T):
+    import ctypes as C
+
+    from warpdecode_amd import capi
+    L = synth.make_layer(H, F, E, k, gate, down, shared, seed=SEED, layer=H + T, router_sigma=1.0 / np.sqrt(H))
+    base = synth.rng_for(SEED, 64, H + T).normal(0, 1, H)
+    xs = np.stack([synth.rms_normed(synth.rng_for(SEED, 65, H + T, t), H) + base for t in range(T)]).astype(np.float32)
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    dx, out = g.dev(xs), g.empty((T, H), np.float32)
+    arr = (C.c_void_p * T)(*[s.h.value for s in scr])
+    capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, arr, 0, g.stream())
+    g.sync()
+    got = g.host(out)
+    for t in range(T):
+        want, d = oracle.moe_layer(L, xs[t])
+        assert np.array_equal(scr[t].get("ids", k, np.int32), d["ids"])
+        assert g.same_bits(got[t], want), t
+    for s in scr:
+        s.close()

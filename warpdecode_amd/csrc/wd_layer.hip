@@ -894,6 +894,43 @@ extern "C" int wd_moe_stack_f32(const wd_moe_layer *layers, int n_layers, float 
 }
 
 namespace {
+template <int TYPE, int FETCH>
+void launch_tokens_b_fetch(const TokenArgs &ta, int items, int cus, hipStream_t st) {
+    const int H = ta.common.H;
+    size_t lds = static_cast<size_t>(ta.T) * (H + sizeof(float) * (H / 256));
+    if (FETCH != 0) lds = ((lds + 15) & ~static_cast<size_t>(15)) + 8 * 2 * static_cast<size_t>(iq_cover_bytes<TYPE>(H / 256));
+    // persistent: as many workgroups as a compute unit holds walk the items
+    if (ta.T <= 4) k_tokens_b<TYPE, 4, FETCH><<<std::min(items, kTokensBPerCu<TYPE, 4, FETCH> * cus), 512, lds, st>>>(ta);
+    else k_tokens_b<TYPE, kMaxTokens, FETCH><<<std::min(items, kTokensBPerCu<TYPE, kMaxTokens, FETCH> * cus), 512, lds, st>>>(ta);
+}
+template <int TYPE>
+void launch_tokens_b(const wd_moe_layer *L, const TokenArgs &ta, int items, int cus, bool table, bool tables_aligned, hipStream_t st) {
+    const int H = L->hidden;
+    // rows of tensors that start on 16-byte boundaries: the aligned fetch, one item ahead
+    auto al16 = [](const void *p, size_t v) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && v % 16 == 0; };
+    const bool words = table ? tables_aligned
+                             : (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && L->slot_gate_bytes % 16 == 0
+                                                  : al16(L->gate, L->gate_stride) && al16(L->up, L->up_stride));
+    if (!words || H > 4096) launch_tokens_b_fetch<TYPE, 0>(ta, items, cus, st);
+    else if (H == 2048) launch_tokens_b_fetch<TYPE, 8>(ta, items, cus, st);
+    else if (H == 2560) launch_tokens_b_fetch<TYPE, 10>(ta, items, cus, st);
+    else if (H <= 2304) launch_tokens_b_fetch<TYPE, 1>(ta, items, cus, st);
+    else launch_tokens_b_fetch<TYPE, 2>(ta, items, cus, st);
+}
+template <int KIND, int PASSES>
+void launch_tokens_c(const TokenArgs &ta, hipStream_t st) {
+    constexpr int kWaves = kTokensCWaves<PASSES>;
+    const size_t lds = kWaves * static_cast<size_t>(layer_c8_wave_bytes<false>(ta.common.F)) + sizeof(float) * 8 * ta.T * (ta.common.k + 1);
+    k_tokens_c<KIND, PASSES><<<ta.common.H / 8, 64 * kWaves, lds, st>>>(ta);
+}
+template <int KIND>
+void launch_tokens_c(const TokenArgs &ta, hipStream_t st) {
+    const int F = ta.common.F;
+    if (F <= 512) launch_tokens_c<KIND, 2>(ta, st);
+    else if (F <= 768) launch_tokens_c<KIND, 3>(ta, st);
+    else if (F <= 1024) launch_tokens_c<KIND, 4>(ta, st);
+    else launch_tokens_c<KIND, 6>(ta, st);
+}
 // gu_table / down_table: null, or device tables of pointers ([entry][2] gate and up, [entry] down) that take the place of
 // the layer's routed tensors, the ids of the pass being entry numbers; tables_aligned: every pointer in them is 16-byte aligned.
 int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int tokens, wd_moe_scratch *const *scratch_per_token,
@@ -909,13 +946,14 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
     hipStream_t st = as_stream(stream);
     const int H = L->hidden, F = L->expert_ffn, k = L->top_k;
     SiteScope total_site(WD_SITE_TOKENS_TOTAL, st);
-    // the union pass over the gate/up tensors needs the IQ types; the multi-token down dispatch needs Q8_0 rows of at
-    // most 16 blocks (other down tensors take the one-token dispatch per token, on the activations the union pass left)
-    const bool union_path = !(flags & WD_MOE_STAGED) && consumes_q8k(L->gate_type) && tokens * k <= 128 &&
+    // the union pass takes every gate/up type (Q8_0 and IQ4_NL rows up to hidden 4096); down rows of more than 48 blocks take the
+    // one-token dispatch per token, on the activations the union pass left
+    const bool iq = consumes_q8k(L->gate_type);
+    const bool union_path = !(flags & WD_MOE_STAGED) && (iq || H <= 4096) && tokens * k <= 128 &&
                             scratch_per_token[0]->gup == nullptr &&
                             !(flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B | WD_MOE_ONLY_C | WD_MOE_DRY));
-    const bool down_tokens = L->down_type == WD_TYPE_Q8_0 && F <= 512;
-    if (gu_table) WD_REQUIRE(union_path, "multi-token pass on a pointer table: IQ3_S / IQ2_S gate and up tensors, at most 128 (token, expert) pairs, no staging flags");
+    const bool down_tokens = F <= 1536;
+    if (gu_table) WD_REQUIRE(union_path && iq, "multi-token pass on a pointer table: IQ3_S / IQ2_S gate and up tensors, at most 128 (token, expert) pairs, no staging flags");
     if (!union_path) {
         // same results, one pass per token (every pass reads its own experts)
         for (int t = 0; t < tokens; ++t)
@@ -943,66 +981,30 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         k_.accum = s->accum, k_.down_f32 = s->down_f32;
     }
     LayerArgs &a = ta.common;
-    a.n_router_wgs = ((a.preselected ? 0 : a.E) + (a.sh_inp ? 1 : 0) + 7) / 8;  // one router row per wave
+    const bool wide = H > 2048 && H <= 4096;  // two waves per router row
+    const int router_rows_n = (a.preselected ? 0 : a.E) + (a.sh_inp ? 1 : 0);
+    a.n_router_wgs = wide ? (router_rows_n + 3) / 4 : (router_rows_n + 7) / 8;
     const int grid_a = tokens_a_grid(a.n_router_wgs, a.sh_inp ? (F + 7) / 8 : 0).total(tokens);
     if (grid_a > 0) {  // router, selection and shared gate/up of every token
         SiteScope site(WD_SITE_TOKENS_A, st);
-        k_tokens_a<<<dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st>>>(ta);
+        if (wide) k_tokens_a<true><<<dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st>>>(ta);
+        else k_tokens_a<false><<<dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st>>>(ta);
         WD_LAUNCH_CHECK();
     }
-    const size_t lds_b = static_cast<size_t>(tokens) * (H + sizeof(float) * (H / 256));
     const int items_b = tokens * k * ((F + 7) / 8);
-    const int grid_b = items_b < 512 ? items_b : 512;  // persistent: two workgroups per compute unit walk the items
-    // rows of eight or ten super-blocks of aligned tensors: the aligned fetch, one item ahead
-    auto al16b = [](const void *p_, size_t v) { return reinterpret_cast<uintptr_t>(p_) % 16 == 0 && v % 16 == 0; };
-    const bool coal_b = (H == 2048 || H == 2560) &&
-                        (gu_table ? tables_aligned
-                                  : (L->slot_of_expert ? al16b(L->slot_pool, L->slot_bytes) && L->slot_gate_bytes % 16 == 0
-                                                       : al16b(L->gate, L->gate_stride) && al16b(L->up, L->up_stride)));
-    const size_t lds_b_coal = ((lds_b + 15) & ~static_cast<size_t>(15)) + 8 * 2 * static_cast<size_t>(H == 2048 ? kIqStageBytes : kIqStage10Bytes);
-    const dim3 gb(grid_b), bb(512);
-#define WD_TOKENS_B(TYPE_)                                                                              \
-    do {                                                                                                \
-        if (coal_b && H == 2048) {                                                                      \
-            if (tokens <= 4) k_tokens_b<TYPE_, 4, 8><<<gb, bb, lds_b_coal, st>>>(ta);                   \
-            else k_tokens_b<TYPE_, kMaxTokens, 8><<<gb, bb, lds_b_coal, st>>>(ta);                      \
-        } else if (coal_b) {                                                                            \
-            if (tokens <= 4) k_tokens_b<TYPE_, 4, 10><<<gb, bb, lds_b_coal, st>>>(ta);                  \
-            else k_tokens_b<TYPE_, kMaxTokens, 10><<<gb, bb, lds_b_coal, st>>>(ta);                     \
-        } else {                                                                                        \
-            if (tokens <= 4) k_tokens_b<TYPE_, 4><<<gb, bb, lds_b, st>>>(ta);                           \
-            else k_tokens_b<TYPE_, kMaxTokens><<<gb, bb, lds_b, st>>>(ta);                              \
-        }                                                                                               \
-    } while (0)
+    const int cus = scratch_per_token[0]->compute_units;
     {
         SiteScope site(WD_SITE_TOKENS_B, st);
-        if (L->gate_type == WD_TYPE_IQ3_S)
-            WD_TOKENS_B(21);
-        else
-            WD_TOKENS_B(22);
+        const size_t lds_q8 = static_cast<size_t>(tokens) * (H + H / 16);
+        switch (L->gate_type) {
+            case WD_TYPE_IQ3_S: launch_tokens_b<21>(L, ta, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
+            case WD_TYPE_IQ2_S: launch_tokens_b<22>(L, ta, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
+            case WD_TYPE_Q8_0: k_tokens_b_q8<0><<<std::min(items_b, 2 * cus), 512, lds_q8, st>>>(ta); break;
+            default: k_tokens_b_q8<1><<<std::min(items_b, 2 * cus), 512, lds_q8, st>>>(ta); break;
+        }
         WD_LAUNCH_CHECK();
     }
-#undef WD_TOKENS_B
-    // down tensors in aligned groups of four 16- or 20-block rows (either type): the dispatch with the aligned fetch
-    auto al16t = [](const void *p_, size_t v) { return reinterpret_cast<uintptr_t>(p_) % 16 == 0 && v % 16 == 0; };
-    const bool down_tokens_nb = (F == 512 || F == 640) && H % 8 == 0 && tokens <= 16 &&
-                                (!L->shared_down || al16t(L->shared_down, 0)) &&
-                                (down_table ? tables_aligned
-                                            : (L->slot_of_expert ? al16t(L->slot_pool, L->slot_bytes) && (L->slot_gate_bytes + L->slot_up_bytes) % 16 == 0
-                                                                 : al16t(L->down, L->down_stride)));
     SiteScope c_site(WD_SITE_TOKENS_C, st);
-    if (down_tokens_nb) {
-        const size_t per_wave_n = (static_cast<size_t>(F) + F / 16 + 15) & ~static_cast<size_t>(15);
-        const size_t lds_n = 16 * per_wave_n + sizeof(float) * 8 * tokens * (k + 1);
-        const dim3 grid(H / 8), block(1024);
-        const bool q8 = L->down_type == WD_TYPE_Q8_0;
-        if (F == 512 && !q8) k_tokens_c_nb<1, 16><<<grid, block, lds_n, st>>>(ta);
-        else if (F == 512) k_tokens_c_nb<0, 16><<<grid, block, lds_n, st>>>(ta);
-        else if (q8) k_tokens_c_nb<0, 20><<<grid, block, lds_n, st>>>(ta);
-        else k_tokens_c_nb<1, 20><<<grid, block, lds_n, st>>>(ta);
-        WD_LAUNCH_CHECK();
-        return WD_OK;
-    }
     if (!down_tokens) {
         WD_REQUIRE(!down_table, "multi-token pass on a pointer table: this down tensor (type %d, %d columns) has no multi-token dispatch", L->down_type, F);
         for (int t = 0; t < tokens; ++t)
@@ -1011,10 +1013,7 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
                 return rc;
         return WD_OK;
     }
-    const int waves_c = 16;
-    const size_t per_wave = (static_cast<size_t>(F) + F / 16 + 15) & ~static_cast<size_t>(15);
-    const size_t lds_c = waves_c * per_wave + sizeof(float) * 8 * tokens * (k + 1);
-    k_tokens_c<<<dim3((H + 7) / 8), dim3(64 * waves_c), lds_c, st>>>(ta);
+    L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c<0>(ta, st) : launch_tokens_c<1>(ta, st);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }

@@ -576,28 +576,23 @@ WD_DEV void iq_rows8_coal(const uint8_t *const (&rows)[NR], const IqTables &t, c
 }
 
 constexpr int kIqStage10Bytes = 1120;  // per row of ten super-blocks: the 70 words that cover 12 + 1100 bytes
-// The aligned fetch of one IQ row of NB = 8 or 10 super-blocks as a request and a store apart (for callers that keep a
-// row in flight while they work on another): the 16-byte words that cover the row (it is 16-byte aligned for NB = 8 and
-// 4-byte aligned for NB = 10), copied to a stage of kIqStageBytes / kIqStage10Bytes; the row then starts `lead` bytes
-// into the stage.
-template <int TYPE, int NB>
-struct IqRowFetch {
-    static constexpr int kBlk = (TYPE == 21) ? 110 : 82, kRow = NB * kBlk;
-    static constexpr bool kTwoLoads = 12 + kRow > 1024;
-    uint4 r0, r1;
+// The aligned fetch of one IQ row as a request and a store apart (for callers that keep a row in flight while they work on
+// another): the 16-byte words that cover it, at most 64 LOADS; the row then starts `lead` bytes into the stage.
+template <int TYPE, int LOADS>
+struct IqRowWords {
+    uint4 u[LOADS];
     uint32_t lead;
     int words;
-    WD_DEV void request(const uint8_t *row, int lane) {
+    WD_DEV void request(const uint8_t *row, int nb, int lane) {
         lead = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(row)) & 15u;  // the same in every lane
-        words = static_cast<int>((lead + kRow + 15) >> 4);
+        words = static_cast<int>((lead + nb * ((TYPE == 21) ? 110 : 82) + 15) >> 4);
         const uint8_t *base = row - lead;
-        r0 = gld_u128_aligned(base + 16 * min(lane, words - 1));
-        if (kTwoLoads) r1 = gld_u128_aligned(base + 16 * min(64 + lane, words - 1));
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) u[i] = gld_u128_aligned(base + 16 * min(64 * i + lane, words - 1));
     }
     WD_DEV void store(uint8_t *stage, int lane) const {  // lanes past the last word repeat it
-        uint4 *st = reinterpret_cast<uint4 *>(stage);
-        st[min(lane, words - 1)] = r0;
-        if (kTwoLoads) st[min(64 + lane, words - 1)] = r1;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) reinterpret_cast<uint4 *>(stage)[min(64 * i + lane, words - 1)] = u[i];
     }
 };
 
@@ -718,21 +713,12 @@ WD_DEV void iq_rows_cover(const uint8_t *const (&rows)[NR], int nb, const IqTabl
     const uint32_t stride = iq_cover_bytes<TYPE>(nb);
     uint32_t lead[NR];
     {
-        uint4 raw[NR][LOADS];
-        int words[NR];
+        IqRowWords<TYPE, LOADS> row[NR];
 #pragma unroll
-        for (int i = 0; i < NR; ++i) {
-            lead[i] = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(rows[i])) & 15u;  // the same in every lane
-            words[i] = static_cast<int>((lead[i] + nb * kBlk + 15) >> 4);
-            const uint8_t *base = rows[i] - lead[i];
-#pragma unroll
-            for (int q = 0; q < LOADS; ++q) raw[i][q] = gld_u128_aligned(base + 16 * min(64 * q + lane, words[i] - 1));
-        }
+        for (int i = 0; i < NR; ++i) row[i].request(rows[i], nb, lane), lead[i] = row[i].lead;
         pre();
 #pragma unroll
-        for (int i = 0; i < NR; ++i)  // lanes past the last word repeat it
-#pragma unroll
-            for (int q = 0; q < LOADS; ++q) reinterpret_cast<uint4 *>(stage + i * stride)[min(64 * q + lane, words[i] - 1)] = raw[i][q];
+        for (int i = 0; i < NR; ++i) row[i].store(stage + i * stride, lane);
     }
     wave_lds_fence();
     float acc[NR];

@@ -3,7 +3,7 @@
 // The reference batches M tokens as M*k (token, expert) pairs and re-reads an expert's weights for
 // every pair that names it (src/qwen38_moe.cuh:1316-1437, :2743-3237).  Here a pass is three dispatches:
 //   A  router, selection and shared gate/up of every token side by side (grid.y = token);
-//   B  routed gate/up + SwiGLU over the union of the selected experts: a weight row is decoded once and applied to
+//   B  routed gate/up + SwiGLU over the union of the selected experts: a weight row is fetched and decoded once and applied to
 //      the activation of every token that selected the expert;
 //   C  down projections over the union (a member's rows are loaded once and applied to the activations of its
 //      tokens) and the ordered combine per token.
@@ -64,6 +64,8 @@ struct TokensAGrid {
 __host__ __device__ inline TokensAGrid tokens_a_grid(int n_router_wgs, int n_shared_wgs) {
     return TokensAGrid{(n_router_wgs + 7) & ~7, (n_shared_wgs + 7) & ~7};
 }
+// WIDE: router rows of 2049..4096 columns, two waves each (n_router_wgs is then for four rows per workgroup).
+template <bool WIDE>
 __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     extern __shared__ __align__(16) uint8_t lds_ta[];
     __shared__ __align__(16) uint8_t s_work[sizeof(Q8RowTile) * 8];
@@ -87,8 +89,12 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     const TokenSlots &s = ta.tok[token];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wg < a.n_router_wgs) {
-        router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, a.preselected ? 0 : a.E, a.H,
-                               a.sh_inp, s.shared_gate, wg);
+        const int rows = a.preselected ? 0 : a.E;
+        if (WIDE)
+            router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.logits, rows, a.H,
+                                  a.sh_inp, s.shared_gate, wg);
+        else
+            router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, rows, a.H, a.sh_inp, s.shared_gate, wg);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
         __syncthreads();
@@ -129,7 +135,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
     const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
     float gu[2];
-    q8_row_wave<0, 2, false>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
+    q8_row_wave<0, 2, WIDE>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
         lds_quantize_q8_0(s.x, a.H, xq, xd, threadIdx.x, 512);
         __syncthreads();
     });
@@ -210,11 +216,14 @@ WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
 // the item, decodes it once and applies it to every token that selected the expert.
 // MAXT: token capacity of the instantiation (4 or kMaxTokens).
 // dynamic LDS: T * (H bytes + H/256 floats): the Q8_K copies of the T inputs.
-// NB: 0, or the super-blocks per row (8 or 10) when the rows can be fetched as aligned words (IqRowFetch): the row pair of
-// the wave's next item is then requested before the current one is worked on.  dynamic LDS then has
-// 8 * 2 * (kIqStageBytes or kIqStage10Bytes) more bytes behind the activations (16-byte aligned).
-template <int TYPE, int MAXT, int NB = 0>
-__global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
+// FETCH: 0, or how the rows come in when they can be fetched as aligned words (IqRowWords): 8 and 10 rows of that many
+// super-blocks, 1 and 2 others of one or two words per lane.  The row pair of the wave's next item is then requested before the
+// current one is worked on.  dynamic LDS then has 8 * 2 * iq_cover_bytes more bytes behind the activations (16-byte aligned).
+// As many workgroups per compute unit as the registers allow without spilling.
+template <int TYPE, int MAXT, int FETCH>
+constexpr int kTokensBPerCu = FETCH == 8 || (FETCH == 10 && TYPE == 22 && MAXT <= 4) ? 3 : 2;
+template <int TYPE, int MAXT, int FETCH = 0>
+__global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k_tokens_b(TokenArgs ta) {
     extern __shared__ __align__(16) uint8_t lds_tb[];
     __shared__ IqTables tables;
     __shared__ TokenUnion un;
@@ -224,7 +233,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
     int8_t *xq = reinterpret_cast<int8_t *>(lds_tb);
     float *xd = reinterpret_cast<float *>(lds_tb + static_cast<size_t>(ta.T) * a.H);
     constexpr int kBlk = (TYPE == 21) ? 110 : 82;
-    const int nb = a.H >> 8;
+    const int nb = FETCH >= 8 ? FETCH : a.H >> 8;
     const size_t rb = static_cast<size_t>(nb) * kBlk;
     mark(a, 1, 0);
     // the T inputs as Q8_K: a wave's blocks (wave, wave + 8, ...) are requested four at a time, the first four before
@@ -261,27 +270,26 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
     __syncthreads();
     mark(a, 1, 2);
     const int n_items = un.count * groups;
-    // rows of eight super-blocks are one pass: the lane layout of iq_rows8_coal_dots then (a chain's lanes two apart inside
-    // a row, no carry between passes, no lane excluded from a chain step)
-    // (NB == 10: the same layout for super-blocks 0..7, and super-blocks 8 and 9 of both rows in one shared pass, as in
-    // iq_rows10_coal)
-    constexpr bool kPairs = NB == 8 || NB == 10;
+    // the aligned forms use the lane layout of iq_rows8_coal_dots (a chain's lanes two apart inside a row, no lane excluded from
+    // a chain step), rows of ten super-blocks with the last two of both rows in one shared pass, as in iq_rows10_coal
+    constexpr bool kPairs = FETCH != 0;
+    constexpr int kLoads = FETCH == 2 || (FETCH == 10 && TYPE == 21) ? 2 : 1;
     const int ib = kPairs ? ((lane >> 4) << 1) | (lane & 1) : lane >> 3, sbl = kPairs ? (lane >> 1) & 7 : lane & 7;
     const bool first = sbl == 0;
-    constexpr int kStage = (NB == 10) ? kIqStage10Bytes : kIqStageBytes;
+    const uint32_t kStage = iq_cover_bytes<TYPE>(nb);
     uint8_t *stage = lds_tb + ((static_cast<size_t>(ta.T) * (a.H + sizeof(float) * nb) + 15) & ~static_cast<size_t>(15)) +
                      static_cast<size_t>(wave) * 2 * kStage;
-    IqRowFetch<TYPE, NB == 0 ? 8 : NB> fetch[2];
+    IqRowWords<TYPE, kLoads> fetch[2];
     auto row_pair = [&](int item, const uint8_t *(&rows)[2]) {
         const int u = item / groups, rg = item - u * groups;
         const int e = un.expert[u];
         const size_t off = static_cast<size_t>(min(rg * 8 + wave, a.F - 1)) * rb;
         rows[0] = uniform_ptr(mat_ptr_entry<0>(a.gate_up, e) + off), rows[1] = uniform_ptr(mat_ptr_entry<1>(a.gate_up, e) + off);
     };
-    if (NB != 0 && static_cast<int>(blockIdx.x) < n_items) {
+    if (FETCH != 0 && static_cast<int>(blockIdx.x) < n_items) {
         const uint8_t *rows[2];
         row_pair(blockIdx.x, rows);
-        fetch[0].request(rows[0], lane), fetch[1].request(rows[1], lane);
+        fetch[0].request(rows[0], nb, lane), fetch[1].request(rows[1], nb, lane);
     }
     for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
         const int u = item / groups, rg = item - u * groups;
@@ -292,7 +300,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
         const uint8_t *rows[2];  // one row pair per wave
         row_pair(item, rows);
         uint32_t lead[2] = {0, 0};
-        if (NB != 0) {
+        if (FETCH != 0) {
             wave_lds_fence();  // the previous item's rows have been read
             fetch[0].store(stage, lane), fetch[1].store(stage + kStage, lane);
             lead[0] = fetch[0].lead, lead[1] = fetch[1].lead;
@@ -300,23 +308,25 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
             if (item + static_cast<int>(gridDim.x) < n_items) {  // the next item's rows, into the registers just written out
                 const uint8_t *next[2];
                 row_pair(item + gridDim.x, next);
-                fetch[0].request(next[0], lane), fetch[1].request(next[1], lane);
+                fetch[0].request(next[0], nb, lane), fetch[1].request(next[1], nb, lane);
             }
         }
         float acc[MAXT][2];
 #pragma unroll
         for (int t = 0; t < MAXT; ++t) acc[t][0] = acc[t][1] = 0.0f;
-        for (int base = 0; base < (NB == 10 ? 8 : nb); base += 8) {
-            const int sb = base + sbl;
-            const bool on = sb < nb;
+        for (int base = 0; base < (FETCH == 10 ? 8 : nb); base += 8) {
+            // (aligned forms: positions past the row's end work on its last super-block and contribute zero)
+            const bool in_row = FETCH >= 8 || base + sbl < nb, on = kPairs || in_row;
+            const int sb = FETCH >= 8 ? base + sbl : min(base + sbl, nb - 1);
             uint32_t w[2][8];
             int ls[2][2];
             float dw[2] = {0.0f, 0.0f};
             if (on) {
                 IqFields f[2];
-                if (NB != 0) {
-                    f[0] = iq_fields_lds<TYPE>(stage + lead[0] + sb * kBlk, ib, sb);
-                    f[1] = iq_fields_lds<TYPE>(stage + kStage + lead[1] + sb * kBlk, ib, sb);
+                if (FETCH != 0) {
+                    const uint32_t o0 = lead[0] + sb * kBlk, o1 = lead[1] + sb * kBlk;
+                    f[0] = iq_fields_shifted<TYPE>(stage + o0, ib, (o0 + 2) & 2u);
+                    f[1] = iq_fields_shifted<TYPE>(stage + kStage + o1, ib, (o1 + 2) & 2u);
                 } else {
                     f[0] = iq_load<TYPE>(rows[0] + static_cast<size_t>(sb) * kBlk, ib);
                     f[1] = iq_load<TYPE>(rows[1] + static_cast<size_t>(sb) * kBlk, ib);
@@ -337,7 +347,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
                     const uint4 a0 = *reinterpret_cast<const uint4 *>(aq);
                     const uint4 a1 = *reinterpret_cast<const uint4 *>(aq + 16);
                     av[0] = a0.x, av[1] = a0.y, av[2] = a0.z, av[3] = a0.w, av[4] = a1.x, av[5] = a1.y, av[6] = a1.z, av[7] = a1.w;
-                    dx = xd[t * nb + sb];
+                    dx = in_row ? xd[t * nb + sb] : 0.0f;
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
@@ -352,9 +362,15 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
                     }
                     if (kPairs) {
                         const float pf = static_cast<float>(reduce_scatter_ib_pairs(p, lane));
-                        float v = __builtin_fmaf(ds, pf, 0.0f);
+                        // the chain's value of the pass before moves to the first position, which keeps it while the others
+                        // converge; past the row's end it passes through, fma(0, finite, acc) == acc
+                        float up = FETCH >= 8 || base == 0 ? 0.0f : dpp_f<kDppShl14>(0.0f, acc[t][i]);
+                        float v = __builtin_fmaf(ds, pf, up);
 #pragma unroll
-                        for (int s = 1; s < 8; ++s) v = __builtin_fmaf(ds, pf, dpp_f<kDppShr2, 0xf, 0xf, true>(0.0f, v));
+                        for (int s = 1; s < 8; ++s) {
+                            up = FETCH >= 8 ? dpp_f<kDppShr2, 0xf, 0xf, true>(0.0f, v) : dpp_f<kDppShr2>(up, v);
+                            v = __builtin_fmaf(ds, pf, up);
+                        }
                         acc[t][i] = v;
                         continue;
                     }
@@ -371,7 +387,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
                 }
             }
         }
-        if (NB == 10) {
+        if (FETCH == 10) {
             // super-blocks 8 and 9: position 0/1 of the pass = row 0, position 2/3 = row 1 (positions 4..7 idle)
             const int ri = min(sbl >> 1, 1), sb = 8 + (sbl & 1);
             const bool on = sbl < 4;
@@ -416,114 +432,132 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b(TokenArgs ta) {
     mark(a, 1, 5);
 }
 
-// ---- dispatch C for T tokens ----------------------------------------------------------------------------
-// grid = ceil(H / 8), 1024 threads: a workgroup owns eight output rows (two groups of four).  Work items are
-// (token, matrix) with matrix = the token's k routed down tensors, then the shared one; wave w takes items w,
-// w + 16, w + 32 of a round of 48: it requests the activations and (as soon as the ids are in) the eight rows of all
-// its items together (F <= 512: one block per lane and row group), then quantises each item's activation once and
-// runs the one-token row code on both row groups.  Items that name the same expert read the same rows within one
-// workgroup, so memory sees them once.  Waves 0..T-1 finally fold token t's results in its own top-k order.
-// dynamic LDS: per wave F bytes + F/32 halves (+pad), then [T][k+1][8] floats.
-__global__ __launch_bounds__(1024) void k_tokens_c(TokenArgs ta) {
-    extern __shared__ __align__(16) uint8_t lds_tc[];
-    __shared__ Q8Tile tiles[16];
+// The same for Q8_0 (KIND 0) and IQ4_NL (KIND 1) gate/up rows.  The waves of the grid take the items (union member, group of
+// four rows) in turn: four gate rows and the same four up rows are the eight rows of q8_rows8_pass, 32 blocks of each in
+// registers at a time and applied to every token that selected the expert.
+// (One row pair per wave with a block per lane runs the chains of two rows on all 64 lanes, 64 steps each, for every token: 61 us
+// for eight tokens, top-5, hidden 3584, ffn 512, against 30.)
+// dynamic LDS: T * (H bytes + H/32 halves), the Q8_0 copies of the T inputs.
+template <int KIND>
+__global__ __launch_bounds__(512, 4) void k_tokens_b_q8(TokenArgs ta) {
+    extern __shared__ __align__(16) uint8_t lds_tq[];
+    __shared__ Q8Tile8 tiles[8];
+    __shared__ TokenUnion un;
     const LayerArgs &a = ta.common;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    constexpr int kWaves = 16, kItems = 3;
-    const size_t per_wave = (static_cast<size_t>(a.F) + a.F / 16 + 15) & ~static_cast<size_t>(15);
-    int8_t *aq = reinterpret_cast<int8_t *>(lds_tc + wave * per_wave);
-    uint16_t *ad = reinterpret_cast<uint16_t *>(lds_tc + wave * per_wave + a.F);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int groups = a.F >> 2, nb = a.H >> 5;  // (F is a multiple of 32, H of 256)
+    constexpr int kBlk = (KIND == 0) ? 34 : 18, kChunk = 4;  // passes of eight blocks
+    const size_t rb = static_cast<size_t>(nb) * kBlk;
+    int8_t *xq = reinterpret_cast<int8_t *>(lds_tq);
+    uint16_t *xd = reinterpret_cast<uint16_t *>(lds_tq + static_cast<size_t>(ta.T) * a.H);
+    if (wave == 0) token_union_build(ta, un, lane);
+    for (int t = 0; t < ta.T; ++t) lds_quantize_q8_0(ta.tok[t].x, a.H, xq + static_cast<size_t>(t) * a.H, xd + t * nb, threadIdx.x, 512);
+    __syncthreads();
+    const int n_items = un.count * groups, row = lane >> 3, b = lane & 7;
+    // (neighbouring workgroups take neighbouring items, a workgroup's waves items far apart: every wave of the grid gets one
+    // before any gets a second)
+    for (int item = wave * static_cast<int>(gridDim.x) + static_cast<int>(blockIdx.x); item < n_items; item += 8 * static_cast<int>(gridDim.x)) {
+        const int u = item / groups, r0 = 4 * (item - u * groups);
+        const int e = __builtin_amdgcn_readfirstlane(un.expert[u]);
+        const uint8_t *const gate = mat_ptr_entry<0>(a.gate_up, e), *const up = mat_ptr_entry<1>(a.gate_up, e);
+        const uint8_t *const mine = (row < 4 ? gate : up) + static_cast<size_t>(r0 + (row & 3)) * rb;
+        int rank[kMaxTokens];
+#pragma unroll
+        for (int t = 0; t < kMaxTokens; ++t) rank[t] = __builtin_amdgcn_readfirstlane(static_cast<int>(un.rank[u][t]));
+        Q8Chain ch[kMaxTokens];
+        for (int base = 0; base < nb; base += 8 * kChunk) {
+            Q8Block w[kChunk];
+#pragma unroll
+            for (int q = 0; q < kChunk; ++q) w[q] = q8_load<KIND>(mine + static_cast<size_t>(min(base + 8 * q + b, nb - 1)) * kBlk);
+#pragma unroll
+            for (int t = 0; t < kMaxTokens; ++t) {
+                if (rank[t] < 0) continue;  // uniform
+#pragma unroll
+                for (int q = 0; q < kChunk; ++q)
+                    if (base + 8 * q < nb)
+                        q8_rows8_pass<KIND, false>(w[q], base + 8 * q, nb, xq + static_cast<size_t>(t) * a.H, xd + t * nb, tiles[wave], lane, ch[t], nullptr);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < kMaxTokens; ++t) {
+            if (rank[t] < 0) continue;
+            const float y = q8_rows8_close<KIND>(ch[t], nb, tiles[wave], lane);
+            const wd_uint2v h = __builtin_amdgcn_permlane32_swap(f_bits(y), f_bits(y), false, false);  // .y in lanes 0..31: the value 32 lanes up
+            if (b == 0 && row < 4) ta.tok[t].act[static_cast<size_t>(rank[t]) * a.F + r0 + row] = silu_ggml(y) * bits_f(h.y);
+        }
+    }
+}
+
+// ---- dispatch C for T tokens ----------------------------------------------------------------------------
+// grid = H / 8: a workgroup owns eight output rows, as the one-token k_layer_c8 does.  Work items are (token, matrix) with
+// matrix = the token's k routed down tensors, then the shared one (always Q8_0); the waves take them in turn: the
+// activation, then the eight rows, one block per lane and pass.  Items that name the same expert read the same rows within one
+// workgroup, so memory sees them once.  Waves 0..T-1 finally fold token t's results in its own top-k order.
+// One item in flight per wave and as many waves as the registers allow - two workgroups of sixteen waves per compute unit for
+// rows of 16 blocks, two of eight for longer ones -, so that grids of more than 256 workgroups (hidden > 2048) still run in one round: with two
+// or three items per wave and one workgroup of sixteen waves per compute unit, hidden 2304 took twice the time of 2048.
+// KIND: down tensor kind; PASSES: of eight blocks per row (F <= 256 PASSES).
+// dynamic LDS: per wave the tile and the quantised activation (layer_c8_wave_bytes<false>), then [T][k+1][8] floats.
+template <int PASSES>
+constexpr int kTokensCWaves = PASSES <= 2 ? 16 : 8;
+template <int KIND, int PASSES>
+__global__ __launch_bounds__(64 * kTokensCWaves<PASSES>) __attribute__((amdgpu_waves_per_eu(PASSES <= 2 ? 8 : (PASSES == 3 ? 5 : 4))))
+void k_tokens_c(TokenArgs ta) {
+    extern __shared__ __align__(16) uint8_t lds_tc[];
+    const LayerArgs &a = ta.common;
+    const int lane = threadIdx.x & 63, tw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    constexpr int kWaves = kTokensCWaves<PASSES>, kActs = (PASSES + 1) / 2;
+    const uint32_t per_wave = layer_c8_wave_bytes<false>(a.F);
+    Q8Tile8 &tile = *reinterpret_cast<Q8Tile8 *>(lds_tc + tw * per_wave);
+    int8_t *aq = reinterpret_cast<int8_t *>(lds_tc + tw * per_wave + sizeof(Q8Tile8));
+    uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
     float *ybuf = reinterpret_cast<float *>(lds_tc + kWaves * per_wave);  // [T][k+1][8]
     const bool shared = a.sh_down != nullptr;
-    const int per_token = a.k + (shared ? 1 : 0);
-    const int n_items = ta.T * per_token;
-    const int r0 = blockIdx.x * 8;
-    const int nb = a.F >> 5;  // <= 16
-    const int r4 = lane >> 4, b = lane & 15, c = lane & 7;
-    const bool act_on = lane * 8 < a.F;
+    const int per_token = a.k + (shared ? 1 : 0), n_items = ta.T * per_token;
+    const int r0 = blockIdx.x * 8, nb = a.F >> 5;  // hidden is a multiple of 8
     mark(a, 2, 0);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
     const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
-    // combine operands of token `wave`, requested early: lane j keeps router weight j, lane 16 the shared gate
-    const int tw = __builtin_amdgcn_readfirstlane(wave);  // uniform index into the argument block
+    // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
     float wreg;
     {
         const TokenSlots &s = ta.tok[min(tw, ta.T - 1)];
         const float *src = (lane == 16 && shared) ? s.shared_gate : s.weights + min(lane, a.k - 1);
         wreg = *src;
     }
-    Q8Tile &tile = tiles[wave];
-    for (int item0 = 0; item0 < n_items; item0 += kWaves * kItems) {
-        int it_t[kItems], it_j[kItems];
-        bool it_on[kItems];
-        float4 v0[kItems], v1[kItems];
-        Q8Block wb[kItems][2];
+    for (int item = tw; item < n_items; item += kWaves) {
+        const int t = item / per_token, j = item - t * per_token;
+        const bool is_shared = j == a.k;
+        float4 v[2 * kActs];
 #pragma unroll
-        for (int i = 0; i < kItems; ++i) {  // unconditional loads: an item past the end repeats the last one
-            const int item = item0 + tw + kWaves * i;
-            it_on[i] = item < n_items;
-            const int ic = min(item, n_items - 1);
-            it_t[i] = ic / per_token, it_j[i] = ic - it_t[i] * per_token;
-            const float *act = ta.tok[it_t[i]].act + static_cast<size_t>(it_j[i]) * a.F + min(lane * 8, a.F - 8);
-            v0[i] = *reinterpret_cast<const float4 *>(act);
-            v1[i] = *reinterpret_cast<const float4 *>(act + 4);
+        for (int q = 0; q < kActs; ++q) {
+            const float *p = ta.tok[t].act + static_cast<size_t>(j) * a.F + min(512 * q + lane * 8, a.F - 8);
+            v[2 * q] = *reinterpret_cast<const float4 *>(p), v[2 * q + 1] = *reinterpret_cast<const float4 *>(p + 4);
         }
-#pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            const bool is_shared = it_j[i] == a.k;
-            const int pair = it_t[i] * a.k + (is_shared ? 0 : it_j[i]);
-            const int e = pair < 64 ? __builtin_amdgcn_readlane(id_lo, pair) : __builtin_amdgcn_readlane(id_hi, pair - 64);
-            const uint8_t *w = is_shared ? a.sh_down : mat_ptr_entry<0>(a.down, e);
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const int row = min(r0 + 4 * g + r4, a.H - 1);
-                wb[i][g] = q8_load<0>(w + (static_cast<size_t>(row) * nb + min(b, nb - 1)) * 34);
-            }
-        }
-        mark(a, 2, 1);
-#pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            if (!it_on[i]) continue;  // uniform
+        const int pair = t * a.k + (is_shared ? 0 : j);
+        const int e = pair < 64 ? __builtin_amdgcn_readlane(id_lo, pair) : __builtin_amdgcn_readlane(id_hi, pair - 64);
+        const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_entry<0>(a.down, e)) + static_cast<size_t>(r0) * nb * (KIND == 0 || is_shared ? 34 : 18));
+        auto run = [&](auto kind) {
+            constexpr int K = decltype(kind)::value;
+            Q8Rows8Blocks<K, PASSES> blocks;
+            // (the longest rows leave no registers to hold the activation beside the blocks: quantised ahead of their request)
+            constexpr bool kActFirst = PASSES > 4;
+            if (!kActFirst) blocks.request(rows, nb, lane);
             wave_lds_fence();
-            lds_quantize_q8_0_step(v0[i], v1[i], act_on, lane * 8, aq, ad, lane);
+#pragma unroll
+            for (int q = 0; q < kActs; ++q)
+                lds_quantize_q8_0_step(v[2 * q], v[2 * q + 1], 512 * q + lane * 8 < a.F, 512 * q + lane * 8, aq, ad, lane);
             wave_lds_fence();
-            uint32_t av[8];
-            float dxa = 0.0f;
-            if (b < nb) {
-                const uint4 a0 = *reinterpret_cast<const uint4 *>(aq + b * 32);
-                const uint4 a1 = *reinterpret_cast<const uint4 *>(aq + b * 32 + 16);
-                av[0] = a0.x, av[1] = a0.y, av[2] = a0.z, av[3] = a0.w, av[4] = a1.x, av[5] = a1.y, av[6] = a1.z, av[7] = a1.w;
-                dxa = h2f(ad[b]);
-            }
+            if (kActFirst) blocks.request(rows, nb, lane);
+            Q8Chain ch;
 #pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                const bool on = r0 + 4 * g + r4 < a.H && b < nb;
-                int p[8];
-                float ds = 0.0f;
-                if (on) {
-                    q8_chunks<0>(wb[i][g], av, p);
-                    ds = h2f(wb[i][g].d) * dxa;
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) p[q] = 0;
-                }
-                wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
-                float4 *dst = reinterpret_cast<float4 *>(&tile.pf[r4 * 136 + b * 8]);
-                dst[0] = make_float4(static_cast<float>(p[0]), static_cast<float>(p[1]), static_cast<float>(p[2]),
-                                     static_cast<float>(p[3]));
-                dst[1] = make_float4(static_cast<float>(p[4]), static_cast<float>(p[5]), static_cast<float>(p[6]),
-                                     static_cast<float>(p[7]));
-                tile.ds[lane] = ds;
-                wave_lds_fence();
-                float acc = 0.0f;
-#pragma unroll
-                for (int s = 0; s < 16; ++s)  // slots past the row's end hold zeros: fma(0, 0, acc) == acc
-                    acc = __builtin_fmaf(tile.ds[r4 * 16 + s], tile.pf[r4 * 136 + s * 8 + c], acc);
-                const float y = close_lanes8(acc);
-                if ((lane & 15) == 0) ybuf[(it_t[i] * (a.k + 1) + it_j[i]) * 8 + 4 * g + r4] = y;
-            }
-            mark(a, 2, 2 + i);
-        }
+            for (int q = 0; q < PASSES; ++q)
+                if (8 * q < nb) q8_rows8_pass<K, false>(blocks.w[q], 8 * q, nb, aq, ad, tile, lane, ch, nullptr);
+            return q8_rows8_close<K>(ch, nb, tile, lane);
+        };
+        const float y = (KIND == 0 || is_shared) ? run(std::integral_constant<int, 0>{}) : run(std::integral_constant<int, KIND>{});
+        if ((lane & 7) == 0) ybuf[(t * (a.k + 1) + j) * 8 + (lane >> 3)] = y;
+        mark(a, 2, item == tw ? 2 : 3);
     }
     __syncthreads();
     mark(a, 2, 5);
@@ -554,129 +588,6 @@ __global__ __launch_bounds__(1024) void k_tokens_c(TokenArgs ta) {
         }
     }
     mark(a, 2, 6);
-}
-
-// The same for IQ4_NL (KIND 1) or Q8_0 (KIND 0) rows of NB = 16 or 20 blocks in 16-byte aligned groups of four, fetched as
-// aligned words (q8_rows4_coal): preferred over k_tokens_c where both apply (aligned Q8_0 rows of 16 blocks).  Eight rows per workgroup, 16 waves, an
-// item is (token, matrix) with the shared expert (always Q8_0) as matrix k; a wave has the two row groups of two items
-// in flight.  dynamic LDS per wave: F bytes + F/32 halves (+ pad), then [T][k+1][8] floats.
-template <int KIND, int NB>
-__global__ __launch_bounds__(1024) void k_tokens_c_nb(TokenArgs ta) {
-    extern __shared__ __align__(16) uint8_t lds_tn[];
-    __shared__ Q8TileNB<NB> tiles[16];
-    const LayerArgs &a = ta.common;
-    const int lane = threadIdx.x & 63;
-    constexpr int kWaves = 16, kItems = 2, kF = NB * 32;
-    using RawQ8 = Q8CoalRaw<0, NB>;
-    using RawW = Q8CoalRaw<KIND, NB>;
-    const int tw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const size_t per_wave = (static_cast<size_t>(kF) + kF / 16 + 15) & ~static_cast<size_t>(15);
-    int8_t *aq = reinterpret_cast<int8_t *>(lds_tn + tw * per_wave);
-    uint16_t *ad = reinterpret_cast<uint16_t *>(lds_tn + tw * per_wave + kF);
-    float *ybuf = reinterpret_cast<float *>(lds_tn + kWaves * per_wave);  // [T][k+1][8]
-    const bool shared = a.sh_down != nullptr;
-    const int per_token = a.k + (shared ? 1 : 0);
-    const int n_items = ta.T * per_token;
-    const int r0 = blockIdx.x * 8;  // hidden is a multiple of 8
-    const int r4 = lane >> 4;
-    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
-    float wreg;
-    {
-        const TokenSlots &s = ta.tok[min(tw, ta.T - 1)];
-        const float *src = (lane == 16 && shared) ? s.shared_gate : s.weights + min(lane, a.k - 1);
-        wreg = *src;
-    }
-    Q8TileNB<NB> &tile = tiles[tw];
-    for (int item0 = 0; item0 < n_items; item0 += kWaves * kItems) {
-        int it_t[kItems], it_j[kItems];
-        bool it_on[kItems];
-        float4 v0[kItems], v1[kItems], v2[kItems], v3[kItems];
-        uint4 raw[kItems][2][RawQ8::kLoads];
-#pragma unroll
-        for (int i = 0; i < kItems; ++i) {  // unconditional loads: an item past the end repeats the last one
-            const int item = item0 + tw + kWaves * i;
-            it_on[i] = item < n_items;
-            const int ic = min(item, n_items - 1);
-            it_t[i] = ic / per_token, it_j[i] = ic - it_t[i] * per_token;
-            const float *act = ta.tok[it_t[i]].act + static_cast<size_t>(it_j[i]) * kF;
-            v0[i] = *reinterpret_cast<const float4 *>(act + lane * 8);
-            v1[i] = *reinterpret_cast<const float4 *>(act + lane * 8 + 4);
-            if (NB == 20) {  // values 512..639: lanes 0..15 (the others repeat them)
-                v2[i] = *reinterpret_cast<const float4 *>(act + 512 + (lane & 15) * 8);
-                v3[i] = *reinterpret_cast<const float4 *>(act + 512 + (lane & 15) * 8 + 4);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            const bool is_shared = it_j[i] == a.k;
-            const int pair = it_t[i] * a.k + (is_shared ? 0 : it_j[i]);
-            const int e = pair < 64 ? __builtin_amdgcn_readlane(id_lo, pair) : __builtin_amdgcn_readlane(id_hi, pair - 64);
-            const uint8_t *w = is_shared ? a.sh_down : mat_ptr_entry<0>(a.down, e);
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                if (KIND == 0 || is_shared) {  // wave-uniform
-                    const RawQ8 r = q8_rows4_coal_request<0, NB>(w + static_cast<size_t>(r0 + 4 * g) * NB * 34, lane);
-#pragma unroll
-                    for (int q = 0; q < RawQ8::kLoads; ++q) raw[i][g][q] = r.u[q];
-                } else {
-                    const RawW r = q8_rows4_coal_request<KIND, NB>(w + static_cast<size_t>(r0 + 4 * g) * NB * RawW::kBlk, lane);
-#pragma unroll
-                    for (int q = 0; q < RawW::kLoads; ++q) raw[i][g][q] = r.u[q];
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kItems; ++i) {
-            if (!it_on[i]) continue;  // uniform
-            const bool is_shared = it_j[i] == a.k;
-            wave_lds_fence();
-            lds_quantize_q8_0_step(v0[i], v1[i], true, lane * 8, aq, ad, lane);
-            if (NB == 20) lds_quantize_q8_0_step(v2[i], v3[i], lane < 16, 512 + (lane & 15) * 8, aq, ad, lane);
-            wave_lds_fence();
-#pragma unroll
-            for (int g = 0; g < 2; ++g) {
-                float y;
-                if (KIND == 0 || is_shared) {
-                    RawQ8 r;
-#pragma unroll
-                    for (int q = 0; q < RawQ8::kLoads; ++q) r.u[q] = raw[i][g][q];
-                    y = q8_rows4_coal_finish<0, NB>(r, aq, ad, tile, lane);
-                } else {
-                    RawW r;
-#pragma unroll
-                    for (int q = 0; q < RawW::kLoads; ++q) r.u[q] = raw[i][g][q];
-                    y = q8_rows4_coal_finish<KIND, NB>(r, aq, ad, tile, lane);
-                }
-                if ((lane & 15) == 0) ybuf[(it_t[i] * (a.k + 1) + it_j[i]) * 8 + 4 * g + r4] = y;
-            }
-        }
-    }
-    __syncthreads();
-    if (tw < ta.T) {
-        const TokenSlots &s = ta.tok[tw];
-        const int row = r0 + lane;
-        const bool row_on = lane < 8;
-        float acc = 0.0f;
-        for (int j = 0; j < a.k; ++j) {
-            const float wj = lane_get(wreg, j);
-            const float y = ybuf[(tw * (a.k + 1) + j) * 8 + (lane & 7)];
-            const float prod = y * wj;
-            acc = acc + prod;
-            if (s.expert_out && row_on) s.expert_out[static_cast<size_t>(j) * a.H + row] = y;
-        }
-        const float gate = lane_get(wreg, 16);
-        if (row_on) {
-            float o = acc;
-            if (shared) {
-                const float y = ybuf[(tw * (a.k + 1) + a.k) * 8 + lane];
-                const float prod = y * gate;
-                o = acc + prod;
-                s.down_f32[row] = y;
-            }
-            s.accum[row] = acc;
-            s.out[row] = o;
-        }
-    }
 }
 
 }  // namespace wd
