@@ -219,6 +219,59 @@ def test_q8_0_gemv_misaligned_base(g, oracle):
     assert g.same_bits(g.host(out), want) and g.same_bits(g.host(out_s), want)
 
 
+# Rows around the chunks of 16, 32 and 64 blocks (a last chunk that repeats all but one of its blocks, none, or half), the
+# changes between the split kernels (5 and 8 chunks of 32, 257 groups), to the unsplit one (1024 groups) and to the general
+# kernel (fewer than 16 blocks, 17..21 with many rows, more than 512), IQ4_NL's unpaired last block in each
+RAGGED_SHAPES = [(9, 480), (8, 512), (9, 544), (8193, 544), (8193, 704), (17, 992), (8203, 1024), (64, 1056), (1003, 1504), (24, 2016),
+                 (8190, 2080), (8200, 2080), (40, 2592), (31, 4128), (10, 5152), (2049, 8160), (2060, 8192), (9, 8224), (8, 16352), (12, 16416)]
+
+
+@pytest.mark.parametrize("shift", [0, 2, 14])
+@pytest.mark.parametrize("t", [synth.Q8_0, synth.IQ4_NL])
+def test_gemv_ragged_rows(g, oracle, t, shift):
+    """The same bits as the oracle for any row length, from any two-byte boundary; nothing next to the outputs is written."""
+    import torch
+    for rows, cols in RAGGED_SHAPES:
+        rng = synth.rng_for(SEED, 41, t, rows, cols)
+        w = synth.matrix(t, rng, rows, cols)
+        qs, d = oracle.quantize_q8_0(rng.normal(0, 1, cols).astype(np.float32))
+        raw = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda")
+        raw[shift:shift + w.size] = torch.from_numpy(w.reshape(-1)).cuda()
+        dq, dd = g.dev(qs), g.dev(d)
+        out = torch.full((rows + 8,), 7.0, dtype=torch.float32, device="cuda")
+        out2, part = torch.full_like(out, 7.0), g.empty((rows, oracle.partials_per_row(t, cols)), np.int32)
+        for o, p in ((out, None), (out2, g.ptr(part))):
+            capi.call("wd_gemv_q8_0_f32", t, C.c_void_p(raw.data_ptr() + shift), rows, cols, g.ptr(dq), g.ptr(dd), g.ptr(o), p, g.stream())
+        g.sync()
+        want, wpart = oracle.gemv(t, w, rows, cols, qs, d, want_partials=True)
+        assert np.array_equal(g.host(part), wpart), (rows, cols)
+        for o in (out, out2):
+            assert g.same_bits(g.host(o)[:rows], want), (rows, cols)
+            assert (o[rows:] == 7.0).all(), (rows, cols)
+
+
+def test_q8_0_gemv_batch_of_ragged_rows(g, oracle):
+    """Items of 81 blocks a row, one of them off its 16-byte boundary, in one launch: the bits of the oracle."""
+    import torch
+    cols, rows_list = 2592, [64, 9, 1003, 8]
+    rng = synth.rng_for(SEED, 42)
+    qs, d = oracle.quantize_q8_0(rng.normal(0, 1, cols).astype(np.float32))
+    dq, dd = g.dev(qs), g.dev(d)
+    items = (capi.GemvItem * len(rows_list))()
+    keep, wants = [], []
+    for i, rows in enumerate(rows_list):
+        w = synth.matrix(synth.Q8_0, rng, rows, cols)
+        raw, out = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda"), g.empty(rows, np.float32)
+        raw[2 * i:2 * i + w.size] = torch.from_numpy(w.reshape(-1)).cuda()
+        keep.append((raw, out))
+        items[i].d_w, items[i].rows, items[i].d_act_qs, items[i].d_act_scales, items[i].d_out = raw.data_ptr() + 2 * i, rows, dq.data_ptr(), dd.data_ptr(), out.data_ptr()
+        wants.append(oracle.gemv(synth.Q8_0, w, rows, cols, qs, d))
+    capi.call("wd_gemv_q8_0_batch_f32", synth.Q8_0, items, len(rows_list), cols, g.stream())
+    g.sync()
+    for (_, out), want in zip(keep, wants):
+        assert g.same_bits(g.host(out), want)
+
+
 # cols, then the rows of every item: the projections of a block on one activation (2048 columns), the long rows of a down
 # projection (8192), a list longer than one launch takes (18 items), and lists with items the shared kernel does not
 # take (fewer than 8 rows; 8192 rows and more; a base 2 bytes into an allocation), which are launched by themselves

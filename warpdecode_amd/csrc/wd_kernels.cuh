@@ -455,87 +455,137 @@ __global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream_batch(GemvBatch b, 
                                        static_cast<int>(blockIdx.x) - b.first_group[item]);
 }
 
-// ---- dense Q8_0 x Q8_0 GEMV, streaming: one lane per (row, chain) ----------------------------------------------
+// ---- dense Q8_0 / IQ4_NL x Q8_0 GEMV, streaming: one lane per (row, chain) --------------------------------------
 // The reference order of a Q8_0 row (src/qwen38_cpu_moe.cuh:690-722) is eight chains, chain c over bytes 4c..4c+3 of
 // every block, each one fma(d_w d_a, float(dot4), acc) per block in block order: the chains of a row are as long as
-// the row, and nothing shortens them.  A wave therefore takes eight rows and gives every (row, chain) pair a lane
+// the row, and nothing shortens them.  IQ4_NL (:377-422) has the same eight chains - c < 4: the low nibbles of bytes
+// 4c..4c+3, c >= 4: the high ones of bytes 4(c-4).. -, each kept twice, over the even and over the odd blocks, and an
+// unpaired last block apart.  A wave therefore takes eight rows and gives every (row, chain) pair a lane
 // (lane = 8 row + chain): each fma instruction then advances 64 chains, no value crosses lanes until the closing tree,
-// and the cost per block and row is under one vector instruction.
-// The eight rows are fetched KB blocks at a time (34 KB bytes per row, whole 16-byte words because KB is a multiple of
-// 8 and rows start on 16-byte boundaries) with lane-contiguous 16-byte loads, one chunk ahead in a second register set,
-// and copied to LDS with a row stride that spreads the eight rows over the banks.  Blocks are 34 bytes, so the four
-// bytes of a lane are dword aligned in the odd blocks of a chunk and two bytes off in the even ones (two dwords and a
-// v_alignbyte); the parity is the same for every lane, so the unrolled loop knows it at compile time.
-// The activation's quants and its scales (as floats) are staged in LDS once per workgroup.
-// dynamic LDS: cols bytes, cols/32 floats, then one stage of 8 * kQ8sRowStride<KB> bytes per wave.
-template <int KB>
-constexpr int kQ8sRowStride = KB == 64 ? 2208 : (KB == 32 ? 1184 : 544);  // 34 KB + padding, 8 (mod 32) dwords
+// and the cost per block and row is under one vector instruction (IQ4_NL: two).
+// The eight rows are fetched KB blocks at a time (whole 16-byte words because KB is a multiple of 8) with lane-contiguous
+// 16-byte loads, one chunk ahead in a second register set, and copied to LDS with a row stride that spreads the eight rows
+// over the banks.  Blocks are 34 or 18 bytes, so the four bytes of a lane are dword aligned in the odd blocks of a chunk and
+// two bytes off in the even ones (two dwords and a v_alignbyte); the parity is the same for every lane, so the unrolled loop
+// knows it at compile time.
+// Rows that are no whole number of chunks end with a chunk of their LAST KB blocks, whose first blocks have been there
+// already and get the scale zero: every chunk is KB blocks long, starts at offset zero of its stage and reads nothing outside
+// its row.  RAGGED: such rows, and rows that do not start on 16-byte boundaries (loads are then two-byte aligned).
+// The activation's quants and its scales (as floats, in the order of the chunks) are staged in LDS once per workgroup.
+// dynamic LDS: cols bytes, a float per block of every chunk, then one stage of 8 * kQ8sRowStride<KIND, KB> bytes per wave.
+template <int KIND>
+constexpr int kQ8sBlk = KIND == 0 ? 34 : 18;
+template <int KIND, int KB>
+constexpr int kQ8sRowStride = KIND == 0 ? (KB == 32 ? 1184 : 544) : (KB == 32 ? 672 : 288);  // a chunk + padding, 8 (mod 32) dwords
 
-template <int KB>
+template <int KIND, int KB>
 struct Q8sFetch {
-    static constexpr int kWordsPerRow = 34 * KB / 16;                 // 16-byte words of a row's chunk
+    static constexpr int kWordsPerRow = kQ8sBlk<KIND> * KB / 16;      // 16-byte words of a row's chunk
     static constexpr int kWords = 8 * kWordsPerRow;                    // of the eight rows
     static constexpr int kLoads = (kWords + 63) / 64;
     uint4 u[kLoads];
 };
+template <bool RAGGED>
+WD_DEV uint4 q8s_load(const uint8_t *p) {
+    return RAGGED ? gld_u128(p) : gld_u128_aligned(p);
+}
 
 // Eight blocks of a lane's row (lane = 8 row + chain) out of a staged chunk: the lane's four bytes of every block, the
 // blocks' scales, the activation's four bytes and scales.  The LDS reads are issued as one group, so that a caller can put
 // the next group's before the arithmetic of this one.
+template <int KIND>
 struct Q8sBatch {
     uint32_t w[12];  // blocks 0 2 4 6 of the batch: two dwords each (w[3i], w[3i+1]); blocks 1 3 5 7: w[3i+2]
     uint32_t dw[8], a[8];
     float4 da[2];
     // my: the lane's bytes of the chunk's first block; row_blocks: the row's first block in the stage; my_a / ad: the
-    // activation's quants at the lane's chain and its scales; b0: the chunk's first block in the row; s: batch in the chunk.
-    WD_DEV void load(const uint8_t *my, const uint8_t *row_blocks, const int8_t *my_a, const float *ad, int b0, int s) {
+    // activation's quants at the lane's chain and its scales, of the chunk's first block; s: batch in the chunk.
+    WD_DEV void load(const uint8_t *my, const uint8_t *row_blocks, const int8_t *my_a, const float *ad, int s) {
+        constexpr int kBlk = kQ8sBlk<KIND>;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint8_t *blk = my + 34 * (8 * s + 2 * i);
+            const uint8_t *blk = my + kBlk * (8 * s + 2 * i);
             w[3 * i] = *reinterpret_cast<const uint32_t *>(blk);
             w[3 * i + 1] = *reinterpret_cast<const uint32_t *>(blk + 4);
-            w[3 * i + 2] = *reinterpret_cast<const uint32_t *>(blk + 36);
+            w[3 * i + 2] = *reinterpret_cast<const uint32_t *>(blk + kBlk + 2);
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            dw[i] = *reinterpret_cast<const uint16_t *>(row_blocks + 34 * (8 * s + i));
-            a[i] = *reinterpret_cast<const uint32_t *>(my_a + 32 * (b0 + 8 * s + i));
+            dw[i] = *reinterpret_cast<const uint16_t *>(row_blocks + kBlk * (8 * s + i));
+            a[i] = *reinterpret_cast<const uint32_t *>(my_a + 32 * (8 * s + i));
         }
-        da[0] = *reinterpret_cast<const float4 *>(ad + b0 + 8 * s);
-        da[1] = *reinterpret_cast<const float4 *>(ad + b0 + 8 * s + 4);
+        da[0] = *reinterpret_cast<const float4 *>(ad + 8 * s);
+        da[1] = *reinterpret_cast<const float4 *>(ad + 8 * s + 4);
     }
-    // block i of the batch: its scale product and its chunk sum
+    // block i of the batch: its scale product and its chunk sum (nibble: 0 or 4, the lane's half of the bytes)
     WD_DEV float scale(int i) const {
         const float d[8] = {da[0].x, da[0].y, da[0].z, da[0].w, da[1].x, da[1].y, da[1].z, da[1].w};
         return h2f(static_cast<uint16_t>(dw[i])) * d[i];
     }
-    WD_DEV int dot(int i) const {
+    WD_DEV int dot(int i, int nibble) const {
         const uint32_t q = (i & 1) ? w[3 * (i >> 1) + 2] : __builtin_amdgcn_alignbyte(w[3 * (i >> 1) + 1], w[3 * (i >> 1)], 2);
-        return sdot4(q, a[i], 0);
+        return sdot4(KIND == 0 ? q : iq4nl_values((q >> nibble) & 0x0f0f0f0fu), a[i], 0);
     }
 };
+// use(batch, s) for the batches s of a chunk in order.  AHEAD: the next eight blocks are requested from LDS before the
+// arithmetic of these, where the registers reach for two batches (72 of them); elsewhere they would be spilled.
+template <int KIND, int KB, bool AHEAD, typename Use>
+WD_DEV void q8s_batches(const uint8_t *my, const uint8_t *row_blocks, const int8_t *my_a, const float *ad, Use &&use) {
+    Q8sBatch<KIND> t0, t1;
+    if (!AHEAD) {
+#pragma unroll
+        for (int s = 0; s < KB / 8; ++s) {
+            t0.load(my, row_blocks, my_a, ad, s);
+            use(t0, s);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
+    t0.load(my, row_blocks, my_a, ad, 0);
+#pragma unroll
+    for (int s = 0; s < KB / 8; s += 2) {
+        t1.load(my, row_blocks, my_a, ad, s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        use(t0, s);
+        if (s + 2 < KB / 8) t0.load(my, row_blocks, my_a, ad, s + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        use(t1, s + 1);
+    }
+}
+// The unpaired last block of an IQ4_NL row: its scale times the whole-block integer sum (exact below 2^24).
+WD_DEV float q8s_tail(float scale, int p) {
+    p += lane_xor(p, 1);
+    p += lane_xor(p, 2);
+    p += lane_xor(p, 4);
+    return scale * static_cast<float>(p);
+}
+// The activation into LDS: its quants, and its scales in the order of chunks of `chunk` blocks (the last one: the row's last
+// `chunk` blocks).
+WD_DEV void q8s_stage_activation(int8_t *aq, float *ad, const int8_t *act_qs, const uint16_t *act_d, int nb, int chunk, int threads) {
+    const int whole = (nb + chunk - 1) / chunk * chunk, last = whole - chunk;
+    for (int i = threadIdx.x; i < nb * 2; i += threads) reinterpret_cast<uint4 *>(aq)[i] = reinterpret_cast<const uint4 *>(act_qs)[i];
+    for (int i = threadIdx.x; i < whole; i += threads) ad[i] = h2f(act_d[i < last ? i : i - whole + nb]);
+}
 
-// SETS: register sets of fetched chunks in flight per wave (2 for grids of single waves, which have nothing else to
-// hide the memory latency with).
-template <int KB, bool PART, int WAVES, int SETS>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES == 1 ? 1 : 4))) void k_gemv_q8_rows8(const uint8_t *__restrict__ w, int rows, int nb,
+template <int KIND, int KB, bool RAGGED, bool PART>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_gemv_q8_rows8(const uint8_t *__restrict__ w, int rows, int nb,
                                                               const int8_t *__restrict__ act_qs, const uint16_t *__restrict__ act_d,
                                                               float *__restrict__ out, int32_t *__restrict__ partials) {
-    using Fetch = Q8sFetch<KB>;
-    constexpr int RS = kQ8sRowStride<KB>;
+    constexpr int WAVES = 4, kBlk = kQ8sBlk<KIND>;
+    using Fetch = Q8sFetch<KIND, KB>;
+    constexpr int RS = kQ8sRowStride<KIND, KB>;
     extern __shared__ __align__(16) uint8_t q8s_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int cols = nb * 32;
+    const int cols = nb * 32, nchunks = (nb + KB - 1) / KB, skipped = nchunks * KB - nb;
     int8_t *aq = reinterpret_cast<int8_t *>(q8s_lds);
     float *ad = reinterpret_cast<float *>(q8s_lds + cols);
-    uint8_t *stage = q8s_lds + cols + nb * 4 + wave * (8 * RS);
-    const size_t rb = static_cast<size_t>(nb) * 34;
+    uint8_t *stage = q8s_lds + cols + nchunks * KB * 4 + wave * (8 * RS);
+    const size_t rb = static_cast<size_t>(nb) * kBlk;
     // the waves of the grid take the groups of eight rows in turn (rows >= 8)
     const int n_groups = (rows + 7) >> 3, n_waves = gridDim.x * WAVES, first = blockIdx.x * WAVES + wave;
     const int my_groups = first < n_groups ? (n_groups - first + n_waves - 1) / n_waves : 0;
-    const int nchunks = nb / KB;
     // where the lane's words of a chunk lie: in memory (relative to the chunk of the group's first row) and in the stage
-    const int row = lane >> 3, c = lane & 7;
+    const int row = lane >> 3, c = lane & 7, nibble = c & 4;
     uint32_t goff[Fetch::kLoads], loff[Fetch::kLoads];
 #pragma unroll
     for (int i = 0; i < Fetch::kLoads; ++i) {
@@ -544,105 +594,107 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
         goff[i] = static_cast<uint32_t>(r * rb + 16 * within);
         loff[i] = static_cast<uint32_t>(r * RS + 16 * within);
     }
-    // the fetch runs SETS chunks ahead of the arithmetic, over the group boundaries
+    // a chunk's first block in its row
+    auto first_block = [&](int chunk) { return RAGGED && chunk == nchunks - 1 ? nb - KB : chunk * KB; };
+    // the fetch runs one chunk ahead of the arithmetic, over the group boundaries
     int f_group = min(first, n_groups - 1), f_chunk = 0, fetched = 0;
     const int items = my_groups * nchunks;
-    Fetch fs[SETS];
-    auto fetch = [&](Fetch &f) {
+    Fetch f;
+    auto fetch = [&]() {
         // a last group of fewer than eight rows is moved up to end with the matrix: it then repeats rows of the group
         // before it, which come out the same
-        const uint8_t *p = uniform_ptr(w + static_cast<size_t>(min(8 * f_group, rows - 8)) * rb + static_cast<size_t>(f_chunk) * (34 * KB));
+        const uint8_t *p = uniform_ptr(w + static_cast<size_t>(min(8 * f_group, rows - 8)) * rb + static_cast<size_t>(first_block(f_chunk)) * kBlk);
 #pragma unroll
-        for (int i = 0; i < Fetch::kLoads; ++i) f.u[i] = gld_u128_aligned(p + goff[i]);
+        for (int i = 0; i < Fetch::kLoads; ++i) f.u[i] = q8s_load<RAGGED>(p + goff[i]);
         // past the wave's last chunk the same chunk is requested again (and not used), so that every turn issues the
         // same number of requests
         if (++fetched < items) {
             if (++f_chunk == nchunks) f_chunk = 0, f_group += n_waves;
         }
     };
-#pragma unroll
-    for (int i = 0; i < SETS; ++i) fetch(fs[i]);
-    for (int i = threadIdx.x; i < cols / 16; i += 64 * WAVES) reinterpret_cast<uint4 *>(aq)[i] = reinterpret_cast<const uint4 *>(act_qs)[i];
-    for (int i = threadIdx.x; i < nb; i += 64 * WAVES) ad[i] = h2f(act_d[i]);
+    fetch();
+    q8s_stage_activation(aq, ad, act_qs, act_d, nb, KB, 64 * WAVES);
     __syncthreads();
     if (my_groups == 0) return;  // wave-uniform
-    const uint8_t *my = stage + row * RS + 4 * c;
-    const int8_t *my_a = aq + 4 * c;
-    float acc = 0.0f;
+    const uint8_t *row_blocks = stage + row * RS, *my = row_blocks + 4 * (KIND == 0 ? c : c & 3);
+    float acc = 0.0f, odd = 0.0f, tail = 0.0f;
     int group = first, chunk = 0;
-    auto turn = [&](Fetch &f) {
+    for (int t = 0; t < items; ++t) {
         wave_lds_fence();  // the previous chunk has been read
 #pragma unroll
         for (int i = 0; i < Fetch::kLoads; ++i) *reinterpret_cast<uint4 *>(stage + loff[i]) = f.u[i];
         wave_lds_fence();
-        fetch(f);  // a later chunk, into the registers just written out
-        const int b0 = chunk * KB;
+        fetch();  // a later chunk, into the registers just written out
+        const bool last = chunk == nchunks - 1;
+        const int b0 = first_block(chunk), skip = RAGGED && last ? skipped : 0;
+        const bool unpaired = KIND == 1 && RAGGED && last && (nb & 1);
+        if (unpaired) {  // (the chunk then starts with an odd block; the closing sum takes the two in either order)
+            const float swap = acc;
+            acc = odd, odd = swap;
+        }
         const int out_row = min(8 * group, rows - 8) + row;
-        int32_t *pp = PART ? partials + (static_cast<size_t>(out_row) * nb) * 8 + c : nullptr;
-        const uint8_t *row_blocks = stage + row * RS;
-        auto compute_batch = [&](const Q8sBatch &bt, int s) {
+        int32_t *pp = PART ? partials + (static_cast<size_t>(out_row) * nb + b0) * 8 + c : nullptr;
+        const int8_t *my_a = aq + 4 * c + 32 * b0;
+        const float *my_d = ad + chunk * KB;
+        auto compute_batch = [&](const Q8sBatch<KIND> &bt, int s) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const int p = bt.dot(i);
-                if (PART) pp[(b0 + 8 * s + i) * 8] = p;
-                acc = __builtin_fmaf(bt.scale(i), static_cast<float>(p), acc);
+                const int at = 8 * s + i, p = bt.dot(i, nibble);
+                float scale = bt.scale(i);
+                if (PART && at >= skip) pp[at * 8] = p;
+                if (RAGGED && at < skip) scale = 0.0f;
+                if (RAGGED && KIND == 1 && at == KB - 1 && unpaired) {
+                    tail = q8s_tail(scale, p);
+                    scale = 0.0f;
+                }
+                float &chain = KIND == 1 && (i & 1) ? odd : acc;
+                chain = __builtin_fmaf(scale, static_cast<float>(p), chain);
             }
+            asm volatile("" : "+v"(acc), "+v"(odd));  // (batch by batch: the products are not kept for later)
         };
-        // eight blocks at a time, the next eight requested from LDS before the arithmetic of these
-        Q8sBatch t0, t1;
-        t0.load(my, row_blocks, my_a, ad, b0, 0);
-#pragma unroll
-        for (int s = 0; s < KB / 8; s += 2) {
-            t1.load(my, row_blocks, my_a, ad, b0, s + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            compute_batch(t0, s);
-            if (s + 2 < KB / 8) t0.load(my, row_blocks, my_a, ad, b0, s + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            compute_batch(t1, s + 1);
-        }
+        q8s_batches<KIND, KB, KB == 16>(my, row_blocks, my_a, my_d, compute_batch);
         if (++chunk == nchunks) {
-            const float y = close_lanes8(acc);
+            float y = close_lanes8(KIND == 1 ? acc + odd : acc);
+            if (RAGGED && KIND == 1 && (nb & 1)) y = y + tail;
             if (c == 0) out[out_row] = y;
-            acc = 0.0f, chunk = 0, group += n_waves;
-        }
-    };
-    for (int t = 0; t < items; t += SETS) {
-#pragma unroll
-        for (int i = 0; i < SETS; ++i) {
-            if (t + i >= items) break;
-            turn(fs[i]);
+            acc = 0.0f, odd = 0.0f, chunk = 0, group += n_waves;
         }
     }
 }
 
-// ---- dense Q8_0 x Q8_0 GEMV, few rows: the waves of a workgroup share the eight rows of a group --------------------
+// ---- the same, few rows: the waves of a workgroup share the eight rows of a group ----------------------------------
 // With few row groups a group's wave runs alone on its SIMD and the time is the length of its chains (about 40 cycles
 // per block: one wave issues an instruction every four cycles and a block is ten of them).  Only the fma itself has to
-// run in block order.  So wave v of a workgroup takes blocks [v NCH*KB, (v+1) NCH*KB) of the eight rows, requests all
-// of them at once, turns them into (d_w d_a, float(dot4)) pairs in registers at its own pace, and then the waves run
-// their parts of the chains one after the other, handing the 64 accumulators on through LDS: NCH*KB dependent fma per
-// wave, nothing else.  Lane = 8 row + chain as in k_gemv_q8_rows8; nb = KB NCH WAVES blocks per row (KB = 16 or 32).
-// dynamic LDS: cols bytes, cols/32 floats, 256 bytes of accumulators, then one stage of 8 * kQ8sRowStride<KB> per wave.
+// run in block order.  So wave v of a workgroup takes blocks [v NCH*KB, (v+1) NCH*KB) of the eight rows (the last one the
+// last NCH*KB), requests all of them at once, turns them into (d_w d_a, float(dot4)) pairs in registers at its own pace, and
+// then the waves run their parts of the chains one after the other, handing the 64 accumulators on through LDS: NCH*KB
+// dependent fma per wave, nothing else.  Lane = 8 row + chain and RAGGED as in k_gemv_q8_rows8; up to eight waves (WAVES, or any
+// number when that is 0), nb > their blocks but those of the last, and nb >= NCH*KB.
+// dynamic LDS: cols bytes, a float per block of every wave, 512 bytes of accumulators, then one stage of
+// 8 * kQ8sRowStride<KIND, KB> per wave.
 // (the body: `group` is the workgroup's group of eight rows)
-template <int KB, int NCH, int WAVES, bool PART>
+template <int KIND, int KB, int NCH, int WAVES, bool RAGGED, bool PART>
 WD_DEV void gemv_q8_rows8_split_body(const uint8_t *__restrict__ w, int rows, int nb, const int8_t *__restrict__ act_qs,
                                      const uint16_t *__restrict__ act_d, float *__restrict__ out, int32_t *__restrict__ partials,
                                      int group) {
-    constexpr int SEG = NCH * KB;
-    using Fetch = Q8sFetch<KB>;
-    constexpr int RS = kQ8sRowStride<KB>;
+    constexpr int SEG = NCH * KB, kBlk = kQ8sBlk<KIND>;
+    using Fetch = Q8sFetch<KIND, KB>;
+    constexpr int RS = kQ8sRowStride<KIND, KB>;
     extern __shared__ __align__(16) uint8_t q8p_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int cols = nb * 32;
+    const int cols = nb * 32, waves = WAVES ? WAVES : (nb + SEG - 1) / SEG;
+    const bool last = wave == waves - 1;
     int8_t *aq = reinterpret_cast<int8_t *>(q8p_lds);
     float *ad = reinterpret_cast<float *>(q8p_lds + cols);
-    float *carry = reinterpret_cast<float *>(q8p_lds + cols + nb * 4);
-    uint8_t *stage = q8p_lds + cols + nb * 4 + 256 + wave * (8 * RS);
-    const size_t rb = static_cast<size_t>(nb) * 34;
-    const int row = lane >> 3, c = lane & 7;
+    float *carry = reinterpret_cast<float *>(q8p_lds + cols + waves * SEG * 4);
+    uint8_t *stage = q8p_lds + cols + waves * SEG * 4 + 512 + wave * (8 * RS);
+    const size_t rb = static_cast<size_t>(nb) * kBlk;
+    const int row = lane >> 3, c = lane & 7, nibble = c & 4;
     // a last group of fewer than eight rows is moved up to end with the matrix (rows >= 8)
     const int base_row = min(8 * group, rows - 8);
-    const uint8_t *src = uniform_ptr(w + static_cast<size_t>(base_row) * rb + static_cast<size_t>(wave) * (34 * SEG));
+    const int first_block = RAGGED && last ? nb - SEG : wave * SEG, skip = RAGGED && last ? waves * SEG - nb : 0;
+    const bool unpaired = KIND == 1 && RAGGED && last && (nb & 1);
+    const uint8_t *src = uniform_ptr(w + static_cast<size_t>(base_row) * rb + static_cast<size_t>(first_block) * kBlk);
     uint32_t loff[Fetch::kLoads];
     Fetch f[NCH];
 #pragma unroll
@@ -652,76 +704,90 @@ WD_DEV void gemv_q8_rows8_split_body(const uint8_t *__restrict__ w, int rows, in
         loff[i] = static_cast<uint32_t>(r * RS + 16 * within);
         const uint32_t goff = static_cast<uint32_t>(r * rb + 16 * within);
 #pragma unroll
-        for (int ch = 0; ch < NCH; ++ch) f[ch].u[i] = gld_u128_aligned(src + goff + ch * (34 * KB));
+        for (int ch = 0; ch < NCH; ++ch) f[ch].u[i] = q8s_load<RAGGED>(src + goff + ch * (kBlk * KB));
     }
-    for (int i = threadIdx.x; i < cols / 16; i += 64 * WAVES) reinterpret_cast<uint4 *>(aq)[i] = reinterpret_cast<const uint4 *>(act_qs)[i];
-    for (int i = threadIdx.x; i < nb; i += 64 * WAVES) ad[i] = h2f(act_d[i]);
+    q8s_stage_activation(aq, ad, act_qs, act_d, nb, SEG, 64 * waves);
     __syncthreads();
-    const uint8_t *my = stage + row * RS + 4 * c;
-    const int8_t *my_a = aq + 4 * c;
-    const int first_block = wave * SEG;
-    int32_t *pp = PART ? partials + (static_cast<size_t>(base_row + row) * nb) * 8 + c : nullptr;
-    float dv[SEG], pv[SEG];
-    const uint8_t *row_blocks = stage + row * RS;
+    const uint8_t *row_blocks = stage + row * RS, *my = row_blocks + 4 * (KIND == 0 ? c : c & 3);
+    int32_t *pp = PART ? partials + (static_cast<size_t>(base_row + row) * nb + first_block) * 8 + c : nullptr;
+    float dv[SEG], pv[SEG], acc = 0.0f, odd = 0.0f, tail = 0.0f;
 #pragma unroll
     for (int ch = 0; ch < NCH; ++ch) {
         wave_lds_fence();  // the previous chunk has been read
 #pragma unroll
         for (int i = 0; i < Fetch::kLoads; ++i) *reinterpret_cast<uint4 *>(stage + loff[i]) = f[ch].u[i];
         wave_lds_fence();
-        const int b0 = first_block + ch * KB;
-        auto pairs = [&](const Q8sBatch &bt, int s) {
+        const int8_t *my_a = aq + 4 * c + 32 * (first_block + ch * KB);
+        const float *my_d = ad + wave * SEG + ch * KB;
+        auto pairs = [&](const Q8sBatch<KIND> &bt, int s) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const int p = bt.dot(i);
-                if (PART) pp[(b0 + 8 * s + i) * 8] = p;
-                dv[ch * KB + 8 * s + i] = bt.scale(i);
-                pv[ch * KB + 8 * s + i] = static_cast<float>(p);
+                const int at = ch * KB + 8 * s + i, p = bt.dot(i, nibble);
+                float scale = bt.scale(i);
+                if (PART && at >= skip) pp[at * 8] = p;
+                if (RAGGED && at < skip) scale = 0.0f;
+                if (RAGGED && KIND == 1 && at == SEG - 1 && unpaired) {
+                    tail = q8s_tail(scale, p);
+                    scale = 0.0f;
+                }
+                dv[at] = scale;
+                pv[at] = static_cast<float>(p);
+                // Made here: left to itself the compiler moves the products into the wave's turn, and the turns are serial
+                // (five waves, 5000 x 5120: 13.7 us instead of 11.6).  Where the number of waves is known it does better.
+                if (WAVES == 0) asm volatile("" : "+v"(dv[at]), "+v"(pv[at]));
             }
         };
-        Q8sBatch t0, t1;
-        t0.load(my, row_blocks, my_a, ad, b0, 0);
-#pragma unroll
-        for (int s = 0; s < KB / 8; s += 2) {
-            t1.load(my, row_blocks, my_a, ad, b0, s + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            pairs(t0, s);
-            if (s + 2 < KB / 8) t0.load(my, row_blocks, my_a, ad, b0, s + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            pairs(t1, s + 1);
-        }
+        q8s_batches<KIND, KB, true>(my, row_blocks, my_a, my_d, pairs);
     }
     // the chains, one wave after the other in block order
-    float acc = 0.0f;
-#pragma unroll
-    for (int turn = 0; turn < WAVES; ++turn) {
+    auto take_turn = [&](int turn) {
         if (wave == turn) {
-            if (turn > 0) acc = carry[lane];
+            if (turn > 0) {
+                acc = carry[lane];
+                if (KIND == 1) odd = carry[64 + lane];
+            }
+            if (unpaired) {  // (the part starts with an odd block; the closing sum takes the two in either order)
+                const float swap = acc;
+                acc = odd, odd = swap;
+            }
 #pragma unroll
-            for (int i = 0; i < SEG; ++i) acc = __builtin_fmaf(dv[i], pv[i], acc);
-            if (turn < WAVES - 1) carry[lane] = acc;
+            for (int i = 0; i < SEG; ++i) {
+                float &chain = KIND == 1 && (i & 1) ? odd : acc;
+                chain = __builtin_fmaf(dv[i], pv[i], chain);
+            }
+            if (turn < waves - 1) {
+                carry[lane] = acc;
+                if (KIND == 1) carry[64 + lane] = odd;
+            }
         }
-        if (turn < WAVES - 1) __syncthreads();
+        if (turn < waves - 1) __syncthreads();
+    };
+    if constexpr (WAVES != 0) {
+#pragma unroll
+        for (int turn = 0; turn < WAVES; ++turn) take_turn(turn);
+    } else {
+        for (int turn = 0; turn < waves; ++turn) take_turn(turn);
     }
-    if (wave == WAVES - 1) {
-        const float y = close_lanes8(acc);
+    if (last) {
+        float y = close_lanes8(KIND == 1 ? acc + odd : acc);
+        if (KIND == 1 && unpaired) y = y + tail;
         if (c == 0) out[base_row + row] = y;
     }
 }
-template <int KB, int NCH, int WAVES, bool PART>
-__global__ __launch_bounds__(64 * WAVES) void k_gemv_q8_rows8_split(const uint8_t *__restrict__ w, int rows, int nb,
+template <int KIND, int KB, int NCH, int WAVES, bool RAGGED, bool PART>
+__global__ __launch_bounds__(WAVES ? 64 * WAVES : 512) void k_gemv_q8_rows8_split(const uint8_t *__restrict__ w, int rows, int nb,
                                                               const int8_t *__restrict__ act_qs, const uint16_t *__restrict__ act_d,
                                                               float *__restrict__ out, int32_t *__restrict__ partials) {
-    gemv_q8_rows8_split_body<KB, NCH, WAVES, PART>(w, rows, nb, act_qs, act_d, out, partials, static_cast<int>(blockIdx.x));
+    gemv_q8_rows8_split_body<KIND, KB, NCH, WAVES, RAGGED, PART>(w, rows, nb, act_qs, act_d, out, partials, static_cast<int>(blockIdx.x));
 }
 // Several matrices of the same row length in ONE launch (the projections a block applies to one or a few activations:
 // each of them alone is bound by its launch, not by its bytes).  Workgroup b belongs to the item whose range of row
 // groups holds b; what it computes is what k_gemv_q8_rows8_split computes for that item alone.
-template <int KB, int NCH, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void k_gemv_q8_rows8_split_batch(GemvBatch b, int nb) {
+template <int KB, int NCH, int WAVES, bool RAGGED>
+__global__ __launch_bounds__(WAVES ? 64 * WAVES : 512) void k_gemv_q8_rows8_split_batch(GemvBatch b, int nb) {
     const int item = gemv_batch_item(b);
-    gemv_q8_rows8_split_body<KB, NCH, WAVES, false>(b.w[item], b.rows[item], nb, b.act_qs[item], b.act_d[item], b.out[item], nullptr,
-                                                   static_cast<int>(blockIdx.x) - b.first_group[item]);
+    gemv_q8_rows8_split_body<0, KB, NCH, WAVES, RAGGED, false>(b.w[item], b.rows[item], nb, b.act_qs[item], b.act_d[item], b.out[item], nullptr,
+                                                       static_cast<int>(blockIdx.x) - b.first_group[item]);
 }
 
 // ---- Q6_K x Q8_K GEMV: the waves of the grid take the rows in turn, pass by pass, one pass fetched ahead -------

@@ -224,20 +224,93 @@ static int launch_gemv_q8k(int type, MatSrc src, int mats, int rows, int cols, c
     return WD_OK;
 }
 
-// The split configuration of the streaming kernel for rows of nb blocks in `groups` groups of eight rows; null when the
-// kernel for that shape is another one.
-struct Q8Split { int nb, kb, nch, waves; };
-static const Q8Split *q8_split_for(int nb, int groups) {
-    static const Q8Split kSplits[] = {{64, 32, 1, 2}, {80, 16, 1, 5}, {128, 32, 1, 4}, {160, 32, 1, 5}, {256, 32, 1, 8},
-                                      {256, 32, 2, 4}, {320, 32, 2, 5}, {512, 32, 2, 8}};
-    for (const Q8Split &sp : kSplits) {
-        if (groups >= 1024 || sp.nb != nb) continue;
-        // 8192 columns: eight waves when a compute unit gets one workgroup, four (two chunks each) when it gets more
-        if (nb == 256 && (sp.waves == 8) != (groups <= 256)) continue;
-        return &sp;
-    }
-    return nullptr;
+// ---- the streaming kernels of Q8_0 and IQ4_NL rows (k_gemv_q8_rows8 and its split form) ---------------------------
+// Rows of at least one chunk, up to what the activation may take of LDS; aligned activations; eight rows or more.  Many rows
+// (no split) of 17 to 21 blocks stay with the general kernel: more than half of them would be repeated to fill the second chunk
+// (9000 x 544 Q8_0: 5.4 us against 4.7).
+static bool q8_streams(int rows, int nb, const int8_t *qs) {
+    if (rows >= 8 * 1023 + 1 && nb > 16 && nb < 22) return false;
+    return rows >= 8 && nb >= 16 && nb <= 512 && reinterpret_cast<uintptr_t>(qs) % 16 == 0;
 }
+// How the waves of a workgroup share rows of nb blocks, given `groups` groups of eight rows: kb * nch blocks per wave, as few
+// repeated ones as the choice allows; kb == 0: rows enough to give every SIMD a group of its own (the kernel without split).
+struct Q8Split {
+    int kb, nch, waves;
+    bool operator==(const Q8Split &o) const { return kb == o.kb && nch == o.nch && waves == o.waves; }
+};
+static Q8Split q8_split_for(int nb, int groups) {
+    const int w16 = (nb + 15) / 16, w32 = (nb + 31) / 32, w64 = (nb + 63) / 64;
+    if (groups >= 1024) return {0, 0, 0};
+    if (nb < 32 || (16 * w16 < 32 * w32 && w16 <= 8)) return {16, 1, w16};
+    // beyond five waves of 32 blocks: that many when a compute unit gets one workgroup, half (two chunks each) when it gets more
+    if (w32 <= 5 || (w32 <= 8 && groups <= 256)) return {32, 1, w32};
+    return {32, 2, w64};
+}
+static size_t q8_split_lds(int kind, const Q8Split &sp, int nb) {
+    const int stride = kind == 0 ? (sp.kb == 32 ? kQ8sRowStride<0, 32> : kQ8sRowStride<0, 16>)
+                                 : (sp.kb == 32 ? kQ8sRowStride<1, 32> : kQ8sRowStride<1, 16>);
+    return static_cast<size_t>(nb) * 32 + static_cast<size_t>(sp.waves) * (sp.kb * sp.nch * 4 + 8 * stride) + 512;
+}
+// Rows of other lengths than whole chunks, or off 16-byte boundaries.
+static bool q8_ragged(const uint8_t *w, int nb, int chunk) { return nb % chunk != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0; }
+
+#define WD_Q8_FIXED_SPLITS \
+    WD_Q8_SPLIT(32, 1, 2) WD_Q8_SPLIT(16, 1, 5) WD_Q8_SPLIT(32, 1, 4) WD_Q8_SPLIT(32, 1, 5) WD_Q8_SPLIT(32, 1, 8) \
+    WD_Q8_SPLIT(32, 2, 4) WD_Q8_SPLIT(32, 2, 5) WD_Q8_SPLIT(32, 2, 8)
+
+}  // extern "C" (a template)
+template <int KIND>
+static void launch_q8_stream(const uint8_t *w, int rows, int nb, const int8_t *qs, const uint16_t *d, float *out, int32_t *partials,
+                             hipStream_t stream) {
+    const int groups = (rows + 7) / 8;
+    const Q8Split sp = q8_split_for(nb, groups);
+    if (sp.kb) {
+        const size_t lds = q8_split_lds(KIND, sp, nb);
+        auto launch = [&](auto kernel) { kernel<<<groups, 64 * sp.waves, lds, stream>>>(w, rows, nb, qs, d, out, partials); };
+        if constexpr (KIND == 0) {
+            // whole chunks on 16-byte boundaries, the usual row lengths (2048, 2560, 4096, 5120, 8192, 10240, 16384 columns):
+            // kernels that know their number of waves (2560 x 2560: 4.97 us, 5.16 with the number taken from nb)
+            if (!partials && !q8_ragged(w, nb, sp.kb * sp.nch)) {
+#define WD_Q8_SPLIT(KB_, NCH_, WAVES_)                                                 \
+    if (sp == Q8Split{KB_, NCH_, WAVES_}) {                                             \
+        launch(k_gemv_q8_rows8_split<0, KB_, NCH_, WAVES_, false, false>);               \
+        return;                                                                          \
+    }
+                WD_Q8_FIXED_SPLITS
+#undef WD_Q8_SPLIT
+            }
+        }
+#define WD_Q8_SPLIT(KB_, NCH_)                                                           \
+    if (sp.kb == KB_ && sp.nch == NCH_) {                                                 \
+        if (partials) launch(k_gemv_q8_rows8_split<KIND, KB_, NCH_, 0, true, true>);       \
+        else launch(k_gemv_q8_rows8_split<KIND, KB_, NCH_, 0, true, false>);               \
+    }
+        WD_Q8_SPLIT(16, 1)
+        WD_Q8_SPLIT(32, 1)
+        WD_Q8_SPLIT(32, 2)
+#undef WD_Q8_SPLIT
+        return;
+    }
+    // Workgroups of four waves, each taking several row groups beyond 1024 workgroups; chunks of about the same bytes for
+    // both kinds
+    const int kb = KIND == 1 && nb >= 64 ? 32 : 16, nchunks = (nb + kb - 1) / kb;
+    const unsigned wgs = static_cast<unsigned>(std::min((groups + 3) / 4, 1024));
+    const size_t lds = static_cast<size_t>(nb) * 32 + static_cast<size_t>(nchunks) * kb * 4 +
+                       4 * 8 * (kb == 32 ? kQ8sRowStride<KIND, 32> : kQ8sRowStride<KIND, 16>);
+    auto launch = [&](auto kernel) { kernel<<<wgs, 256, lds, stream>>>(w, rows, nb, qs, d, out, partials); };
+    const bool ragged = q8_ragged(w, nb, kb);
+    if (KIND == 1 && kb == 32) {
+        if (partials) launch(k_gemv_q8_rows8<1, 32, true, true>);
+        else if (ragged) launch(k_gemv_q8_rows8<1, 32, true, false>);
+        else launch(k_gemv_q8_rows8<1, 32, false, false>);
+    } else {
+        if (partials) launch(k_gemv_q8_rows8<KIND, 16, true, true>);
+        else if (ragged) launch(k_gemv_q8_rows8<KIND, 16, true, false>);
+        else launch(k_gemv_q8_rows8<KIND, 16, false, false>);
+    }
+}
+
+extern "C" {
 
 static int launch_gemv_q8_0(int type, MatSrc src, int mats, int rows, int cols, const int8_t *qs, const uint16_t *d,
                             int act_per_mat, float *out, int32_t *partials, hipStream_t stream) {
@@ -274,46 +347,9 @@ static int launch_gemv_q8_0(int type, MatSrc src, int mats, int rows, int cols, 
         WD_LAUNCH_CHECK();
         return WD_OK;
     }
-    if (type == WD_TYPE_Q8_0 && mats == 1 && src.single && nb % 16 == 0 && cols <= 16384 && rows >= 8 &&
-        reinterpret_cast<uintptr_t>(src.single) % 16 == 0 && reinterpret_cast<uintptr_t>(qs) % 16 == 0) {
-        // whole 16-byte words per row chunk and a 16-byte aligned base: the streaming kernel, eight rows per wave
-        const int groups = (rows + 7) / 8;
-        // few row groups: the waves of a workgroup share a group, the chain runs over prepared pairs
-        if (const Q8Split *found = q8_split_for(nb, groups)) {
-            const Q8Split &sp = *found;
-            const size_t lds = static_cast<size_t>(cols) + static_cast<size_t>(nb) * 4 + 256 +
-                               static_cast<size_t>(sp.waves) * 8 * (sp.kb == 32 ? kQ8sRowStride<32> : kQ8sRowStride<16>);
-            auto launch = [&](auto kernel) { kernel<<<groups, 64 * sp.waves, lds, stream>>>(src.single, rows, nb, qs, d, out, partials); };
-#define WD_Q8_SPLIT(KB_, NCH_, WAVES_)                                                                      \
-    if (sp.kb == KB_ && sp.nch == NCH_ && sp.waves == WAVES_) {                                               \
-        partials ? launch(k_gemv_q8_rows8_split<KB_, NCH_, WAVES_, true>) : launch(k_gemv_q8_rows8_split<KB_, NCH_, WAVES_, false>); \
-    }
-            WD_Q8_SPLIT(32, 1, 2)
-            WD_Q8_SPLIT(16, 1, 5)
-            WD_Q8_SPLIT(32, 1, 4)
-            WD_Q8_SPLIT(32, 1, 5)
-            WD_Q8_SPLIT(32, 1, 8)
-            WD_Q8_SPLIT(32, 2, 4)
-            WD_Q8_SPLIT(32, 2, 5)
-            WD_Q8_SPLIT(32, 2, 8)
-#undef WD_Q8_SPLIT
-            WD_LAUNCH_CHECK();
-            return WD_OK;
-        }
-        // Workgroups of four waves (taking several row groups each beyond 1024 workgroups) when there is a row group
-        // or more per SIMD; otherwise single waves, which keep two chunks in flight to cover the memory latency.
-        const int waves = groups >= 1024 ? 4 : 1;
-        int wgs_wanted = (groups + waves - 1) / waves;
-        wgs_wanted = std::min(wgs_wanted, waves == 4 ? 1024 : 2048);
-        const unsigned wgs = static_cast<unsigned>(wgs_wanted);
-        // single waves: 32-block chunks, two of them in flight; full workgroups: 16-block chunks, one ahead
-        const int kb = (waves == 1 && nb % 32 == 0) ? 32 : 16;
-        const size_t lds = static_cast<size_t>(cols) + static_cast<size_t>(nb) * 4 +
-                           static_cast<size_t>(waves) * 8 * (kb == 32 ? kQ8sRowStride<32> : kQ8sRowStride<16>);
-        auto launch = [&](auto kernel) { kernel<<<wgs, 64 * waves, lds, stream>>>(src.single, rows, nb, qs, d, out, partials); };
-        if (waves == 4) partials ? launch(k_gemv_q8_rows8<16, true, 4, 1>) : launch(k_gemv_q8_rows8<16, false, 4, 1>);
-        else if (kb == 32) partials ? launch(k_gemv_q8_rows8<32, true, 1, 2>) : launch(k_gemv_q8_rows8<32, false, 1, 2>);
-        else partials ? launch(k_gemv_q8_rows8<16, true, 1, 2>) : launch(k_gemv_q8_rows8<16, false, 1, 2>);
+    if (type != WD_TYPE_Q4_0 && mats == 1 && src.single && q8_streams(rows, nb, qs)) {
+        if (type == WD_TYPE_Q8_0) launch_q8_stream<0>(src.single, rows, nb, qs, d, out, partials, stream);
+        else launch_q8_stream<1>(src.single, rows, nb, qs, d, out, partials, stream);
         WD_LAUNCH_CHECK();
         return WD_OK;
     }
@@ -440,22 +476,18 @@ int wd_gemv_q8_0_batch_f32(int type, const wd_gemv_item *items, int n_items, int
                    "batched GEMV: item %d has a null pointer or no rows", i);
     if (type == WD_TYPE_Q4_0) return gemv_q4_0_batch(items, n_items, cols, stream);
     const int nb = cols / 32;
-    // One launch for as many items in a row as take the same kernel: every item must be a shape the split kernel takes
-    // alone (then its workgroups do here exactly what they do there); anything else is launched by itself.
-    auto splits_alike = [&](const wd_gemv_item &it, const Q8Split *want) {
-        const Q8Split *sp = nb % 16 == 0 && cols <= 16384 && it.rows >= 8 && reinterpret_cast<uintptr_t>(it.d_w) % 16 == 0 &&
-                                    reinterpret_cast<uintptr_t>(it.d_act_qs) % 16 == 0
-                                ? q8_split_for(nb, (it.rows + 7) / 8)
-                                : nullptr;
-        return sp != nullptr && (want == nullptr || sp == want) ? sp : nullptr;
+    // One launch for as many items in a row as take the same split kernel: a workgroup does here exactly what it does for its
+    // item alone; anything else is launched by itself.
+    auto split_of = [&](const wd_gemv_item &it) {
+        return q8_streams(it.rows, nb, it.d_act_qs) ? q8_split_for(nb, (it.rows + 7) / 8) : Q8Split{0, 0, 0};
     };
     int i = 0;
     while (i < n_items) {
-        const Q8Split *sp = splits_alike(items[i], nullptr);
+        const Q8Split sp = split_of(items[i]);
         int j = i + 1;
-        if (sp)
-            while (j < n_items && j - i < kGemvBatchMax && splits_alike(items[j], sp)) ++j;
-        if (!sp || j - i == 1) {
+        if (sp.kb)
+            while (j < n_items && j - i < kGemvBatchMax && split_of(items[j]) == sp) ++j;
+        if (!sp.kb || j - i == 1) {
             if (const int rc = wd_gemv_q8_0_f32(type, items[i].d_w, items[i].rows, cols, items[i].d_act_qs, items[i].d_act_scales,
                                                 items[i].d_out, nullptr, stream))
                 return rc;
@@ -465,28 +497,26 @@ int wd_gemv_q8_0_batch_f32(int type, const wd_gemv_item *items, int n_items, int
         GemvBatch b{};
         b.n = j - i;
         int groups = 0;
+        bool ragged = false;
         for (int q = 0; q < b.n; ++q) {
             const wd_gemv_item &it = items[i + q];
             b.w[q] = it.d_w, b.act_qs[q] = it.d_act_qs, b.act_d[q] = it.d_act_scales, b.out[q] = it.d_out, b.rows[q] = it.rows;
             b.first_group[q] = groups;
             groups += (it.rows + 7) / 8;
+            ragged = ragged || q8_ragged(it.d_w, nb, sp.kb * sp.nch);
         }
         for (int q = b.n; q <= kGemvBatchMax; ++q) b.first_group[q] = groups;
-        const size_t lds = static_cast<size_t>(cols) + static_cast<size_t>(nb) * 4 + 256 +
-                           static_cast<size_t>(sp->waves) * 8 * (sp->kb == 32 ? kQ8sRowStride<32> : kQ8sRowStride<16>);
-        const hipStream_t st = as_stream(stream);
-#define WD_Q8_BATCH(KB_, NCH_, WAVES_)                                    \
-    if (sp->kb == KB_ && sp->nch == NCH_ && sp->waves == WAVES_)          \
-        k_gemv_q8_rows8_split_batch<KB_, NCH_, WAVES_><<<groups, 64 * WAVES_, lds, st>>>(b, nb);
-        WD_Q8_BATCH(32, 1, 2)
-        WD_Q8_BATCH(16, 1, 5)
-        WD_Q8_BATCH(32, 1, 4)
-        WD_Q8_BATCH(32, 1, 5)
-        WD_Q8_BATCH(32, 1, 8)
-        WD_Q8_BATCH(32, 2, 4)
-        WD_Q8_BATCH(32, 2, 5)
-        WD_Q8_BATCH(32, 2, 8)
-#undef WD_Q8_BATCH
+        const size_t lds = q8_split_lds(0, sp, nb);
+        auto launch = [&](auto kernel) { kernel<<<groups, 64 * sp.waves, lds, as_stream(stream)>>>(b, nb); };
+        bool fixed = false;
+#define WD_Q8_SPLIT(KB_, NCH_, WAVES_)                                                                                       \
+    if (!ragged && sp == Q8Split{KB_, NCH_, WAVES_}) launch(k_gemv_q8_rows8_split_batch<KB_, NCH_, WAVES_, false>), fixed = true;
+        WD_Q8_FIXED_SPLITS
+#undef WD_Q8_SPLIT
+        if (fixed) {
+        } else if (sp.kb == 16) launch(k_gemv_q8_rows8_split_batch<16, 1, 0, true>);
+        else if (sp.nch == 1) launch(k_gemv_q8_rows8_split_batch<32, 1, 0, true>);
+        else launch(k_gemv_q8_rows8_split_batch<32, 2, 0, true>);
         WD_LAUNCH_CHECK();
         i = j;
     }
