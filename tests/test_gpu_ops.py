@@ -250,6 +250,36 @@ def test_gemv_ragged_rows(g, oracle, t, shift):
             assert (o[rows:] == 7.0).all(), (rows, cols)
 
 
+# super-blocks around the passes of eight and the changes of the number of waves (8, 16, 32, 64), beyond what is staged (65),
+# groups around the end of the split kernel (1023 / 1024) and of one round of the grid (3072), fewer rows than a group
+IQ_SHAPES = [(7, 2048), (8, 256), (9, 512), (15, 1792), (8184, 768), (8185, 768), (8193, 256), (24584, 512), (8190, 2048), (8200, 2304), (8192, 4096), (8199, 5888),
+             (33, 2304), (12, 4096), (10, 4352), (17, 8192), (9, 8448), (21, 12288), (8, 16384), (9, 16640)]
+
+
+@pytest.mark.parametrize("shift", [0, 2])
+@pytest.mark.parametrize("t", [synth.IQ3_S, synth.IQ2_S])
+def test_gemv_iq_row_groups(g, oracle, t, shift):
+    """The same bits as the oracle for any row length, from any two-byte boundary; nothing next to the outputs is written."""
+    import torch
+    for rows, cols in IQ_SHAPES:
+        rng = synth.rng_for(SEED, 43, t, rows, cols)
+        w = synth.matrix(t, rng, rows, cols)
+        qs, d, _ = oracle.quantize_q8_K(rng.normal(0, 1, cols).astype(np.float32))
+        raw = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda")
+        raw[shift:shift + w.size] = torch.from_numpy(w.reshape(-1)).cuda()
+        dq, dd = g.dev(qs), g.dev(d)
+        out = torch.full((rows + 8,), 7.0, dtype=torch.float32, device="cuda")
+        out2, part = torch.full_like(out, 7.0), g.empty((rows, oracle.partials_per_row(t, cols)), np.int32)
+        for o, p in ((out, None), (out2, g.ptr(part))):
+            capi.call("wd_gemv_q8_k_f32", t, C.c_void_p(raw.data_ptr() + shift), rows, cols, g.ptr(dq), g.ptr(dd), g.ptr(o), p, g.stream())
+        g.sync()
+        want, wpart = oracle.gemv(t, w, rows, cols, qs, d, want_partials=True)
+        assert np.array_equal(g.host(part), wpart), (rows, cols)
+        for o in (out, out2):
+            assert g.same_bits(g.host(o)[:rows], want), (rows, cols)
+            assert (o[rows:] == 7.0).all(), (rows, cols)
+
+
 def test_q8_0_gemv_batch_of_ragged_rows(g, oracle):
     """Items of 81 blocks a row, one of them off its 16-byte boundary, in one launch: the bits of the oracle."""
     import torch

@@ -286,6 +286,238 @@ __global__ __launch_bounds__(256) void k_gemv_iq(MatSrc src, int rows, int cols,
     }
 }
 
+// ---- IQ3_S / IQ2_S x Q8_K, one matrix: eight rows at a time, one lane per (row, super-block) ------------------------
+// A lane decodes all eight 32-value blocks of one super-block and keeps the eight chunk sums over them in its registers
+// (integers: any order), which takes the exchange between the lanes of a super-block away that k_gemv_iq pays per row (seven
+// lane swaps and as many additions for eight super-blocks); the sums then go through LDS once, and lane (row, chunk) runs the
+// chain of its chunk over the super-blocks in order, eight rows at a time (the other form: sixteen instructions per row).
+// Eight rows are 8 nb blocks in a row, a whole number of 16-byte words; the words are fetched lane by lane (two-byte aligned
+// where the rows are) and the fields are picked out of LDS.  The activation is staged with a stride of 272 bytes per
+// super-block (eight of them at once fall on different banks).
+template <int TYPE>
+constexpr int kIqBlk = TYPE == 21 ? 110 : 82;
+constexpr int kIqActStride = 272;
+WD_DEV void iq_stage_activation(int8_t *aq, float *ad, const int8_t *act_qs, const float *act_d, int nb, int threads) {
+    for (int i = threadIdx.x; i < nb * 16; i += threads)
+        *reinterpret_cast<uint4 *>(aq + (i >> 4) * kIqActStride + (i & 15) * 16) = reinterpret_cast<const uint4 *>(act_qs)[i];
+    for (int i = threadIdx.x; i < nb; i += threads) ad[i] = act_d[i];
+}
+WD_DEV void iq_load_act(uint32_t (&a)[8], const int8_t *aq) {
+    const uint4 a0 = *reinterpret_cast<const uint4 *>(aq), a1 = *reinterpret_cast<const uint4 *>(aq + 16);
+    a[0] = a0.x, a[1] = a0.y, a[2] = a0.z, a[3] = a0.w, a[4] = a1.x, a[5] = a1.y, a[6] = a1.z, a[7] = a1.w;
+}
+// A super-block in registers: the dwords behind its scale, so that the fields of block ib are picked at compile time.
+template <int TYPE>
+struct IqBlockRegs {
+    static constexpr int kWords = (kIqBlk<TYPE> - 2) / 4;
+    uint32_t v[kWords];
+    float d;
+    // off: the block's (even) offset in the stage; up to four bytes behind the block are read
+    WD_DEV void load(const uint8_t *stage, uint32_t off) {
+        const uint32_t sh = (off + 2) & 2u;
+        const uint32_t *r = reinterpret_cast<const uint32_t *>(stage + (off + 2 - sh));
+        d = h2f(*reinterpret_cast<const uint16_t *>(stage + off));
+        uint32_t lo = r[0];
+#pragma unroll
+        for (int j = 0; j < kWords; ++j) {
+            const uint32_t hi = r[j + 1];
+            v[j] = __builtin_amdgcn_alignbyte(hi, lo, sh);
+            lo = hi;
+        }
+    }
+    WD_DEV IqFields fields(int ib) const {
+        IqFields f;
+        f.d = 0;
+        f.qh = v[16 + (ib >> 2)] >> (8 * (ib & 3));  // (of its bits above the eighth none is used)
+        if (TYPE == 21) {
+            f.qs = make_uint2(v[2 * ib], v[2 * ib + 1]);
+            f.sg = v[18 + ib];
+            f.sc = v[TYPE == 21 ? 26 : 0] >> (8 * (ib >> 1));
+        } else {
+            f.qs = make_uint2(v[ib], v[8 + ib]);
+            f.sg = 0;
+            f.sc = (v[18 + (ib >> 2)] >> (8 * (ib & 3))) & 0xffu;
+        }
+        return f;
+    }
+};
+constexpr int kIqTileRow = 72;                              // [row][super-block][chunk], rows padded (bank spread)
+constexpr int kIqTileWords = 8 * kIqTileRow;
+
+// Many rows: the waves of the grid take the groups of eight rows in turn, eight super-blocks at a time, one such chunk ahead in
+// registers.  Rows that are no whole number of chunks end with a chunk of their last eight super-blocks, of which the first
+// have been there already and get the scale zero; rows of fewer than eight are one chunk with idle lanes.  rows >= 8.
+// dynamic LDS: nb * kIqActStride, nb floats (rounded to 16 bytes), then per wave the stage, later the tile in the same place.
+template <int TYPE>
+constexpr int kIqWaveStage = 64 * kIqBlk<TYPE> + 16;
+template <int TYPE, bool PART>
+__global__ __launch_bounds__(256) void k_gemv_iq_rows8(const uint8_t *__restrict__ w, int rows, int nb, const int8_t *__restrict__ act_qs,
+                                                        const float *__restrict__ act_d, float *__restrict__ out, int32_t *__restrict__ partials) {
+    constexpr int kBlk = kIqBlk<TYPE>, kRowWords = 8 * kBlk / 16, kLoads = (8 * kRowWords + 63) / 64;
+    static_assert(kIqWaveStage<TYPE> >= (kIqTileWords + 64) * 4, "the tile lies where the stage was");
+    __shared__ IqTables tables;
+    extern __shared__ __align__(16) uint8_t iq_lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int8_t *aq = reinterpret_cast<int8_t *>(iq_lds);
+    float *ad = reinterpret_cast<float *>(iq_lds + nb * kIqActStride);
+    uint8_t *stage = iq_lds + nb * kIqActStride + ((nb * 4 + 15) & ~15) + wave * kIqWaveStage<TYPE>;
+    float *tile = reinterpret_cast<float *>(stage), *tile_d = tile + kIqTileWords;
+    const size_t rb = static_cast<size_t>(nb) * kBlk;
+    const int n_groups = (rows + 7) >> 3, n_waves = gridDim.x * 4, first = blockIdx.x * 4 + wave;
+    const int my_groups = first < n_groups ? (n_groups - first + n_waves - 1) / n_waves : 0;
+    const int nchunks = (nb + 7) >> 3, skipped = nb < 8 ? 0 : 8 * nchunks - nb;
+    const int row = lane >> 3, pos = lane & 7;
+    // (fewer than eight super-blocks: the eight rows are one run of words)
+    const int words = nb < 8 ? nb * kBlk / 2 : 8 * kRowWords;
+    uint32_t goff[kLoads], loff[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int u = min(i * 64 + lane, words - 1), r = u / kRowWords;
+        goff[i] = nb < 8 ? 16u * u : static_cast<uint32_t>(r * rb + 16 * (u - r * kRowWords));
+        loff[i] = 16u * u;
+    }
+    const uint32_t my_block = static_cast<uint32_t>((nb < 8 ? row * nb + min(pos, nb - 1) : 8 * row + pos) * kBlk);
+    int f_group = min(first, n_groups - 1), f_chunk = 0, fetched = 0;
+    const int items = my_groups * nchunks;
+    auto chunk_start = [&](int chunk) { return nb < 8 ? 0 : min(8 * chunk, nb - 8); };
+    uint4 f[kLoads];
+    auto fetch = [&]() {
+        // (a last group of fewer than eight rows is moved up to end with the matrix)
+        const uint8_t *p = uniform_ptr(w + static_cast<size_t>(min(8 * f_group, rows - 8)) * rb + static_cast<size_t>(chunk_start(f_chunk)) * kBlk);
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) f[i] = gld_u128(p + goff[i]);
+        if (++fetched < items) {  // (past the wave's last chunk the same one again, not used)
+            if (++f_chunk == nchunks) f_chunk = 0, f_group += n_waves;
+        }
+    };
+    fetch();
+    stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, 256);
+    iq_stage_activation(aq, ad, act_qs, act_d, nb, 256);
+    __syncthreads();
+    if (my_groups == 0) return;  // wave-uniform
+    float acc = 0.0f;
+    int group = first, chunk = 0;
+    for (int t = 0; t < items; ++t) {
+        wave_lds_fence();  // the previous chunk's tile has been read
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) *reinterpret_cast<uint4 *>(stage + loff[i]) = f[i];
+        wave_lds_fence();
+        fetch();
+        const int b0 = chunk_start(chunk), sb = min(b0 + pos, nb - 1);
+        const bool on = b0 + pos < nb && (chunk < nchunks - 1 || pos >= skipped);
+        const int out_row = min(8 * group, rows - 8) + row;
+        IqBlockRegs<TYPE> blk;
+        blk.load(stage, my_block);
+        int sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int ib = 0; ib < 8; ++ib) {
+            uint32_t a[8];
+            iq_load_act(a, aq + sb * kIqActStride + ib * 32);
+            int p[8];
+            iq_chunks<TYPE>(blk.fields(ib), ib, tables, a, p);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) sum[c] += p[c];
+        }
+        if (PART && on) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) partials[(static_cast<size_t>(out_row) * nb + sb) * 8 + c] = sum[c];
+        }
+        wave_lds_fence();  // every lane has its block in registers
+        float4 *dst = reinterpret_cast<float4 *>(tile + row * kIqTileRow + pos * 8);
+        dst[0] = make_float4(static_cast<float>(sum[0]), static_cast<float>(sum[1]), static_cast<float>(sum[2]), static_cast<float>(sum[3]));
+        dst[1] = make_float4(static_cast<float>(sum[4]), static_cast<float>(sum[5]), static_cast<float>(sum[6]), static_cast<float>(sum[7]));
+        tile_d[lane] = on ? blk.d * ad[sb] : 0.0f;
+        wave_lds_fence();
+#pragma unroll
+        for (int s = 0; s < 8; ++s) acc = __builtin_fmaf(tile_d[row * 8 + s], tile[row * kIqTileRow + s * 8 + pos], acc);
+        if (++chunk == nchunks) {
+            const float y = close_lanes8(acc);
+            if (pos == 0) out[out_row] = TYPE == 22 ? 0.125f * y : y;
+            acc = 0.0f, chunk = 0, group += n_waves;
+        }
+    }
+}
+
+// Few rows: one workgroup per group of eight rows, `parts` waves for every eight super-blocks, of which wave `part` takes the
+// 32-value blocks part, part + parts, ...; their chunk sums are added (integers) by the wave that runs the chains.
+// 64 * parts * ceil(nb / 8) threads, rows >= 8.  dynamic LDS: the activation as above, the rows (8 nb blocks and 16 bytes),
+// then a tile per wave.
+template <int TYPE>
+static size_t iq_split_lds(int nb, int parts) {
+    const int nchunks = (nb + 7) / 8;
+    return static_cast<size_t>(nb) * kIqActStride + ((nb * 4 + 15) & ~15) + ((static_cast<size_t>(8) * nb * kIqBlk<TYPE> + 31) & ~size_t(15)) +
+           static_cast<size_t>(nchunks) * (parts * kIqTileWords + 64) * 4;
+}
+template <int TYPE, bool PART>
+__global__ __launch_bounds__(512) void k_gemv_iq_split(const uint8_t *__restrict__ w, int rows, int nb, int parts, const int8_t *__restrict__ act_qs,
+                                                        const float *__restrict__ act_d, float *__restrict__ out, int32_t *__restrict__ partials) {
+    constexpr int kBlk = kIqBlk<TYPE>;
+    __shared__ IqTables tables;
+    extern __shared__ __align__(16) uint8_t iq_lds[];
+    const int threads = blockDim.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nchunks = (nb + 7) >> 3, chunk = wave / parts, part = wave - chunk * parts;
+    int8_t *aq = reinterpret_cast<int8_t *>(iq_lds);
+    float *ad = reinterpret_cast<float *>(iq_lds + nb * kIqActStride);
+    uint8_t *stage = iq_lds + nb * kIqActStride + ((nb * 4 + 15) & ~15);
+    int32_t *tiles = reinterpret_cast<int32_t *>(stage + ((8 * nb * kBlk + 31) & ~15));
+    float *scales = reinterpret_cast<float *>(tiles + nchunks * parts * kIqTileWords);
+    const int base_row = min(8 * static_cast<int>(blockIdx.x), rows - 8);
+    const uint8_t *src = uniform_ptr(w + static_cast<size_t>(base_row) * nb * kBlk);
+    const int words = nb * kBlk / 2;
+    // at most eight words per thread: nb 55 words over 64 ceil(nb / 8) threads or more
+    uint4 f[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (i * threads < words) f[i] = gld_u128(src + 16 * min(i * threads + static_cast<int>(threadIdx.x), words - 1));
+    stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, threads);
+    iq_stage_activation(aq, ad, act_qs, act_d, nb, threads);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (i * threads < words) reinterpret_cast<uint4 *>(stage)[min(i * threads + static_cast<int>(threadIdx.x), words - 1)] = f[i];
+    __syncthreads();
+    const int row = lane >> 3, pos = lane & 7;
+    {
+        const bool on = 8 * chunk + pos < nb;
+        const int sb = min(8 * chunk + pos, nb - 1);
+        const uint32_t off = static_cast<uint32_t>((row * nb + sb) * kBlk);
+        int sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int ib = part; ib < 8; ib += parts) {
+            const IqFields f_ib = iq_fields_shifted<TYPE>(stage + off, ib, (off + 2) & 2u);
+            uint32_t a[8];
+            iq_load_act(a, aq + sb * kIqActStride + ib * 32);
+            int p[8];
+            iq_chunks<TYPE>(f_ib, ib, tables, a, p);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) sum[c] += p[c];
+        }
+        int4 *dst = reinterpret_cast<int4 *>(tiles + wave * kIqTileWords + row * kIqTileRow + pos * 8);
+        dst[0] = make_int4(sum[0], sum[1], sum[2], sum[3]);
+        dst[1] = make_int4(sum[4], sum[5], sum[6], sum[7]);
+        if (part == 0) scales[64 * chunk + lane] = on ? h2f(*reinterpret_cast<const uint16_t *>(stage + off)) * ad[sb] : 0.0f;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float acc = 0.0f;
+    for (int ch = 0; ch < nchunks; ++ch) {
+        const int32_t *tile = tiles + ch * parts * kIqTileWords + row * kIqTileRow + pos;
+        float dv[8];
+        int pv[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) dv[s] = scales[64 * ch + 8 * row + s], pv[s] = tile[8 * s];
+        for (int q = 1; q < parts; ++q) {
+#pragma unroll
+            for (int s = 0; s < 8; ++s) pv[s] += tile[q * kIqTileWords + 8 * s];
+        }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            if (PART && 8 * ch + s < nb) partials[(static_cast<size_t>(base_row + row) * nb + 8 * ch + s) * 8 + pos] = pv[s];
+            acc = __builtin_fmaf(dv[s], static_cast<float>(pv[s]), acc);
+        }
+    }
+    const float y = close_lanes8(acc);
+    if (pos == 0) out[base_row + row] = TYPE == 22 ? 0.125f * y : y;
+}
+
 // ---- Q8_0 / IQ4_NL / Q4_0 x Q8_0 GEMV: 16 rows per workgroup, 4 per wave ----------------------
 // act_stride: elements between the activations of consecutive matrices (0 = one shared activation).
 template <int KIND, bool PART>

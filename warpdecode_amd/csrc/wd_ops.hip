@@ -199,6 +199,31 @@ int wd_topk_softmax(const float *d_logits, int n_experts, int k, float expert_sc
     return WD_OK;
 }
 
+}  // extern "C" (a template)
+// One IQ matrix of eight rows or more, whose rows fit LDS eight at a time; the activation 16-byte aligned.
+static bool iq_streams(int rows, int nb, const int8_t *qs) { return rows >= 8 && nb <= 64 && reinterpret_cast<uintptr_t>(qs) % 16 == 0; }
+template <int TYPE>
+static void launch_iq_stream(const uint8_t *w, int rows, int nb, const int8_t *qs, const float *d, float *out, int32_t *partials,
+                             hipStream_t stream) {
+    const int groups = (rows + 7) / 8, nchunks = (nb + 7) / 8;
+    if (groups < 1024) {
+        // fewer groups than SIMDs: up to eight waves share one
+        const int parts = nchunks <= 2 ? 4 : (nchunks <= 4 ? 2 : 1);
+        const size_t lds = iq_split_lds<TYPE>(nb, parts);
+        auto launch = [&](auto kernel) { kernel<<<groups, 64 * parts * nchunks, lds, stream>>>(w, rows, nb, parts, qs, d, out, partials); };
+        if (partials) launch(k_gemv_iq_split<TYPE, true>);
+        else launch(k_gemv_iq_split<TYPE, false>);
+        return;
+    }
+    // three workgroups of four waves are what LDS holds per compute unit
+    const unsigned wgs = static_cast<unsigned>(std::min((groups + 3) / 4, 768));
+    const size_t lds = static_cast<size_t>(nb) * kIqActStride + ((nb * 4 + 15) & ~15) + 4 * kIqWaveStage<TYPE>;
+    auto launch = [&](auto kernel) { kernel<<<wgs, 256, lds, stream>>>(w, rows, nb, qs, d, out, partials); };
+    if (partials) launch(k_gemv_iq_rows8<TYPE, true>);
+    else launch(k_gemv_iq_rows8<TYPE, false>);
+}
+extern "C" {
+
 // ---- GEMVs --------------------------------------------------------------------------------
 static int launch_gemv_q8k(int type, MatSrc src, int mats, int rows, int cols, const int8_t *qs, const float *d,
                            float *out, int32_t *partials, hipStream_t stream) {
@@ -207,6 +232,12 @@ static int launch_gemv_q8k(int type, MatSrc src, int mats, int rows, int cols, c
     WD_REQUIRE(rows > 0 && cols > 0 && cols % 256 == 0, "invalid low-bit matrix shape %d x %d", rows, cols);
     WD_REQUIRE(mats > 0 && mats <= 64, "expert batch must be in (0, 64] (got %d)", mats);
     WD_REQUIRE(qs && d && out, "low-bit GEMV: null pointer");
+    if (mats == 1 && src.single && iq_streams(rows, cols / 256, qs)) {
+        if (type == WD_TYPE_IQ3_S) launch_iq_stream<21>(src.single, rows, cols / 256, qs, d, out, partials, stream);
+        else launch_iq_stream<22>(src.single, rows, cols / 256, qs, d, out, partials, stream);
+        WD_LAUNCH_CHECK();
+        return WD_OK;
+    }
     const dim3 grid((rows + 15) / 16, mats), block(256);
     const int ppr = partials_per_row(type, cols);
     if (type == WD_TYPE_IQ3_S) {
