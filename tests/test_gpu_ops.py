@@ -280,6 +280,39 @@ def test_gemv_iq_row_groups(g, oracle, t, shift):
             assert (o[rows:] == 7.0).all(), (rows, cols)
 
 
+# blocks around the groups of eight, groups per row that do not divide a wave (3, 9, 33, 63), one and more rows per pass, the
+# ends of what streams (7 / 8 and 512 / 513 blocks; 63 / 64 blocks or 200000 in all), passes around 256 (two or four waves per
+# workgroup)
+Q4_SHAPES = [(40, 224), (25000, 256), (22223, 288), (11764, 544), (11765, 544), (8700, 736), (67, 2016), (61, 2080), (6, 2560), (1003, 2592),
+             (256, 8448), (257, 8448), (9, 16096), (3, 16352), (5, 16416)]
+
+
+@pytest.mark.parametrize("shift", [0, 2])
+def test_q4_0_gemv_ragged_rows(g, oracle, shift):
+    """Block sums exact, results within 1e-5 of the magnitude of their terms (a sum of n float32 terms in any order is off by less
+    than n 2^-24 of it, and n <= 513 terms are added eight to a lane and then in a tree: below 16 2^-24), no row next to them written."""
+    import torch
+    for rows, cols in Q4_SHAPES:
+        rng = synth.rng_for(SEED, 44, rows, cols)
+        w = synth.matrix(synth.Q4_0, rng, rows, cols)
+        qs, d = oracle.quantize_q8_0(rng.normal(0, 1, cols).astype(np.float32))
+        raw = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda")
+        raw[shift:shift + w.size] = torch.from_numpy(w.reshape(-1)).cuda()
+        dq, dd = g.dev(qs), g.dev(d)
+        out = torch.full((rows + 64,), 7.0, dtype=torch.float32, device="cuda")
+        out2, part = torch.full_like(out, 7.0), g.empty((rows, cols // 32), np.int32)
+        for o, p in ((out, None), (out2, g.ptr(part))):
+            capi.call("wd_gemv_q8_0_f32", synth.Q4_0, C.c_void_p(raw.data_ptr() + shift), rows, cols, g.ptr(dq), g.ptr(dd), g.ptr(o), p, g.stream())
+        g.sync()
+        want, wpart = oracle.gemv(synth.Q4_0, w, rows, cols, qs, d, want_partials=True)
+        assert np.array_equal(g.host(part), wpart), (rows, cols)
+        wd = np.stack([oracle.dequant_row(synth.Q4_0, w[r], cols) for r in range(rows)]).astype(np.float64)
+        mag = np.abs(wd) @ np.abs(qs.astype(np.float64) * np.repeat(d.view(np.float16).astype(np.float64), 32))
+        for o in (out, out2):
+            assert (np.abs(g.host(o)[:rows] - want) <= 1e-5 * mag).all(), (rows, cols)
+            assert (o[rows:] == 7.0).all(), (rows, cols)
+
+
 def test_q8_0_gemv_batch_of_ragged_rows(g, oracle):
     """Items of 81 blocks a row, one of them off its 16-byte boundary, in one launch: the bits of the oracle."""
     import torch

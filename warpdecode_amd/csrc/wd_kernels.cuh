@@ -556,20 +556,26 @@ __global__ __launch_bounds__(256) void k_gemv_q8(MatSrc src, int rows, int cols,
 // float and 8 * sum(a) beside it; Block sums are exact; the float side adds a lane's
 // eight blocks in order and folds the row's lanes with an xor tree (Q4_0 has no canonical float order).
 // A wave takes NP consecutive passes and requests all of them before it touches the first.
-// grid.x * WPB waves * NP passes cover ceil(rows / (64 / lpr)) passes.
-// dynamic LDS: lpr * 272 bytes of quants, then nb floats, then nb ints.
+// RAGGED: any row of eight blocks or more and 64 groups or fewer, on any two-byte boundary.  A row is lpr = ceil(nb / 8) groups
+// of which the last holds the row's LAST eight blocks (those that the group before has as well get the scale zero), a pass is
+// floor(64 / lpr) rows, and the words are fetched group by group.  The sum of a row's lanes is the same tree over any lpr.
+// grid.x * WPB waves * NP passes cover ceil(rows / floor(64 / lpr)) passes.
+// dynamic LDS: lpr * 272 bytes of quants, then 8 lpr floats, then 8 lpr ints.
 // (the body: `block` is the workgroup's number among those of its matrix)
-template <bool PART, int NP, int WPB>
+template <bool PART, int NP, int WPB, bool RAGGED>
 WD_DEV void gemv_q4_stream_body(const uint8_t *__restrict__ w, int rows, int nb, const int8_t *__restrict__ act_qs,
                                 const uint16_t *__restrict__ act_d, float *__restrict__ out, int32_t *__restrict__ partials,
                                 int block) {
     __shared__ uint4 stage[WPB][9 * 64];
     extern __shared__ __align__(16) uint8_t q4_act[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lpr = nb >> 3, lpr_shift = __builtin_ctz(lpr), rpp = 64 >> lpr_shift;
-    const int col = lane & (lpr - 1), rsub = lane >> lpr_shift;
+    const int lpr = (nb + 7) >> 3, lpr_shift = __builtin_ctz(lpr), rpp = RAGGED ? 64 / lpr : 64 >> lpr_shift;
+    const int inv = (65535 + lpr) / lpr;  // n / lpr = n inv / 65536 for the n below 64 that are divided here
+    const int rsub = RAGGED ? (lane * inv) >> 16 : lane >> lpr_shift, col = RAGGED ? lane - rsub * lpr : lane & (lpr - 1);
+    const bool last_group = RAGGED && col == lpr - 1;
+    const int skip = last_group ? 8 * lpr - nb : 0, first_block = last_group ? nb - 8 : 8 * col;
     float *ad = reinterpret_cast<float *>(q4_act + lpr * 272);
-    int *corr = reinterpret_cast<int *>(ad + nb);
+    int *corr = reinterpret_cast<int *>(ad + 8 * lpr);
     const size_t rb = static_cast<size_t>(nb) * 18;
     const long long pass0 = (static_cast<long long>(block) * WPB + wave) * NP;
     uint4 v[NP][9];
@@ -580,24 +586,31 @@ WD_DEV void gemv_q4_stream_body(const uint8_t *__restrict__ w, int rows, int nb,
         const uint8_t *base = w + static_cast<size_t>(row0) * rb;
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
-            const size_t off = static_cast<size_t>(k) * 1024 + static_cast<size_t>(lane) * 16;
-            v[slot][k] = off < valid ? gld_u128_aligned(base + off) : make_uint4(0, 0, 0, 0);
+            if constexpr (RAGGED) {
+                const int word = k * 64 + lane, group = word / 9, r = (group * inv) >> 16, g = group - r * lpr;
+                const size_t off = r * rb + (g == lpr - 1 ? rb - 144 : static_cast<size_t>(g) * 144) + 16 * (word - 9 * group);
+                v[slot][k] = r < rpp && off < valid ? gld_u128(base + off) : make_uint4(0, 0, 0, 0);
+            } else {
+                const size_t off = static_cast<size_t>(k) * 1024 + static_cast<size_t>(lane) * 16;
+                v[slot][k] = off < valid ? gld_u128_aligned(base + off) : make_uint4(0, 0, 0, 0);
+            }
         }
     };
     // activation into LDS: thread t takes 16-byte pieces t, t + blockDim.x, ...; a block's two pieces give its sum.  The
     // first piece is requested before the weights so that it can be consumed while they are still in flight.
-    const int n_pieces = nb * 2;
+    const int n_pieces = lpr * 16;
+    auto block_of = [&](int i) { return RAGGED && (i >> 4) == lpr - 1 ? nb - 8 + ((i & 15) >> 1) : i >> 1; };  // of piece i
     uint4 q0 = make_uint4(0, 0, 0, 0);
     uint16_t d0 = 0;
     if (static_cast<int>(threadIdx.x) < n_pieces) {
-        q0 = *reinterpret_cast<const uint4 *>(act_qs + threadIdx.x * 16);
-        d0 = act_d[threadIdx.x >> 1];
+        q0 = *reinterpret_cast<const uint4 *>(act_qs + block_of(threadIdx.x) * 32 + (threadIdx.x & 1) * 16);
+        d0 = act_d[block_of(threadIdx.x)];
     }
 #pragma unroll
     for (int p = 0; p < NP; ++p) fetch(pass0 + p, p);
     for (int i = threadIdx.x; i < n_pieces; i += WPB * 64) {
         const bool first = i == static_cast<int>(threadIdx.x);
-        const uint4 q = first ? q0 : *reinterpret_cast<const uint4 *>(act_qs + i * 16);
+        const uint4 q = first ? q0 : *reinterpret_cast<const uint4 *>(act_qs + block_of(i) * 32 + (i & 1) * 16);
         *reinterpret_cast<uint4 *>(q4_act + (i >> 4) * 272 + (i & 15) * 16) = q;
         int s = sdot4(0x01010101u, q.x, 0);
         s = sdot4(0x01010101u, q.y, s);
@@ -606,7 +619,7 @@ WD_DEV void gemv_q4_stream_body(const uint8_t *__restrict__ w, int rows, int nb,
         s += lane_xor(s, 1);
         if ((i & 1) == 0) {
             corr[i >> 1] = 8 * s;
-            ad[i >> 1] = h2f(first ? d0 : act_d[i >> 1]);
+            ad[i >> 1] = h2f(first ? d0 : act_d[block_of(i)]);
         }
     }
     __syncthreads();
@@ -626,6 +639,7 @@ WD_DEV void gemv_q4_stream_body(const uint8_t *__restrict__ w, int rows, int nb,
         }
         wave_lds_fence();
         const int row = static_cast<int>(row0) + rsub;
+        const bool on = row < rows && (!RAGGED || rsub < rpp);
         float sumf = 0.0f;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -648,19 +662,28 @@ WD_DEV void gemv_q4_stream_body(const uint8_t *__restrict__ w, int rows, int nb,
                 sumi = sdot4(n[l] & 0x0f0f0f0fu, al[l], sumi);
                 sumi = sdot4((n[l] >> 4) & 0x0f0f0f0fu, ah[l], sumi);
             }
-            if (PART && row < rows) partials[static_cast<size_t>(row) * nb + col * 8 + j] = sumi;
-            sumf += h2f(static_cast<uint16_t>(dw)) * ad[col * 8 + j] * static_cast<float>(sumi);
+            if (PART && on && j >= skip) partials[static_cast<size_t>(row) * nb + first_block + j] = sumi;
+            const float term = h2f(static_cast<uint16_t>(dw)) * ad[col * 8 + j] * static_cast<float>(sumi);
+            sumf += RAGGED && j < skip ? 0.0f : term;
         }
-        for (int mask = lpr >> 1; mask >= 1; mask >>= 1) sumf += lane_xor(sumf, mask);
-        if (col == 0 && row < rows) out[row] = sumf;
+        if constexpr (RAGGED) {
+#pragma unroll
+            for (int off = 32; off >= 1; off >>= 1) {
+                const float other = __shfl_down(sumf, off, 64);
+                if (col + off < lpr && col < off) sumf += other;
+            }
+        } else {
+            for (int mask = lpr >> 1; mask >= 1; mask >>= 1) sumf += lane_xor(sumf, mask);
+        }
+        if (col == 0 && on) out[row] = sumf;
     }
 }
-template <bool PART, int NP, int WPB>
+template <bool PART, int NP, int WPB, bool RAGGED>
 __global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream(const uint8_t *__restrict__ w, int rows, int nb,
                                                          const int8_t *__restrict__ act_qs,
                                                          const uint16_t *__restrict__ act_d, float *__restrict__ out,
                                                          int32_t *__restrict__ partials) {
-    gemv_q4_stream_body<PART, NP, WPB>(w, rows, nb, act_qs, act_d, out, partials, static_cast<int>(blockIdx.x));
+    gemv_q4_stream_body<PART, NP, WPB, RAGGED>(w, rows, nb, act_qs, act_d, out, partials, static_cast<int>(blockIdx.x));
 }
 // Several matrices of one row length in one launch (see k_gemv_q8_rows8_split_batch): workgroup b belongs to the item
 // whose range of workgroups holds b and does there what k_gemv_q4_stream does for that item alone.
@@ -680,10 +703,10 @@ WD_DEV int gemv_batch_item(const GemvBatch &b) {
         if (static_cast<int>(blockIdx.x) >= b.first_group[i]) item = i;
     return __builtin_amdgcn_readfirstlane(item);
 }
-template <int WPB>
+template <int WPB, bool RAGGED>
 __global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream_batch(GemvBatch b, int nb) {
     const int item = gemv_batch_item(b);
-    gemv_q4_stream_body<false, 1, WPB>(b.w[item], b.rows[item], nb, b.act_qs[item], b.act_d[item], b.out[item], nullptr,
+    gemv_q4_stream_body<false, 1, WPB, RAGGED>(b.w[item], b.rows[item], nb, b.act_qs[item], b.act_d[item], b.out[item], nullptr,
                                        static_cast<int>(blockIdx.x) - b.first_group[item]);
 }
 

@@ -343,6 +343,24 @@ static void launch_q8_stream(const uint8_t *w, int rows, int nb, const int8_t *q
 
 extern "C" {
 
+// ---- Q4_0: the streaming kernel takes rows of 8 to 512 blocks, aligned activations -------------------------------------
+// Rows that are no whole groups of eight blocks, groups that do not divide a wave, or a matrix off 16-byte boundaries.
+static bool q4_ragged(const uint8_t *w, int nb) { return nb % 8 != 0 || 64 % (nb / 8) != 0 || reinterpret_cast<uintptr_t>(w) % 16 != 0; }
+// Ragged ones only where the rows are long or the matrix is large: below, the general kernel, which stages nothing, ends sooner
+// (us, general / streaming: 640 x 800 2.3 / 3.5, 520 x 1600 3.3 / 3.7, 9000 x 544 3.7 / 4.2; 2560 x 2560 4.5 / 4.1, 3000 x 2592
+// 4.9 / 4.2, 5000 x 5120 9.6 / 7.1, 2048 x 12288 16.7 / 7.2, 100000 x 1056 22.5 / 16.0).
+static bool q4_streams(const uint8_t *w, int rows, int nb, const int8_t *qs) {
+    if (q4_ragged(w, nb < 8 ? 8 : nb) && nb < 64 && static_cast<long long>(rows) * nb < 200000) return false;
+    return nb >= 8 && nb <= 512 && reinterpret_cast<uintptr_t>(qs) % 16 == 0;
+}
+// Its workgroups (waves per workgroup in *wpb): four waves stream best; two when the whole matrix is only a few hundred passes.
+static long long q4_stream_wgs(int rows, int nb, int *wpb) {
+    const int rpp = 64 / ((nb + 7) / 8);
+    const long long passes = (static_cast<long long>(rows) + rpp - 1) / rpp;
+    *wpb = passes <= 256 ? 2 : 4;
+    return (passes + *wpb - 1) / *wpb;
+}
+
 static int launch_gemv_q8_0(int type, MatSrc src, int mats, int rows, int cols, const int8_t *qs, const uint16_t *d,
                             int act_per_mat, float *out, int32_t *partials, hipStream_t stream) {
     WD_REQUIRE(type == WD_TYPE_Q8_0 || type == WD_TYPE_IQ4_NL || type == WD_TYPE_Q4_0,
@@ -354,27 +372,20 @@ static int launch_gemv_q8_0(int type, MatSrc src, int mats, int rows, int cols, 
     const int ppr = partials_per_row(type, cols);
     const int act_stride = act_per_mat ? cols : 0;
     const int nb = cols / 32;
-    if (type == WD_TYPE_Q4_0 && mats == 1 && src.single && nb % 8 == 0 && nb / 8 <= 64 && 64 % (nb / 8) == 0 &&
-        reinterpret_cast<uintptr_t>(src.single) % 16 == 0 && reinterpret_cast<uintptr_t>(qs) % 16 == 0) {
-        // whole 8-block groups per row and a 16-byte aligned base: the streaming kernel
-        const int rpp = 64 / (nb / 8);
-        const long long passes = (static_cast<long long>(rows) + rpp - 1) / rpp;
-        // four waves per workgroup stream best; two when the whole matrix is only a few hundred passes
-        const int wpb = passes <= 256 ? 2 : 4;
-        const unsigned wgs = static_cast<unsigned>((passes + wpb - 1) / wpb);
-        const size_t lds = static_cast<size_t>(nb / 8) * 272 + static_cast<size_t>(nb) * 8;
-#define WD_Q4S_LAUNCH(WPB)                                                                                              \
-    do {                                                                                                                \
-        if (partials)                                                                                                   \
-            k_gemv_q4_stream<true, 1, WPB><<<wgs, WPB * 64, lds, stream>>>(src.single, rows, nb, qs, d, out, partials); \
-        else                                                                                                            \
-            k_gemv_q4_stream<false, 1, WPB><<<wgs, WPB * 64, lds, stream>>>(src.single, rows, nb, qs, d, out, nullptr); \
-    } while (0)
-        if (wpb == 2)
-            WD_Q4S_LAUNCH(2);
-        else
-            WD_Q4S_LAUNCH(4);
-#undef WD_Q4S_LAUNCH
+    if (type == WD_TYPE_Q4_0 && mats == 1 && src.single && q4_streams(src.single, rows, nb, qs)) {
+        const int lpr = (nb + 7) / 8;
+        const bool ragged = q4_ragged(src.single, nb);
+        int wpb = 0;
+        const unsigned wgs = static_cast<unsigned>(q4_stream_wgs(rows, nb, &wpb));
+        const size_t lds = static_cast<size_t>(lpr) * (272 + 64);
+        auto launch = [&](auto kernel) { kernel<<<wgs, wpb * 64, lds, stream>>>(src.single, rows, nb, qs, d, out, partials); };
+        if (partials) {
+            if (wpb == 2) ragged ? launch(k_gemv_q4_stream<true, 1, 2, true>) : launch(k_gemv_q4_stream<true, 1, 2, false>);
+            else ragged ? launch(k_gemv_q4_stream<true, 1, 4, true>) : launch(k_gemv_q4_stream<true, 1, 4, false>);
+        } else {
+            if (wpb == 2) ragged ? launch(k_gemv_q4_stream<false, 1, 2, true>) : launch(k_gemv_q4_stream<false, 1, 2, false>);
+            else ragged ? launch(k_gemv_q4_stream<false, 1, 4, true>) : launch(k_gemv_q4_stream<false, 1, 4, false>);
+        }
         WD_LAUNCH_CHECK();
         return WD_OK;
     }
@@ -449,16 +460,10 @@ int wd_gemv_q8_0_f32(int type, const uint8_t *d_w, int rows, int cols, const int
     return launch_gemv_q8_0(type, src, 1, rows, cols, d_act_qs, d_act_scales, 0, d_out, d_partials, as_stream(stream));
 }
 
-// Q4_0 matrices: the workgroups per item of the streaming kernel (waves per workgroup in *wpb), 0 when the item takes
-// another kernel alone.
-static int q4_stream_wgs(const wd_gemv_item &it, int nb, int *wpb) {
-    if (!(nb % 8 == 0 && nb / 8 <= 64 && 64 % (nb / 8) == 0 && reinterpret_cast<uintptr_t>(it.d_w) % 16 == 0 &&
-          reinterpret_cast<uintptr_t>(it.d_act_qs) % 16 == 0))
-        return 0;
-    const int rpp = 64 / (nb / 8);
-    const long long passes = (static_cast<long long>(it.rows) + rpp - 1) / rpp;
-    *wpb = passes <= 256 ? 2 : 4;
-    const long long wgs = (passes + *wpb - 1) / *wpb;
+// The workgroups of an item of a Q4_0 batch, 0 when the item is launched by itself.
+static int q4_batch_wgs(const wd_gemv_item &it, int nb, int *wpb) {
+    if (!q4_streams(it.d_w, it.rows, nb, it.d_act_qs)) return 0;
+    const long long wgs = q4_stream_wgs(it.rows, nb, wpb);
     return wgs <= 4096 ? static_cast<int>(wgs) : 0;  // (large matrices are not bound by their launch)
 }
 static int gemv_q4_0_batch(const wd_gemv_item *items, int n_items, int cols, void *stream) {
@@ -466,10 +471,10 @@ static int gemv_q4_0_batch(const wd_gemv_item *items, int n_items, int cols, voi
     int i = 0;
     while (i < n_items) {
         int wpb = 0, other = 0;
-        const int wgs0 = q4_stream_wgs(items[i], nb, &wpb);
+        const int wgs0 = q4_batch_wgs(items[i], nb, &wpb);
         int j = i + 1;
         if (wgs0)
-            while (j < n_items && j - i < kGemvBatchMax && q4_stream_wgs(items[j], nb, &other) && other == wpb) ++j;
+            while (j < n_items && j - i < kGemvBatchMax && q4_batch_wgs(items[j], nb, &other) && other == wpb) ++j;
         if (!wgs0 || j - i == 1) {
             if (const int rc = wd_gemv_q8_0_f32(WD_TYPE_Q4_0, items[i].d_w, items[i].rows, cols, items[i].d_act_qs, items[i].d_act_scales,
                                                 items[i].d_out, nullptr, stream))
@@ -480,18 +485,19 @@ static int gemv_q4_0_batch(const wd_gemv_item *items, int n_items, int cols, voi
         GemvBatch b{};
         b.n = j - i;
         int wgs = 0;
+        bool ragged = false;
         for (int q = 0; q < b.n; ++q) {
             const wd_gemv_item &it = items[i + q];
             b.w[q] = it.d_w, b.act_qs[q] = it.d_act_qs, b.act_d[q] = it.d_act_scales, b.out[q] = it.d_out, b.rows[q] = it.rows;
             b.first_group[q] = wgs;
-            wgs += q4_stream_wgs(it, nb, &other);
+            ragged = ragged || q4_ragged(it.d_w, nb);
+            wgs += q4_batch_wgs(it, nb, &other);
         }
         for (int q = b.n; q <= kGemvBatchMax; ++q) b.first_group[q] = wgs;
-        const size_t lds = static_cast<size_t>(nb / 8) * 272 + static_cast<size_t>(nb) * 8;
-        if (wpb == 2)
-            k_gemv_q4_stream_batch<2><<<wgs, 128, lds, as_stream(stream)>>>(b, nb);
-        else
-            k_gemv_q4_stream_batch<4><<<wgs, 256, lds, as_stream(stream)>>>(b, nb);
+        const size_t lds = static_cast<size_t>((nb + 7) / 8) * (272 + 64);
+        auto launch = [&](auto kernel) { kernel<<<wgs, wpb * 64, lds, as_stream(stream)>>>(b, nb); };
+        if (wpb == 2) ragged ? launch(k_gemv_q4_stream_batch<2, true>) : launch(k_gemv_q4_stream_batch<2, false>);
+        else ragged ? launch(k_gemv_q4_stream_batch<4, true>) : launch(k_gemv_q4_stream_batch<4, false>);
         WD_LAUNCH_CHECK();
         i = j;
     }
