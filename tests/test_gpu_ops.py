@@ -94,6 +94,19 @@ def test_topk_softmax(g, oracle, n, k):
             assert g.same_bits(g.host(wts), ow)
 
 
+@pytest.mark.parametrize("n", [64, 128, 256, 512])
+def test_topk_near_tie_at_the_end_of_a_key_cell(g, oracle, n):
+    from test_selection_margin import near_tie_row
+    logits = near_tie_row(n)
+    ids, wts = g.empty(6, np.int32), g.empty(6, np.float32)
+    dl = g.dev(logits)
+    capi.call("wd_topk_softmax", g.ptr(dl), n, 6, 1.0, g.ptr(ids), g.ptr(wts), g.stream())
+    g.sync()
+    oi, ow = oracle.route(logits, 6, 1.0)
+    assert oi[-1] == 30
+    assert np.array_equal(g.host(ids), oi) and g.same_bits(g.host(wts), ow)
+
+
 def _quant_act(oracle, t, x):
     if t in (synth.IQ3_S, synth.IQ2_S):
         qs, d, _ = oracle.quantize_q8_K(x)

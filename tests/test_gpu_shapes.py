@@ -41,6 +41,36 @@ def test_layer_shapes(g, oracle, H, F, E, k, gate, down, shared):
     check_layer(g, oracle, L, x, ids=ids, weights=np.linspace(0.3, 0.05, k).astype(np.float32), flags=1)
 
 
+@pytest.mark.parametrize("H,F,E", [(256, 32, 64), (256, 32, 128), (256, 32, 256), (256, 32, 512), (2048, 512, 64)])
+def test_near_tie_at_the_end_of_a_key_cell(g, oracle, H, F, E):
+    """Router rows whose logits are the near-tie row: the layer, a token batch and a stack of one layer (one launch at
+    2048 / 512) take the expert with the lower id of two equal probabilities."""
+    import ctypes as C
+
+    from test_selection_margin import near_tie_row
+    from warpdecode_amd import capi
+    k, T = 6, 2
+    L = synth.make_layer(H, F, E, k, IQ3, Q8, True, seed=SEED, layer=E, router_sigma=1.0)
+    L["router"] = np.ascontiguousarray(L["router"], np.float32).reshape(E, H).copy()
+    L["router"][:, 0] = near_tie_row(E)
+    x = np.zeros(H, np.float32)
+    x[0] = 1.0
+    got = check_layer(g, oracle, L, x)
+    assert got["ids"][-1] == 30
+    want, _ = oracle.moe_layer(L, x)
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    dx, out = g.dev(np.stack([x] * T)), g.empty((T, H), np.float32)
+    capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, (C.c_void_p * T)(*[s.h.value for s in scr]), 0, g.stream())
+    g.sync()
+    assert all(g.same_bits(g.host(out)[t], want) for t in range(T))
+    dx, out = g.dev(x), g.empty(H, np.float32)
+    capi.call("wd_moe_stack_f32", (capi.MoeLayer * 1)(dl.desc), 1, g.ptr(dx), g.ptr(out), scr[0].h, None, 0.05, 0, g.stream())
+    g.sync()
+    assert g.same_bits(g.host(out), want)
+    for s in scr:
+        s.close()
+
+
 @pytest.mark.parametrize("H,F,k", [(2048, 512, 16), (2560, 640, 4), (3072, 96, 3)])
 def test_tensors_on_two_byte_boundaries(g, oracle, monkeypatch, H, F, k):
     import torch

@@ -38,3 +38,63 @@ def test_without_the_margin_the_order_can_collapse():
     e_a = np.nextafter(e_b, np.float32(np.inf))
     inv = (1.0 / rng.uniform(1.0, 1024.0, e_b.size)).astype(np.float32)
     assert np.any((e_a * inv).astype(np.float32) == (e_b * inv).astype(np.float32))
+
+
+# ---- the one-wave selection: keys of 23 bits ------------------------------------------------------------------------
+def step_a(oracle, logits, k, cell_top=True):
+    """The device's first step restated for one row: (accepted, ids).  Keys are the logits' bits in float order with the
+    low nine replaced by 511 - expert; cell_top: the (k+1)-th exponential is that of the top of its key's cell."""
+    b = logits.view(np.uint32)
+    order = np.where(b >> 31, ~b, b ^ np.uint32(0x80000000)).astype(np.uint32)
+    key = (order & np.uint32(0xFFFFFE00)) | (511 - np.arange(logits.size)).astype(np.uint32)
+    taken = np.argsort(key)[::-1][:k + 1]
+    l = logits[taken].copy()
+    if cell_top:
+        top = key[taken[k]] | np.uint32(0x1FF)
+        l[k] = np.array([top ^ np.uint32(0x80000000) if top >> 31 else ~top], np.uint32).view(np.float32)[0]
+    e = oracle.exp_ggml((l - logits.max()).astype(np.float32))
+    margin = np.full(k, 1.000001, np.float32)
+    margin[k - 1] = 1.000004
+    grid = key[taken] >> 9
+    ok = np.all(grid[:-1] > grid[1:]) and np.all(e[:-1] >= FLOOR) and np.all(e[:-1] > (e[1:] * margin).astype(np.float32))
+    return bool(ok), taken[:k]
+
+
+def near_tie_row(n=64):
+    """Five clear winners; then the first float of a cell (id 40), the last of the cell below (id 30: the same
+    probability, and the lower id) and a float low in that cell (id 20: a higher key than id 30's).  Top-6 takes id 30."""
+    l = np.linspace(-3.0, -0.5, n).astype(np.float32)
+    l[[3, 9, 17, 33, 50]] = np.array([4.0, 3.5, 3.0, 2.5, 2.0], np.float32)
+    l[[40, 30, 20]] = [np.float32(float.fromhex(v)) for v in ("0x1.3d74p-1", "0x1.3d73fep-1", "0x1.3d700ap-1")]
+    return l
+
+
+def test_a_logit_left_out_of_the_last_cell_is_not_forgotten(oracle):
+    l, k = near_tie_row(), 6
+    want, _ = oracle.route(l, k)
+    p = oracle.softmax_row(l)
+    assert p[40] == p[30] and want[-1] == 30
+    accepted, ids = step_a(oracle, l, k, cell_top=False)
+    assert accepted and ids[-1] == 40     # negative control: by the (k+1)-th logit itself the row passes with the wrong id
+    accepted, ids = step_a(oracle, l, k)
+    assert not accepted                   # the row takes the rungs over the probabilities
+
+
+def test_accepted_rows_are_the_selection(oracle):
+    """Rows whose k-th and later logits crowd around the end of a cell, of either sign and several magnitudes."""
+    rng = np.random.default_rng(20261202)
+    accepted = 0
+    for trial in range(3000):
+        n, k = (64, 6) if trial % 2 else (128, 10)
+        l = rng.normal(-6.0, 0.5, n).astype(np.float32)
+        where = rng.permutation(n)
+        l[where[:k - 1]] = (4.0 + np.arange(k - 1)).astype(np.float32)
+        edge = np.array([np.float32(rng.choice([-1.0, 1.0]) * 2.0 ** rng.uniform(-5, 1.5))]).view(np.uint32)[0] & np.uint32(0xFFFFFE00)
+        crowd = where[k - 1:k + 3]
+        reach = int(rng.choice([4, 64, 600, 3000]))   # units in the last place around the end of the cell
+        l[crowd] = (edge + rng.integers(-reach, reach, crowd.size)).astype(np.uint32).view(np.float32)
+        ok, ids = step_a(oracle, l, k)
+        if ok:
+            accepted += 1
+            assert np.array_equal(ids, oracle.route(l, k)[0]), (trial, l[crowd])
+    assert accepted > 300

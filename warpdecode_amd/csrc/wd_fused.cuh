@@ -530,17 +530,18 @@ WD_DEV void topk_wave(const float *logits, int n, int k, float w_scale, int32_t 
 // The keys order the logits up to their low nine bits, so the result is accepted as the selection only when
 //   * the keys' upper 23 bits are strictly decreasing over the k + 1 - any logit that was not taken then lies below
 //     the grid point at or below the k-th taken logit -, and
-//   * the exponentials e_0 > e_1 > ... > e_k of the k + 1 exact logits are strictly decreasing by a relative margin:
-//     exp_ggml is within two units in the last place of the true exponential (relative error below 2^-22) on normal
-//     results, so every logit not above the (k+1)-th has an exponential below e_k (1 + 2^-21), and
-//     e_(k-1) > e_k (1 + 2^-18) puts the k-th selected strictly above everything left, also after the product with the
-//     row's 1/sum has been rounded.
+//   * the exponentials e_0 > e_1 > ... > e_(k-1) of the k taken logits and e_k, that of the top of the (k+1)-th key's cell
+//     (its low nine bits set: a logit that was not taken may lie above the (k+1)-th key's own, but not above its cell),
+//     are strictly decreasing by a relative margin: exp_ggml is within two units in the last place of the true
+//     exponential (relative error below 2^-22) on normal results, so every logit that was not taken has an exponential
+//     below e_k (1 + 2^-21), and e_(k-1) > e_k (1 + 2^-18) puts the k-th selected strictly above everything left, also
+//     after the product with the row's 1/sum has been rounded.
 // Rows the test does not accept (ties, near-ties, NaN, +inf, fewer than k + 1 finite logits, selected exponentials below
 // 2^-100) take the reference's rungs over all probabilities in step B.
 struct SelWaveState {
     float mx;      // the row's largest logit
-    float e;       // lane j <= k: exponential of the j-th largest logit (accepted rows)
-    int id;        // lane j <= k: its expert
+    float e;       // lane j < k: exponential of the j-th largest logit (accepted rows)
+    int id;        // lane j < k: its expert
     bool fast;     // step A accepted the row (the same in every lane)
 };
 
@@ -585,13 +586,15 @@ WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s
     wave_lds_fence();
     const uint32_t key = lane < count ? ck[lane] : 0u;
     const float key_l = s.cl[lane];
+    const uint32_t top = key | 0x1ffu;  // of the key's cell (mapped back here, ahead of the ranks that decide who needs it)
+    const float cell = bits_f(top & 0x80000000u ? top ^ 0x80000000u : ~top);
     int rank = 0;
     const int steps = (min(count, 64) + 3) & ~3;  // lanes past the list hold zero, which is ahead of nothing
     for (int src = 0; src < steps; src += 4) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) rank += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), src + u)) > key ? 1 : 0;
     }
-    if (key != 0u && rank <= k) s.sel[rank] = static_cast<int>(key), s.selp[rank] = key_l;
+    if (key != 0u && rank <= k) s.sel[rank] = static_cast<int>(key), s.selp[rank] = rank == k ? cell : key_l;
     wave_lds_fence();
     const uint32_t mine = lane <= k && lane < count ? static_cast<uint32_t>(s.sel[lane & 15]) : 0u;  // lane j: the j-th largest key of the row
     const int idc = 511 - static_cast<int>(mine & 0x1ffu);
