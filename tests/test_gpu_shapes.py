@@ -27,6 +27,13 @@ SHAPES = [
     (3328, 160, 200, 7, Q8, Q8, True),       # five down blocks
     (4096, 1056, 24, 3, IQ2, Q8, True),      # sixteen super-blocks, 33 down blocks
     (4352, 64, 520, 2, IQ3, Q8, True),       # beyond the aligned fetch and the paired router rows
+    (4352, 1024, 8, 6, IQ3, Q8, True),       # rows taken field by field, in a loop: of every type
+    (4352, 1024, 8, 7, IQ2, IQ4, False),
+    (4608, 1024, 8, 6, Q8, Q8, True),
+    (4352, 1024, 8, 6, IQ4, IQ4, True),
+    (4352, 544, 8, 4, Q8, IQ4, False),       # field by field, an item per workgroup
+    (4352, 96, 16, 5, IQ2, Q8, True),
+    (4608, 64, 8, 3, IQ4, Q8, True),
     (1024, 96, 128, 15, IQ4, Q8, True),      # the largest selection of one wave
     (3072, 1536, 16, 16, IQ3, IQ4, True),    # items beyond the device, 17 matrices
 ]

@@ -956,8 +956,13 @@ __host__ __device__ inline uint32_t layer_ab_stage_bytes(int H) {  // per wave
     return 2 * iq_cover_bytes<TYPE>(H >> 8);
 }
 
+// Workgroups per compute unit: three.  (Two for the rows taken field by field: Q8_0, hidden 5120 / ffn 1024, top-8 and the shared
+// expert 49.5 us against 40.6; IQ4_NL 43.7 against 36.4; IQ2_S 35.7 against 30.6.)  The loop over IQ3_S rows taken field by field
+// does not fit 80 registers - 22 are spilled - and runs two (hidden 4096 / ffn 1536, top-8: 32.5 us against 44.9).
+template <int TYPE, int FETCH, bool LOOP>
+constexpr int kAbPerCu = TYPE == 21 && FETCH == 0 && LOOP ? 2 : 3;
 template <int TYPE, int FETCH, bool LOOP = false, bool PART = false, bool TRACE = false>
-__global__ __launch_bounds__(512, FETCH == 0 ? 4 : 6) void k_layer_ab(LayerArgs a) {
+__global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_layer_ab(LayerArgs a) {
     constexpr bool kIq = kAbIq<TYPE, FETCH>, kWide = FETCH == 10 || FETCH == 2;
     constexpr bool kTwoPasses = kWide;  // Q8_0 rows of 65..128 blocks
     constexpr int kIqType = kIq ? TYPE : 21;

@@ -542,16 +542,19 @@ int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s
     m.n_routed_items = routed ? a.k * groups : 0;
     if (!routed) m.ids_tagged = nullptr;  // nobody waits for them inside this launch
     if (!front || a.preselected) m.ids_known = s->ids;
-    // A compute unit holds three of these workgroups (two without the aligned fetch).  The router and shared ones leave well before the ids are
+    // A compute unit holds three of these workgroups.  The router and shared ones leave well before the ids are
     // published, so a few routed ones that have to wait for their places still start in time.  But when the routed
     // ones alone are more than the device holds at once (hidden 2560: 800 against 768), the surplus would start -
     // quantise x, stage the codebooks - only after others have finished: the grid is then cut to what the device
     // holds and the routed workgroups walk the items in a loop (measured at hidden 2560: 36.4 against 37.4 us per layer;
     // there each router row has two waves, and the routed workgroups keep their number all the same).
     const int fixed_wgs = (router_rows_n + 7) / 8 + m.n_shared_wgs;
-    const int capacity = (fetch == 0 ? 2 : 3) * s->compute_units;
-    const int routed_wgs = m.n_routed_items <= capacity - 8 ? m.n_routed_items
-                                                            : std::min(m.n_routed_items, std::max(capacity - fixed_wgs, groups));
+    const int capacity = 3 * s->compute_units;
+    // (The loop that runs two per compute unit, kAbPerCu, takes all of its places: with the shared expert's workgroups counted among
+    // them hidden 7168 / ffn 2048, top-8, has 256 routed workgroups left and takes 106 us, so 68; 5120 / 1024 40.7, 34.2.)
+    const bool two = fetch == 0 && L->gate_type == WD_TYPE_IQ3_S;
+    const int looping = two ? kAbPerCu<21, 0, true> * s->compute_units : std::max(capacity - fixed_wgs, groups);
+    const int routed_wgs = m.n_routed_items <= capacity - 8 ? m.n_routed_items : std::min(m.n_routed_items, looping);
     const int grid = m.n_router_wgs + m.n_shared_wgs + routed_wgs;
     if (grid == 0) return WD_OK;
     const bool loop = routed_wgs < m.n_routed_items;
