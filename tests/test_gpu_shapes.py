@@ -35,6 +35,8 @@ SHAPES = [
     (4352, 96, 16, 5, IQ2, Q8, True),
     (4608, 64, 8, 3, IQ4, Q8, True),
     (1024, 96, 128, 15, IQ4, Q8, True),      # the largest selection of one wave
+    (512, 64, 136, 16, IQ3, Q8, False),      # top-16: the selection by a whole workgroup, more candidates than it ranks
+    (512, 64, 512, 16, IQ3, Q8, True),
     (3072, 1536, 16, 16, IQ3, IQ4, True),    # items beyond the device, 17 matrices
 ]
 
