@@ -37,6 +37,11 @@ SHAPES = [
     (1024, 96, 128, 15, IQ4, Q8, True),      # the largest selection of one wave
     (512, 64, 136, 16, IQ3, Q8, False),      # top-16: the selection by a whole workgroup, more candidates than it ranks
     (512, 64, 512, 16, IQ3, Q8, True),
+    (256, 288, 16, 16, IQ3, Q8, True),       # seventeen down matrices: two per wave, rows of 9, 16 and 24 blocks
+    (512, 512, 16, 16, IQ2, IQ4, True),
+    (256, 768, 16, 16, Q8, IQ4, True),
+    (512, 544, 16, 16, IQ4, Q8, True),
+    (512, 256, 16, 16, IQ3, IQ4, True),      # eight blocks: the four-row form
     (3072, 1536, 16, 16, IQ3, IQ4, True),    # items beyond the device, 17 matrices
 ]
 

@@ -1269,6 +1269,9 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
 // and 1 fold four rows each.  (Hidden 4096, eight experts with rows of 48 Q8_0 blocks, 53.5 MB: 25.7 us in the four-row form
 // with two matrices per wave, 16.3 so, 15.4 with WORDS - the bytes alone take 9 -; hidden 2560, ten IQ4_NL experts of 20
 // blocks and the shared one: 12.4, 10.9; hidden 2048, ten Q8_0 experts of 16: 6.0, 5.5.)
+// TWO: seventeen matrices (top-16 and the shared expert), nine waves with two each, one after the other: rows of 9..24 blocks.
+// (Hidden 2560, rows of 20 Q8_0 blocks: 13.2 us, in the four-row form with sixteen waves 20.5, here with sixteen 14.8; hidden 2048,
+// 16 blocks: 7.8, 9.7, 7.9; hidden 1024, eight blocks: 6.1, 5.6.)
 // WORDS: the rows come through LDS as aligned words (Q8Rows8Fetch), otherwise a lane loads its own blocks (Q8Rows8Blocks).
 // dynamic LDS: per wave the tile (WORDS: the staging area, which it lies in) and the quantised activation (F bytes + F/32
 // halves, padded), then [n_act][8] floats.
@@ -1277,72 +1280,77 @@ __host__ __device__ inline uint32_t layer_c8_wave_bytes(int F) {
     static_assert(sizeof(Q8Tile8) <= kQ8Rows8StageBytes, "the tile lies in the staging area");
     return (WORDS ? kQ8Rows8StageBytes : static_cast<uint32_t>(sizeof(Q8Tile8))) + (static_cast<uint32_t>(F + F / 16 + 15) & ~15u);
 }
-template <int KIND, int PASSES, bool WORDS, bool PART = false, bool TRACE = false>
-__global__ __launch_bounds__(1024) void k_layer_c8(LayerArgs a) {
+template <int KIND, int PASSES, bool WORDS, bool PART = false, bool TRACE = false, bool TWO = false>
+__global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
     constexpr int STEPS = (PASSES + 1) / 2;  // of sixteen blocks
     extern __shared__ __align__(16) uint8_t lds_c8[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int n_act = a.k + (a.sh_inp ? 1 : 0);
+    const int n_act = a.k + (a.sh_inp ? 1 : 0), n_waves = TWO ? 9 : max(n_act, 2);
     const uint32_t per_wave = layer_c8_wave_bytes<WORDS>(a.F);
     uint8_t *stage = lds_c8 + wave * per_wave;
     Q8Tile8 &tile = *reinterpret_cast<Q8Tile8 *>(stage);
     int8_t *aq = reinterpret_cast<int8_t *>(stage + (WORDS ? kQ8Rows8StageBytes : sizeof(Q8Tile8)));
     uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_c8 + max(n_act, 2) * per_wave);
+    float *ybuf = reinterpret_cast<float *>(lds_c8 + n_waves * per_wave);
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;
     if (a.dry) return;
     if (a.clear_tagged && blockIdx.x == 0)  // (as in k_layer_c)
-        for (int i = threadIdx.x; i < kTagCopies * 16; i += 64 * n_act)
+        for (int i = threadIdx.x; i < kTagCopies * 16; i += 64 * (TWO ? 9 : n_act))
             __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     mark<TRACE>(a, 2, 0);
-    const int m = min(wave, n_act - 1);  // (a second wave without a matrix of its own repeats the first's)
-    const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;
-    // the activation first: its address needs no expert id, and loads return in order - it is quantised while the weights are
-    // still on their way
-    float4 v[2 * STEPS];
-#pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-        const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
-        v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
-    }
-    const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m))) +
-                                            static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
     FoldOps ops;
-    auto run = [&](auto kind, auto part) {
-        constexpr int K = decltype(kind)::value;
-        constexpr bool P = decltype(part)::value;
-        typename std::conditional<WORDS, Q8Rows8Fetch<K, STEPS>, Q8Rows8Blocks<K, PASSES>>::type fetch;
-        fetch.request(rows, nb, lane);
-        if (wave < 2) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+    int m = TWO ? wave : min(wave, n_act - 1);  // (a second wave without a matrix of its own repeats the first's)
+    do {
+        int lane = threadIdx.x & 63;
+        if constexpr (TWO) asm volatile("" : "+v"(lane));  // (nothing per lane is kept from one matrix to the next: it would take 30 registers)
+        const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;
+        // the activation first: its address needs no expert id, and loads return in order - it is quantised while the weights are
+        // still on their way
+        float4 v[2 * STEPS];
 #pragma unroll
-        for (int i = 0; i < STEPS; ++i)
-            lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
-        mark<TRACE>(a, 2, 1);
-        Q8Chain ch;
-        int32_t *pp = P ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;
-#pragma unroll
-        for (int q = 0; q < STEPS; ++q) {
-            Q8Block w0, w1;
-            if constexpr (WORDS) {
-                wave_lds_fence();  // the step before has been read
-                fetch.park(q, stage, lane);
-                wave_lds_fence();
-                // (both blocks of the step before the first pass: its tile takes the parked words' place)
-                w0 = q8_rows8_block<K>(stage, nb, lane >> 3, lane & 7), w1 = q8_rows8_block<K>(stage, nb, lane >> 3, 8 + (lane & 7));
-            } else {
-                if (q == 0) wave_lds_fence();
-                w0 = fetch.w[2 * q], w1 = fetch.w[min(2 * q + 1, PASSES - 1)];
-            }
-            q8_rows8_pass<K, P>(w0, 16 * q, nb, aq, ad, tile, lane, ch, pp);
-            if (2 * q + 1 < PASSES && 16 * q + 8 < nb) q8_rows8_pass<K, P>(w1, 16 * q + 8, nb, aq, ad, tile, lane, ch, pp);
+        for (int i = 0; i < STEPS; ++i) {
+            const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
+            v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
         }
-        return q8_rows8_close<K>(ch, nb, tile, lane);
-    };
-    float y;
-    if (PART && !is_shared) y = run(std::integral_constant<int, KIND>{}, std::integral_constant<bool, PART>{});
-    else if (q8) y = run(std::integral_constant<int, 0>{}, std::false_type{});
-    else y = run(std::integral_constant<int, KIND>{}, std::false_type{});
-    if (wave < n_act && (lane & 7) == 0) ybuf[m * 8 + (lane >> 3)] = y;
+        const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m))) +
+                                                static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
+        auto run = [&](auto kind, auto part) {
+            constexpr int K = decltype(kind)::value;
+            constexpr bool P = decltype(part)::value;
+            typename std::conditional<WORDS, Q8Rows8Fetch<K, STEPS>, Q8Rows8Blocks<K, PASSES>>::type fetch;
+            fetch.request(rows, nb, lane);
+            if (wave < 2 && (!TWO || m < 9)) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+#pragma unroll
+            for (int i = 0; i < STEPS; ++i)
+                lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
+            mark<TRACE>(a, 2, 1);
+            Q8Chain ch;
+            int32_t *pp = P ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;
+#pragma unroll
+            for (int q = 0; q < STEPS; ++q) {
+                Q8Block w0, w1;
+                if constexpr (WORDS) {
+                    wave_lds_fence();  // the step before has been read
+                    fetch.park(q, stage, lane);
+                    wave_lds_fence();
+                    // (both blocks of the step before the first pass: its tile takes the parked words' place)
+                    w0 = q8_rows8_block<K>(stage, nb, lane >> 3, lane & 7), w1 = q8_rows8_block<K>(stage, nb, lane >> 3, 8 + (lane & 7));
+                } else {
+                    if (q == 0) wave_lds_fence();
+                    w0 = fetch.w[2 * q], w1 = fetch.w[min(2 * q + 1, PASSES - 1)];
+                }
+                q8_rows8_pass<K, P>(w0, 16 * q, nb, aq, ad, tile, lane, ch, pp);
+                if (2 * q + 1 < PASSES && 16 * q + 8 < nb) q8_rows8_pass<K, P>(w1, 16 * q + 8, nb, aq, ad, tile, lane, ch, pp);
+            }
+            return q8_rows8_close<K>(ch, nb, tile, lane);
+        };
+        float y;
+        if (PART && !is_shared) y = run(std::integral_constant<int, KIND>{}, std::integral_constant<bool, PART>{});
+        else if (q8) y = run(std::integral_constant<int, 0>{}, std::false_type{});
+        else y = run(std::integral_constant<int, KIND>{}, std::false_type{});
+        if (wave < n_act && (lane & 7) == 0) ybuf[m * 8 + (lane >> 3)] = y;
+        m += 9;
+    } while (TWO && m < n_act);
     mark<TRACE>(a, 2, 2);
     __syncthreads();
     mark<TRACE>(a, 2, 3);

@@ -594,6 +594,15 @@ void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
         k_layer_c8<KIND, PASSES, WORDS><<<grid, block, lds, st>>>(a);
 }
 template <int KIND>
+void launch_layer_c8_two(hipStream_t st, const LayerArgs &a) {
+    const size_t lds = 9 * static_cast<size_t>(layer_c8_wave_bytes<false>(a.F)) + sizeof(float) * 8 * (a.k + 1);
+    const dim3 grid(a.H / 8), block(64 * 9);
+    if (a.F <= 512)
+        k_layer_c8<KIND, 2, false, false, false, true><<<grid, block, lds, st>>>(a);
+    else
+        k_layer_c8<KIND, 3, false, false, false, true><<<grid, block, lds, st>>>(a);
+}
+template <int KIND>
 void launch_layer_c8(bool words, hipStream_t st, const LayerArgs &a) {
     if (a.F <= 512) launch_layer_c8<KIND, 2, false>(st, a);
     else if (a.F <= 768) launch_layer_c8<KIND, 3, false>(st, a);
@@ -629,7 +638,9 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
     SiteScope site(WD_SITE_FUSED_C, st);
     const int n_act = k + (shared ? 1 : 0);
     const bool q8 = L->down_type == WD_TYPE_Q8_0;
-    if (F <= 1536 && n_act <= 16) {
+    if (n_act > 16 && F > 256 && F <= 768 && !a.down_part && !a.trace) {  // (chunk sums and time stamps: the four-row form has them)
+        q8 ? launch_layer_c8_two<0>(st, a) : launch_layer_c8_two<1>(st, a);
+    } else if (F <= 1536 && n_act <= 16) {
         // The aligned fetch where every down tensor starts on a 16-byte boundary and the rows' bytes are what the dispatch
         // waits for: 40 MB and more (53.5 MB: 15.4 us against 16.3; 21 MB: 9.5 against 9.0; 15 MB: 7.5 against 7.0).
         auto al16 = [](const void *p, size_t v) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && v % 16 == 0; };
