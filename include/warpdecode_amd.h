@@ -199,7 +199,9 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
 int wd_moe_scratch_destroy(wd_moe_scratch *s);
 /* 0 when every bounded wait inside the fused dispatches was satisfied so far, 1 when one ran out, 2 when a kernel
  * was asked for an expert whose entry in slot_of_expert is negative (not in the slot pool: the kernel read slot 0
- * instead); the layer's results are then invalid and the fused combine has written NaN.  -1 on error.
+ * instead), 3 when an id given by the caller (a routing trace, a preselection) is not one of the layer's experts (expert 0
+ * was read instead; the one-launch stack reads expert 0 without a report); the layer's results are then invalid and the
+ * fused combine of one token has written NaN.  -1 on error.
  * Synchronous read of one device word. */
 int wd_moe_scratch_status(wd_moe_scratch *s);
 /* The device word behind it (u32), for callers that copy it beside other results instead of a read of its own. */

@@ -299,6 +299,57 @@ def test_status_word_is_clear(g):
     sc.close()
 
 
+@pytest.mark.parametrize("H,F,k,gate_t", [(2048, 512, 4, synth.IQ3_S), (512, 64, 3, synth.Q8_0), (512, 256, 16, synth.IQ2_S)])
+@pytest.mark.parametrize("bad", [-1, 16, 0x7fffffff])
+def test_ids_outside_the_layer(g, oracle, H, F, k, gate_t, bad):
+    """A preselection or a routing trace with an id that the layer does not have: expert 0 is read instead, the status word
+    says so and the one-token results are NaN; a token batch reports it as well.  After the reset the same scratch gives the
+    oracle's result again."""
+    E = 16
+    L = synth.make_layer(H, F, E, k, gate_t, synth.Q8_0, True, seed=SEED, layer=91, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 92, H), H)
+    dl, scs = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(2)]
+    sc, lib = scs[0], capi.load()
+    ids = np.arange(k, dtype=np.int32)
+    ids[k // 2] = bad
+    wts = np.full(k, 0.25, np.float32)
+
+    def select(s, which):
+        capi.call("wd_memcpy_h2d", C.c_void_p(s.raw("ids")), which.ctypes.data_as(C.c_void_p), 4 * k, g.stream())
+        capi.call("wd_memcpy_h2d", C.c_void_p(s.raw("weights")), wts.ctypes.data_as(C.c_void_p), 4 * k, g.stream())
+
+    dx, out = g.dev(x), g.empty(H, np.float32)
+    for flags in (0, capi.MOE_SPLIT_AB, capi.MOE_STAGED):
+        select(sc, ids)
+        capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, flags | capi.MOE_PRESELECTED, g.stream())
+        g.sync()
+        assert lib.wd_moe_scratch_status(sc.h) == 3, flags
+        if flags != capi.MOE_STAGED:
+            assert np.isnan(g.host(out)).all(), flags
+        capi.call("wd_moe_scratch_set_wait_limit", sc.h, 0)
+    trace = g.dev(ids)
+    capi.call("wd_moe_stack_f32", (capi.MoeLayer * 1)(dl.desc), 1, g.ptr(g.dev(x)), g.ptr(out), sc.h, g.ptr(trace), 0.05, 0x200, g.stream())
+    g.sync()
+    assert lib.wd_moe_scratch_status(sc.h) == 3 and np.isnan(g.host(out)).all()
+    capi.call("wd_moe_scratch_set_wait_limit", sc.h, 0)
+    for s in scs:
+        select(s, ids)
+    dx2, out2 = g.dev(np.stack([x, x])), g.empty((2, H), np.float32)
+    arr = (C.c_void_p * 2)(*[s.h.value for s in scs])
+    capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx2), g.ptr(out2), 2, arr, capi.MOE_PRESELECTED, g.stream())
+    g.sync()
+    assert lib.wd_moe_scratch_status(sc.h) == 3
+    capi.call("wd_moe_scratch_set_wait_limit", sc.h, 0)
+    good = np.arange(k, dtype=np.int32)
+    select(sc, good)
+    capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, capi.MOE_PRESELECTED, g.stream())
+    g.sync()
+    want, _ = oracle.moe_layer(L, x, ids=good, weights=wts)
+    assert lib.wd_moe_scratch_status(sc.h) == 0 and g.same_bits(g.host(out), want)
+    for s in scs:
+        s.close()
+
+
 def test_bounded_wait_gives_up_and_recovers(g, oracle):
     """Failure path of the in-dispatch hand-off, forced from the host: with a wait limit of one poll the routed
     workgroups give up before the ids are published, the status word says so, every kernel still ends; with the

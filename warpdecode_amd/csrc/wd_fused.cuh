@@ -1074,7 +1074,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         const int rg = item - j * groups;
         int e;
         if (a.ids_known) {
-            e = sld_i32(a.ids_known + j);
+            e = checked_expert(a.gate_up, sld_i32(a.ids_known + j));
             if (!kBehind) __syncthreads();
         } else {
             if (threadIdx.x == 0) {
@@ -1240,7 +1240,7 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
     for (int m = wave; m < n_act; m += nwaves) {
         const bool is_shared = m == a.k;
         // m is the same for the whole wave: the id comes through the scalar path
-        const uint8_t *const w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m));
+        const uint8_t *const w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)));
         const bool q8 = KIND == 0 || is_shared;  // the same in every lane
         const uint8_t *const rows = w + static_cast<size_t>(r0) * nb * (q8 ? 34 : 18);
         auto quantise = [&]() {
@@ -1312,7 +1312,7 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
             const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
             v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
         }
-        const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, sld_i32(a.ids + m))) +
+        const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)))) +
                                                 static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
         auto run = [&](auto kind, auto part) {
             constexpr int K = decltype(kind)::value;

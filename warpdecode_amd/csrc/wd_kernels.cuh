@@ -22,8 +22,19 @@ struct MatSrc {
     const uint8_t *pool;
     size_t slot_bytes;
     size_t slot_off[2];
-    unsigned *slot_status;  // set to 2 when an expert without a slot is asked for (may be null)
+    unsigned *slot_status;  // set to 2 when an expert without a slot is asked for, to 3 for one that the layer does not have (may be null)
+    unsigned n_experts;     // experts of the tensors (0: not known, ids are taken as they are)
 };
+
+// An id that the caller gave (a routing trace, a selection left in the scratch) may lie outside the layer's experts: such
+// a request is reported through the status word and reads expert 0 instead of an address outside the tensors.
+WD_DEV int checked_expert(const MatSrc &s, int e) {
+    if (s.n_experts != 0u && static_cast<unsigned>(e) >= s.n_experts) {
+        if (s.slot_status) __hip_atomic_store(s.slot_status, 3u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        e = 0;
+    }
+    return e;
+}
 
 // The slot of an expert that is not in the pool is -1: such a request is reported through the status word and reads
 // slot 0 (memory that exists, values that mean nothing) instead of an address before the pool.
@@ -39,7 +50,7 @@ WD_DEV const uint8_t *mat_ptr(const MatSrc &s, int m) {
     if (s.table) return s.table[m];
     if (s.ids) {
         const int j = m / s.per_expert, t = m - j * s.per_expert;
-        const int e = s.ids[j];
+        const int e = checked_expert(s, s.ids[j]);
         if (s.slot_of_expert) return s.pool + checked_slot(s, s.slot_of_expert[e]) * s.slot_bytes + s.slot_off[t];
         return s.base[t] + static_cast<size_t>(e) * s.stride[t];
     }

@@ -277,6 +277,7 @@ MatSrc routed_src(const wd_moe_layer *L, const wd_moe_scratch *s, const int32_t 
     MatSrc m{};
     m.ids = ids;
     m.slot_status = s->status;
+    m.n_experts = static_cast<unsigned>(L->n_experts);
     m.per_expert = down ? 1 : 2;
     if (L->slot_of_expert) {
         m.slot_of_expert = L->slot_of_expert;

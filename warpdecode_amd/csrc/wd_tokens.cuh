@@ -22,8 +22,8 @@ constexpr int kPairEntries = 128;  // entries of a pointer table (wd_moe_layer_t
 
 // Tensor T of "expert" e when the pass was given a table of pointers instead of tensors that hold every expert: e is
 // then an index into the table ([entry][tensors per entry]).  The host fills every one of the kPairEntries entries
-// (those past the caller's with entry 0), and a number outside the table reads entry 0: a wrong id in the scratch gives
-// a wrong result, never a load through a pointer nobody set.
+// (those past the caller's with entry 0), and a number outside the table reads entry 0 (so do numbers past the caller's
+// entries: token_pair_id): a wrong id in the scratch gives a wrong result, never a load through a pointer nobody set.
 template <int T>
 WD_DEV const uint8_t *mat_ptr_entry(const MatSrc &s, int e) {
     if (s.table) return s.table[(static_cast<unsigned>(e) < static_cast<unsigned>(kPairEntries) ? e : 0) * s.per_expert + T];
@@ -143,8 +143,10 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
 }
 
 // The id of pair `pair` (= token * k + rank) for lane-parallel comparisons; pairs past the end get distinct
-// negative values that match nothing.
-WD_DEV int token_pair_id(const TokenArgs &ta, int pair) {
+// negative values that match nothing.  An id outside the layer's experts (only a selection that the caller left in the
+// scratches can hold one) counts as expert 0, as in checked_expert: it also indexes the union's tables.  Dispatch B reports it;
+// here a branch would make every wave wait for the ids alone (checked_expert in this place: 0.8 us per layer).
+WD_DEV int token_pair_id(const TokenArgs &ta, int pair, bool &outside) {
     const int k = ta.common.k, n = ta.T * k;
     const int pc = min(pair, n - 1);  // the load is unconditional (no branch, so that it can overlap with others)
     int t = 0;
@@ -156,7 +158,8 @@ WD_DEV int token_pair_id(const TokenArgs &ta, int pair) {
         p = past ? ta.tok[q].ids : p;
     }
     const int v = p[pc - t * k];
-    return pair < n ? v : -1 - pair;
+    outside = static_cast<unsigned>(v) >= ta.common.down.n_experts;
+    return pair < n ? (outside ? 0 : v) : -1 - pair;
 }
 
 // The union of the T*k routed ids, in order of first appearance, with the rank at which every token selected
@@ -171,7 +174,8 @@ struct TokenUnion {
 
 WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
     const int k = ta.common.k, n = ta.T * k;
-    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
+    bool outside_lo, outside_hi;
+    const int id_lo = token_pair_id(ta, lane, outside_lo), id_hi = token_pair_id(ta, lane + 64, outside_hi);
     const bool on_lo = lane < n, on_hi = lane + 64 < n;
     for (int i = lane; i < 128 * kMaxTokens / 4; i += 64) reinterpret_cast<uint32_t *>(&un.rank[0][0])[i] = 0xffffffffu;
     // lowest pair that names the same expert, through a table indexed by expert id
@@ -207,6 +211,7 @@ WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
     if (on_lo) un.rank[un.upos[fq_lo]][t_lo] = static_cast<int8_t>(lane - t_lo * k);
     if (on_hi) un.rank[un.upos[fq_hi]][t_hi] = static_cast<int8_t>(lane + 64 - t_hi * k);
     wave_lds_fence();
+    if (blockIdx.x == 0 && (outside_lo || outside_hi)) __hip_atomic_store(ta.common.status, 3u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- dispatch B for T tokens ----------------------------------------------------------------------------
@@ -517,7 +522,8 @@ void k_tokens_c(TokenArgs ta) {
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;  // hidden is a multiple of 8
     mark(a, 2, 0);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
-    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
+    bool outside;
+    const int id_lo = token_pair_id(ta, lane, outside), id_hi = token_pair_id(ta, lane + 64, outside);
     // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
     float wreg;
     {

@@ -296,7 +296,7 @@ public:
     int *h_ids() const { return h_ids_; }
     // The scratch's status word travels to the host with the next synchronisation of `stream`; afterwards
     // throw_if_failed() reports a layer pass on this scratch whose results are invalid (a bounded wait that ran out,
-    // an expert that had no slot).
+    // an expert that had no slot, an id that the layer does not have).
     void queue_status_copy(Stream stream) {
         check(wd_memcpy_d2h(h_ids_ + kMoeBatchTokenMax * k_, wd_moe_scratch_status_word(s_), sizeof(int), stream), "status copy failed");
     }
@@ -304,6 +304,7 @@ public:
         const int st = h_ids_[kMoeBatchTokenMax * k_];
         if (st == 1) throw std::runtime_error("MoE layer pass failed: a wait between its workgroups ran out");
         if (st == 2) throw std::runtime_error("MoE layer pass failed: an expert without a cache slot was selected");
+        if (st == 3) throw std::runtime_error("MoE layer pass failed: an expert id outside the layer was given");
         if (st != 0) throw std::runtime_error("MoE layer pass failed");
     }
     float *h_weights() const { return h_weights_; }
