@@ -42,6 +42,12 @@ SHAPES = [
     (256, 768, 16, 16, Q8, IQ4, True),
     (512, 544, 16, 16, IQ4, Q8, True),
     (512, 256, 16, 16, IQ3, IQ4, True),      # eight blocks: the four-row form
+    (4096, 800, 16, 12, IQ3, Q8, True),      # 40 MB and more of down rows: as aligned words; 25, 32, 33 and 48 blocks
+    (4096, 1024, 16, 9, IQ2, Q8, True),
+    (4096, 1056, 16, 9, IQ3, Q8, True),
+    (4096, 1536, 8, 8, IQ2, Q8, False),
+    (4608, 1024, 16, 15, IQ3, IQ4, True),
+    (4096, 1536, 16, 12, IQ2, IQ4, False),
     (3072, 1536, 16, 16, IQ3, IQ4, True),    # items beyond the device, 17 matrices
 ]
 
@@ -111,6 +117,8 @@ def test_tensors_on_two_byte_boundaries(g, oracle, monkeypatch, H, F, k):
     (1792, 512, 32, 5, IQ3, IQ4, False, 3),      # a pass of seven super-blocks
     (2304, 640, 16, 3, IQ2, IQ4, True, 4),       # nine
     (4096, 1056, 16, 3, IQ3, Q8, True, 7),       # sixteen, 33 down blocks
+    (512, 800, 16, 4, IQ3, Q8, True, 5),         # 25 and 32 down blocks
+    (768, 1024, 16, 3, IQ2, IQ4, False, 8),
     (3072, 1536, 16, 10, IQ4, IQ4, True, 2),     # 48 down blocks
     (1024, 1568, 16, 2, IQ2, Q8, True, 6)])      # 49: the one-token dispatch per token
 def test_token_batch_shapes(g, oracle, H, F, E, k, gate, down, shared, T):
