@@ -42,11 +42,11 @@ SHAPES = [
     (256, 768, 16, 16, Q8, IQ4, True),
     (512, 544, 16, 16, IQ4, Q8, True),
     (512, 256, 16, 16, IQ3, IQ4, True),      # eight blocks: the four-row form
-    (4096, 800, 16, 12, IQ3, Q8, True),      # 40 MB and more of down rows: as aligned words; 25, 32, 33 and 48 blocks
+    (4096, 800, 16, 12, IQ3, Q8, True),      # 32 MB and more of down rows: as aligned words; 25, 32, 33 and 48 blocks
     (4096, 1024, 16, 9, IQ2, Q8, True),
     (4096, 1056, 16, 9, IQ3, Q8, True),
     (4096, 1536, 8, 8, IQ2, Q8, False),
-    (4608, 1024, 16, 15, IQ3, IQ4, True),
+    (4608, 1024, 16, 15, IQ3, IQ4, True),    # (as blocks)
     (4096, 1536, 16, 12, IQ2, IQ4, False),
     (3072, 1536, 16, 16, IQ3, IQ4, True),    # items beyond the device, 17 matrices
 ]

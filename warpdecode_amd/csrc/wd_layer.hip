@@ -607,7 +607,7 @@ template <int KIND>
 void launch_layer_c8(bool words, hipStream_t st, const LayerArgs &a) {
     if (a.F <= 512) launch_layer_c8<KIND, 2, false>(st, a);
     else if (a.F <= 768) launch_layer_c8<KIND, 3, false>(st, a);
-    else if (a.F <= 1024) words ? launch_layer_c8<KIND, 4, true>(st, a) : launch_layer_c8<KIND, 4, false>(st, a);
+    else if (a.F <= 1024) KIND == 0 && words ? launch_layer_c8<0, 4, true>(st, a) : launch_layer_c8<KIND, 4, false>(st, a);
     else words ? launch_layer_c8<KIND, 6, true>(st, a) : launch_layer_c8<KIND, 6, false>(st, a);
 }
 
@@ -643,9 +643,11 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
         q8 ? launch_layer_c8_two<0>(st, a) : launch_layer_c8_two<1>(st, a);
     } else if (F <= 1536 && n_act <= 16) {
         // The aligned fetch where every down tensor starts on a 16-byte boundary and the rows' bytes are what the dispatch
-        // waits for: 40 MB and more (53.5 MB: 15.4 us against 16.3; 21 MB: 9.5 against 9.0; 15 MB: 7.5 against 7.0).
+        // waits for: 32 MB and more (Q8_0 rows of 48 blocks, 53.5 MB: 14.7 us against 16.1; 40: 12.6, 13.3; 33: 11.4, 11.7; 26.7: 10.0,
+        // 10.1; 32 blocks, 44.6 MB: 12.5, 13.9; 35.7: 10.7, 11.5; 26.7: 9.2, 9.5; at 21 MB it loses, 9.5 against 9.0).  IQ4_NL rows,
+        // half as long, only beyond 32 blocks (48 blocks, 42.5 MB: 20.0, 20.4; 35.4: 19.1, 19.3; 32 blocks, 37.7 MB: 18.6, 17.2).
         auto al16 = [](const void *p, size_t v) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && v % 16 == 0; };
-        const bool words = static_cast<size_t>(n_act) * wd_tensor_bytes(L->down_type, H, F) >= (40u << 20) && al16(L->shared_down, 0) &&
+        const bool words = static_cast<size_t>(n_act) * wd_tensor_bytes(L->down_type, H, F) >= 32000000 && (q8 || F > 1024) && al16(L->shared_down, 0) &&
                            (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && (L->slot_gate_bytes + L->slot_up_bytes) % 16 == 0
                                               : al16(L->down, L->down_stride));
         q8 ? launch_layer_c8<0>(words, st, a) : launch_layer_c8<1>(words, st, a);
