@@ -468,15 +468,22 @@ WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *w
     const bool dead = sum == 0.0;
     float top_mine = top_e * inv;
     if (!all_good) {
-        float v[8 * M];
+        auto rungs = [&](auto rows) {
+            constexpr int R = decltype(rows)::value;
+            float v[8 * R];
 #pragma unroll
-        for (int m = 0; m < M; ++m)
+            for (int m = 0; m < R; ++m)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int ix = (lane + 64 * m) * 8 + i;
-                v[8 * m + i] = (ix < n && !dead) ? s.p[ix] * inv : -INFINITY;
-            }
-        rungs_on_probs<M>(v, k, lane, top_mine, id_mine);
+                for (int i = 0; i < 8; ++i) {
+                    const int ix = (lane + 64 * m) * 8 + i;
+                    v[8 * m + i] = (ix < n && !dead) ? s.p[ix] * inv : -INFINITY;
+                }
+            rungs_on_probs<R>(v, k, lane, top_mine, id_mine);
+        };
+        // (16 of 72..256 experts: with fewer rows of lanes than there are experts to select the threshold excludes nobody, and this
+        // is the rule; by the rungs for 1024 dispatch AB took 19.7 us instead of 17.1, top-16 of 128)
+        if (M == 1 || n <= 512) rungs(std::integral_constant<int, 1>{});
+        else rungs(std::integral_constant<int, M>{});
         if (override_ids) id_mine = id_given;
         if (tagged) publish_ids(id_mine, k, tagged, copies, lane);
     }
@@ -706,8 +713,6 @@ WD_DEV void topk_block(const float *logits, int n, int k, float w_scale, int32_t
         else if (n <= 128) topk_two_waves<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
         else if (n <= 256) topk_two_waves<4>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
         else topk_two_waves<8>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-    } else if (n <= 512) {  // (top-16 of 128 experts: dispatch AB 17.2 us, by the form for 1024 experts 19.7)
-        topk_block_m<1>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
     } else {
         topk_block_m<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
     }
