@@ -142,11 +142,8 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     if (lane == 0 && r < a.F) s.act[static_cast<size_t>(a.k) * a.F + r] = silu_ggml(gu[0]) * gu[1];
 }
 
-// The id of pair `pair` (= token * k + rank) for lane-parallel comparisons; pairs past the end get distinct
-// negative values that match nothing.  An id outside the layer's experts (only a selection that the caller left in the
-// scratches can hold one) counts as expert 0, as in checked_expert: it also indexes the union's tables.  Dispatch B reports it;
-// here a branch would make every wave wait for the ids alone (checked_expert in this place: 0.8 us per layer).
-WD_DEV int token_pair_id(const TokenArgs &ta, int pair, bool &outside) {
+// The id of pair `pair` (= token * k + rank; at most the last pair's) as it stands in the scratch.
+WD_DEV int token_pair_raw(const TokenArgs &ta, int pair) {
     const int k = ta.common.k, n = ta.T * k;
     const int pc = min(pair, n - 1);  // the load is unconditional (no branch, so that it can overlap with others)
     int t = 0;
@@ -157,9 +154,20 @@ WD_DEV int token_pair_id(const TokenArgs &ta, int pair, bool &outside) {
         t += past ? 1 : 0;
         p = past ? ta.tok[q].ids : p;
     }
-    const int v = p[pc - t * k];
-    outside = static_cast<unsigned>(v) >= ta.common.down.n_experts;
-    return pair < n ? (outside ? 0 : v) : -1 - pair;
+    return p[pc - t * k];
+}
+// The same for lane-parallel comparisons; pairs past the end get distinct negative values that match nothing.  An id outside
+// the layer's experts (only a selection that the caller left in the scratches can hold one) counts as expert 0, as in
+// checked_expert: it also indexes the union's tables.  (checked_expert in this place, a branch between the load and the union,
+// takes 0.8 us per layer: another wave reports it, token_ids_report.)
+WD_DEV int token_pair_id(const TokenArgs &ta, int pair) {
+    const int v = token_pair_raw(ta, pair);
+    return pair < ta.T * ta.common.k ? (static_cast<unsigned>(v) < ta.common.down.n_experts ? v : 0) : -1 - pair;
+}
+
+// One wave: reports an id outside the layer's experts through the status word.
+WD_DEV void token_ids_report(const TokenArgs &ta, int lane) {
+    for (int pair = lane; pair < ta.T * ta.common.k; pair += 64) checked_expert(ta.common.down, token_pair_raw(ta, pair));
 }
 
 // The union of the T*k routed ids, in order of first appearance, with the rank at which every token selected
@@ -174,8 +182,7 @@ struct TokenUnion {
 
 WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
     const int k = ta.common.k, n = ta.T * k;
-    bool outside_lo, outside_hi;
-    const int id_lo = token_pair_id(ta, lane, outside_lo), id_hi = token_pair_id(ta, lane + 64, outside_hi);
+    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
     const bool on_lo = lane < n, on_hi = lane + 64 < n;
     for (int i = lane; i < 128 * kMaxTokens / 4; i += 64) reinterpret_cast<uint32_t *>(&un.rank[0][0])[i] = 0xffffffffu;
     // lowest pair that names the same expert, through a table indexed by expert id
@@ -211,7 +218,6 @@ WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
     if (on_lo) un.rank[un.upos[fq_lo]][t_lo] = static_cast<int8_t>(lane - t_lo * k);
     if (on_hi) un.rank[un.upos[fq_hi]][t_hi] = static_cast<int8_t>(lane + 64 - t_hi * k);
     wave_lds_fence();
-    if (blockIdx.x == 0 && (outside_lo || outside_hi)) __hip_atomic_store(ta.common.status, 3u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- dispatch B for T tokens ----------------------------------------------------------------------------
@@ -265,6 +271,7 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
     };
     load_blocks(wave);
     if (wave == 0) token_union_build(ta, un, lane);
+    if (a.preselected && blockIdx.x == 0 && wave == 1) token_ids_report(ta, lane);  // (ahead of the loads: 0.4 us)
     mark(a, 1, 1);
     stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, 512);
     quantise_blocks(wave);
@@ -456,6 +463,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b_q8(TokenArgs ta) {
     int8_t *xq = reinterpret_cast<int8_t *>(lds_tq);
     uint16_t *xd = reinterpret_cast<uint16_t *>(lds_tq + static_cast<size_t>(ta.T) * a.H);
     if (wave == 0) token_union_build(ta, un, lane);
+    if (a.preselected && blockIdx.x == 0 && wave == 1) token_ids_report(ta, lane);
     for (int t = 0; t < ta.T; ++t) lds_quantize_q8_0(ta.tok[t].x, a.H, xq + static_cast<size_t>(t) * a.H, xd + t * nb, threadIdx.x, 512);
     __syncthreads();
     const int n_items = un.count * groups, row = lane >> 3, b = lane & 7;
@@ -522,8 +530,7 @@ void k_tokens_c(TokenArgs ta) {
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;  // hidden is a multiple of 8
     mark(a, 2, 0);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
-    bool outside;
-    const int id_lo = token_pair_id(ta, lane, outside), id_hi = token_pair_id(ta, lane + 64, outside);
+    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
     // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
     float wreg;
     {
