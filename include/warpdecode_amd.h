@@ -131,9 +131,9 @@ int wd_gemv_q8_0_f32(int type, const uint8_t *d_w, int rows, int cols, const int
  * not by their bytes (a 2048 x 2048 Q8_0 matrix alone reaches a seventh of the device's bandwidth).  Item i computes
  * d_out[rows] = W_i (rows x cols) . activation_i exactly as wd_gemv_q8_0_f32 does for it alone - the same workgroups do
  * the same arithmetic, the results are the same bits.  `items` is host memory; items whose shape the shared kernel does
- * not take (Q8_0: rows < 8, fewer than 64 or more than 512 blocks per row, 8192 or more rows; Q4_0: rows that are not a
- * power-of-two number of 8-block groups up to 64; either: pointers not 16-byte aligned) are launched by themselves, in
- * order.  At most 16 items go into one launch; longer lists are cut.
+ * not take (Q8_0: rows < 8, fewer than 16 or more than 512 blocks per row, more than 8184 rows; Q4_0: fewer than 8 or more
+ * than 512 blocks per row, small matrices of fewer than 64 that do not stream, more than 4096 workgroups; either: an
+ * activation that is not 16-byte aligned) are launched by themselves, in order; matrices may start on any two-byte boundary.  At most 16 items go into one launch; longer lists are cut.
  * reference: the call sites of q38_hc_launch_exact_q8_0_gemv_f32, one launch per projection (src/qwen38_hc.cuh:1020-1049),
  * and of launch_q4_float (src/warodecode.cu:1746-1768). */
 typedef struct wd_gemv_item {
@@ -308,7 +308,7 @@ int wd_moe_layer_noalloc_f32(const wd_moe_layer *layer, const float *d_x, float 
  * `layers` is a host array.  No counterpart in the reference, whose caller loops over layers
  * (Qwen38Decoder::step, src/qwen38_forward.cuh:2923-3371).
  * Stacks of up to 64 layers of the 512-expert layer shape (hidden 2048, ffn 512, at most 512 experts, top-k <= 10,
- * IQ3_S or IQ2_S gate/up, Q8_0 down, 16-byte aligned tensors, experts addressed directly) run as ONE launch of 512
+ * IQ3_S, IQ2_S or Q8_0 gate/up, Q8_0 down, 16-byte aligned tensors, experts addressed directly) run as ONE launch of 512
  * workgroups that stay on the device for the whole step and hand values to each other through global memory; this
  * needs a device that holds the whole grid at once (checked) and flags == 0.  Everything else, and
  * WD_MOE_PER_LAYER, takes the per-layer dispatches.  The results are the same bits either way.  The first call with
@@ -329,8 +329,7 @@ int wd_moe_layer_tokens_f32(const wd_moe_layer *layer, const float *d_x, float *
  * Qwen38MoeTokenBatch::set_pair_weights / run, src/qwen38_moe.cuh:2907-3109).  h_gate / h_up / h_down: host arrays of
  * n_entries (<= 128) device pointers; the ids in the scratches are entry numbers, the weights the router weights, and
  * flags must contain WD_MOE_PRESELECTED.  `layer` supplies geometry, tensor types and (optionally) the shared expert;
- * its routed tensor pointers are ignored.  IQ3_S / IQ2_S gate and up; Q8_0 down with ffn <= 512, or 16-byte aligned
- * down views with ffn 512 / 640.  The table travels through a small pinned ring owned by the first scratch (allocated
+ * its routed tensor pointers are ignored.  IQ3_S / IQ2_S gate and up, ffn <= 1536, two-byte aligned views.  The table travels through a small pinned ring owned by the first scratch (allocated
  * at first use); every expert's bytes are read once for all tokens that selected it, results are those of one pass
  * per token. */
 int wd_moe_layer_tokens_pairs_f32(const wd_moe_layer *layer, const uint8_t *const *h_gate, const uint8_t *const *h_up,

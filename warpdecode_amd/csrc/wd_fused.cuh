@@ -1273,7 +1273,8 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
 // PASSES: of eight blocks per row (F <= 256 PASSES).  grid = H / 8, block = 64 max(n_act, 2) with at most 16 matrices; waves 0
 // and 1 fold four rows each.  (Hidden 4096, eight experts with rows of 48 Q8_0 blocks, 53.5 MB: 25.7 us in the four-row form
 // with two matrices per wave, 16.1 so, 14.7 with WORDS - the bytes alone take 9 -; hidden 2560, ten IQ4_NL experts of 20
-// blocks and the shared one: 12.4, 10.9; hidden 2048, ten Q8_0 experts of 16: 6.0, 5.5.)
+// blocks and the shared one: 11.8, 10.1; hidden 2048, eight Q8_0 experts of 24: 8.9, 6.8; hidden 2048, ten of 16 and the shared one:
+// 6.7, 6.4 with part of the weights in the last-level cache, 6.7, 6.9 with all of them from HBM.)
 // TWO: seventeen matrices (top-16 and the shared expert), nine waves with two each, one after the other: rows of 9..24 blocks.
 // (Hidden 2560, rows of 20 Q8_0 blocks: 13.2 us, in the four-row form with sixteen waves 20.5, here with sixteen 14.8; hidden 2048,
 // 16 blocks: 7.8, 9.7, 7.9; hidden 1024, eight blocks: 6.1, 5.6.)
