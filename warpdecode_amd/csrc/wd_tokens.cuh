@@ -230,7 +230,8 @@ WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
 // FETCH: 0, or how the rows come in when they can be fetched as aligned words (IqRowWords): 8 and 10 rows of that many
 // super-blocks, 1 and 2 others of one or two words per lane.  The row pair of the wave's next item is then requested before the
 // current one is worked on.  dynamic LDS then has 8 * 2 * iq_cover_bytes more bytes behind the activations (16-byte aligned).
-// As many workgroups per compute unit as the registers allow without spilling.
+// As many workgroups per compute unit as the registers allow without spilling (eight tokens and rows of eight super-blocks spill
+// two, which costs nothing: 68.3 us per layer, 68.7 without).
 template <int TYPE, int MAXT, int FETCH>
 constexpr int kTokensBPerCu = FETCH == 8 || (FETCH == 10 && TYPE == 22 && MAXT <= 4) ? 3 : 2;
 template <int TYPE, int MAXT, int FETCH = 0>
