@@ -534,7 +534,7 @@ int wd_expert_cache_create(wd_expert_cache **out, size_t capacity_bytes, size_t 
     const size_t table_n = static_cast<size_t>(n_layers) * n_experts;
     if ((e = hipMalloc(reinterpret_cast<void **>(&c->d_table), table_n * sizeof(int32_t))) != hipSuccess)
         return bail("hipMalloc slot table", e);
-    k_fill_i32<<<dim3(static_cast<unsigned>((table_n + 255) / 256)), dim3(256)>>>(c->d_table, -1, table_n);
+    enqueue(k_fill_i32, dim3(static_cast<unsigned>((table_n + 255) / 256)), dim3(256), 0, nullptr, c->d_table, -1, table_n);
     if ((e = hipDeviceSynchronize()) != hipSuccess) return bail("slot table fill", e);
     if ((e = hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking)) != hipSuccess) return bail("copy stream", e);
     if ((e = hipEventCreateWithFlags(&c->ev_retire, hipEventDisableTiming)) != hipSuccess) return bail("event", e);
@@ -811,7 +811,7 @@ int flush_slot_updates(wd_expert_cache *c, const SlotUpdate *updates, int n_upda
         SlotUpdate *d = c->d_updates + static_cast<size_t>(r) * kMaxUpdates;
         for (int i = 0; i < n; ++i) h[i] = updates[done + i];
         WD_HIP(hipMemcpyAsync(d, h, sizeof(SlotUpdate) * n, hipMemcpyHostToDevice, st));
-        k_apply_slot_updates<<<dim3(1), dim3(64), 0, st>>>(c->d_table, d, n);
+        enqueue(k_apply_slot_updates, dim3(1), dim3(64), 0, st, c->d_table, d, n);
         WD_LAUNCH_CHECK();
         WD_HIP(hipEventRecord(c->ring_free[r], st));  // both copies of ring entry r are free after this point
         c->ring_used[r] = true;
@@ -1081,9 +1081,9 @@ int launch_fill_segments(wd_expert_cache *c, FillSegments &fills, int &n_fill, u
         const dim3 grid(per_seg < most ? (per_seg ? per_seg : 1) : most);
         if (beside) {
             const FillMarks marks{mark_layers ? c->d_fill_done : nullptr, reinterpret_cast<unsigned *>(c->d_fill_done + kRowsLayers), mark_layers, c->mark_seq};
-            k_fill_slots_beside<<<grid, dim3(WD_FILL_THREADS), 0, c->copy_stream>>>(fills, n_fill, marks);
+            enqueue(k_fill_slots_beside, grid, dim3(WD_FILL_THREADS), 0, c->copy_stream, fills, n_fill, marks);
         } else {
-            k_fill_slots<<<grid, dim3(WD_FILL_THREADS), 0, c->copy_stream>>>(fills, n_fill);
+            enqueue(k_fill_slots, grid, dim3(WD_FILL_THREADS), 0, c->copy_stream, fills, n_fill);
         }
         WD_LAUNCH_CHECK();
     }

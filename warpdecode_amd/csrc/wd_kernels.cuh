@@ -703,24 +703,28 @@ __global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream(const uint8_t *__re
 }
 // Several matrices of one row length in one launch (see k_gemv_q8_rows8_split_batch): workgroup b belongs to the item
 // whose range of workgroups holds b and does there what k_gemv_q4_stream does for that item alone.
-constexpr int kGemvBatchMax = 16;
+// The table travels with the launch, whose host time grows with it (40 bytes 2.75 us, 480 bytes 3.5): one for few items (184
+// bytes) beside one for many (648).
+constexpr int kGemvBatchMax = 16, kGemvBatchFew = 4;
+template <int MAX>
 struct GemvBatch {
-    const uint8_t *w[kGemvBatchMax];
-    const int8_t *act_qs[kGemvBatchMax];
-    const uint16_t *act_d[kGemvBatchMax];
-    float *out[kGemvBatchMax];
-    int rows[kGemvBatchMax];
-    int first_group[kGemvBatchMax + 1];  // the item's first workgroup; first_group[n]: all workgroups
+    const uint8_t *w[MAX];
+    const int8_t *act_qs[MAX];
+    const uint16_t *act_d[MAX];
+    float *out[MAX];
+    int rows[MAX];
+    int first_group[MAX + 1];  // the item's first workgroup; first_group[n]: all workgroups
     int n;
 };
-WD_DEV int gemv_batch_item(const GemvBatch &b) {
+template <int MAX>
+WD_DEV int gemv_batch_item(const GemvBatch<MAX> &b) {
     int item = 0;
     for (int i = 1; i < b.n; ++i)
         if (static_cast<int>(blockIdx.x) >= b.first_group[i]) item = i;
     return __builtin_amdgcn_readfirstlane(item);
 }
-template <int WPB, bool RAGGED>
-__global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream_batch(GemvBatch b, int nb) {
+template <int WPB, bool RAGGED, int MAX>
+__global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream_batch(GemvBatch<MAX> b, int nb) {
     const int item = gemv_batch_item(b);
     gemv_q4_stream_body<false, 1, WPB, RAGGED>(b.w[item], b.rows[item], nb, b.act_qs[item], b.act_d[item], b.out[item], nullptr,
                                        static_cast<int>(blockIdx.x) - b.first_group[item]);
@@ -1058,8 +1062,8 @@ __global__ __launch_bounds__(WAVES ? 64 * WAVES : 512) void k_gemv_q8_rows8_spli
 // Several matrices of the same row length in ONE launch (the projections a block applies to one or a few activations:
 // each of them alone is bound by its launch, not by its bytes).  Workgroup b belongs to the item whose range of row
 // groups holds b; what it computes is what k_gemv_q8_rows8_split computes for that item alone.
-template <int KB, int NCH, int WAVES, bool RAGGED>
-__global__ __launch_bounds__(WAVES ? 64 * WAVES : 512) void k_gemv_q8_rows8_split_batch(GemvBatch b, int nb) {
+template <int KB, int NCH, int WAVES, bool RAGGED, int MAX>
+__global__ __launch_bounds__(WAVES ? 64 * WAVES : 512) void k_gemv_q8_rows8_split_batch(GemvBatch<MAX> b, int nb) {
     const int item = gemv_batch_item(b);
     gemv_q8_rows8_split_body<0, KB, NCH, WAVES, RAGGED, false>(b.w[item], b.rows[item], nb, b.act_qs[item], b.act_d[item], b.out[item], nullptr,
                                                        static_cast<int>(blockIdx.x) - b.first_group[item]);

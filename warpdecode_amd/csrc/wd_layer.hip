@@ -303,18 +303,18 @@ template <int TYPE>
 void launch_iq(bool part, dim3 grid, hipStream_t st, MatSrc src, int rows, int cols, const int8_t *qs, const float *d,
                float *out, int32_t *partials, int ppr) {
     if (part)
-        k_gemv_iq<TYPE, true><<<grid, dim3(256), 0, st>>>(src, rows, cols, qs, d, out, partials, ppr);
+        enqueue(k_gemv_iq<TYPE, true>, grid, dim3(256), 0, st, src, rows, cols, qs, d, out, partials, ppr);
     else
-        k_gemv_iq<TYPE, false><<<grid, dim3(256), 0, st>>>(src, rows, cols, qs, d, out, nullptr, 0);
+        enqueue(k_gemv_iq<TYPE, false>, grid, dim3(256), 0, st, src, rows, cols, qs, d, out, nullptr, 0);
 }
 
 template <int KIND>
 void launch_q8(bool part, dim3 grid, hipStream_t st, MatSrc src, int rows, int cols, const int8_t *qs,
                const uint16_t *d, int act_stride, float *out, int32_t *partials, int ppr) {
     if (part)
-        k_gemv_q8<KIND, true><<<grid, dim3(256), 0, st>>>(src, rows, cols, qs, d, act_stride, out, partials, ppr);
+        enqueue(k_gemv_q8<KIND, true>, grid, dim3(256), 0, st, src, rows, cols, qs, d, act_stride, out, partials, ppr);
     else
-        k_gemv_q8<KIND, false><<<grid, dim3(256), 0, st>>>(src, rows, cols, qs, d, act_stride, out, nullptr, 0);
+        enqueue(k_gemv_q8<KIND, false>, grid, dim3(256), 0, st, src, rows, cols, qs, d, act_stride, out, nullptr, 0);
 }
 
 // One grouped GEMV of `mats` matrices of `type` ([rows][cols]) against the layer's quantised input
@@ -359,19 +359,19 @@ int layer_staged(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_s
     if (!pre) {
         {
             SiteScope site(WD_SITE_ROUTER_GEMV, st);
-            k_router_gemv<<<dim3((E + (shared ? 1 : 0) + 7) / 8), dim3(256), 0, st>>>(
+            enqueue(k_router_gemv, dim3((E + (shared ? 1 : 0) + 7) / 8), dim3(256), 0, st,
                 L->router, d_x, s->logits, E, H, shared ? L->shared_gate_inp : nullptr, s->shared_gate);
             WD_LAUNCH_CHECK();
         }
         SiteScope site(WD_SITE_ROUTER_TOPK, st);
-        k_topk_softmax<<<dim3(1), dim3(64), 0, st>>>(s->logits, E, k, L->expert_scale, s->ids, s->weights,
+        enqueue(k_topk_softmax, dim3(1), dim3(64), 0, st, s->logits, E, k, L->expert_scale, s->ids, s->weights,
                                                      shared ? s->shared_gate : nullptr, ids_override);
         WD_LAUNCH_CHECK();
     } else if (shared) {
         SiteScope site(WD_SITE_SHARED_GATE, st);
-        k_router_gemv<<<dim3(1), dim3(256), 0, st>>>(L->router, d_x, s->logits, 0, H, L->shared_gate_inp, s->shared_gate);
+        enqueue(k_router_gemv, dim3(1), dim3(256), 0, st, L->router, d_x, s->logits, 0, H, L->shared_gate_inp, s->shared_gate);
         WD_LAUNCH_CHECK();
-        k_sigmoid1<<<dim3(1), dim3(64), 0, st>>>(s->shared_gate);
+        enqueue(k_sigmoid1, dim3(1), dim3(64), 0, st, s->shared_gate);
         WD_LAUNCH_CHECK();
     }
 
@@ -379,11 +379,11 @@ int layer_staged(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_s
     {
         SiteScope site(WD_SITE_RX_QUANT, st);
         if (consumes_q8k(L->gate_type)) {
-            k_q8_k_quantize<<<dim3((H / 256 + 3) / 4), dim3(256), 0, st>>>(d_x, H / 256, s->xk_qs, s->xk_d, s->xk_bs);
+            enqueue(k_q8_k_quantize, dim3((H / 256 + 3) / 4), dim3(256), 0, st, d_x, H / 256, s->xk_qs, s->xk_d, s->xk_bs);
             WD_LAUNCH_CHECK();
         }
         if (!consumes_q8k(L->gate_type) || shared) {
-            k_q8_0_quantize<<<dim3((H / 32 + 31) / 32), dim3(256), 0, st>>>(d_x, H / 32, s->x0_qs, s->x0_d);
+            enqueue(k_q8_0_quantize, dim3((H / 32 + 31) / 32), dim3(256), 0, st, d_x, H / 32, s->x0_qs, s->x0_d);
             WD_LAUNCH_CHECK();
         }
     }
@@ -409,12 +409,12 @@ int layer_staged(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_s
     const int n_act = k + (shared ? 1 : 0);
     {
         SiteScope site(WD_SITE_SILU, st);
-        k_silu_mul_experts<<<dim3((F + 255) / 256, n_act), dim3(256), 0, st>>>(s->gate_up, s->act, F);
+        enqueue(k_silu_mul_experts, dim3((F + 255) / 256, n_act), dim3(256), 0, st, s->gate_up, s->act, F);
         WD_LAUNCH_CHECK();
     }
     {
         SiteScope site(WD_SITE_Q8_QUANT, st);
-        k_q8_0_quantize<<<dim3((n_act * F / 32 + 31) / 32), dim3(256), 0, st>>>(s->act, n_act * F / 32, s->act_qs, s->act_d);
+        enqueue(k_q8_0_quantize, dim3((n_act * F / 32 + 31) / 32), dim3(256), 0, st, s->act, n_act * F / 32, s->act_qs, s->act_d);
         WD_LAUNCH_CHECK();
     }
 
@@ -437,14 +437,14 @@ int layer_staged(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_s
     // 7. ordered weighted sum and the shared branch
     {
         SiteScope site(WD_SITE_ACCUM, st);
-        k_combine<<<dim3((H + 255) / 256), dim3(256), 0, st>>>(s->expert_out, s->weights, k, shared ? s->down_f32 : nullptr,
+        enqueue(k_combine, dim3((H + 255) / 256), dim3(256), 0, st, s->expert_out, s->weights, k, shared ? s->down_f32 : nullptr,
                                                                 s->shared_gate, s->accum, d_out, hc ? nullptr : residual,
                                                                 residual_scale, H);
         WD_LAUNCH_CHECK();
     }
     if (hc && residual) {
         SiteScope site(WD_SITE_HC_COMBINE, st);
-        k_hc_combine<0><<<dim3((H * hc->hc + 255) / 256), dim3(256), 0, st>>>(residual, d_out, nullptr, nullptr, hc->inject, H,
+        enqueue(k_hc_combine<0>, dim3((H * hc->hc + 255) / 256), dim3(256), 0, st, residual, d_out, nullptr, nullptr, hc->inject, H,
                                                                              hc->hc, hc->round_half);
         WD_LAUNCH_CHECK();
     }
@@ -498,17 +498,17 @@ void launch_layer_ab_fetch(bool loop, int grid, hipStream_t st, const LayerArgs 
     // while the chunk sums are exported)
     const bool trace = m.trace != nullptr && !part;
     if constexpr (TYPE == 21 || TYPE == 22) {
-        if (loop && part) return k_layer_ab<TYPE, FETCH, true, true><<<grid, block, lds, st>>>(m);
-        if (part) return k_layer_ab<TYPE, FETCH, false, true><<<grid, block, lds, st>>>(m);
+        if (loop && part) return enqueue(k_layer_ab<TYPE, FETCH, true, true>, grid, block, lds, st, m);
+        if (part) return enqueue(k_layer_ab<TYPE, FETCH, false, true>, grid, block, lds, st, m);
     }
     if (loop && trace)
-        k_layer_ab<TYPE, FETCH, true, false, true><<<grid, block, lds, st>>>(m);
+        enqueue(k_layer_ab<TYPE, FETCH, true, false, true>, grid, block, lds, st, m);
     else if (loop)
-        k_layer_ab<TYPE, FETCH, true><<<grid, block, lds, st>>>(m);
+        enqueue(k_layer_ab<TYPE, FETCH, true>, grid, block, lds, st, m);
     else if (trace)
-        k_layer_ab<TYPE, FETCH, false, false, true><<<grid, block, lds, st>>>(m);
+        enqueue(k_layer_ab<TYPE, FETCH, false, false, true>, grid, block, lds, st, m);
     else
-        k_layer_ab<TYPE, FETCH, false><<<grid, block, lds, st>>>(m);
+        enqueue(k_layer_ab<TYPE, FETCH, false>, grid, block, lds, st, m);
 }
 template <int TYPE>
 void launch_layer_ab(int fetch, bool loop, int grid, hipStream_t st, const LayerArgs &m) {
@@ -576,11 +576,11 @@ void launch_layer_c(hipStream_t st, const LayerArgs &a) {
     const size_t lds = waves * per_wave + sizeof(float) * 4 * n_act;
     const dim3 grid((a.H + 3) / 4), block(64 * waves);
     if (a.down_part)
-        k_layer_c<KIND, true><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c<KIND, true>, grid, block, lds, st, a);
     else if (a.trace)
-        k_layer_c<KIND, false, true><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c<KIND, false, true>, grid, block, lds, st, a);
     else
-        k_layer_c<KIND><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c<KIND>, grid, block, lds, st, a);
 }
 template <int KIND, int PASSES, bool WORDS>
 void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
@@ -588,20 +588,20 @@ void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
     const size_t lds = waves * static_cast<size_t>(layer_c8_wave_bytes<WORDS>(a.F)) + sizeof(float) * 8 * n_act;
     const dim3 grid(a.H / 8), block(64 * waves);
     if (a.down_part)
-        k_layer_c8<KIND, PASSES, WORDS, true><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c8<KIND, PASSES, WORDS, true>, grid, block, lds, st, a);
     else if (a.trace)
-        k_layer_c8<KIND, PASSES, WORDS, false, true><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c8<KIND, PASSES, WORDS, false, true>, grid, block, lds, st, a);
     else
-        k_layer_c8<KIND, PASSES, WORDS><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c8<KIND, PASSES, WORDS>, grid, block, lds, st, a);
 }
 template <int KIND>
 void launch_layer_c8_two(hipStream_t st, const LayerArgs &a) {
     const size_t lds = 9 * static_cast<size_t>(layer_c8_wave_bytes<false>(a.F)) + sizeof(float) * 8 * (a.k + 1);
     const dim3 grid(a.H / 8), block(64 * 9);
     if (a.F <= 512)
-        k_layer_c8<KIND, 2, false, false, false, true><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c8<KIND, 2, false, false, false, true>, grid, block, lds, st, a);
     else
-        k_layer_c8<KIND, 3, false, false, false, true><<<grid, block, lds, st>>>(a);
+        enqueue(k_layer_c8<KIND, 3, false, false, false, true>, grid, block, lds, st, a);
 }
 template <int KIND>
 void launch_layer_c8(bool words, hipStream_t st, const LayerArgs &a) {
@@ -695,7 +695,7 @@ extern "C" int wd_hc_combine_f32(float *d_residual, const float *d_block_out, co
     WD_REQUIRE(d_residual && d_block_out && d_inject, "combine: null pointer");
     WD_REQUIRE(hidden > 0 && hc > 0 && static_cast<long long>(hidden) * hc < (1LL << 31), "combine: bad geometry %d x %d", hc, hidden);
     SiteScope site(WD_SITE_HC_COMBINE, as_stream(stream));
-    k_hc_combine<0><<<dim3((hidden * hc + 255) / 256), dim3(256), 0, as_stream(stream)>>>(d_residual, d_block_out, nullptr, nullptr,
+    enqueue(k_hc_combine<0>, dim3((hidden * hc + 255) / 256), dim3(256), 0, as_stream(stream), d_residual, d_block_out, nullptr, nullptr,
                                                                                           d_inject, hidden, hc, round_half ? 1 : 0);
     WD_LAUNCH_CHECK();
     return WD_OK;
@@ -709,9 +709,9 @@ extern "C" int wd_hc_combine_moe_f32(float *d_residual, const float *d_routed, c
     SiteScope site(WD_SITE_HC_COMBINE, as_stream(stream));
     const dim3 grid((hidden * hc + 255) / 256), block(256);
     if (shared_is_half)
-        k_hc_combine<2><<<grid, block, 0, as_stream(stream)>>>(d_residual, d_routed, d_shared, d_shared_gate, d_inject, hidden, hc, round_half ? 1 : 0);
+        enqueue(k_hc_combine<2>, grid, block, 0, as_stream(stream), d_residual, d_routed, d_shared, d_shared_gate, d_inject, hidden, hc, round_half ? 1 : 0);
     else
-        k_hc_combine<1><<<grid, block, 0, as_stream(stream)>>>(d_residual, d_routed, d_shared, d_shared_gate, d_inject, hidden, hc, round_half ? 1 : 0);
+        enqueue(k_hc_combine<1>, grid, block, 0, as_stream(stream), d_residual, d_routed, d_shared, d_shared_gate, d_inject, hidden, hc, round_half ? 1 : 0);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -724,11 +724,11 @@ extern "C" int wd_shared_expert_f32(const wd_moe_layer *L, const float *d_x, wd_
     const int H = L->hidden, F = L->expert_ffn, slot = s->max_k;
     const hipStream_t st = as_stream(stream);
     SiteScope site(WD_SITE_SHARED, st);
-    k_router_gemv<<<dim3(1), dim3(256), 0, st>>>(L->router, d_x, s->logits, 0, H, L->shared_gate_inp, s->shared_gate);
+    enqueue(k_router_gemv, dim3(1), dim3(256), 0, st, L->router, d_x, s->logits, 0, H, L->shared_gate_inp, s->shared_gate);
     WD_LAUNCH_CHECK();
-    k_sigmoid1<<<dim3(1), dim3(64), 0, st>>>(s->shared_gate);
+    enqueue(k_sigmoid1, dim3(1), dim3(64), 0, st, s->shared_gate);
     WD_LAUNCH_CHECK();
-    k_q8_0_quantize<<<dim3((H / 32 + 31) / 32), dim3(256), 0, st>>>(d_x, H / 32, s->x0_qs, s->x0_d);
+    enqueue(k_q8_0_quantize, dim3((H / 32 + 31) / 32), dim3(256), 0, st, d_x, H / 32, s->x0_qs, s->x0_d);
     WD_LAUNCH_CHECK();
     MatSrc g{}, u{}, d{};
     g.single = L->shared_gate, u.single = L->shared_up, d.single = L->shared_down;
@@ -738,9 +738,9 @@ extern "C" int wd_shared_expert_f32(const wd_moe_layer *L, const float *d_x, wd_
     uint16_t *ad = s->act_d + static_cast<size_t>(slot) * (F / 32);
     if (const int rc = grouped_gemv(WD_TYPE_Q8_0, g, 1, F, H, s, s->x0_qs, s->x0_d, 0, gu, nullptr, st)) return rc;
     if (const int rc = grouped_gemv(WD_TYPE_Q8_0, u, 1, F, H, s, s->x0_qs, s->x0_d, 0, gu + F, nullptr, st)) return rc;
-    k_silu_mul_experts<<<dim3((F + 255) / 256, 1), dim3(256), 0, st>>>(gu, act, F);
+    enqueue(k_silu_mul_experts, dim3((F + 255) / 256, 1), dim3(256), 0, st, gu, act, F);
     WD_LAUNCH_CHECK();
-    k_q8_0_quantize<<<dim3((F / 32 + 31) / 32), dim3(256), 0, st>>>(act, F / 32, aq, ad);
+    enqueue(k_q8_0_quantize, dim3((F / 32 + 31) / 32), dim3(256), 0, st, act, F / 32, aq, ad);
     WD_LAUNCH_CHECK();
     return grouped_gemv(WD_TYPE_Q8_0, d, 1, H, F, s, aq, ad, 0, s->down_f32, nullptr, st);
 }
@@ -816,9 +816,9 @@ int resident_launch(const ResidentArgs &a, wd_moe_scratch *s, hipStream_t st) {
     if (!s->res_fits) return kTakePerLayer;  // the workgroups would wait for each other without all being on the device
     SiteScope site(WD_SITE_STACK_RESIDENT, st);
     if (a.trace)  // (the variant with the time stamps only when they are asked for)
-        k_stack_resident<TYPE, true><<<dim3(kResWgs), dim3(kResThreads), kResLdsBytes, st>>>(a);
+        enqueue(k_stack_resident<TYPE, true>, dim3(kResWgs), dim3(kResThreads), kResLdsBytes, st, a);
     else
-        k_stack_resident<TYPE, false><<<dim3(kResWgs), dim3(kResThreads), kResLdsBytes, st>>>(a);
+        enqueue(k_stack_resident<TYPE, false>, dim3(kResWgs), dim3(kResThreads), kResLdsBytes, st, a);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -900,7 +900,7 @@ extern "C" int wd_moe_stack_f32(const wd_moe_layer *layers, int n_layers, float 
         if (only && !(only & WD_MOE_ONLY_C) && l % kTagRecords == 0) {
             // no dispatch C to invalidate the published ids: reset all records before they are used again
             const size_t n = static_cast<size_t>(kTagRecords) * kTagCopies * 16;
-            k_fill_u32<<<dim3((n + 255) / 256), dim3(256), 0, as_stream(stream)>>>(s->tagged, kTagInvalid, n);
+            enqueue(k_fill_u32, dim3((n + 255) / 256), dim3(256), 0, as_stream(stream), s->tagged, kTagInvalid, n);
             WD_LAUNCH_CHECK();
         }
         SiteScope layer_site(WD_SITE_ROUTED_TOTAL, as_stream(stream));
@@ -917,8 +917,8 @@ void launch_tokens_b_fetch(const TokenArgs &ta, int items, int cus, hipStream_t 
     size_t lds = static_cast<size_t>(ta.T) * (H + sizeof(float) * (H / 256));
     if (FETCH != 0) lds = ((lds + 15) & ~static_cast<size_t>(15)) + 8 * 2 * static_cast<size_t>(iq_cover_bytes<TYPE>(H / 256));
     // persistent: as many workgroups as a compute unit holds walk the items
-    if (ta.T <= 4) k_tokens_b<TYPE, 4, FETCH><<<std::min(items, kTokensBPerCu<TYPE, 4, FETCH> * cus), 512, lds, st>>>(ta);
-    else k_tokens_b<TYPE, kMaxTokens, FETCH><<<std::min(items, kTokensBPerCu<TYPE, kMaxTokens, FETCH> * cus), 512, lds, st>>>(ta);
+    if (ta.T <= 4) enqueue(k_tokens_b<TYPE, 4, FETCH>, std::min(items, kTokensBPerCu<TYPE, 4, FETCH> * cus), 512, lds, st, ta);
+    else enqueue(k_tokens_b<TYPE, kMaxTokens, FETCH>, std::min(items, kTokensBPerCu<TYPE, kMaxTokens, FETCH> * cus), 512, lds, st, ta);
 }
 template <int TYPE>
 void launch_tokens_b(const wd_moe_layer *L, const TokenArgs &ta, int items, int cus, bool table, bool tables_aligned, hipStream_t st) {
@@ -938,7 +938,7 @@ template <int KIND, int PASSES>
 void launch_tokens_c(const TokenArgs &ta, hipStream_t st) {
     constexpr int kWaves = kTokensCWaves<PASSES>;
     const size_t lds = kWaves * static_cast<size_t>(layer_c8_wave_bytes<false>(ta.common.F)) + sizeof(float) * 8 * ta.T * (ta.common.k + 1);
-    k_tokens_c<KIND, PASSES><<<ta.common.H / 8, 64 * kWaves, lds, st>>>(ta);
+    enqueue(k_tokens_c<KIND, PASSES>, ta.common.H / 8, 64 * kWaves, lds, st, ta);
 }
 template <int KIND>
 void launch_tokens_c(const TokenArgs &ta, hipStream_t st) {
@@ -1004,8 +1004,8 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
     const int grid_a = tokens_a_grid(a.n_router_wgs, a.sh_inp ? (F + 7) / 8 : 0).total(tokens);
     if (grid_a > 0) {  // router, selection and shared gate/up of every token
         SiteScope site(WD_SITE_TOKENS_A, st);
-        if (wide) k_tokens_a<true><<<dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st>>>(ta);
-        else k_tokens_a<false><<<dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st>>>(ta);
+        if (wide) enqueue(k_tokens_a<true>, dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st, ta);
+        else enqueue(k_tokens_a<false>, dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st, ta);
         WD_LAUNCH_CHECK();
     }
     const int items_b = tokens * k * ((F + 7) / 8);
@@ -1016,8 +1016,8 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         switch (L->gate_type) {
             case WD_TYPE_IQ3_S: launch_tokens_b<21>(L, ta, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
             case WD_TYPE_IQ2_S: launch_tokens_b<22>(L, ta, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
-            case WD_TYPE_Q8_0: k_tokens_b_q8<0><<<std::min(items_b, 2 * cus), 512, lds_q8, st>>>(ta); break;
-            default: k_tokens_b_q8<1><<<std::min(items_b, 2 * cus), 512, lds_q8, st>>>(ta); break;
+            case WD_TYPE_Q8_0: enqueue(k_tokens_b_q8<0>, std::min(items_b, 2 * cus), 512, lds_q8, st, ta); break;
+            default: enqueue(k_tokens_b_q8<1>, std::min(items_b, 2 * cus), 512, lds_q8, st, ta); break;
         }
         WD_LAUNCH_CHECK();
     }

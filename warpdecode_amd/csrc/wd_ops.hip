@@ -91,7 +91,7 @@ int wd_memset(void *d_dst, int value, size_t bytes, void *stream) {
     const size_t n = bytes / 4;
     if (n == 0) return WD_OK;
     // a fill kernel rather than hipMemsetAsync, so the call may sit inside a captured graph
-    k_fill_u32<<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, as_stream(stream)>>>(
+    enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, as_stream(stream),
         static_cast<uint32_t *>(d_dst), b * 0x01010101u, n);
     WD_LAUNCH_CHECK();
     return WD_OK;
@@ -123,7 +123,7 @@ int wd_q8_k_quantize_f32(const float *d_x, int elements, int8_t *d_qs, float *d_
                "Q8_K quantisation requires a positive multiple of 256 elements (got %d)", elements);
     WD_REQUIRE(d_x && d_qs && d_scales && d_bsums, "wd_q8_k_quantize_f32: null pointer");
     const int blocks = elements / 256;
-    k_q8_k_quantize<<<dim3((blocks + 3) / 4), dim3(256), 0, as_stream(stream)>>>(d_x, blocks, d_qs, d_scales, d_bsums);
+    enqueue(k_q8_k_quantize, dim3((blocks + 3) / 4), dim3(256), 0, as_stream(stream), d_x, blocks, d_qs, d_scales, d_bsums);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -133,7 +133,7 @@ int wd_q8_0_quantize_f32(const float *d_x, int elements, int8_t *d_qs, uint16_t 
                "Q8_0 quantisation requires a positive multiple of 32 elements (got %d)", elements);
     WD_REQUIRE(d_x && d_qs && d_scales, "wd_q8_0_quantize_f32: null pointer");
     const int blocks = elements / 32;
-    k_q8_0_quantize<<<dim3((blocks + 31) / 32), dim3(256), 0, as_stream(stream)>>>(d_x, blocks, d_qs, d_scales);
+    enqueue(k_q8_0_quantize, dim3((blocks + 31) / 32), dim3(256), 0, as_stream(stream), d_x, blocks, d_qs, d_scales);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -142,7 +142,7 @@ int wd_q8_1_quantize_f32(const float *d_x, int elements, int8_t *d_qs, uint16_t 
     WD_REQUIRE(elements > 0 && elements % 32 == 0, "Q8_1 input must be a positive multiple of 32 (got %d)", elements);
     WD_REQUIRE(d_x && d_qs && d_scales, "wd_q8_1_quantize_f32: null pointer");
     const int blocks = elements / 32;
-    k_q8_1_quantize<<<dim3((blocks + 31) / 32), dim3(256), 0, as_stream(stream)>>>(d_x, blocks, d_qs, d_scales);
+    enqueue(k_q8_1_quantize, dim3((blocks + 31) / 32), dim3(256), 0, as_stream(stream), d_x, blocks, d_qs, d_scales);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -151,7 +151,7 @@ int wd_q8_0_quantize_f16(const uint16_t *d_x, int elements, int8_t *d_qs, uint16
     WD_REQUIRE(d_x && d_qs && d_scales, "wd_q8_0_quantize_f16: null pointer");
     WD_REQUIRE(reinterpret_cast<uintptr_t>(d_x) % 8 == 0, "wd_q8_0_quantize_f16: the input must be 8-byte aligned");
     const int blocks = elements / 32;
-    k_q8_0_quantize_f16<<<dim3((blocks + 31) / 32), dim3(256), 0, as_stream(stream)>>>(d_x, blocks, d_qs, d_scales);
+    enqueue(k_q8_0_quantize_f16, dim3((blocks + 31) / 32), dim3(256), 0, as_stream(stream), d_x, blocks, d_qs, d_scales);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -160,19 +160,19 @@ int wd_gemv_q8_0_q8_1_f32(const uint8_t *d_w, int rows, int cols, const int8_t *
     WD_REQUIRE(rows > 0 && cols > 0 && cols % 32 == 0, "Q8_0 x Q8_1 GEMV geometry mismatch (%d x %d)", rows, cols);
     WD_REQUIRE(d_w && d_qs && d_scales && d_y, "wd_gemv_q8_0_q8_1_f32: null pointer");
     WD_REQUIRE(reinterpret_cast<uintptr_t>(d_qs) % 4 == 0, "wd_gemv_q8_0_q8_1_f32: the quantised input must be 4-byte aligned");
-    k_gemv_q8_0_q8_1<<<dim3((rows + 3) / 4), dim3(256), 0, as_stream(stream)>>>(d_w, rows, cols, d_qs, d_scales, d_y, d_block_sums);
+    enqueue(k_gemv_q8_0_q8_1, dim3((rows + 3) / 4), dim3(256), 0, as_stream(stream), d_w, rows, cols, d_qs, d_scales, d_y, d_block_sums);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
 int wd_convert_f16_to_f32(const uint16_t *d_src, float *d_dst, size_t n, void *stream) {
     WD_REQUIRE(d_src && d_dst && n > 0, "wd_convert_f16_to_f32: invalid arguments");
-    k_f16_to_f32<<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, as_stream(stream)>>>(d_src, d_dst, n);
+    enqueue(k_f16_to_f32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, as_stream(stream), d_src, d_dst, n);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
 int wd_convert_f32_to_f16(const float *d_src, uint16_t *d_dst, size_t n, void *stream) {
     WD_REQUIRE(d_src && d_dst && n > 0, "wd_convert_f32_to_f16: invalid arguments");
-    k_f32_to_f16<<<dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, as_stream(stream)>>>(d_src, d_dst, n);
+    enqueue(k_f32_to_f16, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, as_stream(stream), d_src, d_dst, n);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -181,7 +181,7 @@ int wd_convert_f32_to_f16(const float *d_src, uint16_t *d_dst, size_t n, void *s
 int wd_router_gemv_f32(const float *d_w, const float *d_x, float *d_logits, int rows, int cols, void *stream) {
     WD_REQUIRE(rows > 0 && cols > 0, "router GEMV: invalid shape %d x %d", rows, cols);
     WD_REQUIRE(d_w && d_x && d_logits, "wd_router_gemv_f32: null pointer");
-    k_router_gemv<<<dim3((rows + 7) / 8), dim3(256), 0, as_stream(stream)>>>(d_w, d_x, d_logits, rows, cols, nullptr,
+    enqueue(k_router_gemv, dim3((rows + 7) / 8), dim3(256), 0, as_stream(stream), d_w, d_x, d_logits, rows, cols, nullptr,
                                                                              nullptr);
     WD_LAUNCH_CHECK();
     return WD_OK;
@@ -193,7 +193,7 @@ int wd_topk_softmax(const float *d_logits, int n_experts, int k, float expert_sc
                "top-k softmax: n_experts must be a multiple of 8 in (0, 1024] (got %d)", n_experts);
     WD_REQUIRE(k > 0 && k <= 16 && k <= n_experts, "top-k softmax: k must be in (0, 16] (got %d)", k);
     WD_REQUIRE(d_logits && d_ids && d_weights, "wd_topk_softmax: null pointer");
-    k_topk_softmax<<<dim3(1), dim3(64), 0, as_stream(stream)>>>(d_logits, n_experts, k, expert_scale, d_ids, d_weights,
+    enqueue(k_topk_softmax, dim3(1), dim3(64), 0, as_stream(stream), d_logits, n_experts, k, expert_scale, d_ids, d_weights,
                                                                 nullptr, nullptr);
     WD_LAUNCH_CHECK();
     return WD_OK;
@@ -210,7 +210,7 @@ static void launch_iq_stream(const uint8_t *w, int rows, int nb, const int8_t *q
         // fewer groups than SIMDs: up to eight waves share one
         const int parts = nchunks <= 2 ? 4 : (nchunks <= 4 ? 2 : 1);
         const size_t lds = iq_split_lds<TYPE>(nb, parts);
-        auto launch = [&](auto kernel) { kernel<<<groups, 64 * parts * nchunks, lds, stream>>>(w, rows, nb, parts, qs, d, out, partials); };
+        auto launch = [&](auto kernel) { enqueue(kernel, groups, 64 * parts * nchunks, lds, stream, w, rows, nb, parts, qs, d, out, partials); };
         if (partials) launch(k_gemv_iq_split<TYPE, true>);
         else launch(k_gemv_iq_split<TYPE, false>);
         return;
@@ -218,7 +218,7 @@ static void launch_iq_stream(const uint8_t *w, int rows, int nb, const int8_t *q
     // three workgroups of four waves are what LDS holds per compute unit
     const unsigned wgs = static_cast<unsigned>(std::min((groups + 3) / 4, 768));
     const size_t lds = static_cast<size_t>(nb) * kIqActStride + ((nb * 4 + 15) & ~15) + 4 * kIqWaveStage<TYPE>;
-    auto launch = [&](auto kernel) { kernel<<<wgs, 256, lds, stream>>>(w, rows, nb, qs, d, out, partials); };
+    auto launch = [&](auto kernel) { enqueue(kernel, wgs, 256, lds, stream, w, rows, nb, qs, d, out, partials); };
     if (partials) launch(k_gemv_iq_rows8<TYPE, true>);
     else launch(k_gemv_iq_rows8<TYPE, false>);
 }
@@ -242,14 +242,14 @@ static int launch_gemv_q8k(int type, MatSrc src, int mats, int rows, int cols, c
     const int ppr = partials_per_row(type, cols);
     if (type == WD_TYPE_IQ3_S) {
         if (partials)
-            k_gemv_iq<21, true><<<grid, block, 0, stream>>>(src, rows, cols, qs, d, out, partials, ppr);
+            enqueue(k_gemv_iq<21, true>, grid, block, 0, stream, src, rows, cols, qs, d, out, partials, ppr);
         else
-            k_gemv_iq<21, false><<<grid, block, 0, stream>>>(src, rows, cols, qs, d, out, nullptr, 0);
+            enqueue(k_gemv_iq<21, false>, grid, block, 0, stream, src, rows, cols, qs, d, out, nullptr, 0);
     } else {
         if (partials)
-            k_gemv_iq<22, true><<<grid, block, 0, stream>>>(src, rows, cols, qs, d, out, partials, ppr);
+            enqueue(k_gemv_iq<22, true>, grid, block, 0, stream, src, rows, cols, qs, d, out, partials, ppr);
         else
-            k_gemv_iq<22, false><<<grid, block, 0, stream>>>(src, rows, cols, qs, d, out, nullptr, 0);
+            enqueue(k_gemv_iq<22, false>, grid, block, 0, stream, src, rows, cols, qs, d, out, nullptr, 0);
     }
     WD_LAUNCH_CHECK();
     return WD_OK;
@@ -297,7 +297,7 @@ static void launch_q8_stream(const uint8_t *w, int rows, int nb, const int8_t *q
     const Q8Split sp = q8_split_for(nb, groups);
     if (sp.kb) {
         const size_t lds = q8_split_lds(KIND, sp, nb);
-        auto launch = [&](auto kernel) { kernel<<<groups, 64 * sp.waves, lds, stream>>>(w, rows, nb, qs, d, out, partials); };
+        auto launch = [&](auto kernel) { enqueue(kernel, groups, 64 * sp.waves, lds, stream, w, rows, nb, qs, d, out, partials); };
         if constexpr (KIND == 0) {
             // whole chunks on 16-byte boundaries, the usual row lengths (2048, 2560, 4096, 5120, 8192, 10240, 16384 columns):
             // kernels that know their number of waves (2560 x 2560: 4.97 us, 5.16 with the number taken from nb)
@@ -328,7 +328,7 @@ static void launch_q8_stream(const uint8_t *w, int rows, int nb, const int8_t *q
     const unsigned wgs = static_cast<unsigned>(std::min((groups + 3) / 4, 1024));
     const size_t lds = static_cast<size_t>(nb) * 32 + static_cast<size_t>(nchunks) * kb * 4 +
                        4 * 8 * (kb == 32 ? kQ8sRowStride<KIND, 32> : kQ8sRowStride<KIND, 16>);
-    auto launch = [&](auto kernel) { kernel<<<wgs, 256, lds, stream>>>(w, rows, nb, qs, d, out, partials); };
+    auto launch = [&](auto kernel) { enqueue(kernel, wgs, 256, lds, stream, w, rows, nb, qs, d, out, partials); };
     const bool ragged = q8_ragged(w, nb, kb);
     if (KIND == 1 && kb == 32) {
         if (partials) launch(k_gemv_q8_rows8<1, 32, true, true>);
@@ -378,7 +378,7 @@ static int launch_gemv_q8_0(int type, MatSrc src, int mats, int rows, int cols, 
         int wpb = 0;
         const unsigned wgs = static_cast<unsigned>(q4_stream_wgs(rows, nb, &wpb));
         const size_t lds = static_cast<size_t>(lpr) * (272 + 64);
-        auto launch = [&](auto kernel) { kernel<<<wgs, wpb * 64, lds, stream>>>(src.single, rows, nb, qs, d, out, partials); };
+        auto launch = [&](auto kernel) { enqueue(kernel, wgs, wpb * 64, lds, stream, src.single, rows, nb, qs, d, out, partials); };
         if (partials) {
             if (wpb == 2) ragged ? launch(k_gemv_q4_stream<true, 1, 2, true>) : launch(k_gemv_q4_stream<true, 1, 2, false>);
             else ragged ? launch(k_gemv_q4_stream<true, 1, 4, true>) : launch(k_gemv_q4_stream<true, 1, 4, false>);
@@ -398,9 +398,9 @@ static int launch_gemv_q8_0(int type, MatSrc src, int mats, int rows, int cols, 
 #define WD_Q8_LAUNCH(KIND)                                                                                          \
     do {                                                                                                            \
         if (partials)                                                                                               \
-            k_gemv_q8<KIND, true><<<grid, block, 0, stream>>>(src, rows, cols, qs, d, act_stride, out, partials, ppr); \
+            enqueue(k_gemv_q8<KIND, true>, grid, block, 0, stream, src, rows, cols, qs, d, act_stride, out, partials, ppr); \
         else                                                                                                        \
-            k_gemv_q8<KIND, false><<<grid, block, 0, stream>>>(src, rows, cols, qs, d, act_stride, out, nullptr, 0); \
+            enqueue(k_gemv_q8<KIND, false>, grid, block, 0, stream, src, rows, cols, qs, d, act_stride, out, nullptr, 0); \
     } while (0)
     if (type == WD_TYPE_Q8_0)
         WD_Q8_LAUNCH(0);
@@ -430,7 +430,7 @@ int wd_gemv_q6_k_q8_k_f32(const uint8_t *d_w, int rows, int cols, const int8_t *
     const size_t lds = static_cast<size_t>(nb) * kQ6ActStride + ((nb * 4 + 15) & ~15) + static_cast<size_t>(nb) * 32 + 4 * kQ6StageBytes;
     hipStream_t st = as_stream(stream);
     const bool full = nb % 8 == 0;
-    auto launch = [&](auto kernel) { kernel<<<wgs, 256, lds, st>>>(d_w, rows, cols, d_act_qs, d_act_scales, d_act_bsums, d_out, d_partials); };
+    auto launch = [&](auto kernel) { enqueue(kernel, wgs, 256, lds, st, d_w, rows, cols, d_act_qs, d_act_scales, d_act_bsums, d_out, d_partials); };
     if (d_partials) {
         if (aligned) launch(k_gemv_q6k<true, true, true>);  // aligned implies whole passes
         else if (full) launch(k_gemv_q6k<true, false, true>);
@@ -482,22 +482,26 @@ static int gemv_q4_0_batch(const wd_gemv_item *items, int n_items, int cols, voi
             ++i;
             continue;
         }
-        GemvBatch b{};
-        b.n = j - i;
-        int wgs = 0;
-        bool ragged = false;
-        for (int q = 0; q < b.n; ++q) {
-            const wd_gemv_item &it = items[i + q];
-            b.w[q] = it.d_w, b.act_qs[q] = it.d_act_qs, b.act_d[q] = it.d_act_scales, b.out[q] = it.d_out, b.rows[q] = it.rows;
-            b.first_group[q] = wgs;
-            ragged = ragged || q4_ragged(it.d_w, nb);
-            wgs += q4_batch_wgs(it, nb, &other);
-        }
-        for (int q = b.n; q <= kGemvBatchMax; ++q) b.first_group[q] = wgs;
-        const size_t lds = static_cast<size_t>((nb + 7) / 8) * (272 + 64);
-        auto launch = [&](auto kernel) { kernel<<<wgs, wpb * 64, lds, as_stream(stream)>>>(b, nb); };
-        if (wpb == 2) ragged ? launch(k_gemv_q4_stream_batch<2, true>) : launch(k_gemv_q4_stream_batch<2, false>);
-        else ragged ? launch(k_gemv_q4_stream_batch<4, true>) : launch(k_gemv_q4_stream_batch<4, false>);
+        auto run = [&](auto max) {
+            GemvBatch<decltype(max)::value> b{};
+            b.n = j - i;
+            int wgs = 0;
+            bool ragged = false;
+            for (int q = 0; q < b.n; ++q) {
+                const wd_gemv_item &it = items[i + q];
+                b.w[q] = it.d_w, b.act_qs[q] = it.d_act_qs, b.act_d[q] = it.d_act_scales, b.out[q] = it.d_out, b.rows[q] = it.rows;
+                b.first_group[q] = wgs;
+                ragged = ragged || q4_ragged(it.d_w, nb);
+                wgs += q4_batch_wgs(it, nb, &other);
+            }
+            for (int q = b.n; q <= max; ++q) b.first_group[q] = wgs;
+            const size_t lds = static_cast<size_t>((nb + 7) / 8) * (272 + 64);
+            auto launch = [&](auto kernel) { enqueue(kernel, wgs, wpb * 64, lds, as_stream(stream), b, nb); };
+            if (wpb == 2) ragged ? launch(k_gemv_q4_stream_batch<2, true, max>) : launch(k_gemv_q4_stream_batch<2, false, max>);
+            else ragged ? launch(k_gemv_q4_stream_batch<4, true, max>) : launch(k_gemv_q4_stream_batch<4, false, max>);
+        };
+        if (j - i <= kGemvBatchFew) run(std::integral_constant<int, kGemvBatchFew>{});
+        else run(std::integral_constant<int, kGemvBatchMax>{});
         WD_LAUNCH_CHECK();
         i = j;
     }
@@ -531,29 +535,33 @@ int wd_gemv_q8_0_batch_f32(int type, const wd_gemv_item *items, int n_items, int
             ++i;
             continue;
         }
-        GemvBatch b{};
-        b.n = j - i;
-        int groups = 0;
-        bool ragged = false;
-        for (int q = 0; q < b.n; ++q) {
-            const wd_gemv_item &it = items[i + q];
-            b.w[q] = it.d_w, b.act_qs[q] = it.d_act_qs, b.act_d[q] = it.d_act_scales, b.out[q] = it.d_out, b.rows[q] = it.rows;
-            b.first_group[q] = groups;
-            groups += (it.rows + 7) / 8;
-            ragged = ragged || q8_ragged(it.d_w, nb, sp.kb * sp.nch);
-        }
-        for (int q = b.n; q <= kGemvBatchMax; ++q) b.first_group[q] = groups;
-        const size_t lds = q8_split_lds(0, sp, nb);
-        auto launch = [&](auto kernel) { kernel<<<groups, 64 * sp.waves, lds, as_stream(stream)>>>(b, nb); };
-        bool fixed = false;
+        auto run = [&](auto max) {
+            GemvBatch<decltype(max)::value> b{};
+            b.n = j - i;
+            int groups = 0;
+            bool ragged = false;
+            for (int q = 0; q < b.n; ++q) {
+                const wd_gemv_item &it = items[i + q];
+                b.w[q] = it.d_w, b.act_qs[q] = it.d_act_qs, b.act_d[q] = it.d_act_scales, b.out[q] = it.d_out, b.rows[q] = it.rows;
+                b.first_group[q] = groups;
+                groups += (it.rows + 7) / 8;
+                ragged = ragged || q8_ragged(it.d_w, nb, sp.kb * sp.nch);
+            }
+            for (int q = b.n; q <= max; ++q) b.first_group[q] = groups;
+            const size_t lds = q8_split_lds(0, sp, nb);
+            auto launch = [&](auto kernel) { enqueue(kernel, groups, 64 * sp.waves, lds, as_stream(stream), b, nb); };
+            bool fixed = false;
 #define WD_Q8_SPLIT(KB_, NCH_, WAVES_)                                                                                       \
-    if (!ragged && sp == Q8Split{KB_, NCH_, WAVES_}) launch(k_gemv_q8_rows8_split_batch<KB_, NCH_, WAVES_, false>), fixed = true;
-        WD_Q8_FIXED_SPLITS
+    if (!ragged && sp == Q8Split{KB_, NCH_, WAVES_}) launch(k_gemv_q8_rows8_split_batch<KB_, NCH_, WAVES_, false, max>), fixed = true;
+            WD_Q8_FIXED_SPLITS
 #undef WD_Q8_SPLIT
-        if (fixed) {
-        } else if (sp.kb == 16) launch(k_gemv_q8_rows8_split_batch<16, 1, 0, true>);
-        else if (sp.nch == 1) launch(k_gemv_q8_rows8_split_batch<32, 1, 0, true>);
-        else launch(k_gemv_q8_rows8_split_batch<32, 2, 0, true>);
+            if (fixed) {
+            } else if (sp.kb == 16) launch(k_gemv_q8_rows8_split_batch<16, 1, 0, true, max>);
+            else if (sp.nch == 1) launch(k_gemv_q8_rows8_split_batch<32, 1, 0, true, max>);
+            else launch(k_gemv_q8_rows8_split_batch<32, 2, 0, true, max>);
+        };
+        if (j - i <= kGemvBatchFew) run(std::integral_constant<int, kGemvBatchFew>{});
+        else run(std::integral_constant<int, kGemvBatchMax>{});
         WD_LAUNCH_CHECK();
         i = j;
     }
@@ -583,7 +591,7 @@ int wd_gemv_q8_0_experts_f32(int type, const uint8_t *const *d_w_experts, int ex
 // ---- elementwise ------------------------------------------------------------------------------
 int wd_silu_mul_experts_f32(const float *d_gate_up, float *d_act, int ffn, int experts, void *stream) {
     WD_REQUIRE(ffn > 0 && experts > 0 && d_gate_up && d_act, "silu*up: invalid arguments");
-    k_silu_mul_experts<<<dim3((ffn + 255) / 256, experts), dim3(256), 0, as_stream(stream)>>>(d_gate_up, d_act, ffn);
+    enqueue(k_silu_mul_experts, dim3((ffn + 255) / 256, experts), dim3(256), 0, as_stream(stream), d_gate_up, d_act, ffn);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -591,7 +599,7 @@ int wd_silu_mul_experts_f32(const float *d_gate_up, float *d_act, int ffn, int e
 int wd_weighted_accum_experts_f32(const float *d_experts, const float *d_weights, float *d_accum, int n, int k,
                                   void *stream) {
     WD_REQUIRE(n > 0 && k > 0 && d_experts && d_weights && d_accum, "weighted accumulate: invalid arguments");
-    k_weighted_accum<<<dim3((n + 255) / 256), dim3(256), 0, as_stream(stream)>>>(d_experts, d_weights, d_accum, n, k);
+    enqueue(k_weighted_accum, dim3((n + 255) / 256), dim3(256), 0, as_stream(stream), d_experts, d_weights, d_accum, n, k);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
@@ -599,7 +607,7 @@ int wd_weighted_accum_experts_f32(const float *d_experts, const float *d_weights
 int wd_add_shared_f32(float *d_routed, const float *d_shared, const float *d_gate, int n, void *stream) {
     WD_REQUIRE(n > 0 && d_routed && d_shared && d_gate, "add shared: invalid arguments");
     SiteScope site(WD_SITE_FINISH, as_stream(stream));
-    k_add_shared<<<dim3((n + 255) / 256), dim3(256), 0, as_stream(stream)>>>(d_routed, d_shared, d_gate, d_routed, n);
+    enqueue(k_add_shared, dim3((n + 255) / 256), dim3(256), 0, as_stream(stream), d_routed, d_shared, d_gate, d_routed, n);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
