@@ -61,6 +61,16 @@ def test_layer_shapes(g, oracle, H, F, E, k, gate, down, shared):
     check_layer(g, oracle, L, x, ids=ids, weights=np.linspace(0.3, 0.05, k).astype(np.float32), flags=1)
 
 
+@pytest.mark.parametrize("gate", [Q8, IQ4])
+@pytest.mark.parametrize("H", [256, 768, 1024, 1280, 1536, 2048, 2304, 3072, 3328, 4096, 4352, 6400])
+def test_row_pairs_of_blocks(g, oracle, H, gate):
+    """Gate and up rows (and the shared expert's) of 8 to 200 blocks: passes that end in the first or the second half of the
+    tile, on a whole one, and rows of one, two and more passes."""
+    F, E, k = 96, 16, 3
+    L = synth.make_layer(H, F, E, k, gate, Q8, True, seed=SEED, layer=H, router_sigma=1.0 / np.sqrt(H))
+    check_layer(g, oracle, L, synth.rms_normed(synth.rng_for(SEED, 66, H), H))
+
+
 @pytest.mark.parametrize("H,F,E", [(256, 32, 64), (256, 32, 128), (256, 32, 256), (256, 32, 512), (2048, 512, 64)])
 def test_near_tie_at_the_end_of_a_key_cell(g, oracle, H, F, E):
     """Router rows whose logits are the near-tie row: the layer, a token batch and a stack of one layer (one launch at

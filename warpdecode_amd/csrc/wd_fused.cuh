@@ -1042,7 +1042,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
         const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
         float gu[2];
-        q8_row_wave<0, 2, kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, [&]() {
+        q8_row_pair<0, kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, [&]() {
             lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
             __syncthreads();
         });
@@ -1134,7 +1134,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
             const size_t rb = static_cast<size_t>(nb) * (TYPE == 8 ? 34 : 18);
             const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
             const uint8_t *const rows[2] = {uniform_ptr(gate + off), uniform_ptr(up + off)};
-            q8_row_wave<(TYPE == 8 ? 0 : 1), 2, kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, pre);
+            q8_row_pair<(TYPE == 8 ? 0 : 1), kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, pre);
         }
         if (lane == 0 && r < a.F) act[r] = silu_ggml(gu[0]) * gu[1];
         mark<TRACE>(a, 1, 3);

@@ -655,9 +655,9 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             res_mark<STAMPS>(a, c, l, 11);
             if constexpr (kQ8) {
                 Q8RowTile &tile = *reinterpret_cast<Q8RowTile *>(c.area());
-                float acc[2] = {0.0f, 0.0f};
-                q8_row_wave_pass<0, 2>(gb, true, lane, c.x0q(), c.x0d(), tile, lane, acc, acc);
-                gu[0] = close_lanes8(acc[0]), gu[1] = close_lanes8(acc[1]);
+                float acc = 0.0f;
+                q8_row_pair_pass<0>(gb, true, lane, 64, c.x0q(), c.x0d(), tile, lane, acc, acc);
+                q8_row_pair_close<0>(acc, acc, gu);
             } else {
                 if (decoded) iq_rows8_kept_decoded_dots<kIq>(dec, kept, c.kept(), c.xq(), c.xd(), lane, gu);
                 else iq_rows8_half_decoded_dots<kIq>(dec, tables, c.xq(), c.xd(), lane, gu, c.area());
@@ -793,10 +793,10 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         if (with_shared) {
             res_mark<STAMPS>(a, c, l, 2);
             Q8RowTile &tile = *reinterpret_cast<Q8RowTile *>(c.area());
-            float acc[2] = {0.0f, 0.0f};
-            q8_row_wave_pass<0, 2>(gb, true, lane, c.x0q(), c.x0d(), tile, lane, acc, acc);
-            const float g = close_lanes8(acc[0]), u = close_lanes8(acc[1]);
-            act = silu_ggml(g) * u;
+            float acc = 0.0f, gu[2];
+            q8_row_pair_pass<0>(gb, true, lane, 64, c.x0q(), c.x0d(), tile, lane, acc, acc);
+            q8_row_pair_close<0>(acc, acc, gu);
+            act = silu_ggml(gu[0]) * gu[1];
             res_mark<STAMPS>(a, c, l, 5);
         }
         // Workgroup 0: this wave has time to spare where the router wave has none, so it takes the half of the selection

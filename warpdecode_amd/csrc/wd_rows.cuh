@@ -1252,25 +1252,31 @@ WD_DEV float q8_rows4(const uint8_t *rows, int nrows, int nb, const int8_t *act_
     return q8_rows4_close<KIND>(ch, nb, tile, lane);
 }
 
-// ---- Q8_0 or IQ4_NL x Q8_0, one row per wave ------------------------------------------------------------
-// For long rows (gate/up projections): lane b takes blocks b, b + 64, ...  The chunk sums of a pass
-// are handed over transposed ([chunk][block]) so that the chain lanes read them four at a time.
+// ---- Q8_0 or IQ4_NL x Q8_0, one pair of rows (gate and up) per wave ------------------------------------------------
+// For long rows (gate/up projections): lane b takes blocks b, b + 64, ... of both rows.  The chunk sums are handed over
+// transposed ([chunk][block]) so that the chain lanes read them four at a time, 32 blocks of BOTH rows at a time: columns
+// 0..31 of the tile are the gate row's blocks, columns 32..63 the same blocks of the up row (v_permlane32_swap puts the halves
+// side by side), and lane (m = bit 3, c = bits 0..2) runs chunk c's chain of row m.  What bounds these rows is vector
+// instructions, and the chains were more than half of them: with one row after the other, every lane of the wave repeating
+// the same eight chains, a pair took 128 steps, so 64 - and rows of up to 32 blocks 32 steps, where they took 128 as well.
+// (us per layer, weights from HBM, one row after the other / so: hidden 1024, Q8_0 18.5 / 17.8; 2560 / 640 with a shared expert
+// 29.8 / 28.0; 3072 / 768 IQ4_NL 30.7 / 27.4; 48 layers of 2048 / 512 in one launch, Q8_0 828 / 795, IQ3_S with a shared Q8_0
+// expert and a routing trace 546 / 527.)
 struct Q8RowTile {
-    float pf[8][68];  // [c][block of the pass], rows padded to 68 floats (16-byte aligned, bank spread)
+    float pf[8][68];  // [c][column], rows padded to 68 floats (16-byte aligned, bank spread)
     float ds[64];
 };
 
-// One pass of the row chains: block `bi` of every matrix (wb[i], loaded by the caller; lanes with on == false
-// contribute nothing) against the activation; acc[i] is chunk lane (lane & 7)'s accumulator (IQ4_NL: of the even blocks,
-// acc_odd[i] that of the odd ones).  next(i) runs once the block of matrix i has been used: the place to request the
-// matrix's block of the next pass, so that it travels under this pass's chain.
+// One pass of the row chains: block `bi` of both rows (wb[i], loaded by the caller; lanes with on == false contribute
+// nothing), the pass's `n` blocks being those of lanes 0..n-1, against the activation; acc: the lane's chain (IQ4_NL: of the
+// even blocks, acc_odd that of the odd ones).  next(i) runs once the block of row i has been used: the place to request the
+// row's block of the next pass, so that it travels under this pass's chain.
 struct NoNext {
     WD_DEV void operator()(int) const {}
 };
-template <int KIND, int NM, typename Next = NoNext>
-WD_DEV void q8_row_wave_pass(const Q8Block (&wb)[NM], bool on, int bi, const int8_t *act_qs, const uint16_t *act_d,
-                             Q8RowTile &tile, int lane, float (&acc)[NM], float (&acc_odd)[NM], Next next = Next()) {
-    const int c = lane & 7;
+template <int KIND, typename Next = NoNext>
+WD_DEV void q8_row_pair_pass(const Q8Block (&wb)[2], bool on, int bi, int n, const int8_t *act_qs, const uint16_t *act_d,
+                             Q8RowTile &tile, int lane, float &acc, float &acc_odd, Next next = Next()) {
     uint32_t a[8];
     float dx = 0.0f;
     if (on) {
@@ -1279,73 +1285,92 @@ WD_DEV void q8_row_wave_pass(const Q8Block (&wb)[NM], bool on, int bi, const int
         a[0] = a0.x, a[1] = a0.y, a[2] = a0.z, a[3] = a0.w, a[4] = a1.x, a[5] = a1.y, a[6] = a1.z, a[7] = a1.w;
         dx = h2f(act_d[bi]);
     }
+    float f[2][9];  // the chunk sums, then the scale
 #pragma unroll
-    for (int i = 0; i < NM; ++i) {
+    for (int i = 0; i < 2; ++i) {
         int p[8];
-        float ds = 0.0f;
+        f[i][8] = 0.0f;
         if (on) {
             q8_chunks<KIND>(wb[i], a, p);
-            ds = h2f(wb[i].d) * dx;
+            f[i][8] = h2f(wb[i].d) * dx;
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) p[j] = 0;
         }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[i][j] = static_cast<float>(p[j]);
         next(i);
+    }
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {  // f[0]: blocks 0..31 of the gate row, then of the up row; f[1]: blocks 32..63
+        const wd_uint2v h = __builtin_amdgcn_permlane32_swap(f_bits(f[0][j]), f_bits(f[1][j]), false, false);
+        f[0][j] = bits_f(h.x), f[1][j] = bits_f(h.y);
+    }
+    const int c = lane & 7, col = (lane & 8) * 4;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (half == 1 && n <= 32) break;
         wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
 #pragma unroll
-        for (int j = 0; j < 8; ++j) tile.pf[j][lane] = static_cast<float>(p[j]);
-        tile.ds[lane] = ds;
+        for (int j = 0; j < 8; ++j) tile.pf[j][lane] = f[half][j];
+        tile.ds[lane] = f[half][8];
         wave_lds_fence();
-        // blocks past the end of the row contribute fma(0, 0, acc) == acc
-        // (partial unroll: a full one makes the compiler hold all 128 tile values in registers at once)
-#pragma unroll 4
-        for (int s4 = 0; s4 < 16; ++s4) {
-            const float4 pv = *reinterpret_cast<const float4 *>(&tile.pf[c][4 * s4]);
-            const float4 dv = *reinterpret_cast<const float4 *>(&tile.ds[4 * s4]);
-            float &odd = KIND == 1 ? acc_odd[i] : acc[i];
-            acc[i] = __builtin_fmaf(dv.x, pv.x, acc[i]);
-            odd = __builtin_fmaf(dv.y, pv.y, odd);
-            acc[i] = __builtin_fmaf(dv.z, pv.z, acc[i]);
-            odd = __builtin_fmaf(dv.w, pv.w, odd);
+        // blocks past the end of the rows contribute fma(0, 0, acc) == acc
+        // (sixteen steps at a time: more would have the compiler hold 64 tile values in registers at once)
+#pragma unroll 1
+        for (int q = 0; q < 32 && 32 * half + q < n; q += 16) {
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4) {
+                const float4 pv = *reinterpret_cast<const float4 *>(&tile.pf[c][col + q + 4 * s4]);
+                const float4 dv = *reinterpret_cast<const float4 *>(&tile.ds[col + q + 4 * s4]);
+                float &odd = KIND == 1 ? acc_odd : acc;
+                acc = __builtin_fmaf(dv.x, pv.x, acc);
+                odd = __builtin_fmaf(dv.y, pv.y, odd);
+                acc = __builtin_fmaf(dv.z, pv.z, acc);
+                odd = __builtin_fmaf(dv.w, pv.w, odd);
+            }
         }
     }
 }
+// The results of both rows out of their chains, valid in lane 0.
+template <int KIND>
+WD_DEV void q8_row_pair_close(float acc, float acc_odd, float (&y)[2]) {
+    y[0] = close_lanes8(KIND == 1 ? acc + acc_odd : acc);
+    y[1] = readlane_f(y[0], 8);
+}
 
-// rows[i]: the row of matrix i.  y[i] valid in lane 0 (every aligned group of 8 lanes runs the same chain).
+// rows[i]: row i of the pair; y[i] valid in lane 0.
 // IQ4_NL: an even number of blocks (a trailing unpaired block would not be part of a chain).
-// TWO: rows of 65..128 blocks; the second pass's blocks of a matrix are requested as soon as its first ones have been used
+// TWO: rows of 65..128 blocks; the second pass's blocks of a row are requested as soon as its first ones have been used
 // (otherwise rows of any length, every pass waits for its own blocks).
-template <int KIND, int NM, bool TWO, typename Pre = NoPre>
-WD_DEV void q8_row_wave(const uint8_t *const (&rows)[NM], int nb, const int8_t *act_qs, const uint16_t *act_d,
-                        Q8RowTile &tile, int lane, float (&y)[NM], Pre pre = Pre()) {
+template <int KIND, bool TWO, typename Pre = NoPre>
+WD_DEV void q8_row_pair(const uint8_t *const (&rows)[2], int nb, const int8_t *act_qs, const uint16_t *act_d,
+                        Q8RowTile &tile, int lane, float (&y)[2], Pre pre = Pre()) {
     constexpr int kBlk = (KIND == 0) ? 34 : 18;
-    float acc[NM], acc_odd[NM];
-#pragma unroll
-    for (int i = 0; i < NM; ++i) acc[i] = acc_odd[i] = 0.0f;
+    float acc = 0.0f, acc_odd = 0.0f;
     if constexpr (TWO) {
-        Q8Block wb[NM], wb2[NM];
+        Q8Block wb[2], wb2[2];
 #pragma unroll
-        for (int i = 0; i < NM; ++i) wb[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(lane) * kBlk);
+        for (int i = 0; i < 2; ++i) wb[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(lane) * kBlk);
         pre();
         // (blocks past the row's end are read as its last one and not used, so that no request hangs on a branch)
-        q8_row_wave_pass<KIND, NM>(wb, true, lane, act_qs, act_d, tile, lane, acc, acc_odd, [&](int i) {
+        q8_row_pair_pass<KIND>(wb, true, lane, 64, act_qs, act_d, tile, lane, acc, acc_odd, [&](int i) {
             wb2[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(min(64 + lane, nb - 1)) * kBlk);
         });
-        q8_row_wave_pass<KIND, NM>(wb2, 64 + lane < nb, 64 + lane, act_qs, act_d, tile, lane, acc, acc_odd);
+        q8_row_pair_pass<KIND>(wb2, 64 + lane < nb, 64 + lane, nb - 64, act_qs, act_d, tile, lane, acc, acc_odd);
     } else {
         for (int base = 0; base < nb; base += 64) {
             const int bi = base + lane;
-            Q8Block wb[NM];
+            Q8Block wb[2];
             if (bi < nb) {
 #pragma unroll
-                for (int i = 0; i < NM; ++i) wb[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(bi) * kBlk);
+                for (int i = 0; i < 2; ++i) wb[i] = q8_load<KIND>(rows[i] + static_cast<size_t>(bi) * kBlk);
             }
             if (base == 0) pre();
-            q8_row_wave_pass<KIND, NM>(wb, bi < nb, bi, act_qs, act_d, tile, lane, acc, acc_odd);
+            q8_row_pair_pass<KIND>(wb, bi < nb, bi, min(nb - base, 64), act_qs, act_d, tile, lane, acc, acc_odd);
         }
     }
-#pragma unroll
-    for (int i = 0; i < NM; ++i) y[i] = close_lanes8(KIND == 1 ? acc[i] + acc_odd[i] : acc[i]);
+    q8_row_pair_close<KIND>(acc, acc_odd, y);
 }
 
 // ---- dense Q4_0 x Q8_0 (src/warodecode.cu:1534-1562; no canonical float order) ------------

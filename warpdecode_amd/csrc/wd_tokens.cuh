@@ -135,7 +135,7 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
     const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
     float gu[2];
-    q8_row_wave<0, 2, WIDE>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
+    q8_row_pair<0, WIDE>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
         lds_quantize_q8_0(s.x, a.H, xq, xd, threadIdx.x, 512);
         __syncthreads();
     });
