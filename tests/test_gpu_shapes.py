@@ -61,6 +61,23 @@ def test_layer_shapes(g, oracle, H, F, E, k, gate, down, shared):
     check_layer(g, oracle, L, x, ids=ids, weights=np.linspace(0.3, 0.05, k).astype(np.float32), flags=1)
 
 
+@pytest.mark.parametrize("H,nb,k,down,shared", [
+    (256, 1, 2, IQ4, False),      # one row per workgroup, fewer matrices than waves that fold
+    (512, 16, 3, Q8, False), (768, 17, 6, IQ4, True), (1024, 33, 1, Q8, True), (1024, 48, 8, IQ4, True),
+    (1280, 12, 5, Q8, True), (1280, 13, 3, IQ4, False), (1280, 25, 15, IQ4, True), (1280, 37, 4, Q8, False),
+    (1536, 10, 4, Q8, True), (1536, 9, 4, IQ4, True), (1536, 17, 7, IQ4, False), (1536, 41, 2, IQ4, True),
+    (2304, 13, 6, IQ4, True), (2304, 24, 5, Q8, False), (2304, 36, 8, Q8, True), (2560, 12, 4, IQ4, True), (2560, 37, 6, IQ4, False),
+    (2816, 11, 5, IQ4, False), (2816, 40, 7, Q8, True), (3072, 10, 4, Q8, True), (3072, 31, 5, IQ4, True), (3072, 41, 5, IQ4, False),
+    (3328, 9, 6, IQ4, True), (3328, 27, 5, IQ4, True), (3328, 45, 6, IQ4, False), (3584, 19, 6, IQ4, True), (3584, 37, 7, Q8, False),
+    (3840, 8, 6, Q8, False), (3840, 17, 5, IQ4, True), (4096, 7, 15, IQ4, True), (4096, 33, 6, IQ4, False)])
+def test_rows_per_compute_unit(g, oracle, H, nb, k, down, shared):
+    """Down rows of nb blocks, hidden / 256 rows per workgroup: passes that end on a row's last block, one before and one
+    behind it, an unpaired last IQ4_NL block in passes of even and odd length, rows in one group and in two of equal and unequal size."""
+    F, E = 32 * nb, 16
+    L = synth.make_layer(H, F, E, k, IQ3, down, shared, seed=SEED, layer=H + nb, router_sigma=1.0 / np.sqrt(H))
+    check_layer(g, oracle, L, synth.rms_normed(synth.rng_for(SEED, 67, H + nb), H))
+
+
 @pytest.mark.parametrize("gate", [Q8, IQ4])
 @pytest.mark.parametrize("H", [256, 768, 1024, 1280, 1536, 2048, 2304, 3072, 3328, 4096, 4352, 6400])
 def test_row_pairs_of_blocks(g, oracle, H, gate):

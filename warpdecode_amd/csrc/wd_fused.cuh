@@ -1364,4 +1364,88 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
     mark<TRACE>(a, 2, 4);
 }
 
+// k_layer_c_even: one workgroup for every compute unit, hidden / 256 rows each.  Eight rows per workgroup spread other hidden sizes
+// than 2048 and 4096 unevenly: 2560 is 320 workgroups, two of them on 64 of the 256 compute units, and the dispatch takes as long
+// as those (the second one of a compute unit has its activations quantised 4.3 us after its start, the others 1.9); 1024 leaves
+// half of the compute units without work.  A wave takes its matrix's rows, up to 64 / LPR of them by lanes that hold one block
+// each, or (GROUPS 2) two such groups one after the other: the second one's blocks are requested pass by pass, as the registers of
+// the first one's are free (all of both at once: 2560 / 640 IQ4_NL 8.9 us, so 8.4; 3072 / 768 Q8_0 13.0, 12.4).  As two workgroups per
+// compute unit the groups take 0.3 us more at 2560 and 2.5 more at 3072 / 1024.  (Figures: layer_c_evenly.)
+// grid = 256, block = 64 max(n_act, 2 GROUPS) with at most 16 matrices; waves 0 .. 2 GROUPS - 1 fold up to four rows each.
+// dynamic LDS: per wave the tile and the quantised activation (layer_c_even_wave_bytes), then [n_act][16] floats.
+template <int LPR>
+__host__ __device__ inline uint32_t layer_c_even_wave_bytes(int F) {
+    return ((static_cast<uint32_t>(sizeof(Q8TileN<LPR>)) + 15) & ~15u) + (static_cast<uint32_t>(F + F / 16 + 15) & ~15u);
+}
+template <int KIND, int LPR, int GROUPS, int PASSES>
+__global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
+    constexpr int STEPS = LPR * PASSES <= 48 ? (LPR * PASSES + 15) / 16 : 3;  // of the activation
+    constexpr bool kBoth = GROUPS == 2 && PASSES == 1, kThen = GROUPS == 2 && PASSES > 1;
+    extern __shared__ __align__(16) uint8_t lds_ce[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int n_act = a.k + (a.sh_inp ? 1 : 0), n_waves = max(n_act, 2 * GROUPS);
+    const uint32_t per_wave = layer_c_even_wave_bytes<LPR>(a.F);
+    Q8TileN<LPR> &tile = *reinterpret_cast<Q8TileN<LPR> *>(lds_ce + wave * per_wave);
+    int8_t *aq = reinterpret_cast<int8_t *>(lds_ce + wave * per_wave + ((sizeof(Q8TileN<LPR>) + 15) & ~15u));
+    uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
+    float *ybuf = reinterpret_cast<float *>(lds_ce + n_waves * per_wave);
+    const int R = a.H >> 8, r0 = blockIdx.x * R, nb = a.F >> 5;
+    const int rows0 = GROUPS == 1 ? R : (R + 1) >> 1;
+    if (a.dry) return;
+    if (a.clear_tagged && blockIdx.x == 0)  // (as in k_layer_c)
+        for (int i = threadIdx.x; i < kTagCopies * 16; i += 64 * n_waves)
+            __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    FoldOps ops;
+    const int m = min(wave, n_act - 1);  // (a wave without a matrix of its own repeats the last one's)
+    const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;
+    // (the activation first, as in k_layer_c8)
+    float4 v[2 * STEPS];
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+        const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
+        v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
+    }
+    const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)))) +
+                                            static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
+    auto run = [&](auto kind) {
+        constexpr int K = decltype(kind)::value;
+        const uint8_t *const rows1 = rows + static_cast<uint32_t>(rows0 * nb * (K == 0 ? 34 : 18));
+        const Q8RowsNAt<K, LPR> at0(lane, rows0), at1(lane, R - rows0);
+        Q8Block w[kBoth ? 2 * PASSES : PASSES];
+#pragma unroll
+        for (int q = 0; q < PASSES; ++q) w[q] = q8_rowsn_load<K, LPR>(rows, q * LPR, nb, rows0, at0);
+        if (kBoth) {
+#pragma unroll
+            for (int q = 0; q < PASSES; ++q) w[PASSES + q] = q8_rowsn_load<K, LPR>(rows1, q * LPR, nb, R - rows0, at1);
+        }
+        if (4 * wave < R) ops = layer_c_fold_request(a, r0 + 4 * wave, min(4, R - 4 * wave), lane);
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i)
+            lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
+        wave_lds_fence();
+        Q8Chain ch;
+#pragma unroll
+        for (int q = 0; q < PASSES; ++q) {
+            if (q > 0 && q * LPR >= nb) break;
+            q8_rowsn_pass<K, LPR>(w[q], q * LPR, nb, aq, ad, tile, at0, ch);
+            if (kThen) w[q] = q8_rowsn_load<K, LPR>(rows1, q * LPR, nb, R - rows0, at1);
+        }
+        const float y0 = q8_rowsn_close<K, LPR>(ch, nb, tile, at0);
+        if (wave < n_act && (lane & 7) == 0 && (lane >> 3) < rows0) ybuf[m * 16 + (lane >> 3)] = y0;
+        if constexpr (GROUPS == 1) return;
+        ch = Q8Chain();
+#pragma unroll
+        for (int q = 0; q < PASSES; ++q) {
+            if (q > 0 && q * LPR >= nb) break;
+            q8_rowsn_pass<K, LPR>(w[kBoth ? PASSES + q : q], q * LPR, nb, aq, ad, tile, at1, ch);
+        }
+        const float y1 = q8_rowsn_close<K, LPR>(ch, nb, tile, at1);
+        if (wave < n_act && (lane & 7) == 0 && (lane >> 3) < R - rows0) ybuf[m * 16 + rows0 + (lane >> 3)] = y1;
+    };
+    if (q8) run(std::integral_constant<int, 0>{});
+    else run(std::integral_constant<int, KIND>{});
+    __syncthreads();
+    if (4 * wave < R) layer_c_fold(a, ops, ybuf + 4 * wave, 16, r0 + 4 * wave, min(4, R - 4 * wave), lane);
+}
+
 }  // namespace wd

@@ -611,6 +611,43 @@ void launch_layer_c8(bool words, hipStream_t st, const LayerArgs &a) {
     else words ? launch_layer_c8<KIND, 6, true>(st, a) : launch_layer_c8<KIND, 6, false>(st, a);
 }
 
+template <int KIND, int LPR, int GROUPS, int PASSES = 1>
+void launch_layer_c_even(hipStream_t st, const LayerArgs &a) {
+    // (rows of 48 blocks at most; four passes, then six)
+    if constexpr (PASSES * LPR < 48) {
+        if (a.F > 32 * PASSES * LPR) return launch_layer_c_even<KIND, LPR, GROUPS, (PASSES < 4 ? PASSES + 1 : 6)>(st, a);
+    }
+    const int n_act = a.k + (a.sh_inp ? 1 : 0), waves = std::max(n_act, 2 * GROUPS);
+    const size_t lds = waves * static_cast<size_t>(layer_c_even_wave_bytes<LPR>(a.F)) + sizeof(float) * 16 * n_act;
+    enqueue(k_layer_c_even<KIND, LPR, GROUPS, PASSES>, dim3(256), dim3(64 * waves), lds, st, a);
+}
+template <int KIND>
+void launch_layer_c_even(hipStream_t st, const LayerArgs &a) {
+    const int R = a.H / 256;
+    if (R <= 4) launch_layer_c_even<KIND, 16, 1>(st, a);
+    else if (R == 5) launch_layer_c_even<KIND, 12, 1>(st, a);
+    else if (R == 6) launch_layer_c_even<KIND, 10, 1>(st, a);
+    else if (R <= 10) launch_layer_c_even<KIND, 12, 2>(st, a);
+    else if (R <= 12) launch_layer_c_even<KIND, 10, 2>(st, a);
+    else if (R <= 14) launch_layer_c_even<KIND, 9, 2>(st, a);
+    else launch_layer_c_even<KIND, 8, 2>(st, a);
+}
+// Whether dispatch C takes the form with one workgroup of hidden / 256 rows per compute unit (k_layer_c_even) where the eight-row
+// form would do: us of the dispatch, weights from HBM, eight-row / even.
+//   hidden 512 to 1280, always (256: rows of one workgroup in eight's place, 256 3.3 / 3.5, 1280 8.3 / 7.0): 1024 / 512, ten and the shared expert 6.30 / 5.16; 1024 / 256, eight 4.23 / 4.07; 1280 / 1248, eight 9.83 / 8.69;
+//   1536, where ten lanes a row need fewer passes than eight: 1248 10.2 / 9.1, IQ4_NL 640 6.2 / 5.8, but 512 5.8 / 5.9;
+//   not 1792 (768, eight: 7.0 / 7.2) and 2048 (two groups of four rows, 640 IQ4_NL, ten and the shared one: 7.7 / 8.1);
+//   beyond, where there are waves enough: 2560 / 640 IQ4_NL, ten and the shared one 10.2 / 8.4, 1280 17.9 / 13.1, three matrices of 768 6.1 / 5.8; 3072 /
+//   768, ten and the shared one 13.0 / 12.4, four and the shared one 7.8 / 7.4, but three 6.2 / 6.7; 3328 / 640 IQ4_NL, eight 8.4 / 8.1, four and
+//   the shared one 7.0 / 7.3; 4096 / 256, eight 6.6 / 6.0;
+//   and beyond 3072 not for the bytes that the aligned words are for: 3584 / 1536, eight: 15.1 / 17.4 (2560, ten and the shared one: 19.7 / 16.8).
+bool layer_c_evenly(int H, int F, int n_act, bool words) {
+    const int R = H / 256, nb = F / 32;
+    if (R <= 5) return R > 1 || nb > 16;
+    if (R == 6) return (nb + 9) / 10 < (nb + 7) / 8;
+    return R > 8 && R <= 16 && n_act >= (R <= 12 ? 5 : 6) && !(words && R > 12);
+}
+
 int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
                 const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec = 0,
                 const HcSpec *hc = nullptr) {
@@ -650,7 +687,9 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
         const bool words = static_cast<size_t>(n_act) * wd_tensor_bytes(L->down_type, H, F) >= 32000000 && (q8 || F > 1024) && al16(L->shared_down, 0) &&
                            (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && (L->slot_gate_bytes + L->slot_up_bytes) % 16 == 0
                                               : al16(L->down, L->down_stride));
-        q8 ? launch_layer_c8<0>(words, st, a) : launch_layer_c8<1>(words, st, a);
+        // (chunk sums and time stamps: the eight-row form has them)
+        if (!a.down_part && !a.trace && layer_c_evenly(H, F, n_act, words)) q8 ? launch_layer_c_even<0>(st, a) : launch_layer_c_even<1>(st, a);
+        else q8 ? launch_layer_c8<0>(words, st, a) : launch_layer_c8<1>(words, st, a);
     } else {
         q8 ? launch_layer_c<0>(st, a) : launch_layer_c<1>(st, a);
     }

@@ -1129,6 +1129,70 @@ WD_DEV float q8_rows8_close(const Q8Chain &ch, int nb, const Q8Tile8 &tile, int 
     return (KIND == 1 && (nb & 1)) ? r + tile.tail[lane >> 3] : r;
 }
 
+// ---- the same, LPR lanes per row: up to 64 / LPR rows of LPR blocks each per pass (LPR 8, 9, 10, 12, 16: 8, 7, 6, 5, 4 rows) -----
+// The lanes left over, and those of rows that the group does not have, repeat its last row into parts of the tile that nothing reads.
+template <int LPR>
+struct Q8TileN {
+    static constexpr int kRow = LPR & 1 ? LPR * 8 : LPR * 8 + 8;  // floats: the rows of a read differ in their banks
+    static constexpr int kDs = LPR <= 12 ? 12 : 16;
+    float pf[584];        // [row][b][c]
+    float ds[8 * kDs];    // [row][b]
+    float tail[8];
+};
+template <int KIND, int LPR>
+struct Q8RowsNAt {  // the lane's place: row and block of the pass as it loads, row and chunk as it runs a chain
+    int row, b, chain_row, c;
+    WD_DEV Q8RowsNAt(int lane, int nrows) : row(lane / LPR), b(lane % LPR), chain_row(min(lane >> 3, nrows - 1)), c(lane & 7) {}
+};
+template <int KIND, int LPR>
+WD_DEV Q8Block q8_rowsn_load(const uint8_t *group, int base, int nb, int nrows, const Q8RowsNAt<KIND, LPR> &at) {
+    return q8_load<KIND>(group + static_cast<uint32_t>(min(at.row, nrows - 1) * nb + min(base + at.b, nb - 1)) * (KIND == 0 ? 34 : 18));
+}
+// base: a multiple of LPR that the compiler knows (an IQ4_NL block's accumulator is that of its parity).
+template <int KIND, int LPR>
+WD_DEV void q8_rowsn_pass(const Q8Block &w, int base, int nb, const int8_t *act_qs, const uint16_t *act_d, Q8TileN<LPR> &tile,
+                          const Q8RowsNAt<KIND, LPR> &at, Q8Chain &ch) {
+    using Tile = Q8TileN<LPR>;
+    const int bi = base + at.b, bc = min(bi, nb - 1);
+    const uint4 a0 = *reinterpret_cast<const uint4 *>(act_qs + bc * 32);
+    const uint4 a1 = *reinterpret_cast<const uint4 *>(act_qs + bc * 32 + 16);
+    const uint32_t a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+    int p[8];
+    q8_chunks<KIND>(w, a, p);
+    // (a block past the row's end: fma(0, finite, acc) == acc, the chain's value never being -0)
+    float ds = bi < nb ? h2f(w.d) * h2f(act_d[bc]) : 0.0f;
+    wave_lds_fence();  // earlier reads of the tile are done before it is overwritten
+    if (KIND == 1 && (nb & 1) && bi == nb - 1) {
+        int tot = 0;  // (exact integers below 2^24)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) tot += p[j];
+        tile.tail[at.row] = ds * static_cast<float>(tot);
+        ds = 0.0f;
+    }
+    float4 *dst = reinterpret_cast<float4 *>(&tile.pf[at.row * Tile::kRow + at.b * 8]);
+    dst[0] = make_float4(static_cast<float>(p[0]), static_cast<float>(p[1]), static_cast<float>(p[2]), static_cast<float>(p[3]));
+    dst[1] = make_float4(static_cast<float>(p[4]), static_cast<float>(p[5]), static_cast<float>(p[6]), static_cast<float>(p[7]));
+    tile.ds[at.row * Tile::kDs + at.b] = ds;
+    wave_lds_fence();
+    float dv[Tile::kDs];
+#pragma unroll
+    for (int q = 0; q < (LPR + 3) / 4; ++q) {
+        const float4 d = *reinterpret_cast<const float4 *>(&tile.ds[at.chain_row * Tile::kDs + 4 * q]);
+        dv[4 * q] = d.x, dv[4 * q + 1] = d.y, dv[4 * q + 2] = d.z, dv[4 * q + 3] = d.w;
+    }
+#pragma unroll
+    for (int s = 0; s < LPR; ++s) {
+        float &acc = (KIND == 1 && ((base + s) & 1)) ? ch.odd : ch.acc;
+        acc = __builtin_fmaf(dv[s], tile.pf[at.chain_row * Tile::kRow + s * 8 + at.c], acc);
+    }
+}
+// y of row r, valid in lane 8 r
+template <int KIND, int LPR>
+WD_DEV float q8_rowsn_close(const Q8Chain &ch, int nb, const Q8TileN<LPR> &tile, const Q8RowsNAt<KIND, LPR> &at) {
+    const float r = close_lanes8(KIND == 1 ? ch.acc + ch.odd : ch.acc);
+    return (KIND == 1 && (nb & 1)) ? r + tile.tail[at.chain_row] : r;
+}
+
 // ---- Q8_0 / IQ4_NL x Q8_0, four rows of 16 or 20 blocks, aligned fetch -----------------------------------------
 // Four consecutive rows of NB blocks (NB = 16 or 20; Q8_0 or IQ4_NL) that start on a 16-byte boundary: 4 NB blocks are a
 // whole number of 16-byte words (136 NB or 72 NB bytes), fetched as aligned words, copied to LDS and cut into blocks
