@@ -147,6 +147,15 @@ def test_tensors_on_two_byte_boundaries(g, oracle, monkeypatch, H, F, k):
     (512, 800, 16, 4, IQ3, Q8, True, 5),         # 25 and 32 down blocks
     (768, 1024, 16, 3, IQ2, IQ4, False, 8),
     (3072, 1536, 16, 10, IQ4, IQ4, True, 2),     # 48 down blocks
+    (256, 288, 16, 3, IQ3, IQ4, True, 4),        # hidden / 256 rows per workgroup: nine blocks
+    (768, 1440, 16, 6, IQ3, Q8, True, 7),
+    (1024, 512, 16, 4, IQ2, IQ4, False, 5),
+    (1280, 1184, 16, 5, IQ3, IQ4, True, 8),      # 37
+    (1536, 1312, 16, 10, IQ2, Q8, True, 3),      # 41
+    (2304, 800, 16, 3, IQ3, IQ4, True, 5),       # two groups of five and four rows, 25 blocks
+    (2560, 1152, 16, 6, IQ2, Q8, False, 2),
+    (2816, 1312, 16, 2, IQ3, IQ4, True, 6),      # six and five rows, 41 blocks
+    (3072, 1216, 16, 4, IQ2, Q8, True, 8),
     (1024, 1568, 16, 2, IQ2, Q8, True, 6)])      # 49: the one-token dispatch per token
 def test_token_batch_shapes(g, oracle, H, F, E, k, gate, down, shared, T):
     import ctypes as C

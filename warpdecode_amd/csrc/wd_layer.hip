@@ -973,6 +973,31 @@ void launch_tokens_b(const wd_moe_layer *L, const TokenArgs &ta, int items, int 
     else if (H <= 2304) launch_tokens_b_fetch<TYPE, 1>(ta, items, cus, st);
     else launch_tokens_b_fetch<TYPE, 2>(ta, items, cus, st);
 }
+template <int KIND, int LPR, int PASSES = 1>
+void launch_tokens_c_even(const TokenArgs &ta, hipStream_t st) {
+    if constexpr (PASSES * LPR < 48) {  // (as in launch_layer_c_even)
+        if (ta.common.F > 32 * PASSES * LPR) return launch_tokens_c_even<KIND, LPR, (PASSES < 4 ? PASSES + 1 : 6)>(ta, st);
+    }
+    const size_t lds = kTokensCEvenWaves * static_cast<size_t>(layer_c_even_wave_bytes<LPR>(ta.common.F)) + sizeof(float) * 16 * ta.T * (ta.common.k + 1);
+    enqueue(k_tokens_c_even<KIND, LPR, PASSES>, dim3(256), dim3(64 * kTokensCEvenWaves), lds, st, ta);
+}
+// Lanes per row of the form with hidden / 256 rows per workgroup (k_tokens_c_even), 0 where the eight-row form stays: it pays where
+// the rows take fewer passes than with eight lanes each, for more than 16 blocks (up to hidden 1024: for all).  us per layer of the
+// whole pass, weights from HBM, eight-row / even: four tokens, top-8 and the shared expert, 736: hidden 512 44.3 / 40.8, 1280 47.3 / 44.6, 2304 69.7 /
+// 64.9, but (three passes either way) 1536 47.4 / 47.3, 3072 71.9 / 73.4; seven tokens, top-5, IQ4_NL of 1184: 1024 70.8 / 57.9, 1536
+// 73.7 / 64.6, 2560 96.1 / 86.8, 3072 111 / 104; five, top-4, IQ4_NL of 480: 1024 30.0 / 29.3, but (two passes either way) 2304
+// 40.2 / 41.1.  Beyond hidden 3072, where the groups are of seven and eight rows, nothing is left: 3584 / 1184 113.5 / 113.1, 736 73.9 / 75.3.
+int tokens_c_even_lanes(int H, int F) {
+    const int R = H / 256, nb = F / 32;
+    const int lanes = R <= 4 ? 16 : (R == 5 || R == 9 || R == 10 ? 12 : (R == 6 || R == 11 || R == 12 ? 10 : 8));
+    return (nb > 16 || R <= 4) && (nb + lanes - 1) / lanes < (nb + 7) / 8 ? lanes : 0;
+}
+template <int KIND>
+void launch_tokens_c_even(int lanes, const TokenArgs &ta, hipStream_t st) {
+    if (lanes == 16) launch_tokens_c_even<KIND, 16>(ta, st);
+    else if (lanes == 12) launch_tokens_c_even<KIND, 12>(ta, st);
+    else launch_tokens_c_even<KIND, 10>(ta, st);
+}
 template <int KIND, int PASSES>
 void launch_tokens_c(const TokenArgs &ta, hipStream_t st) {
     constexpr int kWaves = kTokensCWaves<PASSES>;
@@ -1069,7 +1094,8 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
                 return rc;
         return WD_OK;
     }
-    L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c<0>(ta, st) : launch_tokens_c<1>(ta, st);
+    if (const int lanes = tokens_c_even_lanes(H, F)) L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c_even<0>(lanes, ta, st) : launch_tokens_c_even<1>(lanes, ta, st);
+    else L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c<0>(ta, st) : launch_tokens_c<1>(ta, st);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }

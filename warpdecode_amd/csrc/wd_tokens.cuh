@@ -30,6 +30,16 @@ WD_DEV const uint8_t *mat_ptr_entry(const MatSrc &s, int e) {
     return mat_ptr_expert<T>(s, e);
 }
 
+template <int T>
+WD_DEV const uint8_t *mat_ptr_entry_uniform(const MatSrc &s, int e) {  // e the same in every lane: through the scalar path
+    if (s.table) {
+        const uint8_t *const *p = s.table + (static_cast<unsigned>(e) < static_cast<unsigned>(kPairEntries) ? e : 0) * s.per_expert + T;
+        const uint32_t lo = static_cast<uint32_t>(sld_i32(reinterpret_cast<const int32_t *>(p))), hi = static_cast<uint32_t>(sld_i32(reinterpret_cast<const int32_t *>(p) + 1));
+        return reinterpret_cast<const uint8_t *>((static_cast<uintptr_t>(hi) << 32) | lo);
+    }
+    return mat_ptr_expert_uniform<T>(s, e);
+}
+
 struct TokenSlots {
     const float *x;
     float *logits;
@@ -593,6 +603,120 @@ void k_tokens_c(TokenArgs ta) {
             float o = acc;
             if (shared) {
                 const float y = ybuf[(t * (a.k + 1) + a.k) * 8 + lane];
+                const float prod = y * gate;
+                o = acc + prod;
+                s.down_f32[row] = y;
+            }
+            s.accum[row] = acc;
+            s.out[row] = o;
+        }
+    }
+    mark(a, 2, 6);
+}
+
+// The same with one workgroup of sixteen waves for every compute unit, hidden / 256 rows each, as in k_layer_c_even: a work item is
+// (token, matrix, group of up to 64 / LPR rows).  (The next item's activation and rows requested while this one is worked on: 2560 / 640,
+// four tokens 63.8 us per layer instead of 61.7, 4096 / 1536 128.8 instead of 119.2.)  Where it is taken and what it measures: tokens_c_even_lanes.
+// grid = 256.  dynamic LDS: per wave the tile and the quantised activation (layer_c_even_wave_bytes), then [T][k+1][16] floats.
+constexpr int kTokensCEvenWaves = 16;
+template <int KIND, int LPR, int PASSES>
+__global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenArgs ta) {
+    constexpr int kWaves = kTokensCEvenWaves, kActs = LPR * PASSES <= 48 ? (LPR * PASSES + 15) / 16 : 3;
+    extern __shared__ __align__(16) uint8_t lds_tc[];
+    const LayerArgs &a = ta.common;
+    const int lane = threadIdx.x & 63, tw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const uint32_t per_wave = layer_c_even_wave_bytes<LPR>(a.F);
+    Q8TileN<LPR> &tile = *reinterpret_cast<Q8TileN<LPR> *>(lds_tc + tw * per_wave);
+    int8_t *aq = reinterpret_cast<int8_t *>(lds_tc + tw * per_wave + ((sizeof(Q8TileN<LPR>) + 15) & ~15u));
+    uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
+    float *ybuf = reinterpret_cast<float *>(lds_tc + kWaves * per_wave);  // [T][k+1][16]
+    const bool shared = a.sh_down != nullptr;
+    const int rows_per_wg = a.H >> 8, r0 = blockIdx.x * rows_per_wg, nb = a.F >> 5;
+    const int n_groups = rows_per_wg * LPR > 64 ? 2 : 1, rows0 = n_groups == 2 ? (rows_per_wg + 1) >> 1 : rows_per_wg;
+    mark(a, 2, 0);
+    // every routed id of the pass, one vector load per wave; an item's id is then a lane read
+    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
+    // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
+    float wreg;
+    {
+        const TokenSlots &s = ta.tok[min(tw, ta.T - 1)];
+        const float *src = (lane == 16 && shared) ? s.shared_gate : s.weights + min(lane, a.k - 1);
+        wreg = *src;
+    }
+    // items [begin, end): of `per_token` matrices from number `first` on for every token
+    auto run = [&](auto kind, int first, int per_token, int begin, int end) {
+        constexpr int K = decltype(kind)::value, kBlk = K == 0 ? 34 : 18;
+        struct Item {
+            const float *act;
+            const uint8_t *rows;
+            int nrows, y;  // y: where the results go in ybuf
+        };
+        auto item_at = [&](int i) {
+            const int g = n_groups == 2 ? i & 1 : 0, pair = n_groups == 2 ? i >> 1 : i;
+            const int t = pair / per_token, j = first + (pair - t * per_token);
+            const int p = t * a.k + min(j, a.k - 1);
+            const int e = p < 64 ? __builtin_amdgcn_readlane(id_lo, p) : __builtin_amdgcn_readlane(id_hi, p - 64);
+            Item it;
+            it.nrows = g ? rows_per_wg - rows0 : rows0;
+            it.act = ta.tok[t].act + static_cast<size_t>(j) * a.F;
+            it.rows = uniform_ptr((j == a.k ? a.sh_down : mat_ptr_entry_uniform<0>(a.down, e)) + static_cast<size_t>(r0 + g * rows0) * nb * kBlk);
+            it.y = (t * (a.k + 1) + j) * 16 + g * rows0;
+            return it;
+        };
+        for (int i = begin; i < end; i += kWaves) {
+            const Item it = item_at(i);
+            float4 v[2 * kActs];
+#pragma unroll
+            for (int q = 0; q < kActs; ++q) {
+                const float *p = it.act + min(512 * q + lane * 8, a.F - 8);
+                v[2 * q] = *reinterpret_cast<const float4 *>(p), v[2 * q + 1] = *reinterpret_cast<const float4 *>(p + 4);
+            }
+            const Q8RowsNAt<K, LPR> at(lane, it.nrows);
+            Q8Block w[PASSES];
+#pragma unroll
+            for (int q = 0; q < PASSES; ++q) w[q] = q8_rowsn_load<K, LPR>(it.rows, q * LPR, nb, it.nrows, at);
+            wave_lds_fence();
+#pragma unroll
+            for (int q = 0; q < kActs; ++q)
+                lds_quantize_q8_0_step(v[2 * q], v[2 * q + 1], 512 * q + lane * 8 < a.F, 512 * q + lane * 8, aq, ad, lane);
+            wave_lds_fence();
+            Q8Chain ch;
+#pragma unroll
+            for (int q = 0; q < PASSES; ++q)
+                if (q == 0 || q * LPR < nb) q8_rowsn_pass<K, LPR>(w[q], q * LPR, nb, aq, ad, tile, at, ch);
+            const float y = q8_rowsn_close<K, LPR>(ch, nb, tile, at);
+            if ((lane & 7) == 0 && (lane >> 3) < it.nrows) ybuf[it.y + (lane >> 3)] = y;
+            mark(a, 2, i == tw ? 2 : 3);
+        }
+    };
+    if (KIND == 0) {
+        run(std::integral_constant<int, 0>{}, 0, a.k + (shared ? 1 : 0), tw, ta.T * (a.k + (shared ? 1 : 0)) * n_groups);
+    } else {
+        const int routed = ta.T * a.k * n_groups;
+        run(std::integral_constant<int, KIND>{}, 0, a.k, tw, routed);
+        // the waves that have one routed item less begin with the shared ones
+        if (shared) run(std::integral_constant<int, 0>{}, a.k, 1, (tw - routed) & (kWaves - 1), ta.T * n_groups);
+    }
+    __syncthreads();
+    mark(a, 2, 5);
+    if (tw < ta.T) {
+        const TokenSlots &s = ta.tok[tw];
+        const int t = tw;
+        const int row = r0 + lane;
+        const bool row_on = lane < rows_per_wg;
+        float acc = 0.0f;
+        for (int j = 0; j < a.k; ++j) {
+            const float wj = lane_get(wreg, j);
+            const float y = ybuf[(t * (a.k + 1) + j) * 16 + (lane & 15)];
+            const float prod = y * wj;
+            acc = acc + prod;
+            if (s.expert_out && row_on) s.expert_out[static_cast<size_t>(j) * a.H + row] = y;
+        }
+        const float gate = lane_get(wreg, 16);
+        if (row_on) {
+            float o = acc;
+            if (shared) {
+                const float y = ybuf[(t * (a.k + 1) + a.k) * 16 + lane];
                 const float prod = y * gate;
                 o = acc + prod;
                 s.down_f32[row] = y;
