@@ -429,7 +429,9 @@ int wd_expert_cache_set_timing(wd_expert_cache *c, int enabled);
  * the geometry wd_moe_stack_f32 runs as one launch, the whole token is acquired ahead and runs as ONE resident launch
  * that waits, layer by layer, for the fills still on their way (they run beside it on the cache's stream;
  * WD_MOE_PER_LAYER in `flags` keeps the dispatches per layer; the results are the same bits).  Without a trace each
- * layer's ids go to the host first, as in
+ * layer's ids go to the host: with flags 0 or WD_MOE_KEEP_EXPERT_OUT the layer's first dispatch reports them and goes on with
+ * the experts that have slots (those without are computed once the host has acquired them); with other flags, chunk sums kept
+ * or the site profiler on, the host waits for them first, as in
  * the reference's loop (q38_moe_select_experts_f32_x + GpuExpertCache::acquire per selected expert,
  * src/qwen38_moe.cuh:2323-2380, :3650-3779).  Counters: wd_expert_cache_get_stats. */
 int wd_moe_stack_cached_f32(const wd_moe_layer *layers, int n_layers, wd_expert_cache *cache, float *d_x,

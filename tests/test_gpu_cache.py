@@ -351,3 +351,43 @@ def test_monitor_and_shadow_caches(g):
     assert d["tokens"] == 40 and d["intra_gap_ms"] == 0.0 and d["layer_gap_ms"] > 0.0
     assert abs(d["layer_gap_per_token"] - d["layer_gap_ms"] / 40) < 0.011 and d["acquire_per_token"] > 0.0
     capi.call("wd_expert_cache_destroy", cache)
+
+
+@pytest.mark.parametrize("H,F,E,k,gate,down,shared,slots,partition", [
+    (256, 64, 24, 16, synth.IQ3_S, synth.Q8_0, True, 51, 1),    # top-16 of 17 slots per layer
+    (512, 96, 16, 2, synth.Q8_0, synth.IQ4_NL, False, 5, 0),    # fewer slots than a token takes
+    (256, 32, 16, 3, synth.IQ4_NL, synth.Q8_0, True, 48, 0)])   # every expert fits: hits once they are there
+def test_selections_reported_to_the_host(g, H, F, E, k, gate, down, shared, slots, partition):
+    """Stacks without a trace, one call after the other without a synchronisation, selections that hit, miss and evict: the
+    bits of the stack on resident tensors, whose pointers the layers do not have, and every access counted once."""
+    import torch
+    NL, tokens = 3, 12
+    layers = [synth.make_layer(H, F, E, k, gate, down, shared, seed=SEED, layer=200 + l, router_sigma=1.0 / np.sqrt(H)) for l in range(NL)]
+    gb, db = F * synth.row_bytes(gate, H), H * synth.row_bytes(down, F)
+    cache, pinned = C.c_void_p(), []
+    capi.call("wd_expert_cache_create", C.byref(cache), slots * (2 * gb + db), gb, gb, db, NL, E, partition)
+    dls = [g.DeviceLayer(L) for L in layers]
+    whole = (capi.MoeLayer * NL)(*[d.desc for d in dls])
+    bare = (capi.MoeLayer * NL)(*[d.desc for d in dls])
+    for l, L in enumerate(layers):
+        p = [torch.from_numpy(np.ascontiguousarray(L[n]).reshape(-1)).pin_memory() for n in ("gate", "up", "down")]
+        pinned.append(p)
+        capi.call("wd_expert_cache_register_layer", cache, l, *[C.c_void_p(t.data_ptr()) for t in p])
+        bare[l].gate = bare[l].up = bare[l].down = None
+    xs = np.stack([synth.rms_normed(synth.rng_for(SEED, 83, t // 2), H) for t in range(tokens)])   # every input twice
+    sc, sc2 = g.Scratch(H, F, E, k), g.Scratch(H, F, E, k)
+    dx, dx2, out, out2 = g.dev(xs), g.dev(xs), g.empty((tokens, H), np.float32), g.empty((tokens, H), np.float32)
+    for t in range(tokens):
+        at = [C.c_void_p(b.data_ptr() + 4 * H * t) for b in (dx, out, dx2, out2)]
+        capi.call("wd_moe_stack_cached_f32", bare, NL, cache, at[0], at[1], sc.h, None, None, 0.05, 0, g.stream())
+        capi.call("wd_moe_stack_f32", whole, NL, at[2], at[3], sc2.h, None, 0.05, 0, g.stream())
+    g.sync()
+    assert g.same_bits(g.host(dx), g.host(dx2)) and g.same_bits(g.host(out), g.host(out2))
+    assert capi.load().wd_moe_scratch_status(sc.h) == 0
+    st = capi.CacheStats()
+    capi.call("wd_expert_cache_get_stats", cache, C.byref(st))
+    assert st.accesses == tokens * NL * k == st.hits + st.misses and st.misses > 0
+    assert (st.evictions > 0) == (slots < NL * E) and (slots < NL * k or st.hits >= tokens // 2 * NL)
+    sc.close()
+    sc2.close()
+    capi.call("wd_expert_cache_destroy", cache)

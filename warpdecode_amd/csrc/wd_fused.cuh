@@ -52,6 +52,7 @@ struct LayerArgs {
     // the PART variants of the dispatches also store the exact int32 chunk sums of the routed rows:
     int32_t *gup_part;           // [k][2][F][8 * H / 256]
     int32_t *down_part;          // [k][H][8 * F / 32]
+    uint32_t *host_ids;          // null, or [k] in host memory: dispatch AB reports its selection
 };
 
 constexpr int kTagCopies = 16;           // replicas of the published ids, 64 bytes apart, so that pollers spread over lines
@@ -1023,6 +1024,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
                     if (lane < a.k) {
                         a.ids[lane] = lds_ids[lane];
                         a.weights[lane] = lds_w[lane];
+                        if (a.host_ids) __hip_atomic_store(a.host_ids + lane, static_cast<uint32_t>(lds_ids[lane]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                     }
                     if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
                 }

@@ -38,8 +38,9 @@ struct wd_moe_scratch {
     unsigned *arrive = nullptr;           // device counter used inside the fused dispatch A
     unsigned long long *trace = nullptr;  // device [3][16][8] time stamps, see wd_moe_scratch_trace
     int trace_wg = 0;
-    int32_t *h_ids = nullptr;             // pinned [32]: [0..15] routed ids for callers that must see them on the host,
-                                          // [16] mirror of the status word, written by the resident launch when a wait runs out
+    int32_t *h_ids = nullptr;             // pinned [48]: [0..15] routed ids for callers that must see them on the host,
+                                          // [16] mirror of the status word, written by the resident launch when a wait runs out,
+                                          // [32..47] the selection as dispatch AB reports it (cached_routed_reported)
     uint32_t *tagged = nullptr;           // [kTagRecords][kTagCopies][16] ids published inside the merged dispatch
     unsigned *status = nullptr;           // [0] != 0: a bounded wait inside a dispatch ran out
     unsigned spin_limit = kSpinLimit;
@@ -134,12 +135,12 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
     s->status = reinterpret_cast<unsigned *>(b + o_status);
     (void)hipMemset(s->block, 0, c.off);
     (void)hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16);
-    if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 32, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 48, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->block);
         delete s;
         return fail(WD_ERR_HIP, "hipHostMalloc MoE scratch ids failed");
     }
-    std::memset(s->h_ids, 0, sizeof(int32_t) * 32);
+    std::memset(s->h_ids, 0, sizeof(int32_t) * 48);
     *out = s;
     return WD_OK;
 }
@@ -648,12 +649,15 @@ bool layer_c_evenly(int H, int F, int n_act, bool words) {
     return R > 8 && R <= 16 && n_act >= (R <= 12 ? 5 : 6) && !(words && R > 12);
 }
 
+// report: null, or the host words that dispatch AB reports its selection to.  An expert without a slot is then no error: its
+// rows are computed again once it has one.
 int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
                 const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec = 0,
-                const HcSpec *hc = nullptr) {
+                const HcSpec *hc = nullptr, uint32_t *report = nullptr) {
     const int H = L->hidden, F = L->expert_ffn, k = L->top_k;
     const bool shared = L->shared_gate_inp != nullptr;
-    const LayerArgs a = fused_args(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, rec, hc);
+    LayerArgs a = fused_args(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, rec, hc);
+    if (report) a.host_ids = report, a.gate_up.slot_status = nullptr;
     const unsigned only = flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B | WD_MOE_ONLY_C);
     const bool run_a = !only || (only & WD_MOE_ONLY_A), run_b = !only || (only & WD_MOE_ONLY_B);
     // router + selection + shared gate/up + routed gate/up in one launch (the routed workgroups wait for the ids

@@ -5,10 +5,83 @@
 // With a routing trace known to the host and a pool that holds at least two tokens' experts, the experts of all
 // layers are acquired before the first layer is launched and every layer waits for its own fills only: the host
 // link streams the token's misses back to back under the layers' compute.  With a smaller pool the fills of layer
-// l+1 are queued before layer l is launched and waited for after it.  Without one, every layer
-// does what the reference does (src/qwen38_moe.cuh:2323-2380): router and selection, ids to pinned host
-// memory, stream synchronisation, acquire, expert dispatches.
+// l+1 are queued before layer l is launched and waited for after it.  Without one, dispatch AB of a layer reports its
+// selection to the host while it goes on (cached_routed_reported), or every layer does what the reference does
+// (src/qwen38_moe.cuh:2323-2380): router and selection, ids to pinned host memory, stream synchronisation, acquire,
+// expert dispatches.
 using namespace wd;
+
+namespace {
+
+// Waits until dispatch AB has reported its k ids.  The stream is looked at now and then, so that work that ended without a
+// report (an earlier error of the device) ends the wait as well.
+int wait_report(const volatile uint32_t *rec, int k, hipStream_t st) {
+    for (unsigned polls = 1;; ++polls) {
+        bool ended = false;
+        if (polls % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) (void)hipGetLastError();
+            ended = e != hipErrorNotReady;
+        }
+        int there = 0;
+        while (there < k && rec[there] != kTagInvalid) ++there;
+        if (there == k) return WD_OK;
+        if (ended) {
+            WD_HIP(hipStreamSynchronize(st));
+            return fail(WD_ERR_STATE, "cached MoE stack: a layer's selection was not reported");
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+// The merged dispatch AB of a layer reports its selection to host memory and goes on with the experts that are in their slots.
+// Where that is all of them the host launches the layer's dispatch C and the next layer's AB at once, while AB still runs, and keeps
+// the cache's books behind that (an acquire of hits has no work for the device): the device does not wait for the host.  Where an
+// expert is missing, the host acquires and launches the layer's gate/up once more, on the selection that is in the scratch, ahead
+// of C.  (Router and selection as a dispatch of their own, the copied ids and the synchronisation left the device idle for half of
+// every layer: 2048 / 512, 128 experts, eight layers, nearly all hits: 297 us, so 176; three layers of 1792 / 224, all hits, 95 / 55.)
+int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cache *cache, float *d_x, float *d_layer_out, wd_moe_scratch *s,
+                           float residual_scale, unsigned flags, hipStream_t st) {
+    if (cache->fills_pending)
+        if (const int rc = wait_fills(cache, st)) return rc;
+    uint32_t *const report = reinterpret_cast<uint32_t *>(s->h_ids + 32);
+    auto launch = [&](size_t l, unsigned parts, bool reports) {
+        return layer_fused(&bound[l], d_x, d_layer_out, s, flags | parts, nullptr, d_x, residual_scale, st, 0, nullptr, reports ? report : nullptr);
+    };
+    auto launch_ab = [&](size_t l) {
+        for (int j = 0; j < 16; ++j) reinterpret_cast<volatile uint32_t *>(report)[j] = kTagInvalid;
+        return launch(l, WD_MOE_ONLY_A | WD_MOE_ONLY_B, true);
+    };
+    if (const int rc = launch_ab(0)) return rc;
+    for (size_t l = 0; l < bound.size(); ++l) {
+        const int k = bound[l].top_k;
+        if (const int rc = wait_report(report, k, st)) return rc;
+        bool resident = true;
+        for (int j = 0; j < k; ++j) {
+            s->h_ids[j] = static_cast<int32_t>(report[j]);
+            resident = resident && cache->index.find((static_cast<uint64_t>(l) << 32) | report[j]) != cache->index.end();
+        }
+        int rc = WD_OK;
+        if (!resident) {
+            rc = wd_expert_cache_acquire(cache, static_cast<int>(l), s->h_ids, k, nullptr, st);
+            if (rc) {  // (dispatch C, which makes the published ids invalid again, does not follow)
+                enqueue(k_fill_u32, dim3(1), dim3(kTagCopies * 16), 0, st, s->tagged, kTagInvalid, static_cast<size_t>(kTagCopies) * 16);
+                return rc;
+            }
+            rc = launch(l, WD_MOE_ONLY_B, false);
+        }
+        if (rc == WD_OK) rc = launch(l, WD_MOE_ONLY_C, false);
+        if (rc == WD_OK && l + 1 < bound.size()) rc = launch_ab(l + 1);
+        if (resident) {
+            const int rc_books = wd_expert_cache_acquire(cache, static_cast<int>(l), s->h_ids, k, nullptr, st);
+            if (rc == WD_OK) rc = rc_books;
+        }
+        if (rc) return rc;
+    }
+    return WD_OK;
+}
+
+}  // namespace
 
 extern "C" int wd_moe_stack_cached_f32(const wd_moe_layer *layers, int n_layers, wd_expert_cache *cache, float *d_x,
                                        float *d_layer_out, wd_moe_scratch *s, const int32_t *h_ids_trace,
@@ -99,6 +172,21 @@ extern "C" int wd_moe_stack_cached_f32(const wd_moe_layer *layers, int n_layers,
         return WD_OK;
     }
 
+    {
+        // Layers that every acquire can serve, in a call that nobody records or brackets stage by stage
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        bool reported = (flags & ~WD_MOE_KEEP_EXPERT_OUT) == 0 && !per_layer && s->gup == nullptr && !SiteProfiler::instance().enabled() &&
+                        hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+        (void)hipGetLastError();  // (a stream that may not be asked is not an error of this call)
+        std::vector<wd_moe_layer> bound;
+        bound.reserve(n_layers);
+        for (int l = 0; reported && l < n_layers; ++l) {
+            bound.push_back(bind(l));
+            const Partition &P = cache->parts[cache->partitioned ? l : 0];
+            reported = cache->h_gate[l] != nullptr && P.end - P.begin >= static_cast<size_t>(bound[l].top_k);
+        }
+        if (reported) return cached_routed_reported(bound, cache, d_x, d_layer_out, s, residual_scale, flags, st);
+    }
     for (int l = 0; l < n_layers; ++l) {
         const wd_moe_layer L = bind(l);
         // dispatch A also carries the shared expert's gate/up rows and its gate: it runs whenever there is something in it
