@@ -981,15 +981,18 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (a.dry) return;
     const int groups = (a.F + 7) / 8;
+    // (known where the fetch is made for it: the router's row loops then need no bounds.  us per layer from HBM: 2048 / 512, 256 experts 19.4
+    // / 18.4, 2048 / 768 21.4 / 20.4, 2560 / 640 25.9 / 25.2)
+    const int H = FETCH == 8 ? 2048 : (FETCH == 10 ? 2560 : a.H);
 
     mark<TRACE>(a, wg < a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);
     if (wg < a.n_router_wgs) {
         const int rows = a.preselected ? 0 : a.E;
         if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
             router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.logits, rows,
-                                  a.H, a.sh_inp, a.shared_gate, wg);
+                                  H, a.sh_inp, a.shared_gate, wg);
         else
-            router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.logits, rows, a.H, a.sh_inp,
+            router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.logits, rows, H, a.sh_inp,
                                    a.shared_gate, wg);
         mark<TRACE>(a, 0, 1);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -1035,17 +1038,17 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     }
 
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ab);
-    uint8_t *xscale = lds_ab + a.H;  // Q8_K: f32 [H/256]; Q8_0: f16 [H/32]
+    uint8_t *xscale = lds_ab + H;  // Q8_K: f32 [H/256]; Q8_0: f16 [H/32]
     if (wg < a.n_router_wgs + a.n_shared_wgs) {
         Q8RowTile *tiles = reinterpret_cast<Q8RowTile *>(s_union);
         const int r = (wg - a.n_router_wgs) * 8 + wave;
-        const int nb = a.H >> 5;
+        const int nb = H >> 5;
         const size_t rb = static_cast<size_t>(nb) * 34;
         const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
         const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
         float gu[2];
         q8_row_pair<0, kTwoPasses>(rows, nb, xq, reinterpret_cast<const uint16_t *>(xscale), tiles[wave], lane, gu, [&]() {
-            lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
+            lds_quantize_q8_0(a.x, H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
             __syncthreads();
         });
         if (lane == 0 && r < a.F) a.act[static_cast<size_t>(a.k) * a.F + r] = silu_ggml(gu[0]) * gu[1];
@@ -1058,10 +1061,10 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     auto set_up = [&]() {  // what does not need the ids
         if (kIq) {
             stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, 512);
-            for (int b = wave; b < (a.H >> 8); b += 8)
+            for (int b = wave; b < (H >> 8); b += 8)
                 wave_quantize_q8_k_block(a.x + b * 256, xq + b * 256, reinterpret_cast<float *>(xscale) + b, lane);
         } else {
-            lds_quantize_q8_0(a.x, a.H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
+            lds_quantize_q8_0(a.x, H, xq, reinterpret_cast<uint16_t *>(xscale), threadIdx.x, 512);
         }
         mark<TRACE>(a, 1, 1);
     };
@@ -1113,14 +1116,14 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         };
         float gu[2];
         if (kIq) {
-            const int nb = a.H >> 8;
+            const int nb = H >> 8;
             const size_t rb = static_cast<size_t>(nb) * (TYPE == 21 ? 110 : 82);
             const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
             const uint8_t *const rows[2] = {uniform_ptr(gate + off), uniform_ptr(up + off)};  // one row pair per wave
             // (PART) the chunk sums of the pair: gate row r of rung j, the up row F rows further on
             const size_t pg = static_cast<size_t>(nb) * 8;
             int32_t *pp = PART ? a.gup_part + (static_cast<size_t>(j) * 2 * a.F + min(r, a.F - 1)) * pg : nullptr;
-            uint8_t *const stage = lds_ab + layer_ab_stage(a.H) + wave * layer_ab_stage_bytes<TYPE, FETCH>(a.H);
+            uint8_t *const stage = lds_ab + layer_ab_stage(H) + wave * layer_ab_stage_bytes<TYPE, FETCH>(H);
             const float *xd = reinterpret_cast<const float *>(xscale);
             if (FETCH == 10)
                 iq_rows10_coal<kIqType, 2, PART>(rows, tables, xq, xd, lane, gu, stage, pp, a.F * pg, pre);
@@ -1132,7 +1135,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
                 iq_rows_q8k<kIqType, 2, PART>(rows, nb, tables, xq, xd, lane, gu, pp, a.F * pg, pre);
         } else {
             Q8RowTile *tiles = reinterpret_cast<Q8RowTile *>(s_union);
-            const int nb = a.H >> 5;
+            const int nb = H >> 5;
             const size_t rb = static_cast<size_t>(nb) * (TYPE == 8 ? 34 : 18);
             const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
             const uint8_t *const rows[2] = {uniform_ptr(gate + off), uniform_ptr(up + off)};
