@@ -973,7 +973,7 @@ def bench_tokens(args, torch, capi, synth):
                    "union_bytes_per_layer": int(union_bytes), "serial_bytes_per_layer": int(serial_bytes)},
         "roofline": dict(bound="hbm", achieved=round(union_bytes / us_batch / 1e3, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                          frac=round(union_bytes / us_batch / 1e3 / HBM_PEAK_GBS, 4), traffic=None,
-                         kernel="whole pass (k_tokens_a, k_tokens_b, k_tokens_c)")}))
+                         kernel="whole pass (k_tokens_ab, k_tokens_c)")}))
 
 
 def main():

@@ -181,3 +181,32 @@ def test_tokens_on_a_table_of_expert_views(g, oracle, shape):
     assert lib.wd_moe_layer_tokens_pairs_f32(C.byref(d), hg, hu, hd, 129, g.ptr(dx), g.ptr(out), T, arr, capi.MOE_PRESELECTED, g.stream()) == -1
     for s in scs:
         s.close()
+
+
+@pytest.mark.parametrize("gate,F", [(synth.IQ3_S, 64), (synth.Q8_0, 64), (synth.IQ2_S, 1568)])
+def test_bounded_wait_of_a_token_batch(g, oracle, gate, F):
+    """With a wait limit of one poll the routed workgroups give up before the ids are published: every token's status word and
+    data say so; with the default limit the same scratches give the oracle's results, in one launch and in two."""
+    H, E, k, T = 512, 64, 6, 3
+    L = synth.make_layer(H, F, E, k, gate, synth.Q8_0, True, seed=SEED, layer=33, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, T, 9)
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    arr = (C.c_void_p * T)(*[s.h for s in scr])
+    dx, out = g.dev(xs), g.empty((T, H), np.float32)
+    lib = capi.load()
+    capi.call("wd_moe_scratch_set_wait_limit", scr[0].h, 1)
+    capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, arr, 0, g.stream())
+    g.sync()
+    assert [lib.wd_moe_scratch_status(s.h) for s in scr] == [1] * T
+    assert np.isnan(g.host(out)).all()
+    for s in scr:
+        capi.call("wd_moe_scratch_set_wait_limit", s.h, 0)
+    for flags in (0, capi.MOE_SPLIT_AB, 0):
+        capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, arr, flags, g.stream())
+        g.sync()
+        for t in range(T):
+            want, d = oracle.moe_layer(L, xs[t])
+            assert np.array_equal(scr[t].get("ids", k, np.int32), d["ids"]) and g.same_bits(g.host(out)[t], want), (flags, t)
+    assert [lib.wd_moe_scratch_status(s.h) for s in scr] == [0] * T
+    for s in scr:
+        s.close()

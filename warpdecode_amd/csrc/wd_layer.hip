@@ -954,28 +954,31 @@ extern "C" int wd_moe_stack_f32(const wd_moe_layer *layers, int n_layers, float 
 }
 
 namespace {
+// Dispatch AB of a token batch: ta.front_wgs workgroups of the first part, and with `routed` those of the second.
 template <int TYPE, int FETCH>
-void launch_tokens_b_fetch(const TokenArgs &ta, int items, int cus, hipStream_t st) {
+void launch_tokens_ab_fetch(const TokenArgs &ta, bool routed, int items, int cus, hipStream_t st) {
     const int H = ta.common.H;
     size_t lds = static_cast<size_t>(ta.T) * (H + sizeof(float) * (H / 256));
     if (FETCH != 0) lds = ((lds + 15) & ~static_cast<size_t>(15)) + 8 * 2 * static_cast<size_t>(iq_cover_bytes<TYPE>(H / 256));
+    lds = std::max(lds, sizeof(float) * static_cast<size_t>(H) + 16);
     // persistent: as many workgroups as a compute unit holds walk the items
-    if (ta.T <= 4) enqueue(k_tokens_b<TYPE, 4, FETCH>, std::min(items, kTokensBPerCu<TYPE, 4, FETCH> * cus), 512, lds, st, ta);
-    else enqueue(k_tokens_b<TYPE, kMaxTokens, FETCH>, std::min(items, kTokensBPerCu<TYPE, kMaxTokens, FETCH> * cus), 512, lds, st, ta);
+    auto grid = [&](int per_cu) { return dim3(ta.front_wgs + (routed ? std::min(items, per_cu * cus) : 0)); };
+    if (ta.T <= 4) enqueue(k_tokens_ab<TYPE, 4, FETCH>, grid(kTokensBPerCu<TYPE, 4, FETCH>), dim3(512), lds, st, ta);
+    else enqueue(k_tokens_ab<TYPE, kMaxTokens, FETCH>, grid(kTokensBPerCu<TYPE, kMaxTokens, FETCH>), dim3(512), lds, st, ta);
 }
 template <int TYPE>
-void launch_tokens_b(const wd_moe_layer *L, const TokenArgs &ta, int items, int cus, bool table, bool tables_aligned, hipStream_t st) {
+void launch_tokens_ab(const wd_moe_layer *L, const TokenArgs &ta, bool routed, int items, int cus, bool table, bool tables_aligned, hipStream_t st) {
     const int H = L->hidden;
     // rows of tensors that start on 16-byte boundaries: the aligned fetch, one item ahead
     auto al16 = [](const void *p, size_t v) { return reinterpret_cast<uintptr_t>(p) % 16 == 0 && v % 16 == 0; };
     const bool words = table ? tables_aligned
                              : (L->slot_of_expert ? al16(L->slot_pool, L->slot_bytes) && L->slot_gate_bytes % 16 == 0
                                                   : al16(L->gate, L->gate_stride) && al16(L->up, L->up_stride));
-    if (!words || H > 4096) launch_tokens_b_fetch<TYPE, 0>(ta, items, cus, st);
-    else if (H == 2048) launch_tokens_b_fetch<TYPE, 8>(ta, items, cus, st);
-    else if (H == 2560) launch_tokens_b_fetch<TYPE, 10>(ta, items, cus, st);
-    else if (H <= 2304) launch_tokens_b_fetch<TYPE, 1>(ta, items, cus, st);
-    else launch_tokens_b_fetch<TYPE, 2>(ta, items, cus, st);
+    if (!words || H > 4096) launch_tokens_ab_fetch<TYPE, 0>(ta, routed, items, cus, st);
+    else if (H == 2048) launch_tokens_ab_fetch<TYPE, 8>(ta, routed, items, cus, st);
+    else if (H == 2560) launch_tokens_ab_fetch<TYPE, 10>(ta, routed, items, cus, st);
+    else if (H <= 2304) launch_tokens_ab_fetch<TYPE, 1>(ta, routed, items, cus, st);
+    else launch_tokens_ab_fetch<TYPE, 2>(ta, routed, items, cus, st);
 }
 template <int KIND, int LPR, int PASSES = 1>
 void launch_tokens_c_even(const TokenArgs &ta, hipStream_t st) {
@@ -1064,30 +1067,39 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         k_.shared_gate = s->shared_gate, k_.arrive = s->arrive;
         k_.expert_out = (flags & WD_MOE_KEEP_EXPERT_OUT) ? s->expert_out : nullptr;
         k_.accum = s->accum, k_.down_f32 = s->down_f32;
+        k_.tagged = s->tagged, k_.status = s->status;
     }
     LayerArgs &a = ta.common;
     const bool wide = H > 2048 && H <= 4096;  // two waves per router row
     const int router_rows_n = (a.preselected ? 0 : a.E) + (a.sh_inp ? 1 : 0);
     a.n_router_wgs = wide ? (router_rows_n + 3) / 4 : (router_rows_n + 7) / 8;
     const int grid_a = tokens_a_grid(a.n_router_wgs, a.sh_inp ? (F + 7) / 8 : 0).total(tokens);
-    if (grid_a > 0) {  // router, selection and shared gate/up of every token
-        SiteScope site(WD_SITE_TOKENS_A, st);
-        if (wide) enqueue(k_tokens_a<true>, dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st, ta);
-        else enqueue(k_tokens_a<false>, dim3(grid_a), dim3(512), static_cast<size_t>(H) * 4 + 16, st, ta);
-        WD_LAUNCH_CHECK();
-    }
     const int items_b = tokens * k * ((F + 7) / 8);
     const int cus = scratch_per_token[0]->compute_units;
-    {
-        SiteScope site(WD_SITE_TOKENS_B, st);
-        const size_t lds_q8 = static_cast<size_t>(tokens) * (H + H / 16);
+    // The parts that `front` and `routed` name
+    auto launch_ab = [&](bool front, bool routed) {
+        ta.front_wgs = front ? grid_a : 0, ta.wait_ids = front && routed ? 1 : 0;
+        const size_t lds_q8 = std::max(static_cast<size_t>(tokens) * (H + H / 16), sizeof(float) * static_cast<size_t>(H) + 16);
+        const dim3 grid_q8(ta.front_wgs + (routed ? std::min(items_b, 2 * cus) : 0));
         switch (L->gate_type) {
-            case WD_TYPE_IQ3_S: launch_tokens_b<21>(L, ta, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
-            case WD_TYPE_IQ2_S: launch_tokens_b<22>(L, ta, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
-            case WD_TYPE_Q8_0: enqueue(k_tokens_b_q8<0>, std::min(items_b, 2 * cus), 512, lds_q8, st, ta); break;
-            default: enqueue(k_tokens_b_q8<1>, std::min(items_b, 2 * cus), 512, lds_q8, st, ta); break;
+            case WD_TYPE_IQ3_S: launch_tokens_ab<21>(L, ta, routed, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
+            case WD_TYPE_IQ2_S: launch_tokens_ab<22>(L, ta, routed, items_b, cus, gu_table != nullptr, tables_aligned, st); break;
+            case WD_TYPE_Q8_0: enqueue(k_tokens_ab_q8<0>, grid_q8, dim3(512), lds_q8, st, ta); break;
+            default: enqueue(k_tokens_ab_q8<1>, grid_q8, dim3(512), lds_q8, st, ta); break;
         }
         WD_LAUNCH_CHECK();
+        return static_cast<int>(WD_OK);
+    };
+    // One launch where the ids come out of it; ids that are there already need no wait, and the site profiler brackets the parts
+    if (!a.preselected && !(flags & WD_MOE_SPLIT_AB) && !SiteProfiler::instance().enabled()) {
+        if (const int rc = launch_ab(true, true)) return rc;
+    } else {
+        if (grid_a > 0) {  // router, selection and shared gate/up of every token
+            SiteScope site(WD_SITE_TOKENS_A, st);
+            if (const int rc = launch_ab(true, false)) return rc;
+        }
+        SiteScope site(WD_SITE_TOKENS_B, st);
+        if (const int rc = launch_ab(false, true)) return rc;
     }
     SiteScope c_site(WD_SITE_TOKENS_C, st);
     if (!down_tokens) {

@@ -1,13 +1,14 @@
 // M tokens through one MoE layer with every selected expert's weights read once.
 //
 // The reference batches M tokens as M*k (token, expert) pairs and re-reads an expert's weights for
-// every pair that names it (src/qwen38_moe.cuh:1316-1437, :2743-3237).  Here a pass is three dispatches:
-//   A  router, selection and shared gate/up of every token side by side (grid.y = token);
-//   B  routed gate/up + SwiGLU over the union of the selected experts: a weight row is fetched and decoded once and applied to
-//      the activation of every token that selected the expert;
+// every pair that names it (src/qwen38_moe.cuh:1316-1437, :2743-3237).  Here a pass is two dispatches:
+//   AB router, selection and shared gate/up of every token side by side, and the routed gate/up + SwiGLU over the union of the
+//      selected experts: a weight row is fetched and decoded once and applied to the activation of every token that selected the
+//      expert.  The routed workgroups set themselves up while the router runs and wait for the ids inside the dispatch, as in the
+//      one-token dispatch AB; with ids that are known before, and for the site profiler, the two parts (A and B) are launched apart.
 //   C  down projections over the union (a member's rows are loaded once and applied to the activations of its
 //      tokens) and the ordered combine per token.
-// B and C each work the union out for themselves from the T*k ids (one wave per workgroup, in LDS); nothing about
+// AB and C each work the union out for themselves from the T*k ids (one wave per workgroup, in LDS); nothing about
 // it goes through global memory.  Per token, the arithmetic and its order are those of the one-token kernels, so the
 // results are bit-identical to M separate passes.
 #pragma once
@@ -50,23 +51,27 @@ struct TokenSlots {
     unsigned *arrive;
     float *expert_out;   // null or [k][H]
     float *accum, *down_f32, *out;
+    uint32_t *tagged;    // [kTagCopies][16] selected ids published inside dispatch AB (kTagInvalid = not yet)
+    unsigned *status;    // [0] set to 1 when the wait for the ids ran out
 };
 
 struct TokenArgs {
     LayerArgs common;  // the layer; the per-token members are taken from tok[]
     int T;
+    int front_wgs;     // workgroups of dispatch AB that take its first part
+    int wait_ids;      // the ids come out of the same dispatch (otherwise they are in the scratches)
     TokenSlots tok[kMaxTokens];
 };
 
-// ---- dispatch A for T tokens ----------------------------------------------------------------------------
-// grid = T * (router_stride + shared_stride), 512 threads, the strides being the router and the shared workgroups of a
+// ---- dispatch AB for T tokens, first part (A) --------------------------------------------------------------
+// T * (router_stride + shared_stride) workgroups, 512 threads, the strides being the router and the shared workgroups of a
 // token rounded up to a multiple of 8 (tokens_a_grid): first the router workgroups of every token, token by token, then
 // the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
 // token - the same weight rows - lands on the same XCD (workgroups go to the eight XCDs in turn), so its L2 serves the
 // rows to the tokens after the first.  The padding workgroups return at once.  Per token this is the front of the
 // one-token merged dispatch: router rows one per wave, the last router workgroup of the token selects its experts
-// with the whole workgroup, the other workgroups run the shared expert's gate/up.
-// dynamic LDS: 4 * H bytes (x as f32 for the router rows; the shared workgroups use H + H/16 of it).
+// with the whole workgroup and publishes the ids, the other workgroups run the shared expert's gate/up.
+// lds: 4 * H + 16 bytes (x as f32 for the router rows; the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes.
 struct TokensAGrid {
     int router_stride, shared_stride;
     __host__ __device__ int total(int tokens) const { return tokens * (router_stride + shared_stride); }
@@ -74,13 +79,13 @@ struct TokensAGrid {
 __host__ __device__ inline TokensAGrid tokens_a_grid(int n_router_wgs, int n_shared_wgs) {
     return TokensAGrid{(n_router_wgs + 7) & ~7, (n_shared_wgs + 7) & ~7};
 }
+constexpr int kTokensWorkBytes = sizeof(Q8RowTile) * 8;
 // WIDE: router rows of 2049..4096 columns, two waves each (n_router_wgs is then for four rows per workgroup).
-template <bool WIDE>
-__global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
-    extern __shared__ __align__(16) uint8_t lds_ta[];
-    __shared__ __align__(16) uint8_t s_work[sizeof(Q8RowTile) * 8];
-    __shared__ int s_last;
+// HIDDEN: the layer's, where it is known (0: it is not): its row loops then need no bounds, which spill 18 registers.
+template <bool WIDE, int HIDDEN>
+WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, int &s_last) {
     const LayerArgs &a = ta.common;
+    const int H = HIDDEN ? HIDDEN : a.H;
     const int n_shared_wgs = a.sh_inp ? (a.F + 7) / 8 : 0;
     const TokensAGrid gr = tokens_a_grid(a.n_router_wgs, n_shared_wgs);
     int token, wg;
@@ -101,10 +106,10 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
     if (wg < a.n_router_wgs) {
         const int rows = a.preselected ? 0 : a.E;
         if (WIDE)
-            router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.logits, rows, a.H,
+            router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.logits, rows, H,
                                   a.sh_inp, s.shared_gate, wg);
         else
-            router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, rows, a.H, a.sh_inp, s.shared_gate, wg);
+            router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, rows, H, a.sh_inp, s.shared_gate, wg);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
         __syncthreads();
@@ -115,10 +120,10 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
         if (!s_last) return;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         if (!a.preselected) {
-            static_assert(sizeof(s_work) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
+            static_assert(kTokensWorkBytes >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
             int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
             float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
-            topk_block(s.logits, a.E, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave);
+            topk_block(s.logits, a.E, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr, ta.wait_ids ? s.tagged : nullptr, kTagCopies);
             if (wave == 0) {
                 wave_lds_fence();
                 if (lane < a.k) {
@@ -137,16 +142,16 @@ __global__ __launch_bounds__(512, 4) void k_tokens_a(TokenArgs ta) {
         return;
     }
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ta);
-    uint16_t *xd = reinterpret_cast<uint16_t *>(lds_ta + a.H);
+    uint16_t *xd = reinterpret_cast<uint16_t *>(lds_ta + H);
     Q8RowTile *tiles = reinterpret_cast<Q8RowTile *>(s_work);
     const int r = (wg - a.n_router_wgs) * 8 + wave;
-    const int nb = a.H >> 5;
+    const int nb = H >> 5;
     const size_t rb = static_cast<size_t>(nb) * 34;
     const size_t off = static_cast<size_t>(min(r, a.F - 1)) * rb;
     const uint8_t *const rows[2] = {uniform_ptr(a.sh_gate + off), uniform_ptr(a.sh_up + off)};  // one row pair per wave
     float gu[2];
     q8_row_pair<0, WIDE>(rows, nb, xq, xd, tiles[wave], lane, gu, [&]() {
-        lds_quantize_q8_0(s.x, a.H, xq, xd, threadIdx.x, 512);
+        lds_quantize_q8_0(s.x, H, xq, xd, threadIdx.x, 512);
         __syncthreads();
     });
     if (lane == 0 && r < a.F) s.act[static_cast<size_t>(a.k) * a.F + r] = silu_ggml(gu[0]) * gu[1];
@@ -190,9 +195,47 @@ struct TokenUnion {
     int first_pair[1024];            // scratch of the build: lowest pair naming an expert
 };
 
+// The ids of pairs `lane` and `lane + 64` as the first part of the same dispatch publishes them; false: the wait ran out.
+WD_DEV bool token_pairs_wait(const TokenArgs &ta, int lane, int &id_lo, int &id_hi) {
+    const int k = ta.common.k, n = ta.T * k;
+    auto word_of = [&](int pair) {
+        const int pc = min(pair, n - 1);
+        int t = 0;
+        const uint32_t *p = ta.tok[0].tagged;
+#pragma unroll
+        for (int q = 1; q < kMaxTokens; ++q) {
+            const bool past = pc >= q * k;
+            t += past ? 1 : 0;
+            p = past ? ta.tok[q].tagged : p;
+        }
+        return p + (blockIdx.x & (kTagCopies - 1)) * 16 + (pc - t * k);
+    };
+    const uint32_t *const lo = word_of(lane), *const hi = word_of(lane + 64);
+    for (unsigned polls = 1;; ++polls) {
+        const uint32_t v = __hip_atomic_load(lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), w = __hip_atomic_load(hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_ballot_w64(v == kTagInvalid || w == kTagInvalid) == 0ull) {
+            id_lo = lane < n ? static_cast<int>(v) : -1 - lane, id_hi = lane + 64 < n ? static_cast<int>(w) : -65 - lane;
+            return true;
+        }
+        if (polls >= ta.common.spin_limit) return false;
+        __builtin_amdgcn_s_sleep(4);
+    }
+}
+// Returns with un.count < 0 when the ids did not come (the status word is set).
 WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
     const int k = ta.common.k, n = ta.T * k;
-    const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
+    int id_lo, id_hi;
+    if (!ta.wait_ids) {
+        id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
+    } else if (!token_pairs_wait(ta, lane, id_lo, id_hi)) {
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < kMaxTokens; ++q)
+                if (q < ta.T) __hip_atomic_store(ta.tok[q].status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            un.count = -1;
+        }
+        return;
+    }
     const bool on_lo = lane < n, on_hi = lane + 64 < n;
     for (int i = lane; i < 128 * kMaxTokens / 4; i += 64) reinterpret_cast<uint32_t *>(&un.rank[0][0])[i] = 0xffffffffu;
     // lowest pair that names the same expert, through a table indexed by expert id
@@ -230,26 +273,40 @@ WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
     wave_lds_fence();
 }
 
-// ---- dispatch B for T tokens ----------------------------------------------------------------------------
-// Persistent form: grid = min(T * k * ceil(F / 8), a few workgroups per compute unit), 512 threads.  Every
-// workgroup builds the union (wave 0), stages the codebooks and quantises the T inputs once, then walks the items
-// (union member, group of 8 rows) blockIdx.x, blockIdx.x + gridDim.x, ...; a wave takes one (gate, up) row pair of
-// the item, decodes it once and applies it to every token that selected the expert.
+// ---- dispatch AB for T tokens ---------------------------------------------------------------------------
+// grid = front_wgs (the first part, tokens_front) + min(T * k * ceil(F / 8), a few workgroups per compute unit), 512 threads.
+// Every workgroup of the second part (B) stages the codebooks and quantises the T inputs once, builds the union (wave 0) - when the
+// ids come out of this dispatch, behind the set-up, with a bounded wait -, then walks the items (union member, group of 8 rows) in
+// turn with the stride of their number; a wave takes one (gate, up) row pair of the item, decodes it once and applies it to every
+// token that selected the expert.  As a dispatch of its own this part began 2.6 us after the ids and spent 3.5 more on its set-up.
 // MAXT: token capacity of the instantiation (4 or kMaxTokens).
-// dynamic LDS: T * (H bytes + H/256 floats): the Q8_K copies of the T inputs.
+// dynamic LDS: T * (H bytes + H/256 floats), the Q8_K copies of the T inputs, and 4 * H + 16 bytes at least (tokens_front).
 // FETCH: 0, or how the rows come in when they can be fetched as aligned words (IqRowWords): 8 and 10 rows of that many
 // super-blocks, 1 and 2 others of one or two words per lane.  The row pair of the wave's next item is then requested before the
 // current one is worked on.  dynamic LDS then has 8 * 2 * iq_cover_bytes more bytes behind the activations (16-byte aligned).
-// As many workgroups per compute unit as the registers allow without spilling (eight tokens and rows of eight super-blocks spill
-// two, which costs nothing: 68.3 us per layer, 68.7 without).
+// As many workgroups per compute unit as the registers allow without spilling in the routed part (eight tokens and rows of eight
+// super-blocks spill eleven in all: 73.1 us per layer, 75.7 as two dispatches of which one spilled two).
 template <int TYPE, int MAXT, int FETCH>
 constexpr int kTokensBPerCu = FETCH == 8 || (FETCH == 10 && TYPE == 22 && MAXT <= 4) ? 3 : 2;
 template <int TYPE, int MAXT, int FETCH = 0>
-__global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k_tokens_b(TokenArgs ta) {
+__global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k_tokens_ab(TokenArgs ta) {
     extern __shared__ __align__(16) uint8_t lds_tb[];
-    __shared__ IqTables tables;
-    __shared__ TokenUnion un;
+    struct Routed {
+        IqTables tables;
+        TokenUnion un;
+    };
+    __shared__ __align__(16) uint8_t s_area[sizeof(Routed) > kTokensWorkBytes ? sizeof(Routed) : kTokensWorkBytes];
+    __shared__ int s_last;
     const LayerArgs &a = ta.common;
+    if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
+        const bool wide = a.H > 2048 && a.H <= 4096;
+        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, FETCH == 10 ? 2560 : 0>(ta, lds_tb, s_area, s_last);
+        else tokens_front<false, FETCH == 8 ? 2048 : 0>(ta, lds_tb, s_area, s_last);
+        return;
+    }
+    IqTables &tables = reinterpret_cast<Routed *>(s_area)->tables;
+    TokenUnion &un = reinterpret_cast<Routed *>(s_area)->un;
+    const int wg = static_cast<int>(blockIdx.x) - ta.front_wgs, n_wgs = static_cast<int>(gridDim.x) - ta.front_wgs;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int groups = (a.F + 7) / 8;
     int8_t *xq = reinterpret_cast<int8_t *>(lds_tb);
@@ -281,8 +338,8 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
         }
     };
     load_blocks(wave);
-    if (wave == 0) token_union_build(ta, un, lane);
-    if (a.preselected && blockIdx.x == 0 && wave == 1) token_ids_report(ta, lane);  // (ahead of the loads: 0.4 us)
+    if (!ta.wait_ids && wave == 0) token_union_build(ta, un, lane);
+    if (a.preselected && wg == 0 && wave == 1) token_ids_report(ta, lane);  // (ahead of the loads: 0.4 us)
     mark(a, 1, 1);
     stage_tables<TYPE == 21, TYPE == 22>(tables, threadIdx.x, 512);
     quantise_blocks(wave);
@@ -290,7 +347,9 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
         load_blocks(b0);
         quantise_blocks(b0);
     }
+    if (ta.wait_ids && wave == 0) token_union_build(ta, un, lane);
     __syncthreads();
+    if (un.count < 0) return;  // the wait ran out
     mark(a, 1, 2);
     const int n_items = un.count * groups;
     // the aligned forms use the lane layout of iq_rows8_coal_dots (a chain's lanes two apart inside a row, no lane excluded from
@@ -309,12 +368,12 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
         const size_t off = static_cast<size_t>(min(rg * 8 + wave, a.F - 1)) * rb;
         rows[0] = uniform_ptr(mat_ptr_entry<0>(a.gate_up, e) + off), rows[1] = uniform_ptr(mat_ptr_entry<1>(a.gate_up, e) + off);
     };
-    if (FETCH != 0 && static_cast<int>(blockIdx.x) < n_items) {
+    if (FETCH != 0 && wg < n_items) {
         const uint8_t *rows[2];
-        row_pair(blockIdx.x, rows);
+        row_pair(wg, rows);
         fetch[0].request(rows[0], nb, lane), fetch[1].request(rows[1], nb, lane);
     }
-    for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+    for (int item = wg; item < n_items; item += n_wgs) {
         const int u = item / groups, rg = item - u * groups;
         int rank[MAXT];
 #pragma unroll
@@ -328,9 +387,9 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
             fetch[0].store(stage, lane), fetch[1].store(stage + kStage, lane);
             lead[0] = fetch[0].lead, lead[1] = fetch[1].lead;
             wave_lds_fence();
-            if (item + static_cast<int>(gridDim.x) < n_items) {  // the next item's rows, into the registers just written out
+            if (item + n_wgs < n_items) {  // the next item's rows, into the registers just written out
                 const uint8_t *next[2];
-                row_pair(item + gridDim.x, next);
+                row_pair(item + n_wgs, next);
                 fetch[0].request(next[0], nb, lane), fetch[1].request(next[1], nb, lane);
             }
         }
@@ -450,7 +509,7 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
             }
             if (lane == 0 && r < a.F) ta.tok[t].act[static_cast<size_t>(rank[t]) * a.F + r] = silu_ggml(g) * up;
         }
-        mark(a, 1, item == static_cast<int>(blockIdx.x) ? 3 : 4);
+        mark(a, 1, item == wg ? 3 : 4);
     }
     mark(a, 1, 5);
 }
@@ -460,27 +519,41 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
 // registers at a time and applied to every token that selected the expert.
 // (One row pair per wave with a block per lane runs the chains of two rows on all 64 lanes, 64 steps each, for every token: 61 us
 // for eight tokens, top-5, hidden 3584, ffn 512, against 30.)
-// dynamic LDS: T * (H bytes + H/32 halves), the Q8_0 copies of the T inputs.
+// dynamic LDS: T * (H bytes + H/32 halves), the Q8_0 copies of the T inputs, and 4 * H + 16 bytes at least (tokens_front).
 template <int KIND>
-__global__ __launch_bounds__(512, 4) void k_tokens_b_q8(TokenArgs ta) {
+__global__ __launch_bounds__(512, 4) void k_tokens_ab_q8(TokenArgs ta) {
     extern __shared__ __align__(16) uint8_t lds_tq[];
-    __shared__ Q8Tile8 tiles[8];
-    __shared__ TokenUnion un;
+    struct Routed {
+        Q8Tile8 tiles[8];
+        TokenUnion un;
+    };
+    __shared__ __align__(16) uint8_t s_area[sizeof(Routed) > kTokensWorkBytes ? sizeof(Routed) : kTokensWorkBytes];
+    __shared__ int s_last;
     const LayerArgs &a = ta.common;
+    if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
+        if (a.H > 2048) tokens_front<true, 0>(ta, lds_tq, s_area, s_last);  // (hidden 4096 at most)
+        else tokens_front<false, 0>(ta, lds_tq, s_area, s_last);
+        return;
+    }
+    Q8Tile8 *const tiles = reinterpret_cast<Routed *>(s_area)->tiles;
+    TokenUnion &un = reinterpret_cast<Routed *>(s_area)->un;
+    const int wg = static_cast<int>(blockIdx.x) - ta.front_wgs, n_wgs = static_cast<int>(gridDim.x) - ta.front_wgs;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int groups = a.F >> 2, nb = a.H >> 5;  // (F is a multiple of 32, H of 256)
     constexpr int kBlk = (KIND == 0) ? 34 : 18, kChunk = 4;  // passes of eight blocks
     const size_t rb = static_cast<size_t>(nb) * kBlk;
     int8_t *xq = reinterpret_cast<int8_t *>(lds_tq);
     uint16_t *xd = reinterpret_cast<uint16_t *>(lds_tq + static_cast<size_t>(ta.T) * a.H);
-    if (wave == 0) token_union_build(ta, un, lane);
-    if (a.preselected && blockIdx.x == 0 && wave == 1) token_ids_report(ta, lane);
+    if (!ta.wait_ids && wave == 0) token_union_build(ta, un, lane);
+    if (a.preselected && wg == 0 && wave == 1) token_ids_report(ta, lane);
     for (int t = 0; t < ta.T; ++t) lds_quantize_q8_0(ta.tok[t].x, a.H, xq + static_cast<size_t>(t) * a.H, xd + t * nb, threadIdx.x, 512);
+    if (ta.wait_ids && wave == 0) token_union_build(ta, un, lane);
     __syncthreads();
+    if (un.count < 0) return;  // the wait ran out
     const int n_items = un.count * groups, row = lane >> 3, b = lane & 7;
     // (neighbouring workgroups take neighbouring items, a workgroup's waves items far apart: every wave of the grid gets one
     // before any gets a second)
-    for (int item = wave * static_cast<int>(gridDim.x) + static_cast<int>(blockIdx.x); item < n_items; item += 8 * static_cast<int>(gridDim.x)) {
+    for (int item = wave * n_wgs + wg; item < n_items; item += 8 * n_wgs) {
         const int u = item / groups, r0 = 4 * (item - u * groups);
         const int e = __builtin_amdgcn_readfirstlane(un.expert[u]);
         const uint8_t *const gate = mat_ptr_entry<0>(a.gate_up, e), *const up = mat_ptr_entry<1>(a.gate_up, e);
@@ -513,6 +586,13 @@ __global__ __launch_bounds__(512, 4) void k_tokens_b_q8(TokenArgs ta) {
 }
 
 // ---- dispatch C for T tokens ----------------------------------------------------------------------------
+// (workgroup 0) The ids published for the dispatch before are made invalid again.
+WD_DEV void tokens_clear_tagged(const TokenArgs &ta) {
+    if (blockIdx.x != 0) return;
+    for (int t = 0; t < ta.T; ++t)
+        for (int i = threadIdx.x; i < kTagCopies * 16; i += blockDim.x)
+            __hip_atomic_store(ta.tok[t].tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // grid = H / 8: a workgroup owns eight output rows, as the one-token k_layer_c8 does.  Work items are (token, matrix) with
 // matrix = the token's k routed down tensors, then the shared one (always Q8_0); the waves take them in turn: the
 // activation, then the eight rows, one block per lane and pass.  Items that name the same expert read the same rows within one
@@ -540,10 +620,12 @@ void k_tokens_c(TokenArgs ta) {
     const int per_token = a.k + (shared ? 1 : 0), n_items = ta.T * per_token;
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;  // hidden is a multiple of 8
     mark(a, 2, 0);
+    tokens_clear_tagged(ta);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
     const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
     // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
     float wreg;
+    const unsigned bad = __hip_atomic_load(ta.tok[min(tw, ta.T - 1)].status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // 1: a wait of dispatch AB ran out
     {
         const TokenSlots &s = ta.tok[min(tw, ta.T - 1)];
         const float *src = (lane == 16 && shared) ? s.shared_gate : s.weights + min(lane, a.k - 1);
@@ -607,8 +689,8 @@ void k_tokens_c(TokenArgs ta) {
                 o = acc + prod;
                 s.down_f32[row] = y;
             }
-            s.accum[row] = acc;
-            s.out[row] = o;
+            s.accum[row] = bad == 1u ? __builtin_nanf("") : acc;
+            s.out[row] = bad == 1u ? __builtin_nanf("") : o;
         }
     }
     mark(a, 2, 6);
@@ -634,10 +716,12 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
     const int rows_per_wg = a.H >> 8, r0 = blockIdx.x * rows_per_wg, nb = a.F >> 5;
     const int n_groups = rows_per_wg * LPR > 64 ? 2 : 1, rows0 = n_groups == 2 ? (rows_per_wg + 1) >> 1 : rows_per_wg;
     mark(a, 2, 0);
+    tokens_clear_tagged(ta);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
     const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
     // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
     float wreg;
+    const unsigned bad = __hip_atomic_load(ta.tok[min(tw, ta.T - 1)].status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // 1: a wait of dispatch AB ran out
     {
         const TokenSlots &s = ta.tok[min(tw, ta.T - 1)];
         const float *src = (lane == 16 && shared) ? s.shared_gate : s.weights + min(lane, a.k - 1);
@@ -721,8 +805,8 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
                 o = acc + prod;
                 s.down_f32[row] = y;
             }
-            s.accum[row] = acc;
-            s.out[row] = o;
+            s.accum[row] = bad == 1u ? __builtin_nanf("") : acc;
+            s.out[row] = bad == 1u ? __builtin_nanf("") : o;
         }
     }
     mark(a, 2, 6);
