@@ -759,6 +759,48 @@ WD_DEV float router_close32(float s) {
     return s + dpp_f<kDppShl2>(0.0f, s);
 }
 
+// Rows come in spans of 2048 columns, the lower half of the wave's lanes taking the first 1024 and the upper half the rest; a
+// half's part of a span is up to four groups of 256 columns, eight per lane (hidden is a multiple of 256).  The rows lie on the way to
+// the ids; with a test, an address and a select for every column in the groups' place, us per layer from HBM, so / with groups:
+// 1024 / 256 15.7 / 14.1, 1536 / 512 19.0 / 18.2, 2560 / 640 25.2 / 24.5, 3072 / 768 27.0 / 25.7; six variants of dispatch AB spilled.
+struct RouterSpan {
+    int lower, upper;  // groups of the halves
+    WD_DEV explicit RouterSpan(int cols) : lower(min(cols, 1024) >> 8), upper(max(min(cols, 2048) - 1024, 0) >> 8) {}
+};
+// The lane's weights of the span at column c0 (groups that the row does not have: those of the first group, not used).
+WD_DEV void router_span_load(const float *wr, int c0, const RouterSpan &sp, bool upper, int t, float (&wv)[32]) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        const float *p = wr + (c0 + t + (upper ? (g < sp.upper ? 1024 + 256 * g : 0) : (g < sp.lower ? 256 * g : 0)));
+#pragma unroll
+        for (int u = 0; u < 8; ++u) wv[8 * g + u] = p[32 * u];
+    }
+}
+// A half's multiply-adds of the span, continuing the chain from v; x: the half's first column of the lane.
+WD_DEV float router_span_run(const float (&wv)[32], const float *x, int groups, float v) {
+    float xv[2][8];
+    auto read = [&](int g) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) xv[g & 1][u] = x[256 * max(min(g, groups - 1), 0) + 32 * u];
+    };
+    if (groups == 0) return v;
+    read(0);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        if (g < 3) read(g + 1);
+        if (g < groups) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v = __builtin_fmaf(wv[8 * g + u], xv[g & 1][u], v);
+        }
+    }
+    return v;
+}
+// x to LDS, by the whole workgroup.
+WD_DEV void router_stage_x(const float *__restrict__ x, float *xs, int cols) {
+    for (int i = static_cast<int>(threadIdx.x) * 4; i < cols; i += static_cast<int>(blockDim.x) * 4)
+        *reinterpret_cast<float4 *>(xs + i) = *reinterpret_cast<const float4 *>(x + i);
+}
+
 // One row per wave, x staged once per workgroup in LDS (f32 [cols]).
 // Accumulator t (of ggml's 4 x 8) of the row lives in lanes t and t + 32: for every span of 2048 columns lane t
 // runs the multiply-adds of columns [span, span + 1024) and hands the value to lane t + 32, which continues with
@@ -776,72 +818,27 @@ WD_DEV void router_rows_wave(const float *__restrict__ w, const float *__restric
     const int total = rows + (extra_w ? 1 : 0);
     const bool on = row < total;
     const float *wr = on ? (row < rows ? w + static_cast<size_t>(row) * cols : extra_w) : x;
-    if (SCALAR_ROW) {  // the row is the same for the whole wave
-        const uintptr_t v = reinterpret_cast<uintptr_t>(wr);
-        const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-        const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-        wr = reinterpret_cast<const float *>((static_cast<uintptr_t>(hi) << 32) | lo);
-    }
-    const int np = cols & ~31;
-    const int half_off = (upper ? 1024 : 0) + t;
+    if (SCALAR_ROW) wr = uniform_ptr(wr);  // the row is the same for the whole wave
     float wv[32];
-    if (on) {
-#pragma unroll
-        for (int u = 0; u < 32; ++u) {
-            const int c = half_off + 32 * u;
-            wv[u] = (c < np) ? wr[c] : 0.0f;
-        }
-    }
-    for (int i = static_cast<int>(threadIdx.x) * 4; i < cols; i += static_cast<int>(blockDim.x) * 4) {
-        if (i + 4 <= cols) {
-            *reinterpret_cast<float4 *>(xs + i) = *reinterpret_cast<const float4 *>(x + i);
-        } else {
-            for (int c = i; c < cols; ++c) xs[c] = x[c];
-        }
-    }
+    if (on) router_span_load(wr, 0, RouterSpan(cols), upper, t, wv);
+    router_stage_x(x, xs, cols);
     __syncthreads();
     float s = 0.0f;  // the chain value; valid in the half that ran last
     if (on) {
-        for (int i0 = 0; i0 < np; i0 += 2048) {
-            if (i0 > 0) {
-#pragma unroll
-                for (int u = 0; u < 32; ++u) {
-                    const int c = i0 + half_off + 32 * u;
-                    wv[u] = (c < np) ? wr[c] : 0.0f;
-                }
-            }
-            // this lane's 32 multiply-adds of the span, continuing the chain from `start`
-            auto run_half = [&](float start) {
-                float v = start;
-#pragma unroll
-                for (int ub = 0; ub < 32; ub += 8) {
-                    float xv[8];
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) {
-                        const int c = i0 + half_off + 32 * (ub + q);
-                        xv[q] = xs[c < np ? c : 0];
-                    }
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) {
-                        const int c = i0 + half_off + 32 * (ub + q);
-                        const float nv = __builtin_fmaf(wv[ub + q], xv[q], v);
-                        v = (c < np) ? nv : v;
-                    }
-                }
-                return v;
-            };
+        for (int i0 = 0; i0 < cols; i0 += 2048) {
+            const RouterSpan sp(cols - i0);
+            if (i0 > 0) router_span_load(wr, i0, sp, upper, t, wv);
             // the lower half advances the chain (from the upper half's value of the previous span) ...
             const wd_uint2v back = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
-            if (!upper) s = run_half(i0 == 0 ? 0.0f : bits_f(back.y));
+            if (!upper) s = router_span_run(wv, xs + i0 + t, sp.lower, i0 == 0 ? 0.0f : bits_f(back.y));
             // ... and the upper half continues from its result
             const wd_uint2v fwd = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
-            if (upper) s = run_half(bits_f(fwd.x));
+            if (upper) s = router_span_run(wv, xs + i0 + 1024 + t, sp.upper, bits_f(fwd.x));
         }
     }
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
-    float acc = router_close32(s);
+    const float acc = router_close32(s);
     if (on && lane == 32) {
-        for (int c = np; c < cols; ++c) acc = acc + wr[c] * xs[c];
         float *dst = (row < rows) ? logits + row : extra_out;
         __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (another workgroup of the dispatch reads it)
     }
@@ -853,58 +850,27 @@ WD_DEV void router_rows_wave(const float *__restrict__ w, const float *__restric
 // first one leaves in LDS (`hand`: 4 x 32 floats).  Every thread of the (512-thread) workgroup must call it.
 WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *hand, float *logits,
                                   int rows, int cols, const float *__restrict__ extra_w, float *extra_out, int wg) {
-    const int lane = threadIdx.x & 63, t = lane & 31, wave = static_cast<int>(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, t = lane & 31, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const bool upper = lane >= 32, second = (wave & 1) != 0;
     const int row = wg * 4 + (wave >> 1);
     const int total = rows + (extra_w ? 1 : 0);
     const bool on = row < total;
     const float *wr = on ? (row < rows ? w + static_cast<size_t>(row) * cols : extra_w) : x;
-    const int np = cols & ~31;
-    const int c0 = (second ? 2048 : 0) + (upper ? 1024 : 0) + t;  // this lane's first column
+    const int c0 = second ? 2048 : 0;
+    const RouterSpan sp(cols - c0);
     float wv[32];
-    if (on) {
-#pragma unroll
-        for (int u = 0; u < 32; ++u) {
-            const int c = c0 + 32 * u;
-            wv[u] = (c < np) ? wr[c] : 0.0f;
-        }
-    }
-    for (int i = static_cast<int>(threadIdx.x) * 4; i < cols; i += static_cast<int>(blockDim.x) * 4) {
-        if (i + 4 <= cols) {
-            *reinterpret_cast<float4 *>(xs + i) = *reinterpret_cast<const float4 *>(x + i);
-        } else {
-            for (int c = i; c < cols; ++c) xs[c] = x[c];
-        }
-    }
+    if (on) router_span_load(wr, c0, sp, upper, t, wv);
+    router_stage_x(x, xs, cols);
     __syncthreads();
-    auto run_half = [&](float start) {
-        float v = start;
-#pragma unroll
-        for (int ub = 0; ub < 32; ub += 8) {
-            float xv[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int c = c0 + 32 * (ub + q);
-                xv[q] = xs[c < np ? c : 0];
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int c = c0 + 32 * (ub + q);
-                const float nv = __builtin_fmaf(wv[ub + q], xv[q], v);
-                v = (c < np) ? nv : v;
-            }
-        }
-        return v;
-    };
     // one copy of the chain code for both waves of a pair: turn 0 is the first wave's, turn 1 the second's
     float s = 0.0f;
 #pragma unroll 1
     for (int turn = 0; turn < 2; ++turn) {
         if (second == (turn == 1)) {
             const float start = s;
-            if (on && !upper) s = run_half(start);
+            if (on && !upper) s = router_span_run(wv, xs + c0 + t, sp.lower, start);
             const wd_uint2v fwd = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
-            if (upper) s = on ? run_half(bits_f(fwd.x)) : bits_f(fwd.x);
+            if (upper) s = on ? router_span_run(wv, xs + c0 + 1024 + t, sp.upper, bits_f(fwd.x)) : bits_f(fwd.x);
         }
         if (turn == 0) {
             if (!second && upper) hand[(wave >> 1) * 32 + t] = s;
@@ -914,9 +880,8 @@ WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__re
     }
     if (!second) return;
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
-    float acc = router_close32(s);
+    const float acc = router_close32(s);
     if (on && lane == 32) {
-        for (int c = np; c < cols; ++c) acc = acc + wr[c] * xs[c];
         float *dst = (row < rows) ? logits + row : extra_out;
         __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
