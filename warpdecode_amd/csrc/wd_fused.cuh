@@ -12,6 +12,7 @@
 #pragma once
 #include <type_traits>
 
+#include "wd_handword.hpp"
 #include "wd_kernels.cuh"
 
 namespace wd {
@@ -42,7 +43,7 @@ struct LayerArgs {
     int n_shared_wgs;            // those that take the shared expert's gate/up (the rest: routed gate/up)
     int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
     const int32_t *ids_known;    // null, or the k ids where they are known before the launch
-    unsigned *arrive;            // device counter of finished router workgroups (zero between dispatches)
+    uint32_t *hand;              // [E + 2]: the router's logits and the shared gate's on their way to the selection, then a ticket or count; kHandEmpty between passes
     uint32_t *ids_tagged;        // [kTagCopies][16] selected ids published inside the merged dispatch (kTagInvalid = not yet)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
     unsigned *status;            // [0] set to 1 when a bounded wait inside a dispatch ran out
@@ -663,60 +664,114 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
     finish_weights(top_mine, ids_given ? id_given : id_mine, k, w_scale, ids, weights, nullptr, lane);
 }
 
-// The selection of a row of n <= 64 M logits, k <= 15, inside a dispatch that wrote the logits: wave 0 ranks and publishes
-// the ids, wave 1 takes the exponentials and the denominator meanwhile, and wave 0 forms the weights behind one barrier.
-// Every thread of the workgroup must call it.  ids, weights: LDS.
-template <int M>
-WD_DEV void topk_two_waves(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
-                           const int32_t *__restrict__ override_ids, uint8_t *lds, int lane, int wave, unsigned long long *stamps,
-                           uint32_t *tagged, int copies) {
+// ---- selection inside the dispatch that computes the logits ------------------------------------------------------------
+// Every router workgroup hands its logits on as words that cannot be kHandEmpty (hand[e], the shared expert's gate logit in
+// hand[n_slot]); dispatch C sets the words back.  Which workgroup selects:
+//   one token (COUNT false): every workgroup waits until its words are acknowledged and looks at all of the row's.  Of those that end last
+//     at least one finds every word there.  If several do, all of them select, and the one that draws the ticket (hand[n_slot + 1])
+//     first publishes; the draw is under way while it selects.
+//   token batches (COUNT true): the workgroups count themselves in hand[n_slot + 1], without waiting for any acknowledgement, and the last
+//     one polls the words until all are there.  Surplus selections would hold up the routed workgroups that wait for a place.
+// (Counted behind the acknowledgement and the logits requested by the last one then, a round trip more, us per layer from HBM: 2048 / 512
+// 21.2, with tickets 20.0, counted 20.4; 2560 / 640 24.5, 23.7, 24.8; layer_small's 1024 / 256 12.1, 11.7, 12.0; eight tokens of 2048 / 512
+// 73.1, 75.9, 71.4; six of 1024 / 352 33.3, 31.4, 30.9.)
+struct HandRow {
+    uint32_t *hand;
+    int n, n_slot;
+    bool gate;  // hand[n_slot] is one of the row's
+};
+WD_DEV uint32_t hand_load(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+WD_DEV uint32_t hand_draw(uint32_t *hand, int n_slot) { return __hip_atomic_fetch_add(hand + n_slot + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// One thread: whether its workgroup is the last of n_wgs.
+WD_DEV bool hand_count_last(uint32_t *hand, int n_slot, int n_wgs) { return hand_draw(hand, n_slot) + 1u == static_cast<uint32_t>(n_wgs - 1); }
+// lv[j]: logit 64 j + lane; whether the row is complete.  POLL: once it is (it must be about to; the limit is there for a broken device).
+template <int M, bool POLL>
+WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
+    for (unsigned polls = 0; polls < (POLL ? kSpinLimit : 1u); ++polls) {
+        const uint32_t g = r.gate ? hand_load(r.hand + r.n_slot) : 0u;
+        bool there = hand_arrived(g);
+#pragma unroll
+        for (int j = 0; j < M; ++j) {
+            const uint32_t w = (64 * j + lane < r.n) ? hand_load(r.hand + 64 * j + lane) : f_bits(-INFINITY);
+            there = there && hand_arrived(w), lv[j] = bits_f(w);
+        }
+        if (__builtin_amdgcn_ballot_w64(there) == ~0ull) return true;
+    }
+    return false;
+}
+
+// The selections below return 0: some words are not there; 1: selected, but not the one to publish; 2: the one (wave 0; other waves: 1).
+// n <= 64 M logits, k <= 15: wave 0 ranks and publishes the ids, wave 1 takes the exponentials and the denominator meanwhile, and wave 0 forms
+// the weights behind one barrier.  Every thread of the workgroup must call it.  ids, weights, state: LDS.
+template <int M, bool COUNT>
+WD_DEV int topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
+                          uint8_t *lds, int &state, int lane, int wave, unsigned long long *stamps, uint32_t *tagged, int copies) {
 #define WD_STAMP(i) do { if (stamps && wave == 0 && lane == 0) stamps[i] = wall_clock64(); } while (0)
     const TopkLds<1> s(lds);
-    WD_STAMP(0);
+    const int n = row.n;
     SelWaveState st;
     int id_given = 0;
+    bool there = false, won = COUNT;
+    float lv[M];
     if (wave <= 1) {
         if (override_ids && wave == 0 && lane < k) id_given = override_ids[lane];
-        float lv[M];
-#pragma unroll
-        for (int j = 0; j < M; ++j)
-            lv[j] = (64 * j + lane < n) ? __hip_atomic_load(logits + 64 * j + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
-        if (wave == 0) {
-            sel_wave_ids(lv, n, k, s, lane, st);
-            WD_STAMP(3);
-            if (st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
-            WD_STAMP(6);
-        } else {
-            bool dead;
-            const float inv = sel_wave_denominator(lv, n, s, lane, dead);
-            if (lane == 0) s.rest[0] = inv, s.rest[1] = dead ? 1.0f : 0.0f;
-        }
+        there = hand_gather<M, COUNT>(row, lane, lv);
+        if (!COUNT && wave == 0 && lane == 0) state = there ? 1 : 0;
+    }
+    if (!COUNT) {
+        __syncthreads();
+        if (!state) return 0;
+    }
+    WD_STAMP(0);
+    if (wave == 0) {
+        uint32_t ticket = 0u;
+        if (!COUNT && lane == 0) ticket = hand_draw(row.hand, row.n_slot);
+        sel_wave_ids(lv, n, k, s, lane, st);
+        WD_STAMP(3);
+        if (!COUNT) won = __builtin_amdgcn_readfirstlane(ticket) == kHandEmpty;
+        if (won && st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        WD_STAMP(6);
+    } else if (wave == 1) {
+        if (!COUNT && !there) (void)hand_gather<M, true>(row, lane, lv);  // (wave 0 has seen them all)
+        bool dead;
+        const float inv = sel_wave_denominator(lv, n, s, lane, dead);
+        if (lane == 0) s.rest[0] = inv, s.rest[1] = dead ? 1.0f : 0.0f;
     }
     __syncthreads();
     if (wave == 0) {
         const bool fast = st.fast;
         sel_wave_weights(n, k, w_scale, s, lane, st, s.rest[0], s.rest[1] != 0.0f, ids, weights, override_ids != nullptr, id_given);
-        if (!fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        if (won && !fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
         WD_STAMP(7);
     }
 #undef WD_STAMP
+    return won ? 2 : 1;
 }
 
-// Selection inside a dispatch by the workgroup that read the last logit's arrival; every thread must call it.  Two waves do
-// it where one can hold the row (n <= 512, k <= 15); ids and weights are left in LDS by wave 0.
+// Every thread of the workgroup must call it (COUNT: of the one that counted last).  Two waves select where one can hold the row
+// (n <= 512, k <= 15); ids and weights are left in LDS by wave 0.
 // (64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
 // there are experts to select its threshold excludes nobody -; 512 experts, top-10: 2.1, 2.2.)
-WD_DEV void topk_block(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
-                       const int32_t *__restrict__ override_ids, uint8_t *lds, int lane, int wave,
-                       unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
+template <bool COUNT>
+WD_DEV int topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
+                      uint8_t *lds, int &state, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
+    const int n = row.n;
     if (n <= 512 && k <= 15) {
-        if (n <= 64) topk_two_waves<1>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-        else if (n <= 128) topk_two_waves<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-        else if (n <= 256) topk_two_waves<4>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-        else topk_two_waves<8>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-    } else {
-        topk_block_m<2>(logits, n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        if (n <= 64) return topk_two_waves<1, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
+        if (n <= 128) return topk_two_waves<2, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
+        if (n <= 256) return topk_two_waves<4, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
+        return topk_two_waves<8, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
     }
+    __syncthreads();  // (COUNT: state may be the word the count was read from)
+    if (wave == 0) {
+        float lv[16];
+        const bool there = hand_gather<16, COUNT>(row, lane, lv);
+        if (lane == 0) state = COUNT ? 2 : (!there ? 0 : (hand_draw(row.hand, row.n_slot) == kHandEmpty ? 2 : 1));
+    }
+    __syncthreads();
+    const int got = state;
+    if (got) topk_block_m<2>(reinterpret_cast<const float *>(row.hand), n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, got == 2 ? tagged : nullptr, copies);
+    return got;
 }
 
 // Stand-alone softmax/top-k dispatch: one wave (src/qwen38_moe.cuh:711-818).
@@ -809,9 +864,11 @@ WD_DEV void router_stage_x(const float *__restrict__ x, float *xs, int cols) {
 // which lets three workgroups of the merged dispatch share a compute unit).
 // Every thread of the workgroup must call it (it contains a barrier).
 // SCALAR_ROW: keep the wave's row pointer in scalar registers (two vector registers fewer).
+// The row's result goes to hand[row], the extra row's to hand[extra_slot]; it is returned as well (lane 32), with the row in `done`
+// (-1: this wave has none).
 template <bool SCALAR_ROW = false>
-WD_DEV void router_rows_wave(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *logits, int rows,
-                             int cols, const float *__restrict__ extra_w, float *extra_out, int wg) {
+WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restrict__ x, float *xs, uint32_t *hand, int rows,
+                              int cols, const float *__restrict__ extra_w, int extra_slot, int wg, int &done) {
     const int lane = threadIdx.x & 63, t = lane & 31;
     const bool upper = lane >= 32;
     const int row = wg * static_cast<int>(blockDim.x >> 6) + static_cast<int>(threadIdx.x >> 6);
@@ -838,18 +895,17 @@ WD_DEV void router_rows_wave(const float *__restrict__ w, const float *__restric
     }
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
     const float acc = router_close32(s);
-    if (on && lane == 32) {
-        float *dst = (row < rows) ? logits + row : extra_out;
-        __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // (another workgroup of the dispatch reads it)
-    }
+    done = on ? (row < rows ? row : extra_slot) : -1;
+    if (on && lane == 32) __hip_atomic_store(hand + done, hand_word_bits(f_bits(acc)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return acc;
 }
 
 // The same for rows of 2049..4096 columns, two waves per row: wave 2 w takes the first 2048 columns of row (4 wg + w),
 // wave 2 w + 1 the rest, both with every load of theirs in flight from the start - one trip to memory instead of one per
 // span.  The chains still see their columns in ascending order: the second wave starts from the 32 accumulators the
-// first one leaves in LDS (`hand`: 4 x 32 floats).  Every thread of the (512-thread) workgroup must call it.
-WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *hand, float *logits,
-                                  int rows, int cols, const float *__restrict__ extra_w, float *extra_out, int wg) {
+// first one leaves in LDS (`over`: 4 x 32 floats).  Every thread of the (512-thread) workgroup must call it.
+WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *over, uint32_t *hand,
+                                   int rows, int cols, const float *__restrict__ extra_w, int extra_slot, int wg, int &done) {
     const int lane = threadIdx.x & 63, t = lane & 31, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const bool upper = lane >= 32, second = (wave & 1) != 0;
     const int row = wg * 4 + (wave >> 1);
@@ -873,18 +929,18 @@ WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__re
             if (upper) s = on ? router_span_run(wv, xs + c0 + 1024 + t, sp.upper, bits_f(fwd.x)) : bits_f(fwd.x);
         }
         if (turn == 0) {
-            if (!second && upper) hand[(wave >> 1) * 32 + t] = s;
+            if (!second && upper) over[(wave >> 1) * 32 + t] = s;
             __syncthreads();
-            if (second) s = hand[(wave >> 1) * 32 + t];
+            if (second) s = over[(wave >> 1) * 32 + t];
         }
     }
-    if (!second) return;
+    done = -1;
+    if (!second) return 0.0f;
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
     const float acc = router_close32(s);
-    if (on && lane == 32) {
-        float *dst = (row < rows) ? logits + row : extra_out;
-        __hip_atomic_store(dst, acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    done = on ? (row < rows ? row : extra_slot) : -1;
+    if (on && lane == 32) __hip_atomic_store(hand + done, hand_word_bits(f_bits(acc)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return acc;
 }
 
 // ---- dispatch AB ------------------------------------------------------------------------------------------
@@ -896,10 +952,7 @@ WD_DEV void router_rows_wave_pair(const float *__restrict__ w, const float *__re
 // activation set-up from the critical path of the layer.  Where the ids are known before the launch (ids_known: a routing
 // trace, or a selection that is in the scratch) nothing is waited for and the weights are requested ahead of the set-up.
 //
-// Hand-off to the selecting workgroup: logits are published with device-scope atomic stores, each
-// workgroup then waits for its stores to complete and bumps a counter with a relaxed device-scope
-// atomic; the workgroup that reads n_router_wgs - 1 knows every logit is complete and reads them
-// with device-scope atomic loads.  No cache-wide release/acquire is needed for 2 KB of data.
+// Hand-off to the selecting workgroup: see topk_two_waves; no cache-wide release/acquire is needed for 2 KB of data.
 //
 // Publication: id j goes, as one 32-bit word, to ids_tagged[c][j] of every replica c with a device-scope atomic
 // store; a word other than kTagInvalid is the id itself, so a reader needs no second flag.  The words are reset
@@ -953,50 +1006,39 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     mark<TRACE>(a, wg < a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);
     if (wg < a.n_router_wgs) {
         const int rows = a.preselected ? 0 : a.E;
+        int row;
+        float logit;
         if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
-            router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.logits, rows,
-                                  H, a.sh_inp, a.shared_gate, wg);
+            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, rows, H,
+                                          a.sh_inp, a.E, wg, row);
         else
-            router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.logits, rows, H, a.sh_inp,
-                                   a.shared_gate, wg);
+            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, rows, H, a.sh_inp, a.E, wg, row);
         mark<TRACE>(a, 0, 1);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's word has been acknowledged
         __syncthreads();
-        if (threadIdx.x == 0)
-            s_last = (__hip_atomic_fetch_add(a.arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                      static_cast<unsigned>(a.n_router_wgs - 1));
-        __syncthreads();
-        if (s_last) {
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            if (TRACE && a.trace && threadIdx.x == 0) a.trace[(0 * 16 + 8) * 8 + 0] = wall_clock64();
-            if (wave == 5 && lane == 0) {
-                // off the selection's path: the shared expert's gate, and the counter for the next layer pass
-                if (a.sh_inp) {
-                    const float g = __hip_atomic_load(a.shared_gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    a.shared_gate[0] = sigmoid_ggml(g);
-                }
-                a.arrive[0] = 0u;
+        if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
+        if (TRACE && a.trace && threadIdx.x == 0) a.trace[(0 * 16 + 8) * 8 + 0] = wall_clock64();
+        int selected = 1;  // (no selection: the one workgroup with the shared gate's row)
+        // results land behind the selection's own scratch
+        static_assert(sizeof(s_union) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
+        int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
+        float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
+        if (!a.preselected)
+            // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
+            selected = topk_block<false>(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, s_last, lane, wave,
+                                         (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
+        // off the selection's path: the shared expert's gate (by every workgroup that found the row complete: the same value)
+        if (selected && a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(a.hand + a.E)));
+        if (selected == 2 && wave == 0) {
+            wave_lds_fence();
+            // the plain copies for dispatch C
+            if (lane < a.k) {
+                a.ids[lane] = lds_ids[lane];
+                a.weights[lane] = lds_w[lane];
+                if (a.host_ids) __hip_atomic_store(a.host_ids + lane, static_cast<uint32_t>(lds_ids[lane]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
-            if (!a.preselected) {
-                // results land behind the selection's own scratch
-                static_assert(sizeof(s_union) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
-                int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
-                float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
-                // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
-                topk_block(a.logits, a.E, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
-                           (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
-                if (wave == 0) {
-                    wave_lds_fence();
-                    // the plain copies for dispatch C
-                    if (lane < a.k) {
-                        a.ids[lane] = lds_ids[lane];
-                        a.weights[lane] = lds_w[lane];
-                        if (a.host_ids) __hip_atomic_store(a.host_ids + lane, static_cast<uint32_t>(lds_ids[lane]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    }
-                    if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
-                }
-            }
+            if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
         }
         mark<TRACE>(a, 0, 2);
         return;
@@ -1115,6 +1157,14 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     } while (LOOP && item < a.n_routed_items);
 }
 
+// (workgroup 0 of dispatch C) The words of this layer pass are done with: ids published, logits handed on, the ticket.
+WD_DEV void layer_clear_handed(const LayerArgs &a, int threads) {
+    if (!a.clear_tagged || blockIdx.x != 0) return;
+    for (int i = threadIdx.x; i < kTagCopies * 16; i += threads)
+        __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = threadIdx.x; i < a.E + 2; i += threads) __hip_atomic_store(a.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // ---- the combine at the end of dispatch C ---------------------------------------------------------------------
 // The operands of one wave's four rows, requested when the dispatch begins: lane m keeps router weight m, lane 16 the shared
 // gate; the residual values that the rows' owner updates at its end (nothing else writes them meanwhile): lane 4c + r
@@ -1206,9 +1256,7 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
     if (a.dry) return;
     // every routed workgroup of this layer pass finished with the previous dispatch: make the ids published
     // for them invalid again (this dispatch reads the plain copy)
-    if (a.clear_tagged && blockIdx.x == 0)
-        for (int i = threadIdx.x; i < kTagCopies * 16; i += blockDim.x)
-            __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    layer_clear_handed(a, blockDim.x);
     mark<TRACE>(a, 2, 0);
     FoldOps ops;
     if (wave == 0) ops = layer_c_fold_request(a, r0, nrows, lane);
@@ -1270,9 +1318,7 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
     float *ybuf = reinterpret_cast<float *>(lds_c8 + n_waves * per_wave);
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;
     if (a.dry) return;
-    if (a.clear_tagged && blockIdx.x == 0)  // (as in k_layer_c)
-        for (int i = threadIdx.x; i < kTagCopies * 16; i += 64 * (TWO ? 9 : n_act))
-            __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    layer_clear_handed(a, 64 * (TWO ? 9 : n_act));
     mark<TRACE>(a, 2, 0);
     FoldOps ops;
     int m = TWO ? wave : min(wave, n_act - 1);  // (a second wave without a matrix of its own repeats the first's)
@@ -1362,9 +1408,7 @@ __global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
     const int R = a.H >> 8, r0 = blockIdx.x * R, nb = a.F >> 5;
     const int rows0 = GROUPS == 1 ? R : (R + 1) >> 1;
     if (a.dry) return;
-    if (a.clear_tagged && blockIdx.x == 0)  // (as in k_layer_c)
-        for (int i = threadIdx.x; i < kTagCopies * 16; i += 64 * n_waves)
-            __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    layer_clear_handed(a, 64 * n_waves);
     FoldOps ops;
     const int m = min(wave, n_act - 1);  // (a wave without a matrix of its own repeats the last one's)
     const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;

@@ -35,7 +35,7 @@ struct wd_moe_scratch {
     int32_t *gup = nullptr;
     int32_t *dp = nullptr;
     int gup_type = -1, dp_type = -1;
-    unsigned *arrive = nullptr;           // device counter used inside the fused dispatch A
+    uint32_t *hand = nullptr;             // [n_experts + 2] logits on their way to the selection inside dispatch AB (LayerArgs)
     unsigned long long *trace = nullptr;  // device [3][16][8] time stamps, see wd_moe_scratch_trace
     int trace_wg = 0;
     int32_t *h_ids = nullptr;             // pinned [48]: [0..15] routed ids for callers that must see them on the host,
@@ -103,7 +103,7 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
                  o_act = c.take(sizeof(float) * K1 * F), o_aq = c.take(K1 * F),
                  o_ad = c.take(sizeof(uint16_t) * K1 * (F / 32)), o_eo = c.take(sizeof(float) * K1 * H),
                  o_acc = c.take(sizeof(float) * H), o_dn = c.take(sizeof(float) * H), o_sg = c.take(256),
-                 o_arr = c.take(256),
+                 o_hand = c.take(sizeof(uint32_t) * (n_experts + 2)),
                  o_tag = c.take(sizeof(uint32_t) * kTagRecords * kTagCopies * 16), o_status = c.take(256);
     const hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->block), c.off);
     if (e != hipSuccess) {
@@ -130,11 +130,12 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
     s->accum = reinterpret_cast<float *>(b + o_acc);
     s->down_f32 = reinterpret_cast<float *>(b + o_dn);
     s->shared_gate = reinterpret_cast<float *>(b + o_sg);
-    s->arrive = reinterpret_cast<unsigned *>(b + o_arr);
+    s->hand = reinterpret_cast<uint32_t *>(b + o_hand);
     s->tagged = reinterpret_cast<uint32_t *>(b + o_tag);
     s->status = reinterpret_cast<unsigned *>(b + o_status);
     (void)hipMemset(s->block, 0, c.off);
     (void)hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16);
+    (void)hipMemset(s->hand, 0xff, sizeof(uint32_t) * (n_experts + 2));
     if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 48, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->block);
         delete s;
@@ -177,6 +178,7 @@ int wd_moe_scratch_set_wait_limit(wd_moe_scratch *s, unsigned polls) {
     WD_HIP(hipMemset(s->status, 0, sizeof(unsigned)));
     reinterpret_cast<volatile int32_t *>(s->h_ids)[16] = 0;
     WD_HIP(hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16));
+    WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 2)));
     if (s->res_block) WD_HIP(hipMemset(s->res_block, 0xff, kHandEpoch));
     return WD_OK;
 }
@@ -476,7 +478,7 @@ LayerArgs fused_args(const wd_moe_layer *L, const float *d_x, float *d_out, wd_m
     a.dry = (flags & WD_MOE_DRY) ? 1 : 0;
     a.ids_known = ids_override;  // a routing trace: the ids do not depend on the router
     a.trace = s->trace, a.trace_wg = s->trace_wg;
-    a.arrive = s->arrive;
+    a.hand = s->hand;
     a.ids_tagged = s->tagged + static_cast<size_t>(rec % kTagRecords) * kTagCopies * 16;
     a.clear_tagged = 1;
     a.status = s->status;
@@ -676,7 +678,14 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
             if (const int rc = launch_ab(a, L, s, false, true, st)) return rc;
         }
     }
-    if (only && !(only & WD_MOE_ONLY_C)) return WD_OK;
+    if (only && !(only & WD_MOE_ONLY_C)) {
+        // dispatch C, which sets the handed words back, is not part of this call (with a report it follows in the same one)
+        if (run_a && !report && !a.dry) {
+            enqueue(k_fill_u32, dim3((L->n_experts + 2 + 255) / 256), dim3(256), 0, st, s->hand, kHandEmpty, static_cast<size_t>(L->n_experts) + 2);
+            WD_LAUNCH_CHECK();
+        }
+        return WD_OK;
+    }
     SiteScope site(WD_SITE_FUSED_C, st);
     const int n_act = k + (shared ? 1 : 0);
     const bool q8 = L->down_type == WD_TYPE_Q8_0;
@@ -1064,7 +1073,7 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         TokenSlots &k_ = ta.tok[t];
         k_.x = d_x + static_cast<size_t>(t) * H, k_.out = d_out + static_cast<size_t>(t) * H;
         k_.logits = s->logits, k_.ids = s->ids, k_.weights = s->weights, k_.act = s->act;
-        k_.shared_gate = s->shared_gate, k_.arrive = s->arrive;
+        k_.shared_gate = s->shared_gate, k_.hand = s->hand;
         k_.expert_out = (flags & WD_MOE_KEEP_EXPERT_OUT) ? s->expert_out : nullptr;
         k_.accum = s->accum, k_.down_f32 = s->down_f32;
         k_.tagged = s->tagged, k_.status = s->status;

@@ -24,17 +24,17 @@ uint8_t *g_scratch_ptr[kNoAllocMaxDevices];  // the array's address on each devi
 int g_compute_units[kNoAllocMaxDevices];
 
 // Offsets inside the array (fixed, so that the head of the array is the same whatever the layer).
-constexpr size_t kOffStatus = 0, kOffArrive = 256, kOffTagged = 512;              // words that must start clean: 512 + 1024 bytes
-constexpr size_t kOffIds = kOffTagged + sizeof(uint32_t) * kTagCopies * 16;        // int32 [16]
+constexpr size_t kOffStatus = 0, kOffTagged = 256;                                 // words that must start clean: status, tagged, hand
+constexpr size_t kOffHand = kOffTagged + sizeof(uint32_t) * kTagCopies * 16;       // uint32 [experts + 2]
+constexpr size_t kOffIds = (kOffHand + sizeof(uint32_t) * (kNoAllocMaxExperts + 2) + 255) & ~static_cast<size_t>(255);  // int32 [16]
 constexpr size_t kOffWeights = kOffIds + 256, kOffGate = kOffWeights + 256;       // f32 [16], f32 [1]
 constexpr size_t kOffLogits = kOffGate + 256;                                      // f32 [experts]
 constexpr size_t kOffVectors = kOffLogits + sizeof(float) * kNoAllocMaxExperts;    // accum, down_f32: f32 [hidden] each; then act
 
-// status, arrive = 0; the published ids = "not yet"
+// status = 0; the published ids and the handed logits = "not yet"
 __global__ void k_noalloc_clean(uint32_t *head) {
-    const int i = threadIdx.x;
-    if (i < static_cast<int>(kOffTagged / 4)) head[i] = 0u;
-    if (i < kTagCopies * 16) head[kOffTagged / 4 + i] = kTagInvalid;
+    static_assert(kTagInvalid == kHandEmpty, "one fill for both");
+    for (int i = threadIdx.x; i < static_cast<int>(kOffIds / 4); i += blockDim.x) head[i] = i < static_cast<int>(kOffTagged / 4) ? 0u : kTagInvalid;
 }
 
 }  // namespace
@@ -79,7 +79,7 @@ extern "C" int wd_moe_layer_noalloc_f32(const wd_moe_layer *L, const float *d_x,
     wd_moe_scratch view;  // a host-side description of where things lie in the array; owns nothing
     view.hidden = L->hidden, view.ffn = L->expert_ffn, view.n_experts = L->n_experts, view.max_k = L->top_k;
     view.status = reinterpret_cast<unsigned *>(ptr + kOffStatus);
-    view.arrive = reinterpret_cast<unsigned *>(ptr + kOffArrive);
+    view.hand = reinterpret_cast<uint32_t *>(ptr + kOffHand);
     view.tagged = reinterpret_cast<uint32_t *>(ptr + kOffTagged);
     view.ids = reinterpret_cast<int32_t *>(ptr + kOffIds);
     view.weights = reinterpret_cast<float *>(ptr + kOffWeights);

@@ -64,8 +64,10 @@ int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cac
         int rc = WD_OK;
         if (!resident) {
             rc = wd_expert_cache_acquire(cache, static_cast<int>(l), s->h_ids, k, nullptr, st);
-            if (rc) {  // (dispatch C, which makes the published ids invalid again, does not follow)
+            if (rc) {  // (dispatch C, which sets the published ids and the handed logits back, does not follow)
+                const size_t n = static_cast<size_t>(s->n_experts) + 2;
                 enqueue(k_fill_u32, dim3(1), dim3(kTagCopies * 16), 0, st, s->tagged, kTagInvalid, static_cast<size_t>(kTagCopies) * 16);
+                enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
                 return rc;
             }
             rc = launch(l, WD_MOE_ONLY_B, false);

@@ -48,7 +48,7 @@ struct TokenSlots {
     float *weights;
     float *act;          // [k+1][F]
     float *shared_gate;  // [1]
-    unsigned *arrive;
+    uint32_t *hand;      // (LayerArgs)
     float *expert_out;   // null or [k][H]
     float *accum, *down_f32, *out;
     uint32_t *tagged;    // [kTagCopies][16] selected ids published inside dispatch AB (kTagInvalid = not yet)
@@ -105,39 +105,36 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wg < a.n_router_wgs) {
         const int rows = a.preselected ? 0 : a.E;
+        int row;
+        float logit;
         if (WIDE)
-            router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.logits, rows, H,
-                                  a.sh_inp, s.shared_gate, wg);
+            logit = router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.hand, rows, H, a.sh_inp, a.E, wg, row);
         else
-            router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.logits, rows, H, a.sh_inp, s.shared_gate, wg);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's stores have been acknowledged
-        __syncthreads();
-        if (threadIdx.x == 0)
-            s_last = (__hip_atomic_fetch_add(s.arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
-                      static_cast<unsigned>(a.n_router_wgs - 1));
+            logit = router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.hand, rows, H, a.sh_inp, a.E, wg, row);
+        if (lane == 32 && row >= 0 && row < rows) s.logits[row] = logit;  // (the caller's view)
+        __syncthreads();  // (every wave has sent its word)
+        if (threadIdx.x == 0) s_last = hand_count_last(s.hand, a.E, a.n_router_wgs);
         __syncthreads();
         if (!s_last) return;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        if (!a.preselected) {
-            static_assert(kTokensWorkBytes >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
-            int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
-            float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
-            topk_block(s.logits, a.E, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr, ta.wait_ids ? s.tagged : nullptr, kTagCopies);
-            if (wave == 0) {
-                wave_lds_fence();
-                if (lane < a.k) {
-                    s.ids[lane] = lds_ids[lane];
-                    s.weights[lane] = lds_w[lane];
-                }
+        static_assert(kTokensWorkBytes >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
+        int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
+        float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
+        if (a.preselected) {  // (the one row is the shared gate's)
+            if (wave == 5) {
+                float none[1];
+                (void)hand_gather<1, true>(HandRow{s.hand, 0, a.E, true}, lane, none);
             }
+        } else {
+            (void)topk_block<true>(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, s_last, lane, wave, nullptr,
+                                   ta.wait_ids ? s.tagged : nullptr, kTagCopies);
         }
-        if (wave == 5 && lane == 0) {
-            if (a.sh_inp) {
-                const float g = __hip_atomic_load(s.shared_gate, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s.shared_gate[0] = sigmoid_ggml(g);
+        if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(s.hand + a.E)));
+        if (!a.preselected && wave == 0) {
+            wave_lds_fence();
+            if (lane < a.k) {
+                s.ids[lane] = lds_ids[lane];
+                s.weights[lane] = lds_w[lane];
             }
-            s.arrive[0] = 0u;
         }
         return;
     }
@@ -586,12 +583,12 @@ __global__ __launch_bounds__(512, 4) void k_tokens_ab_q8(TokenArgs ta) {
 }
 
 // ---- dispatch C for T tokens ----------------------------------------------------------------------------
-// (workgroup 0) The ids published for the dispatch before are made invalid again.
-WD_DEV void tokens_clear_tagged(const TokenArgs &ta) {
-    if (blockIdx.x != 0) return;
-    for (int t = 0; t < ta.T; ++t)
-        for (int i = threadIdx.x; i < kTagCopies * 16; i += blockDim.x)
-            __hip_atomic_store(ta.tok[t].tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// As layer_clear_handed: workgroup t for token t, by its last wave, which has the fewest items.
+WD_DEV void tokens_clear_handed(const TokenArgs &ta, int waves, int tw, int lane) {
+    if (static_cast<int>(blockIdx.x) >= ta.T || tw != waves - 1) return;
+    const TokenSlots &s = ta.tok[blockIdx.x];
+    for (int i = lane; i < kTagCopies * 16; i += 64) __hip_atomic_store(s.tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = lane; i < ta.common.E + 2; i += 64) __hip_atomic_store(s.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // grid = H / 8: a workgroup owns eight output rows, as the one-token k_layer_c8 does.  Work items are (token, matrix) with
 // matrix = the token's k routed down tensors, then the shared one (always Q8_0); the waves take them in turn: the
@@ -620,7 +617,7 @@ void k_tokens_c(TokenArgs ta) {
     const int per_token = a.k + (shared ? 1 : 0), n_items = ta.T * per_token;
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;  // hidden is a multiple of 8
     mark(a, 2, 0);
-    tokens_clear_tagged(ta);
+    tokens_clear_handed(ta, kWaves, tw, lane);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
     const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
     // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
@@ -716,7 +713,7 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
     const int rows_per_wg = a.H >> 8, r0 = blockIdx.x * rows_per_wg, nb = a.F >> 5;
     const int n_groups = rows_per_wg * LPR > 64 ? 2 : 1, rows0 = n_groups == 2 ? (rows_per_wg + 1) >> 1 : rows_per_wg;
     mark(a, 2, 0);
-    tokens_clear_tagged(ta);
+    tokens_clear_handed(ta, kWaves, tw, lane);
     // every routed id of the pass, one vector load per wave; an item's id is then a lane read
     const int id_lo = token_pair_id(ta, lane), id_hi = token_pair_id(ta, lane + 64);
     // combine operands of token `tw`, requested early: lane j keeps router weight j, lane 16 the shared gate
