@@ -52,10 +52,17 @@ int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cac
         for (int j = 0; j < 16; ++j) reinterpret_cast<volatile uint32_t *>(report)[j] = kTagInvalid;
         return launch(l, WD_MOE_ONLY_A | WD_MOE_ONLY_B, true);
     };
-    if (const int rc = launch_ab(0)) return rc;
+    // (an error behind a dispatch AB: dispatch C, which sets the published ids and the handed logits back, does not follow)
+    auto leave = [&](int rc) {
+        const size_t n = static_cast<size_t>(s->n_experts) + 2;
+        enqueue(k_fill_u32, dim3(1), dim3(kTagCopies * 16), 0, st, s->tagged, kTagInvalid, static_cast<size_t>(kTagCopies) * 16);
+        enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
+        return rc;
+    };
+    if (const int rc = launch_ab(0)) return leave(rc);
     for (size_t l = 0; l < bound.size(); ++l) {
         const int k = bound[l].top_k;
-        if (const int rc = wait_report(report, k, st)) return rc;
+        if (const int rc = wait_report(report, k, st)) return leave(rc);
         bool resident = true;
         for (int j = 0; j < k; ++j) {
             s->h_ids[j] = static_cast<int32_t>(report[j]);
@@ -64,13 +71,7 @@ int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cac
         int rc = WD_OK;
         if (!resident) {
             rc = wd_expert_cache_acquire(cache, static_cast<int>(l), s->h_ids, k, nullptr, st);
-            if (rc) {  // (dispatch C, which sets the published ids and the handed logits back, does not follow)
-                const size_t n = static_cast<size_t>(s->n_experts) + 2;
-                enqueue(k_fill_u32, dim3(1), dim3(kTagCopies * 16), 0, st, s->tagged, kTagInvalid, static_cast<size_t>(kTagCopies) * 16);
-                enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
-                return rc;
-            }
-            rc = launch(l, WD_MOE_ONLY_B, false);
+            if (rc == WD_OK) rc = launch(l, WD_MOE_ONLY_B, false);
         }
         if (rc == WD_OK) rc = launch(l, WD_MOE_ONLY_C, false);
         if (rc == WD_OK && l + 1 < bound.size()) rc = launch_ab(l + 1);
@@ -78,7 +79,7 @@ int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cac
             const int rc_books = wd_expert_cache_acquire(cache, static_cast<int>(l), s->h_ids, k, nullptr, st);
             if (rc == WD_OK) rc = rc_books;
         }
-        if (rc) return rc;
+        if (rc) return leave(rc);
     }
     return WD_OK;
 }
