@@ -391,3 +391,66 @@ def test_selections_reported_to_the_host(g, H, F, E, k, gate, down, shared, slot
     sc.close()
     sc2.close()
     capi.call("wd_expert_cache_destroy", cache)
+
+
+@pytest.mark.parametrize("gate,shared", [(synth.IQ3_S, True), (synth.Q8_0, False)])
+def test_an_error_behind_a_reported_selection(g, oracle, tmp_path, gate, shared):
+    """The file behind the second layer's experts has lost its tail: the call ends with an error when that layer's selection has
+    been reported and its dispatch AB is queued.  On the same scratch the passes after it - a layer, a token batch, and with the
+    file whole again the stack - give the oracle's and the resident stack's results."""
+    import mmap
+    import os
+    H, F, E, k, NL = 512, 64, 16, 4, 2
+    layers = [synth.make_layer(H, F, E, k, gate, synth.Q8_0, shared, seed=SEED, layer=230 + l, router_sigma=1.0 / np.sqrt(H)) for l in range(NL)]
+    gb, db = F * synth.row_bytes(gate, H), H * synth.row_bytes(synth.Q8_0, F)
+    parts = [np.ascontiguousarray(L[n]).view(np.uint8).reshape(-1) for L in layers for n in ("gate", "up", "down")]
+    data = np.concatenate(parts)
+    starts = np.cumsum([0] + [p.size for p in parts])
+    path = tmp_path / "experts.bin"
+    data.tofile(path)
+    fd = os.open(path, os.O_RDWR)
+    mm = mmap.mmap(fd, data.size)
+    base = np.frombuffer(mm, dtype=np.uint8).ctypes.data
+    cache, lib = C.c_void_p(), capi.load()
+    capi.call("wd_expert_cache_create", C.byref(cache), 12 * (2 * gb + db), gb, gb, db, NL, E, 0)
+    dls = [g.DeviceLayer(L) for L in layers]
+    whole, bare = (capi.MoeLayer * NL)(*[d.desc for d in dls]), (capi.MoeLayer * NL)(*[d.desc for d in dls])
+    for l in range(NL):
+        capi.call("wd_expert_cache_register_layer", cache, l, *[C.c_void_p(base + int(starts[3 * l + q])) for q in range(3)])
+        bare[l].gate = bare[l].up = bare[l].down = None
+    capi.call("wd_expert_cache_attach_file", cache, C.c_void_p(base), data.size, fd, 2)
+    xs = np.stack([synth.rms_normed(synth.rng_for(SEED, 84, t), H) for t in range(4)])
+    scr, sc2 = [g.Scratch(H, F, E, k) for _ in range(2)], g.Scratch(H, F, E, k)
+    arr = (C.c_void_p * 2)(*[s.h for s in scr])
+
+    def stack_fails():
+        os.ftruncate(fd, int(starts[3]))
+        x, out = g.dev(xs[0]), g.empty(H, np.float32)
+        rc = lib.wd_moe_stack_cached_f32(bare, NL, cache, g.ptr(x), g.ptr(out), scr[0].h, None, None, 0.05, 0, g.stream())
+        assert rc < 0 and "pread" in lib.wd_last_error().decode()
+        os.ftruncate(fd, data.size)
+        os.pwrite(fd, data[starts[3]:].tobytes(), int(starts[3]))
+
+    for after in ("layer", "batch", "stack"):
+        stack_fails()
+        x, out = g.dev(xs[1:3]), g.empty((2, H), np.float32)
+        if after == "stack":
+            x2, out2 = g.dev(xs[1:3]), g.empty((2, H), np.float32)
+            capi.call("wd_moe_stack_cached_f32", bare, NL, cache, g.ptr(x), g.ptr(out), scr[0].h, None, None, 0.05, 0, g.stream())
+            capi.call("wd_moe_stack_f32", whole, NL, g.ptr(x2), g.ptr(out2), sc2.h, None, 0.05, 0, g.stream())
+            g.sync()
+            assert g.same_bits(g.host(x), g.host(x2)) and g.same_bits(g.host(out), g.host(out2))
+            continue
+        if after == "layer":
+            capi.call("wd_moe_layer_f32", C.byref(dls[0].desc), g.ptr(x), g.ptr(out), scr[0].h, 0, g.stream())
+        else:
+            capi.call("wd_moe_layer_tokens_f32", C.byref(dls[0].desc), g.ptr(x), g.ptr(out), 2, arr, 0, g.stream())
+        g.sync()
+        for t in range(1 if after == "layer" else 2):
+            assert g.same_bits(g.host(out)[t], oracle.moe_layer(layers[0], xs[1 + t])[0]), (after, t)
+    assert lib.wd_moe_scratch_status(scr[0].h) == 0
+    for s in scr + [sc2]:
+        s.close()
+    capi.call("wd_expert_cache_destroy", cache)
+    del base
+    os.close(fd)

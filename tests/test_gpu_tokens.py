@@ -210,3 +210,50 @@ def test_bounded_wait_of_a_token_batch(g, oracle, gate, F):
     assert [lib.wd_moe_scratch_status(s.h) for s in scr] == [0] * T
     for s in scr:
         s.close()
+
+
+@pytest.mark.parametrize("shape", ["eight-blocks", "q8_0", "ids-by-the-block-form"])
+def test_passes_that_end_before_the_down_projections(g, oracle, shape):
+    """Calls of dispatch A or of A and B without C, on one input, leave nothing on the scratch that a pass of another kind takes
+    for its own: one-token layers, token batches and the dispatches one by one, on other inputs, give the oracle's results."""
+    H, F, E, k, gate, shared = {"eight-blocks": (2048, 64, 64, 6, synth.IQ3_S, True), "q8_0": (512, 96, 24, 4, synth.Q8_0, False),
+                                "ids-by-the-block-form": (512, 64, 640, 10, synth.IQ2_S, True)}[shape]
+    T = 3
+    L = synth.make_layer(H, F, E, k, gate, synth.Q8_0, shared, seed=SEED, layer=35, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, 2 * T, 11, mix=0.2)
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    arr = (C.c_void_p * T)(*[s.h for s in scr])
+    stack = (capi.MoeLayer * 3)(dl.desc, dl.desc, dl.desc)
+    dx, out = g.dev(xs), g.empty((T, H), np.float32)
+    want = [oracle.moe_layer(L, x)[0] for x in xs]
+    A, B, CC = capi.MOE_ONLY_A, capi.MOE_ONLY_B, capi.MOE_ONLY_C
+    row = lambda b, t: C.c_void_p(b.data_ptr() + 4 * H * t)
+
+    def layer(t, x, flags):
+        capi.call("wd_moe_layer_f32", C.byref(dl.desc), row(dx, x), row(out, t), scr[t].h, flags, g.stream())
+
+    def one_by_one(t, x):
+        layer(t, x, A)
+        layer(t, x, B | capi.MOE_PRESELECTED)
+        layer(t, x, CC | capi.MOE_PRESELECTED)
+
+    before = {"A": lambda: [layer(t, T + t, A) for t in range(T)],
+              "A and B": lambda: [layer(t, T + t, A | B) for t in range(T)],
+              "A and B apart": lambda: [layer(t, T + t, A | B | capi.MOE_SPLIT_AB) for t in range(T)],
+              "a batch's A and B": lambda: capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), row(dx, T), g.ptr(out), T, arr, A | B, g.stream()),
+              "a stack's A and B": lambda: [capi.call("wd_moe_stack_f32", stack, 3, row(dx, T), row(out, 0), s.h, None, 0.0, A | B, g.stream()) for s in scr]}
+    passes = {"batch": lambda: capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), row(dx, 0), g.ptr(out), T, arr, 0, g.stream()),
+              "batch in two": lambda: capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), row(dx, 0), g.ptr(out), T, arr, capi.MOE_SPLIT_AB, g.stream()),
+              "layer": lambda: [layer(t, t, 0) for t in range(T)], "one by one": lambda: [one_by_one(t, t) for t in range(T)]}
+    for first, ends_early in before.items():
+        for second, whole in passes.items():
+            ends_early()
+            ends_early()
+            out.zero_()
+            whole()
+            g.sync()
+            for t in range(T):
+                assert g.same_bits(g.host(out)[t], want[t]), (first, second, t)
+    assert [capi.load().wd_moe_scratch_status(s.h) for s in scr] == [0] * T
+    for s in scr:
+        s.close()

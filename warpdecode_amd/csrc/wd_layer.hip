@@ -651,11 +651,31 @@ bool layer_c_evenly(int H, int F, int n_act, bool words) {
     return R > 8 && R <= 16 && n_act >= (R <= 12 ? 5 : 6) && !(words && R > 12);
 }
 
+// What dispatches A and AB hand on - the ids published in the scratch's records, the logits and the ticket - is set back by dispatch C.
+// These do it where C does not follow: a pass that finds what another one left takes that one's ids.
+int reset_published(const wd_moe_scratch *s, int first, int records, hipStream_t st) {
+    const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(records) * record;
+    enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->tagged + static_cast<size_t>(first % kTagRecords) * record, kTagInvalid, n);
+    WD_LAUNCH_CHECK();
+    return WD_OK;
+}
+int reset_hand(const wd_moe_scratch *s, hipStream_t st) {
+    const size_t n = static_cast<size_t>(s->n_experts) + 2;
+    enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
+    WD_LAUNCH_CHECK();
+    return WD_OK;
+}
+int reset_handed(const wd_moe_scratch *s, int rec, hipStream_t st) {
+    const int rc = reset_published(s, rec, 1, st), rc_hand = reset_hand(s, st);
+    return rc ? rc : rc_hand;
+}
+
 // report: null, or the host words that dispatch AB reports its selection to.  An expert without a slot is then no error: its
 // rows are computed again once it has one.
-int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
-                const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec = 0,
-                const HcSpec *hc = nullptr, uint32_t *report = nullptr) {
+// rec: which of the scratch's records of published ids the pass uses; chain: the caller sets it back.
+int layer_fused_queue(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
+                      const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec,
+                      const HcSpec *hc, uint32_t *report, bool chain) {
     const int H = L->hidden, F = L->expert_ffn, k = L->top_k;
     const bool shared = L->shared_gate_inp != nullptr;
     LayerArgs a = fused_args(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, rec, hc);
@@ -680,11 +700,10 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
     }
     if (only && !(only & WD_MOE_ONLY_C)) {
         // dispatch C, which sets the handed words back, is not part of this call (with a report it follows in the same one)
-        if (run_a && !report && !a.dry) {
-            enqueue(k_fill_u32, dim3((L->n_experts + 2 + 255) / 256), dim3(256), 0, st, s->hand, kHandEmpty, static_cast<size_t>(L->n_experts) + 2);
-            WD_LAUNCH_CHECK();
-        }
-        return WD_OK;
+        if (report || a.dry) return WD_OK;
+        if (merged && !chain)
+            if (const int rc = reset_published(s, rec, 1, st)) return rc;
+        return run_a ? reset_hand(s, st) : static_cast<int>(WD_OK);
     }
     SiteScope site(WD_SITE_FUSED_C, st);
     const int n_act = k + (shared ? 1 : 0);
@@ -710,14 +729,22 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
     return WD_OK;
 }
 
+int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
+                const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec = 0,
+                const HcSpec *hc = nullptr, uint32_t *report = nullptr, bool chain = false) {
+    const int rc = layer_fused_queue(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, st, rec, hc, report, chain);
+    if (rc != WD_OK) (void)reset_handed(s, rec, st);  // (an error behind dispatch A or AB: C does not follow)
+    return rc;
+}
+
 int layer_dispatch(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_scratch *s, unsigned flags,
                    const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec = 0,
-                   const HcSpec *hc = nullptr) {
+                   const HcSpec *hc = nullptr, bool chain = false) {
     const bool want_partials = s->gup != nullptr;
     const bool fused_exports = consumes_q8k(L->gate_type) && s->gup_type == L->gate_type && s->dp_type == L->down_type;
     if ((flags & WD_MOE_STAGED) || (want_partials && !fused_exports))
         return layer_staged(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, st, hc);
-    return layer_fused(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, st, rec, hc);
+    return layer_fused(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, st, rec, hc, nullptr, chain);
 }
 
 }  // namespace
@@ -946,18 +973,21 @@ extern "C" int wd_moe_stack_f32(const wd_moe_layer *layers, int n_layers, float 
         if (rc != kTakePerLayer) return rc;
     }
     flags &= ~WD_MOE_PER_LAYER;
-    const unsigned only = flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B | WD_MOE_ONLY_C);
+    const hipStream_t st = as_stream(stream);
+    // (layers without dispatch C leave their ids in a record each: all are set back when they have been used, and at the end)
+    const bool chain = (flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B)) && !(flags & WD_MOE_ONLY_C);
     for (int l = 0; l < n_layers; ++l) {
         const int32_t *trace = d_ids_trace ? d_ids_trace + static_cast<size_t>(l) * layers[l].top_k : nullptr;
-        if (only && !(only & WD_MOE_ONLY_C) && l % kTagRecords == 0) {
-            // no dispatch C to invalidate the published ids: reset all records before they are used again
-            const size_t n = static_cast<size_t>(kTagRecords) * kTagCopies * 16;
-            enqueue(k_fill_u32, dim3((n + 255) / 256), dim3(256), 0, as_stream(stream), s->tagged, kTagInvalid, n);
-            WD_LAUNCH_CHECK();
+        int rc = WD_OK;
+        {
+            SiteScope layer_site(WD_SITE_ROUTED_TOTAL, st);
+            rc = layer_dispatch(&layers[l], d_x, d_layer_out, s, flags, trace, d_x, residual_scale, st, l, nullptr, chain);
         }
-        SiteScope layer_site(WD_SITE_ROUTED_TOTAL, as_stream(stream));
-        if (const int rc = layer_dispatch(&layers[l], d_x, d_layer_out, s, flags, trace, d_x, residual_scale, as_stream(stream), l))
-            return rc;
+        if (chain && (rc || l + 1 == n_layers || (l + 1) % kTagRecords == 0)) {
+            const int rc_reset = reset_published(s, 0, kTagRecords, st);
+            if (rc == WD_OK) rc = rc_reset;
+        }
+        if (rc) return rc;
     }
     return WD_OK;
 }
@@ -1099,30 +1129,36 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         WD_LAUNCH_CHECK();
         return static_cast<int>(WD_OK);
     };
-    // One launch where the ids come out of it; ids that are there already need no wait, and the site profiler brackets the parts
-    if (!a.preselected && !(flags & WD_MOE_SPLIT_AB) && !SiteProfiler::instance().enabled()) {
-        if (const int rc = launch_ab(true, true)) return rc;
-    } else {
-        if (grid_a > 0) {  // router, selection and shared gate/up of every token
-            SiteScope site(WD_SITE_TOKENS_A, st);
-            if (const int rc = launch_ab(true, false)) return rc;
+    auto queue = [&]() {
+        // One launch where the ids come out of it; ids that are there already need no wait, and the site profiler brackets the parts
+        if (!a.preselected && !(flags & WD_MOE_SPLIT_AB) && !SiteProfiler::instance().enabled()) {
+            if (const int rc = launch_ab(true, true)) return rc;
+        } else {
+            if (grid_a > 0) {  // router, selection and shared gate/up of every token
+                SiteScope site(WD_SITE_TOKENS_A, st);
+                if (const int rc = launch_ab(true, false)) return rc;
+            }
+            SiteScope site(WD_SITE_TOKENS_B, st);
+            if (const int rc = launch_ab(false, true)) return rc;
         }
-        SiteScope site(WD_SITE_TOKENS_B, st);
-        if (const int rc = launch_ab(false, true)) return rc;
-    }
-    SiteScope c_site(WD_SITE_TOKENS_C, st);
-    if (!down_tokens) {
-        WD_REQUIRE(!down_table, "multi-token pass on a pointer table: this down tensor (type %d, %d columns) has no multi-token dispatch", L->down_type, F);
-        for (int t = 0; t < tokens; ++t)
-            if (const int rc = layer_fused(L, d_x + static_cast<size_t>(t) * H, d_out + static_cast<size_t>(t) * H, scratch_per_token[t],
-                                           flags | WD_MOE_ONLY_C, nullptr, nullptr, 0.0f, st))
-                return rc;
-        return WD_OK;
-    }
-    if (const int lanes = tokens_c_even_lanes(H, F)) L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c_even<0>(lanes, ta, st) : launch_tokens_c_even<1>(lanes, ta, st);
-    else L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c<0>(ta, st) : launch_tokens_c<1>(ta, st);
-    WD_LAUNCH_CHECK();
-    return WD_OK;
+        SiteScope c_site(WD_SITE_TOKENS_C, st);
+        if (!down_tokens) {
+            WD_REQUIRE(!down_table, "multi-token pass on a pointer table: this down tensor (type %d, %d columns) has no multi-token dispatch", L->down_type, F);
+            for (int t = 0; t < tokens; ++t)
+                if (const int rc = layer_fused(L, d_x + static_cast<size_t>(t) * H, d_out + static_cast<size_t>(t) * H, scratch_per_token[t],
+                                               flags | WD_MOE_ONLY_C, nullptr, nullptr, 0.0f, st))
+                    return rc;
+            return static_cast<int>(WD_OK);
+        }
+        if (const int lanes = tokens_c_even_lanes(H, F)) L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c_even<0>(lanes, ta, st) : launch_tokens_c_even<1>(lanes, ta, st);
+        else L->down_type == WD_TYPE_Q8_0 ? launch_tokens_c<0>(ta, st) : launch_tokens_c<1>(ta, st);
+        WD_LAUNCH_CHECK();
+        return static_cast<int>(WD_OK);
+    };
+    const int rc = queue();
+    if (rc != WD_OK)  // (as in layer_fused)
+        for (int t = 0; t < tokens; ++t) (void)reset_handed(scratch_per_token[t], 0, st);
+    return rc;
 }
 }  // namespace
 

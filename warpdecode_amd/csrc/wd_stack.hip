@@ -52,11 +52,10 @@ int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cac
         for (int j = 0; j < 16; ++j) reinterpret_cast<volatile uint32_t *>(report)[j] = kTagInvalid;
         return launch(l, WD_MOE_ONLY_A | WD_MOE_ONLY_B, true);
     };
-    // (an error behind a dispatch AB: dispatch C, which sets the published ids and the handed logits back, does not follow)
+    // (an error behind a dispatch AB: its dispatch C does not follow, and its report must not come into the next call's)
     auto leave = [&](int rc) {
-        const size_t n = static_cast<size_t>(s->n_experts) + 2;
-        enqueue(k_fill_u32, dim3(1), dim3(kTagCopies * 16), 0, st, s->tagged, kTagInvalid, static_cast<size_t>(kTagCopies) * 16);
-        enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
+        (void)reset_handed(s, 0, st);
+        (void)hipStreamSynchronize(st);
         return rc;
     };
     if (const int rc = launch_ab(0)) return leave(rc);
