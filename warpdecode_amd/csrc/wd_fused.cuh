@@ -43,9 +43,10 @@ struct LayerArgs {
     int n_shared_wgs;            // those that take the shared expert's gate/up (the rest: routed gate/up)
     int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
     const int32_t *ids_known;    // null, or the k ids where they are known before the launch
-    uint32_t *hand;              // [E + 2]: the router's logits and the shared gate's on their way to the selection, then a ticket or count; kHandEmpty between passes
+    uint32_t *hand;              // [E + 3]: the router's logits and the shared gate's on their way to the selection, a ticket or count, and the count of hand_close; kHandEmpty between passes
     uint32_t *ids_tagged;        // [kTagCopies][16] selected ids published inside the merged dispatch (kTagInvalid = not yet)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
+    int close_hand;              // no dispatch C follows: the router workgroups set `hand` back themselves
     unsigned *status;            // [0] set to 1 when a bounded wait inside a dispatch ran out
     unsigned spin_limit;         // polls (about a microsecond each) before such a wait gives up
     unsigned long long *trace;   // profiling aid: null, or [3][16][8] time stamps (100 MHz) of workgroup trace_wg
@@ -684,6 +685,18 @@ WD_DEV uint32_t hand_load(const uint32_t *p) { return __hip_atomic_load(p, __ATO
 WD_DEV uint32_t hand_draw(uint32_t *hand, int n_slot) { return __hip_atomic_fetch_add(hand + n_slot + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 // One thread: whether its workgroup is the last of n_wgs.
 WD_DEV bool hand_count_last(uint32_t *hand, int n_slot, int n_wgs) { return hand_draw(hand, n_slot) + 1u == static_cast<uint32_t>(n_wgs - 1); }
+// Sets the words back where no dispatch C does: the router workgroup that is done last, behind every other one's last use of them.  Every
+// thread of each of the n_wgs must call it.  (A fill launched behind the dispatch instead, us per layer with the ids through the host: 2048 / 512
+// 46.2, so 45.0; 1024 / 256 37.9, 36.9; 4096 / 1536 66.5, 65.5.)
+WD_DEV void hand_close(uint32_t *hand, int n_slot, int n_wgs, int &last) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);  // what this wave has asked for of the words is there
+    __syncthreads();
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(hand + n_slot + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == static_cast<uint32_t>(n_wgs - 1);
+    __syncthreads();
+    if (!last) return;
+    for (int i = threadIdx.x; i < n_slot + 3; i += static_cast<int>(blockDim.x)) __hip_atomic_store(hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // lv[j]: logit 64 j + lane; whether the row is complete.  POLL: once it is (it must be about to; the limit is there for a broken device).
 template <int M, bool POLL>
 WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
@@ -1041,6 +1054,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
             if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
         }
         mark<TRACE>(a, 0, 2);
+        if (a.close_hand) hand_close(a.hand, a.E, a.n_router_wgs, s_last);
         return;
     }
 

@@ -35,7 +35,7 @@ struct wd_moe_scratch {
     int32_t *gup = nullptr;
     int32_t *dp = nullptr;
     int gup_type = -1, dp_type = -1;
-    uint32_t *hand = nullptr;             // [n_experts + 2] logits on their way to the selection inside dispatch AB (LayerArgs)
+    uint32_t *hand = nullptr;             // [n_experts + 3] logits on their way to the selection inside dispatch AB (LayerArgs)
     unsigned long long *trace = nullptr;  // device [3][16][8] time stamps, see wd_moe_scratch_trace
     int trace_wg = 0;
     int32_t *h_ids = nullptr;             // pinned [48]: [0..15] routed ids for callers that must see them on the host,
@@ -103,7 +103,7 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
                  o_act = c.take(sizeof(float) * K1 * F), o_aq = c.take(K1 * F),
                  o_ad = c.take(sizeof(uint16_t) * K1 * (F / 32)), o_eo = c.take(sizeof(float) * K1 * H),
                  o_acc = c.take(sizeof(float) * H), o_dn = c.take(sizeof(float) * H), o_sg = c.take(256),
-                 o_hand = c.take(sizeof(uint32_t) * (n_experts + 2)),
+                 o_hand = c.take(sizeof(uint32_t) * (n_experts + 3)),
                  o_tag = c.take(sizeof(uint32_t) * kTagRecords * kTagCopies * 16), o_status = c.take(256);
     const hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->block), c.off);
     if (e != hipSuccess) {
@@ -135,7 +135,7 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
     s->status = reinterpret_cast<unsigned *>(b + o_status);
     (void)hipMemset(s->block, 0, c.off);
     (void)hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16);
-    (void)hipMemset(s->hand, 0xff, sizeof(uint32_t) * (n_experts + 2));
+    (void)hipMemset(s->hand, 0xff, sizeof(uint32_t) * (n_experts + 3));
     if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 48, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->block);
         delete s;
@@ -178,7 +178,7 @@ int wd_moe_scratch_set_wait_limit(wd_moe_scratch *s, unsigned polls) {
     WD_HIP(hipMemset(s->status, 0, sizeof(unsigned)));
     reinterpret_cast<volatile int32_t *>(s->h_ids)[16] = 0;
     WD_HIP(hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16));
-    WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 2)));
+    WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 3)));
     if (s->res_block) WD_HIP(hipMemset(s->res_block, 0xff, kHandEpoch));
     return WD_OK;
 }
@@ -651,23 +651,21 @@ bool layer_c_evenly(int H, int F, int n_act, bool words) {
     return R > 8 && R <= 16 && n_act >= (R <= 12 ? 5 : 6) && !(words && R > 12);
 }
 
-// What dispatches A and AB hand on - the ids published in the scratch's records, the logits and the ticket - is set back by dispatch C.
-// These do it where C does not follow: a pass that finds what another one left takes that one's ids.
+// What dispatches A and AB hand on - the ids published in the scratch's records, the logits and the ticket - is set back by dispatch C,
+// and where C does not follow by the dispatch itself (the logits, close_hand) and by these: a pass that finds what another one left
+// takes that one's ids.
 int reset_published(const wd_moe_scratch *s, int first, int records, hipStream_t st) {
     const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(records) * record;
     enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->tagged + static_cast<size_t>(first % kTagRecords) * record, kTagInvalid, n);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
-int reset_hand(const wd_moe_scratch *s, hipStream_t st) {
-    const size_t n = static_cast<size_t>(s->n_experts) + 2;
+// Both, behind an error after which no dispatch C comes.  (The error stays the one to report.)
+void reset_handed(const wd_moe_scratch *s, int rec, hipStream_t st) {
+    const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(s->n_experts) + 3;
+    enqueue(k_fill_u32, dim3(1), dim3(static_cast<unsigned>(record)), 0, st, s->tagged + static_cast<size_t>(rec % kTagRecords) * record, kTagInvalid, record);
     enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
-    WD_LAUNCH_CHECK();
-    return WD_OK;
-}
-int reset_handed(const wd_moe_scratch *s, int rec, hipStream_t st) {
-    const int rc = reset_published(s, rec, 1, st), rc_hand = reset_hand(s, st);
-    return rc ? rc : rc_hand;
+    (void)hipGetLastError();
 }
 
 // report: null, or the host words that dispatch AB reports its selection to.  An expert without a slot is then no error: its
@@ -682,6 +680,7 @@ int layer_fused_queue(const wd_moe_layer *L, const float *d_x, float *d_out, wd_
     if (report) a.host_ids = report, a.gate_up.slot_status = nullptr;
     const unsigned only = flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B | WD_MOE_ONLY_C);
     const bool run_a = !only || (only & WD_MOE_ONLY_A), run_b = !only || (only & WD_MOE_ONLY_B);
+    a.close_hand = only && !(only & WD_MOE_ONLY_C) && !report;
     // router + selection + shared gate/up + routed gate/up in one launch (the routed workgroups wait for the ids
     // inside the dispatch) unless the caller asked for the two parts apart
     const bool merged = run_a && run_b && !(flags & WD_MOE_SPLIT_AB);
@@ -700,10 +699,7 @@ int layer_fused_queue(const wd_moe_layer *L, const float *d_x, float *d_out, wd_
     }
     if (only && !(only & WD_MOE_ONLY_C)) {
         // dispatch C, which sets the handed words back, is not part of this call (with a report it follows in the same one)
-        if (report || a.dry) return WD_OK;
-        if (merged && !chain)
-            if (const int rc = reset_published(s, rec, 1, st)) return rc;
-        return run_a ? reset_hand(s, st) : static_cast<int>(WD_OK);
+        return merged && !chain && !report && !a.dry ? reset_published(s, rec, 1, st) : static_cast<int>(WD_OK);
     }
     SiteScope site(WD_SITE_FUSED_C, st);
     const int n_act = k + (shared ? 1 : 0);
@@ -733,7 +729,7 @@ int layer_fused(const wd_moe_layer *L, const float *d_x, float *d_out, wd_moe_sc
                 const int32_t *ids_override, float *residual, float residual_scale, hipStream_t st, int rec = 0,
                 const HcSpec *hc = nullptr, uint32_t *report = nullptr, bool chain = false) {
     const int rc = layer_fused_queue(L, d_x, d_out, s, flags, ids_override, residual, residual_scale, st, rec, hc, report, chain);
-    if (rc != WD_OK) (void)reset_handed(s, rec, st);  // (an error behind dispatch A or AB: C does not follow)
+    if (rc != WD_OK) reset_handed(s, rec, st);
     return rc;
 }
 
@@ -1157,7 +1153,7 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
     };
     const int rc = queue();
     if (rc != WD_OK)  // (as in layer_fused)
-        for (int t = 0; t < tokens; ++t) (void)reset_handed(scratch_per_token[t], 0, st);
+        for (int t = 0; t < tokens; ++t) reset_handed(scratch_per_token[t], 0, st);
     return rc;
 }
 }  // namespace

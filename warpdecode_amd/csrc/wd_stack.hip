@@ -54,7 +54,7 @@ int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cac
     };
     // (an error behind a dispatch AB: its dispatch C does not follow, and its report must not come into the next call's)
     auto leave = [&](int rc) {
-        (void)reset_handed(s, 0, st);
+        reset_handed(s, 0, st);
         (void)hipStreamSynchronize(st);
         return rc;
     };
