@@ -212,6 +212,38 @@ def test_bounded_wait_of_a_token_batch(g, oracle, gate, F):
         s.close()
 
 
+@pytest.mark.parametrize("E,k", [(64, 6), (512, 10), (640, 10)])
+@pytest.mark.parametrize("preselected", [False, True])
+def test_logits_that_are_late_are_reported(g, oracle, E, k, preselected):
+    """With a wait limit of one poll the workgroup that selects a token's experts may find logits missing (the parts are launched
+    apart, so nobody else waits): a token's results are then NaN with its status word set, and the oracle's where it is clear."""
+    H, F, T = 512, 64, 5
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=34, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, T, 10)
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    arr = (C.c_void_p * T)(*[s.h for s in scr])
+    dx, out = g.dev(xs), g.empty((T, H), np.float32)
+    lib = capi.load()
+    ids, wts = np.arange(k, dtype=np.int32), np.full(k, 0.125, np.float32)
+    flags = capi.MOE_PRESELECTED if preselected else capi.MOE_SPLIT_AB
+    want = [oracle.moe_layer(L, x, ids=ids, weights=wts)[0] if preselected else oracle.moe_layer(L, x)[0] for x in xs]
+    for limit in (1,) * 12 + (0,):
+        for s in scr:
+            capi.call("wd_moe_scratch_set_wait_limit", s.h, limit)
+            if preselected:
+                capi.call("wd_memcpy_h2d", C.c_void_p(s.raw("ids")), ids.ctypes.data_as(C.c_void_p), 4 * k, g.stream())
+                capi.call("wd_memcpy_h2d", C.c_void_p(s.raw("weights")), wts.ctypes.data_as(C.c_void_p), 4 * k, g.stream())
+        out.zero_()
+        capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, arr, flags, g.stream())
+        g.sync()
+        for t, s in enumerate(scr):
+            late = lib.wd_moe_scratch_status(s.h)
+            assert late in ((0, 1) if limit else (0,))
+            assert np.isnan(g.host(out)[t]).all() if late else g.same_bits(g.host(out)[t], want[t]), (limit, t)
+    for s in scr:
+        s.close()
+
+
 @pytest.mark.parametrize("shape", ["eight-blocks", "q8_0", "ids-by-the-block-form"])
 def test_passes_that_end_before_the_down_projections(g, oracle, shape):
     """Calls of dispatch A or of A and B without C, on one input, leave nothing on the scratch that a pass of another kind takes

@@ -680,6 +680,7 @@ struct HandRow {
     uint32_t *hand;
     int n, n_slot;
     bool gate;  // hand[n_slot] is one of the row's
+    unsigned limit;  // polls before one that waits for the row gives up
 };
 WD_DEV uint32_t hand_load(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 WD_DEV uint32_t hand_draw(uint32_t *hand, int n_slot) { return __hip_atomic_fetch_add(hand + n_slot + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -697,10 +698,11 @@ WD_DEV void hand_close(uint32_t *hand, int n_slot, int n_wgs, int &last) {
     if (!last) return;
     for (int i = threadIdx.x; i < n_slot + 3; i += static_cast<int>(blockDim.x)) __hip_atomic_store(hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// lv[j]: logit 64 j + lane; whether the row is complete.  POLL: once it is (it must be about to; the limit is there for a broken device).
+// lv[j]: logit 64 j + lane; whether the row is complete.  POLL: once it is (it must be about to; the limit is there for a broken device: words
+// that did not come are NaN, what is selected then are experts of the layer, and the status makes the results NaN).
 template <int M, bool POLL>
 WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
-    for (unsigned polls = 0; polls < (POLL ? kSpinLimit : 1u); ++polls) {
+    for (unsigned polls = 0; polls < (POLL ? r.limit : 1u); ++polls) {
         const uint32_t g = r.gate ? hand_load(r.hand + r.n_slot) : 0u;
         bool there = hand_arrived(g);
 #pragma unroll
@@ -713,7 +715,8 @@ WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
     return false;
 }
 
-// The selections below return 0: some words are not there; 1: selected, but not the one to publish; 2: the one (wave 0; other waves: 1).
+// The selections below return 0: some words are not there; 1: selected, but not the one to publish; 2: the one (wave 0; other waves: 1); 3, in the
+// wave that saw it: a poll for the row ran out (the caller sets the status).
 // n <= 64 M logits, k <= 15: wave 0 ranks and publishes the ids, wave 1 takes the exponentials and the denominator meanwhile, and wave 0 forms
 // the weights behind one barrier.  Every thread of the workgroup must call it.  ids, weights, state: LDS.
 template <int M, bool COUNT>
@@ -745,7 +748,7 @@ WD_DEV int topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids
         if (won && st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
         WD_STAMP(6);
     } else if (wave == 1) {
-        if (!COUNT && !there) (void)hand_gather<M, true>(row, lane, lv);  // (wave 0 has seen them all)
+        if (!COUNT && !there) there = hand_gather<M, true>(row, lane, lv);  // (wave 0 has seen them all)
         bool dead;
         const float inv = sel_wave_denominator(lv, n, s, lane, dead);
         if (lane == 0) s.rest[0] = inv, s.rest[1] = dead ? 1.0f : 0.0f;
@@ -758,7 +761,7 @@ WD_DEV int topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids
         WD_STAMP(7);
     }
 #undef WD_STAMP
-    return won ? 2 : 1;
+    return wave <= 1 && !there ? 3 : (won ? 2 : 1);
 }
 
 // Every thread of the workgroup must call it (COUNT: of the one that counted last).  Two waves select where one can hold the row
@@ -776,15 +779,16 @@ WD_DEV int topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, fl
         return topk_two_waves<8, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
     }
     __syncthreads();  // (COUNT: state may be the word the count was read from)
+    bool there = true;
     if (wave == 0) {
         float lv[16];
-        const bool there = hand_gather<16, COUNT>(row, lane, lv);
+        there = hand_gather<16, COUNT>(row, lane, lv);
         if (lane == 0) state = COUNT ? 2 : (!there ? 0 : (hand_draw(row.hand, row.n_slot) == kHandEmpty ? 2 : 1));
     }
     __syncthreads();
     const int got = state;
     if (got) topk_block_m<2>(reinterpret_cast<const float *>(row.hand), n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, got == 2 ? tagged : nullptr, copies);
-    return got;
+    return COUNT && !there ? 3 : got;
 }
 
 // Stand-alone softmax/top-k dispatch: one wave (src/qwen38_moe.cuh:711-818).
@@ -1039,8 +1043,9 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
         if (!a.preselected)
             // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
-            selected = topk_block<false>(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, s_last, lane, wave,
+            selected = topk_block<false>(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, s_last, lane, wave,
                                          (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
+        if (selected == 3 && lane == 0) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // off the selection's path: the shared expert's gate (by every workgroup that found the row complete: the same value)
         if (selected && a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(a.hand + a.E)));
         if (selected == 2 && wave == 0) {

@@ -52,7 +52,7 @@ struct TokenSlots {
     float *expert_out;   // null or [k][H]
     float *accum, *down_f32, *out;
     uint32_t *tagged;    // [kTagCopies][16] selected ids published inside dispatch AB (kTagInvalid = not yet)
-    unsigned *status;    // [0] set to 1 when the wait for the ids ran out
+    unsigned *status;    // [0] set to 1 when a wait for the ids or the logits ran out
 };
 
 struct TokenArgs {
@@ -119,15 +119,17 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         static_assert(kTokensWorkBytes >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
         int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
         float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
+        bool there = true;
         if (a.preselected) {  // (the one row is the shared gate's)
             if (wave == 5) {
                 float none[1];
-                (void)hand_gather<1, true>(HandRow{s.hand, 0, a.E, true}, lane, none);
+                there = hand_gather<1, true>(HandRow{s.hand, 0, a.E, true, a.spin_limit}, lane, none);
             }
         } else {
-            (void)topk_block<true>(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, s_last, lane, wave, nullptr,
-                                   ta.wait_ids ? s.tagged : nullptr, kTagCopies);
+            there = topk_block<true>(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, s_last, lane, wave, nullptr,
+                                     ta.wait_ids ? s.tagged : nullptr, kTagCopies) != 3;
         }
+        if (!there && lane == 0) __hip_atomic_store(s.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(s.hand + a.E)));
         if (!a.preselected && wave == 0) {
             wave_lds_fence();
