@@ -183,6 +183,38 @@ def test_tokens_on_a_table_of_expert_views(g, oracle, shape):
         s.close()
 
 
+def test_a_refused_table_of_expert_views_runs_nothing(g, oracle):
+    """Down rows of more than 48 blocks have no dispatch for a pointer table: the call is refused before anything is launched (the
+    scratches' activations stay as they are), and a preselected and a routed batch on the same scratches are the oracle's."""
+    H, F, E, k, T = 512, 1568, 16, 4, 3
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=36, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, 2 * T, 12)
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    arr = (C.c_void_p * T)(*[s.h for s in scr])
+    ids, wts = np.arange(k, dtype=np.int32), np.full(k, 0.25, np.float32)
+    for s in scr:
+        capi.call("wd_memcpy_h2d", C.c_void_p(s.raw("ids")), ids.ctypes.data_as(C.c_void_p), 4 * k, None)
+        capi.call("wd_memcpy_h2d", C.c_void_p(s.raw("weights")), wts.ctypes.data_as(C.c_void_p), 4 * k, None)
+    d, P, lib = dl.desc, C.c_void_p * E, capi.load()
+    table = [P(*[base + e * stride for e in range(E)]) for base, stride in ((d.gate, d.gate_stride), (d.up, d.up_stride), (d.down, d.down_stride))]
+    dx, out = g.dev(xs), g.empty((T, H), np.float32)
+    for flags in (capi.MOE_PRESELECTED, 0):
+        before = [s.get("act", (k + 1) * F, np.float32) for s in scr]
+        rc = lib.wd_moe_layer_tokens_pairs_f32(C.byref(d), *table, E, C.c_void_p(dx.data_ptr() + 4 * H * T), g.ptr(out), T, arr, capi.MOE_PRESELECTED, g.stream())
+        assert rc == -1 and "no multi-token dispatch" in lib.wd_last_error().decode()
+        g.sync()
+        for s, a in zip(scr, before):
+            assert g.same_bits(s.get("act", (k + 1) * F, np.float32), a)
+        capi.call("wd_moe_layer_tokens_f32", C.byref(d), g.ptr(dx), g.ptr(out), T, arr, flags, g.stream())
+        g.sync()
+        for t in range(T):
+            want = oracle.moe_layer(L, xs[t], ids=ids, weights=wts)[0] if flags else oracle.moe_layer(L, xs[t])[0]
+            assert g.same_bits(g.host(out)[t], want), (flags, t)
+    assert [lib.wd_moe_scratch_status(s.h) for s in scr] == [0] * T
+    for s in scr:
+        s.close()
+
+
 @pytest.mark.parametrize("gate,F", [(synth.IQ3_S, 64), (synth.Q8_0, 64), (synth.IQ2_S, 1568)])
 def test_bounded_wait_of_a_token_batch(g, oracle, gate, F):
     """With a wait limit of one poll the routed workgroups give up before the ids are published: every token's status word and

@@ -1077,6 +1077,8 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
                             !(flags & (WD_MOE_ONLY_A | WD_MOE_ONLY_B | WD_MOE_ONLY_C | WD_MOE_DRY));
     const bool down_tokens = F <= 1536;
     if (gu_table) WD_REQUIRE(union_path && iq, "multi-token pass on a pointer table: IQ3_S / IQ2_S gate and up tensors, at most 128 (token, expert) pairs, no staging flags");
+    // (before anything is launched: what the dispatches hand on is set back by a dispatch C)
+    WD_REQUIRE(!down_table || down_tokens, "multi-token pass on a pointer table: this down tensor (type %d, %d columns) has no multi-token dispatch", L->down_type, F);
     if (!union_path) {
         // same results, one pass per token (every pass reads its own experts)
         for (int t = 0; t < tokens; ++t)
@@ -1139,7 +1141,6 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         }
         SiteScope c_site(WD_SITE_TOKENS_C, st);
         if (!down_tokens) {
-            WD_REQUIRE(!down_table, "multi-token pass on a pointer table: this down tensor (type %d, %d columns) has no multi-token dispatch", L->down_type, F);
             for (int t = 0; t < tokens; ++t)
                 if (const int rc = layer_fused(L, d_x + static_cast<size_t>(t) * H, d_out + static_cast<size_t>(t) * H, scratch_per_token[t],
                                                flags | WD_MOE_ONLY_C, nullptr, nullptr, 0.0f, st))
