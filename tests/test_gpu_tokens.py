@@ -183,6 +183,19 @@ def test_tokens_on_a_table_of_expert_views(g, oracle, shape):
         s.close()
 
 
+@pytest.mark.parametrize("H,T", [(17920, 8), (24064, 6), (35840, 1)])
+def test_the_longest_rows_of_a_token_batch(g, oracle, H, T):
+    """Rows whose inputs fill the LDS: T of them in Q8_K beside the codebooks and the union (162128 of 163840 bytes at 17920 and eight
+    tokens), or one in f32 beside the selection's work area."""
+    F, E, k = 32, 8, 2
+    L = synth.make_layer(H, F, E, k, synth.IQ2_S, synth.Q8_0, True, seed=SEED, layer=37, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, T, 13)
+    dl = g.DeviceLayer(L)
+    r = run_tokens(g, dl, L, xs)
+    for t in range(T):
+        assert g.same_bits(r["out"][t], oracle.moe_layer(L, xs[t])[0]), t
+
+
 def test_a_refused_table_of_expert_views_runs_nothing(g, oracle):
     """Down rows of more than 48 blocks have no dispatch for a pointer table: the call is refused before anything is launched (the
     scratches' activations stay as they are), and a preselected and a routed batch on the same scratches are the oracle's."""

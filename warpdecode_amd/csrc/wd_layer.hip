@@ -995,7 +995,7 @@ void launch_tokens_ab_fetch(const TokenArgs &ta, bool routed, int items, int cus
     const int H = ta.common.H;
     size_t lds = static_cast<size_t>(ta.T) * (H + sizeof(float) * (H / 256));
     if (FETCH != 0) lds = ((lds + 15) & ~static_cast<size_t>(15)) + 8 * 2 * static_cast<size_t>(iq_cover_bytes<TYPE>(H / 256));
-    lds = std::max(lds, sizeof(float) * static_cast<size_t>(H) + 16);
+    lds = tokens_ab_lds(H, lds);
     // persistent: as many workgroups as a compute unit holds walk the items
     auto grid = [&](int per_cu) { return dim3(ta.front_wgs + (routed ? std::min(items, per_cu * cus) : 0)); };
     if (ta.T <= 4) enqueue(k_tokens_ab<TYPE, 4, FETCH>, grid(kTokensBPerCu<TYPE, 4, FETCH>), dim3(512), lds, st, ta);

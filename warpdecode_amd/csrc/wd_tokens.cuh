@@ -71,7 +71,8 @@ struct TokenArgs {
 // rows to the tokens after the first.  The padding workgroups return at once.  Per token this is the front of the
 // one-token merged dispatch: router rows one per wave, the last router workgroup of the token selects its experts
 // with the whole workgroup and publishes the ids, the other workgroups run the shared expert's gate/up.
-// lds: 4 * H + 16 bytes (x as f32 for the router rows; the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes.
+// lds: 4 * H + 16 bytes, x as f32 for the router rows (the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes of the
+// routed part's tables, for the selection; tiles: the shared rows' eight.
 struct TokensAGrid {
     int router_stride, shared_stride;
     __host__ __device__ int total(int tokens) const { return tokens * (router_stride + shared_stride); }
@@ -79,11 +80,11 @@ struct TokensAGrid {
 __host__ __device__ inline TokensAGrid tokens_a_grid(int n_router_wgs, int n_shared_wgs) {
     return TokensAGrid{(n_router_wgs + 7) & ~7, (n_shared_wgs + 7) & ~7};
 }
-constexpr int kTokensWorkBytes = sizeof(Q8RowTile) * 8;
+constexpr int kTokensWorkBytes = kTopkLdsBytes2 + 128;
 // WIDE: router rows of 2049..4096 columns, two waves each (n_router_wgs is then for four rows per workgroup).
 // HIDDEN: the layer's, where it is known (0: it is not): its row loops then need no bounds, which spill 18 registers.
 template <bool WIDE, int HIDDEN>
-WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, int &s_last) {
+WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, Q8RowTile *tiles, int &s_last) {
     const LayerArgs &a = ta.common;
     const int H = HIDDEN ? HIDDEN : a.H;
     const int n_shared_wgs = a.sh_inp ? (a.F + 7) / 8 : 0;
@@ -116,7 +117,6 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         if (threadIdx.x == 0) s_last = hand_count_last(s.hand, a.E, a.n_router_wgs);
         __syncthreads();
         if (!s_last) return;
-        static_assert(kTokensWorkBytes >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
         int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
         float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
         bool there = true;
@@ -142,7 +142,6 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
     }
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ta);
     uint16_t *xd = reinterpret_cast<uint16_t *>(lds_ta + H);
-    Q8RowTile *tiles = reinterpret_cast<Q8RowTile *>(s_work);
     const int r = (wg - a.n_router_wgs) * 8 + wave;
     const int nb = H >> 5;
     const size_t rb = static_cast<size_t>(nb) * 34;
@@ -279,12 +278,19 @@ WD_DEV void token_union_build(const TokenArgs &ta, TokenUnion &un, int lane) {
 // turn with the stride of their number; a wave takes one (gate, up) row pair of the item, decodes it once and applies it to every
 // token that selected the expert.  As a dispatch of its own this part began 2.6 us after the ids and spent 3.5 more on its set-up.
 // MAXT: token capacity of the instantiation (4 or kMaxTokens).
-// dynamic LDS: T * (H bytes + H/256 floats), the Q8_K copies of the T inputs, and 4 * H + 16 bytes at least (tokens_front).
+// dynamic LDS: T * (H bytes + H/256 floats), the Q8_K copies of the T inputs; at least what tokens_front takes (tokens_ab_lds).
 // FETCH: 0, or how the rows come in when they can be fetched as aligned words (IqRowWords): 8 and 10 rows of that many
 // super-blocks, 1 and 2 others of one or two words per lane.  The row pair of the wave's next item is then requested before the
 // current one is worked on.  dynamic LDS then has 8 * 2 * iq_cover_bytes more bytes behind the activations (16-byte aligned).
 // As many workgroups per compute unit as the registers allow without spilling in the routed part (eight tokens and rows of eight
 // super-blocks spill eleven in all: 73.1 us per layer, 75.7 as two dispatches of which one spilled two).
+// The shared rows' tiles of the first part lie behind the quantised x of the same workgroup: in the static area they would make it 2.9 KB larger
+// than the tables and the union, which is what the inputs of eight tokens of 17920 columns leave (162128 of 163840 bytes).
+__host__ __device__ inline uint32_t tokens_front_tiles(int H) { return static_cast<uint32_t>(H + H / 16 + 15) & ~15u; }
+// activations: the T inputs, and the staging behind them.
+inline size_t tokens_ab_lds(int H, size_t activations) {
+    return std::max({activations, sizeof(float) * static_cast<size_t>(H) + 16, tokens_front_tiles(H) + 8 * sizeof(Q8RowTile)});
+}
 template <int TYPE, int MAXT, int FETCH>
 constexpr int kTokensBPerCu = FETCH == 8 || (FETCH == 10 && TYPE == 22 && MAXT <= 4) ? 3 : 2;
 template <int TYPE, int MAXT, int FETCH = 0>
@@ -294,13 +300,15 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
         IqTables tables;
         TokenUnion un;
     };
-    __shared__ __align__(16) uint8_t s_area[sizeof(Routed) > kTokensWorkBytes ? sizeof(Routed) : kTokensWorkBytes];
+    static_assert(sizeof(Routed) >= kTokensWorkBytes, "the selection works in the place of the tables and the union");
+    __shared__ __align__(16) uint8_t s_area[sizeof(Routed)];
     __shared__ int s_last;
     const LayerArgs &a = ta.common;
     if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
         const bool wide = a.H > 2048 && a.H <= 4096;
-        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, FETCH == 10 ? 2560 : 0>(ta, lds_tb, s_area, s_last);
-        else tokens_front<false, FETCH == 8 ? 2048 : 0>(ta, lds_tb, s_area, s_last);
+        Q8RowTile *const tiles = reinterpret_cast<Q8RowTile *>(lds_tb + tokens_front_tiles(a.H));
+        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, FETCH == 10 ? 2560 : 0>(ta, lds_tb, s_area, tiles, s_last);
+        else tokens_front<false, FETCH == 8 ? 2048 : 0>(ta, lds_tb, s_area, tiles, s_last);
         return;
     }
     IqTables &tables = reinterpret_cast<Routed *>(s_area)->tables;
@@ -526,12 +534,14 @@ __global__ __launch_bounds__(512, 4) void k_tokens_ab_q8(TokenArgs ta) {
         Q8Tile8 tiles[8];
         TokenUnion un;
     };
-    __shared__ __align__(16) uint8_t s_area[sizeof(Routed) > kTokensWorkBytes ? sizeof(Routed) : kTokensWorkBytes];
+    static_assert(sizeof(Routed) >= kTokensWorkBytes && sizeof(Routed) >= 8 * sizeof(Q8RowTile), "the first part works in the place of the tiles and the union");
+    __shared__ __align__(16) uint8_t s_area[sizeof(Routed)];
     __shared__ int s_last;
     const LayerArgs &a = ta.common;
     if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
-        if (a.H > 2048) tokens_front<true, 0>(ta, lds_tq, s_area, s_last);  // (hidden 4096 at most)
-        else tokens_front<false, 0>(ta, lds_tq, s_area, s_last);
+        Q8RowTile *const tiles = reinterpret_cast<Q8RowTile *>(s_area);
+        if (a.H > 2048) tokens_front<true, 0>(ta, lds_tq, s_area, tiles, s_last);  // (hidden 4096 at most)
+        else tokens_front<false, 0>(ta, lds_tq, s_area, tiles, s_last);
         return;
     }
     Q8Tile8 *const tiles = reinterpret_cast<Routed *>(s_area)->tiles;
