@@ -334,3 +334,48 @@ def test_passes_that_end_before_the_down_projections(g, oracle, shape):
     assert [capi.load().wd_moe_scratch_status(s.h) for s in scr] == [0] * T
     for s in scr:
         s.close()
+
+
+@pytest.mark.parametrize("E,k", [(64, 6), (640, 10)])
+def test_logits_of_the_reserved_nan(g, E, k):
+    """A router row, then the shared expert's gate row, whose logit is the NaN that stands for "not handed on yet": one-token layers and
+    token batches end with the status word clear and with what any other NaN there gives.  (A NaN among the logits leaves k times the
+    same id with infinite weights, so only the selection and the staged dispatches' results, which hand nothing on, are compared.)"""
+    H, F, T = 512, 64, 3
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=38, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, T, 14)
+    clean = run_tokens(g, g.DeviceLayer(L), L, xs)
+    late = int(clean["ids"][0][k - 1])
+    lib = capi.load()
+    for name, row in (("router", late), ("router", E - 1), ("shared_gate_inp", 0)):
+        seen = []
+        for bits in (0xffffffff, 0x7fc00000):
+            bad = dict(L)
+            bad[name] = np.array(L[name], np.float32)
+            bad[name].reshape(-1, H)[row, 5] = np.array([bits], np.uint32).view(np.float32)[0]
+            dl, scr = g.DeviceLayer(bad), [g.Scratch(H, F, E, k) for _ in range(T)]
+            arr = (C.c_void_p * T)(*[s.h for s in scr])
+            dx = g.dev(xs)
+            for how in ("batch", "batch in two", "layer", "staged"):
+                out = g.empty((T, H), np.float32)
+                if how.startswith("batch"):
+                    capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, arr, 0 if how == "batch" else capi.MOE_SPLIT_AB, g.stream())
+                else:
+                    for t, s in enumerate(scr):
+                        capi.call("wd_moe_layer_f32", C.byref(dl.desc), C.c_void_p(dx.data_ptr() + 4 * H * t), C.c_void_p(out.data_ptr() + 4 * H * t), s.h,
+                                  capi.MOE_STAGED if how == "staged" else 0, g.stream())
+                g.sync()
+                assert [lib.wd_moe_scratch_status(s.h) for s in scr] == [0] * T, (name, row, how)
+                if name == "router":  # (the logits as the caller sees them: the word is the reserved one)
+                    assert [int(s.get("logits", E, np.float32).view(np.uint32)[row]) for s in scr] == [bits] * T, how
+                ids, weights, accum = (np.stack([s.get(n, w, d) for s in scr]) for n, w, d in (("ids", k, np.int32), ("weights", k, np.float32), ("accum", H, np.float32)))
+                seen.append((how, ids, weights, accum, g.host(out)))
+            for s in scr:
+                s.close()
+        _, ids, *staged = seen[-1]
+        for how, ids_h, *values in seen:
+            assert np.array_equal(ids_h, ids), (name, row, how)
+            for a, b in list(zip(values, staged))[:1 if how.startswith("batch") and name == "router" else 3]:
+                assert np.array_equal(np.isnan(a), np.isnan(b)) and g.same_bits(a[~np.isnan(a)], b[~np.isnan(b)]), (name, row, how)
+            if name == "shared_gate_inp":
+                assert np.array_equal(ids_h, clean["ids"]) and g.same_bits(values[1], clean["accum"]) and np.isnan(values[2]).all(), how
