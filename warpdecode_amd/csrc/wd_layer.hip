@@ -630,7 +630,7 @@ void launch_layer_c_even(hipStream_t st, const LayerArgs &a) {
     if (R <= 4) launch_layer_c_even<KIND, 16, 1>(st, a);
     else if (R == 5) launch_layer_c_even<KIND, 12, 1>(st, a);
     else if (R == 6) launch_layer_c_even<KIND, 10, 1>(st, a);
-    else if (R <= 10) launch_layer_c_even<KIND, 12, 2>(st, a);
+    else if (R <= 10) launch_layer_c_even<KIND, 12, 2>(st, a);  // (9 and 10: layer_c_evenly takes neither 7 nor 8)
     else if (R <= 12) launch_layer_c_even<KIND, 10, 2>(st, a);
     else if (R <= 14) launch_layer_c_even<KIND, 9, 2>(st, a);
     else launch_layer_c_even<KIND, 8, 2>(st, a);
@@ -1015,7 +1015,7 @@ void launch_tokens_ab(const wd_moe_layer *L, const TokenArgs &ta, bool routed, i
     else if (H <= 2304) launch_tokens_ab_fetch<TYPE, 1>(ta, routed, items, cus, st);
     else launch_tokens_ab_fetch<TYPE, 2>(ta, routed, items, cus, st);
 }
-template <int KIND, int LPR, int PASSES = 1>
+template <int KIND, int LPR, int PASSES = (LPR == 16 ? 1 : 2)>  // (tokens_c_even_lanes: more than 16 blocks for the others)
 void launch_tokens_c_even(const TokenArgs &ta, hipStream_t st) {
     if constexpr (PASSES * LPR < 48) {  // (as in launch_layer_c_even)
         if (ta.common.F > 32 * PASSES * LPR) return launch_tokens_c_even<KIND, LPR, (PASSES < 4 ? PASSES + 1 : 6)>(ta, st);
