@@ -1016,8 +1016,8 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (a.dry) return;
     const int groups = (a.F + 7) / 8;
-    // (known where the fetch is made for it: the router's row loops then need no bounds.  us per layer from HBM: 2048 / 512, 256 experts 19.4
-    // / 18.4, 2048 / 768 21.4 / 20.4, 2560 / 640 25.9 / 25.2)
+    // (known where the fetch is made for it: 56 registers instead of 80 at 2048 without the loop, 73 and none spilled with it.  us per layer from
+    // HBM, unknown / known: 2048 / 512 19.61 / 19.48, 2048 / 768 20.20 / 20.14, IQ2_S 19.05 / 18.97, 2560 / 640 24.72 / 24.61, IQ2_S 23.16 / 23.20)
     const int H = FETCH == 8 ? 2048 : (FETCH == 10 ? 2560 : a.H);
 
     mark<TRACE>(a, wg < a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);

@@ -82,7 +82,8 @@ __host__ __device__ inline TokensAGrid tokens_a_grid(int n_router_wgs, int n_sha
 }
 constexpr int kTokensWorkBytes = kTopkLdsBytes2 + 128;
 // WIDE: router rows of 2049..4096 columns, two waves each (n_router_wgs is then for four rows per workgroup).
-// HIDDEN: the layer's, where it is known (0: it is not): its row loops then need no bounds, which spill 18 registers.
+// HIDDEN: 2048, where it is known (0: it is not).  With it the dispatch for five and more tokens spills 11 registers instead of 18; us per layer,
+// unknown / known: two tokens 28.3 / 28.3, four 41.1 / 40.3, eight 69.5 / 67.9.  (2560 known: nothing, 55.0 / 55.0 and 84.6 / 84.5.)
 template <bool WIDE, int HIDDEN>
 WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, Q8RowTile *tiles, int &s_last) {
     const LayerArgs &a = ta.common;
@@ -307,7 +308,7 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
     if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
         const bool wide = a.H > 2048 && a.H <= 4096;
         Q8RowTile *const tiles = reinterpret_cast<Q8RowTile *>(lds_tb + tokens_front_tiles(a.H));
-        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, FETCH == 10 ? 2560 : 0>(ta, lds_tb, s_area, tiles, s_last);
+        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, 0>(ta, lds_tb, s_area, tiles, s_last);
         else tokens_front<false, FETCH == 8 ? 2048 : 0>(ta, lds_tb, s_area, tiles, s_last);
         return;
     }
