@@ -1,4 +1,5 @@
-// The bits a 32-bit value travels with between the workgroups of a resident launch (wd_resident.cuh).  A hand-off word
+// The bits a 32-bit value travels with between the workgroups of a resident launch (wd_resident.cuh), and a router logit between those of
+// dispatch AB and of the token batches' (wd_fused.cuh, wd_tokens.cuh).  A hand-off word
 // that still holds kHandEmpty has not been written; consumers poll the data words themselves.  kHandEmpty is also the
 // bit pattern of one particular NaN, which a producer may legitimately compute: it is handed on as the default quiet NaN
 // instead, so that its consumer does not wait for it for ever.  Plain C++: the host tests include this file too.

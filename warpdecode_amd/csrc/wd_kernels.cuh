@@ -703,8 +703,8 @@ __global__ __launch_bounds__(WPB * 64) void k_gemv_q4_stream(const uint8_t *__re
 }
 // Several matrices of one row length in one launch (see k_gemv_q8_rows8_split_batch): workgroup b belongs to the item
 // whose range of workgroups holds b and does there what k_gemv_q4_stream does for that item alone.
-// The table travels with the launch, whose host time grows with it (40 bytes 2.75 us, 480 bytes 3.5): one for few items (184
-// bytes) beside one for many (648).
+// The table travels with the launch, whose host time grows with it (184 bytes 2.2 to 2.3 us, 648 2.35 to 2.4; 2.7 and 3.0 to 3.4 in
+// another process): one for few items (184 bytes) beside one for many (648).
 constexpr int kGemvBatchMax = 16, kGemvBatchFew = 4;
 template <int MAX>
 struct GemvBatch {

@@ -39,7 +39,8 @@ int wait_report(const volatile uint32_t *rec, int k, hipStream_t st) {
 // the cache's books behind that (an acquire of hits has no work for the device): the device does not wait for the host.  Where an
 // expert is missing, the host acquires and launches the layer's gate/up once more, on the selection that is in the scratch, ahead
 // of C.  (Router and selection as a dispatch of their own, the copied ids and the synchronisation left the device idle for half of
-// every layer: 2048 / 512, 128 experts, eight layers, nearly all hits: 297 us, so 176; three layers of 1792 / 224, all hits, 95 / 55.)
+// every layer: 2048 / 512, 128 experts, eight layers, all hits: 293 us, so 158; with 4.8 misses a token 592 / 501, with 23 1398 / 1300, with 55
+// 2570 / 2506; three layers of 1792 / 224, all hits, 96 / 55.)
 int cached_routed_reported(const std::vector<wd_moe_layer> &bound, wd_expert_cache *cache, float *d_x, float *d_layer_out, wd_moe_scratch *s,
                            float residual_scale, unsigned flags, hipStream_t st) {
     if (cache->fills_pending)
