@@ -77,7 +77,7 @@ def parse():
                     help="lru mode: tokens run before the warm-up steps so that the slot pool is in steady state")
     ap.add_argument("--cache-timing", action="store_true",
                     help="lru mode: switch on the cache's device-side timings (the copy stream's waits and fills, in the monitor "
-                         "object); the events they need cost about 4 % of the rate")
+                         "object); the events they need cost about 4 %% of the rate")
     ap.add_argument("--graph", choices=["auto", "on", "off"], default="auto",
                     help="replay the step from a captured HIP graph or launch it eagerly; auto: eagerly when the step is one "
                          "launch (the resident stack: a graph of one kernel costs more than the launch it saves), a graph for "
