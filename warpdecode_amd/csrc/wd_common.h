@@ -36,7 +36,7 @@ int noalloc_setup_current_device();
 
 // A kernel launch through the runtime's own entry point.  The <<<>>> form goes through a stub that parks the launch shape in
 // the runtime and takes it out again: 2.35 to 2.43 us of host time for a launch, 2.22 to 2.28 so (an argument block of 40 bytes, a
-// C++ loop; another process of the same box 2.79 to 2.84, 2.67 to 2.72).  An error is left for WD_LAUNCH_CHECK, as by <<<>>>.
+// C++ loop; another process of the same machine 2.79 to 2.84, 2.67 to 2.72).  An error is left for WD_LAUNCH_CHECK, as by <<<>>>.
 template <typename T>
 struct SameType {
     using type = T;
