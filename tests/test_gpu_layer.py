@@ -376,6 +376,31 @@ def test_bounded_wait_gives_up_and_recovers(g, oracle):
     sc.close()
 
 
+@pytest.mark.parametrize("E,k", [(8, 1), (64, 6), (512, 10), (640, 10), (512, 16)])
+def test_late_logits_are_reported(g, oracle, E, k):
+    """The selecting workgroup starts before the router's and polls their words: with a wait limit of one poll it may give up (the parts
+    are launched apart, so nobody else waits), and then says so in the status word and in the data; with the default limit it is the oracle's."""
+    H, F = 512, 64
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=980, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 70, E), H)
+    want, d = oracle.moe_layer(L, x)
+    dl, sc = g.DeviceLayer(L), g.Scratch(H, F, E, k)
+    dx, out = g.dev(x), g.empty(H, np.float32)
+    for limit in (1, 1, 1, 0, 0):
+        capi.call("wd_moe_scratch_set_wait_limit", sc.h, limit)
+        out.zero_()
+        capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, capi.MOE_SPLIT_AB, g.stream())
+        g.sync()
+        late = capi.load().wd_moe_scratch_status(sc.h)
+        assert late in ((0, 1) if limit else (0,))
+        if late:
+            assert np.isnan(g.host(out)).all()
+        else:
+            assert np.array_equal(sc.get("ids", k, np.int32), d["ids"]) and g.same_bits(sc.get("weights", k, np.float32), d["weights"])
+            assert g.same_bits(g.host(out), want)
+    sc.close()
+
+
 def test_fused_gate_up_tensor_layout(g, oracle):
     """One tensor with 2 * ffn rows per expert (gate rows, then up rows), as the reference's target model stores
     them (src/qwen38_moe.cuh:3462-3514): the layer descriptor addresses it in place, resident and through the

@@ -1,6 +1,6 @@
 // Fused MoE layer: two dispatches per layer (three when the caller asks for the split form).
-//   AB router logits (+ shared-expert gate logit), a wave or two per row; the router workgroup that finishes last
-//      runs softmax/top-k and publishes the ids inside the dispatch; the shared expert's gate/up + SwiGLU and
+//   AB router logits (+ shared-expert gate logit), a wave or two per row; the dispatch's first workgroup waits for
+//      them, runs softmax/top-k and publishes the ids inside the dispatch; the shared expert's gate/up + SwiGLU and
 //      the routed gate/up + SwiGLU run in the same launch: the routed workgroups quantise x and stage the
 //      codebooks while the router runs and pick the ids up as soon as they appear - or request their weights at
 //      once when the ids are known before the launch (given by the caller, or by a routing trace).
@@ -39,11 +39,12 @@ struct LayerArgs {
     int hc, hc_round_half;
     int dry;                     // measurement aid: every workgroup returns at once
     int preselected;
-    int n_router_wgs;            // workgroups of dispatch AB that take router rows,
+    int n_select_wgs;            // workgroups of dispatch AB that select: one, or none,
+    int n_router_wgs;            // those that take router rows,
     int n_shared_wgs;            // those that take the shared expert's gate/up (the rest: routed gate/up)
     int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
     const int32_t *ids_known;    // null, or the k ids where they are known before the launch
-    uint32_t *hand;              // [E + 3]: the router's logits and the shared gate's on their way to the selection, a ticket or count, and the count of hand_close; kHandEmpty between passes
+    uint32_t *hand;              // [E + 2]: the router's logits and the shared gate's on their way to the selection, and the count of hand_close; kHandEmpty between passes
     uint32_t *ids_tagged;        // [kTagCopies][16] selected ids published inside the merged dispatch (kTagInvalid = not yet)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
     int close_hand;              // no dispatch C follows: the router workgroups set `hand` back themselves
@@ -666,16 +667,14 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
 }
 
 // ---- selection inside the dispatch that computes the logits ------------------------------------------------------------
-// Every router workgroup hands its logits on as words that cannot be kHandEmpty (hand[e], the shared expert's gate logit in
-// hand[n_slot]); dispatch C sets the words back.  Which workgroup selects:
-//   one token (COUNT false): every workgroup waits until its words are acknowledged and looks at all of the row's.  Of those that end last
-//     at least one finds every word there.  If several do, all of them select, and the one that draws the ticket (hand[n_slot + 1])
-//     first publishes; the draw is under way while it selects.
-//   token batches (COUNT true): the workgroups count themselves in hand[n_slot + 1], without waiting for any acknowledgement, and the last
-//     one polls the words until all are there.  Surplus selections would hold up the routed workgroups that wait for a place.
-// (Counted behind the acknowledgement and the logits requested by the last one then, a round trip more, us per layer from HBM: 2048 / 512
-// 21.2, with tickets 20.0, counted 20.4; 2560 / 640 24.5, 23.7, 24.8; layer_small's 1024 / 256 12.1, 11.7, 12.0; eight tokens of 2048 / 512
-// 73.1, 75.9, 71.4; six of 1024 / 352 33.3, 31.4, 30.9.)
+// Every router wave hands its logit on as a word that cannot be kHandEmpty (hand[e], the shared expert's gate logit in
+// hand[n_slot]); dispatch C sets the words back.  A workgroup of its own, the dispatch's first, selects: it polls the words until all are
+// there.  No router workgroup waits for its own word, counts itself or looks at the row, and the selection runs where nothing else did
+// before it (its code is in that compute unit's instruction cache from one launch to the next).
+// (Selected by the router workgroups that end last - each waits until its words are acknowledged and looks at the row, a ticket names the
+// one to publish - the ids of 2048 / 512 are out 7.2 us after the dispatch's start, by the first workgroup 5.9; 64 experts of 1024 / 256 5.1, 4.4.
+// us per layer: 2560 / 640 24.6, so 24.4; 2048 / 512 20.5, 19.9; 1024 / 256 12.0, 11.9.  Four tokens of 2048 / 512, whose router workgroups
+// counted themselves and the last one polled, 40.0, 39.5.)
 struct HandRow {
     uint32_t *hand;
     int n, n_slot;
@@ -683,26 +682,23 @@ struct HandRow {
     unsigned limit;  // polls before one that waits for the row gives up
 };
 WD_DEV uint32_t hand_load(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-WD_DEV uint32_t hand_draw(uint32_t *hand, int n_slot) { return __hip_atomic_fetch_add(hand + n_slot + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// One thread: whether its workgroup is the last of n_wgs.
-WD_DEV bool hand_count_last(uint32_t *hand, int n_slot, int n_wgs) { return hand_draw(hand, n_slot) + 1u == static_cast<uint32_t>(n_wgs - 1); }
-// Sets the words back where no dispatch C does: the router workgroup that is done last, behind every other one's last use of them.  Every
-// thread of each of the n_wgs must call it.  (A fill launched behind the dispatch instead, us per layer with the ids through the host: 2048 / 512
+// Sets the words back where no dispatch C does: the one of the router workgroups and the selecting one that is done last, behind every other
+// one's last use of them.  Every thread of each of the n_wgs must call it.  (A fill launched behind the dispatch instead, us per layer with the ids through the host: 2048 / 512
 // 46.2, so 45.0; 1024 / 256 37.9, 36.9; 4096 / 1536 66.5, 65.5.)
 WD_DEV void hand_close(uint32_t *hand, int n_slot, int n_wgs, int &last) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);  // what this wave has asked for of the words is there
     __syncthreads();
-    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(hand + n_slot + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == static_cast<uint32_t>(n_wgs - 1);
+    if (threadIdx.x == 0) last = __hip_atomic_fetch_add(hand + n_slot + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == static_cast<uint32_t>(n_wgs - 1);
     __syncthreads();
     if (!last) return;
-    for (int i = threadIdx.x; i < n_slot + 3; i += static_cast<int>(blockDim.x)) __hip_atomic_store(hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = threadIdx.x; i < n_slot + 2; i += static_cast<int>(blockDim.x)) __hip_atomic_store(hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// lv[j]: logit 64 j + lane; whether the row is complete.  POLL: once it is (it must be about to; the limit is there for a broken device: words
-// that did not come are NaN, what is selected then are experts of the layer, and the status makes the results NaN).
-template <int M, bool POLL>
+// lv[j]: logit 64 j + lane, once the row is complete (the limit is there for a broken device: words that did not come are NaN, what is
+// selected then are experts of the layer, and the status makes the results NaN).  Returns whether it was.
+template <int M>
 WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
-    for (unsigned polls = 0; polls < (POLL ? r.limit : 1u); ++polls) {
+    for (unsigned polls = 0; polls < r.limit; ++polls) {
         const uint32_t g = r.gate ? hand_load(r.hand + r.n_slot) : 0u;
         bool there = hand_arrived(g);
 #pragma unroll
@@ -715,40 +711,30 @@ WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
     return false;
 }
 
-// The selections below return 0: some words are not there; 1: selected, but not the one to publish; 2: the one (wave 0; other waves: 1); 3, in the
-// wave that saw it: a poll for the row ran out (the caller sets the status).
+// The selections below return whether the row's words came (a wave that does not wait for them: true; the caller sets the status otherwise).
 // n <= 64 M logits, k <= 15: wave 0 ranks and publishes the ids, wave 1 takes the exponentials and the denominator meanwhile, and wave 0 forms
-// the weights behind one barrier.  Every thread of the workgroup must call it.  ids, weights, state: LDS.
-template <int M, bool COUNT>
-WD_DEV int topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
-                          uint8_t *lds, int &state, int lane, int wave, unsigned long long *stamps, uint32_t *tagged, int copies) {
+// the weights behind one barrier.  Every thread of the workgroup must call it.  ids, weights: LDS.
+template <int M>
+WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
+                           uint8_t *lds, int lane, int wave, unsigned long long *stamps, uint32_t *tagged, int copies) {
 #define WD_STAMP(i) do { if (stamps && wave == 0 && lane == 0) stamps[i] = wall_clock64(); } while (0)
     const TopkLds<1> s(lds);
     const int n = row.n;
     SelWaveState st;
     int id_given = 0;
-    bool there = false, won = COUNT;
+    bool there = true;
     float lv[M];
     if (wave <= 1) {
         if (override_ids && wave == 0 && lane < k) id_given = override_ids[lane];
-        there = hand_gather<M, COUNT>(row, lane, lv);
-        if (!COUNT && wave == 0 && lane == 0) state = there ? 1 : 0;
-    }
-    if (!COUNT) {
-        __syncthreads();
-        if (!state) return 0;
+        there = hand_gather<M>(row, lane, lv);
     }
     WD_STAMP(0);
     if (wave == 0) {
-        uint32_t ticket = 0u;
-        if (!COUNT && lane == 0) ticket = hand_draw(row.hand, row.n_slot);
         sel_wave_ids(lv, n, k, s, lane, st);
         WD_STAMP(3);
-        if (!COUNT) won = __builtin_amdgcn_readfirstlane(ticket) == kHandEmpty;
-        if (won && st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        if (st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
         WD_STAMP(6);
     } else if (wave == 1) {
-        if (!COUNT && !there) there = hand_gather<M, true>(row, lane, lv);  // (wave 0 has seen them all)
         bool dead;
         const float inv = sel_wave_denominator(lv, n, s, lane, dead);
         if (lane == 0) s.rest[0] = inv, s.rest[1] = dead ? 1.0f : 0.0f;
@@ -757,38 +743,30 @@ WD_DEV int topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids
     if (wave == 0) {
         const bool fast = st.fast;
         sel_wave_weights(n, k, w_scale, s, lane, st, s.rest[0], s.rest[1] != 0.0f, ids, weights, override_ids != nullptr, id_given);
-        if (won && !fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        if (!fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
         WD_STAMP(7);
     }
 #undef WD_STAMP
-    return wave <= 1 && !there ? 3 : (won ? 2 : 1);
+    return there;
 }
 
-// Every thread of the workgroup must call it (COUNT: of the one that counted last).  Two waves select where one can hold the row
-// (n <= 512, k <= 15); ids and weights are left in LDS by wave 0.
+// Every thread of the workgroup must call it.  Two waves select where one can hold the row (n <= 512, k <= 15); ids and weights are left in
+// LDS by wave 0.
 // (64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
 // there are experts to select its threshold excludes nobody -; 512 experts, top-10: 2.1, 2.2.)
-template <bool COUNT>
-WD_DEV int topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
-                      uint8_t *lds, int &state, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
+WD_DEV bool topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
+                       uint8_t *lds, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
     const int n = row.n;
     if (n <= 512 && k <= 15) {
-        if (n <= 64) return topk_two_waves<1, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
-        if (n <= 128) return topk_two_waves<2, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
-        if (n <= 256) return topk_two_waves<4, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
-        return topk_two_waves<8, COUNT>(row, k, w_scale, ids, weights, override_ids, lds, state, lane, wave, stamps, tagged, copies);
+        if (n <= 64) return topk_two_waves<1>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        if (n <= 128) return topk_two_waves<2>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        if (n <= 256) return topk_two_waves<4>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        return topk_two_waves<8>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
     }
-    __syncthreads();  // (COUNT: state may be the word the count was read from)
-    bool there = true;
-    if (wave == 0) {
-        float lv[16];
-        there = hand_gather<16, COUNT>(row, lane, lv);
-        if (lane == 0) state = COUNT ? 2 : (!there ? 0 : (hand_draw(row.hand, row.n_slot) == kHandEmpty ? 2 : 1));
-    }
-    __syncthreads();
-    const int got = state;
-    if (got) topk_block_m<2>(reinterpret_cast<const float *>(row.hand), n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, got == 2 ? tagged : nullptr, copies);
-    return COUNT && !there ? 3 : got;
+    float lv[16];
+    const bool there = hand_gather<16>(row, lane, lv);  // (every wave)
+    topk_block_m<2>(reinterpret_cast<const float *>(row.hand), n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+    return there;
 }
 
 // Stand-alone softmax/top-k dispatch: one wave (src/qwen38_moe.cuh:711-818).
@@ -961,7 +939,7 @@ WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__r
 }
 
 // ---- dispatch AB ------------------------------------------------------------------------------------------
-// Workgroups [0, n_router_wgs): router rows, the last one to finish selects the experts and publishes the ids;
+// One workgroup that selects the experts and publishes the ids, n_router_wgs for the router rows,
 // then n_shared_wgs workgroups for the shared expert's gate/up; the rest for the routed gate/up, one (expert rung,
 // group of eight rows) item each: a (gate, up) row pair per wave.  The routed workgroups are dispatched after the router
 // ones (lower block index first), quantise x and stage the codebooks while the router runs, then poll the published ids;
@@ -969,7 +947,7 @@ WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__r
 // activation set-up from the critical path of the layer.  Where the ids are known before the launch (ids_known: a routing
 // trace, or a selection that is in the scratch) nothing is waited for and the weights are requested ahead of the set-up.
 //
-// Hand-off to the selecting workgroup: see topk_two_waves; no cache-wide release/acquire is needed for 2 KB of data.
+// Hand-off to the selecting workgroup: see hand_gather; no cache-wide release/acquire is needed for 2 KB of data.
 //
 // Publication: id j goes, as one 32-bit word, to ids_tagged[c][j] of every replica c with a device-scope atomic
 // store; a word other than kTagInvalid is the id itself, so a reader needs no second flag.  The words are reset
@@ -1011,8 +989,8 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     constexpr int kIqType = kIq ? TYPE : 21;
     extern __shared__ __align__(16) uint8_t lds_ab[];
     __shared__ __align__(16) uint8_t s_union[sizeof(Q8RowTile) * 8 > sizeof(IqTables) ? sizeof(Q8RowTile) * 8 : sizeof(IqTables)];
-    __shared__ int s_last;
-    const int wg = blockIdx.x;
+    __shared__ int s_last;  // (hand_close)
+    const int blk = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (a.dry) return;
     const int groups = (a.F + 7) / 8;
@@ -1020,35 +998,20 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     // HBM, unknown / known: 2048 / 512 19.61 / 19.48, 2048 / 768 20.20 / 20.14, IQ2_S 19.05 / 18.97, 2560 / 640 24.72 / 24.61, IQ2_S 23.16 / 23.20)
     const int H = FETCH == 8 ? 2048 : (FETCH == 10 ? 2560 : a.H);
 
-    mark<TRACE>(a, wg < a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);
-    if (wg < a.n_router_wgs) {
-        const int rows = a.preselected ? 0 : a.E;
-        int row;
-        float logit;
-        if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
-            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, rows, H,
-                                          a.sh_inp, a.E, wg, row);
-        else
-            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, rows, H, a.sh_inp, a.E, wg, row);
-        mark<TRACE>(a, 0, 1);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_waitcnt(0);  // this wave's word has been acknowledged
-        __syncthreads();
-        if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
-        if (TRACE && a.trace && threadIdx.x == 0) a.trace[(0 * 16 + 8) * 8 + 0] = wall_clock64();
-        int selected = 1;  // (no selection: the one workgroup with the shared gate's row)
+    mark<TRACE>(a, blk < a.n_select_wgs + a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);
+    if (blk < a.n_select_wgs) {
         // results land behind the selection's own scratch
         static_assert(sizeof(s_union) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
         int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
         float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
-        if (!a.preselected)
-            // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
-            selected = topk_block<false>(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, s_last, lane, wave,
-                                         (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
-        if (selected == 3 && lane == 0) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // off the selection's path: the shared expert's gate (by every workgroup that found the row complete: the same value)
-        if (selected && a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(a.hand + a.E)));
-        if (selected == 2 && wave == 0) {
+        if (wave == 0) __builtin_amdgcn_s_setprio(3);
+        // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
+        const bool there = topk_block(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
+                                      (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
+        if (!there && lane == 0) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // off the selection's path: the shared expert's gate
+        if (a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(a.hand + a.E)));
+        if (wave == 0) {
             wave_lds_fence();
             // the plain copies for dispatch C
             if (lane < a.k) {
@@ -1059,7 +1022,25 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
             if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
         }
         mark<TRACE>(a, 0, 2);
-        if (a.close_hand) hand_close(a.hand, a.E, a.n_router_wgs, s_last);
+        if (a.close_hand) hand_close(a.hand, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
+        return;
+    }
+    const int wg = blk - a.n_select_wgs;
+    if (wg < a.n_router_wgs) {
+        const int rows = a.preselected ? 0 : a.E;
+        int row;
+        float logit;
+        if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
+            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, rows, H,
+                                          a.sh_inp, a.E, wg, row);
+        else
+            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, rows, H, a.sh_inp, a.E, wg, row);
+        mark<TRACE>(a, 0, 1);
+        if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
+        // (no selection: the one wave with the shared gate's row)
+        if (a.preselected && row == a.E && lane == 32) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
+        mark<TRACE>(a, 0, 2);
+        if (a.close_hand) hand_close(a.hand, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
         return;
     }
 
@@ -1095,7 +1076,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         mark<TRACE>(a, 1, 1);
     };
     __shared__ int s_expert;
-    const int n_routed_wgs = LOOP ? static_cast<int>(gridDim.x) - a.n_router_wgs - a.n_shared_wgs : 0;
+    const int n_routed_wgs = LOOP ? static_cast<int>(gridDim.x) - a.n_select_wgs - a.n_router_wgs - a.n_shared_wgs : 0;
     // With known ids the set-up is done behind the requests of the first item (the variants named here have no registers
     // to hold these meanwhile).
     constexpr bool kBehind = FETCH != 0 && !(TYPE == 8 && LOOP);
@@ -1176,12 +1157,12 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     } while (LOOP && item < a.n_routed_items);
 }
 
-// (workgroup 0 of dispatch C) The words of this layer pass are done with: ids published, logits handed on, the ticket.
+// (workgroup 0 of dispatch C) The words of this layer pass are done with: ids published, logits handed on.
 WD_DEV void layer_clear_handed(const LayerArgs &a, int threads) {
     if (!a.clear_tagged || blockIdx.x != 0) return;
     for (int i = threadIdx.x; i < kTagCopies * 16; i += threads)
         __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int i = threadIdx.x; i < a.E + 2; i += threads) __hip_atomic_store(a.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = threadIdx.x; i < a.E + 1; i += threads) __hip_atomic_store(a.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---- the combine at the end of dispatch C ---------------------------------------------------------------------

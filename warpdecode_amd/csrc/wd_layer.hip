@@ -35,7 +35,7 @@ struct wd_moe_scratch {
     int32_t *gup = nullptr;
     int32_t *dp = nullptr;
     int gup_type = -1, dp_type = -1;
-    uint32_t *hand = nullptr;             // [n_experts + 3] logits on their way to the selection inside dispatch AB (LayerArgs)
+    uint32_t *hand = nullptr;             // [n_experts + 2] logits on their way to the selection inside dispatch AB (LayerArgs)
     unsigned long long *trace = nullptr;  // device [3][16][8] time stamps, see wd_moe_scratch_trace
     int trace_wg = 0;
     int32_t *h_ids = nullptr;             // pinned [48]: [0..15] routed ids for callers that must see them on the host,
@@ -103,7 +103,7 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
                  o_act = c.take(sizeof(float) * K1 * F), o_aq = c.take(K1 * F),
                  o_ad = c.take(sizeof(uint16_t) * K1 * (F / 32)), o_eo = c.take(sizeof(float) * K1 * H),
                  o_acc = c.take(sizeof(float) * H), o_dn = c.take(sizeof(float) * H), o_sg = c.take(256),
-                 o_hand = c.take(sizeof(uint32_t) * (n_experts + 3)),
+                 o_hand = c.take(sizeof(uint32_t) * (n_experts + 2)),
                  o_tag = c.take(sizeof(uint32_t) * kTagRecords * kTagCopies * 16), o_status = c.take(256);
     const hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->block), c.off);
     if (e != hipSuccess) {
@@ -135,7 +135,7 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
     s->status = reinterpret_cast<unsigned *>(b + o_status);
     (void)hipMemset(s->block, 0, c.off);
     (void)hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16);
-    (void)hipMemset(s->hand, 0xff, sizeof(uint32_t) * (n_experts + 3));
+    (void)hipMemset(s->hand, 0xff, sizeof(uint32_t) * (n_experts + 2));
     if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 48, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->block);
         delete s;
@@ -178,7 +178,7 @@ int wd_moe_scratch_set_wait_limit(wd_moe_scratch *s, unsigned polls) {
     WD_HIP(hipMemset(s->status, 0, sizeof(unsigned)));
     reinterpret_cast<volatile int32_t *>(s->h_ids)[16] = 0;
     WD_HIP(hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16));
-    WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 3)));
+    WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 2)));
     if (s->res_block) WD_HIP(hipMemset(s->res_block, 0xff, kHandEpoch));
     return WD_OK;
 }
@@ -542,6 +542,7 @@ int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s
     LayerArgs m = a;
     const int router_rows_n = front ? (a.preselected ? 0 : a.E) + (shared ? 1 : 0) : 0;
     m.n_router_wgs = wide ? (router_rows_n + 3) / 4 : (router_rows_n + 7) / 8;  // two waves or one per row
+    m.n_select_wgs = front && !a.preselected ? 1 : 0;
     m.n_shared_wgs = front && shared ? groups : 0;
     m.n_routed_items = routed ? a.k * groups : 0;
     if (!routed) m.ids_tagged = nullptr;  // nobody waits for them inside this launch
@@ -559,7 +560,7 @@ int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s
     const bool two = fetch == 0 && L->gate_type == WD_TYPE_IQ3_S;
     const int looping = two ? kAbPerCu<21, 0, true> * s->compute_units : std::max(capacity - fixed_wgs, groups);
     const int routed_wgs = m.n_routed_items <= capacity - 8 ? m.n_routed_items : std::min(m.n_routed_items, looping);
-    const int grid = m.n_router_wgs + m.n_shared_wgs + routed_wgs;
+    const int grid = m.n_select_wgs + m.n_router_wgs + m.n_shared_wgs + routed_wgs;
     if (grid == 0) return WD_OK;
     const bool loop = routed_wgs < m.n_routed_items;
     switch (L->gate_type) {
@@ -651,7 +652,7 @@ bool layer_c_evenly(int H, int F, int n_act, bool words) {
     return R > 8 && R <= 16 && n_act >= (R <= 12 ? 5 : 6) && !(words && R > 12);
 }
 
-// What dispatches A and AB hand on - the ids published in the scratch's records, the logits and the ticket - is set back by dispatch C,
+// What dispatches A and AB hand on - the ids published in the scratch's records, and the logits - is set back by dispatch C,
 // and where C does not follow by the dispatch itself (the logits, close_hand) and by these: a pass that finds what another one left
 // takes that one's ids.
 int reset_published(const wd_moe_scratch *s, int first, int records, hipStream_t st) {
@@ -662,7 +663,7 @@ int reset_published(const wd_moe_scratch *s, int first, int records, hipStream_t
 }
 // Both, behind an error after which no dispatch C comes.  (The error stays the one to report.)
 void reset_handed(const wd_moe_scratch *s, int rec, hipStream_t st) {
-    const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(s->n_experts) + 3;
+    const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(s->n_experts) + 2;
     enqueue(k_fill_u32, dim3(1), dim3(static_cast<unsigned>(record)), 0, st, s->tagged + static_cast<size_t>(rec % kTagRecords) * record, kTagInvalid, record);
     enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
     (void)hipGetLastError();
@@ -1110,7 +1111,7 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
     const bool wide = H > 2048 && H <= 4096;  // two waves per router row
     const int router_rows_n = (a.preselected ? 0 : a.E) + (a.sh_inp ? 1 : 0);
     a.n_router_wgs = wide ? (router_rows_n + 3) / 4 : (router_rows_n + 7) / 8;
-    const int grid_a = tokens_a_grid(a.n_router_wgs, a.sh_inp ? (F + 7) / 8 : 0).total(tokens);
+    const int grid_a = tokens_a_grid(a.n_router_wgs, a.sh_inp ? (F + 7) / 8 : 0).total(tokens, !a.preselected);
     const int items_b = tokens * k * ((F + 7) / 8);
     const int cus = scratch_per_token[0]->compute_units;
     // The parts that `front` and `routed` name

@@ -25,8 +25,8 @@ int g_compute_units[kNoAllocMaxDevices];
 
 // Offsets inside the array (fixed, so that the head of the array is the same whatever the layer).
 constexpr size_t kOffStatus = 0, kOffTagged = 256;                                 // words that must start clean: status, tagged, hand
-constexpr size_t kOffHand = kOffTagged + sizeof(uint32_t) * kTagCopies * 16;       // uint32 [experts + 3]
-constexpr size_t kOffIds = (kOffHand + sizeof(uint32_t) * (kNoAllocMaxExperts + 3) + 255) & ~static_cast<size_t>(255);  // int32 [16]
+constexpr size_t kOffHand = kOffTagged + sizeof(uint32_t) * kTagCopies * 16;       // uint32 [experts + 2]
+constexpr size_t kOffIds = (kOffHand + sizeof(uint32_t) * (kNoAllocMaxExperts + 2) + 255) & ~static_cast<size_t>(255);  // int32 [16]
 constexpr size_t kOffWeights = kOffIds + 256, kOffGate = kOffWeights + 256;       // f32 [16], f32 [1]
 constexpr size_t kOffLogits = kOffGate + 256;                                      // f32 [experts]
 constexpr size_t kOffVectors = kOffLogits + sizeof(float) * kNoAllocMaxExperts;    // accum, down_f32: f32 [hidden] each; then act

@@ -64,35 +64,61 @@ struct TokenArgs {
 };
 
 // ---- dispatch AB for T tokens, first part (A) --------------------------------------------------------------
-// T * (router_stride + shared_stride) workgroups, 512 threads, the strides being the router and the shared workgroups of a
-// token rounded up to a multiple of 8 (tokens_a_grid): first the router workgroups of every token, token by token, then
-// the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
+// kTokensSelectWgs (none where the ids are given) + T * (router_stride + shared_stride) workgroups, 512 threads, the strides being the router and the
+// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first one workgroup per token that selects, then the router workgroups
+// of every token, token by token, then the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
 // token - the same weight rows - lands on the same XCD (workgroups go to the eight XCDs in turn), so its L2 serves the
 // rows to the tokens after the first.  The padding workgroups return at once.  Per token this is the front of the
-// one-token merged dispatch: router rows one per wave, the last router workgroup of the token selects its experts
-// with the whole workgroup and publishes the ids, the other workgroups run the shared expert's gate/up.
+// one-token merged dispatch: router rows one per wave, the token's first workgroup waits for them, selects its experts
+// and publishes the ids, the other workgroups run the shared expert's gate/up.
 // lds: 4 * H + 16 bytes, x as f32 for the router rows (the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes of the
 // routed part's tables, for the selection; tiles: the shared rows' eight.
+constexpr int kTokensSelectWgs = kMaxTokens;
+static_assert(kTokensSelectWgs % 8 == 0, "the workgroups behind keep their XCDs");
 struct TokensAGrid {
     int router_stride, shared_stride;
-    __host__ __device__ int total(int tokens) const { return tokens * (router_stride + shared_stride); }
+    __host__ __device__ int total(int tokens, bool selects) const { return (selects ? kTokensSelectWgs : 0) + tokens * (router_stride + shared_stride); }
 };
 __host__ __device__ inline TokensAGrid tokens_a_grid(int n_router_wgs, int n_shared_wgs) {
     return TokensAGrid{(n_router_wgs + 7) & ~7, (n_shared_wgs + 7) & ~7};
 }
 constexpr int kTokensWorkBytes = kTopkLdsBytes2 + 128;
+// Selects token t's experts as the first workgroup of the one-token dispatch does.
+WD_DEV void tokens_select(const TokenArgs &ta, int t, uint8_t *s_work, int lane, int wave) {
+    const LayerArgs &a = ta.common;
+    const TokenSlots &s = ta.tok[t];
+    int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
+    float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
+    if (wave == 0) __builtin_amdgcn_s_setprio(3);
+    const bool there = topk_block(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr,
+                                  ta.wait_ids ? s.tagged : nullptr, kTagCopies);
+    if (!there && lane == 0) __hip_atomic_store(s.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(s.hand + a.E)));
+    if (wave == 0) {
+        wave_lds_fence();
+        if (lane < a.k) {
+            s.ids[lane] = lds_ids[lane];
+            s.weights[lane] = lds_w[lane];
+        }
+    }
+}
 // WIDE: router rows of 2049..4096 columns, two waves each (n_router_wgs is then for four rows per workgroup).
 // HIDDEN: 2048, where it is known (0: it is not).  With it the dispatch for five and more tokens spills 11 registers instead of 18; us per layer,
 // unknown / known: two tokens 28.3 / 28.3, four 41.1 / 40.3, eight 69.5 / 67.9.  (2560 known: nothing, 55.0 / 55.0 and 84.6 / 84.5.)
 template <bool WIDE, int HIDDEN>
-WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, Q8RowTile *tiles, int &s_last) {
+WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, Q8RowTile *tiles) {
     const LayerArgs &a = ta.common;
     const int H = HIDDEN ? HIDDEN : a.H;
     const int n_shared_wgs = a.sh_inp ? (a.F + 7) / 8 : 0;
     const TokensAGrid gr = tokens_a_grid(a.n_router_wgs, n_shared_wgs);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int token, wg;
     {
-        const int b = blockIdx.x, router_part = ta.T * gr.router_stride;
+        const int first = a.preselected ? 0 : kTokensSelectWgs, b = static_cast<int>(blockIdx.x) - first, router_part = ta.T * gr.router_stride;
+        if (b < 0) {
+            if (b + first < ta.T) tokens_select(ta, b + first, s_work, lane, wave);
+            return;
+        }
         if (b < router_part) {
             token = b / gr.router_stride, wg = b - token * gr.router_stride;
             if (wg >= a.n_router_wgs) return;
@@ -104,7 +130,6 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         }
     }
     const TokenSlots &s = ta.tok[token];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (wg < a.n_router_wgs) {
         const int rows = a.preselected ? 0 : a.E;
         int row;
@@ -114,31 +139,8 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         else
             logit = router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.hand, rows, H, a.sh_inp, a.E, wg, row);
         if (lane == 32 && row >= 0 && row < rows) s.logits[row] = logit;  // (the caller's view)
-        __syncthreads();  // (every wave has sent its word)
-        if (threadIdx.x == 0) s_last = hand_count_last(s.hand, a.E, a.n_router_wgs);
-        __syncthreads();
-        if (!s_last) return;
-        int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
-        float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
-        bool there = true;
-        if (a.preselected) {  // (the one row is the shared gate's)
-            if (wave == 5) {
-                float none[1];
-                there = hand_gather<1, true>(HandRow{s.hand, 0, a.E, true, a.spin_limit}, lane, none);
-            }
-        } else {
-            there = topk_block<true>(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, s_last, lane, wave, nullptr,
-                                     ta.wait_ids ? s.tagged : nullptr, kTagCopies) != 3;
-        }
-        if (!there && lane == 0) __hip_atomic_store(s.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(s.hand + a.E)));
-        if (!a.preselected && wave == 0) {
-            wave_lds_fence();
-            if (lane < a.k) {
-                s.ids[lane] = lds_ids[lane];
-                s.weights[lane] = lds_w[lane];
-            }
-        }
+        // (no selection: the one wave with the shared gate's row)
+        if (a.preselected && row == a.E && lane == 32) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
         return;
     }
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ta);
@@ -303,13 +305,12 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
     };
     static_assert(sizeof(Routed) >= kTokensWorkBytes, "the selection works in the place of the tables and the union");
     __shared__ __align__(16) uint8_t s_area[sizeof(Routed)];
-    __shared__ int s_last;
     const LayerArgs &a = ta.common;
     if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
         const bool wide = a.H > 2048 && a.H <= 4096;
         Q8RowTile *const tiles = reinterpret_cast<Q8RowTile *>(lds_tb + tokens_front_tiles(a.H));
-        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, 0>(ta, lds_tb, s_area, tiles, s_last);
-        else tokens_front<false, FETCH == 8 ? 2048 : 0>(ta, lds_tb, s_area, tiles, s_last);
+        if (FETCH != 8 && (FETCH == 10 || FETCH == 2 || wide)) tokens_front<true, 0>(ta, lds_tb, s_area, tiles);
+        else tokens_front<false, FETCH == 8 ? 2048 : 0>(ta, lds_tb, s_area, tiles);
         return;
     }
     IqTables &tables = reinterpret_cast<Routed *>(s_area)->tables;
@@ -537,12 +538,11 @@ __global__ __launch_bounds__(512, 4) void k_tokens_ab_q8(TokenArgs ta) {
     };
     static_assert(sizeof(Routed) >= kTokensWorkBytes && sizeof(Routed) >= 8 * sizeof(Q8RowTile), "the first part works in the place of the tiles and the union");
     __shared__ __align__(16) uint8_t s_area[sizeof(Routed)];
-    __shared__ int s_last;
     const LayerArgs &a = ta.common;
     if (static_cast<int>(blockIdx.x) < ta.front_wgs) {
         Q8RowTile *const tiles = reinterpret_cast<Q8RowTile *>(s_area);
-        if (a.H > 2048) tokens_front<true, 0>(ta, lds_tq, s_area, tiles, s_last);  // (hidden 4096 at most)
-        else tokens_front<false, 0>(ta, lds_tq, s_area, tiles, s_last);
+        if (a.H > 2048) tokens_front<true, 0>(ta, lds_tq, s_area, tiles);  // (hidden 4096 at most)
+        else tokens_front<false, 0>(ta, lds_tq, s_area, tiles);
         return;
     }
     Q8Tile8 *const tiles = reinterpret_cast<Routed *>(s_area)->tiles;
@@ -601,7 +601,7 @@ WD_DEV void tokens_clear_handed(const TokenArgs &ta, int waves, int tw, int lane
     if (static_cast<int>(blockIdx.x) >= ta.T || tw != waves - 1) return;
     const TokenSlots &s = ta.tok[blockIdx.x];
     for (int i = lane; i < kTagCopies * 16; i += 64) __hip_atomic_store(s.tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (int i = lane; i < ta.common.E + 2; i += 64) __hip_atomic_store(s.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = lane; i < ta.common.E + 1; i += 64) __hip_atomic_store(s.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // grid = H / 8: a workgroup owns eight output rows, as the one-token k_layer_c8 does.  Work items are (token, matrix) with
 // matrix = the token's k routed down tensors, then the shared one (always Q8_0); the waves take them in turn: the
