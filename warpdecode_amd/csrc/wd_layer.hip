@@ -550,15 +550,18 @@ int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s
     // A compute unit holds three of these workgroups.  The router and shared ones leave well before the ids are
     // published, so a few routed ones that have to wait for their places still start in time.  But when the routed
     // ones alone are more than the device holds at once (hidden 2560: 800 against 768), the surplus would start -
-    // quantise x, stage the codebooks - only after others have finished: the grid is then cut to what the device
-    // holds and the routed workgroups walk the items in a loop (measured at hidden 2560: 36.4 against 37.4 us per layer;
-    // there each router row has two waves, and the routed workgroups keep their number all the same).
-    const int fixed_wgs = (router_rows_n + 7) / 8 + m.n_shared_wgs;
-    const int capacity = 3 * s->compute_units;
+    // quantise x, stage the codebooks - only after others have finished: the grid is then cut and the routed workgroups walk the items in a
+    // loop.  Cut by the places of the router's workgroups, which are the last to leave, and not by the shared expert's; by neither
+    // where that saves a round of the loop.  us per layer, cut by both / by the router's / by neither: 2560 / 640 IQ2_S with a shared expert, 800 items, 24.3 /
+    // 23.8 / 24.0 (a workgroup for every item 26.0); 3328 / 864 Q8_0 with one, 972, 31.6 / 28.7 / 28.8; 2048 / 992 Q8_0 with one, 1240, 24.5 / 22.7 /
+    // 23.1; without one 1536 / 832 IQ2_S, 936, 18.0 / 18.0 / 18.4, and 4096 / 1536, 1536 items in three rounds / three / two, 40.0 / 40.0 / 39.3.
+    const int capacity = 3 * s->compute_units, router_places = (router_rows_n + 7) / 8;
+    auto rounds = [&](int wgs) { return (m.n_routed_items + wgs - 1) / wgs; };
     // (The loop that runs two per compute unit, kAbPerCu, takes all of its places: with the shared expert's workgroups counted among
     // them hidden 7168 / ffn 2048, top-8, has 256 routed workgroups left and takes 106 us, so 68; 5120 / 1024 40.7, 34.2.)
     const bool two = fetch == 0 && L->gate_type == WD_TYPE_IQ3_S;
-    const int looping = two ? kAbPerCu<21, 0, true> * s->compute_units : std::max(capacity - fixed_wgs, groups);
+    const int cut = std::max(capacity - router_places, 1);
+    const int looping = two ? kAbPerCu<21, 0, true> * s->compute_units : (rounds(cut) > rounds(capacity) ? capacity : cut);
     const int routed_wgs = m.n_routed_items <= capacity - 8 ? m.n_routed_items : std::min(m.n_routed_items, looping);
     const int grid = m.n_select_wgs + m.n_router_wgs + m.n_shared_wgs + routed_wgs;
     if (grid == 0) return WD_OK;
