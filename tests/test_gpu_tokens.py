@@ -289,6 +289,41 @@ def test_logits_that_are_late_are_reported(g, oracle, E, k, preselected):
         s.close()
 
 
+@pytest.mark.parametrize("E,k", [(64, 6), (2048, 4), (2056, 4)])
+def test_scratches_at_many_addresses(g, oracle, E, k):
+    """What workgroups hand on lies in pieces of the scratch chosen by where the scratch happens to be (and the logits outside of them where
+    they do not fit one): scratches of different sizes, used one by one and as a batch, give the oracle's results, twice."""
+    H, F, T = 512, 64, 8
+    L = synth.make_layer(H, F, 64, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=39, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, T, 13)
+    want = [oracle.moe_layer(L, x)[0] for x in xs]
+    dl = g.DeviceLayer(L)
+    scr = [g.Scratch(H, F, E, k + t) for t in range(T)]
+    arr = (C.c_void_p * T)(*[s.h for s in scr])
+    dx, out = g.dev(xs), g.empty((T, H), np.float32)
+    for turn in range(2):
+        for t, s in enumerate(scr):
+            row = C.c_void_p(dx.data_ptr() + 4 * H * t), C.c_void_p(out.data_ptr() + 4 * H * t)
+            capi.call("wd_moe_layer_f32", C.byref(dl.desc), *row, s.h, 0, g.stream())
+        g.sync()
+        assert g.same_bits(g.host(out), np.stack(want)), ("layers", turn)
+        out.zero_()
+        capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), T, arr, 0, g.stream())
+        g.sync()
+        assert g.same_bits(g.host(out), np.stack(want)), ("batch", turn)
+    stack = (capi.MoeLayer * 35)(*[dl.desc] * 35)    # records of published ids beyond the first piece's
+    x0, o0 = g.dev(xs[0]), g.empty(H, np.float32)
+    for flags in (0, capi.MOE_SPLIT_AB):
+        xc = g.dev(xs[0])
+        capi.call("wd_moe_stack_f32", stack, 35, g.ptr(xc), g.ptr(out), scr[0].h, None, 0.0, flags, g.stream())
+        capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(x0), g.ptr(o0), scr[0].h, 0, g.stream())
+        g.sync()
+        assert g.same_bits(g.host(out)[0], want[0]) and g.same_bits(g.host(o0), want[0]), flags
+    assert [capi.load().wd_moe_scratch_status(s.h) for s in scr] == [0] * T
+    for s in scr:
+        s.close()
+
+
 @pytest.mark.parametrize("shape", ["eight-blocks", "q8_0", "ids-by-the-block-form"])
 def test_passes_that_end_before_the_down_projections(g, oracle, shape):
     """Calls of dispatch A or of A and B without C, on one input, leave nothing on the scratch that a pass of another kind takes

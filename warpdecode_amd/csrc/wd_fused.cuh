@@ -45,7 +45,8 @@ struct LayerArgs {
     int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
     const int32_t *ids_known;    // null, or the k ids where they are known before the launch
     uint32_t *hand;              // [E + 2]: the router's logits and the shared gate's on their way to the selection, and the count of hand_close; kHandEmpty between passes
-    uint32_t *ids_tagged;        // [kTagCopies][16] selected ids published inside the merged dispatch (kTagInvalid = not yet)
+    uint32_t *ids_tagged;        // selected ids published inside the merged dispatch (kTagInvalid = not yet): [kTagCopies / 2][16] for side 0,
+    int tag_side;                // so many words on from these for side 1 (tag_copy)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
     int close_hand;              // no dispatch C follows: the router workgroups set `hand` back themselves
     unsigned *status;            // [0] set to 1 when a bounded wait inside a dispatch ran out
@@ -60,6 +61,18 @@ struct LayerArgs {
 
 constexpr int kTagCopies = 16;           // replicas of the published ids, 64 bytes apart, so that pollers spread over lines
 constexpr uint32_t kTagInvalid = 0xffffffffu;
+
+// Sides.  A word that workgroups hand on has a home in one half of the device's memory, and the XCDs of that half reach it sooner: a device-scope
+// load that misses the L2 takes 350 to 450 clocks near its home and 580 to 700 from the other half (stores 370 to 500 and 600 to 760), a word from
+// XCD 0 to XCD 1 360 ns by way of the near half and 575 by the far one.  Memory alternates between the halves in pieces of kSidePiece bytes; which
+// of two neighbours is whose is measured when a scratch is made (k_scratch_init).  Words lie on their readers' side: workgroup b runs on XCD b mod 8,
+// XCDs 0..3 are side 0, the others side 1.
+constexpr int kSidePiece = 8192;
+WD_DEV int block_side() { return static_cast<int>((blockIdx.x >> 2) & 1u); }
+// The replica of the published ids that workgroup `wg` of the waiting ones polls.
+WD_DEV const uint32_t *tag_copy(const uint32_t *tagged, int tag_side, int wg) {
+    return tagged + (block_side() ? tag_side : 0) + ((wg >> 3) & (kTagCopies / 2 - 1)) * 16;
+}
 constexpr unsigned kSpinLimit = 1u << 16;  // default number of polls before a wait gives up (tens of milliseconds; a wait lasts microseconds)
 
 // Time stamp `i` of dispatch `d` (0 = A, 1 = B, 2 = C) for the traced workgroup; lane 0 of every wave.
@@ -296,16 +309,15 @@ WD_DEV void topk_wave_m(const float *logits, int n, int k, float w_scale, int32_
     finish_weights(top_mine, id_mine, k, w_scale, ids, weights, override_ids, lane);
 }
 
-// The ids held by lanes 0..k-1 (k <= 16) into the `copies` replicas: into every row of 16 lanes first, then four replicas
+// The ids held by lanes 0..k-1 (k <= 16) into the kTagCopies replicas: into every row of 16 lanes first, then four replicas
 // per store instruction, so that the last replica goes out a quarter of the stores after the first.
-WD_DEV void publish_ids(int id_mine, int k, uint32_t *tagged, int copies, int lane) {
+WD_DEV void publish_ids(int id_mine, int k, uint32_t *tagged, int tag_side, int lane) {
     const wd_uint2v t16 = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(id_mine), static_cast<uint32_t>(id_mine), false, false);
     const wd_uint2v t32 = __builtin_amdgcn_permlane32_swap(t16.x, t16.x, false, false);
     const int j = lane & 15, c4 = lane >> 4;
-#pragma unroll 4
-    for (int c0 = 0; c0 < copies; c0 += 4)
-        if (j < k && c0 + c4 < copies)
-            __hip_atomic_store(tagged + (c0 + c4) * 16 + j, t32.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int c0 = 0; c0 < kTagCopies; c0 += 4)  // (the sides in turn)
+        if (j < k) __hip_atomic_store(tagged + ((c0 & 4) ? tag_side : 0) + ((c0 >> 3) * 4 + c4) * 16 + j, t32.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The same selection by a workgroup of eight waves (every thread must call it; it contains barriers).
@@ -328,7 +340,7 @@ WD_DEV void publish_ids(int id_mine, int k, uint32_t *tagged, int copies, int la
 //      reference's rungs over the probabilities themselves.
 // lds: 4 * (512 * M + 600) bytes of scratch.  The results are written by wave 0 (lanes 0..k-1).
 // tagged != null: as soon as the ids are known - before the renormalisation, which only the weights need - id j
-// goes to tagged[c * 16 + j] of the `copies` replicas with device-scope atomic stores (the readers poll them).
+// goes to every replica with device-scope atomic stores (the readers poll them).
 // Ids given by the caller (override_ids) are requested up front, so their round trip is not behind the selection.
 // The three steps as functions of their own, so that a caller with the logits already in registers (or with waves
 // that only keep the barriers company) can compose them.  LDS layout of the selection's scratch:
@@ -413,7 +425,7 @@ WD_DEV void topk_block_step2(const float (&l)[M], int n, int k, const TopkLds<M>
 // id_given: the caller's id for lane j < k when the ids are replaced (override), requested before step 1.
 template <int M>
 WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *weights, bool override_ids, int id_given,
-                             const TopkLds<M> &s, int lane, unsigned long long *stamps, uint32_t *tagged, int copies) {
+                             const TopkLds<M> &s, int lane, unsigned long long *stamps, uint32_t *tagged, int tag_side) {
 #define WD_STAMP(i) do { if (stamps && lane == 0) stamps[i] = wall_clock64(); } while (0)
     auto nan_is_large = [](float v) { return v != v ? INFINITY : v; };
     const int groups = n >> 3;
@@ -459,7 +471,7 @@ WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *w
     const bool all_good = __builtin_amdgcn_ballot_w64(good) == ~0ull;
     int id_mine = override_ids ? id_given : idc;
     if (all_good && tagged) {
-        publish_ids(id_mine, k, tagged, copies, lane);
+        publish_ids(id_mine, k, tagged, tag_side, lane);
     }
     WD_STAMP(6);
 
@@ -489,7 +501,7 @@ WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *w
         if (M == 1 || n <= 512) rungs(std::integral_constant<int, 1>{});
         else rungs(std::integral_constant<int, M>{});
         if (override_ids) id_mine = id_given;
-        if (tagged) publish_ids(id_mine, k, tagged, copies, lane);
+        if (tagged) publish_ids(id_mine, k, tagged, tag_side, lane);
     }
     finish_weights(top_mine, id_mine, k, w_scale, ids, weights, nullptr, lane);
     WD_STAMP(7);
@@ -499,7 +511,7 @@ WD_DEV void topk_block_step3(int n, int k, float w_scale, int32_t *ids, float *w
 template <int M>
 WD_DEV void topk_block_m(const float *logits, int n, int k, float w_scale, int32_t *ids, float *weights,
                          const int32_t *__restrict__ override_ids, uint8_t *lds, int lane, int wave,
-                         unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
+                         unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int tag_side = 0) {
 #define WD_STAMP(i) do { if (stamps && wave == 0 && lane == 0) stamps[i] = wall_clock64(); } while (0)
     const TopkLds<M> s(lds);
     WD_STAMP(0);
@@ -518,7 +530,7 @@ WD_DEV void topk_block_m(const float *logits, int n, int k, float w_scale, int32
     __syncthreads();
     WD_STAMP(2);
     if (wave == 0)
-        topk_block_step3<M>(n, k, w_scale, ids, weights, override_ids != nullptr, id_given, s, lane, stamps, tagged, copies);
+        topk_block_step3<M>(n, k, w_scale, ids, weights, override_ids != nullptr, id_given, s, lane, stamps, tagged, tag_side);
 #undef WD_STAMP
 }
 
@@ -716,7 +728,7 @@ WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
 // the weights behind one barrier.  Every thread of the workgroup must call it.  ids, weights: LDS.
 template <int M>
 WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
-                           uint8_t *lds, int lane, int wave, unsigned long long *stamps, uint32_t *tagged, int copies) {
+                           uint8_t *lds, int lane, int wave, unsigned long long *stamps, uint32_t *tagged, int tag_side) {
 #define WD_STAMP(i) do { if (stamps && wave == 0 && lane == 0) stamps[i] = wall_clock64(); } while (0)
     const TopkLds<1> s(lds);
     const int n = row.n;
@@ -732,7 +744,7 @@ WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *id
     if (wave == 0) {
         sel_wave_ids(lv, n, k, s, lane, st);
         WD_STAMP(3);
-        if (st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        if (st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, tag_side, lane);
         WD_STAMP(6);
     } else if (wave == 1) {
         bool dead;
@@ -743,7 +755,7 @@ WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *id
     if (wave == 0) {
         const bool fast = st.fast;
         sel_wave_weights(n, k, w_scale, s, lane, st, s.rest[0], s.rest[1] != 0.0f, ids, weights, override_ids != nullptr, id_given);
-        if (!fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, copies, lane);
+        if (!fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, tag_side, lane);
         WD_STAMP(7);
     }
 #undef WD_STAMP
@@ -755,17 +767,17 @@ WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *id
 // (64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
 // there are experts to select its threshold excludes nobody -; 512 experts, top-10: 2.1, 2.2.)
 WD_DEV bool topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
-                       uint8_t *lds, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int copies = 0) {
+                       uint8_t *lds, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int tag_side = 0) {
     const int n = row.n;
     if (n <= 512 && k <= 15) {
-        if (n <= 64) return topk_two_waves<1>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-        if (n <= 128) return topk_two_waves<2>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-        if (n <= 256) return topk_two_waves<4>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
-        return topk_two_waves<8>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+        if (n <= 64) return topk_two_waves<1>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, tag_side);
+        if (n <= 128) return topk_two_waves<2>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, tag_side);
+        if (n <= 256) return topk_two_waves<4>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, tag_side);
+        return topk_two_waves<8>(row, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, tag_side);
     }
     float lv[16];
     const bool there = hand_gather<16>(row, lane, lv);  // (every wave)
-    topk_block_m<2>(reinterpret_cast<const float *>(row.hand), n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, copies);
+    topk_block_m<2>(reinterpret_cast<const float *>(row.hand), n, k, w_scale, ids, weights, override_ids, lds, lane, wave, stamps, tagged, tag_side);
     return there;
 }
 
@@ -1007,7 +1019,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         if (wave == 0) __builtin_amdgcn_s_setprio(3);
         // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
         const bool there = topk_block(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
-                                      (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, kTagCopies);
+                                      (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, a.tag_side);
         if (!there && lane == 0) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // off the selection's path: the shared expert's gate
         if (a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(a.hand + a.E)));
@@ -1095,7 +1107,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
             if (!kBehind) __syncthreads();
         } else {
             if (threadIdx.x == 0) {
-                const uint32_t *src = a.ids_tagged + (bw & (kTagCopies - 1)) * 16 + j;
+                const uint32_t *src = tag_copy(a.ids_tagged, a.tag_side, bw) + j;
                 uint32_t id = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 unsigned polls = 0;
                 while (id == kTagInvalid && ++polls < a.spin_limit) {
@@ -1160,8 +1172,10 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
 // (workgroup 0 of dispatch C) The words of this layer pass are done with: ids published, logits handed on.
 WD_DEV void layer_clear_handed(const LayerArgs &a, int threads) {
     if (!a.clear_tagged || blockIdx.x != 0) return;
-    for (int i = threadIdx.x; i < kTagCopies * 16; i += threads)
+    for (int i = threadIdx.x; i < kTagCopies * 8; i += threads) {
         __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(a.ids_tagged + a.tag_side + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     for (int i = threadIdx.x; i < a.E + 1; i += threads) __hip_atomic_store(a.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 

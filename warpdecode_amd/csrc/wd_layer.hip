@@ -13,6 +13,12 @@
 
 using namespace wd;
 
+namespace {
+constexpr int kTagRecords = 64;  // one record per layer of a stack (modulo), so that a chain of layers needs no reset in between
+constexpr int kTagRecordsPerPiece = kSidePiece / (kTagCopies * 8 * 4);
+constexpr int kTagUnits = kTagRecords / kTagRecordsPerPiece;  // of two pieces
+}  // namespace
+
 struct wd_moe_scratch {
     int hidden = 0, ffn = 0, n_experts = 0, max_k = 0;
     uint8_t *block = nullptr;
@@ -41,7 +47,16 @@ struct wd_moe_scratch {
     int32_t *h_ids = nullptr;             // pinned [48]: [0..15] routed ids for callers that must see them on the host,
                                           // [16] mirror of the status word, written by the resident launch when a wait runs out,
                                           // [32..47] the selection as dispatch AB reports it (cached_routed_reported)
-    uint32_t *tagged = nullptr;           // [kTagRecords][kTagCopies][16] ids published inside the merged dispatch
+    // ids published inside the merged dispatch, kTagRecords records.  sided: kTagRecordsPerPiece records' copies of side 0 and those of side 1 in two
+    // pieces of kSidePiece bytes, flip: side 1's first; otherwise [record][kTagCopies][16].
+    uint32_t *tagged = nullptr;
+    bool sided = false;
+    int flip = 0;
+    uint32_t *tags(int rec) const {
+        if (!sided) return tagged + static_cast<size_t>(rec) * kTagCopies * 16;
+        return tagged + (2 * (rec / kTagRecordsPerPiece) + flip) * (kSidePiece / 4) + (rec % kTagRecordsPerPiece) * (kTagCopies * 8);
+    }
+    int tag_side() const { return !sided ? kTagCopies * 8 : (flip ? -kSidePiece / 4 : kSidePiece / 4); }
     unsigned *status = nullptr;           // [0] != 0: a bounded wait inside a dispatch ran out
     unsigned spin_limit = kSpinLimit;
     int compute_units = 256;              // of the device the scratch lives on
@@ -66,10 +81,6 @@ struct wd_moe_scratch {
 constexpr int kPairRing = 4;
 
 namespace {
-constexpr int kTagRecords = 64;  // one record per layer of a stack (modulo), so that a chain of layers needs no reset in between
-}
-
-namespace {
 
 struct Carver {
     size_t off = 0;
@@ -79,6 +90,30 @@ struct Carver {
         return at;
     }
 };
+
+}  // namespace
+
+namespace {
+
+// A scratch's block: zeros, but for the words that are handed on, which are "not yet" (ones_at .. ones_end, in words).  Then workgroup b < 8 (XCD b mod 8)
+// times round trips of device-scope accesses to the first two pieces at `sided`, its loads and stores leaving the words as they are (votes[b] > 0: the
+// second piece is nearer).
+__global__ __launch_bounds__(256) void k_scratch_init(uint32_t *block, unsigned words, unsigned ones_at, unsigned ones_end, uint32_t *sided, int *votes) {
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) block[i] = i >= ones_at && i < ones_end ? kHandEmpty : 0u;
+    if (blockIdx.x >= 8 || threadIdx.x != 0) return;
+    long long sum = 0;
+    for (int turn = 0; turn < 10; ++turn) {
+        uint32_t *p = sided + (turn & 1) * (kSidePiece / 4) + blockIdx.x * 64;
+        const long long t0 = clock64();
+        __hip_atomic_store(p, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint32_t v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(v)::"memory");
+        const long long t = clock64() - t0;
+        if (turn >= 2) sum += (turn & 1) ? -t : t;
+    }
+    votes[blockIdx.x] = static_cast<int>(sum);
+}
 
 }  // namespace
 
@@ -103,8 +138,11 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
                  o_act = c.take(sizeof(float) * K1 * F), o_aq = c.take(K1 * F),
                  o_ad = c.take(sizeof(uint16_t) * K1 * (F / 32)), o_eo = c.take(sizeof(float) * K1 * H),
                  o_acc = c.take(sizeof(float) * H), o_dn = c.take(sizeof(float) * H), o_sg = c.take(256),
-                 o_hand = c.take(sizeof(uint32_t) * (n_experts + 2)),
-                 o_tag = c.take(sizeof(uint32_t) * kTagRecords * kTagCopies * 16), o_status = c.take(256);
+                 o_status = c.take(256);
+    // the words that are handed on: the logits where they do not fit a piece, then (from a boundary of two pieces, within 2 MB, in which the
+    // halves keep their order) two pieces for them and those of the published ids
+    const size_t side_bytes = 2 * static_cast<size_t>(kSidePiece) * (1 + kTagUnits);
+    const size_t o_hand = c.take(sizeof(uint32_t) * (n_experts + 2)), o_side = c.take(2 * side_bytes + 2 * kSidePiece);
     const hipError_t e = hipMalloc(reinterpret_cast<void **>(&s->block), c.off);
     if (e != hipSuccess) {
         delete s;
@@ -131,16 +169,32 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
     s->down_f32 = reinterpret_cast<float *>(b + o_dn);
     s->shared_gate = reinterpret_cast<float *>(b + o_sg);
     s->hand = reinterpret_cast<uint32_t *>(b + o_hand);
-    s->tagged = reinterpret_cast<uint32_t *>(b + o_tag);
+    uintptr_t side = (reinterpret_cast<uintptr_t>(b + o_side) + 2 * kSidePiece - 1) & ~static_cast<uintptr_t>(2 * kSidePiece - 1);
+    constexpr uintptr_t kChunk = 2u << 20;
+    if (side / kChunk != (side + side_bytes - 1) / kChunk) side = (side / kChunk + 1) * kChunk;
+    uint32_t *const units = reinterpret_cast<uint32_t *>(side);
+    s->tagged = units + 2 * kSidePiece / 4, s->sided = true;
     s->status = reinterpret_cast<unsigned *>(b + o_status);
-    (void)hipMemset(s->block, 0, c.off);
-    (void)hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16);
-    (void)hipMemset(s->hand, 0xff, sizeof(uint32_t) * (n_experts + 2));
     if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 48, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->block);
         delete s;
         return fail(WD_ERR_HIP, "hipHostMalloc MoE scratch ids failed");
     }
+    std::memset(s->h_ids, 0, sizeof(int32_t) * 48);
+    enqueue(k_scratch_init, dim3(64), dim3(256), 0, nullptr, reinterpret_cast<uint32_t *>(b), static_cast<unsigned>(c.off / 4), static_cast<unsigned>(o_hand / 4),
+            static_cast<unsigned>(c.off / 4), units, s->h_ids);
+    hipError_t init = hipGetLastError();
+    if (init == hipSuccess) init = hipStreamSynchronize(nullptr);
+    if (init != hipSuccess) {
+        (void)hipHostFree(s->h_ids);
+        (void)hipFree(s->block);
+        delete s;
+        return fail(WD_ERR_HIP, "MoE scratch: the first launch failed: %s", hipGetErrorString(init));
+    }
+    int second = 0;  // workgroups that say that the second piece is side 0's
+    for (int g = 0; g < 8; ++g) second += (s->h_ids[g] > 0) == (g < 4) ? 1 : 0;
+    s->flip = second > 4 ? 1 : 0;
+    if (sizeof(uint32_t) * (static_cast<size_t>(n_experts) + 2) <= kSidePiece) s->hand = units + s->flip * (kSidePiece / 4);
     std::memset(s->h_ids, 0, sizeof(int32_t) * 48);
     *out = s;
     return WD_OK;
@@ -177,7 +231,7 @@ int wd_moe_scratch_set_wait_limit(wd_moe_scratch *s, unsigned polls) {
     WD_HIP(hipDeviceSynchronize());  // (a launch that gave up may still be running and would set the words again)
     WD_HIP(hipMemset(s->status, 0, sizeof(unsigned)));
     reinterpret_cast<volatile int32_t *>(s->h_ids)[16] = 0;
-    WD_HIP(hipMemset(s->tagged, 0xff, sizeof(uint32_t) * kTagRecords * kTagCopies * 16));
+    WD_HIP(hipMemset(s->tagged, 0xff, 2 * static_cast<size_t>(kSidePiece) * kTagUnits));
     WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 2)));
     if (s->res_block) WD_HIP(hipMemset(s->res_block, 0xff, kHandEpoch));
     return WD_OK;
@@ -479,7 +533,7 @@ LayerArgs fused_args(const wd_moe_layer *L, const float *d_x, float *d_out, wd_m
     a.ids_known = ids_override;  // a routing trace: the ids do not depend on the router
     a.trace = s->trace, a.trace_wg = s->trace_wg;
     a.hand = s->hand;
-    a.ids_tagged = s->tagged + static_cast<size_t>(rec % kTagRecords) * kTagCopies * 16;
+    a.ids_tagged = s->tags(rec % kTagRecords), a.tag_side = s->tag_side();
     a.clear_tagged = 1;
     a.status = s->status;
     a.spin_limit = s->spin_limit;
@@ -658,16 +712,28 @@ bool layer_c_evenly(int H, int F, int n_act, bool words) {
 // What dispatches A and AB hand on - the ids published in the scratch's records, and the logits - is set back by dispatch C,
 // and where C does not follow by the dispatch itself (the logits, close_hand) and by these: a pass that finds what another one left
 // takes that one's ids.
-int reset_published(const wd_moe_scratch *s, int first, int records, hipStream_t st) {
-    const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(records) * record;
-    enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->tagged + static_cast<size_t>(first % kTagRecords) * record, kTagInvalid, n);
+__global__ __launch_bounds__(kTagCopies * 8) void k_reset_tags(uint32_t *tags, int tag_side) {
+    tags[threadIdx.x] = kTagInvalid, tags[tag_side + static_cast<int>(threadIdx.x)] = kTagInvalid;
+}
+void reset_tags(const wd_moe_scratch *s, int rec, hipStream_t st) {
+    enqueue(k_reset_tags, dim3(1), dim3(kTagCopies * 8), 0, st, s->tags(rec % kTagRecords), s->tag_side());
+}
+// (of a scratch made by wd_moe_scratch_create)
+int reset_all_published(const wd_moe_scratch *s, hipStream_t st) {
+    const size_t n = 2 * static_cast<size_t>(kSidePiece / 4) * kTagUnits;
+    enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->tagged, kTagInvalid, n);
+    WD_LAUNCH_CHECK();
+    return WD_OK;
+}
+int reset_published(const wd_moe_scratch *s, int rec, hipStream_t st) {
+    reset_tags(s, rec, st);
     WD_LAUNCH_CHECK();
     return WD_OK;
 }
 // Both, behind an error after which no dispatch C comes.  (The error stays the one to report.)
 void reset_handed(const wd_moe_scratch *s, int rec, hipStream_t st) {
-    const size_t record = static_cast<size_t>(kTagCopies) * 16, n = static_cast<size_t>(s->n_experts) + 2;
-    enqueue(k_fill_u32, dim3(1), dim3(static_cast<unsigned>(record)), 0, st, s->tagged + static_cast<size_t>(rec % kTagRecords) * record, kTagInvalid, record);
+    const size_t n = static_cast<size_t>(s->n_experts) + 2;
+    reset_tags(s, rec, st);
     enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
     (void)hipGetLastError();
 }
@@ -703,7 +769,7 @@ int layer_fused_queue(const wd_moe_layer *L, const float *d_x, float *d_out, wd_
     }
     if (only && !(only & WD_MOE_ONLY_C)) {
         // dispatch C, which sets the handed words back, is not part of this call (with a report it follows in the same one)
-        return merged && !chain && !report && !a.dry ? reset_published(s, rec, 1, st) : static_cast<int>(WD_OK);
+        return merged && !chain && !report && !a.dry ? reset_published(s, rec, st) : static_cast<int>(WD_OK);
     }
     SiteScope site(WD_SITE_FUSED_C, st);
     const int n_act = k + (shared ? 1 : 0);
@@ -984,7 +1050,7 @@ extern "C" int wd_moe_stack_f32(const wd_moe_layer *layers, int n_layers, float 
             rc = layer_dispatch(&layers[l], d_x, d_layer_out, s, flags, trace, d_x, residual_scale, st, l, nullptr, chain);
         }
         if (chain && (rc || l + 1 == n_layers || (l + 1) % kTagRecords == 0)) {
-            const int rc_reset = reset_published(s, 0, kTagRecords, st);
+            const int rc_reset = reset_all_published(s, st);
             if (rc == WD_OK) rc = rc_reset;
         }
         if (rc) return rc;
@@ -1108,7 +1174,7 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         k_.shared_gate = s->shared_gate, k_.hand = s->hand;
         k_.expert_out = (flags & WD_MOE_KEEP_EXPERT_OUT) ? s->expert_out : nullptr;
         k_.accum = s->accum, k_.down_f32 = s->down_f32;
-        k_.tagged = s->tagged, k_.status = s->status;
+        k_.tagged = s->tags(0), k_.tag_side = s->tag_side(), k_.status = s->status;
     }
     LayerArgs &a = ta.common;
     const bool wide = H > 2048 && H <= 4096;  // two waves per router row

@@ -51,7 +51,8 @@ struct TokenSlots {
     uint32_t *hand;      // (LayerArgs)
     float *expert_out;   // null or [k][H]
     float *accum, *down_f32, *out;
-    uint32_t *tagged;    // [kTagCopies][16] selected ids published inside dispatch AB (kTagInvalid = not yet)
+    uint32_t *tagged;    // selected ids published inside dispatch AB (ids_tagged, LayerArgs),
+    int tag_side;
     unsigned *status;    // [0] set to 1 when a wait for the ids or the logits ran out
 };
 
@@ -65,7 +66,7 @@ struct TokenArgs {
 
 // ---- dispatch AB for T tokens, first part (A) --------------------------------------------------------------
 // kTokensSelectWgs (none where the ids are given) + T * (router_stride + shared_stride) workgroups, 512 threads, the strides being the router and the
-// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first one workgroup per token that selects, then the router workgroups
+// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first two workgroups per token of which one selects, then the router workgroups
 // of every token, token by token, then the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
 // token - the same weight rows - lands on the same XCD (workgroups go to the eight XCDs in turn), so its L2 serves the
 // rows to the tokens after the first.  The padding workgroups return at once.  Per token this is the front of the
@@ -73,7 +74,8 @@ struct TokenArgs {
 // and publishes the ids, the other workgroups run the shared expert's gate/up.
 // lds: 4 * H + 16 bytes, x as f32 for the router rows (the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes of the
 // routed part's tables, for the selection; tiles: the shared rows' eight.
-constexpr int kTokensSelectWgs = kMaxTokens;
+// (workgroups 4..7 of every eight return at once: the words that a selection waits for lie on side 0)
+constexpr int kTokensSelectWgs = 2 * kMaxTokens;
 static_assert(kTokensSelectWgs % 8 == 0, "the workgroups behind keep their XCDs");
 struct TokensAGrid {
     int router_stride, shared_stride;
@@ -91,7 +93,7 @@ WD_DEV void tokens_select(const TokenArgs &ta, int t, uint8_t *s_work, int lane,
     float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
     if (wave == 0) __builtin_amdgcn_s_setprio(3);
     const bool there = topk_block(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr,
-                                  ta.wait_ids ? s.tagged : nullptr, kTagCopies);
+                                  ta.wait_ids ? s.tagged : nullptr, s.tag_side);
     if (!there && lane == 0) __hip_atomic_store(s.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(s.hand + a.E)));
     if (wave == 0) {
@@ -116,7 +118,8 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
     {
         const int first = a.preselected ? 0 : kTokensSelectWgs, b = static_cast<int>(blockIdx.x) - first, router_part = ta.T * gr.router_stride;
         if (b < 0) {
-            if (b + first < ta.T) tokens_select(ta, b + first, s_work, lane, wave);
+            const int t = (blockIdx.x & 3) + 4 * (blockIdx.x >> 3);
+            if (block_side() == 0 && t < ta.T) tokens_select(ta, t, s_work, lane, wave);
             return;
         }
         if (b < router_part) {
@@ -202,14 +205,14 @@ WD_DEV bool token_pairs_wait(const TokenArgs &ta, int lane, int &id_lo, int &id_
     auto word_of = [&](int pair) {
         const int pc = min(pair, n - 1);
         int t = 0;
-        const uint32_t *p = ta.tok[0].tagged;
+        const uint32_t *p = tag_copy(ta.tok[0].tagged, ta.tok[0].tag_side, static_cast<int>(blockIdx.x));
 #pragma unroll
         for (int q = 1; q < kMaxTokens; ++q) {
             const bool past = pc >= q * k;
             t += past ? 1 : 0;
-            p = past ? ta.tok[q].tagged : p;
+            p = past ? tag_copy(ta.tok[q].tagged, ta.tok[q].tag_side, static_cast<int>(blockIdx.x)) : p;
         }
-        return p + (blockIdx.x & (kTagCopies - 1)) * 16 + (pc - t * k);
+        return p + (pc - t * k);
     };
     const uint32_t *const lo = word_of(lane), *const hi = word_of(lane + 64);
     for (unsigned polls = 1;; ++polls) {
@@ -600,7 +603,10 @@ __global__ __launch_bounds__(512, 4) void k_tokens_ab_q8(TokenArgs ta) {
 WD_DEV void tokens_clear_handed(const TokenArgs &ta, int waves, int tw, int lane) {
     if (static_cast<int>(blockIdx.x) >= ta.T || tw != waves - 1) return;
     const TokenSlots &s = ta.tok[blockIdx.x];
-    for (int i = lane; i < kTagCopies * 16; i += 64) __hip_atomic_store(s.tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = lane; i < kTagCopies * 8; i += 64) {
+        __hip_atomic_store(s.tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(s.tagged + s.tag_side + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     for (int i = lane; i < ta.common.E + 1; i += 64) __hip_atomic_store(s.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // grid = H / 8: a workgroup owns eight output rows, as the one-token k_layer_c8 does.  Work items are (token, matrix) with
