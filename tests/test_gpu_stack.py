@@ -251,6 +251,28 @@ def test_one_launch_stack_matches_per_layer_and_oracle(g, oracle, gate_type, exp
     sc_b.close()
 
 
+def test_one_launch_stack_of_every_depth_the_block_holds(g):
+    """64 layers reach every piece of the hand-off block, whose pieces are chosen by where it happens to lie: several scratches at
+    once, each twice (both sets of buffers), against the dispatches per layer."""
+    L = synth.make_layer(2048, 512, 16, 4, synth.IQ3_S, synth.Q8_0, shared=True, layer=360, router_sigma=1.0 / np.sqrt(2048.0))
+    dls, one = _descs(g, [L])
+    arr = (capi.MoeLayer * 64)(*[one[0]] * 64)
+    x = synth.rms_normed(synth.rng_for(SEED, 85), 2048)
+    tr = np.stack([np.random.default_rng(SEED + l).choice(16, size=4, replace=False) for l in range(64)]).astype(np.int32)
+    ref = g.Scratch(2048, 512, 16, 4)
+    scr = [g.Scratch(2048, 512, 16, 4) for _ in range(3)]
+    for trace in (None, tr):
+        want = _run_stack(g, arr, 64, x, trace, ref, PER_LAYER)
+        for turn in range(2):
+            for sc in scr:
+                got = _run_stack(g, arr, 64, x, trace, sc, 0)
+                assert g.same_bits(got[0], want[0]) and g.same_bits(got[1], want[1]), (turn, trace is None)
+                assert np.array_equal(got[2]["ids"], want[2]["ids"])
+    for sc in scr + [ref]:
+        assert capi.load().wd_moe_scratch_status(sc.h) == 0
+        sc.close()
+
+
 # 150 slots hold three tokens' experts (a token's fills run beside the launch of the token before), 100 two tokens'
 # (they wait for it); 320 (layer, expert) pairs compete for them
 @pytest.mark.parametrize("slots", [150, 100], ids=["three-tokens-of-slots", "two-tokens-of-slots"])

@@ -17,6 +17,7 @@ namespace {
 constexpr int kTagRecords = 64;  // one record per layer of a stack (modulo), so that a chain of layers needs no reset in between
 constexpr int kTagRecordsPerPiece = kSidePiece / (kTagCopies * 8 * 4);
 constexpr int kTagUnits = kTagRecords / kTagRecordsPerPiece;  // of two pieces
+constexpr int kHostWords = 48 + 8 * 2 * kHandChunks;
 }  // namespace
 
 struct wd_moe_scratch {
@@ -44,9 +45,9 @@ struct wd_moe_scratch {
     uint32_t *hand = nullptr;             // [n_experts + 2] logits on their way to the selection inside dispatch AB (LayerArgs)
     unsigned long long *trace = nullptr;  // device [3][16][8] time stamps, see wd_moe_scratch_trace
     int trace_wg = 0;
-    int32_t *h_ids = nullptr;             // pinned [48]: [0..15] routed ids for callers that must see them on the host,
+    int32_t *h_ids = nullptr;             // pinned [kHostWords]: [0..15] routed ids for callers that must see them on the host,
                                           // [16] mirror of the status word, written by the resident launch when a wait runs out,
-                                          // [32..47] the selection as dispatch AB reports it (cached_routed_reported)
+                                          // [32..47] the selection as dispatch AB reports it (cached_routed_reported), [48..] votes (side_vote)
     // ids published inside the merged dispatch, kTagRecords records.  sided: kTagRecordsPerPiece records' copies of side 0 and those of side 1 in two
     // pieces of kSidePiece bytes, flip: side 1's first; otherwise [record][kTagCopies][16].
     uint32_t *tagged = nullptr;
@@ -61,7 +62,8 @@ struct wd_moe_scratch {
     unsigned spin_limit = kSpinLimit;
     int compute_units = 256;              // of the device the scratch lives on
     // the resident stack kernel (wd_resident.cuh): hand-off buffers, device copy of the layer descriptors
-    uint8_t *res_block = nullptr;
+    uint8_t *res_block = nullptr, *res_alloc = nullptr;  // (the block begins on a boundary of kSideChunk inside the allocation)
+    unsigned res_flips = 0;
     // Device copies of the layer descriptors of the stacks this scratch has run ([kResMaxLayers], then one ResidentViews
     // each).  A copy is never overwritten: a captured graph keeps the address of the copy it was recorded with.
     struct ResDescSet {
@@ -95,15 +97,12 @@ struct Carver {
 
 namespace {
 
-// A scratch's block: zeros, but for the words that are handed on, which are "not yet" (ones_at .. ones_end, in words).  Then workgroup b < 8 (XCD b mod 8)
-// times round trips of device-scope accesses to the first two pieces at `sided`, its loads and stores leaving the words as they are (votes[b] > 0: the
-// second piece is nearer).
-__global__ __launch_bounds__(256) void k_scratch_init(uint32_t *block, unsigned words, unsigned ones_at, unsigned ones_end, uint32_t *sided, int *votes) {
-    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) block[i] = i >= ones_at && i < ones_end ? kHandEmpty : 0u;
-    if (blockIdx.x >= 8 || threadIdx.x != 0) return;
+// One thread of a workgroup: whether the second of two pieces of kSidePiece bytes is nearer to it than the first (> 0).  Times round trips of
+// device-scope accesses whose loads and stores leave the words as they are (all ones; every workgroup has a line of its own).
+WD_DEV int side_vote(uint32_t *pieces) {
     long long sum = 0;
     for (int turn = 0; turn < 10; ++turn) {
-        uint32_t *p = sided + (turn & 1) * (kSidePiece / 4) + blockIdx.x * 64;
+        uint32_t *p = pieces + (turn & 1) * (kSidePiece / 4) + (blockIdx.x & 7) * 64;
         const long long t0 = clock64();
         __hip_atomic_store(p, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -112,7 +111,23 @@ __global__ __launch_bounds__(256) void k_scratch_init(uint32_t *block, unsigned 
         const long long t = clock64() - t0;
         if (turn >= 2) sum += (turn & 1) ? -t : t;
     }
-    votes[blockIdx.x] = static_cast<int>(sum);
+    return static_cast<int>(sum);
+}
+// (host) From the votes of workgroups 0..7: 1 where the first piece is side 1's.
+int side_flip_of(const int *votes) {
+    int second = 0;  // workgroups that say that the second piece is side 0's
+    for (int g = 0; g < 8; ++g) second += (votes[g] > 0) == (g < 4) ? 1 : 0;
+    return second > 4 ? 1 : 0;
+}
+// A scratch's block: zeros, but for the words that are handed on, which are "not yet" (ones_at .. ones_end, in words).  Workgroups 0..7 vote on
+// the first two pieces at `sided`.
+__global__ __launch_bounds__(256) void k_scratch_init(uint32_t *block, unsigned words, unsigned ones_at, unsigned ones_end, uint32_t *sided, int *votes) {
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) block[i] = i >= ones_at && i < ones_end ? kHandEmpty : 0u;
+    if (blockIdx.x < 8 && threadIdx.x == 0) votes[blockIdx.x] = side_vote(sided);
+}
+// Workgroups 8 q .. 8 q + 7 vote on the first two pieces of chunk q.
+__global__ __launch_bounds__(64) void k_side_votes(uint32_t *base, int *votes) {
+    if (threadIdx.x == 0) votes[blockIdx.x] = side_vote(base + static_cast<size_t>(blockIdx.x >> 3) * (kSideChunk / 4));
 }
 
 }  // namespace
@@ -170,17 +185,16 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
     s->shared_gate = reinterpret_cast<float *>(b + o_sg);
     s->hand = reinterpret_cast<uint32_t *>(b + o_hand);
     uintptr_t side = (reinterpret_cast<uintptr_t>(b + o_side) + 2 * kSidePiece - 1) & ~static_cast<uintptr_t>(2 * kSidePiece - 1);
-    constexpr uintptr_t kChunk = 2u << 20;
-    if (side / kChunk != (side + side_bytes - 1) / kChunk) side = (side / kChunk + 1) * kChunk;
+    if (side / kSideChunk != (side + side_bytes - 1) / kSideChunk) side = (side / kSideChunk + 1) * kSideChunk;
     uint32_t *const units = reinterpret_cast<uint32_t *>(side);
     s->tagged = units + 2 * kSidePiece / 4, s->sided = true;
     s->status = reinterpret_cast<unsigned *>(b + o_status);
-    if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * 48, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(reinterpret_cast<void **>(&s->h_ids), sizeof(int32_t) * kHostWords, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->block);
         delete s;
         return fail(WD_ERR_HIP, "hipHostMalloc MoE scratch ids failed");
     }
-    std::memset(s->h_ids, 0, sizeof(int32_t) * 48);
+    std::memset(s->h_ids, 0, sizeof(int32_t) * kHostWords);
     enqueue(k_scratch_init, dim3(64), dim3(256), 0, nullptr, reinterpret_cast<uint32_t *>(b), static_cast<unsigned>(c.off / 4), static_cast<unsigned>(o_hand / 4),
             static_cast<unsigned>(c.off / 4), units, s->h_ids);
     hipError_t init = hipGetLastError();
@@ -191,11 +205,9 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
         delete s;
         return fail(WD_ERR_HIP, "MoE scratch: the first launch failed: %s", hipGetErrorString(init));
     }
-    int second = 0;  // workgroups that say that the second piece is side 0's
-    for (int g = 0; g < 8; ++g) second += (s->h_ids[g] > 0) == (g < 4) ? 1 : 0;
-    s->flip = second > 4 ? 1 : 0;
+    s->flip = side_flip_of(s->h_ids);
     if (sizeof(uint32_t) * (static_cast<size_t>(n_experts) + 2) <= kSidePiece) s->hand = units + s->flip * (kSidePiece / 4);
-    std::memset(s->h_ids, 0, sizeof(int32_t) * 48);
+    std::memset(s->h_ids, 0, sizeof(int32_t) * kHostWords);
     *out = s;
     return WD_OK;
 }
@@ -206,7 +218,7 @@ int wd_moe_scratch_destroy(wd_moe_scratch *s) {
     (void)hipFree(s->gup);
     (void)hipFree(s->dp);
     (void)hipFree(s->trace);
-    (void)hipFree(s->res_block);
+    (void)hipFree(s->res_alloc);
     for (wd_moe_scratch::ResDescSet &d : s->res_sets) (void)hipFree(d.dev);
     (void)hipHostFree(s->h_ids);
     (void)hipFree(s->pair_dev);
@@ -895,10 +907,23 @@ namespace {
 // The hand-off buffers of the resident stack kernel, allocated on first use.
 int resident_prepare(wd_moe_scratch *s) {
     if (s->res_block) return WD_OK;
-    uint8_t *b = nullptr;
-    WD_HIP(hipMalloc(reinterpret_cast<void **>(&b), kHandBytes));
+    uint8_t *alloc = nullptr;
+    WD_HIP(hipMalloc(reinterpret_cast<void **>(&alloc), kHandBytes + kSideChunk));
+    uint8_t *const b = reinterpret_cast<uint8_t *>((reinterpret_cast<uintptr_t>(alloc) + kSideChunk - 1) & ~static_cast<uintptr_t>(kSideChunk - 1));
     (void)hipMemset(b, 0xff, kHandEpoch);                        // every hand-off word of both sets "not yet written"
     (void)hipMemset(b + kHandEpoch, 0, kHandBytes - kHandEpoch);  // launches finished
+    int *const votes = s->h_ids + 48;
+    std::memset(votes, 0, sizeof(int) * 8 * 2 * kHandChunks);
+    enqueue(k_side_votes, dim3(8 * 2 * kHandChunks), dim3(64), 0, nullptr, reinterpret_cast<uint32_t *>(b), votes);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) {
+        (void)hipFree(alloc);
+        return fail(WD_ERR_HIP, "MoE stack: the hand-off block's first launch failed: %s", hipGetErrorString(e));
+    }
+    s->res_flips = 0;
+    for (int q = 0; q < 2 * kHandChunks; ++q) s->res_flips |= static_cast<unsigned>(side_flip_of(votes + 8 * q)) << q;
+    s->res_alloc = alloc;
     s->res_block = b;
     return WD_OK;
 }
@@ -1013,7 +1038,7 @@ int stack_resident(const wd_moe_layer *layers, int n_layers, float *d_x, float *
         a.rows_trace = slots->rows_trace, a.fill_need = slots->fill_need, a.fill_done = slots->fill_done, a.row_limit = slots->n_slots;
     }
     a.views = reinterpret_cast<const ResidentViews *>(descriptors + kResMaxLayers);
-    a.hand = s->res_block, a.status = s->status, a.spin_limit = s->spin_limit;
+    a.hand = s->res_block, a.side_flips = s->res_flips, a.status = s->status, a.spin_limit = s->spin_limit;
     a.status_host = reinterpret_cast<unsigned *>(s->h_ids + 16);
     a.trace = s->trace, a.trace_wg = s->trace_wg, a.trace_layer = s->trace_layer;
     switch (layers[0].gate_type) {

@@ -90,29 +90,48 @@ struct ResidentViews {
 // Byte offsets inside the hand-off block.
 // What every workgroup needs from every other - four values of the next input, eleven activations - is
 // written by its producer into kResCopies copies, one per group of workgroups (r % kResCopies; on this device the
-// workgroups of a group share an L2), laid out contiguously: the consumers of a group fetch their copy with coalesced
-// requests, and a line is polled from one L2 only.
+// workgroups of a group share an L2): the consumers of a group fetch their copy with coalesced requests, and a line is polled from one
+// L2 only.  Every word lies on its readers' side of the device (see kSidePiece): the records that workgroup 0 gathers on side 0, a copy on
+// the side of its XCD, half of the ids' replicas on either.  Memory changes sides every kSidePiece bytes: the copies' pieces follow each other and
+// workgroup r reads the one of a pair that is on its side (own_copy); bit q of ResidentArgs::side_flips: in the q-th 2 MB of the block
+// the first piece of two is side 1's.  (48 layers, IQ3_S / Q8_0 rows with the router's ids, IQ3_S with a routing trace, us: copies wherever they fall 780 / 797 /
+// 526, every word on its readers' side 760 / 759 / 525, every word on the other side 806 / 816 / 536.)
 constexpr int kResCopies = 8;
 constexpr unsigned kRecBytes = 16;        // a logit record: word 0 the router logit of row r, word 1 (workgroup 1) the shared expert's gate logit
-constexpr unsigned kHandRec = 0;                                                        // [layers][512] records, gathered by workgroup 0 only
+constexpr unsigned kHandRec = 0;                                                        // [layers][2] pieces, one of them 512 records, gathered by workgroup 0 only
 constexpr unsigned kXcStride = 16;        // bytes from one workgroup's four values of a layer input to the next one's
-constexpr unsigned kXcBytes = kXcStride * kResWgs;                                     // one copy
-constexpr unsigned kHandXc = kHandRec + kRecBytes * kResWgs * kResMaxLayers;            // [layers][copies][512] pieces of four f32: layer inputs
+constexpr unsigned kHandXc = kHandRec + 2u * kSidePiece * kResMaxLayers;               // [layers][copies] pieces of [512] x four f32: layer inputs
 constexpr unsigned kAcRec = 48;                                                        // bytes of a workgroup's activations: slots 0..10, a zero
-constexpr unsigned kAcBytes = kAcRec * kResWgs;                                        // 24 KB per copy
-constexpr unsigned kHandAc = kHandXc + kXcBytes * kResMaxLayers * kResCopies;          // f32 [layers][copies][512][12] activations
+constexpr unsigned kAcBytes = kAcRec * kResWgs;                                        // 24 KB per copy: three pieces
+constexpr unsigned kHandAc = kHandXc + kSidePiece * kResMaxLayers * kResCopies;        // f32 [layers][3][copies] pieces: a copy's three are [512][12] activations
 constexpr int kResIdCopies = 16;          // replicas of the published ids (pollers spread over lines)
-constexpr unsigned kHandIdh = kHandAc + kAcBytes * kResMaxLayers * kResCopies;         // u32 [layers][replicas][16] selected ids
-constexpr unsigned kHandWh = kHandIdh + 4u * kResMaxLayers * kResIdCopies * 16;        // u32 [layers][16] router weights, [15] the shared gate
-constexpr unsigned kHandSet = kHandWh + 4u * kResMaxLayers * 16;             // bytes of one set of hand-off buffers
-// The block holds two such sets and the number of launches finished.  Launch e works in set e % 2 and, layer by layer and
+constexpr int kIdhPerPiece = kSidePiece / (kResIdCopies * 32);
+constexpr unsigned kHandIdh = kHandAc + kAcBytes * kResMaxLayers * kResCopies;         // [layers / kIdhPerPiece][2] pieces of u32 [layers][replicas / 2][16] selected ids
+constexpr unsigned kHandWh = kHandIdh + 2u * kSidePiece * (kResMaxLayers / kIdhPerPiece);  // u32 [layers][16] router weights, [15] the shared gate
+constexpr unsigned kHandSet = (kHandWh + 4u * kResMaxLayers * 16 + kSideChunk - 1) & ~(kSideChunk - 1);  // bytes of one set of hand-off buffers
+// The block (on a boundary of kSideChunk) holds two such sets and the number of launches finished.  Launch e works in set e % 2 and, layer by layer and
 // off its critical path, puts set (e + 1) % 2 back to "not yet written": no launch has to clean up behind itself.
 constexpr unsigned kHandEpoch = 2u * kHandSet;
 constexpr unsigned kHandBytes = kHandEpoch + 256u;
-static_assert(kHandXc % 128 == 0 && kHandAc % 128 == 0 && kHandIdh % 128 == 0 && kHandWh % 16 == 0 && kHandSet % 128 == 0, "hand-off block alignment");
-WD_DEV unsigned rec_off(int l, int wg) { return kHandRec + static_cast<unsigned>(l * kResWgs + wg) * kRecBytes; }
-WD_DEV unsigned xc_off(int l, int copy) { return kHandXc + static_cast<unsigned>(l * kResCopies + copy) * kXcBytes; }
-WD_DEV unsigned ac_off(int l, int copy) { return kHandAc + static_cast<unsigned>(l * kResCopies + copy) * kAcBytes; }
+constexpr int kHandChunks = static_cast<int>(kHandSet / kSideChunk);  // of one set
+static_assert(kRecBytes * kResWgs == kSidePiece && kXcStride * kResWgs == kSidePiece && kAcBytes == 3 * kSidePiece && kResMaxLayers % kIdhPerPiece == 0 && 2 * kHandChunks <= 32,
+              "hand-off block pieces");
+// flips: those of the set's chunks.  1: in the chunk of `off` the first piece of two is side 1's.
+WD_DEV unsigned side_flip(unsigned flips, unsigned off) { return (flips >> (off / kSideChunk)) & 1u; }
+WD_DEV unsigned rec_off(unsigned flips, int l, int wg) {
+    const unsigned at = kHandRec + 2u * kSidePiece * l;
+    return at + kSidePiece * side_flip(flips, at) + kRecBytes * wg;
+}
+// The layer's copies, one piece after the other; the one that workgroup r reads (its side's of the pair of XCDs c and c + 4).
+WD_DEV unsigned xc_off(int l) { return kHandXc + static_cast<unsigned>(kResCopies * kSidePiece) * l; }
+WD_DEV unsigned own_copy(unsigned flips, unsigned at, int r) { return kSidePiece * (2u * (r & 3) + (((r >> 2) & 1u) ^ side_flip(flips, at))); }
+// The layer's activations: the copies' first pieces one after the other, their second, their third; byte o of a copy lies ac_byte(o) behind its first piece.
+WD_DEV unsigned ac_off(int l) { return kHandAc + kAcBytes * kResCopies * l; }
+WD_DEV unsigned ac_byte(unsigned o) { return o + (o / kSidePiece) * ((kResCopies - 1) * kSidePiece); }
+WD_DEV unsigned idh_off(unsigned flips, int l, int side) {
+    const unsigned at = kHandIdh + 2u * kSidePiece * (l / kIdhPerPiece);
+    return at + kSidePiece * (side ^ side_flip(flips, at)) + (kSidePiece / kIdhPerPiece) * (l % kIdhPerPiece);
+}
 
 struct ResidentArgs {
     const ResidentLayer *layers;  // device array [n_layers]
@@ -132,7 +151,8 @@ struct ResidentArgs {
     const uint32_t *fill_done;    // [n_layers], written by the fills while the launch runs
     unsigned row_limit;           // ids (or slot numbers) that address the tensors are below this
     const struct ResidentViews *views;  // device: where the last layer's values go
-    uint8_t *hand;   // the hand-off block (kHand* offsets below)
+    uint8_t *hand;   // the hand-off block (kHand* offsets above)
+    unsigned side_flips;  // of the chunks of both sets
     unsigned *status;
     unsigned *status_host;        // null, or the status word's mirror in pinned host memory (the host reads it without a synchronisation)
     unsigned spin_limit;
@@ -345,10 +365,15 @@ WD_DEV int fresh_s(int v) {  // v is the same in every lane
 }
 
 // What a wave is and where it works.  slot: 0..9 routed rung, 10 the shared expert; -1 for the router wave.
+struct ResHand {
+    __amdgpu_buffer_rsrc_t b;  // a set of hand-off buffers
+    unsigned flips;            // of its chunks
+};
 struct ResCtx {
     uint8_t *lds;
     int r, lane, wave, slot;
     __amdgpu_buffer_rsrc_t hb;  // the hand-off block
+    unsigned flips;
     WD_DEV float *xt() const { return reinterpret_cast<float *>(lds + kResLdsXs); }
     WD_DEV float x_at(int e) const { return xt()[(e & 31) * kResXtRow + (e >> 5)]; }
     WD_DEV int8_t *xq() const { return reinterpret_cast<int8_t *>(lds + kResLdsXq); }
@@ -371,13 +396,13 @@ WD_DEV int fresh_lane() {
     const unsigned all = static_cast<unsigned>(fresh_s(-1));
     return static_cast<int>(__builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0u)));
 }
-WD_DEV ResCtx res_ctx(uint8_t *base, int r, int lane, int wave, int slot, __amdgpu_buffer_rsrc_t hb) {
+WD_DEV ResCtx res_ctx(uint8_t *base, int r, int lane, int wave, int slot, const ResHand &hand) {
     ResCtx c;
     c.lds = base + fresh_s(0);
     (void)lane;
     c.lane = fresh_lane();
     c.r = fresh_s(r), c.wave = fresh_s(wave), c.slot = fresh_s(slot);
-    c.hb = hb;
+    c.hb = hand.b, c.flips = hand.flips;
     return c;
 }
 // Time stamp i of this wave in layer l.  trace_wg >= 0: every wave of that workgroup ([12][16] stamps);
@@ -430,14 +455,14 @@ WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool has
     if (wave == 0 && lane < 3 * kResCopies) {  // piece lane % 3 of the workgroup's 48 bytes, to copy lane / 3
         const int piece = lane % 3, copy = lane / 3;
         const float4 p = reinterpret_cast<const float4 *>(c.actv())[piece];
-        hand_store16(c.hb, ac_off(l, copy) + kAcRec * c.r + 16u * piece, make_uint4(hand_word(p.x), hand_word(p.y), hand_word(p.z), hand_word(p.w)));
+        hand_store16(c.hb, ac_off(l) + kSidePiece * copy + ac_byte(kAcRec * c.r + 16u * piece), make_uint4(hand_word(p.x), hand_word(p.y), hand_word(p.z), hand_word(p.w)));
     }
     res_mark<STAMPS>(a, c, l, 10);
     early();
     if (wave < 8) {  // the group's copy, three 16-byte words per lane: word w is piece w % 3 of workgroup w / 3
         const int i = wave * 64 + lane;
-        const unsigned base = ac_off(l, c.r & (kResCopies - 1)) + 16u * i;
-        const unsigned off[3] = {base, base + 16u * 512, base + 16u * 1024};
+        const unsigned base = ac_off(l) + own_copy(c.flips, ac_off(l), c.r) + 16u * i;
+        const unsigned off[3] = {base, base + kResCopies * kSidePiece, base + 2u * kResCopies * kSidePiece};
         uint4 v[3];
         {
             // the first third alone until it is complete, then the rest: by then most of it is there, and a third of the
@@ -498,7 +523,7 @@ WD_DEV void res_down(const ResidentArgs &a, const ResCtx &c, int l, Q8CoalRaw<0,
 // both, chosen at run time, costs the compiler's merging of registers that either form defines in its own place).
 template <int TYPE, bool STAMPS, bool TRACED>
 WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, int lane0, int wave0, int slot0,
-                            __amdgpu_buffer_rsrc_t hb, bool &dead) {
+                            const ResHand &hand, bool &dead) {
     // TYPE 21 / 22: gate/up rows of eight IQ3_S / IQ2_S super-blocks against the Q8_K form of the input; TYPE 8: Q8_0 rows,
     // one 34-byte block per lane, against its Q8_0 form (the row routine of the shared expert's wave).
     constexpr bool kQ8 = TYPE == 8;
@@ -562,7 +587,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         draw_asked = true;
     }
     for (int l = 0; l < a.n_layers; ++l) {
-        const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, slot0, hb);
+        const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, slot0, hand);
         const int r = c.r, lane = c.lane, wave = c.wave, rung = c.slot;
         // (the tables at an LDS address written out as a number - the kernel has no LDS but its dynamic block, which
         // therefore starts at 0, as the kernel checks when it begins)
@@ -592,7 +617,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
                 // (the other waves of the workgroup come here while rung 0 still folds the previous layer: nothing
                 // can have arrived yet)
                 if (rung != 0 && !decoded) __builtin_amdgcn_s_sleep(kResSleepFold);
-                const unsigned off[1] = {xc_off(l, r & (kResCopies - 1)) + kXcStride * i};
+                const unsigned off[1] = {xc_off(l) + own_copy(c.flips, xc_off(l), r) + kXcStride * i};
                 uint4 v[1];
                 hand_wait16<1>(a, c.hb, off, true, v, dead);
                 xv = make_float4(bits_f(v[0].x), bits_f(v[0].y), bits_f(v[0].z), bits_f(v[0].w));
@@ -615,7 +640,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         res_mark<STAMPS>(a, c, l, 2);
         const float res_pre = c.x_at(4 * r + (lane & 3));  // (rung 0 adds the layer's output to these)
         if (!traced && on) {  // the id this rung works on, from one of the replicas workgroup 0 publishes
-            e = hand_wait4(a, c.hb, kHandIdh + static_cast<unsigned>(((l * kResIdCopies + (r & (kResIdCopies - 1))) * 16 + rung) * 4), true, dead);
+            e = hand_wait4(a, c.hb, idh_off(c.flips, l, (r >> 2) & 1) + 64u * ((r >> 3) & (kResIdCopies / 2 - 1)) + 4u * rung, true, dead);
             e = expert_in_range(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(e)));
             gate_up_rows(gate_base, up_base, e, r, lane);
         }
@@ -751,7 +776,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             } else {
                 const uint4 piece = make_uint4(hand_word(readlane_f(xn, 0)), hand_word(readlane_f(xn, 1)), hand_word(readlane_f(xn, 2)),
                                                hand_word(readlane_f(xn, 3)));
-                if (lane < kResCopies) hand_store16(c.hb, xc_off(l + 1, lane) + kXcStride * r, piece);
+                if (lane < kResCopies) hand_store16(c.hb, xc_off(l + 1) + kSidePiece * lane + kXcStride * r, piece);
             }
             res_mark<STAMPS>(a, c, l, 9);
             if (r != 0) __builtin_amdgcn_s_setprio(0);
@@ -774,7 +799,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
 // ---- the shared expert's wave ------------------------------------------------------------------------------------
 template <bool STAMPS>
 WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, int lane0, int wave0,
-                            __amdgpu_buffer_rsrc_t hb, bool &dead) {
+                            const ResHand &hand, bool &dead) {
     Q8Block gb[2];
     Q8CoalRaw<0, 16> draw;
     auto fetch = [&](const ResidentLayer *L, int r, int lane) {
@@ -785,7 +810,7 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
     const bool traced = a.ids_trace != nullptr;
     if (a.shared) fetch(a.layers, r0, lane0);
     for (int l = 0; l < a.n_layers; ++l) {
-        const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, kResSharedSlot, hb);
+        const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, kResSharedSlot, hand);
         const int r = c.r, lane = c.lane;
         const bool with_shared = fresh_s(a.shared) != 0;  // (a scalar of this layer, not a vector register kept for the launch)
         __syncthreads();  // B1
@@ -813,7 +838,7 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         auto gather_logits = [&](bool patient) {
             uint32_t lb[8];
             const unsigned all_in = 11u * static_cast<unsigned>(l + 1);
-            const bool got = hand_wait4<8>(a, c.hb, rec_off(l, lane), 64u * kRecBytes, want, lb, dead, [&] {
+            const bool got = hand_wait4<8>(a, c.hb, rec_off(c.flips, l, lane), 64u * kRecBytes, want, lb, dead, [&] {
                 return !patient && __hip_atomic_load(c.arrived(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= all_in;
             });
 #pragma unroll
@@ -856,11 +881,11 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
 // the fold at the end of the layer needs - follow behind the next barrier.  With a routing trace nobody waits for the
 // ids, and workgroup 0 must not hold up its own rungs: ranks and weights are then taken between the barriers of the
 // activation exchange, while the rungs wait for the activations.
-// The wave also puts the other set of hand-off buffers (`ob`) back to "not yet written": in layer l this workgroup's
+// The wave also puts the other set of hand-off buffers (`other`) back to "not yet written": in layer l this workgroup's
 // share of layers l, l + n, l + 2n, ... of that set (all kResMaxLayers layers, whatever the launch that wrote them used).
 template <bool STAMPS>
 WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, int lane0, int wave0,
-                            __amdgpu_buffer_rsrc_t hb, __amdgpu_buffer_rsrc_t ob, bool &dead) {
+                            const ResHand &hand, const ResHand &other, bool &dead) {
     const bool has_row = r0 < a.E;
     const bool traced = a.ids_trace != nullptr;
     // The wave's few instructions are on the critical path of the whole grid (the logit; in workgroup 0 the ranks), while
@@ -871,7 +896,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
     float wv[32];
     res_router_fetch(res_field(&a.layers->router) + static_cast<size_t>(has_row ? r0 : 0) * kResH, wv, lane0);
     for (int l = 0; l < a.n_layers; ++l) {
-        const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, -1, hb);
+        const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, -1, hand);
         const int r = c.r, lane = c.lane;
         const bool last = l == a.n_layers - 1;
         const ResidentLayer *L = a.layers + l;
@@ -887,7 +912,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         res_mark<STAMPS>(a, c, l, 2);
         {
             const float s = res_router_dot(wv, c.xt(), lane);
-            if (has_row && lane == 32) hand_store4(c.hb, rec_off(l, r), hand_word(s));
+            if (has_row && lane == 32) hand_store4(c.hb, rec_off(c.flips, l, r), hand_word(s));
             res_mark<STAMPS>(a, c, l, 3);
         }
         // (before the selection's values exist: this dot and they together would not fit the registers)
@@ -895,7 +920,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             float gw[32];  // (an array of its own: the router row's registers keep one definition per layer)
             res_router_fetch(res_field(&L->sh_inp), gw, lane);
             const float s = res_router_dot(gw, c.xt(), lane);
-            if (lane == 32) hand_store4(c.hb, rec_off(l, 1) + 4u, hand_word(s));
+            if (lane == 32) hand_store4(c.hb, rec_off(c.flips, l, 1) + 4u, hand_word(s));
         }
         bool want[8];
         float lv[8];
@@ -908,7 +933,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         auto gather_logits = [&](bool patient) {
             uint32_t lb[8];
             const unsigned all_in = 11u * static_cast<unsigned>(l + 1);
-            const bool got = hand_wait4<8>(a, c.hb, rec_off(l, lane), 64u * kRecBytes, want, lb, dead, [&] {
+            const bool got = hand_wait4<8>(a, c.hb, rec_off(c.flips, l, lane), 64u * kRecBytes, want, lb, dead, [&] {
                 return !patient && __hip_atomic_load(c.arrived(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= all_in;
             });
 #pragma unroll
@@ -921,8 +946,8 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             wave_lds_fence();
             const int j = lane & 15;
 #pragma unroll
-            for (int c0 = 0; c0 < kResIdCopies; c0 += 4)
-                if (j < a.k) hand_store4(c.hb, kHandIdh + static_cast<unsigned>(((l * kResIdCopies + c0 + (lane >> 4)) * 16 + j) * 4), static_cast<uint32_t>(lds_ids[j]));
+            for (int c0 = 0; c0 < kResIdCopies; c0 += 4)  // (the sides in turn)
+                if (j < a.k) hand_store4(c.hb, idh_off(c.flips, l, (c0 >> 2) & 1) + 64u * ((c0 >> 3) * 4 + (lane >> 4)) + 4u * j, static_cast<uint32_t>(lds_ids[j]));
             res_mark<STAMPS>(a, c, l, 13);
         };
         // what every fold needs: the weights and the shared expert's gate; the last layer's values for the caller
@@ -941,7 +966,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
                     if (want[j]) a.views->logits[64 * j + lane] = lv[j];
             }
             if (a.shared) {
-                const float g = bits_f(hand_wait4(a, c.hb, rec_off(l, 1) + 4u, true, dead));
+                const float g = bits_f(hand_wait4(a, c.hb, rec_off(c.flips, l, 1) + 4u, true, dead));
                 const float sg = sigmoid_ggml(g);
                 if (lane == 0) {
                     hand_store4(c.hb, kHandWh + static_cast<unsigned>((l * 16 + kResGateSlot) * 4), hand_word(sg));
@@ -978,12 +1003,12 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         for (int ll = l; ll < kResMaxLayers; ll += a.n_layers) {
             const uint4 empty4 = make_uint4(kResEmpty, kResEmpty, kResEmpty, kResEmpty);
             // lane 0 the workgroup's logit record, 8 lanes its 128 bytes of the layer's input copies, 24 its 384 bytes of the activations'
-            const unsigned off = lane < 8 ? rec_off(ll, r)
-                               : lane < 16 ? xc_off(ll, 0) + kXcStride * (8 * r + lane - 8) : ac_off(ll, 0) + 16u * (24 * r + lane - 16);
-            if (lane == 0 || (lane >= 8 && lane < 40)) hand_store16(ob, off, empty4);
+            const unsigned off = lane < 8 ? rec_off(other.flips, ll, r)
+                               : lane < 16 ? xc_off(ll) + kXcStride * (8 * r + lane - 8) : ac_off(ll) + 16u * (24 * r + lane - 16);
+            if (lane == 0 || (lane >= 8 && lane < 40)) hand_store16(other.b, off, empty4);
             if (r == 0) {
-                hand_store16(ob, kHandIdh + static_cast<unsigned>(ll * kResIdCopies * 64 + 16 * lane), empty4);
-                if (lane < 4) hand_store16(ob, kHandWh + static_cast<unsigned>(ll * 64 + 16 * lane), empty4);
+                hand_store16(other.b, idh_off(other.flips, ll, lane >> 5) + 16u * (lane & 31), empty4);
+                if (lane < 4) hand_store16(other.b, kHandWh + static_cast<unsigned>(ll * 64 + 16 * lane), empty4);
             }
         }
         // The exchange of the activations: this wave (never one of waves 0..7) only keeps its three barriers company.
@@ -1030,7 +1055,9 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(6, 
     }
     const unsigned epoch = __hip_atomic_load(reinterpret_cast<const unsigned *>(a.hand + kHandEpoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned set_base = (epoch & 1u) ? kHandSet : 0u;
-    const __amdgpu_buffer_rsrc_t hb = hand_rsrc(a.hand + set_base, kHandSet), ob = hand_rsrc(a.hand + (kHandSet - set_base), kHandSet);
+    const unsigned odd = epoch & 1u;
+    const ResHand hand{hand_rsrc(a.hand + set_base, kHandSet), a.side_flips >> (odd ? kHandChunks : 0)};
+    const ResHand other{hand_rsrc(a.hand + (kHandSet - set_base), kHandSet), a.side_flips >> (odd ? 0 : kHandChunks)};
     stage_tables<TYPE == 21, TYPE == 22>(*reinterpret_cast<IqTables *>(lds_res + kResLdsTables), threadIdx.x, kResThreads);
 
     // Roles.  The twelve waves of a workgroup sit three to a SIMD (waves w, w + 4, w + 8 share one), and two
@@ -1072,12 +1099,12 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(6, 
     if (r == 0) __builtin_amdgcn_s_setprio(kResPrioWg0);
     bool dead = false;
     if (slot < 0)
-        res_router_role<STAMPS>(a, lds_res, r, fresh_lane(), wave, hb, ob, dead);
+        res_router_role<STAMPS>(a, lds_res, r, fresh_lane(), wave, hand, other, dead);
     else if (slot == kResSharedSlot)
-        res_shared_role<STAMPS>(a, lds_res, r, fresh_lane(), wave, hb, dead);
+        res_shared_role<STAMPS>(a, lds_res, r, fresh_lane(), wave, hand, dead);
     else
-        if (a.ids_trace) res_routed_role<TYPE, STAMPS, true>(a, lds_res, r, fresh_lane(), wave, slot, hb, dead);
-        else res_routed_role<TYPE, STAMPS, false>(a, lds_res, r, fresh_lane(), wave, slot, hb, dead);
+        if (a.ids_trace) res_routed_role<TYPE, STAMPS, true>(a, lds_res, r, fresh_lane(), wave, slot, hand, dead);
+        else res_routed_role<TYPE, STAMPS, false>(a, lds_res, r, fresh_lane(), wave, slot, hand, dead);
 
     // the next launch takes the other set (workgroup 0 can only get here after every workgroup has read the number)
     if (r == 0 && wave == 0 && fresh_lane() == 0 && !dead)
