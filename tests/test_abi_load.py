@@ -59,3 +59,58 @@ def test_profiler_switched_off_touches_nothing():
     buf = C.create_string_buffer(need + 1)
     assert lib.wd_profile_report(buf, need + 1) == need
     assert buf.value == b"[moe-profile] tokens=0 unit=ms_per_token\n"
+
+
+SPAN = (C.c_uint8 * 4096)()
+CALLS = [
+    ("wd_q8_k_quantize_f32", None, 100, None, None, None, None), ("wd_q8_0_quantize_f32", C.c_void_p(8), 33, SPAN, 8, None),
+    ("wd_topk_softmax", None, 12, 2, 1.0, None, None, None), ("wd_topk_softmax", None, 12, 2, 1, None, None, None),
+    ("wd_topk_softmax", None, 12, 2, "1", None, None, None), ("wd_topk_softmax", None, 12.0, 2, 1.0, None, None, None),
+    ("wd_topk_softmax", None, (1 << 32) + 12, -5, 1.0, None, None, None), ("wd_topk_softmax", True, 12, True, 1.0, None, -1, 1 << 70),
+    ("wd_topk_softmax", C.byref(SPAN), C.c_int(12), 2, C.c_float(1), C.POINTER(C.c_uint8)(), None, None),
+    ("wd_topk_softmax", b"x", 12, 2, 1.0, "x", None, None), ("wd_topk_softmax", None, 12, 2, 1.0, None, None),
+    ("wd_topk_softmax", None, 12, 2, 1.0, None, None, None, None), ("wd_topk_softmax",), ("wd_no_such_thing", 1), (1, 2), (),
+    ("wd_gemv_q8_k_f32", synth.Q8_0, C.c_void_p(8), 4, 256, None, None, None, None, None),
+    ("wd_gemv_q8_0_f32", synth.Q8_0, SPAN, 0, 256, SPAN, None, 8, None, None), ("wd_gemv_q8_0_f32", synth.Q8_0, 1.5, 0, 256, SPAN, None, 8, None, None),
+    ("wd_moe_scratch_create", C.byref(C.c_void_p()), 100, 512, 64, 8),
+]
+
+
+@pytest.mark.parametrize("args", CALLS, ids=lambda a: "-".join(str(x)[:8] for x in a[:1]) or "nothing")
+def test_calls_without_ctypes_answer_as_with_it(args):
+    """Every form of an argument is taken, or refused with the same words, on both ways to an entry point."""
+    assert capi._fast is not None and capi.call is capi._fast.call, "the extension is not built"
+    capi.load()
+
+    def outcome(call):
+        try:
+            return call(*args)
+        except Exception as e:   # noqa: BLE001 (whatever it is has to be alike)
+            return type(e), str(e).replace("_call", "call")
+    want = outcome(capi._call)
+    assert want is not None and outcome(capi.call) == want
+
+
+def test_arguments_arrive_as_with_ctypes():
+    """What each form of an argument becomes: entry points that hand their own arguments back."""
+    seen = []
+    kind = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_void_p, C.c_void_p, C.c_void_p)
+    stand_in = kind(lambda *a: seen.append(a) or 0)
+    lib = capi.load()
+    true_fn = lib.wd_topk_softmax
+    rows = [(None, 8, 2, 1.5, SPAN, C.c_void_p(), C.c_void_p(77)), ((1 << 64) - 8, -3, (1 << 32) + 5, -0.0, True, -1, 1 << 63),
+            (0, 2**31, -2**31, 1e300, None, (1 << 64) + 9, (C.c_void_p * 2)())]
+    try:
+        capi._fast.prepare(capi._call, capi.check, C.c_void_p, C.Array)
+        capi._fast.bind("wd_topk_softmax", C.cast(stand_in, C.c_void_p).value)
+        for r in rows:
+            assert capi.call("wd_topk_softmax", *r) is None
+            stand_in.argtypes = true_fn.argtypes
+            stand_in(*r)
+            assert repr(seen[-1]) == repr(seen[-2])
+        with pytest.raises(ValueError):
+            capi._fast.bind("wd_topk_softmax", 8)
+    finally:
+        capi._fast.prepare(capi._call, capi.check, C.c_void_p, C.Array)
+        for name in capi._fast.names():
+            capi._fast.bind(name, C.cast(getattr(lib, name), C.c_void_p).value)

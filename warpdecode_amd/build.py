@@ -2,10 +2,12 @@
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libwarpdecode_amd.so")
+FAST = os.path.join(HERE, "_fast.so")   # capi.call for the stand-alone operators (csrc/wd_python.cpp)
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -17,6 +19,11 @@ FLAGS = [
 
 def build(verbose=False):
     cmd = ["hipcc"] + FLAGS + ["-o", LIB, os.path.join(CSRC, "wd_lib.hip")]
+    if verbose:
+        print(" ".join(cmd))
+    subprocess.check_call(cmd)
+    cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-Wextra", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "wd_python.cpp"), "-o", FAST]
     if verbose:
         print(" ".join(cmd))
     subprocess.check_call(cmd)

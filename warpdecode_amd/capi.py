@@ -8,6 +8,11 @@ import ctypes as C
 import os
 import re
 
+try:
+    from . import _fast
+except ImportError:    # not built: every call goes through ctypes
+    _fast = None
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libwarpdecode_amd.so")
 HEADER = os.path.join(os.path.dirname(HERE), "include", "warpdecode_amd.h")
@@ -189,6 +194,11 @@ def load():
                     raise WdError("libwarpdecode_amd.so does not export " + name)
                 continue
             fn.restype, fn.argtypes = res, args
+        if _fast:
+            for name in _fast.names():
+                if not set(_SIGS[name][1]) <= {vp, i32, f32, sz}:
+                    raise WdError("_fast does not take the arguments of " + name)
+                _fast.bind(name, C.cast(getattr(lib, name), vp).value)
         _lib = lib
     return _lib
 
@@ -201,10 +211,19 @@ def check(rc):
 _fns = {}     # bound functions by name: a decode step makes hundreds of calls of a few microseconds each
 
 
-def call(name, *args):
+def _call(name, *args):
     fn = _fns.get(name)
     if fn is None:
         fn = _fns[name] = getattr(load(), name)
     rc = fn(*args)
     if rc:
         check(rc)
+
+
+# call(name, *args): the entry point of that name, WdError where it reports an error.  The stand-alone operators go
+# without ctypes where the extension is built (from the first call on, which loads the library).
+if _fast:
+    _fast.prepare(_call, check, vp, C.Array)
+    call = _fast.call
+else:
+    call = _call
