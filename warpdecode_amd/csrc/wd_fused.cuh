@@ -65,14 +65,18 @@ constexpr uint32_t kTagInvalid = 0xffffffffu;
 // Sides.  A word that workgroups hand on has a home in one half of the device's memory, and the XCDs of that half reach it sooner: a device-scope
 // load that misses the L2 takes 350 to 450 clocks near its home and 580 to 700 from the other half (stores 370 to 500 and 600 to 760), a word from
 // XCD 0 to XCD 1 360 ns by way of the near half and 575 by the far one.  Memory alternates between the halves in pieces of kSidePiece bytes; which
-// of two neighbours is whose is measured when a scratch is made (side_vote).  Words lie on their readers' side: workgroup b runs on XCD b mod 8,
-// XCDs 0..3 are side 0, the others side 1.
+// of two neighbours is whose is measured when a scratch is made (side_vote).  Words lie on their readers' side: XCDs 0..3 are side 0, the others
+// side 1; workgroup b runs on XCD b mod 8 in the queues that begin at XCD 0.
 constexpr int kSidePiece = 8192;
 constexpr unsigned kSideChunk = 2u << 20;  // within which the halves keep their order
 WD_DEV int block_side() { return static_cast<int>((blockIdx.x >> 2) & 1u); }
+// Where a reader may choose among copies it goes by the XCD that it does run on (HW_REG XCC_ID): block 0 of a dispatch is on the XCD at which its
+// hardware queue begins, 0 for one stream and 7 for another.
+WD_DEV unsigned xcc_id() { return static_cast<unsigned>(__builtin_amdgcn_s_getreg(20 | (3 << 11))) & 7u; }
+WD_DEV int xcc_side() { return static_cast<int>(xcc_id() >> 2); }
 // The replica of the published ids that workgroup `wg` of the waiting ones polls.
 WD_DEV const uint32_t *tag_copy(const uint32_t *tagged, int tag_side, int wg) {
-    return tagged + (block_side() ? tag_side : 0) + ((wg >> 3) & (kTagCopies / 2 - 1)) * 16;
+    return tagged + (xcc_side() ? tag_side : 0) + ((wg >> 3) & (kTagCopies / 2 - 1)) * 16;
 }
 constexpr unsigned kSpinLimit = 1u << 16;  // default number of polls before a wait gives up (tens of milliseconds; a wait lasts microseconds)
 

@@ -97,7 +97,7 @@ struct Carver {
 
 namespace {
 
-// One thread of a workgroup: whether the second of two pieces of kSidePiece bytes is nearer to it than the first (> 0).  Times round trips of
+// One thread of a workgroup: whether the second of two pieces of kSidePiece bytes is nearer to side 0 than the first (> 0).  Times round trips of
 // device-scope accesses whose loads and stores leave the words as they are (all ones; every workgroup has a line of its own).
 WD_DEV int side_vote(uint32_t *pieces) {
     long long sum = 0;
@@ -111,12 +111,12 @@ WD_DEV int side_vote(uint32_t *pieces) {
         const long long t = clock64() - t0;
         if (turn >= 2) sum += (turn & 1) ? -t : t;
     }
-    return static_cast<int>(sum);
+    return static_cast<int>(xcc_side() ? -sum : sum);
 }
 // (host) From the votes of workgroups 0..7: 1 where the first piece is side 1's.
 int side_flip_of(const int *votes) {
     int second = 0;  // workgroups that say that the second piece is side 0's
-    for (int g = 0; g < 8; ++g) second += (votes[g] > 0) == (g < 4) ? 1 : 0;
+    for (int g = 0; g < 8; ++g) second += votes[g] > 0 ? 1 : 0;
     return second > 4 ? 1 : 0;
 }
 // A scratch's block: zeros, but for the words that are handed on, which are "not yet" (ones_at .. ones_end, in words).  Workgroups 0..7 vote on
@@ -124,6 +124,13 @@ int side_flip_of(const int *votes) {
 __global__ __launch_bounds__(256) void k_scratch_init(uint32_t *block, unsigned words, unsigned ones_at, unsigned ones_end, uint32_t *sided, int *votes) {
     for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) block[i] = i >= ones_at && i < ones_end ? kHandEmpty : 0u;
     if (blockIdx.x < 8 && threadIdx.x == 0) votes[blockIdx.x] = side_vote(sided);
+}
+// The resident stack's hand-off block: every word of both sets "not yet written", no launch finished.
+__global__ __launch_bounds__(256) void k_hand_block_init(uint4 *block) {
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < kHandBytes / 16; i += gridDim.x * 256) {
+        const uint32_t v = i < kHandEpoch / 16 ? kHandEmpty : 0u;
+        block[i] = make_uint4(v, v, v, v);
+    }
 }
 // Workgroups 8 q .. 8 q + 7 vote on the first two pieces of chunk q.
 __global__ __launch_bounds__(64) void k_side_votes(uint32_t *base, int *votes) {
@@ -621,6 +628,7 @@ int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s
     // where that saves a round of the loop.  us per layer, cut by both / by the router's / by neither: 2560 / 640 IQ2_S with a shared expert, 800 items, 24.3 /
     // 23.8 / 24.0 (a workgroup for every item 26.0); 3328 / 864 Q8_0 with one, 972, 31.6 / 28.7 / 28.8; 2048 / 992 Q8_0 with one, 1240, 24.5 / 22.7 /
     // 23.1; without one 1536 / 832 IQ2_S, 936, 18.0 / 18.0 / 18.4, and 4096 / 1536, 1536 items in three rounds / three / two, 40.0 / 40.0 / 39.3.
+    // (Rows of two waves, beyond 2048 columns, count as one: the figures above are with that.)
     const int capacity = 3 * s->compute_units, router_places = (router_rows_n + 7) / 8;
     auto rounds = [&](int wgs) { return (m.n_routed_items + wgs - 1) / wgs; };
     // (The loop that runs two per compute unit, kAbPerCu, takes all of its places: with the shared expert's workgroups counted among
@@ -910,10 +918,9 @@ int resident_prepare(wd_moe_scratch *s) {
     uint8_t *alloc = nullptr;
     WD_HIP(hipMalloc(reinterpret_cast<void **>(&alloc), kHandBytes + kSideChunk));
     uint8_t *const b = reinterpret_cast<uint8_t *>((reinterpret_cast<uintptr_t>(alloc) + kSideChunk - 1) & ~static_cast<uintptr_t>(kSideChunk - 1));
-    (void)hipMemset(b, 0xff, kHandEpoch);                        // every hand-off word of both sets "not yet written"
-    (void)hipMemset(b + kHandEpoch, 0, kHandBytes - kHandEpoch);  // launches finished
     int *const votes = s->h_ids + 48;
     std::memset(votes, 0, sizeof(int) * 8 * 2 * kHandChunks);
+    enqueue(k_hand_block_init, dim3(kHandBytes / 16 / 256 / 4 + 1), dim3(256), 0, nullptr, reinterpret_cast<uint4 *>(b));
     enqueue(k_side_votes, dim3(8 * 2 * kHandChunks), dim3(64), 0, nullptr, reinterpret_cast<uint32_t *>(b), votes);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);

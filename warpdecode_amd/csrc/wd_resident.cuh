@@ -91,14 +91,14 @@ struct ResidentViews {
 // What every workgroup needs from every other - four values of the next input, eleven activations - is
 // written by its producer into kResCopies copies, one per group of workgroups (r % kResCopies; on this device the
 // workgroups of a group share an L2): the consumers of a group fetch their copy with coalesced requests, and a line is polled from one
-// L2 only.  Every word lies on its readers' side of the device (see kSidePiece): the records that workgroup 0 gathers on side 0, a copy on
+// L2 only.  Every word lies on its readers' side of the device (see kSidePiece): the records that workgroup 0 gathers on both, a copy on
 // the side of its XCD, half of the ids' replicas on either.  Memory changes sides every kSidePiece bytes: the copies' pieces follow each other and
-// workgroup r reads the one of a pair that is on its side (own_copy); bit q of ResidentArgs::side_flips: in the q-th 2 MB of the block
+// a workgroup reads the one of a pair that is on its side (own_copy); bit q of ResidentArgs::side_flips: in the q-th 2 MB of the block
 // the first piece of two is side 1's.  (48 layers, IQ3_S / Q8_0 rows with the router's ids, IQ3_S with a routing trace, us: copies wherever they fall 780 / 797 /
 // 526, every word on its readers' side 760 / 759 / 525, every word on the other side 806 / 816 / 536.)
 constexpr int kResCopies = 8;
 constexpr unsigned kRecBytes = 16;        // a logit record: word 0 the router logit of row r, word 1 (workgroup 1) the shared expert's gate logit
-constexpr unsigned kHandRec = 0;                                                        // [layers][2] pieces, one of them 512 records, gathered by workgroup 0 only
+constexpr unsigned kHandRec = 0;                                                        // [layers][2] pieces of 512 records, both written, one gathered by workgroup 0 only
 constexpr unsigned kXcStride = 16;        // bytes from one workgroup's four values of a layer input to the next one's
 constexpr unsigned kHandXc = kHandRec + 2u * kSidePiece * kResMaxLayers;               // [layers][copies] pieces of [512] x four f32: layer inputs
 constexpr unsigned kAcRec = 48;                                                        // bytes of a workgroup's activations: slots 0..10, a zero
@@ -118,13 +118,14 @@ static_assert(kRecBytes * kResWgs == kSidePiece && kXcStride * kResWgs == kSideP
               "hand-off block pieces");
 // flips: those of the set's chunks.  1: in the chunk of `off` the first piece of two is side 1's.
 WD_DEV unsigned side_flip(unsigned flips, unsigned off) { return (flips >> (off / kSideChunk)) & 1u; }
-WD_DEV unsigned rec_off(unsigned flips, int l, int wg) {
-    const unsigned at = kHandRec + 2u * kSidePiece * l;
-    return at + kSidePiece * side_flip(flips, at) + kRecBytes * wg;
-}
-// The layer's copies, one piece after the other; the one that workgroup r reads (its side's of the pair of XCDs c and c + 4).
+WD_DEV unsigned rec_piece(int l, int piece, int wg) { return kHandRec + kSidePiece * (2u * l + piece) + kRecBytes * wg; }
+WD_DEV unsigned rec_off(unsigned flips, int l, int wg, int side) { return rec_piece(l, side ^ static_cast<int>(side_flip(flips, kHandRec + 2u * kSidePiece * l)), wg); }
+// The layer's copies, one piece after the other; the one that a workgroup reads (its side's of the pair of XCDs c and c + 4).
 WD_DEV unsigned xc_off(int l) { return kHandXc + static_cast<unsigned>(kResCopies * kSidePiece) * l; }
-WD_DEV unsigned own_copy(unsigned flips, unsigned at, int r) { return kSidePiece * (2u * (r & 3) + (((r >> 2) & 1u) ^ side_flip(flips, at))); }
+WD_DEV unsigned own_copy(unsigned flips, unsigned at) {
+    const unsigned x = xcc_id();
+    return kSidePiece * (2u * (x & 3u) + ((x >> 2) ^ side_flip(flips, at)));
+}
 // The layer's activations: the copies' first pieces one after the other, their second, their third; byte o of a copy lies ac_byte(o) behind its first piece.
 WD_DEV unsigned ac_off(int l) { return kHandAc + kAcBytes * kResCopies * l; }
 WD_DEV unsigned ac_byte(unsigned o) { return o + (o / kSidePiece) * ((kResCopies - 1) * kSidePiece); }
@@ -461,7 +462,7 @@ WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool has
     early();
     if (wave < 8) {  // the group's copy, three 16-byte words per lane: word w is piece w % 3 of workgroup w / 3
         const int i = wave * 64 + lane;
-        const unsigned base = ac_off(l) + own_copy(c.flips, ac_off(l), c.r) + 16u * i;
+        const unsigned base = ac_off(l) + own_copy(c.flips, ac_off(l)) + 16u * i;
         const unsigned off[3] = {base, base + kResCopies * kSidePiece, base + 2u * kResCopies * kSidePiece};
         uint4 v[3];
         {
@@ -617,7 +618,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
                 // (the other waves of the workgroup come here while rung 0 still folds the previous layer: nothing
                 // can have arrived yet)
                 if (rung != 0 && !decoded) __builtin_amdgcn_s_sleep(kResSleepFold);
-                const unsigned off[1] = {xc_off(l) + own_copy(c.flips, xc_off(l), r) + kXcStride * i};
+                const unsigned off[1] = {xc_off(l) + own_copy(c.flips, xc_off(l)) + kXcStride * i};
                 uint4 v[1];
                 hand_wait16<1>(a, c.hb, off, true, v, dead);
                 xv = make_float4(bits_f(v[0].x), bits_f(v[0].y), bits_f(v[0].z), bits_f(v[0].w));
@@ -640,7 +641,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         res_mark<STAMPS>(a, c, l, 2);
         const float res_pre = c.x_at(4 * r + (lane & 3));  // (rung 0 adds the layer's output to these)
         if (!traced && on) {  // the id this rung works on, from one of the replicas workgroup 0 publishes
-            e = hand_wait4(a, c.hb, idh_off(c.flips, l, (r >> 2) & 1) + 64u * ((r >> 3) & (kResIdCopies / 2 - 1)) + 4u * rung, true, dead);
+            e = hand_wait4(a, c.hb, idh_off(c.flips, l, xcc_side()) + 64u * ((r >> 3) & (kResIdCopies / 2 - 1)) + 4u * rung, true, dead);
             e = expert_in_range(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(e)));
             gate_up_rows(gate_base, up_base, e, r, lane);
         }
@@ -838,7 +839,7 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         auto gather_logits = [&](bool patient) {
             uint32_t lb[8];
             const unsigned all_in = 11u * static_cast<unsigned>(l + 1);
-            const bool got = hand_wait4<8>(a, c.hb, rec_off(c.flips, l, lane), 64u * kRecBytes, want, lb, dead, [&] {
+            const bool got = hand_wait4<8>(a, c.hb, rec_off(c.flips, l, lane, xcc_side()), 64u * kRecBytes, want, lb, dead, [&] {
                 return !patient && __hip_atomic_load(c.arrived(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= all_in;
             });
 #pragma unroll
@@ -912,7 +913,8 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         res_mark<STAMPS>(a, c, l, 2);
         {
             const float s = res_router_dot(wv, c.xt(), lane);
-            if (has_row && lane == 32) hand_store4(c.hb, rec_off(c.flips, l, r), hand_word(s));
+            const uint32_t word = hand_word(readlane_f(s, 32));
+            if (has_row && lane < 2) hand_store4(c.hb, rec_piece(l, lane, r), word);
             res_mark<STAMPS>(a, c, l, 3);
         }
         // (before the selection's values exist: this dot and they together would not fit the registers)
@@ -920,7 +922,8 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             float gw[32];  // (an array of its own: the router row's registers keep one definition per layer)
             res_router_fetch(res_field(&L->sh_inp), gw, lane);
             const float s = res_router_dot(gw, c.xt(), lane);
-            if (lane == 32) hand_store4(c.hb, rec_off(c.flips, l, 1) + 4u, hand_word(s));
+            const uint32_t word = hand_word(readlane_f(s, 32));
+            if (lane < 2) hand_store4(c.hb, rec_piece(l, lane, 1) + 4u, word);
         }
         bool want[8];
         float lv[8];
@@ -933,7 +936,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         auto gather_logits = [&](bool patient) {
             uint32_t lb[8];
             const unsigned all_in = 11u * static_cast<unsigned>(l + 1);
-            const bool got = hand_wait4<8>(a, c.hb, rec_off(c.flips, l, lane), 64u * kRecBytes, want, lb, dead, [&] {
+            const bool got = hand_wait4<8>(a, c.hb, rec_off(c.flips, l, lane, xcc_side()), 64u * kRecBytes, want, lb, dead, [&] {
                 return !patient && __hip_atomic_load(c.arrived(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >= all_in;
             });
 #pragma unroll
@@ -966,7 +969,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
                     if (want[j]) a.views->logits[64 * j + lane] = lv[j];
             }
             if (a.shared) {
-                const float g = bits_f(hand_wait4(a, c.hb, rec_off(c.flips, l, 1) + 4u, true, dead));
+                const float g = bits_f(hand_wait4(a, c.hb, rec_off(c.flips, l, 1, xcc_side()) + 4u, true, dead));
                 const float sg = sigmoid_ggml(g);
                 if (lane == 0) {
                     hand_store4(c.hb, kHandWh + static_cast<unsigned>((l * 16 + kResGateSlot) * 4), hand_word(sg));
@@ -1002,10 +1005,10 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         }
         for (int ll = l; ll < kResMaxLayers; ll += a.n_layers) {
             const uint4 empty4 = make_uint4(kResEmpty, kResEmpty, kResEmpty, kResEmpty);
-            // lane 0 the workgroup's logit record, 8 lanes its 128 bytes of the layer's input copies, 24 its 384 bytes of the activations'
-            const unsigned off = lane < 8 ? rec_off(other.flips, ll, r)
+            // lanes 0 and 1 the workgroup's logit record in either piece, 8 lanes its 128 bytes of the layer's input copies, 24 its 384 bytes of the activations'
+            const unsigned off = lane < 8 ? rec_piece(ll, lane & 1, r)
                                : lane < 16 ? xc_off(ll) + kXcStride * (8 * r + lane - 8) : ac_off(ll) + 16u * (24 * r + lane - 16);
-            if (lane == 0 || (lane >= 8 && lane < 40)) hand_store16(other.b, off, empty4);
+            if (lane < 2 || (lane >= 8 && lane < 40)) hand_store16(other.b, off, empty4);
             if (r == 0) {
                 hand_store16(other.b, idh_off(other.flips, ll, lane >> 5) + 16u * (lane & 31), empty4);
                 if (lane < 4) hand_store16(other.b, kHandWh + static_cast<unsigned>(ll * 64 + 16 * lane), empty4);
