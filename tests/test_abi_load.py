@@ -1,6 +1,9 @@
 """CPU-side checks of the drop-in boundary: the shared library loads without a GPU, exports every
 symbol the public header declares, and reports errors instead of computing without a device."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -114,3 +117,54 @@ def test_arguments_arrive_as_with_ctypes():
         capi._fast.prepare(capi._call, capi.check, C.c_void_p, C.Array)
         for name in capi._fast.names():
             capi._fast.bind(name, C.cast(getattr(lib, name), C.c_void_p).value)
+
+
+FIRST_CALLS = """
+import sys, threading, time
+from warpdecode_amd import capi
+real, gate, answers = capi.C.CDLL, threading.Barrier(8), []
+def slow_load(path):    # every thread that gets this far is in the load together
+    time.sleep(0.05)
+    return real(path)
+capi.C.CDLL = slow_load
+def first():
+    gate.wait()
+    try:
+        answers.append(capi.call("wd_topk_softmax", None, 12, 2, 1.0, None, None, None))
+    except Exception as e:
+        answers.append((type(e).__name__, str(e)))
+threads = [threading.Thread(target=first) for _ in range(8)]
+[t.start() for t in threads]
+[t.join() for t in threads]
+assert len(answers) == 8 and set(answers) == {answers[0]} and answers[0][0] == "WdError" and "multiple of 8" in answers[0][1], answers
+"""
+LOAD_AGAIN = """
+from warpdecode_amd import capi
+real = capi._fast
+class FailsOnTheWay:
+    bound = 0
+    names = staticmethod(real.names)
+    @classmethod
+    def bind(cls, *a):
+        if cls.bound == 3: raise MemoryError("on the way")
+        cls.bound += 1
+        real.bind(*a)
+capi._fast = FailsOnTheWay
+for _ in range(2):
+    FailsOnTheWay.bound = 0
+    try:
+        capi.load()
+        raise SystemExit("the load did not fail")
+    except MemoryError:
+        pass
+capi._fast = real
+assert capi.load() is capi.load()
+"""
+
+
+@pytest.mark.parametrize("program", [FIRST_CALLS, LOAD_AGAIN], ids=["several_threads", "after_a_failure"])
+def test_first_load(program):
+    """In a process of its own: the first calls of several threads all get the library's answer, and a load that failed can be tried again."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = subprocess.run([sys.executable, "-c", program], cwd=root, capture_output=True, text=True, timeout=120)
+    assert got.returncode == 0, got.stderr

@@ -7,6 +7,7 @@ There is no fallback: if the HIP library has not been built, loading raises.
 import ctypes as C
 import os
 import re
+import threading
 
 try:
     from . import _fast
@@ -177,30 +178,38 @@ def declared_symbols():
 
 
 _lib = None
+_load_lock = threading.RLock()
 
 
 def load():
-    global _lib
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
-            raise WdError("libwarpdecode_amd.so is not built: run `python -m warpdecode_amd.build` "
-                          "(there is no CPU fallback for the HIP kernels)")
-        lib = C.CDLL(LIB_PATH)
-        lib.wd_last_error.restype = C.c_char_p
-        for name, (res, args) in list(_SIGS.items()) + list(_OPTIONAL.items()):
-            fn = getattr(lib, name, None)
-            if fn is None:
-                if name in _SIGS:
-                    raise WdError("libwarpdecode_amd.so does not export " + name)
-                continue
-            fn.restype, fn.argtypes = res, args
-        if _fast:
-            for name in _fast.names():
-                if not set(_SIGS[name][1]) <= {vp, i32, f32, sz}:
-                    raise WdError("_fast does not take the arguments of " + name)
-                _fast.bind(name, C.cast(getattr(lib, name), vp).value)
-        _lib = lib
+        with _load_lock:    # first calls of several threads; loading the library lets go of the interpreter
+            _load()
     return _lib
+
+
+def _load():
+    global _lib
+    if _lib is not None:
+        return
+    if not os.path.exists(LIB_PATH):
+        raise WdError("libwarpdecode_amd.so is not built: run `python -m warpdecode_amd.build` "
+                      "(there is no CPU fallback for the HIP kernels)")
+    lib = C.CDLL(LIB_PATH)
+    lib.wd_last_error.restype = C.c_char_p
+    for name, (res, args) in list(_SIGS.items()) + list(_OPTIONAL.items()):
+        fn = getattr(lib, name, None)
+        if fn is None:
+            if name in _SIGS:
+                raise WdError("libwarpdecode_amd.so does not export " + name)
+            continue
+        fn.restype, fn.argtypes = res, args
+    if _fast:
+        for name in _fast.names():
+            if not set(_SIGS[name][1]) <= {vp, i32, f32, sz}:
+                raise WdError("_fast does not take the arguments of " + name)
+            _fast.bind(name, C.cast(getattr(lib, name), vp).value)
+    _lib = lib
 
 
 def check(rc):

@@ -155,7 +155,8 @@ PyObject *names(PyObject *, PyObject *) {
     }
     return list;
 }
-// bind(name, address): calls of this entry point go to the address from now on
+// bind(name, address): calls of this entry point go to the address from now on.  The same address may be bound again (a load that failed
+// on the way is tried once more), another one may not.
 PyObject *bind(PyObject *, PyObject *args) {
     const char *name;
     PyObject *address;
@@ -163,7 +164,7 @@ PyObject *bind(PyObject *, PyObject *args) {
     void *const fn = PyLong_AsVoidPtr(address);
     if (PyErr_Occurred()) return nullptr;
     for (Entry &e : g_entries)
-        if (g_table && fn && !e.fn && std::strcmp(e.name, name) == 0) {
+        if (g_table && fn && (!e.fn || e.fn == fn) && std::strcmp(e.name, name) == 0) {
             PyObject *const capsule = PyCapsule_New(&e, nullptr, nullptr);
             if (!capsule) return nullptr;
             e.fn = fn;
