@@ -488,3 +488,14 @@ def test_alignment_chooses_the_fetch_path(g, oracle):
         assert capi.load().wd_moe_scratch_status(sc.h) == 0
         for s in scs:
             s.close()
+
+
+def test_scratch_behind_an_older_error(g):
+    """An error that an older call of this thread has left behind is none of a scratch that is made now."""
+    hip = capi.load()   # (the runtime's functions resolve through the library)
+    hip.hipSetDevice.argtypes, hip.hipSetDevice.restype, hip.hipPeekAtLastError.restype = [C.c_int], C.c_int, C.c_int
+    try:
+        assert hip.hipSetDevice(1 << 20) != 0 and hip.hipPeekAtLastError() != 0
+        g.Scratch(1024, 256, 64, 6).close()
+    finally:
+        hip.hipGetLastError()

@@ -36,15 +36,20 @@ int noalloc_setup_current_device();
 
 // A kernel launch through the runtime's own entry point.  The <<<>>> form goes through a stub that parks the launch shape in
 // the runtime and takes it out again: 2.35 to 2.43 us of host time for a launch, 2.22 to 2.28 so (an argument block of 40 bytes, a
-// C++ loop; another process of the same machine 2.79 to 2.84, 2.67 to 2.72).  An error is left for WD_LAUNCH_CHECK, as by <<<>>>.
+// C++ loop; another process of the same machine 2.79 to 2.84, 2.67 to 2.72).  An error is left for WD_LAUNCH_CHECK, as by <<<>>>; enqueue_reported returns
+// it as well, for a caller to whom an older error of the thread must not look like this launch's.
 template <typename T>
 struct SameType {
     using type = T;
 };
 template <typename... P>
-inline void enqueue(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, const typename SameType<P>::type &...args) {
+inline hipError_t enqueue_reported(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, const typename SameType<P>::type &...args) {
     const void *ptrs[] = {&args...};
-    (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, const_cast<void **>(ptrs), lds, stream);
+    return hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, const_cast<void **>(ptrs), lds, stream);
+}
+template <typename... P>
+inline void enqueue(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t stream, const typename SameType<P>::type &...args) {
+    (void)enqueue_reported(kernel, grid, block, lds, stream, args...);
 }
 
 inline int block_elems(int type) {

@@ -202,9 +202,9 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
         return fail(WD_ERR_HIP, "hipHostMalloc MoE scratch ids failed");
     }
     std::memset(s->h_ids, 0, sizeof(int32_t) * kHostWords);
-    enqueue(k_scratch_init, dim3(64), dim3(256), 0, nullptr, reinterpret_cast<uint32_t *>(b), static_cast<unsigned>(c.off / 4), static_cast<unsigned>(o_hand / 4),
-            static_cast<unsigned>(c.off / 4), units, s->h_ids);
-    hipError_t init = hipGetLastError();
+    // (its own code and not the thread's last error, which may be of an older call of the caller's)
+    hipError_t init = enqueue_reported(k_scratch_init, dim3(64), dim3(256), 0, nullptr, reinterpret_cast<uint32_t *>(b), static_cast<unsigned>(c.off / 4),
+                                       static_cast<unsigned>(o_hand / 4), static_cast<unsigned>(c.off / 4), units, s->h_ids);
     if (init == hipSuccess) init = hipStreamSynchronize(nullptr);
     if (init != hipSuccess) {
         (void)hipHostFree(s->h_ids);
@@ -920,9 +920,8 @@ int resident_prepare(wd_moe_scratch *s) {
     uint8_t *const b = reinterpret_cast<uint8_t *>((reinterpret_cast<uintptr_t>(alloc) + kSideChunk - 1) & ~static_cast<uintptr_t>(kSideChunk - 1));
     int *const votes = s->h_ids + 48;
     std::memset(votes, 0, sizeof(int) * 8 * 2 * kHandChunks);
-    enqueue(k_hand_block_init, dim3(kHandBytes / 16 / 256 / 4 + 1), dim3(256), 0, nullptr, reinterpret_cast<uint4 *>(b));
-    enqueue(k_side_votes, dim3(8 * 2 * kHandChunks), dim3(64), 0, nullptr, reinterpret_cast<uint32_t *>(b), votes);
-    hipError_t e = hipGetLastError();
+    hipError_t e = enqueue_reported(k_hand_block_init, dim3(kHandBytes / 16 / 256 / 4 + 1), dim3(256), 0, nullptr, reinterpret_cast<uint4 *>(b));
+    if (e == hipSuccess) e = enqueue_reported(k_side_votes, dim3(8 * 2 * kHandChunks), dim3(64), 0, nullptr, reinterpret_cast<uint32_t *>(b), votes);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         (void)hipFree(alloc);
