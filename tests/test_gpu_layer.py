@@ -4,6 +4,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from warpdecode_amd import capi, synth
 
@@ -499,3 +500,38 @@ def test_scratch_behind_an_older_error(g):
         g.Scratch(1024, 256, 64, 6).close()
     finally:
         hip.hipGetLastError()
+
+
+@pytest.mark.parametrize("E,k", [(64, 6), (160, 16), (512, 10), (640, 10)])
+def test_a_layer_on_every_stream(g, oracle, E, k):
+    """Readers of handed-on words take the copy of the side of the XCD that they run on, and where a dispatch begins differs from
+    stream to stream: merged, split, A alone and then the rest, a stack and a token batch, each in turn on six streams."""
+    H, F, T = 512, 64, 2
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=981, router_sigma=1.0 / np.sqrt(H))
+    xs = np.stack([synth.rms_normed(synth.rng_for(SEED, 71 + t, E), H) for t in range(T)])
+    want = [oracle.moe_layer(L, x)[0] for x in xs]
+    dl, scr = g.DeviceLayer(L), [g.Scratch(H, F, E, k) for _ in range(T)]
+    arr, stack = (C.c_void_p * T)(*[s.h for s in scr]), (capi.MoeLayer * 3)(*[dl.desc] * 3)
+    dx, out, outs = g.dev(xs), g.empty(H, np.float32), g.empty((T, H), np.float32)
+    only_rest = capi.MOE_ONLY_B | capi.MOE_ONLY_C
+    g.sync()
+    for turn in range(2):
+        for stream in [torch.cuda.default_stream()] + [torch.cuda.Stream() for _ in range(5)]:
+            with torch.cuda.stream(stream):
+                for flags in ((0,), (capi.MOE_SPLIT_AB,), (capi.MOE_ONLY_A, only_rest)):
+                    out.zero_()
+                    for f in flags:
+                        capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), scr[0].h, f, g.stream())
+                    assert g.same_bits(g.host(out), want[0]), flags
+                capi.call("wd_moe_layer_noalloc_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), 0, g.stream())
+                assert g.same_bits(g.host(out), want[0])
+                capi.call("wd_moe_stack_f32", stack, 3, g.ptr(dx), g.ptr(out), scr[0].h, None, 0.0, capi.MOE_PER_LAYER, g.stream())
+                assert g.same_bits(g.host(out), want[0])
+                for flags in (0, capi.MOE_SPLIT_AB):
+                    outs.zero_()
+                    capi.call("wd_moe_layer_tokens_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(outs), T, arr, flags, g.stream())
+                    assert g.same_bits(g.host(outs), np.stack(want)), flags
+            stream.synchronize()
+    assert [capi.load().wd_moe_scratch_status(s.h) for s in scr] == [0] * T
+    for s in scr:
+        s.close()

@@ -44,7 +44,8 @@ struct LayerArgs {
     int n_shared_wgs;            // those that take the shared expert's gate/up (the rest: routed gate/up)
     int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
     const int32_t *ids_known;    // null, or the k ids where they are known before the launch
-    uint32_t *hand;              // [E + 2]: the router's logits and the shared gate's on their way to the selection, and the count of hand_close; kHandEmpty between passes
+    uint32_t *hand;              // [E + 2]: the router's logits and the shared gate's on their way to the selection, for side 0, and the count of hand_close; kHandEmpty between passes
+    int hand_side;               // so many words on from these the logits for side 1 (0: one copy for both)
     uint32_t *ids_tagged;        // selected ids published inside the merged dispatch (kTagInvalid = not yet): [kTagCopies / 2][16] for side 0,
     int tag_side;                // so many words on from these for side 1 (tag_copy)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
@@ -65,13 +66,11 @@ constexpr uint32_t kTagInvalid = 0xffffffffu;
 // Sides.  A word that workgroups hand on has a home in one half of the device's memory, and the XCDs of that half reach it sooner: a device-scope
 // load that misses the L2 takes 350 to 450 clocks near its home and 580 to 700 from the other half (stores 370 to 500 and 600 to 760), a word from
 // XCD 0 to XCD 1 360 ns by way of the near half and 575 by the far one.  Memory alternates between the halves in pieces of kSidePiece bytes; which
-// of two neighbours is whose is measured when a scratch is made (side_vote).  Words lie on their readers' side: XCDs 0..3 are side 0, the others
-// side 1; workgroup b runs on XCD b mod 8 in the queues that begin at XCD 0.
+// of two neighbours is whose is measured when a scratch is made (side_vote).  XCDs 0..3 are side 0, the others side 1.
+// What has readers on either side is written once for each, and a reader takes the copy of the side of the XCD that it does run on (HW_REG XCC_ID) and not of
+// its block number: block 0 of a dispatch is on the XCD at which its hardware queue begins, 0 for one stream and 7 for another.
 constexpr int kSidePiece = 8192;
 constexpr unsigned kSideChunk = 2u << 20;  // within which the halves keep their order
-WD_DEV int block_side() { return static_cast<int>((blockIdx.x >> 2) & 1u); }
-// Where a reader may choose among copies it goes by the XCD that it does run on (HW_REG XCC_ID): block 0 of a dispatch is on the XCD at which its
-// hardware queue begins, 0 for one stream and 7 for another.
 WD_DEV unsigned xcc_id() { return static_cast<unsigned>(__builtin_amdgcn_s_getreg(20 | (3 << 11))) & 7u; }
 WD_DEV int xcc_side() { return static_cast<int>(xcc_id() >> 2); }
 // The replica of the published ids that workgroup `wg` of the waiting ones polls.
@@ -685,7 +684,7 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
 
 // ---- selection inside the dispatch that computes the logits ------------------------------------------------------------
 // Every router wave hands its logit on as a word that cannot be kHandEmpty (hand[e], the shared expert's gate logit in
-// hand[n_slot]); dispatch C sets the words back.  A workgroup of its own, the dispatch's first, selects: it polls the words until all are
+// hand[n_slot]; for either side); dispatch C sets the words back.  A workgroup of its own, the dispatch's first, selects: it polls the words until all are
 // there.  No router workgroup waits for its own word, counts itself or looks at the row, and the selection runs where nothing else did
 // before it (its code is in that compute unit's instruction cache from one launch to the next).
 // (Selected by the router workgroups that end last - each waits until its words are acknowledged and looks at the row, a ticket names the
@@ -693,23 +692,31 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
 // us per layer: 2560 / 640 24.6, so 24.4; 2048 / 512 20.5, 19.9; 1024 / 256 12.0, 11.9.  Four tokens of 2048 / 512, whose router workgroups
 // counted themselves and the last one polled, 40.0, 39.5.)
 struct HandRow {
-    uint32_t *hand;
+    const uint32_t *hand;  // the copy of the reader's side
     int n, n_slot;
     bool gate;  // hand[n_slot] is one of the row's
     unsigned limit;  // polls before one that waits for the row gives up
 };
+WD_DEV const uint32_t *hand_copy(const uint32_t *hand, int hand_side) { return hand + (xcc_side() ? hand_side : 0); }
 WD_DEV uint32_t hand_load(const uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// `words` of them back to "not yet", in both copies (the count in the second one's place is as it was).
+WD_DEV void hand_clear(uint32_t *hand, int hand_side, int words, int thread, int threads) {
+    for (int i = thread; i < words; i += threads) {
+        __hip_atomic_store(hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(hand + hand_side + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
 // Sets the words back where no dispatch C does: the one of the router workgroups and the selecting one that is done last, behind every other
 // one's last use of them.  Every thread of each of the n_wgs must call it.  (A fill launched behind the dispatch instead, us per layer with the ids through the host: 2048 / 512
 // 46.2, so 45.0; 1024 / 256 37.9, 36.9; 4096 / 1536 66.5, 65.5.)
-WD_DEV void hand_close(uint32_t *hand, int n_slot, int n_wgs, int &last) {
+WD_DEV void hand_close(uint32_t *hand, int hand_side, int n_slot, int n_wgs, int &last) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);  // what this wave has asked for of the words is there
     __syncthreads();
     if (threadIdx.x == 0) last = __hip_atomic_fetch_add(hand + n_slot + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == static_cast<uint32_t>(n_wgs - 1);
     __syncthreads();
     if (!last) return;
-    for (int i = threadIdx.x; i < n_slot + 2; i += static_cast<int>(blockDim.x)) __hip_atomic_store(hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    hand_clear(hand, hand_side, n_slot + 2, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x));
 }
 // lv[j]: logit 64 j + lane, once the row is complete (the limit is there for a broken device: words that did not come are NaN, what is
 // selected then are experts of the layer, and the status makes the results NaN).  Returns whether it was.
@@ -862,6 +869,11 @@ WD_DEV float router_span_run(const float (&wv)[32], const float *x, int groups, 
     }
     return v;
 }
+// The logit in lane 32 of the wave, to both copies of hand[slot] by one instruction.
+WD_DEV void router_hand_on(float logit, uint32_t *hand, int hand_side, int slot, int lane) {
+    const uint32_t word = hand_word_bits(f_bits(readlane_f(logit, 32)));
+    if (lane < 2) __hip_atomic_store(hand + (lane == 0 ? 0 : hand_side) + slot, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 // x to LDS, by the whole workgroup.
 WD_DEV void router_stage_x(const float *__restrict__ x, float *xs, int cols) {
     for (int i = static_cast<int>(threadIdx.x) * 4; i < cols; i += static_cast<int>(blockDim.x) * 4)
@@ -876,10 +888,10 @@ WD_DEV void router_stage_x(const float *__restrict__ x, float *xs, int cols) {
 // which lets three workgroups of the merged dispatch share a compute unit).
 // Every thread of the workgroup must call it (it contains a barrier).
 // SCALAR_ROW: keep the wave's row pointer in scalar registers (two vector registers fewer).
-// The row's result goes to hand[row], the extra row's to hand[extra_slot]; it is returned as well (lane 32), with the row in `done`
+// The row's result goes to hand[row], the extra row's to hand[extra_slot] (of both sides' copies); it is returned as well (lane 32), with the row in `done`
 // (-1: this wave has none).
 template <bool SCALAR_ROW = false>
-WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restrict__ x, float *xs, uint32_t *hand, int rows,
+WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restrict__ x, float *xs, uint32_t *hand, int hand_side, int rows,
                               int cols, const float *__restrict__ extra_w, int extra_slot, int wg, int &done) {
     const int lane = threadIdx.x & 63, t = lane & 31;
     const bool upper = lane >= 32;
@@ -908,7 +920,7 @@ WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restri
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
     const float acc = router_close32(s);
     done = on ? (row < rows ? row : extra_slot) : -1;
-    if (on && lane == 32) __hip_atomic_store(hand + done, hand_word_bits(f_bits(acc)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (on) router_hand_on(acc, hand, hand_side, done, lane);
     return acc;
 }
 
@@ -916,7 +928,7 @@ WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restri
 // wave 2 w + 1 the rest, both with every load of theirs in flight from the start - one trip to memory instead of one per
 // span.  The chains still see their columns in ascending order: the second wave starts from the 32 accumulators the
 // first one leaves in LDS (`over`: 4 x 32 floats).  Every thread of the (512-thread) workgroup must call it.
-WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *over, uint32_t *hand,
+WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__restrict__ x, float *xs, float *over, uint32_t *hand, int hand_side,
                                    int rows, int cols, const float *__restrict__ extra_w, int extra_slot, int wg, int &done) {
     const int lane = threadIdx.x & 63, t = lane & 31, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const bool upper = lane >= 32, second = (wave & 1) != 0;
@@ -951,7 +963,7 @@ WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__r
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
     const float acc = router_close32(s);
     done = on ? (row < rows ? row : extra_slot) : -1;
-    if (on && lane == 32) __hip_atomic_store(hand + done, hand_word_bits(f_bits(acc)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (on) router_hand_on(acc, hand, hand_side, done, lane);
     return acc;
 }
 
@@ -1023,11 +1035,12 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
         if (wave == 0) __builtin_amdgcn_s_setprio(3);
         // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
-        const bool there = topk_block(HandRow{a.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
+        const uint32_t *const hand = hand_copy(a.hand, a.hand_side);
+        const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
                                       (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, a.tag_side);
         if (!there && lane == 0) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // off the selection's path: the shared expert's gate
-        if (a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(a.hand + a.E)));
+        if (a.sh_inp && wave == 5 && lane == 0) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(hand + a.E)));
         if (wave == 0) {
             wave_lds_fence();
             // the plain copies for dispatch C
@@ -1039,7 +1052,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
             if (TRACE && a.trace && lane == 0) a.trace[(0 * 16 + 8) * 8 + 1] = wall_clock64();
         }
         mark<TRACE>(a, 0, 2);
-        if (a.close_hand) hand_close(a.hand, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
+        if (a.close_hand) hand_close(a.hand, a.hand_side, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
         return;
     }
     const int wg = blk - a.n_select_wgs;
@@ -1048,16 +1061,16 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         int row;
         float logit;
         if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
-            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, rows, H,
+            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, a.hand_side, rows, H,
                                           a.sh_inp, a.E, wg, row);
         else
-            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, rows, H, a.sh_inp, a.E, wg, row);
+            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, a.hand_side, rows, H, a.sh_inp, a.E, wg, row);
         mark<TRACE>(a, 0, 1);
         if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
         // (no selection: the one wave with the shared gate's row)
         if (a.preselected && row == a.E && lane == 32) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
         mark<TRACE>(a, 0, 2);
-        if (a.close_hand) hand_close(a.hand, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
+        if (a.close_hand) hand_close(a.hand, a.hand_side, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
         return;
     }
 
@@ -1181,7 +1194,7 @@ WD_DEV void layer_clear_handed(const LayerArgs &a, int threads) {
         __hip_atomic_store(a.ids_tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(a.ids_tagged + a.tag_side + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    for (int i = threadIdx.x; i < a.E + 1; i += threads) __hip_atomic_store(a.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    hand_clear(a.hand, a.hand_side, a.E + 1, static_cast<int>(threadIdx.x), threads);
 }
 
 // ---- the combine at the end of dispatch C ---------------------------------------------------------------------

@@ -42,7 +42,8 @@ struct wd_moe_scratch {
     int32_t *gup = nullptr;
     int32_t *dp = nullptr;
     int gup_type = -1, dp_type = -1;
-    uint32_t *hand = nullptr;             // [n_experts + 2] logits on their way to the selection inside dispatch AB (LayerArgs)
+    uint32_t *hand = nullptr;             // [n_experts + 2] logits on their way to the selection inside dispatch AB,
+    int hand_side = 0;                    // and those of side 1 (LayerArgs)
     unsigned long long *trace = nullptr;  // device [3][16][8] time stamps, see wd_moe_scratch_trace
     int trace_wg = 0;
     int32_t *h_ids = nullptr;             // pinned [kHostWords]: [0..15] routed ids for callers that must see them on the host,
@@ -213,7 +214,8 @@ int wd_moe_scratch_create(wd_moe_scratch **out, int hidden, int expert_ffn, int 
         return fail(WD_ERR_HIP, "MoE scratch: the first launch failed: %s", hipGetErrorString(init));
     }
     s->flip = side_flip_of(s->h_ids);
-    if (sizeof(uint32_t) * (static_cast<size_t>(n_experts) + 2) <= kSidePiece) s->hand = units + s->flip * (kSidePiece / 4);
+    if (sizeof(uint32_t) * (static_cast<size_t>(n_experts) + 2) <= kSidePiece)
+        s->hand = units + s->flip * (kSidePiece / 4), s->hand_side = s->flip ? -kSidePiece / 4 : kSidePiece / 4;
     std::memset(s->h_ids, 0, sizeof(int32_t) * kHostWords);
     *out = s;
     return WD_OK;
@@ -251,7 +253,7 @@ int wd_moe_scratch_set_wait_limit(wd_moe_scratch *s, unsigned polls) {
     WD_HIP(hipMemset(s->status, 0, sizeof(unsigned)));
     reinterpret_cast<volatile int32_t *>(s->h_ids)[16] = 0;
     WD_HIP(hipMemset(s->tagged, 0xff, 2 * static_cast<size_t>(kSidePiece) * kTagUnits));
-    WD_HIP(hipMemset(s->hand, 0xff, sizeof(uint32_t) * (s->n_experts + 2)));
+    for (uint32_t *hand : {s->hand, s->hand + s->hand_side}) WD_HIP(hipMemset(hand, 0xff, sizeof(uint32_t) * (s->n_experts + 2)));
     if (s->res_block) WD_HIP(hipMemset(s->res_block, 0xff, kHandEpoch));
     return WD_OK;
 }
@@ -551,7 +553,7 @@ LayerArgs fused_args(const wd_moe_layer *L, const float *d_x, float *d_out, wd_m
     a.dry = (flags & WD_MOE_DRY) ? 1 : 0;
     a.ids_known = ids_override;  // a routing trace: the ids do not depend on the router
     a.trace = s->trace, a.trace_wg = s->trace_wg;
-    a.hand = s->hand;
+    a.hand = s->hand, a.hand_side = s->hand_side;
     a.ids_tagged = s->tags(rec % kTagRecords), a.tag_side = s->tag_side();
     a.clear_tagged = 1;
     a.status = s->status;
@@ -754,7 +756,7 @@ int reset_published(const wd_moe_scratch *s, int rec, hipStream_t st) {
 void reset_handed(const wd_moe_scratch *s, int rec, hipStream_t st) {
     const size_t n = static_cast<size_t>(s->n_experts) + 2;
     reset_tags(s, rec, st);
-    enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, s->hand, kHandEmpty, n);
+    for (uint32_t *hand : {s->hand, s->hand + s->hand_side}) enqueue(k_fill_u32, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, hand, kHandEmpty, n);
     (void)hipGetLastError();
 }
 
@@ -1202,7 +1204,7 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
         TokenSlots &k_ = ta.tok[t];
         k_.x = d_x + static_cast<size_t>(t) * H, k_.out = d_out + static_cast<size_t>(t) * H;
         k_.logits = s->logits, k_.ids = s->ids, k_.weights = s->weights, k_.act = s->act;
-        k_.shared_gate = s->shared_gate, k_.hand = s->hand;
+        k_.shared_gate = s->shared_gate, k_.hand = s->hand, k_.hand_side = s->hand_side;
         k_.expert_out = (flags & WD_MOE_KEEP_EXPERT_OUT) ? s->expert_out : nullptr;
         k_.accum = s->accum, k_.down_f32 = s->down_f32;
         k_.tagged = s->tags(0), k_.tag_side = s->tag_side(), k_.status = s->status;

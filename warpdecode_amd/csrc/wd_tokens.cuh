@@ -48,7 +48,8 @@ struct TokenSlots {
     float *weights;
     float *act;          // [k+1][F]
     float *shared_gate;  // [1]
-    uint32_t *hand;      // (LayerArgs)
+    uint32_t *hand;      // (LayerArgs),
+    int hand_side;
     float *expert_out;   // null or [k][H]
     float *accum, *down_f32, *out;
     uint32_t *tagged;    // selected ids published inside dispatch AB (ids_tagged, LayerArgs),
@@ -66,7 +67,7 @@ struct TokenArgs {
 
 // ---- dispatch AB for T tokens, first part (A) --------------------------------------------------------------
 // kTokensSelectWgs (none where the ids are given) + T * (router_stride + shared_stride) workgroups, 512 threads, the strides being the router and the
-// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first two workgroups per token of which one selects, then the router workgroups
+// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first the workgroups that select, one per token, then the router workgroups
 // of every token, token by token, then the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
 // token - the same weight rows - lands on the same XCD (workgroups go to the eight XCDs in turn), so its L2 serves the
 // rows to the tokens after the first.  The padding workgroups return at once.  Per token this is the front of the
@@ -74,8 +75,7 @@ struct TokenArgs {
 // and publishes the ids, the other workgroups run the shared expert's gate/up.
 // lds: 4 * H + 16 bytes, x as f32 for the router rows (the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes of the
 // routed part's tables, for the selection; tiles: the shared rows' eight.
-// (workgroups 4..7 of every eight return at once: the words that a selection waits for lie on side 0)
-constexpr int kTokensSelectWgs = 2 * kMaxTokens;
+constexpr int kTokensSelectWgs = kMaxTokens;
 static_assert(kTokensSelectWgs % 8 == 0, "the workgroups behind keep their XCDs");
 struct TokensAGrid {
     int router_stride, shared_stride;
@@ -92,10 +92,11 @@ WD_DEV void tokens_select(const TokenArgs &ta, int t, uint8_t *s_work, int lane,
     int32_t *lds_ids = reinterpret_cast<int32_t *>(s_work + kTopkLdsBytes2);  // behind the selection's own scratch
     float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
     if (wave == 0) __builtin_amdgcn_s_setprio(3);
-    const bool there = topk_block(HandRow{s.hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr,
+    const uint32_t *const hand = hand_copy(s.hand, s.hand_side);
+    const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr,
                                   ta.wait_ids ? s.tagged : nullptr, s.tag_side);
     if (!there && lane == 0) __hip_atomic_store(s.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(s.hand + a.E)));
+    if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(hand + a.E)));
     if (wave == 0) {
         wave_lds_fence();
         if (lane < a.k) {
@@ -118,8 +119,7 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
     {
         const int first = a.preselected ? 0 : kTokensSelectWgs, b = static_cast<int>(blockIdx.x) - first, router_part = ta.T * gr.router_stride;
         if (b < 0) {
-            const int t = (blockIdx.x & 3) + 4 * (blockIdx.x >> 3);
-            if (block_side() == 0 && t < ta.T) tokens_select(ta, t, s_work, lane, wave);
+            if (static_cast<int>(blockIdx.x) < ta.T) tokens_select(ta, blockIdx.x, s_work, lane, wave);
             return;
         }
         if (b < router_part) {
@@ -138,9 +138,9 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         int row;
         float logit;
         if (WIDE)
-            logit = router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.hand, rows, H, a.sh_inp, a.E, wg, row);
+            logit = router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.hand, s.hand_side, rows, H, a.sh_inp, a.E, wg, row);
         else
-            logit = router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.hand, rows, H, a.sh_inp, a.E, wg, row);
+            logit = router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.hand, s.hand_side, rows, H, a.sh_inp, a.E, wg, row);
         if (lane == 32 && row >= 0 && row < rows) s.logits[row] = logit;  // (the caller's view)
         // (no selection: the one wave with the shared gate's row)
         if (a.preselected && row == a.E && lane == 32) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
@@ -607,7 +607,7 @@ WD_DEV void tokens_clear_handed(const TokenArgs &ta, int waves, int tw, int lane
         __hip_atomic_store(s.tagged + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(s.tagged + s.tag_side + i, kTagInvalid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    for (int i = lane; i < ta.common.E + 1; i += 64) __hip_atomic_store(s.hand + i, kHandEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    hand_clear(s.hand, s.hand_side, ta.common.E + 1, lane, 64);
 }
 // grid = H / 8: a workgroup owns eight output rows, as the one-token k_layer_c8 does.  Work items are (token, matrix) with
 // matrix = the token's k routed down tensors, then the shared one (always Q8_0); the waves take them in turn: the
