@@ -206,9 +206,12 @@ int wd_moe_scratch_destroy(wd_moe_scratch *s);
 int wd_moe_scratch_status(wd_moe_scratch *s);
 /* The device word behind it (u32), for callers that copy it beside other results instead of a read of its own. */
 const unsigned *wd_moe_scratch_status_word(wd_moe_scratch *s);
-/* Sets the number of polls after which such a wait gives up (0 = the default, seconds of waiting) and clears the
- * status word.  For tests of the failure path: with a limit of 1 the waiting workgroups give up at once, set the
- * status and leave without touching memory; every kernel still ends normally.  Synchronous. */
+/* Sets the number of polls after which such a wait gives up (0 = the default: 25 ms for an id that another workgroup publishes,
+ * 0.25 s for the router's logits) and clears the status word.  For tests of the failure path: with a limit of 1 the waiting
+ * workgroups give up at once, set the status and leave without touching memory; every kernel still ends normally.  Where no
+ * workgroup of a dispatch waits for the ids - they are given, or WD_MOE_SPLIT_AB or WD_MOE_ONLY_A keep the routed part out of it - the
+ * limit does not apply: the selection waits for the logits as long as the device takes to run the router's workgroups (a
+ * quarter of a minute, if it never does).  Synchronous. */
 int wd_moe_scratch_set_wait_limit(wd_moe_scratch *s, unsigned polls);
 /* Device views, named after Qwen38MoeScratch accessors (src/qwen38_moe.cuh:1701-2150). */
 float *wd_moe_scratch_logits(wd_moe_scratch *s);      /* f32 [n_experts] */
@@ -254,7 +257,7 @@ unsigned long long *wd_moe_scratch_trace_resident(wd_moe_scratch *s, int wg, int
 #define WD_MOE_ONLY_A 0x10u /* router + selection + shared gate/up */
 #define WD_MOE_ONLY_B 0x20u /* routed gate/up + SwiGLU */
 #define WD_MOE_ONLY_C 0x40u /* down projections + combine */
-#define WD_MOE_SPLIT_AB 0x100u /* router and routed gate/up as two launches instead of one with an in-dispatch hand-off */
+#define WD_MOE_SPLIT_AB 0x100u /* router and routed gate/up as two launches instead of one that hands the ids over inside */
 #define WD_MOE_DRY 0x80u    /* every workgroup of the fused dispatches returns at once: the launch floor */
 #define WD_MOE_PER_LAYER 0x200u /* wd_moe_stack_f32: launch every layer's dispatches instead of one resident launch for the stack */
 

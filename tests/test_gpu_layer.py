@@ -379,8 +379,8 @@ def test_bounded_wait_gives_up_and_recovers(g, oracle):
 
 @pytest.mark.parametrize("E,k", [(8, 1), (64, 6), (512, 10), (640, 10), (512, 16)])
 def test_late_logits_are_reported(g, oracle, E, k):
-    """The selecting workgroup starts before the router's and polls their words: with a wait limit of one poll it may give up (the parts
-    are launched apart, so nobody else waits), and then says so in the status word and in the data; with the default limit it is the oracle's."""
+    """The selecting workgroup polls the router's words, and the routed ones the ids: with a wait limit of one poll they may give up, and
+    then say so in the status word and in the data; with the default limit the results are the oracle's."""
     H, F = 512, 64
     L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=980, router_sigma=1.0 / np.sqrt(H))
     x = synth.rms_normed(synth.rng_for(SEED, 70, E), H)
@@ -390,7 +390,7 @@ def test_late_logits_are_reported(g, oracle, E, k):
     for limit in (1, 1, 1, 0, 0):
         capi.call("wd_moe_scratch_set_wait_limit", sc.h, limit)
         out.zero_()
-        capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, capi.MOE_SPLIT_AB, g.stream())
+        capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, 0, g.stream())
         g.sync()
         late = capi.load().wd_moe_scratch_status(sc.h)
         assert late in ((0, 1) if limit else (0,))
@@ -535,3 +535,32 @@ def test_a_layer_on_every_stream(g, oracle, E, k):
     assert [capi.load().wd_moe_scratch_status(s.h) for s in scr] == [0] * T
     for s in scr:
         s.close()
+
+
+@pytest.mark.parametrize("form", ["split", "trace", "split-trace", "A alone"])
+@pytest.mark.parametrize("E,k", [(8, 1), (64, 6), (512, 10), (640, 10), (512, 16)])
+def test_where_nobody_waits_for_the_ids_nothing_gives_up(g, oracle, E, k, form):
+    """Ids that are known before the launch, or a routed part in a launch of its own: nothing in a dispatch waits for the ids, and a wait limit of
+    one poll, as short as another stream's kernel could make the default one seem, changes nothing."""
+    H, F = 512, 64
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=980, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 70, E), H)
+    want, d = oracle.moe_layer(L, x)
+    dl, sc = g.DeviceLayer(L), g.Scratch(H, F, E, k)
+    out, trace = g.empty(H, np.float32), g.dev(d["ids"].astype(np.int32))
+    stack = (capi.MoeLayer * 1)(dl.desc)
+    for limit in (1,) * 8 + (0,):
+        capi.call("wd_moe_scratch_set_wait_limit", sc.h, limit)
+        dx = g.dev(x)
+        out.zero_()
+        if form == "A alone":
+            for flags in (capi.MOE_ONLY_A, capi.MOE_ONLY_B | capi.MOE_ONLY_C):
+                capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, flags, g.stream())
+        else:
+            flags = capi.MOE_PER_LAYER | (capi.MOE_SPLIT_AB if "split" in form else 0)
+            capi.call("wd_moe_stack_f32", stack, 1, g.ptr(dx), g.ptr(out), sc.h, g.ptr(trace) if "trace" in form else None, 0.0, flags, g.stream())
+        g.sync()
+        assert capi.load().wd_moe_scratch_status(sc.h) == 0, limit
+        assert np.array_equal(sc.get("ids", k, np.int32), d["ids"]) and g.same_bits(sc.get("weights", k, np.float32), d["weights"])
+        assert g.same_bits(g.host(out), want), limit
+    sc.close()

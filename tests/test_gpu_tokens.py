@@ -258,10 +258,12 @@ def test_bounded_wait_of_a_token_batch(g, oracle, gate, F):
 
 
 @pytest.mark.parametrize("E,k", [(64, 6), (512, 10), (640, 10)])
-@pytest.mark.parametrize("preselected", [False, True])
-def test_logits_that_are_late_are_reported(g, oracle, E, k, preselected):
-    """With a wait limit of one poll the workgroup that selects a token's experts may find logits missing (the parts are launched
-    apart, so nobody else waits): a token's results are then NaN with its status word set, and the oracle's where it is clear."""
+@pytest.mark.parametrize("form", ["one launch", "split", "preselected"])
+def test_logits_that_are_late_are_reported(g, oracle, E, k, form):
+    """With a wait limit of one poll the workgroup that selects a token's experts may find logits missing, and those that wait for the ids the
+    ids: a token's results are then NaN with its status word set, and the oracle's where it is clear.  Where nobody in the dispatch
+    waits for the ids - the routed part is a launch of its own, or the ids are given - nothing is ever late."""
+    preselected = form == "preselected"
     H, F, T = 512, 64, 5
     L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=34, router_sigma=1.0 / np.sqrt(H))
     xs = correlated_tokens(H, T, 10)
@@ -270,7 +272,7 @@ def test_logits_that_are_late_are_reported(g, oracle, E, k, preselected):
     dx, out = g.dev(xs), g.empty((T, H), np.float32)
     lib = capi.load()
     ids, wts = np.arange(k, dtype=np.int32), np.full(k, 0.125, np.float32)
-    flags = capi.MOE_PRESELECTED if preselected else capi.MOE_SPLIT_AB
+    flags = {"one launch": 0, "split": capi.MOE_SPLIT_AB, "preselected": capi.MOE_PRESELECTED}[form]
     want = [oracle.moe_layer(L, x, ids=ids, weights=wts)[0] if preselected else oracle.moe_layer(L, x)[0] for x in xs]
     for limit in (1,) * 12 + (0,):
         for s in scr:
@@ -283,7 +285,7 @@ def test_logits_that_are_late_are_reported(g, oracle, E, k, preselected):
         g.sync()
         for t, s in enumerate(scr):
             late = lib.wd_moe_scratch_status(s.h)
-            assert late in ((0, 1) if limit else (0,))
+            assert late in ((0, 1) if limit and form == "one launch" else (0,))
             assert np.isnan(g.host(out)[t]).all() if late else g.same_bits(g.host(out)[t], want[t]), (limit, t)
     for s in scr:
         s.close()

@@ -1,5 +1,5 @@
 // Fused MoE layer: two dispatches per layer (three when the caller asks for the split form).
-//   AB router logits (+ shared-expert gate logit), a wave or two per row; the dispatch's first workgroup waits for
+//   AB router logits (+ shared-expert gate logit), a wave or two per row; a workgroup behind them waits for
 //      them, runs softmax/top-k and publishes the ids inside the dispatch; the shared expert's gate/up + SwiGLU and
 //      the routed gate/up + SwiGLU run in the same launch: the routed workgroups quantise x and stage the
 //      codebooks while the router runs and pick the ids up as soon as they appear - or request their weights at
@@ -39,8 +39,8 @@ struct LayerArgs {
     int hc, hc_round_half;
     int dry;                     // measurement aid: every workgroup returns at once
     int preselected;
-    int n_select_wgs;            // workgroups of dispatch AB that select: one, or none,
-    int n_router_wgs;            // those that take router rows,
+    int n_router_wgs;            // workgroups of dispatch AB that take router rows,
+    int n_select_wgs;            // those that wait for these and select: one, or none,
     int n_shared_wgs;            // those that take the shared expert's gate/up (the rest: routed gate/up)
     int n_routed_items;          // (expert rung, group of eight rows) items shared by the routed workgroups
     const int32_t *ids_known;    // null, or the k ids where they are known before the launch
@@ -51,7 +51,8 @@ struct LayerArgs {
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
     int close_hand;              // no dispatch C follows: the router workgroups set `hand` back themselves
     unsigned *status;            // [0] set to 1 when a bounded wait inside a dispatch ran out
-    unsigned spin_limit;         // polls (about a microsecond each) before such a wait gives up
+    unsigned spin_limit;         // polls (about half a microsecond each) before such a wait gives up,
+    unsigned hand_limit;         // and before the selection's for the logits does (hand_gather)
     unsigned long long *trace;   // profiling aid: null, or [3][16][8] time stamps (100 MHz) of workgroup trace_wg
     int trace_wg;
     // the PART variants of the dispatches also store the exact int32 chunk sums of the routed rows:
@@ -684,11 +685,11 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
 
 // ---- selection inside the dispatch that computes the logits ------------------------------------------------------------
 // Every router wave hands its logit on as a word that cannot be kHandEmpty (hand[e], the shared expert's gate logit in
-// hand[n_slot]; for either side); dispatch C sets the words back.  A workgroup of its own, the dispatch's first, selects: it polls the words until all are
-// there.  No router workgroup waits for its own word, counts itself or looks at the row, and the selection runs where nothing else did
-// before it (its code is in that compute unit's instruction cache from one launch to the next).
+// hand[n_slot]; for either side); dispatch C sets the words back.  A workgroup of its own, behind the router's, selects: it polls the words
+// until all are there.  It waits for workgroups with lower indices only, as every wait inside a dispatch does.  No router workgroup waits for its own word,
+// counts itself or looks at the row.
 // (Selected by the router workgroups that end last - each waits until its words are acknowledged and looks at the row, a ticket names the
-// one to publish - the ids of 2048 / 512 are out 7.2 us after the dispatch's start, by the first workgroup 5.9; 64 experts of 1024 / 256 5.1, 4.4.
+// one to publish - the ids of 2048 / 512 are out 7.2 us after the dispatch's start, by a workgroup of its own 5.9; 64 experts of 1024 / 256 5.1, 4.4.
 // us per layer: 2560 / 640 24.6, so 24.4; 2048 / 512 20.5, 19.9; 1024 / 256 12.0, 11.9.  Four tokens of 2048 / 512, whose router workgroups
 // counted themselves and the last one polled, 40.0, 39.5.)
 struct HandRow {
@@ -718,11 +719,17 @@ WD_DEV void hand_close(uint32_t *hand, int hand_side, int n_slot, int n_wgs, int
     if (!last) return;
     hand_clear(hand, hand_side, n_slot + 2, static_cast<int>(threadIdx.x), static_cast<int>(blockDim.x));
 }
-// lv[j]: logit 64 j + lane, once the row is complete (the limit is there for a broken device: words that did not come are NaN, what is
-// selected then are experts of the layer, and the status makes the results NaN).  Returns whether it was.
+// lv[j]: logit 64 j + lane, once the row is complete (beyond the limit words that did not come are NaN, what is selected then are experts of
+// the layer, and the status makes the results NaN).  Returns whether it was.
+// Another stream's kernel may keep router workgroups from their places for a while.  Where workgroups of the dispatch wait for the ids, these give up
+// after spin_limit polls, 25 ms by default, and the selection, which begins before them, must not do so ahead of them: beyond the tens of microseconds
+// in which the words are due a poll takes 4 us, so the same number of polls is 0.25 s.  Where nobody waits for the ids (they are known before the launch, or the
+// routed part is another one), nobody gives up, so the selection must not either: kHandPatient polls, a quarter of a minute, are there for a broken device.
+constexpr unsigned kHandFastPolls = 64, kHandPatient = 1u << 22;
 template <int M>
 WD_DEV bool hand_gather(const HandRow &r, int lane, float (&lv)[M]) {
     for (unsigned polls = 0; polls < r.limit; ++polls) {
+        if (polls > kHandFastPolls) __builtin_amdgcn_s_sleep(127);
         const uint32_t g = r.gate ? hand_load(r.hand + r.n_slot) : 0u;
         bool there = hand_arrived(g);
 #pragma unroll
@@ -968,7 +975,7 @@ WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__r
 }
 
 // ---- dispatch AB ------------------------------------------------------------------------------------------
-// One workgroup that selects the experts and publishes the ids, n_router_wgs for the router rows,
+// n_router_wgs workgroups for the router rows, one that selects the experts and publishes the ids,
 // then n_shared_wgs workgroups for the shared expert's gate/up; the rest for the routed gate/up, one (expert rung,
 // group of eight rows) item each: a (gate, up) row pair per wave.  The routed workgroups are dispatched after the router
 // ones (lower block index first), quantise x and stage the codebooks while the router runs, then poll the published ids;
@@ -1028,7 +1035,24 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
     const int H = FETCH == 8 ? 2048 : (FETCH == 10 ? 2560 : a.H);
 
     mark<TRACE>(a, blk < a.n_select_wgs + a.n_router_wgs + a.n_shared_wgs ? 0 : 1, 0);
-    if (blk < a.n_select_wgs) {
+    if (blk < a.n_router_wgs) {
+        const int rows = a.preselected ? 0 : a.E;
+        int row;
+        float logit;
+        if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
+            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, a.hand_side, rows, H,
+                                          a.sh_inp, a.E, blk, row);
+        else
+            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, a.hand_side, rows, H, a.sh_inp, a.E, blk, row);
+        mark<TRACE>(a, 0, 1);
+        if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
+        // (no selection: the one wave with the shared gate's row)
+        if (a.preselected && row == a.E && lane == 32) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
+        mark<TRACE>(a, 0, 2);
+        if (a.close_hand) hand_close(a.hand, a.hand_side, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
+        return;
+    }
+    if (blk < a.n_router_wgs + a.n_select_wgs) {
         // results land behind the selection's own scratch
         static_assert(sizeof(s_union) >= kTopkLdsBytes2 + 128, "selection scratch, ids and weights must fit the shared area");
         int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
@@ -1036,7 +1060,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         if (wave == 0) __builtin_amdgcn_s_setprio(3);
         // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
         const uint32_t *const hand = hand_copy(a.hand, a.hand_side);
-        const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
+        const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.hand_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
                                       (TRACE && a.trace) ? a.trace + (0 * 16 + 9) * 8 : nullptr, a.ids_known ? nullptr : a.ids_tagged, a.tag_side);
         if (!there && lane == 0) __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // off the selection's path: the shared expert's gate
@@ -1056,23 +1080,6 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         return;
     }
     const int wg = blk - a.n_select_wgs;
-    if (wg < a.n_router_wgs) {
-        const int rows = a.preselected ? 0 : a.E;
-        int row;
-        float logit;
-        if (kWide)  // two waves per row, four rows per workgroup (the host sizes the grid for it)
-            logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, a.hand_side, rows, H,
-                                          a.sh_inp, a.E, wg, row);
-        else
-            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, a.hand_side, rows, H, a.sh_inp, a.E, wg, row);
-        mark<TRACE>(a, 0, 1);
-        if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
-        // (no selection: the one wave with the shared gate's row)
-        if (a.preselected && row == a.E && lane == 32) a.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
-        mark<TRACE>(a, 0, 2);
-        if (a.close_hand) hand_close(a.hand, a.hand_side, a.E, a.n_select_wgs + a.n_router_wgs, s_last);
-        return;
-    }
 
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ab);
     uint8_t *xscale = lds_ab + H;  // Q8_K: f32 [H/256]; Q8_0: f16 [H/32]

@@ -622,6 +622,7 @@ int launch_ab(const LayerArgs &a, const wd_moe_layer *L, const wd_moe_scratch *s
     m.n_routed_items = routed ? a.k * groups : 0;
     if (!routed) m.ids_tagged = nullptr;  // nobody waits for them inside this launch
     if (!front || a.preselected) m.ids_known = s->ids;
+    m.hand_limit = routed && !m.ids_known ? a.spin_limit : kHandPatient;
     // A compute unit holds three of these workgroups.  The router and shared ones leave well before the ids are
     // published, so a few routed ones that have to wait for their places still start in time.  But when the routed
     // ones alone are more than the device holds at once (hidden 2560: 800 against 768), the surplus would start -
@@ -1218,7 +1219,8 @@ int tokens_pass(const wd_moe_layer *L, const float *d_x, float *d_out, int token
     const int cus = scratch_per_token[0]->compute_units;
     // The parts that `front` and `routed` name
     auto launch_ab = [&](bool front, bool routed) {
-        ta.front_wgs = front ? grid_a : 0, ta.wait_ids = front && routed ? 1 : 0;
+        ta.front_wgs = front ? grid_a : 0, ta.wait_ids = front && routed ? 1 : 0;  // (the ids are not in the scratches then)
+        a.hand_limit = ta.wait_ids ? a.spin_limit : kHandPatient;
         const size_t lds_q8 = std::max(static_cast<size_t>(tokens) * (H + H / 16), sizeof(float) * static_cast<size_t>(H) + 16);
         const dim3 grid_q8(ta.front_wgs + (routed ? std::min(items_b, 2 * cus) : 0));
         switch (L->gate_type) {

@@ -66,12 +66,12 @@ struct TokenArgs {
 };
 
 // ---- dispatch AB for T tokens, first part (A) --------------------------------------------------------------
-// kTokensSelectWgs (none where the ids are given) + T * (router_stride + shared_stride) workgroups, 512 threads, the strides being the router and the
-// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first the workgroups that select, one per token, then the router workgroups
-// of every token, token by token, then the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
+// T * (router_stride + shared_stride) + kTokensSelectWgs (none where the ids are given) workgroups, 512 threads, the strides being the router and the
+// shared workgroups of a token rounded up to a multiple of 8 (tokens_a_grid): first the router workgroups of every token, token by token, then the workgroups
+// that select, one per token, then the shared ones.  The router workgroups are on the pass's critical path and start first; and workgroup w of every
 // token - the same weight rows - lands on the same XCD (workgroups go to the eight XCDs in turn), so its L2 serves the
 // rows to the tokens after the first.  The padding workgroups return at once.  Per token this is the front of the
-// one-token merged dispatch: router rows one per wave, the token's first workgroup waits for them, selects its experts
+// one-token merged dispatch: router rows one per wave, the token's selecting workgroup waits for them, selects its experts
 // and publishes the ids, the other workgroups run the shared expert's gate/up.
 // lds: 4 * H + 16 bytes, x as f32 for the router rows (the shared workgroups use H + H/16 of it); s_work: kTokensWorkBytes of the
 // routed part's tables, for the selection; tiles: the shared rows' eight.
@@ -85,7 +85,7 @@ __host__ __device__ inline TokensAGrid tokens_a_grid(int n_router_wgs, int n_sha
     return TokensAGrid{(n_router_wgs + 7) & ~7, (n_shared_wgs + 7) & ~7};
 }
 constexpr int kTokensWorkBytes = kTopkLdsBytes2 + 128;
-// Selects token t's experts as the first workgroup of the one-token dispatch does.
+// Selects token t's experts as the selecting workgroup of the one-token dispatch does.
 WD_DEV void tokens_select(const TokenArgs &ta, int t, uint8_t *s_work, int lane, int wave) {
     const LayerArgs &a = ta.common;
     const TokenSlots &s = ta.tok[t];
@@ -93,7 +93,7 @@ WD_DEV void tokens_select(const TokenArgs &ta, int t, uint8_t *s_work, int lane,
     float *lds_w = reinterpret_cast<float *>(s_work + kTopkLdsBytes2 + 64);
     if (wave == 0) __builtin_amdgcn_s_setprio(3);
     const uint32_t *const hand = hand_copy(s.hand, s.hand_side);
-    const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.spin_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr,
+    const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.hand_limit}, a.k, a.w_scale, lds_ids, lds_w, nullptr, s_work, lane, wave, nullptr,
                                   ta.wait_ids ? s.tagged : nullptr, s.tag_side);
     if (!there && lane == 0) __hip_atomic_store(s.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (a.sh_inp && wave == 5 && lane == 0) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_load(hand + a.E)));
@@ -117,23 +117,24 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int token, wg;
     {
-        const int first = a.preselected ? 0 : kTokensSelectWgs, b = static_cast<int>(blockIdx.x) - first, router_part = ta.T * gr.router_stride;
-        if (b < 0) {
-            if (static_cast<int>(blockIdx.x) < ta.T) tokens_select(ta, blockIdx.x, s_work, lane, wave);
-            return;
-        }
+        const int router_part = ta.T * gr.router_stride, selecting = a.preselected ? 0 : kTokensSelectWgs;
+        int b = blockIdx.x;
         if (b < router_part) {
             token = b / gr.router_stride, wg = b - token * gr.router_stride;
             if (wg >= a.n_router_wgs) return;
+        } else if (b < router_part + selecting) {
+            token = b - router_part, wg = -1;
+            if (token >= ta.T) return;
         } else {
-            token = (b - router_part) / gr.shared_stride;
-            const int w = b - router_part - token * gr.shared_stride;
+            b -= router_part + selecting;
+            token = b / gr.shared_stride;
+            const int w = b - token * gr.shared_stride;
             if (w >= n_shared_wgs) return;
             wg = a.n_router_wgs + w;
         }
     }
     const TokenSlots &s = ta.tok[token];
-    if (wg < a.n_router_wgs) {
+    if (wg >= 0 && wg < a.n_router_wgs) {
         const int rows = a.preselected ? 0 : a.E;
         int row;
         float logit;
@@ -146,6 +147,7 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         if (a.preselected && row == a.E && lane == 32) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
         return;
     }
+    if (wg < 0) return tokens_select(ta, token, s_work, lane, wave);
     int8_t *xq = reinterpret_cast<int8_t *>(lds_ta);
     uint16_t *xd = reinterpret_cast<uint16_t *>(lds_ta + H);
     const int r = (wg - a.n_router_wgs) * 8 + wave;
