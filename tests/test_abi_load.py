@@ -143,7 +143,7 @@ from warpdecode_amd import capi
 real = capi._fast
 class FailsOnTheWay:
     bound = 0
-    names = staticmethod(real.names)
+    names, signature = staticmethod(real.names), staticmethod(real.signature)
     @classmethod
     def bind(cls, *a):
         if cls.bound == 3: raise MemoryError("on the way")
@@ -162,9 +162,34 @@ assert capi.load() is capi.load()
 """
 
 
-@pytest.mark.parametrize("program", [FIRST_CALLS, LOAD_AGAIN], ids=["several_threads", "after_a_failure"])
+OTHER_PROTOTYPE = """
+from warpdecode_amd import capi
+real, bound = capi._fast, []
+class OfOtherSources:
+    names = staticmethod(real.names)
+    signature = staticmethod(lambda name: "piizppp" if name == "wd_topk_softmax" else real.signature(name))
+    bind = staticmethod(lambda *a: bound.append(a[0]) or real.bind(*a))
+capi._fast = OfOtherSources
+capi.load()
+assert sorted(bound) == sorted(set(real.names()) - {"wd_topk_softmax"}), bound
+try:
+    capi.call("wd_topk_softmax", None, 12, 2, 1.0, None, None, None)
+except capi.WdError as e:
+    assert "multiple of 8" in str(e)
+"""
+
+
+@pytest.mark.parametrize("program", [FIRST_CALLS, LOAD_AGAIN, OTHER_PROTOTYPE], ids=["several_threads", "after_a_failure", "another_prototype"])
 def test_first_load(program):
-    """In a process of its own: the first calls of several threads all get the library's answer, and a load that failed can be tried again."""
+    """In a process of its own: the first calls of several threads all get the library's answer, a load that failed can be tried again, and
+    an entry point that the extension knows with other arguments is called through ctypes."""
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     got = subprocess.run([sys.executable, "-c", program], cwd=root, capture_output=True, text=True, timeout=120)
     assert got.returncode == 0, got.stderr
+
+
+def test_extension_has_these_prototypes():
+    assert len(capi._fast.names()) == 17
+    for name in capi._fast.names():
+        res, args = capi._SIGS[name]
+        assert res is capi.i32 and [capi._CODES[a] for a in args] == list(capi._fast.signature(name)), name

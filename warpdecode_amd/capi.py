@@ -11,7 +11,8 @@ import threading
 
 try:
     from . import _fast
-except ImportError:    # not built: every call goes through ctypes
+    _fast.signature
+except (ImportError, AttributeError):    # not built, or of older sources: every call goes through ctypes
     _fast = None
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -25,6 +26,7 @@ MOE_ONLY_A, MOE_ONLY_B, MOE_ONLY_C, MOE_DRY, MOE_SPLIT_AB = 0x10, 0x20, 0x40, 0x
 MOE_PER_LAYER = 0x200
 
 vp, i32, f32, sz, u32 = C.c_void_p, C.c_int, C.c_float, C.c_size_t, C.c_uint
+_CODES = {vp: "p", i32: "i", f32: "f", sz: "z"}   # as in _fast.signature
 
 
 class WdError(RuntimeError):
@@ -206,9 +208,9 @@ def _load():
         fn.restype, fn.argtypes = res, args
     if _fast:
         for name in _fast.names():
-            if not set(_SIGS[name][1]) <= {vp, i32, f32, sz}:
-                raise WdError("_fast does not take the arguments of " + name)
-            _fast.bind(name, C.cast(getattr(lib, name), vp).value)
+            # (only where it was compiled with the arguments that ctypes would pass)
+            if name in _SIGS and _SIGS[name][0] is i32 and "".join(_CODES.get(t, "?") for t in _SIGS[name][1]) == _fast.signature(name):
+                _fast.bind(name, C.cast(getattr(lib, name), vp).value)
     _lib = lib
 
 

@@ -14,6 +14,7 @@
 
 #include <cstring>
 #include <tuple>
+#include <type_traits>
 #include <utility>
 
 #include "../../include/warpdecode_amd.h"
@@ -89,12 +90,23 @@ struct Bound<int(P...)> {
     }
 };
 
+// A letter per argument, from which the caller tells whether the prototype is the one it would use.
+template <typename T>
+constexpr char code_of = std::is_pointer_v<T> ? 'p' : std::is_same_v<T, int> ? 'i' : std::is_same_v<T, float> ? 'f' : std::is_same_v<T, size_t> ? 'z' : '?';
+template <typename F>
+struct Codes;
+template <typename... P>
+struct Codes<int(P...)> {
+    static constexpr char text[] = {code_of<P>..., 0};
+};
+
 struct Entry {
     const char *name;
+    const char *codes;
     Thunk thunk;
     void *fn;
 };
-#define WD_BIND(f) {#f, Bound<decltype(f)>::run, nullptr}
+#define WD_BIND(f) {#f, Codes<decltype(f)>::text, Bound<decltype(f)>::run, nullptr}
 Entry g_entries[] = {
     WD_BIND(wd_q8_k_quantize_f32),    WD_BIND(wd_q8_0_quantize_f32),   WD_BIND(wd_q8_0_quantize_f16),
     WD_BIND(wd_q8_1_quantize_f32),    WD_BIND(wd_gemv_q8_0_q8_1_f32),  WD_BIND(wd_gemv_q8_k_f32),
@@ -155,6 +167,15 @@ PyObject *names(PyObject *, PyObject *) {
     }
     return list;
 }
+// signature(name) -> the arguments that bind() takes an entry point to have: p(ointer), i(nt), f(loat), z (size_t)
+PyObject *signature(PyObject *, PyObject *args) {
+    const char *name;
+    if (!PyArg_ParseTuple(args, "s", &name)) return nullptr;
+    for (const Entry &e : g_entries)
+        if (std::strcmp(e.name, name) == 0) return PyUnicode_FromString(e.codes);
+    PyErr_Format(PyExc_ValueError, "warpdecode_amd._fast: no %s here", name);
+    return nullptr;
+}
 // bind(name, address): calls of this entry point go to the address from now on.  The same address may be bound again (a load that failed
 // on the way is tried once more), another one may not.
 PyObject *bind(PyObject *, PyObject *args) {
@@ -182,6 +203,7 @@ PyMethodDef g_methods[] = {
      "call(name, *args): the entry point of that name; capi.check's error where it reports one"},
     {"prepare", prepare, METH_VARARGS, "prepare(slow, check, c_void_p, Array)"},
     {"names", names, METH_NOARGS, "the entry points that bind takes"},
+    {"signature", signature, METH_VARARGS, "signature(name): a letter per argument, p, i, f or z"},
     {"bind", bind, METH_VARARGS, "bind(name, address)"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_fast", "capi.call without ctypes' argument conversion", -1, g_methods, nullptr, nullptr, nullptr, nullptr};
