@@ -4,10 +4,11 @@ import ctypes as C
 import os
 import subprocess
 import sys
+import sysconfig
 
 import pytest
 
-from warpdecode_amd import capi, synth
+from warpdecode_amd import build, capi, synth
 
 
 def test_exports_every_declared_symbol():
@@ -188,7 +189,8 @@ def test_first_load(program):
     assert got.returncode == 0, got.stderr
 
 
-def test_extension_has_these_prototypes():
+def test_extension_belongs_to_this_interpreter_and_these_prototypes():
+    assert capi._fast.__file__ == build.FAST and build.FAST.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
     assert len(capi._fast.names()) == 17
     for name in capi._fast.names():
         res, args = capi._SIGS[name]

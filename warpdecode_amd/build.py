@@ -7,7 +7,8 @@ import sysconfig
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libwarpdecode_amd.so")
-FAST = os.path.join(HERE, "_fast.so")   # capi.call for the stand-alone operators (csrc/wd_python.cpp)
+# capi.call for the stand-alone operators (csrc/wd_python.cpp), under a name that only this interpreter's version imports
+FAST = os.path.join(HERE, "_fast" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -22,12 +23,20 @@ def build(verbose=False):
     if verbose:
         print(" ".join(cmd))
     subprocess.check_call(cmd)
+    build_fast(verbose)
+    return LIB
+
+
+def build_fast(verbose=False):
+    for old in (FAST, os.path.join(HERE, "_fast.so")):   # never one of older sources beside a newer library
+        if os.path.exists(old):
+            os.remove(old)
     cmd = ["g++", "-std=c++17", "-O2", "-Wall", "-Wextra", "-fPIC", "-shared", "-I" + sysconfig.get_paths()["include"],
            os.path.join(CSRC, "wd_python.cpp"), "-o", FAST]
     if verbose:
         print(" ".join(cmd))
     subprocess.check_call(cmd)
-    return LIB
+    return FAST
 
 
 def build_host_test(verbose=False):
