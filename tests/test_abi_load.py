@@ -195,3 +195,18 @@ def test_extension_belongs_to_this_interpreter_and_these_prototypes():
     for name in capi._fast.names():
         res, args = capi._SIGS[name]
         assert res is capi.i32 and [capi._CODES[a] for a in args] == list(capi._fast.signature(name)), name
+
+
+@pytest.mark.parametrize("missing", ["header", "compiler"])
+def test_a_machine_that_cannot_build_the_extension(monkeypatch, tmp_path, capfd, missing):
+    """It is left out, with a word on stderr and without an older one staying behind."""
+    monkeypatch.setattr(build, "HERE", str(tmp_path))
+    monkeypatch.setattr(build, "FAST", str(tmp_path / "_fast.old"))
+    for name in ("_fast.old", "_fast.so"):
+        (tmp_path / name).write_bytes(b"of older sources")
+    if missing == "header":
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    else:
+        monkeypatch.setenv("PATH", str(tmp_path))
+    assert build.build_fast() is None
+    assert not os.listdir(tmp_path) and "not built" in capfd.readouterr().err

@@ -28,6 +28,7 @@ def build(verbose=False):
 
 
 def build_fast(verbose=False):
+    """The extension, or None where this machine cannot build one (no Python.h, say): calls then go through ctypes."""
     for old in (FAST, os.path.join(HERE, "_fast.so")):   # never one of older sources beside a newer library
         if os.path.exists(old):
             os.remove(old)
@@ -35,7 +36,11 @@ def build_fast(verbose=False):
            os.path.join(CSRC, "wd_python.cpp"), "-o", FAST]
     if verbose:
         print(" ".join(cmd))
-    subprocess.check_call(cmd)
+    try:
+        subprocess.check_call(cmd)
+    except (OSError, subprocess.CalledProcessError) as e:
+        print("warpdecode_amd._fast is not built, calls go through ctypes: %s" % e, file=sys.stderr)
+        return None
     return FAST
 
 
