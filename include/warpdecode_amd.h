@@ -234,9 +234,10 @@ int32_t *wd_moe_scratch_down_partials(wd_moe_scratch *s);
 int wd_moe_scratch_enable_partials(wd_moe_scratch *s, int gate_type, int down_type);
 
 /* Profiling aid: makes the fused layer dispatches record 100 MHz time stamps of workgroup `wg` and returns the
- * device buffer (NULL on failure): uint64 [3][16][8] = [dispatch][wave][point]; dispatch 0 = router and shared
- * workgroups of the merged launch (wave rows 8 and 9: begin/end and the phases of the selection), 1 = routed gate/up
- * workgroups, 2 = dispatch C.  Only the traced workgroup pays for it.
+ * device buffer (NULL on failure): uint64 [3][16][8] = [dispatch][wave][point]; dispatch 0 = router, selecting and shared
+ * workgroups of the merged launch, 1 = its routed gate/up workgroups (block indices in this order), 2 = dispatch C.  Wave rows 8 and
+ * 9 of dispatch 0, whichever workgroup is traced: begin (point 0) and end (1) of the selecting workgroup; the phases of the selection
+ * (row 9, point 0: every logit has been seen).  Only the traced and the selecting workgroup pay for it.
  * Counterpart of the reference's kernel profiler sites, src/qwen38_moe.cuh:296-535. */
 unsigned long long *wd_moe_scratch_trace(wd_moe_scratch *s, int wg);
 /* The same for the one-launch form of wd_moe_stack_f32: uint64 [12][16] = [wave][point] of workgroup `wg` in layer

@@ -564,3 +564,27 @@ def test_where_nobody_waits_for_the_ids_nothing_gives_up(g, oracle, E, k, form):
         assert np.array_equal(sc.get("ids", k, np.int32), d["ids"]) and g.same_bits(sc.get("weights", k, np.float32), d["weights"])
         assert g.same_bits(g.host(out), want), limit
     sc.close()
+
+
+@pytest.mark.parametrize("E,k", [(64, 6), (640, 10)])
+def test_time_stamps_of_the_selection(g, E, k):
+    """Whichever workgroup is traced: the selecting one begins, sees every logit, and ends, in this order, on the launch's own clock."""
+    H, F = 1024, 64
+    L = synth.make_layer(H, F, E, k, synth.IQ3_S, synth.Q8_0, True, seed=SEED, layer=982, router_sigma=1.0 / np.sqrt(H))
+    dl, sc = g.DeviceLayer(L), g.Scratch(H, F, E, k)
+    dx, out = g.dev(synth.rms_normed(synth.rng_for(SEED, 73, E), H)), g.empty(H, np.float32)
+    n_router = (E + 1 + 7) // 8
+    for wg in (0, n_router, n_router + 1):
+        at = capi.load().wd_moe_scratch_trace(sc.h, wg)
+
+        def stamps():    # of dispatch 0; (row 15 holds no times)
+            return g.view(at, 128, np.uint64).reshape(16, 8)[:15]
+        for turn in range(2):    # (the second pass overwrites the first one's)
+            before = int(stamps().max())
+            capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), sc.h, 0, g.stream())
+            g.sync()
+            st = stamps()
+            begin, seen, end, mine = int(st[8, 0]), int(st[9, 0]), int(st[8, 1]), int(st[0, 0])
+            assert before < begin <= seen <= end and before < mine, (wg, turn)
+            assert abs(begin - mine) < 100 * 1000, (wg, turn)    # (100 MHz: a millisecond)
+    sc.close()

@@ -1058,6 +1058,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         int32_t *lds_ids = reinterpret_cast<int32_t *>(s_union + kTopkLdsBytes2);
         float *lds_w = reinterpret_cast<float *>(s_union + kTopkLdsBytes2 + 64);
         if (wave == 0) __builtin_amdgcn_s_setprio(3);
+        if (TRACE && a.trace && threadIdx.x == 0) a.trace[(0 * 16 + 8) * 8 + 0] = wall_clock64();
         // the selection itself publishes the replicas that the routed workgroups wait for, ahead of the weights
         const uint32_t *const hand = hand_copy(a.hand, a.hand_side);
         const bool there = topk_block(HandRow{hand, a.E, a.E, a.sh_inp != nullptr, a.hand_limit}, a.k, a.w_scale, lds_ids, lds_w, a.ids_override, s_union, lane, wave,
