@@ -689,9 +689,11 @@ WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, i
 // until all are there.  It waits for workgroups with lower indices only, as every wait inside a dispatch does.  No router workgroup waits for its own word,
 // counts itself or looks at the row.
 // (Selected by the router workgroups that end last - each waits until its words are acknowledged and looks at the row, a ticket names the
-// one to publish - the ids of 2048 / 512 are out 7.2 us after the dispatch's start, by a workgroup of its own 5.9; 64 experts of 1024 / 256 5.1, 4.4.
-// us per layer: 2560 / 640 24.6, so 24.4; 2048 / 512 20.5, 19.9; 1024 / 256 12.0, 11.9.  Four tokens of 2048 / 512, whose router workgroups
-// counted themselves and the last one polled, 40.0, 39.5.)
+// one to publish - the ids of 2048 / 512 are out 7.2 us after the dispatch's start, by a workgroup of its own 5.6; 64 experts of 1024 / 256 5.1, 3.9.
+// us per layer: 2560 / 640 24.64, so 24.39; 2048 / 512 20.0, 19.65; 1024 / 256 11.75, 11.67.  Four tokens of 2048 / 512, whose router workgroups
+// counted themselves and the last one polled, 39.95, 39.55.)
+// (By the last router workgroup where nobody waits for the ids, whichever the others do: split 2048 / 512 24.8, by a workgroup of its own 23.4; split
+// 2560 / 640 30.5, 28.3; dispatch A alone 8.8, 7.6 and 9.9, 8.9.)
 struct HandRow {
     const uint32_t *hand;  // the copy of the reader's side
     int n, n_slot;
