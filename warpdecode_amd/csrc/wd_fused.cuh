@@ -49,7 +49,7 @@ struct LayerArgs {
     uint32_t *ids_tagged;        // selected ids published inside the merged dispatch (kTagInvalid = not yet): [kTagCopies / 2][16] for side 0,
     int tag_side;                // so many words on from these for side 1 (tag_copy)
     int clear_tagged;            // dispatch C resets ids_tagged when it is done with the layer
-    int close_hand;              // no dispatch C follows: the router workgroups set `hand` back themselves
+    int close_hand;              // no dispatch C follows: the router and the selecting workgroups set `hand` back themselves (hand_close)
     unsigned *status;            // [0] set to 1 when a bounded wait inside a dispatch ran out
     unsigned spin_limit;         // polls (about half a microsecond each) before such a wait gives up,
     unsigned hand_limit;         // and before the selection's for the logits does (hand_gather)
