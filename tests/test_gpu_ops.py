@@ -107,6 +107,46 @@ def test_topk_near_tie_at_the_end_of_a_key_cell(g, oracle, n):
     assert np.array_equal(g.host(ids), oi) and g.same_bits(g.host(wts), ow)
 
 
+def _selection_rows(n, k):
+    """Rows at the edges of the counted selection: lists of candidates of one place, of about 32 and of more than 64 (the
+    largest logits all in lanes equal modulo 16), differences around what it accepts, ties at the last place, NaN, infinities."""
+    rng = np.random.default_rng(n * 100 + k)
+    base = rng.normal(0, 1, n).astype(np.float32)
+    for lead in (1, 20, 33, 40, 70):
+        row = base.copy()
+        row[::16][:lead] += np.float32(20)
+        yield row
+    order = np.argsort(base)[::-1]
+    for place in {0, k - 2, k - 1, min(k, n - 1) - 1} - {-1}:
+        if place + 1 >= n:
+            continue
+        for gap in (0.0, 2.0 ** -24, 2.0 ** -20, 2.0 ** -19, 2.0 ** -18, 2.0 ** -17, 2.0 ** -16):
+            row = (base * np.float32(2.0 ** -6)).astype(np.float32)   # a unit in the last place well below the differences
+            row[order[place + 1]] = row[order[place]] - np.float32(gap)
+            yield row
+    for value in (np.float32(np.nan), -np.float32(np.nan), np.float32(-np.inf), np.float32(np.inf)):
+        row = base.copy()
+        row[order[n // 2]] = value
+        yield row
+    yield np.where(np.arange(n) < k, base, np.float32(-np.inf)).astype(np.float32)
+    yield (base * np.float32(60)).astype(np.float32)
+
+
+@pytest.mark.parametrize("n,k", [(8, 1), (8, 8), (16, 15), (56, 6), (64, 11), (64, 12), (72, 8), (128, 10), (256, 12), (264, 8), (504, 10), (512, 11),
+                                 (512, 12), (512, 15)])
+def test_topk_edges_of_the_counted_selection(g, oracle, n, k):
+    for i, logits in enumerate(_selection_rows(n, k)):
+        dl, ids, wts = g.dev(logits), g.empty(k, np.int32), g.empty(k, np.float32)
+        capi.call("wd_topk_softmax", g.ptr(dl), n, k, 1.0, g.ptr(ids), g.ptr(wts), g.stream())
+        g.sync()
+        oi, ow = oracle.route(logits, k, 1.0)
+        if not np.isfinite(ow).all():   # a row of NaN or infinite probabilities: experts of the layer, and no finite weight
+            assert ((g.host(ids) >= 0) & (g.host(ids) < n)).all() and not np.isfinite(g.host(wts)).any(), i
+            continue
+        assert np.array_equal(g.host(ids), oi), (i, g.host(ids), oi)
+        assert g.same_bits(g.host(wts), ow), i
+
+
 def _quant_act(oracle, t, x):
     if t in (synth.IQ3_S, synth.IQ2_S):
         qs, d, _ = oracle.quantize_q8_K(x)

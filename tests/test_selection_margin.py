@@ -98,3 +98,21 @@ def test_accepted_rows_are_the_selection(oracle):
             accepted += 1
             assert np.array_equal(ids, oracle.route(l, k)[0]), (trial, l[crowd])
     assert accepted > 300
+
+
+# ---- the one-wave selection: differences of the logits --------------------------------------------------------------
+def test_differences_of_the_logits_order_the_probabilities(oracle):
+    """The one-wave selection accepts on d = fl(l - l_0) alone: a fall of 2^-19 from one selected logit to the next, of 2^-17 to the
+    first that is not, nothing selected below -69.  The tightest such pairs, through the reference's exponential: separated by
+    the margins above, and by anything that is left, up to the first that is not selected, too."""
+    rng = np.random.default_rng(20261204)
+    d_a = -np.concatenate([rng.uniform(0.0, 69.0, 300_000), 2.0 ** rng.uniform(-18, 6, 300_000)]).astype(np.float32)
+    d_a = d_a[d_a >= np.float32(-69.0)]
+    for gap, margin in ((np.float32(2.0 ** -19), MARGIN), (np.float32(2.0 ** -17), np.float32(1.000004))):
+        d_b = (d_a - gap).astype(np.float32)
+        d_b = np.where((d_a - d_b).astype(np.float32) >= gap, d_b, np.nextafter(d_b, np.float32(-np.inf)))
+        assert np.all((d_a - d_b).astype(np.float32) >= gap)
+        e_a, e_b = oracle.exp_ggml(d_a), oracle.exp_ggml(d_b)
+        assert np.all(e_a >= FLOOR) and np.all(e_a > (e_b * margin).astype(np.float32))
+        below = oracle.exp_ggml((d_b * (1 + rng.uniform(0, 2.0 ** -18, d_b.size))).astype(np.float32))
+        assert np.all(e_a > (below * MARGIN).astype(np.float32))

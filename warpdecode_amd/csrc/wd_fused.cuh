@@ -314,15 +314,20 @@ WD_DEV void topk_wave_m(const float *logits, int n, int k, float w_scale, int32_
     finish_weights(top_mine, id_mine, k, w_scale, ids, weights, override_ids, lane);
 }
 
-// The ids held by lanes 0..k-1 (k <= 16) into the kTagCopies replicas: into every row of 16 lanes first, then four replicas
+// The ids held by lanes 0..k-1 (k <= 16) of every row of lanes into the kTagCopies replicas: four replicas
 // per store instruction, so that the last replica goes out a quarter of the stores after the first.
+WD_DEV void publish_ids_of_rows(int id, int k, uint32_t *tagged, int tag_side, int lane) {
+    const int j = lane & 15, c4 = lane >> 4;
+    if (j >= k) return;
+#pragma unroll
+    for (int c0 = 0; c0 < kTagCopies; c0 += 4)  // (the sides in turn)
+        __hip_atomic_store(tagged + ((c0 & 4) ? tag_side : 0) + ((c0 >> 3) * 4 + c4) * 16 + j, static_cast<uint32_t>(id), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The ids held by lanes 0..k-1 only.
 WD_DEV void publish_ids(int id_mine, int k, uint32_t *tagged, int tag_side, int lane) {
     const wd_uint2v t16 = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(id_mine), static_cast<uint32_t>(id_mine), false, false);
     const wd_uint2v t32 = __builtin_amdgcn_permlane32_swap(t16.x, t16.x, false, false);
-    const int j = lane & 15, c4 = lane >> 4;
-#pragma unroll
-    for (int c0 = 0; c0 < kTagCopies; c0 += 4)  // (the sides in turn)
-        if (j < k) __hip_atomic_store(tagged + ((c0 & 4) ? tag_side : 0) + ((c0 >> 3) * 4 + c4) * 16 + j, t32.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    publish_ids_of_rows(static_cast<int>(t32.x), k, tagged, tag_side, lane);
 }
 
 // The same selection by a workgroup of eight waves (every thread must call it; it contains barriers).
@@ -548,95 +553,146 @@ WD_DEV void topk_wave(const float *logits, int n, int k, float w_scale, int32_t 
 }
 
 // ---- the same selection by ONE wave that holds M = 1, 2, 4 or 8 logits per lane --------------------------------------
-// lv[j] is the logit of expert 64 j + lane (-inf at and beyond n; n <= 64 M, k <= 15).  A single wave's time is the length
-// of its dependent steps, so step A counts instead of searching: every logit becomes a 32-bit key - its bits mapped so that
-// unsigned order is float order, the low nine bits replaced by 511 - expert, so that keys are distinct -; the largest keys
-// of groups of lanes (pairs; quads when a lane has one key) are ranked among themselves by counting, one uniform read, a
-// compare and an add for each; T, the (k+1)-th largest of them, is a lower bound of the (k+1)-th largest key, and the keys
-// not below T - 16 or so of 512 - are compacted into LDS, one per lane, and ranked the same way.  (k + 1 rounds of "largest
-// head of any lane" over sorted lanes took 1.9 us for 512 experts, this 1.1.)
-// The keys order the logits up to their low nine bits, so the result is accepted as the selection only when
-//   * the keys' upper 23 bits are strictly decreasing over the k + 1 - any logit that was not taken then lies below
-//     the grid point at or below the k-th taken logit -, and
-//   * the exponentials e_0 > e_1 > ... > e_(k-1) of the k taken logits and e_k, that of the top of the (k+1)-th key's cell
-//     (its low nine bits set: a logit that was not taken may lie above the (k+1)-th key's own, but not above its cell),
-//     are strictly decreasing by a relative margin: exp_ggml is within two units in the last place of the true
-//     exponential (relative error below 2^-22) on normal results, so every logit that was not taken has an exponential
-//     below e_k (1 + 2^-21), and e_(k-1) > e_k (1 + 2^-18) puts the k-th selected strictly above everything left, also
-//     after the product with the row's 1/sum has been rounded.
+// lv[j] is the logit of expert 64 j + lane (-inf at and beyond n; n <= 64 M, k <= 15).  Everybody behind the selection waits for it and a
+// single wave's time is the length of its dependent steps, so step A counts instead of searching and keeps what is not needed for the
+// ids out of the way:
+//   * every logit becomes a 32-bit key, its bits mapped so that unsigned order is float order;
+//   * the largest keys of the sixteen groups of lanes that are equal modulo 16 are ranked among themselves, four comparisons in each row of
+//     lanes (the rows hold the same sixteen, each turned by four lanes more than the one before); T, the (k+1)-th of them, is a lower bound of the
+//     (k+1)-th largest key.  From k = 12 on sixteen groups exclude too little: 32 groups of lanes equal modulo 32;
+//   * the keys not below T - 18 or so of 512 - are compacted into LDS with their experts and ranked by counting, one half of the wave against the
+//     first sixteen of the list and the other against the second (a longer list, by uniform reads);
+//   * rank r goes to slot r.  Equal keys collide there and leave the slot behind them empty.
+// The slots are accepted as the selection only when the first k are filled, and the (k+1)-th too unless every expert is selected, and the
+// differences d_j = l_j - l_0, as the reference takes them ahead of its exponentials, fall by kSelGap from one to the next and by kSelGapLast from the k-th to the
+// (k+1)-th, and the k-th is not below kSelFloor.  exp_ggml is within two units in the last place of the true exponential (relative error below 2^-22) on
+// normal results, so the exponentials then fall by a factor of more than 1 + 2^-19.5 (1 + 2^-17.2 at the end, where what was not taken may be anything up
+// to the (k+1)-th): probabilities, products with one 1/sum in [2^-10, 1], stay strictly ordered, and exp itself is not needed before the ids are out.
 // Rows the test does not accept (ties, near-ties, NaN, +inf, fewer than k + 1 finite logits, selected exponentials below
 // 2^-100) take the reference's rungs over all probabilities in step B.
+// Alone on the device, from the logits in registers until the ids are on their way: 512 experts of which 10 1,810 cycles (0.75 us), 256 of which
+// 8 1,510, 128 of which 8 1,390, 64 of which 6 1,220.  (Groups of two lanes, keys of 23 bits ranked by uniform reads, a branch for every key that may go
+// into the list, and the exponentials ahead of the ids: 3,770 (1.45 us), 2,970, 2,640, 2,130.  The stack of 48 layers with the router's ids: 795, so 752 us;
+// 64 experts of Q8_0 756, 718; layers of 2560 / 640 24.5, 23.4 each; 64 experts of 1024 / 256 11.7, 11.1.)
 struct SelWaveState {
-    float mx;      // the row's largest logit
-    float e;       // lane j < k: exponential of the j-th largest logit (accepted rows)
-    int id;        // lane j < k: its expert
+    float d;       // every row of lanes, lane j < k of it: the j-th largest logit minus the largest (accepted rows)
+    int id;        // its expert
     bool fast;     // step A accepted the row (the same in every lane)
 };
+constexpr float kSelGap = 0x1p-19f, kSelGapLast = 0x1p-17f, kSelFloor = -69.0f;  // (e^-69 > 2^-100)
+constexpr uint32_t kSelFinite = 0x00800000u;  // keys from here on are above -inf's
 
-// Step A.  Returns with st.fast, and for accepted rows the ids of the selection in lanes 0..k-1 of st.id.
-// Of the scratch it uses the candidates' and the selection's places only (cl, cid, sel, selp).
-template <int M>
+// Step A.  Returns with st.fast, and for accepted rows the ids of the selection in lanes 0..k-1 of every row of lanes of st.id.
+// Of the scratch it uses the candidates' and the selection's places only (rmx, cl, ce; sel, selp).
+// LONG false (k < 12 only): a list of more than 32 is not accepted; fewer registers.
+template <int M, bool LONG = true>
 WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s, int lane, SelWaveState &st) {
-    uint32_t h[M];
-    bool odd = false;
-    float lm = lv[0];
-    uint32_t head = 0u;
+    constexpr int kEq = 32, kUgt = 34, kUge = 35, kOge = 3;  // of the compares into scalar masks
+    uint32_t *const ck = reinterpret_cast<uint32_t *>(s.rmx);  // [64] keys of the candidates,
+    int *const cid = reinterpret_cast<int *>(s.rmx) + 64;      // [64] their experts
+    ck[lane & 31] = 0u;  // (behind the end of the list nothing is ahead of anything)
+    s.sel[lane & 15] = 0;
+    const int j = lane & 15;
+    const unsigned long long first_k = ((1ull << k) - 1ull) * 0x0001000100010001ull;  // lanes 0..k-1 of every row of lanes
+    const float gap_needed = j == k - 1 ? kSelGapLast : kSelGap;
+    uint32_t h[M], head = 0u, least = 0xffffffffu;
 #pragma unroll
-    for (int j = 0; j < M; ++j) {
-        const int id = 64 * j + lane;
-        odd = odd || lv[j] != lv[j];
-        lm = __builtin_fmaxf(lm, lv[j]);
-        const uint32_t b = f_bits(lv[j]);
-        const uint32_t ord = b ^ ((b & 0x80000000u) ? 0xffffffffu : 0x80000000u);  // unsigned order = float order
-        h[j] = id < n ? ((ord & ~0x1ffu) | static_cast<uint32_t>(511 - id)) : 0u;
-        head = max(head, h[j]);
+    for (int i = 0; i < M; ++i) {
+        const uint32_t b = f_bits(lv[i]);
+        h[i] = b ^ (static_cast<uint32_t>(static_cast<int>(b) >> 31) | 0x80000000u);
+        head = max(head, h[i]), least = min(least, h[i]);
     }
-    const float mx = wave_max(lm);
-    constexpr int kGroup = M == 1 ? 4 : 2;
-    head = umax_step<kDppXor1>(head);
-    if (M == 1) head = umax_step<kDppXor2>(head);
+    // (NaN with the sign set is below -inf; others are above +inf and fail as the largest)
+    const unsigned long long below_inf = __builtin_amdgcn_uicmp(kSelFinite - 1u, least, kUgt);
+    auto swap16 = [](uint32_t v) { return __builtin_amdgcn_permlane16_swap(v, v, false, false); };
+    auto swap32 = [](uint32_t v) { return __builtin_amdgcn_permlane32_swap(v, v, false, false); };
+    const wd_uint2v h32 = swap32(head);
+    head = max(h32.x, h32.y);
     int larger = 0;
+    if (!LONG || M == 1 || __builtin_expect(k < 12, 1)) {
+        const wd_uint2v h16 = swap16(head);
+        head = max(h16.x, h16.y);
+        int turned = dpp_i<kDppRor4, 0xa>(static_cast<int>(head), static_cast<int>(head));
+        turned = dpp_i<kDppRor8, 0xc>(turned, turned);
+        larger = static_cast<uint32_t>(turned) > head ? 1 : 0;
+        larger += static_cast<uint32_t>(dpp_i<0x121, 0xf, 0xf, true>(0, turned)) > head ? 1 : 0;
+        larger += static_cast<uint32_t>(dpp_i<0x122, 0xf, 0xf, true>(0, turned)) > head ? 1 : 0;
+        larger += static_cast<uint32_t>(dpp_i<0x123, 0xf, 0xf, true>(0, turned)) > head ? 1 : 0;
+        const wd_uint2v a = swap16(static_cast<uint32_t>(larger));
+        const wd_uint2v b = swap32(a.x + a.y);
+        larger = static_cast<int>(b.x + b.y);
+    } else {
+#pragma nounroll
+        for (int g = 0; g < 32; g += 4) {
 #pragma unroll
-    for (int g = 0; g < 64 / kGroup; ++g) larger += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(head), g * kGroup)) > head ? 1 : 0;
+            for (int u = 0; u < 4; ++u) larger += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(head), g + u)) > head ? 1 : 0;
+        }
+    }
     // (with k groups or fewer that hold experts - at most 64 of these then - every key is a candidate)
-    const unsigned long long at = __builtin_amdgcn_ballot_w64(larger == k);
-    const uint32_t thr = at ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(head), __builtin_ctzll(at))) : 0u;
-    uint32_t *const ck = reinterpret_cast<uint32_t *>(s.cid);
-    int count = 0;
+    const unsigned long long at = __builtin_amdgcn_uicmp(static_cast<uint32_t>(larger), static_cast<uint32_t>(k), kEq);
+    const uint32_t kth = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(head), __builtin_ctzll(at | (1ull << 63))));
+    const uint32_t thr = at ? max(kth, kSelFinite) : kSelFinite;
+    unsigned long long m[M];
+    int first[M + 1];
+    first[0] = 0;
 #pragma unroll
-    for (int j = 0; j < M; ++j) {
-        const bool c = h[j] >= thr && h[j] != 0u;
-        const unsigned long long m = __builtin_amdgcn_ballot_w64(c);
-        const int pos = count + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u)));
-        if (c && pos < 64) ck[pos] = h[j], s.cl[pos] = lv[j];
-        count += static_cast<int>(__builtin_popcountll(m));
+    for (int i = 0; i < M; ++i) m[i] = __builtin_amdgcn_uicmp(h[i], thr, kUge);
+#pragma unroll
+    for (int i = 0; i < M; ++i) first[i + 1] = first[i] + static_cast<int>(__builtin_popcountll(m[i]));
+    const int count = first[M];
+    // every lane writes each of its keys, no branch: what is no candidate, and what a list of more than 32 has too much, goes behind the 32 places
+#pragma unroll
+    for (int i = 0; i < M; ++i) {
+        const int before = first[i] + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m[i] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m[i]), 0u)));
+        const int place = min(h[i] >= thr ? before : 63, lane | 32);
+        ck[place] = h[i], cid[place] = 64 * i + lane;
     }
     wave_lds_fence();
-    const uint32_t key = lane < count ? ck[lane] : 0u;
-    const float key_l = s.cl[lane];
-    const uint32_t top = key | 0x1ffu;  // of the key's cell (mapped back here, ahead of the ranks that decide who needs it)
-    const float cell = bits_f(top & 0x80000000u ? top ^ 0x80000000u : ~top);
-    int rank = 0;
-    const int steps = (min(count, 64) + 3) & ~3;  // lanes past the list hold zero, which is ahead of nothing
-    for (int src = 0; src < steps; src += 4) {
+    uint32_t key = ck[lane & 31];
+    int id = cid[lane & 31], rank = 0;
+    uint4 q[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) rank += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), src + u)) > key ? 1 : 0;
+    for (int i = 0; i < 4; ++i) q[i] = reinterpret_cast<const uint4 *>(ck)[4 * (lane >> 5) + i];
+    asm volatile("" : "+v"(id));  // (asked for here and not where it is used)
+    if (!LONG || __builtin_expect(count <= 32, 1)) {
+        unsigned long long ahead[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            ahead[4 * i] = __builtin_amdgcn_uicmp(q[i].x, key, kUgt), ahead[4 * i + 1] = __builtin_amdgcn_uicmp(q[i].y, key, kUgt),
+            ahead[4 * i + 2] = __builtin_amdgcn_uicmp(q[i].z, key, kUgt), ahead[4 * i + 3] = __builtin_amdgcn_uicmp(q[i].w, key, kUgt);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) rank += __builtin_amdgcn_inverse_ballot_w64(ahead[i]) ? 1 : 0;
+        const wd_uint2v t = swap32(static_cast<uint32_t>(rank));
+        rank = static_cast<int>(t.x + t.y);
+    } else {
+        ck[lane] = 0u;
+        wave_lds_fence();
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+            const int before = first[i] + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m[i] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m[i]), 0u)));
+            if (h[i] >= thr) ck[min(before, 63)] = h[i], cid[min(before, 63)] = 64 * i + lane;  // (a list of more than 64 is not used)
+        }
+        wave_lds_fence();
+        key = ck[lane], id = cid[lane];
+#pragma nounroll
+        for (int src = 0; src < 64; src += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) rank += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), src + u)) > key ? 1 : 0;
+        }
     }
-    if (key != 0u && rank <= k) s.sel[rank] = static_cast<int>(key), s.selp[rank] = rank == k ? cell : key_l;
+    if (key != 0u && rank <= k) s.sel[rank] = static_cast<int>(key), s.selp[rank] = bits_f(static_cast<uint32_t>(id));
     wave_lds_fence();
-    const uint32_t mine = lane <= k && lane < count ? static_cast<uint32_t>(s.sel[lane & 15]) : 0u;  // lane j: the j-th largest key of the row
-    const int idc = 511 - static_cast<int>(mine & 0x1ffu);
-    const bool have = mine != 0u && idc < n;
-    const float l = have ? s.selp[lane & 15] : -INFINITY;
+    const uint32_t mine = static_cast<uint32_t>(s.sel[j]);  // the j-th largest key of the row, 0 if there is none
+    const int idc = static_cast<int>(f_bits(s.selp[j]));
     wave_lds_fence();
-    const float e = (have && l > -INFINITY) ? exp_ggml(l - mx) : 0.0f;
-    const float nxt = dpp_f<kDppShl1>(0.0f, e);  // k + 1 <= 16: these lanes are one row
-    const uint32_t grid = mine >> 9, grid_nxt = static_cast<uint32_t>(dpp_i<kDppShl1>(0, static_cast<int>(grid)));
+    const float l = mine ? bits_f(mine ^ (~static_cast<uint32_t>(static_cast<int>(mine) >> 31) | 0x80000000u)) : -INFINITY;
+    const float d = l - readlane_f(l, 0);
+    const float nxt = dpp_f<kDppShl1>(-INFINITY, d);  // k + 1 <= 16: a row of lanes holds them
+    const unsigned long long apart = __builtin_amdgcn_fcmpf(d - nxt, gap_needed, kOge) & __builtin_amdgcn_fcmpf(d, kSelFloor, kOge);
     // (with every expert selected there is no (k+1)-th, and nothing left that could be above the last)
-    const bool good = lane > k || (lane == k && n == k) || (have && l > -INFINITY &&
-                                   (lane == k || (grid > grid_nxt && e >= 0x1p-100f && e > nxt * (lane == k - 1 ? 1.000004f : 1.000001f))));
-    st.mx = mx, st.e = e, st.id = idc;
-    st.fast = count <= 64 && __builtin_amdgcn_ballot_w64(odd) == 0ull && mx < INFINITY && __builtin_amdgcn_ballot_w64(good) == ~0ull;
+    const unsigned long long filled = __builtin_amdgcn_uicmp(mine, 0u, kUgt) | (n == k ? ~0ull : 0ull);
+    st.d = d, st.id = idc;
+    st.fast = (~apart & first_k) == 0ull && (filled >> k & 1ull) != 0ull && below_inf == 0ull && count <= (LONG ? 64 : 32);
 }
 
 // Step B, first half (any wave that holds the logits; it need not be the wave of step A): every exponential into s.p,
@@ -668,7 +724,7 @@ WD_DEV float sel_wave_denominator(const float (&lv)[M], int n, const TopkLds<1> 
 // 0..k-1 write the weights and the ids (ids_given: id_given instead).
 WD_DEV void sel_wave_weights(int n, int k, float w_scale, const TopkLds<1> &s, int lane, SelWaveState &st, float inv, bool dead,
                              int32_t *ids, float *weights, bool ids_given, int id_given) {
-    float top_mine = st.e * inv;
+    float top_mine = exp_ggml(st.d) * inv;
     int id_mine = st.id;
     if (!st.fast) {
         float v[8];
@@ -765,7 +821,10 @@ WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *id
     if (wave == 0) {
         sel_wave_ids(lv, n, k, s, lane, st);
         WD_STAMP(3);
-        if (st.fast && tagged) publish_ids(override_ids ? id_given : st.id, k, tagged, tag_side, lane);
+        if (st.fast && tagged) {
+            if (override_ids) publish_ids(id_given, k, tagged, tag_side, lane);
+            else publish_ids_of_rows(st.id, k, tagged, tag_side, lane);
+        }
         WD_STAMP(6);
     } else if (wave == 1) {
         bool dead;
@@ -785,7 +844,7 @@ WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *id
 
 // Every thread of the workgroup must call it.  Two waves select where one can hold the row (n <= 512, k <= 15); ids and weights are left in
 // LDS by wave 0.
-// (64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
+// (Before the former's differences: 64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
 // there are experts to select its threshold excludes nobody -; 512 experts, top-10: 2.1, 2.2.)
 WD_DEV bool topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
                        uint8_t *lds, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int tag_side = 0) {

@@ -930,7 +930,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
 #pragma unroll
         for (int j = 0; j < 8; ++j) want[j] = 64 * j + lane < a.E, lv[j] = -INFINITY;
         SelWaveState st;
-        st.mx = 0.0f, st.e = 0.0f, st.id = 0, st.fast = false;
+        st.d = 0.0f, st.id = 0, st.fast = false;
         // all logits of the layer, eight per lane (expert 64 j + lane); patient == false: only until every other wave of the
         // workgroup has handed in its activation.  True when they are all there.
         auto gather_logits = [&](bool patient) {
@@ -944,13 +944,12 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             if (got) res_mark<STAMPS>(a, c, l, 12);
             return got;
         };
-        // the ids to every rung of the grid: replica c, rung j at word c * 16 + j
-        auto publish_ids = [&]() {
-            wave_lds_fence();
+        // the ids to every rung of the grid (lane j of every row of lanes holds the j-th): replica c, rung j at word c * 16 + j
+        auto publish_ids = [&](int id) {
             const int j = lane & 15;
 #pragma unroll
             for (int c0 = 0; c0 < kResIdCopies; c0 += 4)  // (the sides in turn)
-                if (j < a.k) hand_store4(c.hb, idh_off(c.flips, l, (c0 >> 2) & 1) + 64u * ((c0 >> 3) * 4 + (lane >> 4)) + 4u * j, static_cast<uint32_t>(lds_ids[j]));
+                if (j < a.k) hand_store4(c.hb, idh_off(c.flips, l, (c0 >> 2) & 1) + 64u * ((c0 >> 3) * 4 + (lane >> 4)) + 4u * j, static_cast<uint32_t>(id));
             res_mark<STAMPS>(a, c, l, 13);
         };
         // what every fold needs: the weights and the shared expert's gate; the last layer's values for the caller
@@ -988,17 +987,17 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         bool weights_out = false;
         if (r == 0 && !traced) {
             (void)gather_logits(true);
-            sel_wave_ids(lv, a.E, a.k, scratch, lane, st);
+            sel_wave_ids<8, false>(lv, a.E, a.k, scratch, lane, st);
             if (st.fast) {
-                if (lane < a.k) lds_ids[lane] = st.id;
-                publish_ids();
+                publish_ids(st.id);
             } else {
                 // the reference's rungs need every probability, and the rungs of the grid are waiting: no time for the
                 // other wave (which computes the very same values into the same places)
                 bool dead_row;
                 const float inv = sel_wave_denominator(lv, a.E, scratch, lane, dead_row);
                 sel_wave_weights(a.E, a.k, w_scale, scratch, lane, st, inv, dead_row, lds_ids, lds_w, false, 0);
-                publish_ids();
+                wave_lds_fence();
+                publish_ids(lds_ids[lane & 15]);
                 publish_weights();
                 weights_out = true;
             }
@@ -1023,7 +1022,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         if (r == 0 && !traced && !weights_out) weights_from_lds();
         if (r == 0 && traced) {
             if (!got) (void)gather_logits(true);
-            sel_wave_ids(lv, a.E, a.k, scratch, lane, st);
+            sel_wave_ids<8, false>(lv, a.E, a.k, scratch, lane, st);
             res_mark<STAMPS>(a, c, l, 13);
         }
         __syncthreads();  // B3
