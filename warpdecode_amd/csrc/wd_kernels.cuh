@@ -801,7 +801,7 @@ struct Q8sBatch {
     }
     WD_DEV int dot(int i, int nibble) const {
         const uint32_t q = (i & 1) ? w[3 * (i >> 1) + 2] : __builtin_amdgcn_alignbyte(w[3 * (i >> 1) + 1], w[3 * (i >> 1)], 2);
-        return sdot4(KIND == 0 ? q : iq4nl_values((q >> nibble) & 0x0f0f0f0fu), a[i], 0);
+        return sdot4(KIND == 0 ? q : iq4nl_low(q >> nibble), a[i], 0);
     }
 };
 // use(batch, s) for the batches s of a chunk in order.  AHEAD: the next eight blocks are requested from LDS before the
