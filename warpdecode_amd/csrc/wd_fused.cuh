@@ -1271,9 +1271,29 @@ WD_DEV void layer_clear_handed(const LayerArgs &a, int threads) {
 // gate; the residual values that the rows' owner updates at its end (nothing else writes them meanwhile): lane 4c + r
 // holds stream c of row r0 + r.
 struct FoldOps {
-    float w = 0.0f, res = 0.0f, inject = 0.0f;
+    float w = 0.0f, res = 0.0f, stream_w = 0.0f;
     unsigned bad = 0u;  // a bounded wait of this layer pass ran out: the results below are replaced by NaN
 };
+// What the weight of the lane's residual stream is made of, asked for ahead of the dispatch's weights so that it can be
+// worked out (layer_c_stream_weight) while these are on their way and not behind the last barrier.  (2560 / 640, ten Q8_0 experts and the shared one, four streams:
+// 23.9 us per layer behind it, so 23.0.)
+struct StreamOps {
+    float inject = 0.0f;
+    uint64_t entry = 0u;
+};
+WD_DEV StreamOps layer_c_stream_request(const LayerArgs &a, bool folds, int lane) {
+    StreamOps s;
+    if (folds && a.hc > 0) s.inject = a.hc_inject[min(lane >> 2, a.hc - 1)], s.entry = exp2f_entry(lane);
+    return s;
+}
+WD_DEV float layer_c_stream_weight(const LayerArgs &a, const StreamOps &s, bool folds) {
+    float w = 0.0f;
+    if (folds && a.hc > 0) {
+        w = hc_weight_of_wave(s.inject, a.hc, s.entry);
+        asm volatile("" : "+v"(w));  // (here and not where it is used)
+    }
+    return w;
+}
 WD_DEV FoldOps layer_c_fold_request(const LayerArgs &a, int r0, int nrows, int lane) {
     FoldOps o;
     o.bad = __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1282,45 +1302,66 @@ WD_DEV FoldOps layer_c_fold_request(const LayerArgs &a, int r0, int nrows, int l
     if (a.residual) {
         const int c = a.hc > 0 ? min(lane >> 2, a.hc - 1) : 0;
         o.res = a.residual[static_cast<size_t>(c) * a.H + r0 + min(lane & 3, nrows - 1)];
-        if (a.hc > 0) o.inject = a.hc_inject[c];
     }
     return o;
 }
-// Rows r0 .. r0 + nrows - 1 (at most four): matrix m's result for row r0 + q at ybuf[m * stride + q].  One wave.
-WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *ybuf, int stride, int r0, int nrows, int lane) {
+// The weighted sum in order over k <= 16 matrices: y[m * STRIDE] is matrix m's result (memory up to y[15 * STRIDE]), lane m of w its weight.  Behind the
+// last barrier of a dispatch a single wave runs it: results are requested from LDS eight at once, weights are lane reads, and in the
+// last four terms what has no matrix adds -0.0, which leaves every sum as it is.  (A loop that reads term and weight through LDS when it
+// needs them: a layer of 1024 / 256, six of 64 experts and the shared one, 11.09 us, so 10.87.)
+template <int STRIDE>
+WD_DEV float fold_in_order(const float *y, float w, int k) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (half == 1 && k <= 8) break;
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = y[(8 * half + u) * STRIDE];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int m = 8 * half + 4 * q;
+            if (m + 4 <= k) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc = acc + v[4 * q + u] * readlane_f(w, m + u);
+            } else if (m < k) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float prod = v[4 * q + u] * readlane_f(w, m + u);
+                    acc = acc + (m + u < k ? prod : -0.0f);
+                }
+            }
+        }
+    }
+    return acc;
+}
+// A dispatch C's dynamic LDS: the results ([n_act][stride] floats) and behind them what its waves own; at least as much as fold_in_order
+// reads, which is up to fifteen matrices past the last one's.
+constexpr size_t layer_c_lds(size_t n_act, size_t stride, size_t of_waves) {
+    const size_t results = 4 * n_act * stride, read = 4 * (n_act + 15) * stride;
+    return results + of_waves > read ? results + of_waves : read;
+}
+// Rows r0 .. r0 + nrows - 1 (at most four): matrix m's result for row r0 + q at ybuf[m * STRIDE + q].  One wave.
+template <int STRIDE>
+WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *ybuf, int r0, int nrows, int lane) {
     const bool shared = a.sh_inp != nullptr;
     // every lane folds row r0 + (lane & 3); lanes 0..3 store it
     const int row = r0 + lane;
     const bool on = lane < nrows;
-    float acc = 0.0f;
-    for (int m = 0; m < a.k; ++m) {
-        const float wm = lane_get(ops.w, m);
-        const float y = ybuf[m * stride + (lane & 3)];
-        const float prod = y * wm;
-        acc = acc + prod;
-        if (a.expert_out && on) a.expert_out[static_cast<size_t>(m) * a.H + row] = y;
-    }
-    const float gate = lane_get(ops.w, 16);
+    const float *const mine = ybuf + (lane & 3);
+    const float y_shared = shared ? mine[a.k * STRIDE] : 0.0f;
+    float acc = fold_in_order<STRIDE>(mine, ops.w, a.k);
     float o = acc;
     if (shared) {
-        const float y = ybuf[a.k * stride + (lane & 3)];
-        const float prod = y * gate;
+        const float prod = y_shared * readlane_f(ops.w, 16);
         o = acc + prod;
-        if (on) a.down_f32[row] = y;
     }
-    // an expert without a slot was reported by the waves above (or by the dispatch before)
-    unsigned bad = ops.bad;
-    if (a.down.slot_of_expert) bad |= __hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (bad) acc = o = __builtin_nanf("");  // the caller sees the failure in its data, without a synchronisation
-    if (on) {
-        a.accum[row] = acc;
-        a.out[row] = o;
-    }
+    if (ops.bad) acc = o = __builtin_nanf("");  // the caller sees the failure in its data, without a synchronisation
     if (a.residual) {
         if (a.hc > 0) {
             const int c = lane >> 2;
             if (c < a.hc && (lane & 3) < nrows) {
-                const float weighted = o * hc_weight(ops.inject, a.hc);
+                const float weighted = o * ops.stream_w;
                 const float v = ops.res + weighted;
                 a.residual[static_cast<size_t>(c) * a.H + r0 + (lane & 3)] = a.hc_round_half ? round_half(v) : v;
             }
@@ -1329,7 +1370,15 @@ WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *yb
             a.residual[row] = ops.res + scaled;
         }
     }
+    if (!on) return;
+    a.out[row] = o;
+    a.accum[row] = acc;
+    if (shared) a.down_f32[row] = y_shared;
+    if (a.expert_out)
+        for (int m = 0; m < a.k; ++m) a.expert_out[static_cast<size_t>(m) * a.H + row] = mine[m * STRIDE];
 }
+// What a wave's matrix gives: NaN for an expert that has no slot (reported through the status word), so that every sum it goes into is one.
+WD_DEV float or_nan(float y, bool missing) { return missing ? __builtin_nanf("") : y; }
 
 // ---- dispatch C -----------------------------------------------------------------------------------------
 // All down projections of a few output rows per workgroup, a wave per matrix (the k routed down tensors, then the shared
@@ -1339,7 +1388,7 @@ WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *yb
 //
 // k_layer_c: four rows, pass by pass: rows of any length, any number of matrices (waves take the matrices in turn).
 // grid = ceil(H / 4), block = 64 * min(n_act, 16) with n_act = k + 1 matrices (k without the shared expert).
-// dynamic LDS per wave: F bytes + F/32 halves (+ pad), then [n_act][4] floats.
+// dynamic LDS (layer_c_lds): [n_act][4] floats, then per wave F bytes + F/32 halves (+ pad).
 template <int KIND, bool PART = false, bool TRACE = false>
 __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
     extern __shared__ __align__(16) uint8_t lds_c[];
@@ -1348,9 +1397,9 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nwaves = blockDim.x >> 6;
     const size_t per_wave = (static_cast<size_t>(a.F) + a.F / 16 + 15) & ~static_cast<size_t>(15);
-    int8_t *aq = reinterpret_cast<int8_t *>(lds_c + wave * per_wave);
-    uint16_t *ad = reinterpret_cast<uint16_t *>(lds_c + wave * per_wave + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_c + nwaves * per_wave);  // [n_act][4]
+    float *ybuf = reinterpret_cast<float *>(lds_c);  // [n_act][4]
+    int8_t *aq = reinterpret_cast<int8_t *>(lds_c + 16 * n_act + wave * per_wave);
+    uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
     const int r0 = blockIdx.x * 4;
     const int nrows = min(4, a.H - r0);
     const int nb = a.F >> 5;
@@ -1359,12 +1408,15 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
     // for them invalid again (this dispatch reads the plain copy)
     layer_clear_handed(a, blockDim.x);
     mark<TRACE>(a, 2, 0);
+    const StreamOps stream = layer_c_stream_request(a, wave == 0, lane);
     FoldOps ops;
     if (wave == 0) ops = layer_c_fold_request(a, r0, nrows, lane);
+    ops.stream_w = layer_c_stream_weight(a, stream, wave == 0);
     for (int m = wave; m < n_act; m += nwaves) {
         const bool is_shared = m == a.k;
         // m is the same for the whole wave: the id comes through the scalar path
-        const uint8_t *const w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)));
+        bool missing = false;
+        const uint8_t *const w = is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)), missing);
         const bool q8 = KIND == 0 || is_shared;  // the same in every lane
         const uint8_t *const rows = w + static_cast<size_t>(r0) * nb * (q8 ? 34 : 18);
         auto quantise = [&]() {
@@ -1378,12 +1430,12 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
         if (PART && !is_shared) y = q8_rows4<KIND, true>(rows, nrows, nb, aq, ad, tiles[wave], lane, pp, quantise);
         else if (q8) y = q8_rows4<0, false>(rows, nrows, nb, aq, ad, tiles[wave], lane, nullptr, quantise);
         else y = q8_rows4<KIND, false>(rows, nrows, nb, aq, ad, tiles[wave], lane, nullptr, quantise);
-        if ((lane & 15) == 0) ybuf[m * 4 + (lane >> 4)] = y;
+        if ((lane & 15) == 0) ybuf[m * 4 + (lane >> 4)] = or_nan(y, missing);
         mark<TRACE>(a, 2, 2);
     }
     __syncthreads();
     mark<TRACE>(a, 2, 3);
-    if (wave == 0) layer_c_fold(a, ops, ybuf, 4, r0, nrows, lane);
+    if (wave == 0) layer_c_fold<4>(a, ops, ybuf, r0, nrows, lane);
     mark<TRACE>(a, 2, 4);
 }
 
@@ -1398,8 +1450,8 @@ __global__ __launch_bounds__(1024) void k_layer_c(LayerArgs a) {
 // (Hidden 2560, rows of 20 Q8_0 blocks: 13.2 us, in the four-row form with sixteen waves 20.5, here with sixteen 14.8; hidden 2048,
 // 16 blocks: 7.8, 9.7, 7.9; hidden 1024, eight blocks: 6.1, 5.6.)
 // WORDS: the rows come through LDS as aligned words (Q8Rows8Fetch), otherwise a lane loads its own blocks (Q8Rows8Blocks).
-// dynamic LDS: per wave the tile (WORDS: the staging area, which it lies in) and the quantised activation (F bytes + F/32
-// halves, padded), then [n_act][8] floats.
+// dynamic LDS (layer_c_lds): [n_act][8] floats, then per wave the tile (WORDS: the staging area, which it lies in) and the quantised
+// activation (F bytes + F/32 halves, padded).
 template <bool WORDS>
 __host__ __device__ inline uint32_t layer_c8_wave_bytes(int F) {
     static_assert(sizeof(Q8Tile8) <= kQ8Rows8StageBytes, "the tile lies in the staging area");
@@ -1410,18 +1462,20 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
     constexpr int STEPS = (PASSES + 1) / 2;  // of sixteen blocks
     extern __shared__ __align__(16) uint8_t lds_c8[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int n_act = a.k + (a.sh_inp ? 1 : 0), n_waves = TWO ? 9 : max(n_act, 2);
+    const int n_act = a.k + (a.sh_inp ? 1 : 0);
     const uint32_t per_wave = layer_c8_wave_bytes<WORDS>(a.F);
-    uint8_t *stage = lds_c8 + wave * per_wave;
+    float *ybuf = reinterpret_cast<float *>(lds_c8);
+    uint8_t *stage = lds_c8 + 32 * n_act + wave * per_wave;
     Q8Tile8 &tile = *reinterpret_cast<Q8Tile8 *>(stage);
     int8_t *aq = reinterpret_cast<int8_t *>(stage + (WORDS ? kQ8Rows8StageBytes : sizeof(Q8Tile8)));
     uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_c8 + n_waves * per_wave);
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;
     if (a.dry) return;
     layer_clear_handed(a, 64 * (TWO ? 9 : n_act));
     mark<TRACE>(a, 2, 0);
+    const StreamOps stream = layer_c_stream_request(a, wave < 2, lane);
     FoldOps ops;
+    float stream_w = 0.0f;
     int m = TWO ? wave : min(wave, n_act - 1);  // (a second wave without a matrix of its own repeats the first's)
     do {
         int lane = threadIdx.x & 63;
@@ -1435,7 +1489,8 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
             const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
             v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
         }
-        const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)))) +
+        bool missing = false;
+        const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)), missing)) +
                                                 static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
         auto run = [&](auto kind, auto part) {
             constexpr int K = decltype(kind)::value;
@@ -1446,6 +1501,7 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
 #pragma unroll
             for (int i = 0; i < STEPS; ++i)
                 lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
+            if (!TWO || m < 9) stream_w = layer_c_stream_weight(a, stream, wave < 2);
             mark<TRACE>(a, 2, 1);
             Q8Chain ch;
             int32_t *pp = P ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;
@@ -1471,13 +1527,14 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
         if (PART && !is_shared) y = run(std::integral_constant<int, KIND>{}, std::integral_constant<bool, PART>{});
         else if (q8) y = run(std::integral_constant<int, 0>{}, std::false_type{});
         else y = run(std::integral_constant<int, KIND>{}, std::false_type{});
-        if (wave < n_act && (lane & 7) == 0) ybuf[m * 8 + (lane >> 3)] = y;
+        if (wave < n_act && (lane & 7) == 0) ybuf[m * 8 + (lane >> 3)] = or_nan(y, missing);
         m += 9;
     } while (TWO && m < n_act);
     mark<TRACE>(a, 2, 2);
     __syncthreads();
     mark<TRACE>(a, 2, 3);
-    if (wave < 2) layer_c_fold(a, ops, ybuf + 4 * wave, 8, r0 + 4 * wave, 4, lane);
+    ops.stream_w = stream_w;
+    if (wave < 2) layer_c_fold<8>(a, ops, ybuf + 4 * wave, r0 + 4 * wave, 4, lane);
     mark<TRACE>(a, 2, 4);
 }
 
@@ -1489,7 +1546,7 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
 // the first one's are free (all of both at once: 2560 / 640 IQ4_NL 8.9 us, so 8.4; 3072 / 768 Q8_0 13.0, 12.4).  As two workgroups per
 // compute unit the groups take 0.3 us more at 2560 and 2.5 more at 3072 / 1024.  (Figures: layer_c_evenly.)
 // grid = 256, block = 64 max(n_act, 2 GROUPS) with at most 16 matrices; waves 0 .. 2 GROUPS - 1 fold up to four rows each.
-// dynamic LDS: per wave the tile and the quantised activation (layer_c_even_wave_bytes), then [n_act][16] floats.
+// dynamic LDS (layer_c_lds): [n_act][16] floats, then per wave the tile and the quantised activation (layer_c_even_wave_bytes).
 template <int LPR>
 __host__ __device__ inline uint32_t layer_c_even_wave_bytes(int F) {
     return ((static_cast<uint32_t>(sizeof(Q8TileN<LPR>)) + 15) & ~15u) + (static_cast<uint32_t>(F + F / 16 + 15) & ~15u);
@@ -1502,15 +1559,18 @@ __global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int n_act = a.k + (a.sh_inp ? 1 : 0), n_waves = max(n_act, 2 * GROUPS);
     const uint32_t per_wave = layer_c_even_wave_bytes<LPR>(a.F);
-    Q8TileN<LPR> &tile = *reinterpret_cast<Q8TileN<LPR> *>(lds_ce + wave * per_wave);
-    int8_t *aq = reinterpret_cast<int8_t *>(lds_ce + wave * per_wave + ((sizeof(Q8TileN<LPR>) + 15) & ~15u));
+    float *ybuf = reinterpret_cast<float *>(lds_ce);
+    uint8_t *const mine = lds_ce + 64 * n_act + wave * per_wave;
+    Q8TileN<LPR> &tile = *reinterpret_cast<Q8TileN<LPR> *>(mine);
+    int8_t *aq = reinterpret_cast<int8_t *>(mine + ((sizeof(Q8TileN<LPR>) + 15) & ~15u));
     uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_ce + n_waves * per_wave);
     const int R = a.H >> 8, r0 = blockIdx.x * R, nb = a.F >> 5;
     const int rows0 = GROUPS == 1 ? R : (R + 1) >> 1;
     if (a.dry) return;
     layer_clear_handed(a, 64 * n_waves);
+    const StreamOps stream = layer_c_stream_request(a, 4 * wave < R, lane);
     FoldOps ops;
+    float stream_w = 0.0f;
     const int m = min(wave, n_act - 1);  // (a wave without a matrix of its own repeats the last one's)
     const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;
     // (the activation first, as in k_layer_c8)
@@ -1520,7 +1580,8 @@ __global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
         const float *p = a.act + static_cast<size_t>(m) * a.F + min(512 * i + lane * 8, a.F - 8);
         v[2 * i] = *reinterpret_cast<const float4 *>(p), v[2 * i + 1] = *reinterpret_cast<const float4 *>(p + 4);
     }
-    const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)))) +
+    bool missing = false;
+    const uint8_t *const rows = uniform_ptr((is_shared ? a.sh_down : mat_ptr_expert_uniform<0>(a.down, checked_expert(a.down, sld_i32(a.ids + m)), missing)) +
                                             static_cast<size_t>(r0) * nb * (q8 ? 34 : 18));
     auto run = [&](auto kind) {
         constexpr int K = decltype(kind)::value;
@@ -1537,6 +1598,7 @@ __global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
 #pragma unroll
         for (int i = 0; i < STEPS; ++i)
             lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
+        stream_w = layer_c_stream_weight(a, stream, 4 * wave < R);
         wave_lds_fence();
         Q8Chain ch;
 #pragma unroll
@@ -1546,7 +1608,7 @@ __global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
             if (kThen) w[q] = q8_rowsn_load<K, LPR>(rows1, q * LPR, nb, R - rows0, at1);
         }
         const float y0 = q8_rowsn_close<K, LPR>(ch, nb, tile, at0);
-        if (wave < n_act && (lane & 7) == 0 && (lane >> 3) < rows0) ybuf[m * 16 + (lane >> 3)] = y0;
+        if (wave < n_act && (lane & 7) == 0 && (lane >> 3) < rows0) ybuf[m * 16 + (lane >> 3)] = or_nan(y0, missing);
         if constexpr (GROUPS == 1) return;
         ch = Q8Chain();
 #pragma unroll
@@ -1555,12 +1617,13 @@ __global__ __launch_bounds__(1024) void k_layer_c_even(LayerArgs a) {
             q8_rowsn_pass<K, LPR>(w[kBoth ? PASSES + q : q], q * LPR, nb, aq, ad, tile, at1, ch);
         }
         const float y1 = q8_rowsn_close<K, LPR>(ch, nb, tile, at1);
-        if (wave < n_act && (lane & 7) == 0 && (lane >> 3) < R - rows0) ybuf[m * 16 + rows0 + (lane >> 3)] = y1;
+        if (wave < n_act && (lane & 7) == 0 && (lane >> 3) < R - rows0) ybuf[m * 16 + rows0 + (lane >> 3)] = or_nan(y1, missing);
     };
     if (q8) run(std::integral_constant<int, 0>{});
     else run(std::integral_constant<int, KIND>{});
     __syncthreads();
-    if (4 * wave < R) layer_c_fold(a, ops, ybuf + 4 * wave, 16, r0 + 4 * wave, min(4, R - 4 * wave), lane);
+    ops.stream_w = stream_w;
+    if (4 * wave < R) layer_c_fold<16>(a, ops, ybuf + 4 * wave, r0 + 4 * wave, min(4, R - 4 * wave), lane);
 }
 
 }  // namespace wd

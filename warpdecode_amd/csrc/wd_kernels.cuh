@@ -68,10 +68,20 @@ WD_DEV const uint8_t *mat_ptr_expert(const MatSrc &s, int e) {
 
 // The same for an e that is the same in every lane: the slot comes through the scalar path, so the lookup neither
 // waits for nor is counted among the wave's vector loads.
+// `missing` is set when it has none.
+template <int T>
+WD_DEV const uint8_t *mat_ptr_expert_uniform(const MatSrc &s, int e, bool &missing) {
+    if (s.slot_of_expert) {
+        const int slot = sld_i32(s.slot_of_expert + e);
+        missing = slot < 0;
+        return s.pool + checked_slot(s, slot) * s.slot_bytes + s.slot_off[T];
+    }
+    return s.base[T] + static_cast<size_t>(e) * s.stride[T];
+}
 template <int T>
 WD_DEV const uint8_t *mat_ptr_expert_uniform(const MatSrc &s, int e) {
-    if (s.slot_of_expert) return s.pool + checked_slot(s, sld_i32(s.slot_of_expert + e)) * s.slot_bytes + s.slot_off[T];
-    return s.base[T] + static_cast<size_t>(e) * s.stride[T];
+    bool missing;
+    return mat_ptr_expert_uniform<T>(s, e, missing);
 }
 
 __global__ void k_fill_u32(uint32_t *dst, uint32_t v, size_t n) {

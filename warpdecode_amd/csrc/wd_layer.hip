@@ -657,7 +657,7 @@ template <int KIND>
 void launch_layer_c(hipStream_t st, const LayerArgs &a) {
     const int n_act = a.k + (a.sh_inp ? 1 : 0), waves = std::min(n_act, 16);
     const size_t per_wave = (static_cast<size_t>(a.F) + a.F / 16 + 15) & ~static_cast<size_t>(15);
-    const size_t lds = waves * per_wave + sizeof(float) * 4 * n_act;
+    const size_t lds = layer_c_lds(n_act, 4, waves * per_wave);
     const dim3 grid((a.H + 3) / 4), block(64 * waves);
     if (a.down_part)
         enqueue(k_layer_c<KIND, true>, grid, block, lds, st, a);
@@ -669,7 +669,7 @@ void launch_layer_c(hipStream_t st, const LayerArgs &a) {
 template <int KIND, int PASSES, bool WORDS>
 void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
     const int n_act = a.k + (a.sh_inp ? 1 : 0), waves = std::max(n_act, 2);
-    const size_t lds = waves * static_cast<size_t>(layer_c8_wave_bytes<WORDS>(a.F)) + sizeof(float) * 8 * n_act;
+    const size_t lds = layer_c_lds(n_act, 8, waves * static_cast<size_t>(layer_c8_wave_bytes<WORDS>(a.F)));
     const dim3 grid(a.H / 8), block(64 * waves);
     if (a.down_part)
         enqueue(k_layer_c8<KIND, PASSES, WORDS, true>, grid, block, lds, st, a);
@@ -680,7 +680,7 @@ void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
 }
 template <int KIND>
 void launch_layer_c8_two(hipStream_t st, const LayerArgs &a) {
-    const size_t lds = 9 * static_cast<size_t>(layer_c8_wave_bytes<false>(a.F)) + sizeof(float) * 8 * (a.k + 1);
+    const size_t lds = layer_c_lds(a.k + 1, 8, 9 * static_cast<size_t>(layer_c8_wave_bytes<false>(a.F)));
     const dim3 grid(a.H / 8), block(64 * 9);
     if (a.F <= 512)
         enqueue(k_layer_c8<KIND, 2, false, false, false, true>, grid, block, lds, st, a);
@@ -702,7 +702,7 @@ void launch_layer_c_even(hipStream_t st, const LayerArgs &a) {
         if (a.F > 32 * PASSES * LPR) return launch_layer_c_even<KIND, LPR, GROUPS, (PASSES < 4 ? PASSES + 1 : 6)>(st, a);
     }
     const int n_act = a.k + (a.sh_inp ? 1 : 0), waves = std::max(n_act, 2 * GROUPS);
-    const size_t lds = waves * static_cast<size_t>(layer_c_even_wave_bytes<LPR>(a.F)) + sizeof(float) * 16 * n_act;
+    const size_t lds = layer_c_lds(n_act, 16, waves * static_cast<size_t>(layer_c_even_wave_bytes<LPR>(a.F)));
     enqueue(k_layer_c_even<KIND, LPR, GROUPS, PASSES>, dim3(256), dim3(64 * waves), lds, st, a);
 }
 template <int KIND>
@@ -1124,7 +1124,7 @@ void launch_tokens_c_even(const TokenArgs &ta, hipStream_t st) {
     if constexpr (PASSES * LPR < 48) {  // (as in launch_layer_c_even)
         if (ta.common.F > 32 * PASSES * LPR) return launch_tokens_c_even<KIND, LPR, (PASSES < 4 ? PASSES + 1 : 6)>(ta, st);
     }
-    const size_t lds = kTokensCEvenWaves * static_cast<size_t>(layer_c_even_wave_bytes<LPR>(ta.common.F)) + sizeof(float) * 16 * ta.T * (ta.common.k + 1);
+    const size_t lds = layer_c_lds(static_cast<size_t>(ta.T) * (ta.common.k + 1), 16, kTokensCEvenWaves * static_cast<size_t>(layer_c_even_wave_bytes<LPR>(ta.common.F)));
     enqueue(k_tokens_c_even<KIND, LPR, PASSES>, dim3(256), dim3(64 * kTokensCEvenWaves), lds, st, ta);
 }
 // Lanes per row of the form with hidden / 256 rows per workgroup (k_tokens_c_even), 0 where the eight-row form stays: it pays where
@@ -1147,7 +1147,7 @@ void launch_tokens_c_even(int lanes, const TokenArgs &ta, hipStream_t st) {
 template <int KIND, int PASSES>
 void launch_tokens_c(const TokenArgs &ta, hipStream_t st) {
     constexpr int kWaves = kTokensCWaves<PASSES>;
-    const size_t lds = kWaves * static_cast<size_t>(layer_c8_wave_bytes<false>(ta.common.F)) + sizeof(float) * 8 * ta.T * (ta.common.k + 1);
+    const size_t lds = layer_c_lds(static_cast<size_t>(ta.T) * (ta.common.k + 1), 8, kWaves * static_cast<size_t>(layer_c8_wave_bytes<false>(ta.common.F)));
     enqueue(k_tokens_c<KIND, PASSES>, ta.common.H / 8, 64 * kWaves, lds, st, ta);
 }
 template <int KIND>

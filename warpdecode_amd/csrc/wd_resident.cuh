@@ -738,23 +738,13 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
 #pragma unroll
             for (int m = 0; m < kResMaxK; ++m) yv[m] = ybuf[m * 4 + (lane & 3)];
             float ysh = ybuf[kResSharedSlot * 4 + (lane & 3)];
+            // (slots not in use hold -0.0, which leaves every sum as it is: no select between two additions of the one chain that the whole
+            // grid waits for)
             float acc = 0.0f;
-            if (traced && fresh_s(a.k) == kResMaxK) {  // (with a routing trace only: the other form of the role came out slower with it)
-                // (every term in use, the usual case: no select between two additions of the one chain the whole grid waits
-                // for - the compiler keeps the selects' ten lane masks parked in lanes of a vector register and fetches one
-                // back, two instructions and their wait states, per term)
 #pragma unroll
-                for (int m = 0; m < kResMaxK; ++m) {
-                    const float prod = yv[m] * readlane_f(wreg, m);
-                    acc = acc + prod;
-                }
-            } else {
-#pragma unroll
-                for (int m = 0; m < kResMaxK; ++m) {
-                    const float prod = yv[m] * readlane_f(wreg, m);
-                    const float next = acc + prod;
-                    acc = m < a.k ? next : acc;
-                }
+            for (int m = 0; m < kResMaxK; ++m) {
+                const float prod = yv[m] * readlane_f(wreg, m);
+                acc = acc + prod;
             }
             float o = acc;
             if (!shared) ysh = 0.0f;
@@ -1067,6 +1057,7 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(6, 
     // third waves of SIMDs 0 and 1 in one of the two workgroups and of SIMDs 2 and 3 in the other, so that every SIMD
     // of the compute unit carries five of the twenty routed waves.
     if (threadIdx.x < 16) reinterpret_cast<float *>(lds_res + kResLdsActv)[threadIdx.x] = 0.0f;  // slots not in use hand on zeros
+    if (threadIdx.x < 4 * kResMaxK) reinterpret_cast<float *>(lds_res + kResLdsY)[threadIdx.x] = -0.0f;  // and add nothing to the fold (times a weight of +0)
     int *simd_of = reinterpret_cast<int *>(lds_res + kResLdsRoles);
     if (fresh_lane() == 0) simd_of[wave] = static_cast<int>((__builtin_amdgcn_s_getreg(4 | (31 << 11)) >> 4) & 3u);  // HW_ID.SIMD_ID
     __syncthreads();

@@ -619,7 +619,7 @@ WD_DEV void tokens_clear_handed(const TokenArgs &ta, int waves, int tw, int lane
 // rows of 16 blocks, two of eight for longer ones -, so that grids of more than 256 workgroups (hidden > 2048) still run in one round: with two
 // or three items per wave and one workgroup of sixteen waves per compute unit, hidden 2304 took twice the time of 2048.
 // KIND: down tensor kind; PASSES: of eight blocks per row (F <= 256 PASSES).
-// dynamic LDS: per wave the tile and the quantised activation (layer_c8_wave_bytes<false>), then [T][k+1][8] floats.
+// dynamic LDS (layer_c_lds): [T][k+1][8] floats, then per wave the tile and the quantised activation (layer_c8_wave_bytes<false>).
 template <int PASSES>
 constexpr int kTokensCWaves = PASSES <= 2 ? 16 : 8;
 template <int KIND, int PASSES>
@@ -630,10 +630,11 @@ void k_tokens_c(TokenArgs ta) {
     const int lane = threadIdx.x & 63, tw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     constexpr int kWaves = kTokensCWaves<PASSES>, kActs = (PASSES + 1) / 2;
     const uint32_t per_wave = layer_c8_wave_bytes<false>(a.F);
-    Q8Tile8 &tile = *reinterpret_cast<Q8Tile8 *>(lds_tc + tw * per_wave);
-    int8_t *aq = reinterpret_cast<int8_t *>(lds_tc + tw * per_wave + sizeof(Q8Tile8));
+    float *ybuf = reinterpret_cast<float *>(lds_tc);  // [T][k+1][8]
+    uint8_t *const own = lds_tc + 32 * ta.T * (a.k + 1) + tw * per_wave;
+    Q8Tile8 &tile = *reinterpret_cast<Q8Tile8 *>(own);
+    int8_t *aq = reinterpret_cast<int8_t *>(own + sizeof(Q8Tile8));
     uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_tc + kWaves * per_wave);  // [T][k+1][8]
     const bool shared = a.sh_down != nullptr;
     const int per_token = a.k + (shared ? 1 : 0), n_items = ta.T * per_token;
     const int r0 = blockIdx.x * 8, nb = a.F >> 5;  // hidden is a multiple of 8
@@ -690,23 +691,19 @@ void k_tokens_c(TokenArgs ta) {
         const int t = tw;
         const int row = r0 + lane;
         const bool row_on = lane < 8 && row < a.H;
-        float acc = 0.0f;
-        for (int j = 0; j < a.k; ++j) {
-            const float wj = lane_get(wreg, j);
-            const float y = ybuf[(t * (a.k + 1) + j) * 8 + (lane & 7)];
-            const float prod = y * wj;
-            acc = acc + prod;
-            if (s.expert_out && row_on) s.expert_out[static_cast<size_t>(j) * a.H + row] = y;
-        }
-        const float gate = lane_get(wreg, 16);
+        const float *const mine = ybuf + t * (a.k + 1) * 8 + (lane & 7);
+        const float y_shared = shared ? mine[a.k * 8] : 0.0f;
+        const float acc = fold_in_order<8>(mine, wreg, a.k);
+        const float gate = readlane_f(wreg, 16);
         if (row_on) {
             float o = acc;
             if (shared) {
-                const float y = ybuf[(t * (a.k + 1) + a.k) * 8 + lane];
-                const float prod = y * gate;
+                const float prod = y_shared * gate;
                 o = acc + prod;
-                s.down_f32[row] = y;
+                s.down_f32[row] = y_shared;
             }
+            if (s.expert_out)
+                for (int j = 0; j < a.k; ++j) s.expert_out[static_cast<size_t>(j) * a.H + row] = mine[j * 8];
             s.accum[row] = bad == 1u ? __builtin_nanf("") : acc;
             s.out[row] = bad == 1u ? __builtin_nanf("") : o;
         }
@@ -717,7 +714,7 @@ void k_tokens_c(TokenArgs ta) {
 // The same with one workgroup of sixteen waves for every compute unit, hidden / 256 rows each, as in k_layer_c_even: a work item is
 // (token, matrix, group of up to 64 / LPR rows).  (The next item's activation and rows requested while this one is worked on: 2560 / 640,
 // four tokens 63.8 us per layer instead of 61.7, 4096 / 1536 128.8 instead of 119.2.)  Where it is taken and what it measures: tokens_c_even_lanes.
-// grid = 256.  dynamic LDS: per wave the tile and the quantised activation (layer_c_even_wave_bytes), then [T][k+1][16] floats.
+// grid = 256.  dynamic LDS (layer_c_lds): [T][k+1][16] floats, then per wave the tile and the quantised activation (layer_c_even_wave_bytes).
 constexpr int kTokensCEvenWaves = 16;
 template <int KIND, int LPR, int PASSES>
 __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenArgs ta) {
@@ -726,10 +723,11 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
     const LayerArgs &a = ta.common;
     const int lane = threadIdx.x & 63, tw = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const uint32_t per_wave = layer_c_even_wave_bytes<LPR>(a.F);
-    Q8TileN<LPR> &tile = *reinterpret_cast<Q8TileN<LPR> *>(lds_tc + tw * per_wave);
-    int8_t *aq = reinterpret_cast<int8_t *>(lds_tc + tw * per_wave + ((sizeof(Q8TileN<LPR>) + 15) & ~15u));
+    float *ybuf = reinterpret_cast<float *>(lds_tc);  // [T][k+1][16]
+    uint8_t *const own = lds_tc + 64 * ta.T * (a.k + 1) + tw * per_wave;
+    Q8TileN<LPR> &tile = *reinterpret_cast<Q8TileN<LPR> *>(own);
+    int8_t *aq = reinterpret_cast<int8_t *>(own + ((sizeof(Q8TileN<LPR>) + 15) & ~15u));
     uint16_t *ad = reinterpret_cast<uint16_t *>(aq + a.F);
-    float *ybuf = reinterpret_cast<float *>(lds_tc + kWaves * per_wave);  // [T][k+1][16]
     const bool shared = a.sh_down != nullptr;
     const int rows_per_wg = a.H >> 8, r0 = blockIdx.x * rows_per_wg, nb = a.F >> 5;
     const int n_groups = rows_per_wg * LPR > 64 ? 2 : 1, rows0 = n_groups == 2 ? (rows_per_wg + 1) >> 1 : rows_per_wg;
@@ -806,23 +804,19 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
         const int t = tw;
         const int row = r0 + lane;
         const bool row_on = lane < rows_per_wg;
-        float acc = 0.0f;
-        for (int j = 0; j < a.k; ++j) {
-            const float wj = lane_get(wreg, j);
-            const float y = ybuf[(t * (a.k + 1) + j) * 16 + (lane & 15)];
-            const float prod = y * wj;
-            acc = acc + prod;
-            if (s.expert_out && row_on) s.expert_out[static_cast<size_t>(j) * a.H + row] = y;
-        }
-        const float gate = lane_get(wreg, 16);
+        const float *const mine = ybuf + t * (a.k + 1) * 16 + (lane & 15);
+        const float y_shared = shared ? mine[a.k * 16] : 0.0f;
+        const float acc = fold_in_order<16>(mine, wreg, a.k);
+        const float gate = readlane_f(wreg, 16);
         if (row_on) {
             float o = acc;
             if (shared) {
-                const float y = ybuf[(t * (a.k + 1) + a.k) * 16 + lane];
-                const float prod = y * gate;
+                const float prod = y_shared * gate;
                 o = acc + prod;
-                s.down_f32[row] = y;
+                s.down_f32[row] = y_shared;
             }
+            if (s.expert_out)
+                for (int j = 0; j < a.k; ++j) s.expert_out[static_cast<size_t>(j) * a.H + row] = mine[j * 16];
             s.accum[row] = bad == 1u ? __builtin_nanf("") : acc;
             s.out[row] = bad == 1u ? __builtin_nanf("") : o;
         }
