@@ -281,6 +281,7 @@ typedef uint32_t __attribute__((aligned(2))) wd_u32a;
 typedef uint32_t wd_u64a __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t wd_u128a __attribute__((ext_vector_type(4), aligned(2)));
 #define WD_GLOBAL __attribute__((address_space(1)))
+WD_DEV float gld_f32(const float *p) { return *((const WD_GLOBAL float *)(p)); }
 WD_DEV uint32_t gld_u8(const uint8_t *p) { return *((const WD_GLOBAL uint8_t *)(p)); }
 WD_DEV uint16_t gld_u16(const uint8_t *p) { return *((const WD_GLOBAL wd_u16a *)(p)); }
 WD_DEV uint32_t gld_u32(const uint8_t *p) { return *((const WD_GLOBAL wd_u32a *)(p)); }

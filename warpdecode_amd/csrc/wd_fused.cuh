@@ -915,24 +915,25 @@ WD_DEV void router_span_load(const float *wr, int c0, const RouterSpan &sp, bool
     for (int g = 0; g < 4; ++g) {
         const float *p = wr + (c0 + t + (upper ? (g < sp.upper ? 1024 + 256 * g : 0) : (g < sp.lower ? 256 * g : 0)));
 #pragma unroll
-        for (int u = 0; u < 8; ++u) wv[8 * g + u] = p[32 * u];
+        for (int u = 0; u < 8; ++u) wv[8 * g + u] = gld_f32(p + 32 * u);
     }
 }
-// A half's multiply-adds of the span, continuing the chain from v; x: the half's first column of the lane.
-WD_DEV float router_span_run(const float (&wv)[32], const float *x, int groups, float v) {
-    float xv[2][8];
-    auto read = [&](int g) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) xv[g & 1][u] = x[256 * max(min(g, groups - 1), 0) + 32 * u];
-    };
-    if (groups == 0) return v;
-    read(0);
+// The values of x that the lane's weights of the span meet, all at once.  x: the half's first column of the lane.
+WD_DEV void router_span_x(const float *x, const RouterSpan &sp, bool upper, float (&xv)[32]) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-        if (g < 3) read(g + 1);
+        const float *p = x + 256 * max(min(g, (upper ? sp.upper : sp.lower) - 1), 0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) xv[8 * g + u] = p[32 * u];
+    }
+}
+// A half's multiply-adds of the span, continuing the chain from v.
+WD_DEV float router_span_run(const float (&wv)[32], const float (&xv)[32], int groups, float v) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
         if (g < groups) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v = __builtin_fmaf(wv[8 * g + u], xv[g & 1][u], v);
+            for (int u = 0; u < 8; ++u) v = __builtin_fmaf(wv[8 * g + u], xv[8 * g + u], v);
         }
     }
     return v;
@@ -942,11 +943,24 @@ WD_DEV void router_hand_on(float logit, uint32_t *hand, int hand_side, int slot,
     const uint32_t word = hand_word_bits(f_bits(readlane_f(logit, 32)));
     if (lane < 2) __hip_atomic_store(hand + (lane == 0 ? 0 : hand_side) + slot, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// x to LDS, by the whole workgroup.
-WD_DEV void router_stage_x(const float *__restrict__ x, float *xs, int cols) {
-    for (int i = static_cast<int>(threadIdx.x) * 4; i < cols; i += static_cast<int>(blockDim.x) * 4)
-        *reinterpret_cast<float4 *>(xs + i) = *reinterpret_cast<const float4 *>(x + i);
-}
+// x to LDS, by the whole workgroup of 512 threads.  The first 4096 columns are requested ahead of the row's weights: loads return in order, and so x is in LDS and in the
+// lanes' registers (router_span_x) while the weights are on their way.  (Behind them, and x read from LDS
+// between the multiply-adds, us per layer: 2048 / 512 18.7, so 18.4; 2560 / 640 22.9, 22.5; 1024 / 1024 17.6, 17.3; four tokens of 2048 / 512 38.2, 37.8.)
+struct RouterX {
+    float4 first, second = make_float4(0.f, 0.f, 0.f, 0.f);
+    WD_DEV RouterX(const float *__restrict__ x, int cols) {
+        const int i = static_cast<int>(threadIdx.x) * 4;
+        first = *reinterpret_cast<const float4 *>(x + min(i, cols - 4));
+        if (cols > 2048) second = *reinterpret_cast<const float4 *>(x + min(i + 2048, cols - 4));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    WD_DEV void stage(const float *__restrict__ x, float *xs, int cols) const {
+        const int i = static_cast<int>(threadIdx.x) * 4;
+        if (i < cols) *reinterpret_cast<float4 *>(xs + i) = first;
+        if (i + 2048 < cols) *reinterpret_cast<float4 *>(xs + i + 2048) = second;
+        for (int j = i + 4096; j < cols; j += 2048) *reinterpret_cast<float4 *>(xs + j) = *reinterpret_cast<const float4 *>(x + j);
+    }
+};
 
 // One row per wave, x staged once per workgroup in LDS (f32 [cols]).
 // Accumulator t (of ggml's 4 x 8) of the row lives in lanes t and t + 32: for every span of 2048 columns lane t
@@ -955,10 +969,8 @@ WD_DEV void router_stage_x(const float *__restrict__ x, float *xs, int cols) {
 // ascending order while a lane holds only 32 weights (half the registers of the 32-lanes-per-row version,
 // which lets three workgroups of the merged dispatch share a compute unit).
 // Every thread of the workgroup must call it (it contains a barrier).
-// SCALAR_ROW: keep the wave's row pointer in scalar registers (two vector registers fewer).
 // The row's result goes to hand[row], the extra row's to hand[extra_slot] (of both sides' copies); it is returned as well (lane 32), with the row in `done`
 // (-1: this wave has none).
-template <bool SCALAR_ROW = false>
 WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restrict__ x, float *xs, uint32_t *hand, int hand_side, int rows,
                               int cols, const float *__restrict__ extra_w, int extra_slot, int wg, int &done) {
     const int lane = threadIdx.x & 63, t = lane & 31;
@@ -967,22 +979,24 @@ WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restri
     const int total = rows + (extra_w ? 1 : 0);
     const bool on = row < total;
     const float *wr = on ? (row < rows ? w + static_cast<size_t>(row) * cols : extra_w) : x;
-    if (SCALAR_ROW) wr = uniform_ptr(wr);  // the row is the same for the whole wave
-    float wv[32];
-    if (on) router_span_load(wr, 0, RouterSpan(cols), upper, t, wv);
-    router_stage_x(x, xs, cols);
+    wr = uniform_ptr(wr);  // the row is the same for the whole wave (two vector registers fewer)
+    const RouterX rx(x, cols);
+    float wv[32], xv[32];
+    router_span_load(wr, 0, RouterSpan(cols), upper, t, wv);  // (a wave without a row: from x; behind a branch x would be waited for with everything else)
+    rx.stage(x, xs, cols);
     __syncthreads();
     float s = 0.0f;  // the chain value; valid in the half that ran last
     if (on) {
         for (int i0 = 0; i0 < cols; i0 += 2048) {
             const RouterSpan sp(cols - i0);
             if (i0 > 0) router_span_load(wr, i0, sp, upper, t, wv);
+            if (!upper || sp.upper > 0) router_span_x(xs + i0 + t + (upper ? 1024 : 0), sp, upper, xv);
             // the lower half advances the chain (from the upper half's value of the previous span) ...
             const wd_uint2v back = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
-            if (!upper) s = router_span_run(wv, xs + i0 + t, sp.lower, i0 == 0 ? 0.0f : bits_f(back.y));
+            if (!upper) s = router_span_run(wv, xv, sp.lower, i0 == 0 ? 0.0f : bits_f(back.y));
             // ... and the upper half continues from its result
             const wd_uint2v fwd = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
-            if (upper) s = router_span_run(wv, xs + i0 + 1024 + t, sp.upper, bits_f(fwd.x));
+            if (upper) s = router_span_run(wv, xv, sp.upper, bits_f(fwd.x));
         }
     }
     // the 32 accumulators are final in the upper half (lanes 32..63): ggml's closing tree
@@ -1004,21 +1018,24 @@ WD_DEV float router_rows_wave_pair(const float *__restrict__ w, const float *__r
     const int total = rows + (extra_w ? 1 : 0);
     const bool on = row < total;
     const float *wr = on ? (row < rows ? w + static_cast<size_t>(row) * cols : extra_w) : x;
+    wr = uniform_ptr(wr);
     const int c0 = second ? 2048 : 0;
     const RouterSpan sp(cols - c0);
-    float wv[32];
-    if (on) router_span_load(wr, c0, sp, upper, t, wv);
-    router_stage_x(x, xs, cols);
+    const RouterX rx(x, cols);
+    float wv[32], xv[32];
+    router_span_load(wr, c0, sp, upper, t, wv);
+    rx.stage(x, xs, cols);
     __syncthreads();
+    if (!upper || sp.upper > 0) router_span_x(xs + c0 + t + (upper ? 1024 : 0), sp, upper, xv);
     // one copy of the chain code for both waves of a pair: turn 0 is the first wave's, turn 1 the second's
     float s = 0.0f;
 #pragma unroll 1
     for (int turn = 0; turn < 2; ++turn) {
         if (second == (turn == 1)) {
             const float start = s;
-            if (on && !upper) s = router_span_run(wv, xs + c0 + t, sp.lower, start);
+            if (on && !upper) s = router_span_run(wv, xv, sp.lower, start);
             const wd_uint2v fwd = __builtin_amdgcn_permlane32_swap(f_bits(s), f_bits(s), false, false);
-            if (upper) s = on ? router_span_run(wv, xs + c0 + 1024 + t, sp.upper, bits_f(fwd.x)) : bits_f(fwd.x);
+            if (upper) s = on ? router_span_run(wv, xv, sp.upper, bits_f(fwd.x)) : bits_f(fwd.x);
         }
         if (turn == 0) {
             if (!second && upper) over[(wave >> 1) * 32 + t] = s;
@@ -1104,7 +1121,7 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
             logit = router_rows_wave_pair(a.router, a.x, reinterpret_cast<float *>(lds_ab), reinterpret_cast<float *>(s_union), a.hand, a.hand_side, rows, H,
                                           a.sh_inp, a.E, blk, row);
         else
-            logit = router_rows_wave<>(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, a.hand_side, rows, H, a.sh_inp, a.E, blk, row);
+            logit = router_rows_wave(a.router, a.x, reinterpret_cast<float *>(lds_ab), a.hand, a.hand_side, rows, H, a.sh_inp, a.E, blk, row);
         mark<TRACE>(a, 0, 1);
         if (lane == 32 && row >= 0 && row < rows) a.logits[row] = logit;  // (the caller's view)
         // (no selection: the one wave with the shared gate's row)

@@ -141,7 +141,7 @@ WD_DEV void tokens_front(const TokenArgs &ta, uint8_t *lds_ta, uint8_t *s_work, 
         if (WIDE)
             logit = router_rows_wave_pair(a.router, s.x, reinterpret_cast<float *>(lds_ta), reinterpret_cast<float *>(s_work), s.hand, s.hand_side, rows, H, a.sh_inp, a.E, wg, row);
         else
-            logit = router_rows_wave<true>(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.hand, s.hand_side, rows, H, a.sh_inp, a.E, wg, row);
+            logit = router_rows_wave(a.router, s.x, reinterpret_cast<float *>(lds_ta), s.hand, s.hand_side, rows, H, a.sh_inp, a.E, wg, row);
         if (lane == 32 && row >= 0 && row < rows) s.logits[row] = logit;  // (the caller's view)
         // (no selection: the one wave with the shared gate's row)
         if (a.preselected && row == a.E && lane == 32) s.shared_gate[0] = sigmoid_ggml(bits_f(hand_word_bits(f_bits(logit))));
