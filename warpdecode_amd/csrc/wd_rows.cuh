@@ -61,29 +61,25 @@ __device__ const SignMask k_signmask = make_signmask();
 
 // LDS copies staged once per workgroup.
 struct IqTables {
+    static constexpr bool kTight = false;
     uint32_t grid3[512];
     uint64_t grid2[1024];
     uint2 sign[16];
-    WD_DEV uint32_t grid3_at(uint32_t idx) const { return grid3[idx]; }
     WD_DEV uint32_t grid3_bytes(uint32_t off) const { return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const uint8_t *>(grid3) + off); }  // off = 4 idx
-    WD_DEV uint64_t grid2_at(uint32_t idx) const { return grid2[idx]; }
-    WD_DEV uint2 sign_at(uint32_t nibble) const { return sign[nibble]; }
+    WD_DEV uint64_t grid2_bytes(uint32_t off) const { return *reinterpret_cast<const uint64_t *>(reinterpret_cast<const uint8_t *>(grid2) + off); }  // off = 8 idx
+    WD_DEV uint2 sign_bytes(uint32_t off) const { return *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint8_t *>(sign) + off); }         // off = 8 nibble
 };
 // The same tables for a kernel that knows their LDS byte address when it is compiled (BASE: the address of an IqTables
 // in the workgroup's LDS): a lookup's address is then the scaled index alone, the rest goes into the load's offset field.
 template <unsigned BASE>
 struct IqTablesAt {
+    static constexpr bool kTight = true;  // (the resident stack has no registers for all of a block's look-ups at once)
     typedef const __attribute__((address_space(3))) uint32_t *Lds32;
     typedef const __attribute__((address_space(3))) uint64_t *Lds64;
-    WD_DEV uint32_t grid3_at(uint32_t idx) const {
-        return *(Lds32)(uintptr_t)(BASE + static_cast<unsigned>(offsetof(IqTables, grid3)) + 4u * idx);
-    }
     WD_DEV uint32_t grid3_bytes(uint32_t off) const { return *(Lds32)(uintptr_t)(BASE + static_cast<unsigned>(offsetof(IqTables, grid3)) + off); }
-    WD_DEV uint64_t grid2_at(uint32_t idx) const {
-        return *(Lds64)(uintptr_t)(BASE + static_cast<unsigned>(offsetof(IqTables, grid2)) + 8u * idx);
-    }
-    WD_DEV uint2 sign_at(uint32_t nibble) const {
-        const uint64_t v = *(Lds64)(uintptr_t)(BASE + static_cast<unsigned>(offsetof(IqTables, sign)) + 8u * nibble);
+    WD_DEV uint64_t grid2_bytes(uint32_t off) const { return *(Lds64)(uintptr_t)(BASE + static_cast<unsigned>(offsetof(IqTables, grid2)) + off); }
+    WD_DEV uint2 sign_bytes(uint32_t off) const {
+        const uint64_t v = *(Lds64)(uintptr_t)(BASE + static_cast<unsigned>(offsetof(IqTables, sign)) + off);
         return make_uint2(static_cast<uint32_t>(v), static_cast<uint32_t>(v >> 32));
     }
 };
@@ -160,69 +156,130 @@ WD_DEV IqFields iq_load(const uint8_t *blk, int ib) {
     return f;
 }
 
-template <int TYPE, typename Tables>
-WD_DEV void iq_chunks(const IqFields &f, int ib, const Tables &t, const uint32_t (&a)[8], int (&p)[8]) {
+// Where a block's look-ups go in the tables, byte offsets.  An index is a byte with one or two more bits above it, and a dispatch that decodes is bound by
+// vector instructions: so the bits above are spread over bytes for all indices at once, one byte permute puts two indices
+// together, one in each half of a register, and an instruction that reads half a register makes it an offset; the nibbles of signs are brought
+// to where they are worth eight for four bytes at once, and one that reads a byte takes each.  29 instructions for the sixteen look-ups of an IQ3_S block, each
+// by itself took 48; 20 for the twelve of IQ2_S in place of 32.  (4096 / 1536 IQ3_S, eight of 128 experts: 39.4 us per layer, so
+// 38.0; four tokens of 2048 / 512 38.7, 38.2.)
+// (Those two through assembly: the compiler folds the shift of a half, or the mask of a byte, into a shift and a mask of the whole register, two instructions.  Nothing
+// but plain vector instructions produces the operand, and LDS instructions take the result, so that there are no wait states to be known.)
+// (The amount in a scalar register for IQ3_S, in a vector register for IQ2_S: the other way round dispatch AB gets a scratch frame.)
+#define WD_HALF_SHIFTED(AMOUNT, WORD) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" WORD : "=v"(r) : AMOUNT(SHIFT), "v"(x))
+template <int SHIFT, int HALF>
+WD_DEV uint32_t half_shifted(uint32_t x) {
+    uint32_t r;
+    if (SHIFT == 2 && HALF == 0) WD_HALF_SHIFTED("s", "WORD_0");
+    else if (SHIFT == 2) WD_HALF_SHIFTED("s", "WORD_1");
+    else if (HALF == 0) WD_HALF_SHIFTED("v", "WORD_0");
+    else WD_HALF_SHIFTED("v", "WORD_1");
+    return r;
+}
+#undef WD_HALF_SHIFTED
+template <int BYTE>
+WD_DEV uint32_t byte_masked(uint32_t mask, uint32_t x) {
+    uint32_t r;
+    if (BYTE == 0) asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(r) : "s"(mask), "v"(x));
+    else if (BYTE == 1) asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(r) : "s"(mask), "v"(x));
+    else if (BYTE == 2) asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "s"(mask), "v"(x));
+    else asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(r) : "s"(mask), "v"(x));
+    return r;
+}
+// chunk c's sign nibble (of four sign bytes: c >> 1, its half c & 1), for chunks 4 HALF .. 4 HALF + 3
+template <int HALF>
+WD_DEV void iq_sign_offsets(uint32_t sg, uint32_t (&off)[4]) {
+    const uint32_t lo = sg << 3, hi = sg >> 1;  // the low nibble of every byte, and the high one, where they are worth eight
+    off[0] = byte_masked<2 * HALF>(0x78u, lo), off[1] = byte_masked<2 * HALF>(0x78u, hi);
+    off[2] = byte_masked<2 * HALF + 1>(0x78u, lo), off[3] = byte_masked<2 * HALF + 1>(0x78u, hi);
+}
+// IQ3_S: eight indices, byte c with bit c of qh above it; for chunks 4 HALF .. 4 HALF + 3
+template <int HALF>
+WD_DEV void iq3_grid_offsets(uint2 qs, uint32_t qh, uint32_t (&off)[4]) {
+    // bit 2 j of the factor goes from 2 j to 8 j by the summand shifted by 6 j; where summands meet, at 6, 12 and 18, a sum does not reach the bits kept
+    const uint32_t even = __umul24(qh & 0x55u, 0x41041u) & 0x01010101u, odd = __umul24((qh >> 1) & 0x55u, 0x41041u) & 0x01010101u;
+    const uint32_t q = HALF ? qs.y : qs.x;
+    const uint32_t i02 = __builtin_amdgcn_perm(even, q, HALF ? 0x07020600u : 0x05020400u), i13 = __builtin_amdgcn_perm(odd, q, HALF ? 0x07030601u : 0x05030401u);
+    off[0] = half_shifted<2, 0>(i02), off[2] = half_shifted<2, 1>(i02), off[1] = half_shifted<2, 0>(i13), off[3] = half_shifted<2, 1>(i13);
+}
+// IQ2_S: four indices, byte g with bits 2 g and 2 g + 1 of qh above it; for g = 2 HALF, 2 HALF + 1
+template <int HALF>
+WD_DEV void iq2_grid_offsets(uint32_t qs, uint32_t qh, uint32_t (&off)[2]) {
+    qh &= 0xffu;  // (some callers' has other fields above)
+    const uint32_t wide = (qh | (qh << 12)) & 0x000f000fu, above = (wide | (wide << 6)) & 0x03030303u;
+    const uint32_t i = __builtin_amdgcn_perm(above, qs, HALF ? 0x07030602u : 0x05010400u);
+    off[0] = half_shifted<3, 0>(i), off[1] = half_shifted<3, 1>(i);
+}
+// Chunks 4 HALF .. 4 HALF + 3 of a block: magnitudes and sign masks looked up.
+template <int TYPE, int HALF, typename Tables>
+WD_DEV void iq_look_up(const IqFields &f, const Tables &t, uint32_t (&g)[4], uint2 (&sm)[4]) {
+    uint32_t so[4];
+    iq_sign_offsets<HALF>(TYPE == 21 ? f.sg : f.qs.y, so);
     if (TYPE == 21) {
-        const int ls = 1 + 2 * static_cast<int>((f.sc >> (4 * (ib & 1))) & 15u);
-        // all sixteen lookups first, the arithmetic after: a lane's block then waits for the LDS once, not eight times
-        uint32_t g[8];
-        uint2 sm[8];
+        uint32_t go[4];
+        iq3_grid_offsets<HALF>(f.qs, f.qh, go);
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            // (the entry's byte offset, 4 (q | high bit << 8), put together from parts that are one instruction each)
-            const uint32_t q4 = (((c < 4 ? f.qs.x : f.qs.y) >> (8 * (c & 3))) & 0xffu) << 2;
-            const uint32_t off = q4 | ((f.qh << (10 - c)) & 0x400u);
-            const uint32_t sbits = (f.sg >> (4 * c)) & 15u;  // sign byte c>>1, nibble c&1
-            g[c] = t.grid3_bytes(off);
-            sm[c] = t.sign_at(sbits);
+        for (int c = 0; c < 4; ++c) g[c] = t.grid3_bytes(go[c]), sm[c] = t.sign_bytes(so[c]);
+    } else {
+        uint32_t go[2];
+        iq2_grid_offsets<HALF>(f.qs.x, f.qh, go);
+        if (Tables::kTight) {  // (the constants of the assembly took 36 registers too many)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int q = 2 * HALF + i;
+                const uint32_t s8 = (f.qs.y >> (8 * q)) & 0xffu;
+                go[i] = (((f.qs.x >> (8 * q)) & 0xffu) | ((f.qh << (8 - 2 * q)) & 0x300u)) << 3;
+                so[2 * i] = (s8 & 15u) << 3, so[2 * i + 1] = (s8 >> 4) << 3;
+            }
         }
 #pragma unroll
-        for (int c = 0; c < 8; ++c) p[c] = __mul24(ls, sdot4(apply_signs(g[c], sm[c]), a[c], 0));
-    } else {
-        const int ls_lo = 1 + 2 * static_cast<int>(f.sc & 15u);
-        const int ls_hi = 1 + 2 * static_cast<int>(f.sc >> 4);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t idx = ((f.qs.x >> (8 * g)) & 0xffu) | ((f.qh << (8 - 2 * g)) & 0x300u);
-            const uint64_t mags = t.grid2_at(idx);
-            const uint32_t s8 = (f.qs.y >> (8 * g)) & 0xffu;
-            const int ls = (g < 2) ? ls_lo : ls_hi;  // chunks 0..3 low nibble, 4..7 high nibble
-            p[2 * g] = __mul24(ls, sdot4(apply_signs(static_cast<uint32_t>(mags), t.sign_at(s8 & 15u)), a[2 * g], 0));
-            p[2 * g + 1] = __mul24(ls, sdot4(apply_signs(static_cast<uint32_t>(mags >> 32), t.sign_at(s8 >> 4)), a[2 * g + 1], 0));
+        for (int i = 0; i < 2; ++i) {
+            const uint64_t mags = t.grid2_bytes(go[i]);
+            g[2 * i] = static_cast<uint32_t>(mags), g[2 * i + 1] = static_cast<uint32_t>(mags >> 32);
+            sm[2 * i] = t.sign_bytes(so[2 * i]), sm[2 * i + 1] = t.sign_bytes(so[2 * i + 1]);
         }
     }
+}
+// The 32 signed weights of a block as eight packed dwords.  All look-ups first, the arithmetic after: a lane's block then waits for the
+// LDS once; with tight registers, half by half.
+template <int TYPE, typename Tables>
+WD_DEV void iq_weights(const IqFields &f, const Tables &t, uint32_t (&w)[8]) {
+    uint32_t g0[4], g1[4];
+    uint2 s0[4], s1[4];
+    iq_look_up<TYPE, 0>(f, t, g0, s0);
+    if (Tables::kTight) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w[c] = apply_signs(g0[c], s0[c]);
+    }
+    iq_look_up<TYPE, 1>(f, t, g1, s1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (!Tables::kTight) w[c] = apply_signs(g0[c], s0[c]);
+        w[4 + c] = apply_signs(g1[c], s1[c]);
+    }
+}
+// The odd sub-scales of chunks 0..3 and 4..7.
+template <int TYPE>
+WD_DEV void iq_sub_scales(const IqFields &f, int ib, int (&ls)[2]) {
+    if (TYPE == 21) ls[0] = ls[1] = 1 + 2 * static_cast<int>((f.sc >> (4 * (ib & 1))) & 15u);
+    else ls[0] = 1 + 2 * static_cast<int>(f.sc & 15u), ls[1] = 1 + 2 * static_cast<int>(f.sc >> 4);
+}
+
+template <int TYPE, typename Tables>
+WD_DEV void iq_chunks(const IqFields &f, int ib, const Tables &t, const uint32_t (&a)[8], int (&p)[8]) {
+    int ls[2];
+    uint32_t w[8];
+    iq_sub_scales<TYPE>(f, ib, ls);
+    iq_weights<TYPE>(f, t, w);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) p[c] = __mul24(ls[c >> 2], sdot4(w[c], a[c], 0));
 }
 
 // The same in two steps, for callers that apply one decoded sub-block to several activations: the 32 signed
 // weights (eight packed dwords) and the odd sub-scale of every chunk first, the chunk sums per activation after.
 template <int TYPE, typename Tables>
 WD_DEV void iq_decode(const IqFields &f, int ib, const Tables &t, uint32_t (&w)[8], int (&ls)[2]) {
-    if (TYPE == 21) {
-        ls[0] = ls[1] = 1 + 2 * static_cast<int>((f.sc >> (4 * (ib & 1))) & 15u);
-        uint32_t g[8];
-        uint2 sm[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const uint32_t q4 = (((c < 4 ? f.qs.x : f.qs.y) >> (8 * (c & 3))) & 0xffu) << 2;
-            const uint32_t off = q4 | ((f.qh << (10 - c)) & 0x400u);
-            const uint32_t sbits = (f.sg >> (4 * c)) & 15u;
-            g[c] = t.grid3_bytes(off);
-            sm[c] = t.sign_at(sbits);
-        }
-#pragma unroll
-        for (int c = 0; c < 8; ++c) w[c] = apply_signs(g[c], sm[c]);
-    } else {
-        ls[0] = 1 + 2 * static_cast<int>(f.sc & 15u);  // chunks 0..3
-        ls[1] = 1 + 2 * static_cast<int>(f.sc >> 4);   // chunks 4..7
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t idx = ((f.qs.x >> (8 * g)) & 0xffu) | ((f.qh << (8 - 2 * g)) & 0x300u);
-            const uint64_t mags = t.grid2_at(idx);
-            const uint32_t s8 = (f.qs.y >> (8 * g)) & 0xffu;
-            w[2 * g] = apply_signs(static_cast<uint32_t>(mags), t.sign_at(s8 & 15u));
-            w[2 * g + 1] = apply_signs(static_cast<uint32_t>(mags >> 32), t.sign_at(s8 >> 4));
-        }
-    }
+    iq_sub_scales<TYPE>(f, ib, ls);
+    iq_weights<TYPE>(f, t, w);
 }
 WD_DEV void iq_dot_decoded(const uint32_t (&w)[8], const int (&ls)[2], const uint32_t (&a)[8], int (&p)[8]) {
     // (The sub-scales pass through a statement the compiler cannot look into.  It knows that they are small, drops
