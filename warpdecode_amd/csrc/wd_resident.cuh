@@ -297,7 +297,7 @@ WD_DEV void fill_wait(const ResidentArgs &a, int l, uint32_t need, bool &dead) {
 WD_DEV void res_router_fetch(const float *__restrict__ row, float (&wv)[32], int lane) {
     const float *p = uniform_ptr(row) + ((lane >= 32) ? 1024 : 0) + (lane & 31);
 #pragma unroll
-    for (int u = 0; u < 32; ++u) wv[u] = p[32 * u];
+    for (int u = 0; u < 32; ++u) wv[u] = gld_f32(p + 32 * u);  // (as generic loads they were counted with the LDS's, and every barrier waited for them)
 }
 // The row's dot product with the input (LDS, transposed: xt[t][v] = x[32 v + t], rows of kResXtRow floats); valid in lane 32.
 WD_DEV float res_router_dot(const float (&wv)[32], const float *xt, int lane) {
@@ -419,14 +419,8 @@ WD_DEV void res_mark(const ResidentArgs &a, const ResCtx &c, int l, int i) {
         a.trace[(c.r * 4 + (c.wave == 0 ? 0 : c.wave - 8)) * 16 + i] = wall_clock64();
     }
 }
-// A pointer field of a layer descriptor, read again (the descriptors lie in global memory) and made wave-uniform.
-template <typename T>
-WD_DEV T *res_field(T *const *field) {
-    return uniform_ptr(*const_cast<T *const volatile *>(field));
-}
-
-// The same through the scalar path (the descriptors are written before the launch): the value is wave-uniform, costs no
-// vector register and no vector-memory wait, and is there long before the request that needs it.
+// A pointer field of a layer descriptor, read again through the scalar path (the descriptors are written before the launch): the value is wave-uniform,
+// costs no vector register and no vector-memory wait, and is there long before the request that needs it.
 template <typename T>
 WD_DEV T *res_field_s(T *const *field) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(field);
@@ -794,9 +788,9 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
     Q8Block gb[2];
     Q8CoalRaw<0, 16> draw;
     auto fetch = [&](const ResidentLayer *L, int r, int lane) {
-        gb[0] = q8_load<0>(res_field(&L->sh_gate) + static_cast<size_t>(r) * (64 * 34) + lane * 34);
-        gb[1] = q8_load<0>(res_field(&L->sh_up) + static_cast<size_t>(r) * (64 * 34) + lane * 34);
-        draw = q8_rows4_coal_request<0, 16>(res_field(&L->sh_down) + static_cast<size_t>(r) * (4 * 16 * 34), lane);
+        gb[0] = q8_load<0>(res_field_s(&L->sh_gate) + static_cast<size_t>(r) * (64 * 34) + lane * 34);
+        gb[1] = q8_load<0>(res_field_s(&L->sh_up) + static_cast<size_t>(r) * (64 * 34) + lane * 34);
+        draw = q8_rows4_coal_request<0, 16>(res_field_s(&L->sh_down) + static_cast<size_t>(r) * (4 * 16 * 34), lane);
     };
     const bool traced = a.ids_trace != nullptr;
     if (a.shared) fetch(a.layers, r0, lane0);
@@ -885,7 +879,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
     // (a workgroup without a row keeps row 0 company: one definition of the row's registers per layer, no merge of an
     // old and a new value - the compiler then holds them as 32 registers, not as one value of 32 that it copies whole)
     float wv[32];
-    res_router_fetch(res_field(&a.layers->router) + static_cast<size_t>(has_row ? r0 : 0) * kResH, wv, lane0);
+    res_router_fetch(res_field_s(&a.layers->router) + static_cast<size_t>(has_row ? r0 : 0) * kResH, wv, lane0);
     for (int l = 0; l < a.n_layers; ++l) {
         const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, -1, hand);
         const int r = c.r, lane = c.lane;
@@ -898,7 +892,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         // (both asked for ahead of the logits)
         int id_given = 0;
         if (traced && r == 0 && lane < a.k) id_given = a.ids_trace[l * a.k + lane];  // (the expert's name, whatever addresses its rows)
-        const float w_scale = *const_cast<const volatile float *>(&L->w_scale);
+        const float w_scale = bits_f(static_cast<uint32_t>(sld_i32(reinterpret_cast<const int32_t *>(&L->w_scale))));
         __syncthreads();  // B1
         res_mark<STAMPS>(a, c, l, 2);
         {
@@ -910,7 +904,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         // (before the selection's values exist: this dot and they together would not fit the registers)
         if (a.shared && r == 1) {  // the shared expert's gate logit: one more row of the router's kind (the fold needs it)
             float gw[32];  // (an array of its own: the router row's registers keep one definition per layer)
-            res_router_fetch(res_field(&L->sh_inp), gw, lane);
+            res_router_fetch(res_field_s(&L->sh_inp), gw, lane);
             const float s = res_router_dot(gw, c.xt(), lane);
             const uint32_t word = hand_word(readlane_f(s, 32));
             if (lane < 2) hand_store4(c.hb, rec_piece(l, lane, 1) + 4u, word);
@@ -1020,7 +1014,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         if (r == 0 && traced) weights_from_lds();
         // the next layer's row: requested behind the selection, so that its registers are not held while the selection runs,
         // and behind the exchange, whose polls it would delay
-        res_router_fetch(res_field(&a.layers[last ? l : l + 1].router) + static_cast<size_t>(has_row ? r : 0) * kResH, wv, lane);
+        res_router_fetch(res_field_s(&a.layers[last ? l : l + 1].router) + static_cast<size_t>(has_row ? r : 0) * kResH, wv, lane);
         __syncthreads();  // B5
     }
 }
