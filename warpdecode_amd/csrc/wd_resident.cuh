@@ -512,7 +512,7 @@ WD_DEV void res_down(const ResidentArgs &a, const ResCtx &c, int l, Q8CoalRaw<0,
 
 // ---- the ten routed waves -------------------------------------------------------------------------------------
 // Rungs 0..7 (always waves 0..7) also fetch and quantise the layer's input.
-// Barriers of a layer, the same for every wave of the workgroup: B1 (input in LDS), B2..B4 (exchange of the
+// Barriers of a layer, the same for every wave of the workgroup: without a routing trace B1x (input in LDS), B1 (with its quantised forms), B2..B4 (exchange of the
 // activations), B5 (down results in LDS).
 // TRACED: the launch has a routing trace (the two forms of the role differ in when they can ask for what: one body for
 // both, chosen at run time, costs the compiler's merging of registers that either form defines in its own place).
@@ -603,9 +603,9 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         if (traced && on) e = traced_expert(l, rung), e_next = traced_expert(l + 1, rung);
         const uint32_t need_next = traced && on ? fill_needed(l + 1) : 0u;
         // ---- the layer's input: 16 bytes per lane of waves 0..7, quantised from the registers they arrive in
+        float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
         if (wave < 8) {
             const int i = wave * 64 + lane;
-            float4 xv;
             if (l == 0) {
                 xv = reinterpret_cast<const float4 *>(a.x)[i];
             } else {
@@ -622,6 +622,12 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
                 float *dst = c.xt() + (4 * (i & 7)) * kResXtRow + (i >> 3);
                 dst[0] = xv.x, dst[kResXtRow] = xv.y, dst[2 * kResXtRow] = xv.z, dst[3 * kResXtRow] = xv.w;
             }
+        }
+        // (Without a routing trace everybody waits for the router's logits, which need the input itself only: its quantised forms are made on the
+        // far side of a barrier of its own.  48 layers, made ahead of the one barrier / so: IQ3_S 713 / 671 us, Q8_0 728 / 711.)
+        if constexpr (!traced) __syncthreads();  // B1x: x is in LDS
+        if (wave < 8) {
+            const int i = wave * 64 + lane;
             if constexpr (!kQ8) wave_quantize_q8_k_regs(xv, c.xq() + 256 * wave, c.xd() + wave, lane);
             if (shared || kQ8) {  // Q8_0: a block is eight lanes
                 float amax = __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(xv.x), __builtin_fabsf(xv.y)),
@@ -798,6 +804,7 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         const ResCtx c = res_ctx(lds_base, r0, lane0, wave0, kResSharedSlot, hand);
         const int r = c.r, lane = c.lane;
         const bool with_shared = fresh_s(a.shared) != 0;  // (a scalar of this layer, not a vector register kept for the launch)
+        if (!traced) __syncthreads();  // B1x
         __syncthreads();  // B1
         float act = 0.0f;
         if (with_shared) {
@@ -893,7 +900,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         int id_given = 0;
         if (traced && r == 0 && lane < a.k) id_given = a.ids_trace[l * a.k + lane];  // (the expert's name, whatever addresses its rows)
         const float w_scale = bits_f(static_cast<uint32_t>(sld_i32(reinterpret_cast<const int32_t *>(&L->w_scale))));
-        __syncthreads();  // B1
+        __syncthreads();  // B1, or without a routing trace B1x: x is in LDS
         res_mark<STAMPS>(a, c, l, 2);
         {
             const float s = res_router_dot(wv, c.xt(), lane);
@@ -901,6 +908,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             if (has_row && lane < 2) hand_store4(c.hb, rec_piece(l, lane, r), word);
             res_mark<STAMPS>(a, c, l, 3);
         }
+        if (!traced) __syncthreads();  // B1
         // (before the selection's values exist: this dot and they together would not fit the registers)
         if (a.shared && r == 1) {  // the shared expert's gate logit: one more row of the router's kind (the fold needs it)
             float gw[32];  // (an array of its own: the router row's registers keep one definition per layer)
