@@ -588,3 +588,32 @@ def test_time_stamps_of_the_selection(g, E, k):
             assert before < begin <= seen <= end and before < mine, (wg, turn)
             assert abs(begin - mine) < 100 * 1000, (wg, turn)    # (100 MHz: a millisecond)
     sc.close()
+
+
+@pytest.mark.parametrize("H,F,gate_t,down_t,shared", [(2048, 512, synth.IQ3_S, synth.Q8_0, True), (1024, 256, synth.Q8_0, synth.Q8_0, True),
+                                                      (2560, 640, synth.IQ2_S, synth.IQ4_NL, True), (2048, 672, synth.Q8_0, synth.IQ4_NL, False)])
+def test_activation_blocks_of_any_magnitude(g, oracle, H, F, gate_t, down_t, shared):
+    """The activations' quantisers have a form for ordinary blocks: blocks of zeros, below and above its range and next to ordinary ones, through
+    dispatch C and through the one-launch stack where it takes the shape."""
+    E, k = 16, 4
+    L = synth.make_layer(H, F, E, k, gate_t, down_t, shared, seed=SEED, layer=H + F, router_sigma=1.0 / np.sqrt(H))
+    L["gate"] = L["gate"].copy()
+    L["gate"].reshape(E, F, -1)[:, 32:64] = 0        # one block of zeros in every expert's activation
+    if shared:
+        L["shared_gate"] = np.ascontiguousarray(L["shared_gate"]).copy()
+        L["shared_gate"].reshape(F, -1)[F - 32:] = 0
+    x = synth.rms_normed(synth.rng_for(SEED, 91, H), H)
+    for gain in (1e-17, 1e-13, 1e-3, 1.0, 1e15, 1e17):   # activations from 1e-35 (127 over a smaller block's largest is infinite) to 1e34
+        xg = (x * np.float32(gain)).astype(np.float32)
+        want, d = oracle.moe_layer(L, xg)
+        got = run_layer(g, L, xg, partials=False, flags=0)
+        assert g.same_bits(got["act"], d["act"]) and g.same_bits(got["accum"], d["routed"]) and g.same_bits(got["out"], want), gain
+        dl, outs = g.DeviceLayer(L), []
+        for flags in (0, capi.MOE_PER_LAYER):
+            sc, stack = g.Scratch(H, F, E, k), (capi.MoeLayer * 2)(dl.desc, dl.desc)
+            dx, out = g.dev(xg), g.empty(H, np.float32)
+            capi.call("wd_moe_stack_f32", stack, 2, g.ptr(dx), g.ptr(out), sc.h, None, 1e-6, flags, g.stream())
+            g.sync()
+            outs.append((g.host(dx), g.host(out)))
+            sc.close()
+        assert g.same_bits(outs[0][0], outs[1][0]) and g.same_bits(outs[0][1], outs[1][1]), gain

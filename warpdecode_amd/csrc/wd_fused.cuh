@@ -91,23 +91,44 @@ WD_DEV void mark(const LayerArgs &a, int d, int i) {
 
 // ---- in-workgroup quantisers (results in LDS) ------------------------------------------------
 // Q8_0 of n values (multiple of 32): four threads per block, eight values per thread.
-// The step on eight loaded values (v0, v1 = x[base .. base + 8)); all four threads of a block must call it.
-WD_DEV void lds_quantize_q8_0_step(const float4 &v0, const float4 &v1, bool on, int base, int8_t *qs, uint16_t *d, int tid) {
+// The general form of the step on eight loaded values (v0, v1 = x[base .. base + 8)); all four threads of a block must call it.  The quants, and the scale's bits.
+WD_DEV uint2 quantize_q8_0_general(const float4 &v0, const float4 &v1, uint16_t &scale) {
     float amax = __builtin_fmaxf(
         __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v0.x), __builtin_fabsf(v0.y)),
                         __builtin_fmaxf(__builtin_fabsf(v0.z), __builtin_fabsf(v0.w))),
         __builtin_fmaxf(__builtin_fmaxf(__builtin_fabsf(v1.x), __builtin_fabsf(v1.y)),
                         __builtin_fmaxf(__builtin_fabsf(v1.z), __builtin_fabsf(v1.w))));
     amax = quad_max_nonneg(amax);
+    uint2 packed = make_uint2(0u, 0u);
+    if (amax != 0.0f) {  // (one division for the eight values)
+        const float inv = 127.0f / amax;
+        packed.x = q8_0_pack4_scaled(v0, inv);
+        packed.y = q8_0_pack4_scaled(v1, inv);
+    }
+    scale = f2h_ref(amax / 127.0f);
+    return packed;
+}
+// The step, for what comes between a dispatch's activations and its dot products (on: the thread's values are of a block; the whole wave must call it).
+// ORDINARY false: the general form only, which takes fewer registers.
+template <bool ORDINARY = true>
+WD_DEV void lds_quantize_q8_0_step(const float4 &v0, const float4 &v1, bool on, int base, int8_t *qs, uint16_t *d, int tid) {
+    uint2 packed;
+    uint16_t scale;
+    if constexpr (ORDINARY) {
+        uint32_t m = umax_step<kDppXor1>(f_bits(max3_abs(max3_abs(max3_abs(v0.x, v0.y, v0.z), v0.w, v1.x), max3_abs(v1.y, v1.z, v1.w), 0.0f)));
+        m = umax_step<kDppXor2>(m);
+        const float most = bits_f(m), inverse = quot_ordinary(127.0f, most);
+        uint32_t worst = 0u;
+        packed.x = quants_ordinary(v0, inverse, worst);
+        packed.y = quants_ordinary(v1, inverse, worst);
+        scale = f2h_number(over_127(most));
+        if (__builtin_expect(quants_not_ordinary(worst, m, on), 0)) packed = quantize_q8_0_general(v0, v1, scale);
+    } else {
+        packed = quantize_q8_0_general(v0, v1, scale);
+    }
     if (on) {
-        uint2 packed = make_uint2(0u, 0u);
-        if (amax != 0.0f) {  // (one division for the eight values)
-            const float inv = 127.0f / amax;
-            packed.x = q8_0_pack4_scaled(v0, inv);
-            packed.y = q8_0_pack4_scaled(v1, inv);
-        }
         *reinterpret_cast<uint2 *>(qs + base) = packed;
-        if ((tid & 3) == 0) d[base >> 5] = f2h_ref(amax / 127.0f);
+        if ((tid & 3) == 0) d[base >> 5] = scale;
     }
 }
 WD_DEV void lds_quantize_q8_0(const float *__restrict__ x, int n, int8_t *qs, uint16_t *d, int tid, int nthreads) {
@@ -120,7 +141,7 @@ WD_DEV void lds_quantize_q8_0(const float *__restrict__ x, int n, int8_t *qs, ui
             v0 = *reinterpret_cast<const float4 *>(x + base);
             v1 = *reinterpret_cast<const float4 *>(x + base + 4);
         }
-        lds_quantize_q8_0_step(v0, v1, on, base, qs, d, tid);
+        lds_quantize_q8_0_step<false>(v0, v1, on, base, qs, d, tid);  // (beside other things that nobody waits for)
     }
 }
 
@@ -975,7 +996,7 @@ WD_DEV float router_rows_wave(const float *__restrict__ w, const float *__restri
                               int cols, const float *__restrict__ extra_w, int extra_slot, int wg, int &done) {
     const int lane = threadIdx.x & 63, t = lane & 31;
     const bool upper = lane >= 32;
-    const int row = wg * static_cast<int>(blockDim.x >> 6) + static_cast<int>(threadIdx.x >> 6);
+    const int row = wg * static_cast<int>(blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int total = rows + (extra_w ? 1 : 0);
     const bool on = row < total;
     const float *wr = on ? (row < rows ? w + static_cast<size_t>(row) * cols : extra_w) : x;

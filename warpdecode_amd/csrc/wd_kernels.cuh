@@ -139,6 +139,52 @@ WD_DEV uint32_t q8_0_pack4(float4 v, float amax) {
     return (q0 & 0xff) | ((q1 & 0xff) << 8) | ((q2 & 0xff) << 16) | (static_cast<uint32_t>(q3 & 0xff) << 24);
 }
 
+// ---- the quantisers' arithmetic on ordinary blocks ----------------------------------------------------------------
+// In dispatch C the quantisation of 512 values by a wave was 100 vector instructions, of 164 with the down rows behind it.  On blocks whose largest
+// magnitude is between 2^-100 and 2^100 and which hold no NaN it takes 55, with the same bits:
+//   * a quotient by one step of Newton's iteration on the reciprocal and one correction of the quotient: what remains of an IEEE division without the scaling
+//     and the special cases (equal to it for every float of the range, 1,677,721,600 of them, for 127 / a and for a / 127);
+//   * a value times the inverse scale rounded to an integer by adding 1.5 * 2^23: the sum's low byte is the quant, and anything that is not a number
+//     of the range shows in the upper bits, of eight values at once.
+// A wave with any other block takes the general form for all of its blocks.  (us per layer: 2560 / 640, IQ4_NL down 21.7, so 21.4; 4096 / 1536 37.6, 37.2.  The
+// resident stack, 48 layers: the same within noise; the token batches' dispatch has no registers for it.)
+constexpr float kQuantAdd = 0x1.8p23f;
+constexpr uint32_t kQuantTop = 0x4b400000u + 127u;   // bits of the sum for 127; smaller ones down to -128 are below
+constexpr uint32_t kQuantLo = (127u - 100u) << 23, kQuantSpan = 200u << 23;  // bits of 2^-100, up to 2^100
+WD_DEV float quot_ordinary(float n, float a) {
+    float y = __builtin_amdgcn_rcpf(a);
+    y = __builtin_fmaf(__builtin_fmaf(-a, y, 1.0f), y, y);
+    const float q = n * y;
+    return __builtin_fmaf(__builtin_fmaf(-a, q, n), y, q);
+}
+WD_DEV float over_127(float a) {
+    constexpr float c = 1.0f / 127.0f;
+    const float q = a * c;
+    return __builtin_fmaf(__builtin_fmaf(-127.0f, q, a), c, q);
+}
+// max(|a|, |b|, |c|).  (fmaxf of values from memory takes an instruction more per value, which quiets signalling NaN; here a NaN shows in the quants.)
+WD_DEV float max3_abs(float a, float b, float c) {
+    float m;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+}
+WD_DEV uint32_t quants_ordinary(const float4 &v, float inv, uint32_t &worst) {
+    const uint32_t t0 = f_bits(v.x * inv + kQuantAdd), t1 = f_bits(v.y * inv + kQuantAdd), t2 = f_bits(v.z * inv + kQuantAdd), t3 = f_bits(v.w * inv + kQuantAdd);
+    worst = max(max(worst, t0), t1), worst = max(max(worst, t2), t3);
+    const uint32_t lo = __builtin_amdgcn_perm(t1, t0, 0x0c0c0400u), hi = __builtin_amdgcn_perm(t3, t2, 0x0c0c0400u);
+    return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+// any lane's (the same in every lane)
+WD_DEV bool quants_not_ordinary(uint32_t worst, uint32_t amax_bits, bool on = true) {
+    return __builtin_amdgcn_ballot_w64(on && (worst > kQuantTop || amax_bits - kQuantLo > kQuantSpan)) != 0ull;
+}
+// f2h_ref of a number that is not NaN
+WD_DEV uint16_t f2h_number(float v) {
+    const uint16_t h = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
+    return __builtin_fabsf(v) < 0x1p-24f ? static_cast<uint16_t>(h & 0x8000u) : h;
+}
+
+
 __global__ __launch_bounds__(256) void k_q8_0_quantize(const float *__restrict__ x, int blocks,
                                                         int8_t *__restrict__ qs, uint16_t *__restrict__ scales) {
     const int sub = threadIdx.x & 7;

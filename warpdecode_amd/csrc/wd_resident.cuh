@@ -503,7 +503,7 @@ WD_DEV void res_down(const ResidentArgs &a, const ResCtx &c, int l, Q8CoalRaw<0,
     wave_lds_fence();
     q8_rows4_coal_stage<0, 16>(draw, stage, lane);
     staged();
-    lds_quantize_q8_0_step(v0, v1, true, lane * 8, aq, ad, lane);
+    lds_quantize_q8_0_step<false>(v0, v1, true, lane * 8, aq, ad, lane);
     wave_lds_fence();
     const float y = q8_rows4_coal_dots<0, 16>(stage, aq, ad, tile, lane);
     if ((lane & 15) == 0) c.ybuf()[c.slot * 4 + (lane >> 4)] = y;

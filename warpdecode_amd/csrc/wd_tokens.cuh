@@ -671,7 +671,7 @@ void k_tokens_c(TokenArgs ta) {
             wave_lds_fence();
 #pragma unroll
             for (int q = 0; q < kActs; ++q)
-                lds_quantize_q8_0_step(v[2 * q], v[2 * q + 1], 512 * q + lane * 8 < a.F, 512 * q + lane * 8, aq, ad, lane);
+                lds_quantize_q8_0_step<false>(v[2 * q], v[2 * q + 1], 512 * q + lane * 8 < a.F, 512 * q + lane * 8, aq, ad, lane);
             wave_lds_fence();
             if (kActFirst) blocks.request(rows, nb, lane);
             Q8Chain ch;
@@ -778,7 +778,7 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
             wave_lds_fence();
 #pragma unroll
             for (int q = 0; q < kActs; ++q)
-                lds_quantize_q8_0_step(v[2 * q], v[2 * q + 1], 512 * q + lane * 8 < a.F, 512 * q + lane * 8, aq, ad, lane);
+                lds_quantize_q8_0_step<false>(v[2 * q], v[2 * q + 1], 512 * q + lane * 8 < a.F, 512 * q + lane * 8, aq, ad, lane);
             wave_lds_fence();
             Q8Chain ch;
 #pragma unroll
