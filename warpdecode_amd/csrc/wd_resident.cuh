@@ -346,7 +346,7 @@ constexpr int kResLdsRoles = kResLdsSel + kTopkLdsBytes1 + 128;       // int [12
 constexpr int kResLdsActv = kResLdsRoles + 64;                        // f32 [12] this workgroup's activations (word 11 zero), u32 [1] arrivals
 constexpr int kResLdsKept = kResLdsActv + 64;                         // per routed rung: 2048 bytes, the next layer's up row decoded ahead
 constexpr int kResLdsBytes = kResLdsKept + kResMaxK * 2048;
-constexpr int kResLdsLand = kResLdsWave;  // f32 [11][512] all activations of the layer, while no slot area is in use
+constexpr int kResLdsLand = kResLdsWave;  // (with a routing trace) f32 [11][512] all activations of the layer, while no slot area is in use
 static_assert(kResLdsXq % 16 == 0 && kResLdsTables % 16 == 0 && kResLdsWave % 16 == 0 && kResWaveBytes % 16 == 0 && kResLdsSel % 16 == 0, "LDS alignment");
 static_assert(sizeof(Q8RowTile) <= sizeof(Q8TileNB<16>) && 2 * kIqStageBytes <= kResTileBytes, "a slot's area serves every stage");
 static_assert(kResLdsBytes <= 81920, "LDS of the resident stack kernel: two workgroups per compute unit");
@@ -385,7 +385,12 @@ struct ResCtx {
     WD_DEV float *actv() const { return reinterpret_cast<float *>(lds + kResLdsActv); }
     // how many waves have handed in their activation of a layer, summed over the layers so far (every wave but the router's: 11 per layer)
     WD_DEV unsigned *arrived() const { return reinterpret_cast<unsigned *>(lds + kResLdsActv + 48); }
-    WD_DEV float *land() const { return reinterpret_cast<float *>(lds + kResLdsLand); }
+    // Where the layer's activations land, slot by slot.  With a routing trace in the slots' areas; without one where nothing else lies then, so that a wave's down
+    // rows can be in its area before they come: the rungs' in the places of the rows decoded ahead, the shared expert's in that of the codebook that the launch has not staged.
+    // (In the areas in either mode, the rows staged behind a barrier more: 48 layers, IQ3_S 652 / so 633 us, Q8_0 710 / 701.)
+    WD_DEV float *land(bool apart, int s, int spare) const {
+        return reinterpret_cast<float *>(lds + (apart ? (s < kResMaxK ? kResLdsKept + 2048 * s : spare) : kResLdsLand + 2048 * s));
+    }
     WD_DEV uint8_t *kept() const { return lds + kResLdsKept + slot * 2048; }  // (routed rungs only)
 };
 // The context of one layer: the indices made opaque (see fresh_v); `base` is the workgroup's dynamic LDS.
@@ -429,6 +434,10 @@ WD_DEV T *res_field_s(T *const *field) {
     return reinterpret_cast<T *>(static_cast<uintptr_t>(v));
 }
 
+// (a 2 KB codebook or the first 2 KB of the other: whichever TYPE does not stage)
+template <int TYPE>
+constexpr int res_spare() { return kResLdsTables + static_cast<int>(TYPE == 22 ? offsetof(IqTables, grid3) : offsetof(IqTables, grid2)); }
+
 // Between the gate/up rows and the down rows of a layer (every wave of the workgroup calls it, the router wave through its
 // own three barriers; `mine`: this wave's activation, for routed rungs in use and the shared expert).  The workgroup's
 // eleven activations go out as one store of its record; waves 0..7 then wait for the records of all 512 workgroups and
@@ -437,7 +446,7 @@ WD_DEV T *res_field_s(T *const *field) {
 // record is on its way (no record can be complete before the slowest workgroup's has crossed the device); meanwhile():
 // work for a wave that does not gather (waves 8..11) while the others wait for the records.
 template <bool STAMPS, typename Before, typename Early, typename Meanwhile>
-WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool has, float mine, float4 &v0, float4 &v1, bool &dead, Before &&before,
+WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool apart, int spare, bool has, float mine, float4 &v0, float4 &v1, bool &dead, Before &&before,
                          Early &&early, Meanwhile &&meanwhile) {
     const int lane = c.lane, wave = c.wave;
     if (lane == 0) {
@@ -445,7 +454,7 @@ WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool has
         __hip_atomic_fetch_add(c.arrived(), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     before();
-    __syncthreads();  // B2: the workgroup's activations are in LDS, and no slot area is in use any more
+    __syncthreads();  // B2: the workgroup's activations are in LDS (and, with a routing trace, no slot area is in use any more)
     if (wave == 0 && lane < 3 * kResCopies) {  // piece lane % 3 of the workgroup's 48 bytes, to copy lane / 3
         const int piece = lane % 3, copy = lane / 3;
         const float4 p = reinterpret_cast<const float4 *>(c.actv())[piece];
@@ -472,8 +481,9 @@ WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool has
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             const int w = i + 512 * t, wg = w / 3, piece = w - 3 * wg;
-            float *land = c.land() + (4 * piece) * 512 + wg;
-            land[0] = bits_f(v[t].x), land[512] = bits_f(v[t].y), land[1024] = bits_f(v[t].z);
+            float *land = c.land(apart, 0, spare) + (4 * piece) * 512 + wg;
+            land[0] = bits_f(v[t].x), land[512] = bits_f(v[t].y);
+            (piece < 2 ? land + 1024 : c.land(apart, kResSharedSlot, spare) + wg)[0] = bits_f(v[t].z);
             if (piece < 2) land[1536] = bits_f(v[t].w);
         }
     } else {
@@ -482,10 +492,31 @@ WD_DEV void res_exchange(const ResidentArgs &a, const ResCtx &c, int l, bool has
     __syncthreads();  // B3: every activation of the layer is in LDS
     res_mark<STAMPS>(a, c, l, 6);
     if (has) {
-        const float4 *row = reinterpret_cast<const float4 *>(c.land() + c.slot * 512 + 8 * lane);
+        const float4 *row = reinterpret_cast<const float4 *>(c.land(apart, c.slot, spare) + 8 * lane);
         v0 = row[0], v1 = row[1];
     }
-    __syncthreads();  // B4: the slot areas are free again
+    if (!apart) __syncthreads();  // B4: the slot areas are free again
+}
+
+// The lane's block of the wave's down rows, ahead of the activations (which then land elsewhere).
+WD_DEV Q8Block res_down_block(const ResCtx &c, const Q8CoalRaw<0, 16> &draw) {
+    uint8_t *const stage = c.area();  // (the tile, as in res_down)
+    wave_lds_fence();
+    q8_rows4_coal_stage<0, 16>(draw, stage, c.lane);
+    wave_lds_fence();
+    return q8_block_from_lds<0>(stage, c.lane);
+}
+template <bool STAMPS>
+WD_DEV void res_down_of_block(const ResidentArgs &a, const ResCtx &c, int l, const Q8Block &w, const float4 &v0, const float4 &v1) {
+    const int lane = c.lane;
+    int8_t *aq = reinterpret_cast<int8_t *>(c.area() + kResTileBytes);
+    uint16_t *ad = reinterpret_cast<uint16_t *>(c.area() + kResTileBytes + kResF);
+    Q8TileNB<16> &tile = *reinterpret_cast<Q8TileNB<16> *>(c.area());
+    lds_quantize_q8_0_step<false>(v0, v1, true, lane * 8, aq, ad, lane);
+    wave_lds_fence();
+    const float y = q8_rows4_block_dots<0, 16>(w, w, aq, ad, tile, lane);
+    if ((lane & 15) == 0) c.ybuf()[c.slot * 4 + (lane >> 4)] = y;
+    res_mark<STAMPS>(a, c, l, 7);
 }
 
 // The down rows 4r..4r+3 of one matrix against the activation values v0, v1 (8 lane .. 8 lane + 7) of slot `c.slot`:
@@ -511,8 +542,8 @@ WD_DEV void res_down(const ResidentArgs &a, const ResCtx &c, int l, Q8CoalRaw<0,
 
 // ---- the ten routed waves -------------------------------------------------------------------------------------
 // Rungs 0..7 (always waves 0..7) also fetch and quantise the layer's input.
-// Barriers of a layer, the same for every wave of the workgroup: without a routing trace B1x (input in LDS), B1 (with its quantised forms), B2..B4 (exchange of the
-// activations), B5 (down results in LDS).
+// Barriers of a layer, the same for every wave of the workgroup: without a routing trace B1x (input in LDS), B1 (with its quantised forms), B2 and B3 (exchange of the
+// activations), with a routing trace B4 (the areas that these landed in are free), B5 (down results in LDS).
 // TRACED: the launch has a routing trace (the two forms of the role differ in when they can ask for what: one body for
 // both, chosen at run time, costs the compiler's merging of registers that either form defines in its own place).
 template <int TYPE, bool STAMPS, bool TRACED>
@@ -703,14 +734,19 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         uint32_t wbits = kResEmpty;
         if (wlane && !dead) wbits = hand_load4(c.hb, woff);
         float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
-        res_exchange<STAMPS>(a, c, l, on, act, v0, v1, dead, [] {},
+        Q8Block down_block{};
+        res_exchange<STAMPS>(a, c, l, !traced, res_spare<TYPE>(), on, act, v0, v1, dead, [] {},
             [&] {  // the next layer's up row, requested behind this layer's dot products: decoded while the records travel
-                if constexpr (!kQ8) {
+                if constexpr (!traced) {
+                    if (on) down_block = res_down_block(c, draw);
+                } else if constexpr (!kQ8) {
                     if (traced && on && !last && rows_asked) iq_row8_coal_decode_kept<kIq>(raw.u[1], tables, lane, c.kept(), kept);
                 }
             },
             [] {});
-        if (on) {
+        if constexpr (!traced) {
+            if (on) res_down_of_block<STAMPS>(a, c, l, down_block, v0, v1);
+        } else if (on) {
             res_down<STAMPS>(a, c, l, draw, v0, v1, [&] {
                 if constexpr (traced) {  // the next layer's down rows (its slots filled, if they are slots)
                     draw_asked = !last && rows_asked;
@@ -787,7 +823,7 @@ WD_DEV void res_routed_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
 }
 
 // ---- the shared expert's wave ------------------------------------------------------------------------------------
-template <bool STAMPS>
+template <int TYPE, bool STAMPS>
 WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, int lane0, int wave0,
                             const ResHand &hand, bool &dead) {
     Q8Block gb[2];
@@ -848,7 +884,7 @@ WD_DEV void res_shared_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         }
         bool got = false;
         float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
-        res_exchange<STAMPS>(a, c, l, with_shared, act, v0, v1, dead,
+        res_exchange<STAMPS>(a, c, l, !traced, res_spare<TYPE>(), with_shared, act, v0, v1, dead,
             [&] { if (r == 0 && traced) got = gather_logits(false); },  // the logits ahead of the barrier, if that holds nobody up
             [] {},
             [&] {
@@ -1017,7 +1053,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
             res_mark<STAMPS>(a, c, l, 13);
         }
         __syncthreads();  // B3
-        __syncthreads();  // B4
+        if (traced) __syncthreads();  // B4
         if (r == 0 && traced) weights_from_lds();
         // the next layer's row: requested behind the selection, so that its registers are not held while the selection runs,
         // and behind the exchange, whose polls it would delay
@@ -1095,7 +1131,7 @@ __global__ __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(6, 
     if (slot < 0)
         res_router_role<STAMPS>(a, lds_res, r, fresh_lane(), wave, hand, other, dead);
     else if (slot == kResSharedSlot)
-        res_shared_role<STAMPS>(a, lds_res, r, fresh_lane(), wave, hand, dead);
+        res_shared_role<TYPE, STAMPS>(a, lds_res, r, fresh_lane(), wave, hand, dead);
     else
         if (a.ids_trace) res_routed_role<TYPE, STAMPS, true>(a, lds_res, r, fresh_lane(), wave, slot, hand, dead);
         else res_routed_role<TYPE, STAMPS, false>(a, lds_res, r, fresh_lane(), wave, slot, hand, dead);

@@ -1306,17 +1306,12 @@ WD_DEV void q8_rows4_coal_stage(const Q8CoalRaw<KIND, NB> &raw, uint8_t *stage, 
 #pragma unroll
     for (int i = 0; i < Raw::kLoads; ++i) reinterpret_cast<uint4 *>(stage)[min(i * 64 + lane, Raw::kWords - 1)] = raw.u[i];
 }
-// The dot products of the four staged rows; `stage` may be the tile itself (its chunk-sum area is overwritten only
-// after the staged bytes have been read).  y of row r4 valid in lane 16 r4.  The float order is that of q8_rows4_multi.
-// partials (PART): int32 [4 rows][NB blocks][8 chunk lanes].
+// The same with the lane's blocks (number `lane` of the four rows, and number 64 + lane where NB is 20) in registers.
 template <int KIND, int NB, bool PART = false>
-WD_DEV float q8_rows4_coal_dots(const uint8_t *stage, const int8_t *act_qs, const uint16_t *act_d, Q8TileNB<NB> &tile, int lane,
-                                int32_t *partials = nullptr) {
+WD_DEV float q8_rows4_block_dots(const Q8Block &w0, const Q8Block &w1, const int8_t *act_qs, const uint16_t *act_d, Q8TileNB<NB> &tile, int lane,
+                                 int32_t *partials = nullptr) {
     constexpr int kSecond = 4 * NB - 64, kRow = Q8TileNB<NB>::kRow;
     const int t1 = 64 + min(lane, max(kSecond, 1) - 1);
-    const Q8Block w0 = q8_block_from_lds<KIND>(stage, lane);
-    Q8Block w1 = w0;
-    if (kSecond > 0) w1 = q8_block_from_lds<KIND>(stage, t1);
     wave_lds_fence();  // the staged bytes (and, by an earlier call, the tile) have been read; the tile now takes the chunk sums
     auto sums = [&](const Q8Block &w, int t) {
         const int row = t / NB, bi = t - row * NB;
@@ -1348,6 +1343,18 @@ WD_DEV float q8_rows4_coal_dots(const uint8_t *stage, const int8_t *act_qs, cons
             acc = __builtin_fmaf(dv, pv, acc);
     }
     return close_lanes8(KIND == 1 ? acc + acc_odd : acc);
+}
+// The dot products of the four staged rows; `stage` may be the tile itself (its chunk-sum area is overwritten only
+// after the staged bytes have been read).  y of row r4 valid in lane 16 r4.  The float order is that of q8_rows4_multi.
+// partials (PART): int32 [4 rows][NB blocks][8 chunk lanes].
+template <int KIND, int NB, bool PART = false>
+WD_DEV float q8_rows4_coal_dots(const uint8_t *stage, const int8_t *act_qs, const uint16_t *act_d, Q8TileNB<NB> &tile, int lane,
+                                int32_t *partials = nullptr) {
+    constexpr int kSecond = 4 * NB - 64;
+    const Q8Block w0 = q8_block_from_lds<KIND>(stage, lane);
+    Q8Block w1 = w0;
+    if (kSecond > 0) w1 = q8_block_from_lds<KIND>(stage, 64 + min(lane, max(kSecond, 1) - 1));
+    return q8_rows4_block_dots<KIND, NB, PART>(w0, w1, act_qs, act_d, tile, lane, partials);
 }
 template <int KIND, int NB, bool PART = false>
 WD_DEV float q8_rows4_coal_finish(const Q8CoalRaw<KIND, NB> &raw, const int8_t *act_qs, const uint16_t *act_d, Q8TileNB<NB> &tile,
