@@ -114,6 +114,19 @@ def test_more_routed_items_than_the_device_holds(g, oracle, H, F, gate_t, down_t
     check_layer(g, oracle, L, x)
 
 
+@pytest.mark.parametrize("given", [False, True], ids=["selected", "given"])
+@pytest.mark.parametrize("H,F,gate_t", [(1024, 1536, synth.IQ4_NL), (1024, 1536, synth.IQ3_S), (2560, 1536, synth.IQ2_S),
+                                        (4096, 1536, synth.IQ3_S), (5120, 1024, synth.IQ3_S)])
+def test_routed_items_round_after_round(g, oracle, H, F, gate_t, given):
+    """2048 or 3072 items: three rounds of the loop and more, whose waves go from item to item by themselves, in every
+    form of the row fetch, with ids that come from the selection and with ids known before the launch."""
+    E, k = 24, 16
+    L = synth.make_layer(H, F, E, k, gate_t, synth.Q8_0, False, seed=SEED, layer=83, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 53, H), H)
+    kw = dict(ids=np.arange(k, dtype=np.int32)[::-1] + 5, weights=np.linspace(0.2, 0.01, k, dtype=np.float32), flags=capi.MOE_PRESELECTED) if given else {}
+    check_layer(g, oracle, L, x, **kw)
+
+
 @pytest.mark.parametrize("H,F,E,k,gate_t,down_t,shared", [
     (256, 32, 8, 1, synth.IQ3_S, synth.Q8_0, False),          # the smallest layer the limits allow
     (256, 32, 1024, 16, synth.IQ2_S, synth.IQ4_NL, True),     # most experts, largest top-k
