@@ -630,3 +630,35 @@ def test_activation_blocks_of_any_magnitude(g, oracle, H, F, gate_t, down_t, sha
             outs.append((g.host(dx), g.host(out)))
             sc.close()
         assert g.same_bits(outs[0][0], outs[1][0]) and g.same_bits(outs[0][1], outs[1][1]), gain
+
+
+@pytest.mark.parametrize("H,F,E,k,gate_t,down_t,shared", [(512, 64, 32, 16, synth.Q8_0, synth.Q8_0, True), (2048, 512, 16, 4, synth.IQ3_S, synth.Q8_0, True),
+                                                          (2560, 640, 16, 4, synth.IQ2_S, synth.IQ4_NL, True), (1024, 512, 32, 16, synth.Q8_0, synth.IQ4_NL, True),
+                                                          (1792, 672, 16, 4, synth.Q8_0, synth.Q8_0, False)])
+def test_one_buffer_for_two_results(g, oracle, H, F, E, k, gate_t, down_t, shared):
+    """A caller without use for the layer's output gives it the residual's buffer, or the scratch's view of the routed sum: the residual is
+    stored over the output, and the output over the view, in every form of the down projections."""
+    L = synth.make_layer(H, F, E, k, gate_t, down_t, shared, seed=SEED, layer=H + F + 5, router_sigma=1.0 / np.sqrt(H))
+    x = synth.rms_normed(synth.rng_for(SEED, 95, H), H)
+    want, _ = oracle.moe_layer(L, x)
+    dl, sc = g.DeviceLayer(L), g.Scratch(H, F, E, k)
+    scale = np.float32(2.0 ** -4)
+    both, stack = g.dev(x), (capi.MoeLayer * 2)(dl.desc, dl.desc)
+    capi.call("wd_moe_stack_f32", stack, 2, g.ptr(both), g.ptr(both), sc.h, None, float(scale), capi.MOE_PER_LAYER, g.stream())
+    g.sync()
+    after = x
+    for _ in range(2):
+        after = (after + (oracle.moe_layer(L, after)[0] * scale).astype(np.float32)).astype(np.float32)
+    assert g.same_bits(g.host(both), after)
+    rng = synth.rng_for(SEED, 96, H)
+    res0, inject = rng.normal(0, 1, (4, H)).astype(np.float32), rng.normal(0, 2, 4).astype(np.float32)
+    dx, res, d_inject = g.dev(x), g.dev(res0), g.dev(inject)
+    for stream in (0, 3):
+        res.copy_(g.dev(res0))
+        capi.call("wd_moe_layer_hc_f32", C.byref(dl.desc), g.ptr(dx), res.data_ptr() + 4 * stream * H, g.ptr(res), g.ptr(d_inject), 4, 0, sc.h, 0, g.stream())
+        g.sync()
+        assert g.same_bits(g.host(res), oracle.hc_combine(res0, want, inject, 0)), stream
+    capi.call("wd_moe_layer_f32", C.byref(dl.desc), g.ptr(dx), sc.raw("accum"), sc.h, 0, g.stream())
+    g.sync()
+    assert g.same_bits(sc.get("accum", H, np.float32), want)
+    sc.close()

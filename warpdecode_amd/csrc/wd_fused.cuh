@@ -1406,6 +1406,14 @@ WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *yb
         o = acc + prod;
     }
     if (ops.bad) acc = o = __builtin_nanf("");  // the caller sees the failure in its data, without a synchronisation
+    // (The order counts where a caller passed one buffer twice: the output over any view of the scratch, the residual over the output.)
+    if (on) {
+        if (a.expert_out)
+            for (int m = 0; m < a.k; ++m) a.expert_out[static_cast<size_t>(m) * a.H + row] = mine[m * STRIDE];
+        if (shared) a.down_f32[row] = y_shared;
+        a.accum[row] = acc;
+        a.out[row] = o;
+    }
     if (a.residual) {
         if (a.hc > 0) {
             const int c = lane >> 2;
@@ -1419,12 +1427,6 @@ WD_DEV void layer_c_fold(const LayerArgs &a, const FoldOps &ops, const float *yb
             a.residual[row] = ops.res + scaled;
         }
     }
-    if (!on) return;
-    a.out[row] = o;
-    a.accum[row] = acc;
-    if (shared) a.down_f32[row] = y_shared;
-    if (a.expert_out)
-        for (int m = 0; m < a.k; ++m) a.expert_out[static_cast<size_t>(m) * a.H + row] = mine[m * STRIDE];
 }
 // What a wave's matrix gives: NaN for an expert that has no slot (reported through the status word), so that every sum it goes into is one.
 WD_DEV float or_nan(float y, bool missing) { return missing ? __builtin_nanf("") : y; }

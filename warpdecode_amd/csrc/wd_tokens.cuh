@@ -697,13 +697,13 @@ void k_tokens_c(TokenArgs ta) {
         const float gate = readlane_f(wreg, 16);
         if (row_on) {
             float o = acc;
+            if (s.expert_out)
+                for (int j = 0; j < a.k; ++j) s.expert_out[static_cast<size_t>(j) * a.H + row] = mine[j * 8];
             if (shared) {
                 const float prod = y_shared * gate;
                 o = acc + prod;
                 s.down_f32[row] = y_shared;
             }
-            if (s.expert_out)
-                for (int j = 0; j < a.k; ++j) s.expert_out[static_cast<size_t>(j) * a.H + row] = mine[j * 8];
             s.accum[row] = bad == 1u ? __builtin_nanf("") : acc;
             s.out[row] = bad == 1u ? __builtin_nanf("") : o;
         }
@@ -810,13 +810,13 @@ __global__ __launch_bounds__(64 * kTokensCEvenWaves) void k_tokens_c_even(TokenA
         const float gate = readlane_f(wreg, 16);
         if (row_on) {
             float o = acc;
+            if (s.expert_out)
+                for (int j = 0; j < a.k; ++j) s.expert_out[static_cast<size_t>(j) * a.H + row] = mine[j * 16];
             if (shared) {
                 const float prod = y_shared * gate;
                 o = acc + prod;
                 s.down_f32[row] = y_shared;
             }
-            if (s.expert_out)
-                for (int j = 0; j < a.k; ++j) s.expert_out[static_cast<size_t>(j) * a.H + row] = mine[j * 16];
             s.accum[row] = bad == 1u ? __builtin_nanf("") : acc;
             s.out[row] = bad == 1u ? __builtin_nanf("") : o;
         }
