@@ -91,6 +91,26 @@ def test_layer_with_combine(g, oracle, flags, shape):
         sc.close()
 
 
+@pytest.mark.parametrize("H,F,k,gate_t,down_t,shared", [(2304, 800, 3, synth.IQ2_S, synth.IQ4_NL, True), (4352, 1024, 10, synth.IQ2_S, synth.IQ4_NL, True),
+                                                        (4352, 800, 11, synth.Q8_0, synth.Q8_0, False), (2560, 544, 16, synth.IQ2_S, synth.Q8_0, True),
+                                                        (2304, 768, 16, synth.Q8_0, synth.IQ4_NL, True)])
+def test_combine_where_two_down_workgroups_share_a_compute_unit(g, oracle, H, F, k, gate_t, down_t, shared):
+    """More than 256 workgroups of the down projections: the forms of 25..32 blocks per row and of two matrices per wave that are made for two per compute unit."""
+    E = 24
+    L = synth.make_layer(H, F, E, k, gate_t, down_t, shared, seed=SEED, layer=900 + k, router_sigma=1.0 / np.sqrt(H))
+    rng = synth.rng_for(SEED, 503, H, k)
+    x = synth.rms_normed(rng, H)
+    res0, inject = rng.normal(0, 1, (4, H)).astype(np.float32), rng.normal(0, 2, 4).astype(np.float32)
+    want_out, _ = oracle.moe_layer(L, x)
+    dl, sc = g.DeviceLayer(L), g.Scratch(H, F, E, k)
+    res, out, dx, d_inject = g.dev(res0), g.empty(H, np.float32), g.dev(x), g.dev(inject)
+    capi.call("wd_moe_layer_hc_f32", C.byref(dl.desc), g.ptr(dx), g.ptr(out), g.ptr(res), g.ptr(d_inject), 4, 0, sc.h, 0, g.stream())
+    g.sync()
+    assert g.same_bits(g.host(out), want_out)
+    assert g.same_bits(g.host(res), oracle.hc_combine(res0, want_out, inject, 0))
+    sc.close()
+
+
 def test_hc_error_paths(g):
     x = g.empty(64, np.float32)
     lib = capi.load()

@@ -1508,9 +1508,15 @@ __host__ __device__ inline uint32_t layer_c8_wave_bytes(int F) {
     static_assert(sizeof(Q8Tile8) <= kQ8Rows8StageBytes, "the tile lies in the staging area");
     return (WORDS ? kQ8Rows8StageBytes : static_cast<uint32_t>(sizeof(Q8Tile8))) + (static_cast<uint32_t>(F + F / 16 + 15) & ~15u);
 }
-template <int KIND, int PASSES, bool WORDS, bool PART = false, bool TRACE = false, bool TWO = false>
-__global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
+// Registers: grids of more than 256 workgroups (hidden beyond 2048) want two on a compute unit, which with nine to twelve waves each takes six waves per SIMD, so
+// at most 80 registers.  Rows of 25..32 blocks that a lane loads itself stay below by asking for what the fold needs behind the quantisation
+// (kLate; eleven IQ4_NL matrices, 5120 / 1024: 46.2 us per layer with 83 registers, 42.8 with 78); two matrices per wave of 17..24 blocks by the
+// general quantisation (ORDINARY false: 5120 / 768 IQ4_NL 53.2 with 87, 50.7 with 79; where one workgroup per compute unit is all there is, 2048 / 768, the
+// ordinary one is the faster, 22.3 against 23.1).
+template <int KIND, int PASSES, bool WORDS, bool PART = false, bool TRACE = false, bool TWO = false, bool ORDINARY = true>
+__global__ __launch_bounds__(TWO ? 576 : 1024, (TWO ? !ORDINARY : PASSES == 4 && !WORDS && !PART && !TRACE) ? 6 : 1) void k_layer_c8(LayerArgs a) {
     constexpr int STEPS = (PASSES + 1) / 2;  // of sixteen blocks
+    constexpr bool kLate = PASSES == 4 && !WORDS;
     extern __shared__ __align__(16) uint8_t lds_c8[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int n_act = a.k + (a.sh_inp ? 1 : 0);
@@ -1548,11 +1554,13 @@ __global__ __launch_bounds__(TWO ? 576 : 1024) void k_layer_c8(LayerArgs a) {
             constexpr bool P = decltype(part)::value;
             typename std::conditional<WORDS, Q8Rows8Fetch<K, STEPS>, Q8Rows8Blocks<K, PASSES>>::type fetch;
             fetch.request(rows, nb, lane);
-            if (wave < 2 && (!TWO || m < 9)) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+            if (!kLate && wave < 2 && (!TWO || m < 9)) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+            if (kLate) stream_w = layer_c_stream_weight(a, stream, wave < 2);
 #pragma unroll
             for (int i = 0; i < STEPS; ++i)
-                lds_quantize_q8_0_step(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
-            if (!TWO || m < 9) stream_w = layer_c_stream_weight(a, stream, wave < 2);
+                lds_quantize_q8_0_step<ORDINARY>(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
+            if (kLate && wave < 2) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+            if (!kLate && (!TWO || m < 9)) stream_w = layer_c_stream_weight(a, stream, wave < 2);
             mark<TRACE>(a, 2, 1);
             Q8Chain ch;
             int32_t *pp = P ? a.down_part + (static_cast<size_t>(m) * a.H + r0) * (static_cast<size_t>(nb) * 8) : nullptr;

@@ -684,8 +684,10 @@ void launch_layer_c8_two(hipStream_t st, const LayerArgs &a) {
     const dim3 grid(a.H / 8), block(64 * 9);
     if (a.F <= 512)
         enqueue(k_layer_c8<KIND, 2, false, false, false, true>, grid, block, lds, st, a);
-    else
+    else if (a.H <= 2048)
         enqueue(k_layer_c8<KIND, 3, false, false, false, true>, grid, block, lds, st, a);
+    else  // more workgroups than compute units: the form of which two fit one
+        enqueue(k_layer_c8<KIND, 3, false, false, false, true, false>, grid, block, lds, st, a);
 }
 template <int KIND>
 void launch_layer_c8(bool words, hipStream_t st, const LayerArgs &a) {
