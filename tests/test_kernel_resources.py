@@ -1,5 +1,6 @@
-"""What the compiler gave the kernels that several workgroups of a compute unit depend on: vector registers, scratch and spills, from
-the metadata of the library that was built here.  (A compute unit has four SIMDs of 512 registers per lane: six waves on each need at most 80.)"""
+"""The kernels of the library that was built here, as they came out of the compiler.  Vector registers, scratch and spills where several workgroups are meant to
+share a compute unit (it has four SIMDs of 512 registers per lane: six waves on each need at most 80); and the statements in assembly whose wait
+states the compiler does not know."""
 import os
 import re
 import subprocess
@@ -12,8 +13,7 @@ BIN = "/opt/rocm/llvm/bin/"
 
 
 @pytest.fixture(scope="module")
-def kernels(tmp_path_factory):
-    """name -> (vector registers, bytes of scratch per lane, spilled vector registers)"""
+def code_object(tmp_path_factory):
     if not os.path.exists(BIN + "clang-offload-bundler"):
         pytest.skip("no LLVM tools")
     if not os.path.exists(build.LIB):
@@ -23,6 +23,13 @@ def kernels(tmp_path_factory):
     subprocess.check_call([BIN + "llvm-objcopy", "--dump-section", ".hip_fatbin=" + fat, build.LIB, os.devnull])
     subprocess.check_call([BIN + "clang-offload-bundler", "--type=o", "--unbundle", "--input=" + fat, "--output=" + co,
                            "--targets=hipv4-amdgcn-amd-amdhsa--gfx950"])
+    return co
+
+
+@pytest.fixture(scope="module")
+def kernels(code_object):
+    """name -> (vector registers, bytes of scratch per lane, spilled vector registers)"""
+    co = code_object
     notes = subprocess.run([BIN + "llvm-readelf", "--notes", co], check=True, capture_output=True, text=True).stdout
     field = lambda text, name: int(re.search(r"\.%s:\s+(\d+)" % name, text).group(1))
     out = {}
@@ -46,3 +53,21 @@ def _kernel(kernels, name, *args):
 def test_two_workgroups_of_down_projections_fit_a_compute_unit(kernels, args):
     vgprs, scratch, spills = _kernel(kernels, "k_layer_c8", *args)
     assert vgprs <= 80 and scratch == 0 and spills == 0, (vgprs, scratch, spills)
+
+
+def test_scalar_operands_of_the_look_ups_come_from_their_own_statement(code_object):
+    """A vector instruction that reads a scalar register needs two wait states behind a vector instruction that writes it.  The compiler keeps them
+    for its own instructions, not for those of a statement in assembly: the byte and half-word selects of the IQ look-ups
+    find their constant written by a scalar instruction right ahead of the two that use it, whatever the compiler puts in front."""
+    dis = subprocess.Popen([BIN + "llvm-objdump", "-d", "--no-show-raw-insn", code_object], stdout=subprocess.PIPE, text=True)
+    selects, before = 0, ["", ""]
+    for line in dis.stdout:
+        text = line.split("//")[0].strip()
+        if text.startswith(("v_and_b32_sdwa", "v_lshlrev_b32_sdwa")):
+            scalar = re.search(r", (s\d+), ", text)
+            if scalar:
+                selects += 1
+                wrote = re.compile(r"(s_movk_i32|s_mov_b32) %s, " % scalar.group(1))
+                assert any(wrote.match(b) for b in before), (before, text)
+        before = [before[1], text]
+    assert dis.wait() == 0 and selects > 1000

@@ -162,35 +162,32 @@ WD_DEV IqFields iq_load(const uint8_t *blk, int ib) {
 // to where they are worth eight for four bytes at once, and one that reads a byte takes each.  29 instructions for the sixteen look-ups of an IQ3_S block, each
 // by itself took 48; 20 for the twelve of IQ2_S in place of 32.  (4096 / 1536 IQ3_S, eight of 128 experts: 39.4 us per layer, so
 // 38.0; four tokens of 2048 / 512 38.7, 38.2.)
-// (Those two through assembly: the compiler folds the shift of a half, or the mask of a byte, into a shift and a mask of the whole register, two instructions.  Nothing
-// but plain vector instructions produces the operand, and LDS instructions take the result, so that there are no wait states to be known.)
-// (The amount in a scalar register for IQ3_S, in a vector register for IQ2_S: the other way round dispatch AB gets a scratch frame.)
-#define WD_HALF_SHIFTED(AMOUNT, WORD) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" WORD : "=v"(r) : AMOUNT(SHIFT), "v"(x))
-template <int SHIFT, int HALF>
-WD_DEV uint32_t half_shifted(uint32_t x) {
-    uint32_t r;
-    if (SHIFT == 2 && HALF == 0) WD_HALF_SHIFTED("s", "WORD_0");
-    else if (SHIFT == 2) WD_HALF_SHIFTED("s", "WORD_1");
-    else if (HALF == 0) WD_HALF_SHIFTED("v", "WORD_0");
-    else WD_HALF_SHIFTED("v", "WORD_1");
-    return r;
+// (Those two through assembly: the compiler folds the shift of a half, or the mask of a byte, into a shift and a mask of the whole register, two instructions.  It also
+// knows nothing of the two wait states between a vector instruction that writes a scalar register, such as the reload of a spilled one, and its use here: so a
+// constant in a scalar register is written by a scalar instruction of the same statement, one for the two that use it.  The vector operands come from plain vector
+// instructions, and LDS instructions take the results.  IQ2_S takes its amount from a vector register: in a scalar one dispatch AB gets a scratch frame.)
+WD_DEV void halves_times_four(uint32_t x, uint32_t &lo, uint32_t &hi) {
+    uint32_t by;
+    asm("s_mov_b32 %2, 2\n\tv_lshlrev_b32_sdwa %0, %2, %3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0\n\t"
+        "v_lshlrev_b32_sdwa %1, %2, %3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=&v"(lo), "=v"(hi), "=&s"(by) : "v"(x));
 }
-#undef WD_HALF_SHIFTED
+#define WD_TWO_BYTES(BYTE) asm("s_movk_i32 %2, 0x78\n\tv_and_b32_sdwa %0, %2, %3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" BYTE "\n\t" \
+    "v_and_b32_sdwa %1, %2, %4 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" BYTE : "=&v"(a), "=v"(b), "=&s"(mask) : "v"(lo), "v"(hi))
 template <int BYTE>
-WD_DEV uint32_t byte_masked(uint32_t mask, uint32_t x) {
-    uint32_t r;
-    if (BYTE == 0) asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0" : "=v"(r) : "s"(mask), "v"(x));
-    else if (BYTE == 1) asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_1" : "=v"(r) : "s"(mask), "v"(x));
-    else if (BYTE == 2) asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_2" : "=v"(r) : "s"(mask), "v"(x));
-    else asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_3" : "=v"(r) : "s"(mask), "v"(x));
-    return r;
+WD_DEV void bytes_masked(uint32_t lo, uint32_t hi, uint32_t &a, uint32_t &b) {
+    uint32_t mask;
+    if (BYTE == 0) WD_TWO_BYTES("BYTE_0");
+    else if (BYTE == 1) WD_TWO_BYTES("BYTE_1");
+    else if (BYTE == 2) WD_TWO_BYTES("BYTE_2");
+    else WD_TWO_BYTES("BYTE_3");
 }
+#undef WD_TWO_BYTES
 // chunk c's sign nibble (of four sign bytes: c >> 1, its half c & 1), for chunks 4 HALF .. 4 HALF + 3
 template <int HALF>
 WD_DEV void iq_sign_offsets(uint32_t sg, uint32_t (&off)[4]) {
     const uint32_t lo = sg << 3, hi = sg >> 1;  // the low nibble of every byte, and the high one, where they are worth eight
-    off[0] = byte_masked<2 * HALF>(0x78u, lo), off[1] = byte_masked<2 * HALF>(0x78u, hi);
-    off[2] = byte_masked<2 * HALF + 1>(0x78u, lo), off[3] = byte_masked<2 * HALF + 1>(0x78u, hi);
+    bytes_masked<2 * HALF>(lo, hi, off[0], off[1]);
+    bytes_masked<2 * HALF + 1>(lo, hi, off[2], off[3]);
 }
 // IQ3_S: eight indices, byte c with bit c of qh above it; for chunks 4 HALF .. 4 HALF + 3
 template <int HALF>
@@ -199,7 +196,8 @@ WD_DEV void iq3_grid_offsets(uint2 qs, uint32_t qh, uint32_t (&off)[4]) {
     const uint32_t even = __umul24(qh & 0x55u, 0x41041u) & 0x01010101u, odd = __umul24((qh >> 1) & 0x55u, 0x41041u) & 0x01010101u;
     const uint32_t q = HALF ? qs.y : qs.x;
     const uint32_t i02 = __builtin_amdgcn_perm(even, q, HALF ? 0x07020600u : 0x05020400u), i13 = __builtin_amdgcn_perm(odd, q, HALF ? 0x07030601u : 0x05030401u);
-    off[0] = half_shifted<2, 0>(i02), off[2] = half_shifted<2, 1>(i02), off[1] = half_shifted<2, 0>(i13), off[3] = half_shifted<2, 1>(i13);
+    halves_times_four(i02, off[0], off[2]);
+    halves_times_four(i13, off[1], off[3]);
 }
 // IQ2_S: four indices, byte g with bits 2 g and 2 g + 1 of qh above it; for g = 2 HALF, 2 HALF + 1
 template <int HALF>
@@ -207,7 +205,8 @@ WD_DEV void iq2_grid_offsets(uint32_t qs, uint32_t qh, uint32_t (&off)[2]) {
     qh &= 0xffu;  // (some callers' has other fields above)
     const uint32_t wide = (qh | (qh << 12)) & 0x000f000fu, above = (wide | (wide << 6)) & 0x03030303u;
     const uint32_t i = __builtin_amdgcn_perm(above, qs, HALF ? 0x07030602u : 0x05010400u);
-    off[0] = half_shifted<3, 0>(i), off[1] = half_shifted<3, 1>(i);
+    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(off[0]) : "v"(3), "v"(i));
+    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=v"(off[1]) : "v"(3), "v"(i));
 }
 // Chunks 4 HALF .. 4 HALF + 3 of a block: magnitudes and sign masks looked up.
 template <int TYPE, int HALF, typename Tables>
