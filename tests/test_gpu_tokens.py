@@ -99,6 +99,18 @@ def test_tokens_equal_single_passes(g, oracle, gate_t, down_t, shared, H, F, E, 
         assert g.same_bits(got["out"][t], want)
 
 
+@pytest.mark.parametrize("T,F", [(2, 32), (3, 640), (4, 96)])
+def test_up_to_four_tokens_on_ten_super_blocks_of_iq2_s(g, oracle, T, F):
+    """The kernel of up to four tokens whose look-ups are made half a block at a time."""
+    H, E, k = 2560, 16, 6
+    L = synth.make_layer(H, F, E, k, synth.IQ2_S, synth.IQ4_NL, True, seed=SEED, layer=17 + T, router_sigma=1.0 / np.sqrt(H))
+    xs = correlated_tokens(H, T, H + T)
+    got = run_tokens(g, g.DeviceLayer(L), L, xs)
+    for t in range(T):
+        want, d = oracle.moe_layer(L, xs[t])
+        assert np.array_equal(got["ids"][t], d["ids"]) and g.same_bits(got["accum"][t], d["routed"]) and g.same_bits(got["out"][t], want)
+
+
 def test_tokens_preselected_full_overlap(g, oracle):
     """All tokens name the same experts in different orders: one union entry per expert."""
     L = synth.make_c2(n_experts=32)

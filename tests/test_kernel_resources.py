@@ -55,6 +55,12 @@ def test_two_workgroups_of_down_projections_fit_a_compute_unit(kernels, args):
     assert vgprs <= 80 and scratch == 0 and spills == 0, (vgprs, scratch, spills)
 
 
+def test_spills_of_the_token_batch_at_ten_super_blocks(kernels):
+    """Three workgroups per compute unit, bought with a few spills: not with more than when the figures beside the kernel were taken."""
+    vgprs, scratch, spills = _kernel(kernels, "k_tokens_ab", 22, 4, 10)
+    assert vgprs <= 80 and scratch <= 24 and spills <= 5, (vgprs, scratch, spills)
+
+
 def test_scalar_operands_of_the_look_ups_come_from_their_own_statement(code_object):
     """A vector instruction that reads a scalar register needs two wait states behind a vector instruction that writes it.  The compiler keeps them
     for its own instructions, not for those of a statement in assembly: the byte and half-word selects of the IQ look-ups

@@ -69,6 +69,10 @@ struct IqTables {
     WD_DEV uint64_t grid2_bytes(uint32_t off) const { return *reinterpret_cast<const uint64_t *>(reinterpret_cast<const uint8_t *>(grid2) + off); }  // off = 8 idx
     WD_DEV uint2 sign_bytes(uint32_t off) const { return *reinterpret_cast<const uint2 *>(reinterpret_cast<const uint8_t *>(sign) + off); }         // off = 8 nibble
 };
+// The same for a kernel without registers for all of a block's look-ups at once, or for the constants of the IQ2_S offsets.
+struct IqTablesTight : IqTables {
+    static constexpr bool kTight = true;
+};
 // The same tables for a kernel that knows their LDS byte address when it is compiled (BASE: the address of an IqTables
 // in the workgroup's LDS): a lookup's address is then the scaled index alone, the rest goes into the load's offset field.
 template <unsigned BASE>
@@ -221,7 +225,7 @@ WD_DEV void iq_look_up(const IqFields &f, const Tables &t, uint32_t (&g)[4], uin
     } else {
         uint32_t go[2];
         iq2_grid_offsets<HALF>(f.qs.x, f.qh, go);
-        if (Tables::kTight) {  // (the constants of the assembly took 36 registers too many)
+        if (Tables::kTight) {  // (the constants of the assembly took 36 registers too many in the resident stack)
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int q = 2 * HALF + i;

@@ -319,6 +319,9 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
         return;
     }
     IqTables &tables = reinterpret_cast<Routed *>(s_area)->tables;
+    // (IQ2_S, ten super-blocks, three workgroups per compute unit: with all look-ups of a block at once 11 registers are spilled, half by half 5.  2560 / 640, two
+    // tokens 31.8 us per layer, so 31.1, three 41.6, 41.0, four 49.1, 49.0.)
+    const auto &look_up = static_cast<const typename std::conditional<TYPE == 22 && FETCH == 10 && kTokensBPerCu<TYPE, MAXT, FETCH> == 3, IqTablesTight, IqTables>::type &>(tables);
     TokenUnion &un = reinterpret_cast<Routed *>(s_area)->un;
     const int wg = static_cast<int>(blockIdx.x) - ta.front_wgs, n_wgs = static_cast<int>(gridDim.x) - ta.front_wgs;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -429,7 +432,7 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
                 }
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    iq_decode<TYPE>(f[i], ib, tables, w[i], ls[i]);
+                    iq_decode<TYPE>(f[i], ib, look_up, w[i], ls[i]);
                     dw[i] = h2f(f[i].d);
                 }
             }
@@ -490,7 +493,7 @@ __global__ __launch_bounds__(512, (2 * kTokensBPerCu<TYPE, MAXT, FETCH>)) void k
             const IqFields f = iq_fields_lds<TYPE>(stage + ri * kStage + (ri ? lead[1] : lead[0]) + sb * kBlk, ib, sb);
             uint32_t w[8];
             int ls[2];
-            iq_decode<TYPE>(f, ib, tables, w, ls);
+            iq_decode<TYPE>(f, ib, look_up, w, ls);
             const float dw = h2f(f.d);
 #pragma unroll
             for (int t = 0; t < MAXT; ++t) {
