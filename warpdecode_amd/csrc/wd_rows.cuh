@@ -169,39 +169,57 @@ WD_DEV IqFields iq_load(const uint8_t *blk, int ib) {
 // (Those two through assembly: the compiler folds the shift of a half, or the mask of a byte, into a shift and a mask of the whole register, two instructions.  It also
 // knows nothing of the two wait states between a vector instruction that writes a scalar register, such as the reload of a spilled one, and its use here: so a
 // constant in a scalar register is written by a scalar instruction of the same statement, one for the two that use it.  The vector operands come from plain vector
-// instructions, and LDS instructions take the results.  IQ2_S takes its amount from a vector register: in a scalar one dispatch AB gets a scratch frame.)
-WD_DEV void halves_times_four(uint32_t x, uint32_t &lo, uint32_t &hi) {
-    uint32_t by;
-    asm("s_mov_b32 %2, 2\n\tv_lshlrev_b32_sdwa %0, %2, %3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0\n\t"
-        "v_lshlrev_b32_sdwa %1, %2, %3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=&v"(lo), "=v"(hi), "=&s"(by) : "v"(x));
+// instructions, and LDS instructions take the results.  In vector registers - TIGHT: the resident stack, which has two left and whose waves wait for every
+// instruction - the constants need no instruction; 48 layers with a routing trace 521 us, 527 with the scalar ones.  The amount of IQ2_S too: in a scalar one
+// dispatch AB gets a scratch frame.)
+#define WD_SELECT(OP, OUT, BY, IN, PART) OP "_sdwa " OUT ", " BY ", " IN " dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" PART
+// lo and hi: the low and the high half of x times 2^SHIFT
+template <int SHIFT, bool TIGHT>
+WD_DEV void halves_shifted(uint32_t x, uint32_t &lo, uint32_t &hi) {
+    if constexpr (TIGHT || SHIFT != 2) {
+        asm(WD_SELECT("v_lshlrev_b32", "%0", "%1", "%2", "WORD_0") : "=v"(lo) : "v"(SHIFT), "v"(x));
+        asm(WD_SELECT("v_lshlrev_b32", "%0", "%1", "%2", "WORD_1") : "=v"(hi) : "v"(SHIFT), "v"(x));
+    } else {
+        uint32_t by;
+        asm("s_mov_b32 %2, 2\n\t" WD_SELECT("v_lshlrev_b32", "%0", "%2", "%3", "WORD_0") "\n\t" WD_SELECT("v_lshlrev_b32", "%1", "%2", "%3", "WORD_1")
+            : "=&v"(lo), "=v"(hi), "=&s"(by) : "v"(x));
+    }
 }
-#define WD_TWO_BYTES(BYTE) asm("s_movk_i32 %2, 0x78\n\tv_and_b32_sdwa %0, %2, %3 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" BYTE "\n\t" \
-    "v_and_b32_sdwa %1, %2, %4 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:" BYTE : "=&v"(a), "=v"(b), "=&s"(mask) : "v"(lo), "v"(hi))
-template <int BYTE>
-WD_DEV void bytes_masked(uint32_t lo, uint32_t hi, uint32_t &a, uint32_t &b) {
+// from_lo and from_hi: byte BYTE of lo and of hi, and 0x78
+template <int BYTE, bool TIGHT>
+WD_DEV void bytes_masked(uint32_t lo, uint32_t hi, uint32_t &from_lo, uint32_t &from_hi) {
     uint32_t mask;
-    if (BYTE == 0) WD_TWO_BYTES("BYTE_0");
-    else if (BYTE == 1) WD_TWO_BYTES("BYTE_1");
-    else if (BYTE == 2) WD_TWO_BYTES("BYTE_2");
-    else WD_TWO_BYTES("BYTE_3");
+#define WD_BOTH(PART)                                                                                                                       \
+    if constexpr (TIGHT) {                                                                                                                  \
+        asm(WD_SELECT("v_and_b32", "%0", "%1", "%2", PART) : "=v"(from_lo) : "v"(0x78u), "v"(lo));                                             \
+        asm(WD_SELECT("v_and_b32", "%0", "%1", "%2", PART) : "=v"(from_hi) : "v"(0x78u), "v"(hi));                                             \
+    } else {                                                                                                                                \
+        asm("s_movk_i32 %2, 0x78\n\t" WD_SELECT("v_and_b32", "%0", "%2", "%3", PART) "\n\t" WD_SELECT("v_and_b32", "%1", "%2", "%4", PART)     \
+            : "=&v"(from_lo), "=v"(from_hi), "=&s"(mask) : "v"(lo), "v"(hi));                                                               \
+    }
+    if constexpr (BYTE == 0) { WD_BOTH("BYTE_0") }
+    else if constexpr (BYTE == 1) { WD_BOTH("BYTE_1") }
+    else if constexpr (BYTE == 2) { WD_BOTH("BYTE_2") }
+    else { WD_BOTH("BYTE_3") }
+#undef WD_BOTH
 }
-#undef WD_TWO_BYTES
+#undef WD_SELECT
 // chunk c's sign nibble (of four sign bytes: c >> 1, its half c & 1), for chunks 4 HALF .. 4 HALF + 3
-template <int HALF>
+template <int HALF, bool TIGHT>
 WD_DEV void iq_sign_offsets(uint32_t sg, uint32_t (&off)[4]) {
     const uint32_t lo = sg << 3, hi = sg >> 1;  // the low nibble of every byte, and the high one, where they are worth eight
-    bytes_masked<2 * HALF>(lo, hi, off[0], off[1]);
-    bytes_masked<2 * HALF + 1>(lo, hi, off[2], off[3]);
+    bytes_masked<2 * HALF, TIGHT>(lo, hi, off[0], off[1]);
+    bytes_masked<2 * HALF + 1, TIGHT>(lo, hi, off[2], off[3]);
 }
 // IQ3_S: eight indices, byte c with bit c of qh above it; for chunks 4 HALF .. 4 HALF + 3
-template <int HALF>
+template <int HALF, bool TIGHT>
 WD_DEV void iq3_grid_offsets(uint2 qs, uint32_t qh, uint32_t (&off)[4]) {
     // bit 2 j of the factor goes from 2 j to 8 j by the summand shifted by 6 j; where summands meet, at 6, 12 and 18, a sum does not reach the bits kept
     const uint32_t even = __umul24(qh & 0x55u, 0x41041u) & 0x01010101u, odd = __umul24((qh >> 1) & 0x55u, 0x41041u) & 0x01010101u;
     const uint32_t q = HALF ? qs.y : qs.x;
     const uint32_t i02 = __builtin_amdgcn_perm(even, q, HALF ? 0x07020600u : 0x05020400u), i13 = __builtin_amdgcn_perm(odd, q, HALF ? 0x07030601u : 0x05030401u);
-    halves_times_four(i02, off[0], off[2]);
-    halves_times_four(i13, off[1], off[3]);
+    halves_shifted<2, TIGHT>(i02, off[0], off[2]);
+    halves_shifted<2, TIGHT>(i13, off[1], off[3]);
 }
 // IQ2_S: four indices, byte g with bits 2 g and 2 g + 1 of qh above it; for g = 2 HALF, 2 HALF + 1
 template <int HALF>
@@ -209,17 +227,16 @@ WD_DEV void iq2_grid_offsets(uint32_t qs, uint32_t qh, uint32_t (&off)[2]) {
     qh &= 0xffu;  // (some callers' has other fields above)
     const uint32_t wide = (qh | (qh << 12)) & 0x000f000fu, above = (wide | (wide << 6)) & 0x03030303u;
     const uint32_t i = __builtin_amdgcn_perm(above, qs, HALF ? 0x07030602u : 0x05010400u);
-    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_0" : "=v"(off[0]) : "v"(3), "v"(i));
-    asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:WORD_1" : "=v"(off[1]) : "v"(3), "v"(i));
+    halves_shifted<3, false>(i, off[0], off[1]);
 }
 // Chunks 4 HALF .. 4 HALF + 3 of a block: magnitudes and sign masks looked up.
 template <int TYPE, int HALF, typename Tables>
 WD_DEV void iq_look_up(const IqFields &f, const Tables &t, uint32_t (&g)[4], uint2 (&sm)[4]) {
     uint32_t so[4];
-    iq_sign_offsets<HALF>(TYPE == 21 ? f.sg : f.qs.y, so);
+    iq_sign_offsets<HALF, Tables::kTight>(TYPE == 21 ? f.sg : f.qs.y, so);
     if (TYPE == 21) {
         uint32_t go[4];
-        iq3_grid_offsets<HALF>(f.qs, f.qh, go);
+        iq3_grid_offsets<HALF, Tables::kTight>(f.qs, f.qh, go);
 #pragma unroll
         for (int c = 0; c < 4; ++c) g[c] = t.grid3_bytes(go[c]), sm[c] = t.sign_bytes(so[c]);
     } else {
