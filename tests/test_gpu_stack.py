@@ -416,3 +416,32 @@ def test_one_launch_stack_keeps_the_descriptors_of_a_recorded_graph(g):
     assert capi.load().wd_moe_scratch_status(sc.h) == 0
     sc.close()
     ref.close()
+
+
+def test_one_launch_stack_lists_of_any_length(g, oracle):
+    """Routers whose favourites crowd into few residues: the one launch ranks up to 64 candidates as the layers by themselves do, and
+    leaves what is longer to the rungs over the probabilities."""
+    import selection_rule as rule
+    E, k, nl = 512, 10, 2
+    L = synth.make_layer(2048, 512, E, k, synth.IQ2_S, synth.Q8_0, shared=True, layer=370, router_sigma=1.0 / np.sqrt(2048.0))
+    dls, one = _descs(g, [L])
+    sc_a, sc_b = g.Scratch(2048, 512, E, k), g.Scratch(2048, 512, E, k)
+    x = synth.rms_normed(synth.rng_for(SEED, 87), 2048)
+    lengths = []
+    for _, row in rule.crowded_rows(E, k):
+        Lr = dict(L, router=np.outer(row, x / np.float32(np.dot(x, x))).astype(np.float32))
+        d_router, arr = g.dev(Lr["router"]), (capi.MoeLayer * nl)(one[0], one[0])
+        for l in range(nl):
+            arr[l].router = d_router.data_ptr()
+        got = _run_stack(g, arr, nl, x, None, sc_a, 0)
+        want = _run_stack(g, arr, nl, x, None, sc_b, PER_LAYER)
+        wx = x.copy()
+        for l in range(nl):
+            wout, dump = oracle.moe_layer(Lr, wx)
+            wx = (wx + (wout * np.float32(2.0 ** -12)).astype(np.float32)).astype(np.float32)
+        assert g.same_bits(got[0], wx) and g.same_bits(got[1], wout) and np.array_equal(got[2]["ids"], dump["ids"])
+        assert g.same_bits(want[0], wx) and g.same_bits(want[1], wout)
+        lengths.append(rule.list_lengths(got[2]["logits"], k))
+    assert any(32 < f <= 64 for f, _ in lengths) and any(f > 64 >= s for f, s in lengths) and any(s > 64 for _, s in lengths), lengths
+    sc_a.close()
+    sc_b.close()
