@@ -71,6 +71,17 @@ def build_host_test(verbose=False):
     return exe
 
 
+def build_device_test(verbose=False):
+    """Kernels that only tests launch (tests/device), compiled as the library is."""
+    d = os.path.join(os.path.dirname(HERE), "tests", "device")
+    out = os.path.join(d, "libtest_quantiser.so")
+    cmd = ["hipcc"] + FLAGS + ["-I" + CSRC, "-o", out, os.path.join(d, "test_quantiser.hip")]
+    if verbose:
+        print(" ".join(cmd))
+    subprocess.check_call(cmd)
+    return out
+
+
 if __name__ == "__main__":
     build(verbose=True)
     print("built", LIB)

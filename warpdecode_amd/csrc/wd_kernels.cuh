@@ -143,7 +143,7 @@ WD_DEV uint32_t q8_0_pack4(float4 v, float amax) {
 // In dispatch C the quantisation of 512 values by a wave was 100 vector instructions, of 164 with the down rows behind it.  On blocks whose largest
 // magnitude is between 2^-100 and 2^100 and which hold no NaN it takes 55, with the same bits:
 //   * a quotient by one step of Newton's iteration on the reciprocal and one correction of the quotient: what remains of an IEEE division without the scaling
-//     and the special cases (equal to it for every float of the range, 1,677,721,600 of them, for 127 / a and for a / 127);
+//     and the special cases (equal to it for every float of the range, 1,677,721,601 of them, for 127 / a and for a / 127: test_gpu_quantiser);
 //   * a value times the inverse scale rounded to an integer by adding 1.5 * 2^23: the sum's low byte is the quant, and anything that is not a number
 //     of the range shows in the upper bits, of eight values at once.
 // A wave with any other block takes the general form for all of its blocks.  (us per layer: 2560 / 640, IQ4_NL down 21.7, so 21.4; 4096 / 1536 37.6, 37.2.  The
