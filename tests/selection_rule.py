@@ -11,28 +11,21 @@ def keys(logits):
     return np.where(b >> 31, ~b, b ^ np.uint32(0x80000000)).astype(np.int64)
 
 
-def list_lengths(logits, k, wide=True):
-    """Candidates by the first threshold, the (k+1)-th largest key of sixteen groups (32 from k = 12 on), and - where these are more than 64 - by the second, that of 64 lanes.
+def list_length(logits, k, wide=True):
+    """Candidates: the keys not below the (k+1)-th largest of the best of sixteen groups (32 from k = 12 on).
     wide: the row lies eight logits to a lane, however short it is."""
     n = logits.size
     padded = np.full(512 if wide else max(64, 1 << (n - 1).bit_length()), FINITE - 1, np.int64)
     padded[:n] = keys(logits)
-
-    def largest(groups):
-        return np.sort(padded.reshape(-1, groups).max(axis=0))[::-1]
-
-    heads = largest(16 if k < 12 or padded.size == 64 else 32)
+    heads = padded.reshape(-1, 16 if k < 12 or padded.size == 64 else 32).max(axis=0)
     exact = heads[(heads[:, None] < heads[None, :]).sum(axis=1) == k]
-    first = int((padded >= max(exact[0] if exact.size else 0, FINITE)).sum())
-    if first <= 64:
-        return first, first
-    return first, int((padded >= max(largest(64)[k], FINITE)).sum())
+    return int((padded >= max(exact[0] if exact.size else 0, FINITE)).sum())
 
 
 def select(logits, k, gap=GAP, gap_last=GAP_LAST, wide=True):
     """(accepted, ids): ids only if accepted."""
     key, n = keys(logits), logits.size
-    if (key < FINITE - 1).any() or list_lengths(logits, k, wide)[1] > 64:   # (NaN with its sign set)
+    if (key < FINITE - 1).any() or list_length(logits, k, wide) > 64:   # (NaN with its sign set)
         return False, None
     order = np.argsort(key, kind="stable")[::-1][:k + 1]
     slots = [int(e) for e in order if key[e] >= FINITE]
@@ -49,10 +42,10 @@ def select(logits, k, gap=GAP, gap_last=GAP_LAST, wide=True):
 
 
 def crowded_rows(n, k, seed=0):
-    """Rows whose favourites crowd into few residues modulo 16 or 64, so that the first list, and the second, comes out long: (lengths, row)."""
+    """Rows whose favourites crowd into few residues modulo 16 or 64, so that the list comes out long: (its length, row)."""
     rng = np.random.default_rng(1000 * n + k + seed)
     for modulo, residues, each in [(16, 1, 32), (16, 2, 16), (16, 3, 12), (16, 4, 10), (16, 5, 16), (16, k, 8), (64, k, 8), (64, k - 1, 8), (16, 1, 14), (32, k, 4)]:
         row = rng.normal(0, 1, n).astype(np.float32)
         for r in rng.permutation(modulo)[:max(residues, 1)]:
             row[r::modulo][:each] += np.float32(8)
-        yield list_lengths(row, k), row
+        yield list_length(row, k), row

@@ -666,14 +666,14 @@ def test_one_buffer_for_two_results(g, oracle, H, F, E, k, gate_t, down_t, share
 
 @pytest.mark.parametrize("E,k", [(64, 10), (64, 12), (128, 10), (128, 14), (256, 8), (256, 13), (512, 10), (512, 12)])
 def test_selection_lists_of_any_length(g, oracle, E, k):
-    """Routers whose favourites crowd into few residues, so that the list of candidates is made a second time, for every number of logits per lane."""
+    """Routers whose favourites crowd into few residues, so that the list of candidates is ranked in the long form, for every number of logits per lane."""
     import selection_rule as rule
     H, F = 512, 32
     L = synth.make_layer(H, F, E, k, synth.Q8_0, synth.Q8_0, False, seed=SEED, layer=E + k)
     x = synth.rms_normed(synth.rng_for(SEED, 97, E), H)
     long = 0
-    for lengths, row in rule.crowded_rows(E, k):
+    for _, row in rule.crowded_rows(E, k):
         Lr = dict(L, router=np.outer(row, x / np.float32(np.dot(x, x))).astype(np.float32))
         check_layer(g, oracle, Lr, x)
-        long += rule.list_lengths(oracle.router_logits(Lr["router"], x), k, wide=False)[0] > 32
+        long += rule.list_length(oracle.router_logits(Lr["router"], x), k, wide=False) > 32
     assert long > 0 or E == 64

@@ -582,8 +582,7 @@ WD_DEV void topk_wave(const float *logits, int n, int k, float w_scale, int32_t 
 //     lanes (the rows hold the same sixteen, each turned by four lanes more than the one before); T, the (k+1)-th of them, is a lower bound of the
 //     (k+1)-th largest key.  From k = 12 on sixteen groups exclude too little: 32 groups of lanes equal modulo 32;
 //   * the keys not below T - 18 or so of 512 - are compacted into LDS with their experts and ranked by counting, one half of the wave against the
-//     first sixteen of the list and the other against the second; a longer one, by uniform reads, one of more than 64 after it was made
-//     again with T from the largest keys of the 64 lanes;
+//     first sixteen of the list and the other against the second (a longer list, by uniform reads);
 //   * rank r goes to slot r.  Equal keys collide there and leave the slot behind them empty.
 // The slots are accepted as the selection only when the first k are filled, and the (k+1)-th too unless every expert is selected, and the
 // differences d_j = l_j - l_0, as the reference takes them ahead of its exponentials, fall by kSelGap from one to the next and by kSelGapLast from the k-th to the
@@ -606,8 +605,8 @@ constexpr uint32_t kSelFinite = 0x00800000u;  // keys from here on are above -in
 
 // Step A.  Returns with st.fast, and for accepted rows the ids of the selection in lanes 0..k-1 of every row of lanes of st.id.
 // Of the scratch it uses the candidates' and the selection's places only (rmx, cl, ce; sel, selp).
-// MORE false: k < 12 only.
-template <int M, bool MORE = true>
+// FEW (k < 12 only): fewer registers, for the resident stack.
+template <int M, bool FEW = false>
 WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s, int lane, SelWaveState &st) {
     constexpr int kEq = 32, kUgt = 34, kUge = 35, kOge = 3;  // of the compares into scalar masks
     uint32_t *const ck = reinterpret_cast<uint32_t *>(s.rmx);  // [64] keys of the candidates,
@@ -631,7 +630,7 @@ WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s
     const wd_uint2v h32 = swap32(head);
     head = max(h32.x, h32.y);
     int larger = 0;
-    if (!MORE || M == 1 || __builtin_expect(k < 12, 1)) {
+    if (FEW || M == 1 || __builtin_expect(k < 12, 1)) {
         const wd_uint2v h16 = swap16(head);
         head = max(h16.x, h16.y);
         int turned = dpp_i<kDppRor4, 0xa>(static_cast<int>(head), static_cast<int>(head));
@@ -661,7 +660,7 @@ WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s
     for (int i = 0; i < M; ++i) m[i] = __builtin_amdgcn_uicmp(h[i], thr, kUge);
 #pragma unroll
     for (int i = 0; i < M; ++i) first[i + 1] = first[i] + static_cast<int>(__builtin_popcountll(m[i]));
-    int count = first[M];
+    const int count = first[M];
     // every lane writes each of its keys, no branch: what is no candidate, and what a list of more than 32 has too much, goes behind the 32 places
 #pragma unroll
     for (int i = 0; i < M; ++i) {
@@ -676,57 +675,41 @@ WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s
 #pragma unroll
     for (int i = 0; i < 4; ++i) q[i] = reinterpret_cast<const uint4 *>(ck)[4 * (lane >> 5) + i];
     asm volatile("" : "+v"(id));  // (asked for here and not where it is used)
-    unsigned long long ahead[16];
+    if (__builtin_expect(count <= 32, 1)) {
+        unsigned long long ahead[16];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        ahead[4 * i] = __builtin_amdgcn_uicmp(q[i].x, key, kUgt), ahead[4 * i + 1] = __builtin_amdgcn_uicmp(q[i].y, key, kUgt),
-        ahead[4 * i + 2] = __builtin_amdgcn_uicmp(q[i].z, key, kUgt), ahead[4 * i + 3] = __builtin_amdgcn_uicmp(q[i].w, key, kUgt);
+        for (int i = 0; i < 4; ++i)
+            ahead[4 * i] = __builtin_amdgcn_uicmp(q[i].x, key, kUgt), ahead[4 * i + 1] = __builtin_amdgcn_uicmp(q[i].y, key, kUgt),
+            ahead[4 * i + 2] = __builtin_amdgcn_uicmp(q[i].z, key, kUgt), ahead[4 * i + 3] = __builtin_amdgcn_uicmp(q[i].w, key, kUgt);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) rank += __builtin_amdgcn_inverse_ballot_w64(ahead[i]) ? 1 : 0;
-    const wd_uint2v both = swap32(static_cast<uint32_t>(rank));
-    rank = static_cast<int>(both.x + both.y);
-    if (__builtin_expect(count > 32, 0)) {  // about one row in a thousand of random logits (ten of 512), and every row whose favourites crowd into few groups
-        // (the keys worked out again, one at a time: held until here they cost the resident stack its last registers)
-        auto again = [&](int i) {
-            uint32_t b = f_bits(lv[i]);
-            asm volatile("" : "+v"(b));
-            return b ^ (static_cast<uint32_t>(static_cast<int>(b) >> 31) | 0x80000000u);
-        };
-        uint32_t from = thr;
-        if (count > 64) {  // by the largest key of every lane the list is as short as any grouping can make it: at most (k + 1) M
-            uint32_t best = 0u;
-#pragma unroll
-            for (int i = 0; i < M; ++i) best = max(best, again(i));
-            larger = 0;
-#pragma nounroll
-            for (int src = 0; src < 64; src += 4) {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) larger += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(best), src + u)) > best ? 1 : 0;
-            }
-            unsigned long long on = 0ull;  // lanes of the (k+1)-th: of equal ones none need have k above it, and the largest has none
-#pragma nounroll
-            for (int above = k; on == 0ull; --above) on = __builtin_amdgcn_uicmp(static_cast<uint32_t>(larger), static_cast<uint32_t>(above), kEq);
-            from = max(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(best), __builtin_ctzll(on))), kSelFinite);
-        }
+        for (int i = 0; i < 16; ++i) rank += __builtin_amdgcn_inverse_ballot_w64(ahead[i]) ? 1 : 0;
+        const wd_uint2v t = swap32(static_cast<uint32_t>(rank));
+        rank = static_cast<int>(t.x + t.y);
+    } else if (!FEW || count <= 64) {
+        int base = 0;
         ck[lane] = 0u;
         wave_lds_fence();
-        count = 0;
 #pragma unroll
         for (int i = 0; i < M; ++i) {
-            const uint32_t h_i = again(i);
-            const unsigned long long in = __builtin_amdgcn_uicmp(h_i, from, kUge);
-            const int place = min(count + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(in >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(in), 0u))), 63);
-            if (h_i >= from) ck[place] = h_i, cid[place] = 64 * i + lane;
-            count += static_cast<int>(__builtin_popcountll(in));
+            uint32_t h_i = h[i];
+            unsigned long long in = m[i];
+            int before = first[i];
+            if (FEW) {  // (worked out again: held until here they cost the resident stack its last registers)
+                h_i = f_bits(lv[i]);
+                asm volatile("" : "+v"(h_i));
+                h_i ^= static_cast<uint32_t>(static_cast<int>(h_i) >> 31) | 0x80000000u;
+                in = __builtin_amdgcn_uicmp(h_i, thr, kUge), before = base;
+                base += static_cast<int>(__builtin_popcountll(in));
+            }
+            before += static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(in >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(in), 0u)));
+            if (h_i >= thr) ck[min(before, 63)] = h_i, cid[min(before, 63)] = 64 * i + lane;  // (a list of more than 64 is not used)
         }
         wave_lds_fence();
-        key = ck[lane], id = cid[lane], rank = 0;
-        if (count <= 64) {  // (a longer one is not used)
+        key = ck[lane], id = cid[lane];
 #pragma nounroll
-            for (int src = 0; src < count; src += 4) {
+        for (int src = 0; src < 64; src += 4) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) rank += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), src + u)) > key ? 1 : 0;
-            }
+            for (int u = 0; u < 4; ++u) rank += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), src + u)) > key ? 1 : 0;
         }
     }
     if (key != 0u && rank <= k) s.sel[rank] = static_cast<int>(key), s.selp[rank] = bits_f(static_cast<uint32_t>(id));

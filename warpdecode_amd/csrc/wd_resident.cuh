@@ -1014,7 +1014,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         bool weights_out = false;
         if (r == 0 && !traced) {
             (void)gather_logits(true);
-            sel_wave_ids<8, false>(lv, a.E, a.k, scratch, lane, st);
+            sel_wave_ids<8, true>(lv, a.E, a.k, scratch, lane, st);
             if (st.fast) {
                 publish_ids(st.id);
             } else {
@@ -1049,7 +1049,7 @@ WD_DEV void res_router_role(const ResidentArgs &a, uint8_t *lds_base, int r0, in
         if (r == 0 && !traced && !weights_out) weights_from_lds();
         if (r == 0 && traced) {
             if (!got) (void)gather_logits(true);
-            sel_wave_ids<8, false>(lv, a.E, a.k, scratch, lane, st);
+            sel_wave_ids<8, true>(lv, a.E, a.k, scratch, lane, st);
             res_mark<STAMPS>(a, c, l, 13);
         }
         __syncthreads();  // B3
