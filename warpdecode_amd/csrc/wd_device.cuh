@@ -244,10 +244,6 @@ template <typename T>
 WD_DEV T lane_down(T v, int delta) {
     return __shfl_down(v, delta, kWave);
 }
-template <typename T>
-WD_DEV T lane_get(T v, int src) {
-    return __shfl(v, src, kWave);
-}
 
 // Orders this wave's LDS traffic for cross-lane hand-offs through LDS.  The hardware
 // executes a wave's LDS instructions in order; the fence keeps the compiler from moving

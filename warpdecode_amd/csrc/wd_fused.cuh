@@ -379,14 +379,16 @@ template <int M>
 struct TopkLds {
     float *p, *gsum, *rmx, *cl, *ce, *rest, *selp;
     int *cid, *ncand, *sel;
+    static constexpr int kRows = 32, kList = 64;
+    static_assert(kRows + 2 * kList >= 2 * 64, "rmx, cl and ce as one: the one-wave form's 64 keys and their 64 experts");
     WD_DEV explicit TopkLds(uint8_t *lds) {
         p = reinterpret_cast<float *>(lds);        // [512 M] exponentials by expert id
         gsum = p + 512 * M;                        // [64 M] per-8 sums by group
-        rmx = gsum + 64 * M;                       // [32] largest logit of every row of 16 lanes
-        cl = rmx + 32;                             // [64] candidates: logit,
-        ce = cl + 64;                              // [64] exponential,
-        cid = reinterpret_cast<int *>(ce + 64);    // [64] id
-        ncand = cid + 64;                          // [4] their number
+        rmx = gsum + 64 * M;                       // [kRows] largest logit of every row of 16 lanes
+        cl = rmx + kRows;                          // [kList] candidates: logit,
+        ce = cl + kList;                           // [kList] exponential,
+        cid = reinterpret_cast<int *>(ce + kList); // [kList] id
+        ncand = cid + kList;                       // [4] their number
         sel = ncand + 4;                           // [16] the r-th selected id
         selp = reinterpret_cast<float *>(sel + 16);  // [16] its exponential
         rest = selp + 16;                          // [8] largest exponential outside the candidates, by wave
@@ -582,7 +584,8 @@ WD_DEV void topk_wave(const float *logits, int n, int k, float w_scale, int32_t 
 //     lanes (the rows hold the same sixteen, each turned by four lanes more than the one before); T, the (k+1)-th of them, is a lower bound of the
 //     (k+1)-th largest key.  From k = 12 on sixteen groups exclude too little: 32 groups of lanes equal modulo 32;
 //   * the keys not below T - 18 or so of 512 - are compacted into LDS with their experts and ranked by counting, one half of the wave against the
-//     first sixteen of the list and the other against the second (a longer list, by uniform reads);
+//     first sixteen of the list and the other against the second; lists of 33 to 64 (one row in a thousand of random logits, ten of 512, and rows whose
+//     favourites crowd into few groups), by uniform reads; longer ones are not accepted;
 //   * rank r goes to slot r.  Equal keys collide there and leave the slot behind them empty.
 // The slots are accepted as the selection only when the first k are filled, and the (k+1)-th too unless every expert is selected, and the
 // differences d_j = l_j - l_0, as the reference takes them ahead of its exponentials, fall by kSelGap from one to the next and by kSelGapLast from the k-th to the
@@ -591,10 +594,8 @@ WD_DEV void topk_wave(const float *logits, int n, int k, float w_scale, int32_t 
 // to the (k+1)-th): probabilities, products with one 1/sum in [2^-10, 1], stay strictly ordered, and exp itself is not needed before the ids are out.
 // Rows the test does not accept (ties, near-ties, NaN, +inf, fewer than k + 1 finite logits, selected exponentials below
 // 2^-100) take the reference's rungs over all probabilities in step B.
-// Alone on the device, from the logits in registers until the ids are on their way: 512 experts of which 10 1,810 cycles (0.75 us), 256 of which
-// 8 1,510, 128 of which 8 1,390, 64 of which 6 1,220.  (Groups of two lanes, keys of 23 bits ranked by uniform reads, a branch for every key that may go
-// into the list, and the exponentials ahead of the ids: 3,770 (1.45 us), 2,970, 2,640, 2,130.  The stack of 48 layers with the router's ids: 795, so 752 us;
-// 64 experts of Q8_0 756, 718; layers of 2560 / 640 24.5, 23.4 each; 64 experts of 1024 / 256 11.7, 11.1.)
+// Alone on the device, from the logits in registers until the ids are on their way: 512 experts of which 10 1,810 cycles (0.75 us), 64 of which 6 1,220; by uniform
+// reads over keys of 23 bits, with the exponentials ahead of the ids, 3,770 and 2,130.
 struct SelWaveState {
     float d;       // every row of lanes, lane j < k of it: the j-th largest logit minus the largest (accepted rows)
     int id;        // its expert
@@ -605,7 +606,7 @@ constexpr uint32_t kSelFinite = 0x00800000u;  // keys from here on are above -in
 
 // Step A.  Returns with st.fast, and for accepted rows the ids of the selection in lanes 0..k-1 of every row of lanes of st.id.
 // Of the scratch it uses the candidates' and the selection's places only (rmx, cl, ce; sel, selp).
-// FEW (k < 12 only): fewer registers, for the resident stack.
+// FEW (k < 12 only): fewer registers, for the resident stack.  (48 layers whose lists are of 33 to 64: 13.45 us each, left to step B 16.6; with a trace 10.3, 12.25.)
 template <int M, bool FEW = false>
 WD_DEV void sel_wave_ids(const float (&lv)[M], int n, int k, const TopkLds<1> &s, int lane, SelWaveState &st) {
     constexpr int kEq = 32, kUgt = 34, kUge = 35, kOge = 3;  // of the compares into scalar masks
@@ -876,8 +877,8 @@ WD_DEV bool topk_two_waves(const HandRow &row, int k, float w_scale, int32_t *id
 
 // Every thread of the workgroup must call it.  Two waves select where one can hold the row (n <= 512, k <= 15); ids and weights are left in
 // LDS by wave 0.
-// (Before the former's differences: 64 experts, top-6: the ids are out 1.5 us after the logits, by the block form 3.0 - with fewer rows of lanes than
-// there are experts to select its threshold excludes nobody -; 512 experts, top-10: 2.1, 2.2.)
+// (The block form takes 3.0 us from the logits to the ids for 6 of 64 experts - with fewer rows of lanes than there are experts to select its threshold
+// excludes nobody - and 2.2 for 10 of 512.)
 WD_DEV bool topk_block(const HandRow &row, int k, float w_scale, int32_t *ids, float *weights, const int32_t *__restrict__ override_ids,
                        uint8_t *lds, int lane, int wave, unsigned long long *stamps = nullptr, uint32_t *tagged = nullptr, int tag_side = 0) {
     const int n = row.n;
@@ -1245,10 +1246,8 @@ __global__ __launch_bounds__(512, (2 * kAbPerCu<TYPE, FETCH, LOOP>)) void k_laye
         return static_cast<int>(id);
     };
     // One item per workgroup unless the grid was capped (LOOP).  Behind the first one the waves go on by themselves: nothing of what they share is
-    // written again, and the ids come together, so that each wave reads the next item's where it lies.  (With the first wave reading it for all,
-    // between two barriers, an item begins when the slowest wave of the one before is done.  us per layer, so / as it is: 4096 / 1536 IQ3_S, 128
-    // experts top-8, 36.8 / 36.0; 5120 / 1024 40.8 / 39.9; 2560 / 640, where an eighth of the workgroups has a second item, 22.35 / 22.41, IQ2_S 21.2 / 21.2.
-    // The id asked for an item ahead was 0.2 faster at 4096 and 0.05 slower at 2560.)
+    // written again, and the ids come together, so that each wave reads the next item's where it lies.  (Between two barriers an item begins when the slowest
+    // wave of the one before is done: 4096 / 1536 IQ3_S, eight of 128 experts, 36.8 us per layer, so 36.0; 2560 / 640, where few workgroups have a second item, the same.)
     int item = bw;
     bool first = true;
     do {

@@ -387,7 +387,7 @@ struct ResCtx {
     WD_DEV unsigned *arrived() const { return reinterpret_cast<unsigned *>(lds + kResLdsActv + 48); }
     // Where the layer's activations land, slot by slot.  With a routing trace in the slots' areas; without one where nothing else lies then, so that a wave's down
     // rows can be in its area before they come: the rungs' in the places of the rows decoded ahead, the shared expert's in that of the codebook that the launch has not staged.
-    // (In the areas in either mode, the rows staged behind a barrier more: 48 layers, IQ3_S 652 / so 633 us, Q8_0 710 / 701.)
+    // (48 layers in the areas, the rows staged behind a barrier more: IQ3_S 652 us, so 633.)
     WD_DEV float *land(bool apart, int s, int spare) const {
         return reinterpret_cast<float *>(lds + (apart ? (s < kResMaxK ? kResLdsKept + 2048 * s : spare) : kResLdsLand + 2048 * s));
     }

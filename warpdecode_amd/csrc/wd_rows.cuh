@@ -1005,7 +1005,7 @@ WD_DEV Q8Block q8_load(const uint8_t *blk) {
 // The IQ4_NL codebook values of the low and of the high 4-bit codes of four bytes, each as four int8: the 16 values are four dwords, v_perm_b32
 // picks among eight bytes, so the codes' low three bits select in both halves of the table and bit 3, moved to where it is worth four, picks one of the
 // two results in a third step (src/lowbit.cuh:1648-1668 reads kvalues_iq4nl[code]).  (As a byte mask instead - bit 3 times 255 - it takes the 32-bit multiply, which runs
-// at a quarter of the rate: 2560 / 640, ten IQ4_NL experts and the shared one, with the fold as it is now 22.6 us per layer, so 22.3; four tokens 57.9, 57.3.)
+// at a quarter of the rate; layers of 2560 / 640, ten IQ4_NL experts and the shared one, take the same either way, 20.9 us, and four tokens 59.4.)
 WD_DEV uint32_t iq4nl_pick(uint32_t sel, uint32_t bit3_at_2) {
     // {-127, -104, -83, -65}, {-49, -35, -22, -10}, {1, 13, 25, 38}, {53, 69, 89, 113}
     constexpr uint32_t t0 = 0xbfad9881u, t1 = 0xf6eaddcfu, t2 = 0x26190d01u, t3 = 0x71594535u;
