@@ -93,9 +93,10 @@ def test_layer_with_combine(g, oracle, flags, shape):
 
 @pytest.mark.parametrize("H,F,k,gate_t,down_t,shared", [(2304, 800, 3, synth.IQ2_S, synth.IQ4_NL, True), (4352, 1024, 10, synth.IQ2_S, synth.IQ4_NL, True),
                                                         (4352, 800, 11, synth.Q8_0, synth.Q8_0, False), (2560, 544, 16, synth.IQ2_S, synth.Q8_0, True),
-                                                        (2304, 768, 16, synth.Q8_0, synth.IQ4_NL, True)])
+                                                        (2304, 768, 16, synth.Q8_0, synth.IQ4_NL, True), (4352, 544, 15, synth.IQ2_S, synth.IQ4_NL, True),
+                                                        (4608, 768, 13, synth.Q8_0, synth.Q8_0, False), (4352, 640, 13, synth.Q8_0, synth.IQ4_NL, False), (4352, 704, 15, synth.IQ2_S, synth.Q8_0, True)])
 def test_combine_where_two_down_workgroups_share_a_compute_unit(g, oracle, H, F, k, gate_t, down_t, shared):
-    """More than 256 workgroups of the down projections: the forms of 25..32 blocks per row and of two matrices per wave that are made for two per compute unit."""
+    """More than 256 workgroups of the down projections: the forms of 25..32 blocks per row, of two matrices per wave and of thirteen matrices and more that are made for two per compute unit."""
     E = 24
     L = synth.make_layer(H, F, E, k, gate_t, down_t, shared, seed=SEED, layer=900 + k, router_sigma=1.0 / np.sqrt(H))
     rng = synth.rng_for(SEED, 503, H, k)

@@ -55,6 +55,12 @@ def test_two_workgroups_of_down_projections_fit_a_compute_unit(kernels, args):
     assert vgprs <= 80 and scratch == 0 and spills == 0, (vgprs, scratch, spills)
 
 
+@pytest.mark.parametrize("kind", [0, 1])
+def test_two_workgroups_of_sixteen_waves_fit_a_compute_unit(kernels, kind):
+    vgprs, scratch, spills = _kernel(kernels, "k_layer_c8", kind, 3, False, False, False, False, False)
+    assert vgprs <= 64 and scratch == 0 and spills == 0, (vgprs, scratch, spills)
+
+
 def test_spills_of_the_token_batch_at_ten_super_blocks(kernels):
     """Three workgroups per compute unit, bought with a few spills: not with more than when the figures beside the kernel were taken."""
     vgprs, scratch, spills = _kernel(kernels, "k_tokens_ab", 22, 4, 10)

@@ -1522,11 +1522,13 @@ __host__ __device__ inline uint32_t layer_c8_wave_bytes(int F) {
 // at most 80 registers.  Rows of 25..32 blocks that a lane loads itself stay below by asking for what the fold needs behind the quantisation
 // (kLate; eleven IQ4_NL matrices, 5120 / 1024: 46.2 us per layer with 83 registers, 42.8 with 78); two matrices per wave of 17..24 blocks by the
 // general quantisation (ORDINARY false: 5120 / 768 IQ4_NL 53.2 with 87, 50.7 with 79; where one workgroup per compute unit is all there is, 2048 / 768, the
-// ordinary one is the faster, 22.3 against 23.1).
+// ordinary one is the faster, 22.3 against 23.1).  Thirteen to sixteen matrices of 17..24 blocks need eight waves per SIMD, 64 registers: the general quantisation, and
+// what the fold needs asked for behind the chains (kLast; us of the dispatch at 5120 / 768 with 73 registers, asked for behind the quantisation with 70, so: thirteen IQ4_NL
+// 14.3, 15.5, 12.0, sixteen 16.2, 17.4, 13.8; Q8_0, 73, 60 and 60 registers, 15.5, 13.7, 13.7 and 18.8, 17.0, 17.1).
 template <int KIND, int PASSES, bool WORDS, bool PART = false, bool TRACE = false, bool TWO = false, bool ORDINARY = true>
-__global__ __launch_bounds__(TWO ? 576 : 1024, (TWO ? !ORDINARY : PASSES == 4 && !WORDS && !PART && !TRACE) ? 6 : 1) void k_layer_c8(LayerArgs a) {
+__global__ __launch_bounds__(TWO ? 576 : 1024, TWO ? (ORDINARY ? 1 : 6) : !ORDINARY ? 8 : PASSES == 4 && !WORDS && !PART && !TRACE ? 6 : 1) void k_layer_c8(LayerArgs a) {
     constexpr int STEPS = (PASSES + 1) / 2;  // of sixteen blocks
-    constexpr bool kLate = PASSES == 4 && !WORDS;
+    constexpr bool kLast = !TWO && !ORDINARY, kLate = (PASSES == 4 && !WORDS) || kLast;
     extern __shared__ __align__(16) uint8_t lds_c8[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int n_act = a.k + (a.sh_inp ? 1 : 0);
@@ -1540,13 +1542,14 @@ __global__ __launch_bounds__(TWO ? 576 : 1024, (TWO ? !ORDINARY : PASSES == 4 &&
     if (a.dry) return;
     layer_clear_handed(a, 64 * (TWO ? 9 : n_act));
     mark<TRACE>(a, 2, 0);
-    const StreamOps stream = layer_c_stream_request(a, wave < 2, lane);
+    StreamOps stream;
+    if (!kLast) stream = layer_c_stream_request(a, wave < 2, lane);
     FoldOps ops;
     float stream_w = 0.0f;
     int m = TWO ? wave : min(wave, n_act - 1);  // (a second wave without a matrix of its own repeats the first's)
     do {
         int lane = threadIdx.x & 63;
-        if constexpr (TWO) asm volatile("" : "+v"(lane));  // (nothing per lane is kept from one matrix to the next: it would take 30 registers)
+        if constexpr (TWO || kLast) asm volatile("" : "+v"(lane));  // (nothing per lane is kept from one matrix to the next: it would take 30 registers)
         const bool is_shared = m == a.k, q8 = KIND == 0 || is_shared;
         // the activation first: its address needs no expert id, and loads return in order - it is quantised while the weights are
         // still on their way
@@ -1565,11 +1568,11 @@ __global__ __launch_bounds__(TWO ? 576 : 1024, (TWO ? !ORDINARY : PASSES == 4 &&
             typename std::conditional<WORDS, Q8Rows8Fetch<K, STEPS>, Q8Rows8Blocks<K, PASSES>>::type fetch;
             fetch.request(rows, nb, lane);
             if (!kLate && wave < 2 && (!TWO || m < 9)) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
-            if (kLate) stream_w = layer_c_stream_weight(a, stream, wave < 2);
+            if (kLate && !kLast) stream_w = layer_c_stream_weight(a, stream, wave < 2);
 #pragma unroll
             for (int i = 0; i < STEPS; ++i)
                 lds_quantize_q8_0_step<ORDINARY>(v[2 * i], v[2 * i + 1], 512 * i + lane * 8 < a.F, 512 * i + lane * 8, aq, ad, lane);
-            if (kLate && wave < 2) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+            if (kLate && !kLast && wave < 2) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
             if (!kLate && (!TWO || m < 9)) stream_w = layer_c_stream_weight(a, stream, wave < 2);
             mark<TRACE>(a, 2, 1);
             Q8Chain ch;
@@ -1599,6 +1602,11 @@ __global__ __launch_bounds__(TWO ? 576 : 1024, (TWO ? !ORDINARY : PASSES == 4 &&
         if (wave < n_act && (lane & 7) == 0) ybuf[m * 8 + (lane >> 3)] = or_nan(y, missing);
         m += 9;
     } while (TWO && m < n_act);
+    if (kLast) {
+        stream = layer_c_stream_request(a, wave < 2, lane);
+        if (wave < 2) ops = layer_c_fold_request(a, r0 + 4 * wave, 4, lane);
+        stream_w = layer_c_stream_weight(a, stream, wave < 2);
+    }
     mark<TRACE>(a, 2, 2);
     __syncthreads();
     mark<TRACE>(a, 2, 3);

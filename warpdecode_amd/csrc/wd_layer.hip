@@ -675,6 +675,8 @@ void launch_layer_c8(hipStream_t st, const LayerArgs &a) {
         enqueue(k_layer_c8<KIND, PASSES, WORDS, true>, grid, block, lds, st, a);
     else if (a.trace)
         enqueue(k_layer_c8<KIND, PASSES, WORDS, false, true>, grid, block, lds, st, a);
+    else if (PASSES == 3 && n_act > 12 && a.H > 2048)  // more workgroups than compute units: the form of which two fit one
+        enqueue(k_layer_c8<KIND, PASSES, WORDS, false, false, false, PASSES != 3>, grid, block, lds, st, a);
     else
         enqueue(k_layer_c8<KIND, PASSES, WORDS>, grid, block, lds, st, a);
 }
